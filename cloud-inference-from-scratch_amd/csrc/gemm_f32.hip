@@ -1,85 +1,486 @@
-// True float32 matrix product for the 32-bit path: C = A * W^T (+ bias).
-//   A [M, K] row-major (row stride lda), W [N, K] row-major (a Linear's weight), C [M, N].
-// Plain fused multiply-adds in float32, no matrix-core reduced-precision mode.
-// Every output element is a sum over k in one fixed order (blocks of 256 k summed one after the other, the
-// blocks' sums added in turn: the rounding error grows with 256 + K/256 terms, not with K), so a row's result
-// does not depend on how many other rows are in the batch.
-// 64x64 output tile per workgroup, 16-deep k slices through LDS, 4x4 per thread.
+// True float32 matrix product for the 32-bit path: C = A * W^T (+ bias), or the gated unit of its two halves.
+//   A [M, K] row-major (row stride lda), W [N, K] row-major (a Linear's weight), C [M, N] (row stride ldc);
+//   with the gate: C [M, N / 2] = silu(first half of the columns) * (second half).
+// Float32 matrix instructions (v_mfma_f32_16x16x4_f32: float32 products and sums, no reduced-precision mode).
+//
+// Every output element is the same sum in the same order in every form below, so a row's result does not depend on
+// how many other rows are in the batch: K in blocks of 256, the sum of two chains of 128 in which
+// k ascends (an instruction takes four neighbouring k); the sums of four blocks are added one after the other, and so are the sums of these stretches of 1,024 k
+// (the rounding error grows with 128 + 1 + 4 + K/1024 terms, not with K).
+//
+// Two forms:
+//
+// * gemm_f32_rows_kernel, few rows: bound by the stream of W.  A workgroup owns 8 to 32 columns and 8 to 32 rows and
+//   goes on to the next columns until none are left; its waves take the blocks of K in turn, each wave fetching W and
+//   A as 128-byte row segments (8 lanes to a segment: a load in which every lane reads another row keeps the address
+//   unit busy four times as long), four 32-wide pieces ahead in registers and across the end of a tile, and turning
+//   them into operand order in 2 KB of LDS per 16 rows of its own.  The blocks' sums meet in LDS and are added in
+//   order.
+// * gemm_f32_tile_kernel, more rows: bound by the matrix cores (256 flops a cycle and unit; 157 TFLOP/s).  Four waves
+//   share a tile of 64 x 64 through two stages of LDS in 32-wide slices, the four following slices on their way in
+//   registers (one slice ahead a tile alone on its unit took twice as long: 89 -> 45 us at 256 rows, N = K = 2,048).
+//   Where the tiles leave units idle a workgroup takes one stretch of K and leaves its sum in a workspace, and
+//   gemm_f32_join_kernel adds the stretches in order.
+//
+// Measured (MI355X, us): 4 rows: N 22,016, K 2,048 42 (4.3 TB/s), N 2,048, K 11,008 27 (3.4 TB/s), N = K = 2,048 10;
+// 517 rows: 473 (99 TFLOP/s), 264 with K in stretches (88 TFLOP/s; 420 without), 68; 2,048 rows: 1,622 (114 TFLOP/s),
+// 824, 170.  Plain fused multiply-adds in tiles of 64 x 64, whatever the rows, took 370 for the median product of a step
+// of 4 rows and 833 of one of 517 (23 TFLOP/s).
 #include "common.h"
 
 namespace {
-constexpr int BM = 64, BN = 64, BK = 16;
-constexpr int kSlicesPerBlock = 16;  // 256 k: a block's sum joins the total
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kBlockK = 256;   // a block of K: its sum joins the total
+constexpr int kPiece = 32;     // k of a piece: 128 bytes of a row
+constexpr int kPiecesPerBlock = kBlockK / kPiece;
+constexpr int kPiecesPerChain = kPiecesPerBlock / 2;
+constexpr int kBlocksPerStretch = 4;
+constexpr int kStretch = kBlockK * kBlocksPerStretch;
+constexpr int kTileFloats = 16 * kPiece;  // 16 rows of a piece
+
+// 16-byte chunk `c` (0..7) of row `row` in a tile whose rows are 128 bytes: the chunks of 16 rows that a quarter wave
+// reads at one time lie in different banks.
+__device__ __forceinline__ int chunk_at(int row, int c) { return row * kPiece + 4 * (c ^ ((row >> 1) & 7)); }
+
+// The numbers k = 16 g + 4 t + q of a row for t = 0..3, where q is the lane's quarter: what four instructions in turn take
+// of 16 k.  (Four 4-byte reads; one 16-byte read and a transposition over the quarters with row swaps made the products
+// of many rows 20 % slower, and one 16-byte read with the k in another order 2 % faster.)
+__device__ __forceinline__ floatx4 operand(const float* tile, int row, int g, int q) {
+    floatx4 v;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[t] = tile[chunk_at(row, 4 * g + t) + q];
+    return v;
 }
 
-__global__ void __launch_bounds__(256)
-gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                const float* __restrict__ bias, float* __restrict__ C, int M, int N, int K,
-                int lda, int ldc) {
-    __shared__ float a_tile[BK][BM + 4];
-    __shared__ float w_tile[BK][BN + 4];
-    const int m0 = blockIdx.y * BM;
-    const int n0 = blockIdx.x * BN;
-    const int tx = threadIdx.x % 16;
-    const int ty = threadIdx.x / 16;
-    float acc[4][4] = {}, total[4][4] = {};
-    int slice = 0;
-    for (int k0 = 0; k0 < K; k0 += BK) {
+// Four values of a row from k on; what lies past K is 0 (`inside`).  kVec: K and the row's start are multiples of
+// four numbers.  The load stands under no condition (a piece past the end reads the row's start again), so that the
+// compiler can count the loads that are under way.
+template <bool kVec>
+__device__ __forceinline__ floatx4 load4(const float* __restrict__ row, int k, int K) {
+    if constexpr (kVec) {
+        return *reinterpret_cast<const floatx4*>(row + (k < K ? k : 0));
+    } else {
+        floatx4 v;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = threadIdx.x + 256 * r;
-            const int row = idx / BK;
-            const int kk = idx % BK;
-            const int k = k0 + kk;
-            const int m = m0 + row;
-            const int n = n0 + row;
-            a_tile[kk][row] = (m < M && k < K) ? A[static_cast<size_t>(m) * lda + k] : 0.f;
-            w_tile[kk][row] = (n < N && k < K) ? W[static_cast<size_t>(n) * K + k] : 0.f;
+        for (int j = 0; j < 4; ++j) v[j] = row[k + j < K ? k + j : 0];
+        return v;
+    }
+}
+
+template <bool kVec>
+__device__ __forceinline__ floatx4 inside(floatx4 v, int k, int K) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (kVec ? k : k + j) < K ? v[j] : 0.f;
+    return v;
+}
+
+__device__ __forceinline__ float gated(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
+
+// kRows rows (8, 16 or 32) by kColumns columns (8, 16 or 32; with the gate kColumns / 2 of each half), in tiles of 16
+// of which the last may be half empty.  kWaves waves share K.  Workgroup x takes the columns' tiles x, x + gridDim.x, ...
+template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec>
+__global__ void __launch_bounds__(kWaves * kWave)
+gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                     float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
+    constexpr int kRowTiles = (kRows + 15) / 16, kColumnTiles = (kColumns + 15) / 16;
+    constexpr int kTiles = kRowTiles + kColumnTiles;
+    constexpr int kSums = kRowTiles * kColumnTiles * 256;
+    constexpr int kAhead = kPiecesPerChain;  // pieces on their way
+    constexpr int kThreads = kWaves * kWave;
+    constexpr int kOwned = (kSums + kThreads - 1) / kThreads;
+    constexpr int kStep = kGate ? kColumns / 2 : kColumns;  // output columns of a tile
+    static_assert(!kGate || kColumns == 32 || kColumns == 16, "a gate's tile holds as many columns of either half");
+    __shared__ float stage_all[kWaves * kTiles * kTileFloats];
+    __shared__ float sums[2][kWaves * kSums];
+    const int lane = threadIdx.x % kWave;
+    const int wave = threadIdx.x / kWave;
+    float* stage = stage_all + wave * kTiles * kTileFloats;
+    const int m0 = blockIdx.y * kRows;
+    const int width = kGate ? N / 2 : N;  // output columns
+    const int column_tiles = (width + kStep - 1) / kStep;
+    const int blocks = (K + kBlockK - 1) / kBlockK;
+    const int rounds = (blocks + kWaves - 1) / kWaves;
+
+    // row r (0..kColumns - 1) of a tile of W
+    auto weight_row = [&](int tile, int r) {
+        const int n = kGate ? min(tile * kStep + r % kStep, width - 1) + (r / kStep) * width : min(tile * kStep + r, N - 1);
+        return W + static_cast<size_t>(n) * K;
+    };
+    constexpr int kWLoads = kColumns / 8, kALoads = kRows / 8;
+    const int chunk = lane % 8;
+    const float* a_row[kALoads];
+#pragma unroll
+    for (int i = 0; i < kALoads; ++i) a_row[i] = A + static_cast<size_t>(min(m0 + 8 * i + lane / 8, M - 1)) * lda;
+
+    // the piece that is fetched next: its place in the block, the round and the tile
+    int f_piece = 0, f_round = 0, f_tile = blockIdx.x;
+    const float* w_row[kWLoads];
+#pragma unroll
+    for (int i = 0; i < kWLoads; ++i) w_row[i] = weight_row(f_tile, 8 * i + lane / 8);
+    floatx4 w_ahead[kAhead][kWLoads], a_ahead[kAhead][kALoads];
+    auto fetch = [&](floatx4 (&w)[kWLoads], floatx4 (&a)[kALoads]) {
+        const int k = (wave + f_round * kWaves) * kBlockK + f_piece * kPiece + 4 * chunk;
+#pragma unroll
+        for (int i = 0; i < kWLoads; ++i) w[i] = load4<kVec>(w_row[i], k, K);
+#pragma unroll
+        for (int i = 0; i < kALoads; ++i) a[i] = load4<kVec>(a_row[i], k, K);
+        if (++f_piece == kPiecesPerBlock) {
+            f_piece = 0;
+            if (++f_round == rounds) {
+                f_round = 0;
+                f_tile = min(f_tile + static_cast<int>(gridDim.x), column_tiles - 1);
+#pragma unroll
+                for (int i = 0; i < kWLoads; ++i) w_row[i] = weight_row(f_tile, 8 * i + lane / 8);
+            }
         }
-        __syncthreads();
+    };
 #pragma unroll
-        for (int kk = 0; kk < BK; ++kk) {
-            float a[4], w[4];
+    for (int s = 0; s < kAhead; ++s) fetch(w_ahead[s], a_ahead[s]);
+
+    int turn = 0;  // two sets of sums take turns: the next block's are written while others still read this one's
+    for (int tile = blockIdx.x; tile < column_tiles; tile += gridDim.x) {
+        float total[kOwned] = {}, stretch[kOwned] = {};
+        for (int round = 0; round < rounds; ++round) {
+            floatx4 block[kColumnTiles][kRowTiles] = {};
+            for (int half = 0; half < 2; ++half) {
+                floatx4 acc[kColumnTiles][kRowTiles] = {};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = a_tile[kk][ty * 4 + i];
+                for (int s = 0; s < kAhead; ++s) {
+                    const int k = (wave + round * kWaves) * kBlockK + (half * kAhead + s) * kPiece + 4 * chunk;
+                    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int j = 0; j < 4; ++j) w[j] = w_tile[kk][tx * 4 + j];
+                    for (int i = 0; i < kWLoads; ++i)
+                        *reinterpret_cast<floatx4*>(stage + chunk_at(8 * i + lane / 8, chunk)) = inside<kVec>(w_ahead[s][i], k, K);
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+                    for (int i = 0; i < kALoads; ++i)
+                        *reinterpret_cast<floatx4*>(stage + kColumnTiles * kTileFloats + chunk_at(8 * i + lane / 8, chunk)) =
+                            inside<kVec>(a_ahead[s][i], k, K);
+                    fetch(w_ahead[s], a_ahead[s]);
+                    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-        }
-        if (++slice == kSlicesPerBlock) {
-            slice = 0;
+                    for (int g = 0; g < kPiece / 16; ++g) {
+                        floatx4 f[kTiles];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+                        for (int t = 0; t < kTiles; ++t) {
+                            // (a half empty tile reads its 8 rows twice; what comes of the copies is not stored)
+                            const int r = (t < kColumnTiles ? kColumns : kRows) == 8 ? lane % 8 : lane % 16;
+                            f[t] = operand(stage + t * kTileFloats, r, g, lane / 16);
+                        }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    total[i][j] += acc[i][j];
-                    acc[i][j] = 0.f;
+                        for (int j = 0; j < 4; ++j)
+#pragma unroll
+                            for (int ct = 0; ct < kColumnTiles; ++ct)
+#pragma unroll
+                                for (int rt = 0; rt < kRowTiles; ++rt)
+                                    acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[ct][j], f[kColumnTiles + rt][j],
+                                                                                       acc[ct][rt], 0, 0, 0);
+                    }
                 }
+#pragma unroll
+                for (int ct = 0; ct < kColumnTiles; ++ct)
+#pragma unroll
+                    for (int rt = 0; rt < kRowTiles; ++rt) block[ct][rt] += acc[ct][rt];
+            }
+            float* all = sums[turn];
+            turn ^= 1;
+#pragma unroll
+            for (int ct = 0; ct < kColumnTiles; ++ct)
+#pragma unroll
+                for (int rt = 0; rt < kRowTiles; ++rt)
+                    *reinterpret_cast<floatx4*>(all + wave * kSums + ((ct * kRowTiles + rt) * kWave + lane) * 4) = block[ct][rt];
+            __syncthreads();
+            const int here = min(kWaves, blocks - round * kWaves);
+#pragma unroll
+            for (int o = 0; o < kOwned; ++o) {
+                const int e = threadIdx.x + o * kThreads;
+                if (e < kSums)
+                    for (int w = 0; w < here; ++w) {
+                        stretch[o] += all[w * kSums + e];
+                        const int block = round * kWaves + w;
+                        if (block % kBlocksPerStretch == kBlocksPerStretch - 1 || block == blocks - 1) {
+                            total[o] += stretch[o];
+                            stretch[o] = 0.f;
+                        }
+                    }
+            }
         }
-        __syncthreads();
-    }
+        // a thread's sum: tile e / 256 (column tiles outer), column 4 * (place / 16) + e % 4, row place % 16
+        if constexpr (kGate) {
+            // the two halves of a column belong to two threads (or to one thread's two sums): they meet in LDS
+            float* all = sums[turn];
+            turn ^= 1;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= M) continue;
+            for (int o = 0; o < kOwned; ++o) {
+                const int e = threadIdx.x + o * kThreads;
+                if (e < kSums) all[e] = total[o];
+            }
+            __syncthreads();
+            for (int at = threadIdx.x; at < kRows * kStep; at += kThreads) {
+                const int c = at % kStep, r = at / kStep;
+                const int n = tile * kStep + c, m = m0 + r;
+                auto sum_of = [&](int column) {
+                    return all[(column / 16 * kRowTiles + r / 16) * 256 + ((column % 16) / 4 * 16 + r % 16) * 4 + column % 4];
+                };
+                if (m < M && n < width)
+                    C[static_cast<size_t>(m) * ldc + n] = gated(sum_of(c), sum_of(kStep + c));
+            }
+        } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n < N) C[static_cast<size_t>(m) * ldc + n] = (total[i][j] + acc[i][j]) + (bias ? bias[n] : 0.f);
+            for (int o = 0; o < kOwned; ++o) {
+                const int e = threadIdx.x + o * kThreads;
+                const int at = (e / 4) % kWave;
+                const int c = 16 * (e / 256 / kRowTiles) + 4 * (at / 16) + e % 4, r = 16 * (e / 256 % kRowTiles) + at % 16;
+                const int n = tile * kStep + c, m = m0 + r;
+                if (e < kSums && c < kColumns && r < kRows && m < M && n < N)
+                    C[static_cast<size_t>(m) * ldc + n] = total[o] + (bias ? bias[n] : 0.f);
+            }
         }
     }
 }
 
-CIE_API int cie_gemm_f32(void* stream, const float* A, const float* W, const float* bias, float* C,
-                         int M, int N, int K, int lda, int ldc) {
-    if (M < 0 || N <= 0 || K <= 0 || lda < K || ldc < N) return CIE_BAD_ARGUMENT;
+// kN x kM tiles of 16 per wave, two by two waves: 32 * kN columns (with the gate half of them of each half, one tile of
+// either in turn), 32 * kM rows per workgroup; kAhead slices on their way.
+template <int kN, int kM, int kAhead, bool kGate, bool kVec>
+__global__ void __launch_bounds__(256, 2)
+gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int row_blocks, int tiles,
+                     float* __restrict__ parts) {
+    constexpr int kRows = 32 * (kN + kM);  // of W, then of A, in a stage
+    constexpr int kStep = kGate ? 16 * kN : 32 * kN;
+    static_assert(kN % 2 == 0 && kAhead % 2 == 0 && kPiecesPerBlock % kAhead == 0, "");
+    __shared__ float stage[2][kRows * kPiece];
+    const int lane = threadIdx.x % kWave;
+    const int wave = threadIdx.x / kWave;
+    // workgroups come to the 8 XCDs in turn: each XCD takes a run of neighbouring tiles, row blocks first, so that
+    // the tiles that read the same rows of W share an L2
+    const int per = (tiles + 7) / 8;
+    const int tile = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= per || tile >= tiles) return;
+    const int m0 = (tile % row_blocks) * 32 * kM;
+    const int n0 = (tile / row_blocks) * kStep;
+    const int width = kGate ? N / 2 : N;
+    // with `parts` workgroup y takes stretch y of K and leaves its sum in parts[y] [M, N]
+    const int k_first = parts ? blockIdx.y * kStretch : 0;
+    const int k_end = parts ? min(K, k_first + kStretch) : K;
+
+    const int chunk = threadIdx.x % 8;
+    const float* row_of[kN + kM];
+#pragma unroll
+    for (int i = 0; i < kN + kM; ++i) {
+        const int r = threadIdx.x / 8 + 32 * i;
+        const int n = kGate ? min(n0 + r / 32 * 16 + r % 16, width - 1) + (r / 16 % 2) * width : min(n0 + r, N - 1);
+        row_of[i] = i < kN ? W + static_cast<size_t>(n) * K : A + static_cast<size_t>(min(m0 + r - 32 * kN, M - 1)) * lda;
+    }
+    floatx4 ahead[kAhead][kN + kM];
+    auto fetch = [&](floatx4 (&to)[kN + kM], int slice) {
+#pragma unroll
+        for (int i = 0; i < kN + kM; ++i) to[i] = load4<kVec>(row_of[i], k_first + slice * kPiece + 4 * chunk, k_end);
+    };
+    auto put = [&](const floatx4 (&from)[kN + kM], int slice, float* to) {
+#pragma unroll
+        for (int i = 0; i < kN + kM; ++i)
+            *reinterpret_cast<floatx4*>(to + chunk_at(threadIdx.x / 8 + 32 * i, chunk)) =
+                inside<kVec>(from[i], k_first + slice * kPiece + 4 * chunk, k_end);
+    };
+
+    auto join = [](floatx4 (&to)[kN][kM], floatx4 (&from)[kN][kM]) {
+#pragma unroll
+        for (int in = 0; in < kN; ++in)
+#pragma unroll
+            for (int im = 0; im < kM; ++im) {
+                to[in][im] += from[in][im];
+                from[in][im] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
+    };
+    const int slices = (k_end - k_first + kPiece - 1) / kPiece;
+    floatx4 acc[kN][kM] = {}, block[kN][kM] = {}, stretch[kN][kM] = {}, total[kN][kM] = {};
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) fetch(ahead[a], a);
+    const int wn = (wave % 2) * 16 * kN, wm = 32 * kN + (wave / 2) * 16 * kM;  // this wave's rows in a stage
+    for (int first = 0; first < slices; first += kAhead) {
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a) {
+            const int slice = first + a;
+            float* here = stage[a % 2];
+            // (this stage was read two slices ago, and all waves have passed the barrier since)
+            put(ahead[a], slice, here);
+            fetch(ahead[a], slice + kAhead);
+            __syncthreads();
+#pragma unroll
+            for (int g = 0; g < kPiece / 16; ++g) {
+                floatx4 w[kN], x[kM];
+#pragma unroll
+                for (int i = 0; i < kN; ++i)
+                    w[i] = operand(here, wn + 16 * i + lane % 16, g, lane / 16);
+#pragma unroll
+                for (int i = 0; i < kM; ++i)
+                    x[i] = operand(here, wm + 16 * i + lane % 16, g, lane / 16);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int in = 0; in < kN; ++in)
+#pragma unroll
+                        for (int im = 0; im < kM; ++im)
+                            acc[in][im] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[in][j], x[im][j], acc[in][im], 0, 0, 0);
+            }
+        }
+        // (what stands behind the last slice adds zeros)
+        const int past = first + kAhead;
+        const bool end = past >= slices;
+        if (end || past % kPiecesPerChain == 0) join(block, acc);
+        if (end || past % kPiecesPerBlock == 0) join(stretch, block);
+        if (end || past % (kPiecesPerBlock * kBlocksPerStretch) == 0) join(total, stretch);
+    }
+    if (parts) C = parts + static_cast<size_t>(blockIdx.y) * M * N;
+    const bool wide = ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+#pragma unroll
+    for (int in = 0; in < kN; in += kGate ? 2 : 1) {
+        const int n = n0 + (kGate ? wn / 2 + 8 * in : wn + 16 * in) + 4 * (lane / 16);
+        floatx4 b = {0.f, 0.f, 0.f, 0.f};
+        if (bias)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b[i] = bias[min(n + i, N - 1)];
+#pragma unroll
+        for (int im = 0; im < kM; ++im) {
+            const int m = m0 + (wm - 32 * kN) + 16 * im + lane % 16;
+            if (m >= M) continue;
+            floatx4 v = total[in][im];
+            if constexpr (kGate) {
+                const floatx4 u = total[in + 1][im];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = gated(v[i], u[i]);
+            } else {
+                v += b;
+            }
+            float* to = C + static_cast<size_t>(m) * ldc + n;
+            if (wide && n + 3 < width) {
+                *reinterpret_cast<floatx4*>(to) = v;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n + i < width) to[i] = v[i];
+            }
+        }
+    }
+}
+
+// C = the sums of `stretches` parts [M, N] in order (+ bias), or the gated unit of their halves; a thread an output number.
+template <bool kGate>
+__global__ void __launch_bounds__(256)
+gemm_f32_join_kernel(const float* __restrict__ parts, int stretches, const float* __restrict__ bias, float* __restrict__ C,
+                     int M, int N, int ldc) {
+    const int width = kGate ? N / 2 : N;
+    const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+    if (n >= width) return;
+    const size_t apart = static_cast<size_t>(M) * N;
+    const float* from = parts + static_cast<size_t>(m) * N + n;
+    float total = 0.f, up = 0.f;
+    for (int first = 0; first < stretches; first += 4) {
+        float v[4], u[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // (a part past the last is read again and dropped)
+            v[i] = from[min(first + i, stretches - 1) * apart];
+            if constexpr (kGate) u[i] = from[min(first + i, stretches - 1) * apart + width];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (first + i >= stretches) break;
+            total += v[i];
+            if constexpr (kGate) up += u[i];
+        }
+    }
+    C[static_cast<size_t>(m) * ldc + n] = kGate ? gated(total, up) : total + (bias ? bias[n] : 0.f);
+}
+
+struct Product {
+    const float *A, *W, *bias;
+    float *C, *parts;
+    int M, N, K, lda, ldc, units;
+};
+
+template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec>
+void run_rows(hipStream_t s, const Product& p) {
+    const int step = kGate ? kColumns / 2 : kColumns;
+    const int tiles = ((kGate ? p.N / 2 : p.N) + step - 1) / step;
+    // as many workgroups as the units hold at a time by their LDS (two of the wide ones, four of the others)
+    const int most = p.units * ((kColumns == 32 || kRows == 32 || kWaves == 16 ? 2 : 4) * (kWaves == 4 ? 2 : 1));
+    dim3 grid(tiles < most ? tiles : most, (p.M + kRows - 1) / kRows);
+    gemm_f32_rows_kernel<kRows, kColumns, kWaves, kGate, kVec><<<grid, kWaves * kWave, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc);
+}
+
+template <bool kGate, bool kVec>
+void run_tiles(hipStream_t s, const Product& p) {
+    const int step = kGate ? 32 : 64;
+    const int row_blocks = (p.M + 63) / 64;
+    const int tiles = row_blocks * (((kGate ? p.N / 2 : p.N) + step - 1) / step);
+    gemm_f32_tile_kernel<2, 2, kVec ? 4 : 2, kGate, kVec><<<(tiles + 7) / 8 * 8, 256, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, row_blocks, tiles, nullptr);
+}
+
+template <bool kVec>
+void run_stretches(hipStream_t s, const Product& p, bool gate) {
+    const int row_blocks = (p.M + 63) / 64;
+    const int tiles = row_blocks * ((p.N + 63) / 64);
+    const int stretches = (p.K + kStretch - 1) / kStretch;
+    dim3 grid((tiles + 7) / 8 * 8, stretches);
+    gemm_f32_tile_kernel<2, 2, kVec ? 4 : 2, false, kVec><<<grid, 256, 0, s>>>(p.A, p.W, nullptr, nullptr, p.M, p.N, p.K, p.lda, p.N, row_blocks, tiles, p.parts);
+    dim3 join(((gate ? p.N / 2 : p.N) + 255) / 256, p.M);
+    if (gate) gemm_f32_join_kernel<true><<<join, 256, 0, s>>>(p.parts, stretches, nullptr, p.C, p.M, p.N, p.ldc);
+    else gemm_f32_join_kernel<false><<<join, 256, 0, s>>>(p.parts, stretches, p.bias, p.C, p.M, p.N, p.ldc);
+}
+
+template <bool kGate>
+void run_few(hipStream_t s, const Product& p, bool vec) {
+    if (!vec) return run_rows<16, 16, 8, kGate, false>(s, p);
+    // columns enough for two workgroups of 32 on every unit; a short K has blocks for four waves only
+    const bool wide = p.N >= 64 * p.units, shallow = p.K <= 4 * kBlockK;
+    if (p.M > 16) {
+        if (shallow) wide ? run_rows<32, 32, 4, kGate, true>(s, p) : run_rows<32, 16, 4, kGate, true>(s, p);
+        else wide ? run_rows<32, 32, 8, kGate, true>(s, p) : run_rows<32, 16, 8, kGate, true>(s, p);
+        return;
+    }
+    const bool eight = p.M <= 8;
+    if (wide) {
+        if (shallow) eight ? run_rows<8, 32, 4, kGate, true>(s, p) : run_rows<16, 32, 4, kGate, true>(s, p);
+        else eight ? run_rows<8, 32, 8, kGate, true>(s, p) : run_rows<16, 32, 8, kGate, true>(s, p);
+        return;
+    }
+    if constexpr (!kGate) {
+        // a long K and too few columns for a workgroup of 16 on every unit: 8 columns (a unit streams some 30 GB/s
+        // however many loads it has under way: N 2,048, K 11,008 at 4 rows 32 -> 26 us; K 2,048 is as fast with 16)
+        if (p.K > 8 * kBlockK && p.N < 16 * p.units) {
+            eight ? run_rows<8, 8, 16, false, true>(s, p) : run_rows<16, 8, 16, false, true>(s, p);
+            return;
+        }
+    }
+    if (shallow) eight ? run_rows<8, 16, 4, kGate, true>(s, p) : run_rows<16, 16, 4, kGate, true>(s, p);
+    else eight ? run_rows<8, 16, 8, kGate, true>(s, p) : run_rows<16, 16, 8, kGate, true>(s, p);
+}
+
+template <bool kGate>
+void run_form(hipStream_t s, const Product& p, int form, bool vec) {
+    if (form == 0) run_few<kGate>(s, p, vec);
+    else if (form == 1) vec ? run_tiles<kGate, true>(s, p) : run_tiles<kGate, false>(s, p);
+    else vec ? run_stretches<true>(s, p, kGate) : run_stretches<false>(s, p, kGate);
+}
+
+}  // namespace
+
+// `form`: 0 = few rows, 1 = tiles, 2 = tiles with a stretch of K each, and with
+// `parts` a workspace of ceil(K / 1024) * M * N numbers.  `gate`: the gated unit of the product's halves (N even, no
+// bias).  `units`: compute units of the device.
+CIE_API int cie_gemm_f32(void* stream, const float* A, const float* W, const float* bias, float* C, float* parts,
+                         int M, int N, int K, int lda, int ldc, int gate, int form, int units) {
+    if (M < 0 || N <= 0 || K <= 0 || lda < K || ldc < (gate ? N / 2 : N) || form < 0 || form > 2 || units < 1) return CIE_BAD_ARGUMENT;
+    if ((gate && (N % 2 || bias)) || (form == 2 && !parts)) return CIE_BAD_ARGUMENT;
     if (M == 0) return CIE_OK;
-    const int grid_y = (M + BM - 1) / BM;
-    if (grid_y > 65535) return CIE_BAD_ARGUMENT;
-    dim3 grid((N + BN - 1) / BN, grid_y);
-    gemm_f32_kernel<<<grid, 256, 0, static_cast<hipStream_t>(stream)>>>(A, W, bias, C, M, N, K, lda, ldc);
+    if (static_cast<long>((M + 63) / 64) * ((N + 31) / 32) > (1L << 30)) return CIE_BAD_ARGUMENT;
+    if ((form == 0 && M > 8 * 65535) || (form == 2 && (M > 65535 || K > 65535 * kStretch))) return CIE_BAD_ARGUMENT;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0;
+    const Product p{A, W, bias, C, parts, M, N, K, lda, ldc, units};
+    if (gate) run_form<true>(s, p, form, vec);
+    else run_form<false>(s, p, form, vec);
     return cie_after_launch();
 }

@@ -435,9 +435,34 @@ def paged_attention_mfma(q: torch.Tensor, q_row_stride: int, k_pool: torch.Tenso
         _i(keys_per_split), _ptr(max_context_dev), _i(tile_waves)))
 
 
+F32_STRETCH = 1024  # k that one workgroup takes where the float32 product cuts K
+
+
+def plan_gemm_f32(rows: int, columns: int, k: int) -> int:
+    """Which form of the float32 product runs (the numbers of ``cie_gemm_f32``): 0 few rows, 1 tiles of 64 x 64, 2 such
+    tiles with K cut in stretches.  Up to 16 rows the first, bound by the weight's stream; beyond that the one whose
+    turns over the units take least, in us as measured on MI355X: a turn of workgroups of 32 rows and 16 columns takes
+    9.5 per 2,048 k (eight waves; 3.9 where K is up to 1,024 and four waves do), a tile 21.5 per 1,000 k when alone on its
+    unit and 17.5 behind another, a stretch 19 and the join behind it 10.  (N = K = 2,048: 64 / 128 rows 13 / 23 in
+    the first, 47 / 48 in the second, 28 / 29 in the third form; N 22,016: 101 / 177, 81 / 115, 69 / 125; N 2,048, K
+    11,008: 53 / 106, 236 / 237, 52 / 75.)"""
+    if rows <= 16:
+        return 0
+    units = compute_units()
+    turns = -(-(-(-rows // 32) * -(-columns // 16)) // units)
+    few = 3 + turns * (3.9 if k <= 1024 else 9.5 * -(-k // 2048))
+    tiles = -(-rows // 64) * -(-columns // 64)
+    whole = 2 + k / 1000 * (21.5 + 17.5 * (-(-tiles // units) - 1))
+    stretches = -(-k // F32_STRETCH)
+    cut = 10 + 19 * min(k, F32_STRETCH) / F32_STRETCH * -(-tiles * stretches // units) if stretches > 1 and rows <= 65535 else whole
+    return 0 if few <= min(whole, cut) else 1 if whole <= cut else 2
+
+
 def gemm_f32(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
-             out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """True float32 ``a @ weight.T + bias``; a [M, K] (rows may be strided), weight [N, K]."""
+             out: Optional[torch.Tensor] = None, gate: bool = False, form: Optional[int] = None) -> torch.Tensor:
+    """True float32 ``a @ weight.T + bias``; a [M, K] (rows may be strided), weight [N, K].  ``gate``: the gated unit of
+    the product's halves instead, ``silu(first N / 2 columns) * (the others)`` (no bias).  ``form``: one of the kernel's
+    forms instead of the planned one (every form gives a row the same bits)."""
     if not (a.is_cuda and a.dtype == torch.float32 and a.dim() == 2 and a.stride(1) == 1):
         raise ValueError("a must be a float32 GPU matrix with unit inner stride")
     _gpu("weight", weight, torch.float32, 2)
@@ -445,18 +470,27 @@ def gemm_f32(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
     n = weight.shape[0]
     if not (weight.shape[1] == k):
         raise ValueError(f"a is [{m},{k}] but weight is {tuple(weight.shape)}")
+    if gate and (bias is not None or n % 2):
+        raise ValueError("a gated unit takes an even number of weight rows and no bias")
     if bias is not None:
         _gpu("bias", bias, torch.float32, 1)
         if not (bias.shape[0] == n):
             raise ValueError(f"bias must be [{n}]")
+    width = n // 2 if gate else n
     if out is None:
-        out = torch.empty((m, n), dtype=torch.float32, device=a.device)
+        out = torch.empty((m, width), dtype=torch.float32, device=a.device)
     _gpu("out", out, torch.float32, 2)
-    if not (out.shape == (m, n)):
-        raise ValueError(f"out must be {(m, n)}")
+    if not (out.shape == (m, width)):
+        raise ValueError(f"out must be {(m, width)}")
     lda = a.stride(0) if m > 1 else max(a.stride(0), k)
-    _run("cie_gemm_f32", load_library().cie_gemm_f32(_stream(), _ptr(a), _ptr(weight), _ptr(bias), _ptr(out),
-                                                     _i(m), _i(n), _i(k), _i(lda), _i(n)))
+    if form is None:
+        form = plan_gemm_f32(m, n, k)
+    parts = None
+    if form == 2:
+        parts = torch.empty((-(-k // F32_STRETCH), m, n), dtype=torch.float32, device=a.device)
+    _run("cie_gemm_f32", load_library().cie_gemm_f32(_stream(), _ptr(a), _ptr(weight), _ptr(bias), _ptr(out), _ptr(parts),
+                                                     _i(m), _i(n), _i(k), _i(lda), _i(width), _i(bool(gate)), _i(form),
+                                                     _i(compute_units(a.device))))
     return out
 
 

@@ -1,6 +1,7 @@
 """``x @ W^T + b`` for a Linear's weight ``[out, in]``, and its fused forms.
 
-float32: the hand-written true-float32 kernel, always.  bfloat16 with up to
+float32: the hand-written true-float32 kernels, always (the gated unit in their
+epilogue).  bfloat16 with up to
 ``FUSED_ROWS`` rows (decode steps, the output head), and up to 64 or 128 rows where
 it is the faster one (a small weight, a long K): the hand-written
 matrix-core kernels that stream the weight once and take over their neighbours'
@@ -301,6 +302,8 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
         elif not silu:
             return ops.gemm_fused(weight, ops.EPI_F32 if wants_f32 else ops.EPI_BF16, x, bias=bias)
     if weight.dtype == torch.float32:
+        if silu and n % 2 == 0 and bias is None:
+            return ops.gemm_f32(x, weight, gate=True)
         out = ops.gemm_f32(x, weight, bias)
     elif wants_f32:
         # a shape the kernel refuses (a width that is no multiple of 8): widened operands, exact products,

@@ -99,6 +99,28 @@ def test_gemm_f32(ops, shape):
     assert torch.equal(ops.gemm_f32(a[:1].contiguous(), w, b), ops.gemm_f32(a, w, b)[:1])
 
 
+# (rows, columns, K): single and half empty tiles, an odd K (no 16-byte loads), K at the edges of pieces, blocks and
+# stretches, columns for the narrow, the middle and the wide workgroups of the few-row form
+@pytest.mark.parametrize("shape", [(1, 8, 4), (9, 7, 33), (64, 66, 256), (65, 64, 1024), (17, 258, 1028), (33, 70, 2047),
+                                   (8, 2048, 2052), (5, 16384, 64), (20, 16386, 40), (130, 130, 4100)])
+def test_gemm_f32_forms(ops, shape):
+    """Every form of the float32 product gives the same bits, also for rows that lie apart, and its gated unit the bits
+    of the unit's own kernel behind the product.  The bound is what K + 8 roundings of half a unit in the last place
+    (6e-8) can add up to."""
+    m, n, k = shape
+    a, w, b = rand((m, k), torch.float32, 13), rand((n, k), torch.float32, 14), rand((n,), torch.float32, 15)
+    wide = torch.zeros((m, k + 12)).cuda()
+    wide[:, :k] = a
+    exact = a.double() @ w.double().t() + b.double()
+    bound = 6e-8 * (k + 8) * (a.double().abs() @ w.double().abs().t() + b.double().abs())
+    outs = [ops.gemm_f32(a, w, b, form=form) for form in (0, 1, 2)] + [ops.gemm_f32(wide[:, :k], w, b), ops.gemm_f32(a, w, b)]
+    assert ((outs[0].double() - exact).abs() <= bound).all()
+    assert all(torch.equal(out, outs[0]) for out in outs[1:])
+    if n % 2 == 0:
+        unit = ops.silu_mul(ops.gemm_f32(a, w))
+        assert all(torch.equal(ops.gemm_f32(a, w, gate=True, form=form), unit) for form in (0, 1, 2))
+
+
 @pytest.mark.parametrize("shape", [(1, 40, 24), (5, 515, 96), (16, 64, 128), (17, 130, 200), (33, 70, 1032),
                                    (64, 256, 264), (150, 99, 72)])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
