@@ -94,6 +94,18 @@ __device__ __forceinline__ float rows_sum(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// A 4 x 4 transposition over the four 16-lane rows of a wave: row q comes with x[4 q + j] in v[j] and leaves with
+// x[4 t + q] in v[t].
+typedef float quarter_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ quarter_t across_quarters(quarter_t v) {
+    const swap_pair_t a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[2]), false, false);
+    const swap_pair_t b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[1]), __float_as_uint(v[3]), false, false);
+    const swap_pair_t c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    const swap_pair_t d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    return quarter_t{__uint_as_float(c[0]), __uint_as_float(c[1]), __uint_as_float(d[0]), __uint_as_float(d[1])};
+}
+
 // Sum over a workgroup of up to 16 waves; every thread gets the result.
 // `scratch` is at least 16 floats of LDS; the call contains barriers.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {

@@ -343,6 +343,68 @@ def paged_attention_generic(q: torch.Tensor, q_row_stride: int, k_pool: torch.Te
     return out
 
 
+F32_HEAD_DIMS = (32, 64, 96, 128)  # head sizes of the float32 attention on the matrix cores
+F32_TILE_ROWS = 64   # (token, head) rows of its tiles
+F32_BLOCK_KEYS = 64  # keys of its blocks
+
+
+def paged_attention_f32(q: torch.Tensor, q_row_stride: int, k_pool: torch.Tensor, v_pool: torch.Tensor,
+                        block_table: torch.Tensor, tile_seq: Optional[torch.Tensor], tile_q0: Optional[torch.Tensor],
+                        n_tiles: int, seq_slot: torch.Tensor, seq_start: torch.Tensor, seq_q_len: torch.Tensor,
+                        q_start_loc: torch.Tensor, out: torch.Tensor, q_heads: int, kv_heads: int, head_dim: int,
+                        window: Optional[int], scale: float, tokens_per_tile: int, first_tile: int = 0, turns: int = 0,
+                        blocks: int = 0, part_o: Optional[torch.Tensor] = None,
+                        part_ml: Optional[torch.Tensor] = None) -> None:
+    """True float32 attention on the matrix cores for the tiles ``first_tile .. first_tile + n_tiles - 1``: tile i holds
+    up to ``tokens_per_tile`` tokens of sequence ``tile_seq[i]`` from its ``tile_q0[i]``-th token of this step on (both
+    ``None``: tile i starts sequence i).  Rows of other tokens of ``out`` are left alone.  ``turns=0``: a workgroup to a
+    tile and key head.  Otherwise that many waves to 16 rows of a tile, which take its blocks of 64 keys in turn and leave
+    them in workspaces, of ``blocks`` blocks a tile (as many as any tile's keys need), that a second kernel joins.  Both
+    give a row the same bits."""
+    if not (q.is_cuda and q.dtype == torch.float32 and q.dim() == 2 and q.stride(1) == 1 and q.stride(0) == q_row_stride):
+        raise ValueError("q must be a float32 GPU matrix with unit inner stride")
+    if not (q.shape[1] >= q_heads * head_dim and q_row_stride % 4 == 0):
+        raise ValueError(f"q {tuple(q.shape)} does not fit")
+    if head_dim not in F32_HEAD_DIMS or q_heads % kv_heads:
+        raise ValueError(f"head_dim must be one of {F32_HEAD_DIMS}, is {head_dim}, and {kv_heads} key heads divide {q_heads}")
+    group = q_heads // kv_heads
+    if not (1 <= tokens_per_tile and tokens_per_tile * group <= F32_TILE_ROWS):
+        raise ValueError(f"{tokens_per_tile} tokens of {group} heads do not fit {F32_TILE_ROWS} rows")
+    page_size = _check_pools(k_pool, v_pool, torch.float32, kv_heads, head_dim)
+    if not (page_size >= 4 and page_size & (page_size - 1) == 0):
+        raise ValueError(f"page size must be a power of two >= 4, is {page_size}")
+    _gpu("block_table", block_table, torch.int32, 2)
+    if (tile_seq is None) != (tile_q0 is None):
+        raise ValueError("tile_seq and tile_q0 come together, or neither (tile i is then the first tile of sequence i)")
+    for name, meta in (("tile_seq", tile_seq), ("tile_q0", tile_q0)):
+        if meta is not None:
+            _gpu(name, meta, torch.int32, 1)
+            if not (meta.shape[0] >= first_tile + n_tiles):
+                raise ValueError(f"{name} has {meta.shape[0]} entries for {first_tile + n_tiles} tiles")
+    if first_tile < 0 or (tile_seq is None and seq_q_len.shape[0] < first_tile + n_tiles):
+        raise ValueError(f"{n_tiles} tiles from {first_tile} on for {seq_q_len.shape[0]} sequences")
+    for name, meta in (("seq_slot", seq_slot), ("seq_start", seq_start), ("seq_q_len", seq_q_len),
+                       ("q_start_loc", q_start_loc)):
+        _gpu(name, meta, torch.int32, 1)
+    _gpu("out", out, torch.float32, 2)
+    if not (out.shape[1] == q_heads * head_dim and out.shape[0] <= q.shape[0]):
+        raise ValueError(f"out is {tuple(out.shape)}")
+    rows = tokens_per_tile * group
+    if turns:
+        if part_o is None or part_ml is None or blocks < 1:
+            raise ValueError("attention in blocks needs its workspaces")
+        _gpu("part_o", part_o, torch.float32)
+        _gpu("part_ml", part_ml, torch.float32)
+        units = n_tiles * kv_heads * blocks * rows
+        if not (part_o.numel() >= units * head_dim and part_ml.numel() >= units * 2):
+            raise ValueError("attention workspaces are too small")
+    _run("cie_paged_attention_f32", load_library().cie_paged_attention_f32(
+        _stream(), _ptr(q), _i(q_row_stride), _ptr(k_pool), _ptr(v_pool), _ptr(block_table), _i(block_table.shape[1]),
+        _ptr(tile_seq), _ptr(tile_q0), _i(first_tile), _i(n_tiles), _ptr(seq_slot), _ptr(seq_start), _ptr(seq_q_len),
+        _ptr(q_start_loc), _ptr(out), _ptr(part_o), _ptr(part_ml), _i(rows), _i(blocks), _i(turns), _i(q_heads),
+        _i(kv_heads), _i(head_dim), _i(page_size), _i(window or 0), _f(scale), _i(tokens_per_tile)))
+
+
 MFMA_HEAD_DIMS = (32, 64, 96, 128, 256)
 TILE_WAVES = 4  # waves per workgroup of the prompt form of the matrix-core attention
 PROMPT_WAVES = 8  # ... and of its form with tiles of 128 rows whose keys and values go through LDS

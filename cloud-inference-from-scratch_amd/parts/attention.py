@@ -196,13 +196,16 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
     bfloat16 with a head size the matrix-core kernel takes: sequences that bring
     one token go to the split-context decode form, prompt portions to the tiled
     form with up to 64 rows per tile (four waves per tile where pages hold at
-    least 16 keys, one wave otherwise).  Everything else (float32, other head
-    sizes, groups of more than 16 heads, pages of fewer than 4 tokens): the
-    generic kernel."""
+    least 16 keys, one wave otherwise).  float32 with heads of 32 to 128
+    dimensions: :func:`attend_f32`.  Everything else (other head sizes, groups of
+    more than 64 heads, pages of fewer than 4 tokens): the generic kernel."""
     group = num_heads // num_kv_heads
     decode_tiles = 1 if group <= 16 else 2 if group <= 32 else 4  # 16-row tiles that hold one token's heads
     page_size = view.page_size
     cus = ops.compute_units()  # compute units of the GPU
+    if (qkv.dtype == torch.float32 and head_dim in ops.F32_HEAD_DIMS and group <= ops.F32_TILE_ROWS
+            and page_size >= 4 and page_size & (page_size - 1) == 0):
+        return attend_f32(qkv, batch, view, num_heads, num_kv_heads, head_dim, window, scale)
     # (a token's heads of one key head share a tile: up to 64 rows, 16 where the head has 256 dimensions)
     if (qkv.dtype != torch.bfloat16 or head_dim not in ops.MFMA_HEAD_DIMS or group > (64 if head_dim <= 128 else 16)
             or page_size < 4 or page_size & (page_size - 1)):
@@ -335,6 +338,62 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
                                  n_tiles, *common, tokens_per_tile=per_tile, row_tiles=row_tiles,
                                  n_splits=n_splits, keys_per_split=per_split, part_o=part_o, part_ml=part_ml,
                                  tile_waves=tile_waves, max_context_dev=longest_dev if n_splits > 1 else None)
+    return out
+
+
+# Float32: contexts up to which single tokens take the prompt form too (a workgroup's two blocks of 64 keys in turn cost
+# less than the second kernel that joins blocks), and the bytes that the blocks' workspace may take (sequences beyond
+# that go in further launches, which share it)
+F32_WHOLE_KEYS = 128
+F32_WORKSPACE_BYTES = 64 << 20
+
+
+def attend_f32(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, head_dim: int,
+               window: Optional[int], scale: float) -> torch.Tensor:
+    """Attention in true float32 on the matrix cores: single tokens in blocks of keys (a wave each, joined behind),
+    prompt portions a workgroup per 64 rows, or in blocks too where such tiles would leave half of the units idle."""
+    out = torch.empty((batch.tokens, num_heads * head_dim), dtype=qkv.dtype, device=qkv.device)
+    group = num_heads // num_kv_heads
+    per_tile = ops.F32_TILE_ROWS // group
+    cus = ops.compute_units()
+    plan = batch.static_plan
+    bound = plan.max_keys if plan is not None else batch.max_context
+    common = (batch.seq_slot, batch.seq_start, batch.seq_q_len, batch.q_start_loc, out, num_heads, num_kv_heads, head_dim,
+              window, scale)
+
+    def run(tiles: tuple, tokens: int, whole: bool) -> None:
+        tile_seq, tile_q0, n_tiles = tiles
+        blocks = -(-bound // ops.F32_BLOCK_KEYS)
+        if window is not None:  # (a window may begin inside a block)
+            blocks = min(blocks, -(-(window + tokens) // ops.F32_BLOCK_KEYS) + 1)
+        rows = tokens * group
+        per = num_kv_heads * blocks * rows
+        if whole or (tokens > 1 and (2 * n_tiles * num_kv_heads > cus
+                                     or n_tiles * per * (head_dim + 2) * 4 > F32_WORKSPACE_BYTES)):
+            ops.paged_attention_f32(qkv, qkv.stride(0), view.k_pool, view.v_pool, view.block_table, tile_seq, tile_q0,
+                                    n_tiles, *common, tokens)
+            return
+        at_once = max(1, min(n_tiles, F32_WORKSPACE_BYTES // (per * (head_dim + 2) * 4)))
+        part_o = torch.empty(at_once * per * head_dim, dtype=torch.float32, device=qkv.device)
+        part_ml = torch.empty(at_once * per * 2, dtype=torch.float32, device=qkv.device)
+        for first in range(0, n_tiles, at_once):
+            count = min(at_once, n_tiles - first)
+            waves = count * num_kv_heads * -(-rows // 16)  # (some 16 waves a unit; more blocks than that are taken in turn)
+            ops.paged_attention_f32(qkv, qkv.stride(0), view.k_pool, view.v_pool, view.block_table, tile_seq, tile_q0, count,
+                                    *common, tokens, first_tile=first, turns=min(blocks, max(1, -(-16 * cus // waves))),
+                                    blocks=blocks, part_o=part_o, part_ml=part_ml)
+
+    single = batch.sequences if plan is not None and plan.decode_rows is None else plan.decode_rows if plan is not None else None
+    if bound <= F32_WHOLE_KEYS:
+        run((None, None, batch.sequences) if single == batch.sequences else batch.tiles(per_tile, decode=None), per_tile, True)
+        return out
+    tiles = (None, None, single) if single is not None else batch.tiles(1, decode=True)
+    if tiles[2]:
+        run(tiles, 1, False)
+    if single != batch.sequences:
+        tiles = batch.tiles(per_tile, decode=False)
+        if tiles[2]:
+            run(tiles, per_tile, False)
     return out
 
 

@@ -211,6 +211,78 @@ def test_paged_attention_generic(ops, dtype, geometry):
     torch.testing.assert_close(out.float().cpu(), torch.cat(expected), **tol(dtype))
 
 
+def run_f32(ops, q_all, contexts, q_lens, k_pool, v_pool, table, slots, q_heads, kv_heads, head_dim, window, scale, per_tile,
+            turns):
+    """Drive the float32 attention of the matrix cores: tiles of ``per_tile`` tokens, whole or in blocks of keys."""
+    as_dev = lambda values: torch.tensor(values, dtype=torch.int32).cuda()  # noqa: E731
+    loc = [sum(q_lens[:i]) for i in range(len(q_lens) + 1)]
+    tiles = [(s, first) for s, n in enumerate(q_lens) for first in range(0, n, per_tile)]
+    stride = (q_heads + 2 * kv_heads) * head_dim
+    buffer = torch.zeros((sum(q_lens), stride)).cuda()
+    buffer[:, : q_heads * head_dim] = q_all.cuda()
+    out = torch.full((sum(q_lens), q_heads * head_dim), float("nan")).cuda()
+    spaces = {}
+    if turns:
+        blocks, rows = max(-(-(c + n) // 64) for c, n in zip(contexts, q_lens)), per_tile * (q_heads // kv_heads)
+        units = len(tiles) * kv_heads * blocks * rows
+        spaces = dict(turns=turns, blocks=blocks, part_o=torch.full((units * head_dim,), float("nan")).cuda(),
+                      part_ml=torch.full((units * 2,), float("nan")).cuda())
+    ops.paged_attention_f32(buffer, stride, k_pool, v_pool, table, as_dev([s for s, _ in tiles]), as_dev([q for _, q in tiles]),
+                            len(tiles), as_dev(slots), as_dev(contexts), as_dev(q_lens), as_dev(loc), out, q_heads, kv_heads,
+                            head_dim, window, scale, per_tile, **spaces)
+    return out.cpu()
+
+
+@pytest.mark.parametrize("geometry", [(16, 2, 128, 16), (3, 1, 32, 4), (14, 2, 64, 8), (16, 1, 96, 32), (64, 1, 32, 128),
+                                      (40, 8, 128, 64)])
+@pytest.mark.parametrize("window", [None, 1, 50, 300])
+def test_paged_attention_f32(ops, geometry, window):
+    """The float32 attention of the matrix cores on the ragged batch of the bfloat16 forms: near the plain
+    implementation, and the same bits whole or in blocks, in large tiles or token by token."""
+    q_heads, kv_heads, head_dim, page_size = geometry
+    contexts = [0, 15, 16, 17, 127, 511, 1, 40, 100]
+    q_lens = [7, 1, 2, 16, 1, 33, 64, 5, 200]
+    lengths = [c + q for c, q in zip(contexts, q_lens)]
+    k_pool, v_pool, table, slots, dense = build_cache(torch.float32, lengths, kv_heads, head_dim, page_size, seed=70)
+    scale = 1.0 / math.sqrt(head_dim)
+    g = torch.Generator().manual_seed(71)
+    qs, expected = [], []
+    for s, (c, n) in enumerate(zip(contexts, q_lens)):
+        q = torch.randn((n, q_heads, head_dim), generator=g) * 2
+        qs.append(q.reshape(n, -1))
+        expected.append(plain_qwen2.causal_attention(q, *dense[s], scale, past_len=c, window=window))
+    most = 64 // (q_heads // kv_heads)
+    outs = [run_f32(ops, torch.cat(qs), contexts, q_lens, k_pool, v_pool, table, slots, q_heads, kv_heads, head_dim, window,
+                    scale, per_tile, turns) for per_tile, turns in ((most, 0), (1, 0), (most, 1), (most, 3), (1, 16))]
+    torch.testing.assert_close(outs[0], torch.cat(expected), **tol(torch.float32))
+    assert all(torch.equal(out, outs[0]) for out in outs[1:])
+
+
+@pytest.mark.parametrize("turns", [0, 2])
+def test_paged_attention_f32_odd_values_reach_the_rows_that_see_them(ops, turns):
+    """An infinity and a NaN among the cached values: the rows before them in the same tile stay as they are, the rows
+    that see them have the generic kernel's infinities and NaN."""
+    q_heads, kv_heads, head_dim, page_size, n = 16, 2, 128, 16, 100
+    k_pool, v_pool, table, slots, _ = build_cache(torch.float32, [n], kv_heads, head_dim, page_size, seed=74)
+    odd = v_pool.clone()
+    page = int(table[slots[0], 3])
+    odd[page, :, 5, 2] = float("inf")
+    odd[page, 0, 7, 3] = float("nan")
+    q = rand((n, q_heads * head_dim), torch.float32, 75)
+    run = lambda values: run_f32(ops, q, [0], [n], k_pool, values, table, slots, q_heads, kv_heads, head_dim, None, 0.1, 8, turns)  # noqa: E731
+    plain, got = run(v_pool), run(odd)
+    as_dev = lambda values: torch.tensor(values, dtype=torch.int32).cuda()  # noqa: E731
+    buffer = torch.zeros((n, (q_heads + 2 * kv_heads) * head_dim)).cuda()
+    buffer[:, : q_heads * head_dim] = q
+    generic = ops.paged_attention_generic(buffer, buffer.shape[1], k_pool, odd, table, as_dev(list(range(n))), as_dev([0] * n),
+                                          as_dev(slots), n, q_heads, kv_heads, head_dim, None, 0.1).cpu()
+    assert torch.equal(got[:50], plain[:50])
+    assert torch.equal(torch.isnan(got), torch.isnan(generic)) and torch.equal(torch.isinf(got), torch.isinf(generic))
+    finite = torch.isfinite(generic)
+    assert not finite.all()
+    torch.testing.assert_close(got[finite], generic[finite], **tol(torch.float32))
+
+
 def run_mfma(ops, q_all, contexts, q_lens, k_pool, v_pool, table, slots, q_heads, kv_heads, head_dim, window,
              scale, per_tile, row_tiles, n_splits=1, keys_per_split=0, decode_only=None, tile_waves=1,
              max_context_dev=None):
