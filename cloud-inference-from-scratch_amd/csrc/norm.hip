@@ -1,6 +1,6 @@
 // Fused residual-add + RMSNorm.
 //
-//   x   = residual[row] (+ branch[row])        float32
+//   x   = residual[row] (+ branch[row]) (+ sum_p parts[p, row], float32, in order)        float32
 //   var = mean(x^2);  y = x * (1 / sqrt(var + eps)) * weight
 //
 // The statistics, the scaling and the residual sum are float32; the output is
@@ -14,20 +14,20 @@ template <typename T, typename W>
 __global__ void add_rmsnorm_kernel(float* __restrict__ residual, const T* __restrict__ branch,
                                    const W* __restrict__ weight, T* __restrict__ out,
                                    const int* __restrict__ rows, int hidden, float eps,
-                                   int write_residual) {
+                                   int write_residual, const float* __restrict__ parts, int n_parts, size_t apart) {
     extern __shared__ float staged[];
     __shared__ float scratch[16];
     const int out_row = blockIdx.x;
     const int row = rows ? rows[out_row] : out_row;
     float* res = residual + static_cast<size_t>(row) * hidden;
     const T* add = branch ? branch + static_cast<size_t>(row) * hidden : nullptr;
+    const float* extra = parts + static_cast<size_t>(row) * hidden;  // (not read without parts)
     float sum_sq = 0.f;
     for (int h = threadIdx.x; h < hidden; h += blockDim.x) {
         float x = res[h];
-        if (add) {
-            x += to_float(add[h]);
-            if (write_residual) res[h] = x;
-        }
+        if (add) x += to_float(add[h]);
+        for (int p = 0; p < n_parts; ++p) x += extra[p * apart + h];
+        if ((add || n_parts) && write_residual) res[h] = x;
         staged[h] = x;
         sum_sq += x * x;
     }
@@ -41,11 +41,12 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ residual, const T* __rest
 // bf16 activations and weight, hidden a multiple of 8: eight elements per thread, 16-byte accesses.
 __global__ void add_rmsnorm_vec8_kernel(float* __restrict__ residual, const bf16_t* __restrict__ branch,
                                         const bf16_t* __restrict__ weight, bf16_t* __restrict__ out,
-                                        int hidden, float eps) {
+                                        int hidden, float eps, const float* __restrict__ parts, int n_parts, size_t apart) {
     extern __shared__ float staged[];
     __shared__ float scratch[16];
     const int row = blockIdx.x;
     float* res = residual + static_cast<size_t>(row) * hidden;
+    const float* extra = parts + static_cast<size_t>(row) * hidden;  // (not read without parts)
     const bf16_t* add = branch ? branch + static_cast<size_t>(row) * hidden : nullptr;
     float sum_sq = 0.f;
     for (int h = threadIdx.x * 8; h < hidden; h += blockDim.x * 8) {
@@ -57,6 +58,23 @@ __global__ void add_rmsnorm_vec8_kernel(float* __restrict__ residual, const bf16
             x0.z += __uint_as_float(raw.y << 16); x0.w += __uint_as_float(raw.y & 0xffff0000u);
             x1.x += __uint_as_float(raw.z << 16); x1.y += __uint_as_float(raw.z & 0xffff0000u);
             x1.z += __uint_as_float(raw.w << 16); x1.w += __uint_as_float(raw.w & 0xffff0000u);
+        }
+        for (int first = 0; first < n_parts; first += 4) {
+            float4 a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {  // (four under way at a time; a part past the last is read again and dropped)
+                const float* from = extra + min(first + i, n_parts - 1) * apart + h;
+                a[i] = *reinterpret_cast<const float4*>(from);
+                b[i] = *reinterpret_cast<const float4*>(from + 4);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (first + i >= n_parts) break;
+                x0.x += a[i].x; x0.y += a[i].y; x0.z += a[i].z; x0.w += a[i].w;
+                x1.x += b[i].x; x1.y += b[i].y; x1.z += b[i].z; x1.w += b[i].w;
+            }
+        }
+        if (add || n_parts) {
             *reinterpret_cast<float4*>(res + h) = x0;
             *reinterpret_cast<float4*>(res + h + 4) = x1;
         }
@@ -84,10 +102,10 @@ __global__ void add_rmsnorm_vec8_kernel(float* __restrict__ residual, const bf16
 template <typename T, typename W>
 static int launch_norm(hipStream_t s, float* residual, const void* branch, const void* weight,
                        void* out, const int* rows, int n_out, int hidden, float eps,
-                       int write_residual) {
+                       int write_residual, const float* parts, int n_parts, size_t apart) {
     add_rmsnorm_kernel<T, W><<<n_out, n_out <= 64 ? 1024 : 256, hidden * sizeof(float), s>>>(
         residual, static_cast<const T*>(branch), static_cast<const W*>(weight), static_cast<T*>(out),
-        rows, hidden, eps, write_residual);
+        rows, hidden, eps, write_residual, parts, n_parts, apart);
     return cie_after_launch();
 }
 
@@ -125,27 +143,30 @@ CIE_API int cie_rmsnorm_from_sumsq(void* stream, int wdtype, const float* residu
     return cie_after_launch();
 }
 
-// dtype: activation type of branch/out; wdtype: storage type of the weight.
+// dtype: activation type of branch/out; wdtype: storage type of the weight.  `parts` [n_parts, tokens, hidden] float32
+// (n_parts 0: none) are added to the stream too, in order; tokens counts the rows of the stream.
 CIE_API int cie_add_rmsnorm(void* stream, int dtype, int wdtype, float* residual, const void* branch,
                             const void* weight, void* out, const int* rows, int n_out, int hidden,
-                            float eps, int write_residual) {
-    if (n_out < 0 || hidden <= 0 || hidden * sizeof(float) > 64 * 1024 || !(eps > 0.f))
+                            float eps, int write_residual, const float* parts, int n_parts, int tokens) {
+    if (n_out < 0 || hidden <= 0 || hidden * sizeof(float) > 64 * 1024 || !(eps > 0.f) || n_parts < 0 || (n_parts && !parts) ||
+        tokens < 0)
         return CIE_BAD_ARGUMENT;
+    const size_t apart = static_cast<size_t>(tokens) * hidden;
     if (rows && write_residual) return CIE_BAD_ARGUMENT;
     if (n_out == 0) return CIE_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == CIE_F32 && wdtype == CIE_F32)
-        return launch_norm<float, float>(s, residual, branch, weight, out, rows, n_out, hidden, eps, write_residual);
+        return launch_norm<float, float>(s, residual, branch, weight, out, rows, n_out, hidden, eps, write_residual, parts, n_parts, apart);
     if (dtype == CIE_BF16 && wdtype == CIE_BF16 && !rows && write_residual && hidden % 8 == 0) {
         add_rmsnorm_vec8_kernel<<<n_out, n_out <= 64 ? 1024 : 256, hidden * sizeof(float), s>>>(
             residual, static_cast<const bf16_t*>(branch), static_cast<const bf16_t*>(weight), static_cast<bf16_t*>(out),
-            hidden, eps);
+            hidden, eps, parts, n_parts, apart);
         return cie_after_launch();
     }
     if (dtype == CIE_BF16 && wdtype == CIE_BF16)
-        return launch_norm<bf16_t, bf16_t>(s, residual, branch, weight, out, rows, n_out, hidden, eps, write_residual);
+        return launch_norm<bf16_t, bf16_t>(s, residual, branch, weight, out, rows, n_out, hidden, eps, write_residual, parts, n_parts, apart);
     if (dtype == CIE_BF16 && wdtype == CIE_F32)
-        return launch_norm<bf16_t, float>(s, residual, branch, weight, out, rows, n_out, hidden, eps, write_residual);
+        return launch_norm<bf16_t, float>(s, residual, branch, weight, out, rows, n_out, hidden, eps, write_residual, parts, n_parts, apart);
     return CIE_BAD_ARGUMENT;
 }
 

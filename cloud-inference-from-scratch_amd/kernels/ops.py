@@ -183,11 +183,11 @@ MAX_NORM_WIDTH = 16384  # a row of the norm kernels is held in 64 KB of LDS as f
 
 def add_rmsnorm(residual: torch.Tensor, branch: Optional[torch.Tensor], weight: torch.Tensor, eps: float,
                 out_dtype: torch.dtype, rows: Optional[torch.Tensor] = None,
-                out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                out: Optional[torch.Tensor] = None, parts: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``residual += branch`` (if given; written back unless ``rows``), then RMS-normalise.
 
     residual float32 [T, H]; branch and the result in ``out_dtype``; weight [H]
-    in ``out_dtype`` or float32.  With ``rows`` (int32 [n]) only those rows are
+    in ``out_dtype`` or float32.  ``parts`` (float32 [P, T, H]) join the residual too, one after the other.  With ``rows`` (int32 [n]) only those rows are
     produced, in that order, and the residual is left as it is."""
     _gpu("residual", residual, torch.float32, 2)
     tokens, hidden = residual.shape
@@ -204,6 +204,10 @@ def add_rmsnorm(residual: torch.Tensor, branch: Optional[torch.Tensor], weight: 
         _gpu("branch", branch, out_dtype, 2)
         if not (branch.shape == residual.shape):
             raise ValueError(f"branch {tuple(branch.shape)} vs residual {tuple(residual.shape)}")
+    if parts is not None:
+        _gpu("parts", parts, torch.float32, 3)
+        if not (parts.shape[1:] == residual.shape):
+            raise ValueError(f"parts {tuple(parts.shape)} vs residual {tuple(residual.shape)}")
     if rows is not None:
         _gpu("rows", rows, torch.int32, 1)
         n_out = rows.shape[0]
@@ -216,7 +220,8 @@ def add_rmsnorm(residual: torch.Tensor, branch: Optional[torch.Tensor], weight: 
         raise ValueError(f"out must be {(n_out, hidden)}, is {tuple(out.shape)}")
     _run("cie_add_rmsnorm", load_library().cie_add_rmsnorm(
         _stream(), _i(_code(out_dtype)), _i(_code(weight.dtype)), _ptr(residual), _ptr(branch), _ptr(weight),
-        _ptr(out), _ptr(rows), _i(n_out), _i(hidden), _f(eps), _i(0 if rows is not None else 1)))
+        _ptr(out), _ptr(rows), _i(n_out), _i(hidden), _f(eps), _i(0 if rows is not None else 1), _ptr(parts),
+        _i(0 if parts is None else parts.shape[0]), _i(tokens)))
     return out
 
 
@@ -828,6 +833,84 @@ FOLDED_NORM_ROWS = 16      # the most rows whose norm the q/k/v product makes it
 def folds_norm(rows: int, k: int) -> bool:
     """Whether ``gemm_qkv_rope`` takes ``folded=`` for this many rows of ``k`` values."""
     return 1 <= rows <= FOLDED_NORM_ROWS and k >= 8 and k % 8 == 0
+
+
+TILE_BF16, TILE_SILU, TILE_RESID, TILE_PARTS = 0, 1, 2, 3
+TILE_SHAPES = ((64, 64), (128, 64), (128, 128), (128, 256))  # columns x rows of a workgroup's tile
+
+
+def _tile_rows(a: torch.Tensor, weight: torch.Tensor) -> tuple[int, int, int, int]:
+    """(rows, columns, K, row stride) of a product that goes to the tile kernel, checked."""
+    _gpu("weight", weight, torch.bfloat16, 2)
+    if not (a.is_cuda and a.dtype == torch.bfloat16 and a.dim() == 2 and a.stride(1) == 1):
+        raise ValueError("a must be a bf16 GPU matrix with unit inner stride")
+    m, k = a.shape
+    n = weight.shape[0]
+    lda = a.stride(0) if m > 1 else max(a.stride(0), k)
+    if not (m >= 1 and weight.shape[1] == k and k % 8 == 0 and lda % 8 == 0):
+        raise ValueError(f"a {tuple(a.shape)} with row stride {lda} and weight {tuple(weight.shape)}: K and the stride are multiples of 8")
+    if a.data_ptr() % 16 or weight.data_ptr() % 16:
+        raise ValueError("operands must be 16-byte aligned")
+    return m, n, k, lda
+
+
+def gemm_tiles(weight: torch.Tensor, epilogue: int, a: torch.Tensor, columns: int, rows: int,
+               bias: Optional[torch.Tensor] = None, into: Optional[torch.Tensor] = None, parts: int = 1) -> torch.Tensor:
+    """``a @ weight.T + bias`` in bfloat16 for some hundred rows, in tiles of ``columns`` x ``rows``: the bf16 result, its
+    gated unit (``TILE_SILU``), added in place to the float32 stream ``into`` (``TILE_RESID``), or K in ``parts`` parts
+    whose float32 sums come back as [parts, M, N] (``TILE_PARTS``)."""
+    m, n, k, lda = _tile_rows(a, weight)
+    if (columns, rows) not in TILE_SHAPES:
+        raise ValueError(f"tiles are one of {TILE_SHAPES}, not {(columns, rows)}")
+    if bias is not None:
+        _gpu("bias", bias, torch.bfloat16, 1)
+        if not (bias.shape[0] == n and epilogue != TILE_SILU):
+            raise ValueError("bias does not fit")
+    if epilogue == TILE_RESID:
+        _gpu("into", into, torch.float32, 2)
+        if not (into.shape == (m, n) and into.data_ptr() % 16 == 0):
+            raise ValueError(f"into must be {(m, n)}, is {tuple(into.shape)}")
+        out = into
+    elif epilogue == TILE_PARTS:
+        out = torch.empty((parts, m, n), dtype=torch.float32, device=a.device)
+    else:
+        out = torch.empty((m, n // 2 if epilogue == TILE_SILU else n), dtype=torch.bfloat16, device=a.device)
+    _run("cie_gemm_tiles", load_library().cie_gemm_tiles(
+        _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(out), _i(out.shape[-1]), _i(m), _i(n), _i(k), _i(epilogue),
+        _i(columns), _i(rows), _i(parts)))
+    return out
+
+
+def gemm_tiles_rope(weight: torch.Tensor, a: torch.Tensor, bias: Optional[torch.Tensor], cos: torch.Tensor,
+                    sin: torch.Tensor, positions: torch.Tensor, seq_of_token: torch.Tensor, seq_slot: torch.Tensor,
+                    block_table: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, q_heads: int, kv_heads: int,
+                    head_dim: int, columns: int, rows: int, rotate: bool = True, write_kv: bool = True) -> torch.Tensor:
+    """What :func:`gemm_qkv_rope` does, for some hundred rows in tiles of ``columns`` x ``rows``."""
+    m, n, k, lda = _tile_rows(a, weight)
+    if (columns, rows) not in TILE_SHAPES or head_dim % 32 or n != (q_heads + 2 * kv_heads) * head_dim:
+        raise ValueError(f"tiles of {columns} x {rows}, heads of {head_dim}, {n} weight rows do not fit")
+    if bias is not None:
+        _gpu("bias", bias, torch.bfloat16, 1)
+        if not (bias.shape[0] == n):
+            raise ValueError("bias does not fit")
+    for name, table in (("cos", cos), ("sin", sin)):
+        _gpu(name, table, torch.float32, 2)
+        if rotate and not (table.shape[1] == head_dim // 2 and table.data_ptr() % 16 == 0 and cos.shape == sin.shape):
+            raise ValueError(f"{name} must be [max_position, {head_dim // 2}]")
+    for name, meta in (("positions", positions), ("seq_of_token", seq_of_token)):
+        _gpu(name, meta, torch.int32, 1)
+        if not (meta.shape[0] >= m):
+            raise ValueError(f"{name} has {meta.shape[0]} entries for {m} rows")
+    _gpu("seq_slot", seq_slot, torch.int32, 1)
+    _gpu("block_table", block_table, torch.int32, 2)
+    page_size = _check_pools(k_pool, v_pool, torch.bfloat16, kv_heads, head_dim)
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=a.device)
+    _run("cie_gemm_tiles_rope", load_library().cie_gemm_tiles_rope(
+        _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k), _i(columns), _i(rows),
+        _ptr(cos), _ptr(sin), _ptr(positions), _ptr(seq_of_token), _ptr(seq_slot), _ptr(block_table),
+        _i(block_table.shape[1]), _ptr(k_pool), _ptr(v_pool), _i(q_heads), _i(kv_heads), _i(head_dim), _i(page_size),
+        _i(1 if rotate else 0), _i(1 if write_kv else 0)))
+    return out
 
 
 def gemm_qkv_rope(weight: torch.Tensor, a: Optional[torch.Tensor], bias: Optional[torch.Tensor], cos: torch.Tensor,

@@ -22,7 +22,11 @@ from ..config.specs import PartSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import Part, build_part, register_part
-from .linear import FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, linear
+from .linear import (BEHIND_RATE, FUSED_PARTS_ROWS, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, linear,
+                     plan_tiles)
+
+
+ROTATION_US = 5.0  # what the rotation's kernel costs behind the library's q/k/v product, beside its traffic
 
 
 class Attention(Part):
@@ -30,6 +34,7 @@ class Attention(Part):
     adds_to_residual = True
     folds_next_norm = True  # its output product can leave the next norm's rows short of their scale
     takes_raw_rows = True  # its first product can make the norm of a few rows itself
+    sums_parts = True  # its last product may come back as parts of K
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int,
                  qkv_bias: bool, out_bias: bool, position: PartSpec, window: Optional[int] = None,
                  scale: Optional[float] = None) -> None:
@@ -114,7 +119,7 @@ class Attention(Part):
         return qkv
 
     def forward(self, x, batch, view, writes: bool = True, residual: Optional[torch.Tensor] = None,
-                next_norm=None):
+                next_norm=None, sums_parts: bool = False):
         if batch.max_context > self.position.max_position and self.position.rotates:
             raise ValueError(
                 f"position {batch.max_context - 1} is beyond the rotary table of {self.position.max_position}"
@@ -136,10 +141,18 @@ class Attention(Part):
                     folded=(x.residual, x.norm.weight_f32, x.norm.eps))
                 context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, head_dim,
                                  self.window, self.scale)
-                return linear(context, self.w_o, self.b_o, into=residual, then_norm=next_norm)
+                return linear(context, self.w_o, self.b_o, into=residual, then_norm=next_norm, sums_parts=sums_parts)
             x = x.complete()
-        if (x.dtype == torch.bfloat16 and few and untouched and head_dim % 32 == 0
-                and x.shape[1] % 8 == 0 and (rows == 1 or x.stride(0) % 8 == 0)):
+        fused = (x.dtype == torch.bfloat16 and untouched and head_dim % 32 == 0
+                 and x.shape[1] % 8 == 0 and (rows == 1 or x.stride(0) % 8 == 0))
+        # (the tiles' epilogue saves the rotation's kernel)
+        tiles = (plan_tiles(rows, self.w_qkv.shape[0], x.shape[1], behind_us=ROTATION_US + rows * self.w_qkv.shape[0] * 4e-6 / BEHIND_RATE)
+                 if fused and not few and rows > FUSED_PARTS_ROWS and x.data_ptr() % 16 == 0 else None)
+        if tiles is not None:
+            qkv = ops.gemm_tiles_rope(self.w_qkv, x, self.b_qkv, self.cos, self.sin, batch.positions, batch.seq_of_token,
+                                      batch.seq_slot, view.block_table, view.k_pool, view.v_pool, self.num_heads,
+                                      self.num_kv_heads, head_dim, *tiles[:2], rotate=self.position.rotates, write_kv=writes)
+        elif fused and few:
             # few rows (where the hand-written product is the faster one): its epilogue rotates and writes the cache
             qkv = ops.gemm_qkv_rope(self.w_qkv, x, self.b_qkv, self.cos, self.sin, batch.positions,
                                     batch.seq_of_token, batch.seq_slot, view.block_table, view.k_pool, view.v_pool,
@@ -152,7 +165,7 @@ class Attention(Part):
                               head_dim, rotate=self.position.rotates, write_kv=writes, rotary_dim=rotary_dim)
         context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, head_dim,
                          self.window, self.scale)
-        return linear(context, self.w_o, self.b_o, into=residual, then_norm=next_norm)
+        return linear(context, self.w_o, self.b_o, into=residual, then_norm=next_norm, sums_parts=sums_parts)
 
 
 WIDE_DECODE_KEYS = 2048  # contexts from which decode rows go to the four-wave form

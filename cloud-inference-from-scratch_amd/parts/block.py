@@ -32,7 +32,7 @@ from ..config.specs import LayerSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import build_part, register_part
-from .linear import Added, RawRows, RowSumsq, StreamRows, WeightedPair, linear, linear_beside
+from .linear import Added, KParts, RawRows, RowSumsq, StreamRows, WeightedPair, linear, linear_beside
 
 
 class PreNormBlock:
@@ -99,6 +99,8 @@ class PreNormBlock:
 
     def _behind_first_norm(self, x, residual: torch.Tensor, batch, view, writes: bool):
         extra = {"residual": residual} if getattr(self.mixer, "adds_to_residual", False) else {}
+        if extra and getattr(self.mixer, "sums_parts", False):
+            extra["sums_parts"] = True
         if (extra and self.has_feed_forward and getattr(self.mixer, "folds_next_norm", False)
                 and getattr(self.norm2, "folds_into_products", False)
                 and getattr(self.feed_forward, "takes_scaled_rows", False)):
@@ -108,6 +110,8 @@ class PreNormBlock:
             return residual, mixed  # (the next norm adds it)
         x = normalise(self.norm2, residual, mixed, self.dtype)
         extra = {"residual": residual} if getattr(self.feed_forward, "adds_to_residual", False) else {}
+        if extra and getattr(self.feed_forward, "sums_parts", False):
+            extra["sums_parts"] = True
         return residual, self.feed_forward.forward(x, **extra)
 
 
@@ -115,7 +119,9 @@ def normalise(norm, residual: torch.Tensor, pending, dtype: torch.dtype, rows=No
     """Run ``norm`` on the residual stream plus what is pending.  Only a norm that
     says so (``takes_row_sumsq``) is shown the fused forms of a branch; for any
     other an already added branch becomes ``None``."""
-    if not getattr(norm, "takes_row_sumsq", False) and isinstance(pending, (RowSumsq, Added)):
+    if not getattr(norm, "takes_row_sumsq", False) and isinstance(pending, (RowSumsq, Added, KParts)):
+        if isinstance(pending, KParts):
+            pending.join(residual)
         pending = None
     if isinstance(pending, WeightedPair):
         pending = pending.combined()
@@ -128,6 +134,9 @@ def whole_stream(residual: torch.Tensor, pending) -> torch.Tensor:
     """The float32 stream with what is pending added to it."""
     if isinstance(pending, WeightedPair):
         pending = pending.combined()
+    if isinstance(pending, KParts):
+        pending.join(residual)
+        return residual
     if isinstance(pending, torch.Tensor):
         return residual + pending.float()
     if pending is None or isinstance(pending, (Added, RowSumsq, NormedRows)):

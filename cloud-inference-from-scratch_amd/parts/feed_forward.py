@@ -20,6 +20,7 @@ class GatedMLP(Part):
     graph_safe = True
     adds_to_residual = True
     takes_scaled_rows = True  # its first product applies the scale of rows that come without it
+    sums_parts = True  # its last product may come back as parts of K
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str = "silu",
                  names: tuple[str, str, str] = ("gate_proj.weight", "up_proj.weight", "down_proj.weight")) -> None:
         if activation != "silu":
@@ -45,8 +46,8 @@ class GatedMLP(Part):
     def warm_up(self, rows: int) -> None:
         self.forward(torch.zeros((rows, self.hidden_size), dtype=self.w_down.dtype, device=self.w_down.device))
 
-    def forward(self, x, residual: Optional[torch.Tensor] = None):
-        return linear(linear(x, self.w_gate_up, epilogue="silu"), self.w_down, into=residual)
+    def forward(self, x, residual: Optional[torch.Tensor] = None, sums_parts: bool = False):
+        return linear(linear(x, self.w_gate_up, epilogue="silu"), self.w_down, into=residual, sums_parts=sums_parts)
 
 
 class ClampedGatedMLP(Part):

@@ -10,13 +10,16 @@ residual stream (``into=residual``), or float32 results for the logits.  They
 come in two forms: waves that share K and own all rows (few rows; the q/k/v,
 o_proj and head products), and waves that own columns and share the rows through
 LDS (the SiLU-gate product up to 64 rows and every product whose K is cut).
-bfloat16 with more rows: the vendor library's product (hipBLASLt through a
-thin cached interface of this package), as the reference leaves its products to
-a library (src/cloud_engine/model.py:89-137), with the small kernels around it.
+bfloat16 with more rows: tiles of this package's own (``csrc/gemm_tiles.hip``) where
+few tiles or a kernel behind the product would cost the library more, else the
+vendor library's product (hipBLASLt through a thin cached interface of this
+package), as the reference leaves its products to a library
+(src/cloud_engine/model.py:89-137), with the small kernels around it.
 """
 
 from __future__ import annotations
 
+import functools
 import weakref
 from dataclasses import dataclass
 from typing import Any, Optional, Union
@@ -95,6 +98,54 @@ def plan_shared_parts(tiles: int, k: int) -> tuple[int, int, int]:
     return column_tiles, waves, parts
 
 
+# Products of more rows than the kernels above take (beyond ``FUSED_PARTS_ROWS``) go to tiles of this package or to the
+# vendor library, whichever the two models below say is faster.
+# Tiles: us per slice of 64 k of a workgroup alone on its unit, and of every further one that meets it there (measured on
+# MI355X at the 3B shape's widths, one to eleven workgroups a unit; what bounds them is the rate at which a unit is fed
+# from its L2, some 20 bytes a cycle, hence the advantage of large tiles where they are many).
+TILE_SLICE_US = {(64, 64): (0.28, 0.17), (128, 64): (0.39, 0.35), (128, 128): (0.63, 0.55), (128, 256): (0.94, 1.20)}
+TILE_PARTS = (1, 2, 3, 4, 6, 8)
+TILE_START_US = 5.0
+# parts of K: float32 sums written by the product and read by the norm, MB per us
+TILE_PARTS_RATE = 4.5
+# The library, whose algorithms do not cut K: some 0.95 PFLOP/s (GFLOP per us) where tiles of 128 x 128 give every unit
+# one, less by the root of the share that have one, a little more where several meet on one, up to 1.25; and never faster
+# than 9 us and 2.8 per 1,000 k (measured, modelled in brackets, us: 3B down at 256 / 613 / 1,024 / 2,048 rows 38 / 63 /
+# 73 / 100 (40 / 52 / 69 / 97), gate/up 37 / 64 / 86 / 139 (24 / 49 / 75 / 147); o_proj 15-18 (15-17)).
+LIBRARY_RATE, LIBRARY_MOST = 0.95, 1.25
+LIBRARY_START_US, LIBRARY_K_US = 9.0, 2.8e-3
+# what a kernel behind the library's product costs that an epilogue saves: its launch, and its traffic
+BEHIND_US = 5.0
+BEHIND_RATE = 5.0
+TILES_MARGIN = 1.03  # the tiles are taken where they are modelled to be faster by this
+
+
+@functools.lru_cache(maxsize=4096)
+def _plan_tiles(rows: int, n: int, k: int, most_parts: int, behind_us: float, units: int) -> Optional[tuple[int, int, int]]:
+    best = None
+    for (columns, tile_rows), (first, further) in TILE_SLICE_US.items():
+        tiles = -(-rows // tile_rows) * -(-n // columns)
+        for parts in TILE_PARTS:
+            per_part = -(-(-(-k // parts)) // 64) * 64
+            if parts > most_parts or per_part * (parts - 1) >= k:
+                continue
+            cost = TILE_START_US + per_part / 64 * (first + (-(-tiles * parts // units) - 1) * further)
+            if parts > 1:
+                cost += parts * rows * n * 8e-6 / TILE_PARTS_RATE
+            if best is None or cost < best[0]:
+                best = (cost, (columns, tile_rows, parts))
+    share = -(-rows // 128) * -(-n // 128) / units
+    rate = min(LIBRARY_MOST, LIBRARY_RATE * share ** (0.5 if share < 1.0 else 0.15))
+    library = max(LIBRARY_START_US + LIBRARY_K_US * k, 2e-9 * rows * n * k / rate) + behind_us
+    return best[1] if best[0] * TILES_MARGIN < library else None
+
+
+def plan_tiles(rows: int, n: int, k: int, most_parts: int = 1, behind_us: float = 0.0) -> Optional[tuple[int, int, int]]:
+    """(columns, rows, parts of K) of the tiles that a bfloat16 product of some hundred rows takes, or ``None`` where the
+    library's product (and a kernel of ``behind_us`` behind it, which the tiles' epilogue would save) is the faster one."""
+    return _plan_tiles(rows, n, k, most_parts, behind_us, ops.compute_units())
+
+
 @dataclass
 class RowSumsq:
     """Stands where a branch output would: the branch was already added into the
@@ -134,6 +185,19 @@ class Added:
     """Stands where a branch output would: the branch was already added into the residual stream, and
     nothing else is known of the stream's rows (a product whose K was cut into parts, each of which added
     its share with atomic adds)."""
+
+
+@dataclass
+class KParts:
+    """Stands where a branch output would: the branch is the sum of ``parts`` [P, rows, hidden] (float32), still to be
+    added into the stream, in order: a product whose K was cut.  A norm that says ``takes_row_sumsq`` sums them itself."""
+
+    parts: torch.Tensor
+
+    def join(self, residual: torch.Tensor) -> None:
+        """Add the branch into the stream (for a reader that cannot sum the parts)."""
+        for part in self.parts:
+            residual.add_(part)
 
 
 @dataclass
@@ -232,7 +296,8 @@ def _fusable(rows: int, k: int, row_stride: int, weight: torch.Tensor) -> bool:
 
 def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out_dtype: Optional[torch.dtype] = None, epilogue: Optional[str] = None,
-           into: Optional[torch.Tensor] = None, then_norm: Any = None) -> Union[torch.Tensor, RowSumsq, Added]:
+           into: Optional[torch.Tensor] = None, then_norm: Any = None,
+           sums_parts: bool = False) -> Union[torch.Tensor, RowSumsq, Added, KParts]:
     """``x @ weight.T + bias``.
 
     ``epilogue="silu"``: weight stacks gate rows over up rows; returns
@@ -241,6 +306,7 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
     :class:`RowSumsq` comes back, or (a product whose K was cut into parts that
     each add their share) an :class:`Added`; otherwise the plain
     result comes back and the caller adds it (the next norm kernel does).
+    ``sums_parts`` (with ``into``): the caller's block takes :class:`KParts` too.
     ``then_norm`` (with ``into``): the norm that follows, if it can be folded into
     this product and the next (``RMSNorm.folds_into_products``): the residual
     epilogue then also leaves that norm's output short of the rows' scale.
@@ -301,6 +367,23 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
             return ops.gemm_fused(weight, ops.EPI_SILU, x)
         elif not silu:
             return ops.gemm_fused(weight, ops.EPI_F32 if wants_f32 else ops.EPI_BF16, x, bias=bias)
+    if fusable and rows > FUSED_PARTS_ROWS and not wants_f32 and x.data_ptr() % 16 == 0:
+        tiles = None
+        if into is not None and not silu and into.is_contiguous() and tuple(into.shape) == (rows, n):
+            tiles = plan_tiles(rows, n, k, most_parts=TILE_PARTS[-1] if sums_parts else 1)
+            if tiles is not None and tiles[2] > 1:
+                return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, *tiles[:2], bias=bias, parts=tiles[2]))
+            if tiles is not None:
+                ops.gemm_tiles(weight, ops.TILE_RESID, x, *tiles[:2], bias=bias, into=into)
+                return Added()
+        elif into is None and silu and n % 2 == 0 and bias is None:
+            tiles = plan_tiles(rows, n, k, behind_us=BEHIND_US + rows * n * 3e-6 / BEHIND_RATE)
+            if tiles is not None:
+                return ops.gemm_tiles(weight, ops.TILE_SILU, x, *tiles[:2])
+        elif into is None and not silu:
+            tiles = plan_tiles(rows, n, k)
+            if tiles is not None:
+                return ops.gemm_tiles(weight, ops.TILE_BF16, x, *tiles[:2], bias=bias)
     if weight.dtype == torch.float32:
         if silu and n % 2 == 0 and bias is None:
             return ops.gemm_f32(x, weight, gate=True)

@@ -15,7 +15,7 @@ import torch
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import Part, register_part
-from .linear import Added, RowSumsq, ScaledRows, SummedBranch, WeightedPair
+from .linear import Added, KParts, RowSumsq, ScaledRows, SummedBranch, WeightedPair
 
 
 class RMSNorm(Part):
@@ -44,10 +44,12 @@ class RMSNorm(Part):
     def forward(self, residual: torch.Tensor, branch, out_dtype: torch.dtype,
                 rows: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``branch`` is a tensor still to be added into ``residual``, ``None``, an
-        ``Added`` (already added) or a ``RowSumsq`` (already added; the rows' sums
-        of squares are known, so the norm needs no reduction)."""
+        ``Added`` (already added), ``KParts`` (summed here) or a ``RowSumsq`` (already
+        added; the rows' sums of squares are known, so the norm needs no reduction)."""
         if isinstance(branch, Added):
             branch = None
+        if isinstance(branch, KParts):
+            return ops.add_rmsnorm(residual, None, self.weight, self.eps, out_dtype, rows=rows, parts=branch.parts)
         if isinstance(branch, RowSumsq):
             if branch.scaled is not None and branch.norm is self and rows is None and out_dtype == torch.bfloat16:
                 return ScaledRows(branch.scaled, branch.sumsq, self.eps, residual, self)

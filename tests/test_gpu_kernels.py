@@ -145,6 +145,78 @@ def test_gemm_fused_plain_any_size(ops, shape, out_dtype):
     torch.testing.assert_close(ops.gemm_fused(w, ops.EPI_F32, wide[:, :k]), ops.gemm_fused(w, ops.EPI_F32, a), rtol=0, atol=0)
 
 
+# (rows, columns, K): less than a tile, edges of 16 and of the tiles, a K that ends inside a slice, odd columns
+@pytest.mark.parametrize("shape", [(1, 32, 8), (63, 64, 64), (65, 130, 136), (129, 256, 200), (200, 99, 72), (257, 96, 1032)])
+@pytest.mark.parametrize("tile", [(64, 64), (128, 64), (128, 128), (128, 256)])
+def test_gemm_tiles(ops, shape, tile):
+    """Products of some hundred rows in tiles: the plain result with bias, its gated unit, the add into the stream and the
+    parts of K (which sum to the same), for rows that lie apart too."""
+    m, n, k = shape
+    wide = torch.zeros((m, k + 24), dtype=torch.bfloat16).cuda()
+    wide[:, :k] = rand((m, k), torch.bfloat16, 16)
+    a, w, b = wide[:, :k], rand((n, k), torch.bfloat16, 17), rand((n,), torch.bfloat16, 18)
+    product = a.double() @ w.double().t()
+    sums = dict(rtol=1e-4, atol=1e-4 * math.sqrt(k))       # float32 sums of k products of numbers about 1
+    rounded = dict(rtol=1e-2, atol=1e-2 * math.sqrt(k))    # ... rounded to bfloat16
+    torch.testing.assert_close(ops.gemm_tiles(w, ops.TILE_BF16, a, *tile, bias=b).double(), product + b.double(), **rounded)
+    if n % 2 == 0:
+        gate, up = product[:, : n // 2], product[:, n // 2:]
+        torch.testing.assert_close(ops.gemm_tiles(w, ops.TILE_SILU, a, *tile).double(), torch.nn.functional.silu(gate) * up,
+                                   rtol=1e-2, atol=1e-2 * k)
+    stream = rand((m, n), torch.float32, 19)
+    expect = stream.double() + product + b.double()
+    ops.gemm_tiles(w, ops.TILE_RESID, a, *tile, bias=b, into=stream)
+    torch.testing.assert_close(stream.double(), expect, **sums)
+    for parts in (1, 2, 3):
+        if (parts - 1) * (-(-(-(-k // parts)) // 64) * 64) < k:  # (every part has some of K)
+            got = ops.gemm_tiles(w, ops.TILE_PARTS, a, *tile, bias=b, parts=parts)
+            assert got.shape == (parts, m, n)
+            torch.testing.assert_close(got.double().sum(0), product + b.double(), **sums)
+
+
+@pytest.mark.parametrize("heads", [(4, 2, 128), (3, 1, 96), (14, 2, 64), (2, 2, 32)])
+@pytest.mark.parametrize("tile", [(64, 64), (128, 64), (128, 128), (128, 256)])
+@pytest.mark.parametrize("rotate,write", [(True, True), (False, True), (True, False)])
+def test_gemm_tiles_rope(ops, heads, tile, rotate, write):
+    """The q/k/v product whose epilogue rotates and writes the cache: the bits of the plain epilogue and the rotation's
+    kernel behind it, with rows of two sequences in pages that are not in order."""
+    q_heads, kv_heads, dim = heads
+    m, k, page = 133, 200, 8
+    n = (q_heads + 2 * kv_heads) * dim
+    a, w, b = rand((m, k), torch.bfloat16, 20), rand((n, k), torch.bfloat16, 21), rand((n,), torch.bfloat16, 22)
+    as_dev = lambda values: torch.tensor(values, dtype=torch.int32).cuda()  # noqa: E731
+    first = 70
+    positions = as_dev(list(range(5, 5 + first)) + list(range(m - first)))
+    seqs, slots = as_dev([0] * first + [1] * (m - first)), as_dev([2, 0])
+    table = torch.randperm(48, generator=torch.Generator().manual_seed(23)).to(torch.int32).reshape(3, 16).cuda()
+    cos, sin = rand((128, dim // 2), torch.float32, 24), rand((128, dim // 2), torch.float32, 25)
+    pools = [torch.zeros((48, kv_heads, page, dim), dtype=torch.bfloat16).cuda(), torch.zeros((48, kv_heads, dim, page), dtype=torch.bfloat16).cuda()]
+    plain_pools = [p.clone() for p in pools]
+    got = ops.gemm_tiles_rope(w, a, b, cos, sin, positions, seqs, slots, table, *pools, q_heads, kv_heads, dim, *tile,
+                              rotate=rotate, write_kv=write)
+    expect = ops.gemm_tiles(w, ops.TILE_BF16, a, *tile, bias=b)
+    ops.rope_kv_write(expect, cos, sin, positions, seqs, slots, table, *plain_pools, q_heads, kv_heads, dim, rotate=rotate, write_kv=write)
+    assert torch.equal(got[:, : q_heads * dim], expect[:, : q_heads * dim])
+    assert all(torch.equal(x, y) for x, y in zip(pools, plain_pools))
+
+
+@pytest.mark.parametrize("dtype,hidden", [(torch.bfloat16, 64), (torch.bfloat16, 100), (torch.float32, 96)])
+@pytest.mark.parametrize("parts", [1, 3, 6])
+def test_add_rmsnorm_sums_parts(ops, dtype, hidden, parts):
+    """Parts of a branch join the stream in order, in the whole step's form and for chosen rows."""
+    stream, weight = rand((37, hidden), torch.float32, 26), rand((hidden,), dtype, 27)
+    pieces = rand((parts, 37, hidden), torch.float32, 28)
+    whole = stream.clone()
+    for piece in pieces:
+        whole += piece
+    expect = ops.add_rmsnorm(whole.clone(), None, weight, 1e-6, dtype)
+    rows = torch.tensor([36, 0, 5], dtype=torch.int32).cuda()
+    chosen = ops.add_rmsnorm(stream, None, weight, 1e-6, dtype, rows=rows, parts=pieces)
+    assert torch.equal(chosen, ops.add_rmsnorm(whole.clone(), None, weight, 1e-6, dtype, rows=rows))
+    assert torch.equal(ops.add_rmsnorm(stream, None, weight, 1e-6, dtype, parts=pieces), expect)
+    assert torch.equal(stream, whole)
+
+
 def build_cache(dtype, lengths, kv_heads, head_dim, page_size, seed, shuffle=True):
     """Random keys/values for sequences of the given lengths, scattered over the
     pages of a pool in a shuffled order.  Returns pools, block table and the
