@@ -1351,6 +1351,7 @@ def retention(proj: torch.Tensor, offsets: tuple[int, int, int, int], cos: Optio
 
 
 MAX_CONV_TAPS = 16
+MAX_SCAN_SEGMENTS = 64
 
 
 def causal_conv(x: torch.Tensor, taps_w: torch.Tensor, bias: Optional[torch.Tensor], past: torch.Tensor,
@@ -1416,7 +1417,7 @@ def gated_recurrence(y_pre: torch.Tensor, x_in: torch.Tensor, u: torch.Tensor, g
     ``a = exp(rate * sigmoid(r))``, ``S = a * S + sqrt(1 - a^2) * sigmoid(i) * u``, ``out = S * gelu_tanh(y_pre)``,
     with r and i from ``gates`` (float32 [T, 2C], per block of ``block_width`` channels its r then its i).  ``state``
     float32 [slots, C]; ``past`` float32 [slots, max(taps - 1, 1), C] is moved on with the step's ``x_in``.
-    ``segments`` (1 to 16) stretches of a sequence's tokens run side by side and are joined by the recurrence's
+    ``segments`` (1 to 64) stretches of a sequence's tokens run side by side and are joined by the recurrence's
     own linearity (for long portions; the result differs from the walk in order by float32 rounding only)."""
     tokens, channels = u.shape
     for name, t in (("y_pre", y_pre), ("x_in", x_in)):
@@ -1429,7 +1430,7 @@ def gated_recurrence(y_pre: torch.Tensor, x_in: torch.Tensor, u: torch.Tensor, g
     _gpu("past", past, torch.float32, 3)
     if (tuple(gates.shape) != (tokens, 2 * channels) or rate.shape[0] != channels or state.shape[1] != channels
             or tuple(past.shape[1:]) != (max(taps - 1, 1), channels) or channels % block_width
-            or not 1 <= taps <= MAX_CONV_TAPS or not 1 <= segments <= 16):
+            or not 1 <= taps <= MAX_CONV_TAPS or not 1 <= segments <= MAX_SCAN_SEGMENTS):
         raise ValueError("gates, rate, state or past do not fit the channels")
     for name, meta, least in (("seq_slot", seq_slot, sequences), ("q_start_loc", q_start_loc, sequences + 1)):
         _gpu(name, meta, torch.int32, 1)

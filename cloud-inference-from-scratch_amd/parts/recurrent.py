@@ -179,6 +179,15 @@ class LightningAttention(Part):
 SCAN_SEGMENT_TOKENS = 64  # portions from which the recurrence's tokens are cut into stretches
 
 
+def scan_segments(longest: int) -> int:
+    """How many stretches the recurrence cuts a portion of ``longest`` tokens into: 16, and beyond 512 tokens as many
+    (in steps of 16) as keep a stretch within the 32 tokens that a thread holds in registers (1,999 tokens of 2,048
+    channels: 107 us in 16 stretches read twice, 44 in 64; some 80 tokens: 13 us in 16, 32 in 64)."""
+    if longest < SCAN_SEGMENT_TOKENS:
+        return 1
+    return min(ops.MAX_SCAN_SEGMENTS, max(16, -(-longest // (32 * 16)) * 16))
+
+
 class GatedLinearRecurrence(Part):
     graph_safe = True
 
@@ -230,7 +239,7 @@ class GatedLinearRecurrence(Part):
         u = ops.causal_conv(x_in, self.conv_w, self.conv_b, past, batch.seq_of_token, batch.seq_slot, batch.q_start_loc)
         gates = ops.block_linear(u, self.w_gates, self.b_gates, out_dtype=torch.float32)
         # long portions run as stretches side by side (the portion lengths are the host's, and a captured step's own)
-        segments = 16 if batch.max_q_len >= SCAN_SEGMENT_TOKENS else 1
+        segments = scan_segments(batch.max_q_len)
         out = ops.gated_recurrence(y_pre, x_in, u, gates, w // self.blocks, self.rate, state, past, batch.seq_slot,
                                    batch.q_start_loc, batch.sequences, self.taps, segments)
         return linear(out, self.w_o)

@@ -365,3 +365,87 @@ def test_layer_boundary_kernel(dtype):
         nothing, normed = ops.depth_stream(x, gains=(3.0, 1.0), out_dtype=dtype, eps=1e-5, want_stream=False)
         unit = x.double() / torch.sqrt((x.double() ** 2).mean(-1, keepdim=True) + 1e-5)
         assert nothing is None and torch.allclose(normed[0].double(), 3.0 * unit, atol=tol, rtol=tol)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,hidden,terms,newest", [
+    (1, 4, 1, 0), (5, 2048, 9, 8), (5, 2048, 8, 3), (3, 4096, 10, 9), (2, 4100, 17, 16), (2, 6144, 18, 0), (4, 260, 3, 4)])
+def test_layer_boundary_kernel_over_depths_and_widths(dtype, rows, hidden, terms, newest):
+    """The boundary with four numbers a thread: one piece and several a thread, a width that ends inside a wave, up to
+    eight earlier rows asked for at once and more, the row just made first, in the middle, last and outside the average;
+    and the same over views that start off a 16-byte line, which take the form of single numbers."""
+    from cie_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(2)
+    layers = max(terms, newest + 1)
+    weights = torch.randn(terms, generator=g)
+    for shift in (0, 1):
+        def rand(*shape, kind=torch.float32):  # (a tensor whose first number lies `shift` numbers off the allocation's start)
+            n = torch.Size(shape).numel()
+            return torch.randn(n + shift, generator=g).to(kind).cuda()[shift:].view(shape)
+        history, x = rand(layers, rows, hidden), rand(rows, hidden)
+        a, b = rand(rows, hidden, kind=dtype), rand(rows, hidden, kind=dtype)
+        kept = history.clone()
+        stream, normed = ops.depth_stream(x, a, b, mult=0.7, history=history, newest=newest, weights=weights.cuda(),
+                                          gains=(1.5, 0.25), out_dtype=dtype, eps=1e-5)
+        new = x.double() + 0.7 * (a.double() + b.double())
+        rest = [j for j in range(layers) if j != newest]
+        assert torch.allclose(history[newest].double(), new, atol=1e-5) and torch.equal(history[rest], kept[rest])
+        parts = [weights[j].double().item() * (new if j == newest else kept[j].double()) for j in range(terms)]
+        want, size = sum(parts), sum(p.abs() for p in parts)
+        # each of the sum's `terms` roundings is at most half a unit in the last place of a partial sum below `size`; three
+        # more make the row just made
+        assert torch.all((stream.double() - want).abs() <= (terms + 3) * 2.0 ** -24 * (size + 2.0))
+        unit = want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-5)
+        tol = 1e-5 if dtype == torch.float32 else 2e-2
+        assert torch.allclose(normed[0].double(), unit * 1.5, atol=tol, rtol=tol)
+        assert torch.allclose(normed[1].double(), unit * 0.25, atol=tol, rtol=tol)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lengths,channels,taps,segments", [
+    ((64, 1, 129), 48, 4, 64), ((63, 65), 16, 4, 64), ((2048,), 128, 4, 64), ((2049, 70), 40, 3, 64), ((4100,), 16, 4, 64),
+    ((300, 5), 24, 4, 2), ((97,), 40, 4, 16), ((9, 2, 3), 72, 4, 1)])
+def test_gated_recurrence_and_its_convolution(dtype, lengths, channels, taps, segments):
+    """Stretches of one token and of the most a round has, portions one short of a round, one round, and one longer than
+    it, fewer tokens than stretches, workgroups that end behind the last channel; against the walk in order in 64 bits."""
+    from cie_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(3)
+    tokens, width = sum(lengths), channels // 2
+    slots = list(range(len(lengths)))[::-1]
+    proj = torch.randn(tokens, 2 * channels, generator=g).to(dtype).cuda()
+    y_pre, x_in = proj[:, :channels], proj[:, channels:]
+    taps_w = torch.randn(channels, taps, generator=g).to(dtype).cuda()
+    bias = torch.randn(channels, generator=g).to(dtype).cuda()
+    past = torch.randn(len(lengths), taps - 1, channels, generator=g).cuda()
+    state = torch.randn(len(lengths), channels, generator=g).cuda()
+    gates = torch.randn(tokens, 2 * channels, generator=g).cuda()
+    rate = -8.0 * torch.rand(channels, generator=g).cuda()
+    starts = [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    meta = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+    of_token = meta([i for i, n in enumerate(lengths) for _ in range(n)])
+    old_past, old_state = past.clone(), state.clone()
+    u = ops.causal_conv(x_in, taps_w, bias, past, of_token, meta(slots), meta(starts))
+    out = ops.gated_recurrence(y_pre, x_in, u, gates, width, rate, state, past, meta(slots), meta(starts), len(lengths),
+                               taps, segments)
+    # a bfloat16 result is rounded once; float32 sums of up to 17 and of some ten terms in front of it
+    tol = dict(atol=3e-5, rtol=3e-5) if dtype == torch.float32 else dict(atol=3e-5, rtol=2.0 ** -8)
+    for i, n in enumerate(lengths):
+        at, slot = starts[i], slots[i]
+        series = torch.cat([old_past[slot], x_in[at: at + n].float()])
+        window = series.double().unfold(0, taps, 1)  # [n, channels, taps]
+        conv = (window * taps_w.double()).sum(-1) + bias.double()
+        assert torch.allclose(u[at: at + n].double(), conv, **tol)
+        assert torch.equal(past[slot], series[-(taps - 1):])
+        gate = gates[at: at + n].double().view(n, 2, 2, width).cpu()
+        log_a = rate.double().cpu() * torch.sigmoid(gate[:, :, 0].reshape(n, channels))
+        moved = torch.sqrt(-torch.expm1(2 * log_a)) * torch.sigmoid(gate[:, :, 1].reshape(n, channels)) * u[at: at + n].double().cpu()
+        S, walked = old_state[slot].double().cpu(), []
+        for t in range(n):
+            S = torch.exp(log_a[t]) * S + moved[t]
+            walked.append(S)
+        want = torch.stack(walked) * torch.nn.functional.gelu(y_pre[at: at + n].double().cpu(), approximate="tanh")
+        # (S fades by 1 - a^2 against what it takes in: its float32 roundings do not add up over the tokens)
+        assert torch.allclose(out[at: at + n].double().cpu(), want, **tol)
+        assert torch.allclose(state[slot].double().cpu(), S, atol=3e-5, rtol=3e-5)
