@@ -38,72 +38,96 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ residual, const T* __rest
         dst[h] = from_float<T>((staged[h] * inv) * to_float(weight[h]));
 }
 
-// bf16 activations and weight, hidden a multiple of 8: eight elements per thread, 16-byte accesses.
-__global__ void add_rmsnorm_vec8_kernel(float* __restrict__ residual, const bf16_t* __restrict__ branch,
-                                        const bf16_t* __restrict__ weight, bf16_t* __restrict__ out,
-                                        int hidden, float eps, const float* __restrict__ parts, int n_parts, size_t apart) {
-    extern __shared__ float staged[];
+// Eight neighbouring numbers as float32, in 16-byte pieces.
+typedef float eight_t __attribute__((ext_vector_type(8)));
+typedef float half_eight_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ eight_t load_eight(const float* p) {
+    const half_eight_t lo = reinterpret_cast<const half_eight_t*>(p)[0], hi = reinterpret_cast<const half_eight_t*>(p)[1];
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+__device__ __forceinline__ eight_t load_eight(const bf16_t* p) {
+    const uint4 raw = *reinterpret_cast<const uint4*>(p);
+    return eight_t{__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xffff0000u), __uint_as_float(raw.y << 16),
+                   __uint_as_float(raw.y & 0xffff0000u), __uint_as_float(raw.z << 16), __uint_as_float(raw.z & 0xffff0000u),
+                   __uint_as_float(raw.w << 16), __uint_as_float(raw.w & 0xffff0000u)};
+}
+__device__ __forceinline__ void store_eight(float* p, eight_t v) {
+    reinterpret_cast<half_eight_t*>(p)[0] = __builtin_shufflevector(v, v, 0, 1, 2, 3);
+    reinterpret_cast<half_eight_t*>(p)[1] = __builtin_shufflevector(v, v, 4, 5, 6, 7);
+}
+__device__ __forceinline__ void store_eight(bf16_t* p, eight_t v) {
+    *reinterpret_cast<uint4*>(p) = uint4{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
+}
+
+// The same with eight elements a thread, where a row's 16-byte pieces lie on 16-byte lines.  What bounds it is the chain
+// launch, loads, two barriers, stores: a workgroup has as many waves as its row has pieces (idle waves cost the barriers
+// their time), the weight is on its way before the reduction, and parts, which few calls bring, are a kernel of their own.
+template <typename T, typename W, bool kParts>
+__global__ void __launch_bounds__(1024)
+add_rmsnorm_vec8_kernel(float* __restrict__ residual, const T* __restrict__ branch, const W* __restrict__ weight,
+                        T* __restrict__ out, const int* __restrict__ rows, int hidden, float eps, int write_residual,
+                        const float* __restrict__ parts, int n_parts, size_t apart) {
+    extern __shared__ float staged[];  // (the pieces of threads that have more than one)
     __shared__ float scratch[16];
-    const int row = blockIdx.x;
+    const int row = rows ? rows[blockIdx.x] : blockIdx.x;
     float* res = residual + static_cast<size_t>(row) * hidden;
-    const float* extra = parts + static_cast<size_t>(row) * hidden;  // (not read without parts)
-    const bf16_t* add = branch ? branch + static_cast<size_t>(row) * hidden : nullptr;
+    const T* add = branch ? branch + static_cast<size_t>(row) * hidden : nullptr;
+    const bool store = write_residual && (add || kParts);
+    const int h0 = threadIdx.x * 8;
+    const eight_t gain = load_eight(weight + min(h0, hidden - 8));
+    eight_t own = {};
     float sum_sq = 0.f;
-    for (int h = threadIdx.x * 8; h < hidden; h += blockDim.x * 8) {
-        float4 x0 = *reinterpret_cast<const float4*>(res + h);
-        float4 x1 = *reinterpret_cast<const float4*>(res + h + 4);
-        if (add) {
-            const uint4 raw = *reinterpret_cast<const uint4*>(add + h);
-            x0.x += __uint_as_float(raw.x << 16); x0.y += __uint_as_float(raw.x & 0xffff0000u);
-            x0.z += __uint_as_float(raw.y << 16); x0.w += __uint_as_float(raw.y & 0xffff0000u);
-            x1.x += __uint_as_float(raw.z << 16); x1.y += __uint_as_float(raw.z & 0xffff0000u);
-            x1.z += __uint_as_float(raw.w << 16); x1.w += __uint_as_float(raw.w & 0xffff0000u);
-        }
-        for (int first = 0; first < n_parts; first += 4) {
-            float4 a[4], b[4];
+    for (int h = h0; h < hidden; h += blockDim.x * 8) {
+        eight_t x = load_eight(res + h);
+        if (add) x += load_eight(add + h);
+        if constexpr (kParts) {
+            const float* extra = parts + static_cast<size_t>(row) * hidden + h;
+            for (int first = 0; first < n_parts; first += 4) {
+                eight_t piece[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {  // (four under way at a time; a part past the last is read again and dropped)
-                const float* from = extra + min(first + i, n_parts - 1) * apart + h;
-                a[i] = *reinterpret_cast<const float4*>(from);
-                b[i] = *reinterpret_cast<const float4*>(from + 4);
-            }
+                for (int i = 0; i < 4; ++i)  // (four under way at a time; a part past the last is read again and dropped)
+                    piece[i] = load_eight(extra + min(first + i, n_parts - 1) * apart);
+                __builtin_amdgcn_sched_barrier(0);  // (no load may move to its use, where each would be waited for alone)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (first + i >= n_parts) break;
-                x0.x += a[i].x; x0.y += a[i].y; x0.z += a[i].z; x0.w += a[i].w;
-                x1.x += b[i].x; x1.y += b[i].y; x1.z += b[i].z; x1.w += b[i].w;
+                for (int i = 0; i < 4; ++i) {
+                    const eight_t with = x + piece[i];
+                    x = first + i < n_parts ? with : x;
+                }
             }
         }
-        if (add || n_parts) {
-            *reinterpret_cast<float4*>(res + h) = x0;
-            *reinterpret_cast<float4*>(res + h + 4) = x1;
-        }
-        *reinterpret_cast<float4*>(staged + h) = x0;
-        *reinterpret_cast<float4*>(staged + h + 4) = x1;
-        sum_sq += (x0.x * x0.x + x0.y * x0.y) + (x0.z * x0.z + x0.w * x0.w) + (x1.x * x1.x + x1.y * x1.y) +
-                  (x1.z * x1.z + x1.w * x1.w);
+        if (store) store_eight(res + h, x);
+        if (h == h0) own = x;
+        else store_eight(staged + h, x);
+        sum_sq += ((x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3])) +
+                  ((x[4] * x[4] + x[5] * x[5]) + (x[6] * x[6] + x[7] * x[7]));
     }
     const float total = block_sum(sum_sq, scratch);
     const float inv = 1.0f / sqrtf(total / static_cast<float>(hidden) + eps);
-    bf16_t* dst = out + static_cast<size_t>(row) * hidden;
-    for (int h = threadIdx.x * 8; h < hidden; h += blockDim.x * 8) {
-        const float4 x0 = *reinterpret_cast<const float4*>(staged + h);
-        const float4 x1 = *reinterpret_cast<const float4*>(staged + h + 4);
-        const uint4 raw = *reinterpret_cast<const uint4*>(weight + h);
-        uint4 packed;
-        packed.x = pack_bf16((x0.x * inv) * __uint_as_float(raw.x << 16), (x0.y * inv) * __uint_as_float(raw.x & 0xffff0000u));
-        packed.y = pack_bf16((x0.z * inv) * __uint_as_float(raw.y << 16), (x0.w * inv) * __uint_as_float(raw.y & 0xffff0000u));
-        packed.z = pack_bf16((x1.x * inv) * __uint_as_float(raw.z << 16), (x1.y * inv) * __uint_as_float(raw.z & 0xffff0000u));
-        packed.w = pack_bf16((x1.z * inv) * __uint_as_float(raw.w << 16), (x1.w * inv) * __uint_as_float(raw.w & 0xffff0000u));
-        *reinterpret_cast<uint4*>(dst + h) = packed;
-    }
+    T* dst = out + static_cast<size_t>(blockIdx.x) * hidden;
+    if (h0 < hidden) store_eight(dst + h0, (own * inv) * gain);
+    for (int h = h0 + blockDim.x * 8; h < hidden; h += blockDim.x * 8)
+        store_eight(dst + h, (load_eight(staged + h) * inv) * load_eight(weight + h));
 }
 
 template <typename T, typename W>
 static int launch_norm(hipStream_t s, float* residual, const void* branch, const void* weight,
                        void* out, const int* rows, int n_out, int hidden, float eps,
                        int write_residual, const float* parts, int n_parts, size_t apart) {
-    add_rmsnorm_kernel<T, W><<<n_out, n_out <= 64 ? 1024 : 256, hidden * sizeof(float), s>>>(
+    const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    const size_t bytes = hidden * sizeof(float);
+    if (hidden % 8 == 0 && aligned(residual) && aligned(branch) && aligned(weight) && aligned(out) && aligned(parts)) {
+        const int threads = min(1024, (hidden / 8 + kWave - 1) / kWave * kWave);
+#define CIE_NORM8(PARTS)                                                                                              \
+    add_rmsnorm_vec8_kernel<T, W, PARTS><<<n_out, threads, hidden > 8 * threads ? bytes : 0, s>>>(                       \
+        residual, static_cast<const T*>(branch), static_cast<const W*>(weight), static_cast<T*>(out), rows, hidden, eps, \
+        write_residual, parts, n_parts, apart)
+        if (n_parts) CIE_NORM8(true);
+        else CIE_NORM8(false);
+#undef CIE_NORM8
+        return cie_after_launch();
+    }
+    add_rmsnorm_kernel<T, W><<<n_out, n_out <= 64 ? 1024 : 256, bytes, s>>>(
         residual, static_cast<const T*>(branch), static_cast<const W*>(weight), static_cast<T*>(out),
         rows, hidden, eps, write_residual, parts, n_parts, apart);
     return cie_after_launch();
@@ -157,12 +181,6 @@ CIE_API int cie_add_rmsnorm(void* stream, int dtype, int wdtype, float* residual
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == CIE_F32 && wdtype == CIE_F32)
         return launch_norm<float, float>(s, residual, branch, weight, out, rows, n_out, hidden, eps, write_residual, parts, n_parts, apart);
-    if (dtype == CIE_BF16 && wdtype == CIE_BF16 && !rows && write_residual && hidden % 8 == 0) {
-        add_rmsnorm_vec8_kernel<<<n_out, n_out <= 64 ? 1024 : 256, hidden * sizeof(float), s>>>(
-            residual, static_cast<const bf16_t*>(branch), static_cast<const bf16_t*>(weight), static_cast<bf16_t*>(out),
-            hidden, eps, parts, n_parts, apart);
-        return cie_after_launch();
-    }
     if (dtype == CIE_BF16 && wdtype == CIE_BF16)
         return launch_norm<bf16_t, bf16_t>(s, residual, branch, weight, out, rows, n_out, hidden, eps, write_residual, parts, n_parts, apart);
     if (dtype == CIE_BF16 && wdtype == CIE_F32)
