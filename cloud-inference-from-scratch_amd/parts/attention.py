@@ -172,6 +172,7 @@ WIDE_DECODE_KEYS = 2048  # contexts from which decode rows go to the four-wave f
 # (the four-wave form cuts long contexts for as many workgroups as the GPU has compute units)
 FEW_DECODE_UNITS = 8  # (sequence, kv head) pairs below which they do not: parts of one wave fill the GPU better
 MANY_DECODE_UNITS = 96  # (sequence, kv head) pairs from which decode rows take the four-wave form at any context
+MANY_PART_BYTES = 300 << 10  # keys and values of one pair below which its keys are not cut then
 SHARED_DECODE_KEYS = 96  # contexts from which four waves share a decode row's keys without cutting them
 SPLIT_MIN_KEYS = 32  # the fewest keys of a one-wave part
 SPLIT_DECODE_KEYS = 192  # contexts from which the keys of decode rows are cut into parts at all
@@ -262,9 +263,13 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
         if wide and bound >= WIDE_DECODE_KEYS and units >= FEW_DECODE_UNITS:
             return ops.TILE_WAVES, dict(target_waves=cus, min_keys=32 * ops.TILE_WAVES)
         # Many pairs fill the GPU by themselves: the same form with the keys whole or in large parts
-        # (64 sequences x 2 heads x 256 keys: 9.2 us against 11.1 us with one wave per part)
+        # (64 sequences x 2 heads x 256 keys: 9.2 us against 11.1 us with one wave per part).  A second part pays for
+        # its merge where a unit has more to read than MANY_PART_BYTES (64 x 2 heads of 128, us, whole against two
+        # parts: 512 keys 12.5, 15.5; 1,024 keys 20.2, 21.5; 1,200 keys 24.7, 24.1; 1,536 keys 29.6, 28.0; 48 x 2
+        # heads: 700 keys 14.8, 15.7; 1,024 keys 19.8, 18.8; 64 x 2 heads of 64: 1,280 keys 14.1, 16.5).
         if wide and units >= MANY_DECODE_UNITS and bound >= SHARED_DECODE_KEYS:
-            return ops.TILE_WAVES, dict(target_waves=4 * cus // ops.TILE_WAVES, min_keys=512)
+            return ops.TILE_WAVES, dict(target_waves=4 * cus // ops.TILE_WAVES,
+                                        min_keys=max(512, MANY_PART_BYTES // (4 * head_dim)))
         # Otherwise one wave per part, parts down to one block of 32 keys (8 x 256 keys: 7.3 us in 8 parts,
         # 10.2 us in 2; 8 x 512 keys: 8.1 us in 16 parts, 10.6 us in 4) ...
         if bound >= SPLIT_DECODE_KEYS:
