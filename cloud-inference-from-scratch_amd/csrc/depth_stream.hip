@@ -1,14 +1,15 @@
 // The float32 stream of a decoder whose layers add their branches in parallel and whose next input is a
 // weighted average over the depth: one kernel per layer boundary.
 //
-//   v      = x + mult * (branch_a + branch_b)        (each branch optional; float32 sum)
+//   v      = x + mult * (branch_a + branch_b + sum_p parts[p])        (each optional; float32 sum, the parts in order)
 //   history[newest] = v                              (what the layer left, before any averaging)
 //   v      = sum_j weights[j] * history[j], j < terms (terms = 0: no averaging)
 //   stream = v
 //   out1   = v / sqrt(mean(v^2) + eps) * gain1       (RMS norms with one gain for all coordinates; each optional)
 //   out2   = v / sqrt(mean(v^2) + eps) * gain2
 //
-// x [rows, hidden] float32; branches and outputs in the activation type; history [layers + 1, rows, hidden]
+// x [rows, hidden] float32; branches and outputs in the activation type; parts [n_parts, rows, hidden] float32 (a branch
+// that comes as the parts of a product whose K was cut); history [layers + 1, rows, hidden]
 // float32.  One workgroup per row; the row passes through LDS, so hidden * 4 bytes must fit in 64 KB.
 #include "common.h"
 
@@ -17,16 +18,19 @@ __global__ void depth_stream_kernel(const float* __restrict__ x, const T* __rest
                                     const T* __restrict__ branch_b, float mult, float* __restrict__ history,
                                     long layer_stride, int newest, const float* __restrict__ weights, int terms,
                                     float* __restrict__ stream, T* __restrict__ out1, float gain1,
-                                    T* __restrict__ out2, float gain2, int hidden, float eps) {
+                                    T* __restrict__ out2, float gain2, int hidden, float eps,
+                                    const float* __restrict__ parts, int n_parts) {
     extern __shared__ float staged[];
     __shared__ float scratch[16];
     const size_t row = static_cast<size_t>(blockIdx.x) * hidden;
+    const size_t apart = static_cast<size_t>(gridDim.x) * hidden;
     float sum_sq = 0.f;
     for (int h = threadIdx.x; h < hidden; h += blockDim.x) {
         float v = x[row + h];
         if (branch_a) {
             float s = to_float(branch_a[row + h]);
             if (branch_b) s += to_float(branch_b[row + h]);
+            for (int p = 0; p < n_parts; ++p) s += parts[p * apart + row + h];
             v = v + mult * s;
         }
         if (newest >= 0) history[static_cast<size_t>(newest) * layer_stride + row + h] = v;
@@ -77,12 +81,13 @@ __device__ __forceinline__ void store_four(bf16_t* p, four_t v) {
 
 constexpr int kDepthAhead = 8;
 
-template <typename T>
+template <typename T, int kBranches, bool kParts>
 __global__ void __launch_bounds__(1024)
 depth_stream_vec4_kernel(const float* __restrict__ x, const T* __restrict__ branch_a, const T* __restrict__ branch_b,
                          float mult, float* __restrict__ history, long layer_stride, int newest,
                          const float* __restrict__ weights, int terms, float* __restrict__ stream, T* __restrict__ out1,
-                         float gain1, T* __restrict__ out2, float gain2, int hidden, float eps) {
+                         float gain1, T* __restrict__ out2, float gain2, int hidden, float eps,
+                         const float* __restrict__ parts, int n_parts) {
     extern __shared__ four_t staged4[];
     __shared__ float scratch[16];
     const size_t row = static_cast<size_t>(blockIdx.x) * hidden;
@@ -90,11 +95,35 @@ depth_stream_vec4_kernel(const float* __restrict__ x, const T* __restrict__ bran
     const int earlier = own < terms ? terms - 1 : terms;
     float sum_sq = 0.f;
     for (int h = threadIdx.x * 4; h < hidden; h += blockDim.x * 4) {
+        // (no load stands behind a condition, and none may move to its use: each would be waited for alone)
         const float* past = history + row + h;
-        four_t v = load_four(x + row + h);
-        if (branch_a) {
-            four_t s = load_four(branch_a + row + h);
-            if (branch_b) s += load_four(branch_b + row + h);
+        four_t v = load_four(x + row + h), branch[kBranches + 1], ahead[kDepthAhead];
+        if constexpr (kBranches > 0) branch[0] = load_four(branch_a + row + h);
+        if constexpr (kBranches > 1) branch[1] = load_four(branch_b + row + h);
+        const auto ask = [&](four_t (&piece)[kDepthAhead], const float* from, size_t apart, int first, int count, int leave_out) {
+#pragma unroll
+            for (int k = 0; k < kDepthAhead; ++k) {  // (a piece past the last reads the last again and is dropped)
+                const int j = min(first + k, count - 1);
+                piece[k] = load_four(from + static_cast<size_t>(j + (j >= leave_out)) * apart);
+            }
+        };
+        if (earlier > 0) ask(ahead, past, layer_stride, 0, earlier, own);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kBranches > 0) {
+            four_t s = branch[0];
+            if constexpr (kBranches > 1) s += branch[1];
+            if constexpr (kParts) {
+                for (int p0 = 0; p0 < n_parts; p0 += kDepthAhead) {
+                    four_t piece[kDepthAhead];
+                    ask(piece, parts + row + h, static_cast<size_t>(gridDim.x) * hidden, p0, n_parts, n_parts);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int k = 0; k < kDepthAhead; ++k) {
+                        const four_t with = s + piece[k];
+                        s = p0 + k < n_parts ? with : s;
+                    }
+                }
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = v[i] + mult * s[i];
         }
@@ -103,19 +132,16 @@ depth_stream_vec4_kernel(const float* __restrict__ x, const T* __restrict__ bran
             // (the terms in the layers' order, the row just made last, from its register)
             four_t acc = {0.f, 0.f, 0.f, 0.f};
             for (int j0 = 0; j0 < earlier; j0 += kDepthAhead) {
-                four_t piece[kDepthAhead];
-#pragma unroll
-                for (int k = 0; k < kDepthAhead; ++k) {  // (no load stands behind a condition; one past the last term
-                    const int j = min(j0 + k, earlier - 1);  // reads the last again and is dropped)
-                    piece[k] = load_four(past + static_cast<size_t>(j + (j >= own)) * layer_stride);
-                }
+                if (j0 > 0) ask(ahead, past, layer_stride, j0, earlier, own);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int k = 0; k < kDepthAhead; ++k) {
-                    const int j = j0 + k;
-                    if (j >= earlier) break;
+                    const int j = min(j0 + k, earlier - 1);
                     const float weight = weights[j + (j >= own)];
+                    four_t with;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[i] = fmaf(weight, piece[k][i], acc[i]);
+                    for (int i = 0; i < 4; ++i) with[i] = fmaf(weight, ahead[k][i], acc[i]);
+                    acc = j0 + k < earlier ? with : acc;
                 }
             }
             if (own < terms) {
@@ -142,27 +168,38 @@ depth_stream_vec4_kernel(const float* __restrict__ x, const T* __restrict__ bran
 CIE_API int cie_depth_stream(void* stream_handle, int dtype, const float* x, const void* branch_a, const void* branch_b,
                              float mult, float* history, long layer_stride, int newest, const float* weights,
                              int terms, float* stream, void* out1, float gain1, void* out2, float gain2, int rows,
-                             int hidden, float eps) {
+                             int hidden, float eps, const float* parts, int n_parts) {
     if (rows < 0 || hidden <= 0 || hidden * sizeof(float) > 64 * 1024 || !(eps > 0.f) || terms < 0) return CIE_BAD_ARGUMENT;
     if ((newest >= 0 || terms > 0) && (!history || layer_stride < static_cast<long>(rows) * hidden)) return CIE_BAD_ARGUMENT;
     if (terms > 0 && !weights) return CIE_BAD_ARGUMENT;
-    if (branch_b && !branch_a) return CIE_BAD_ARGUMENT;
+    if ((branch_b || n_parts) && !branch_a) return CIE_BAD_ARGUMENT;
+    if (n_parts < 0 || (n_parts && !parts)) return CIE_BAD_ARGUMENT;
     if (rows == 0) return CIE_OK;
     hipStream_t s = static_cast<hipStream_t>(stream_handle);
     const auto aligned = [](const void* p, size_t bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; };
     const auto wide = [&](size_t piece) {  // (a piece of the activation type: four numbers)
         return hidden % 4 == 0 && (!history || layer_stride % 4 == 0) && aligned(x, 16) && aligned(history, 16) &&
                aligned(stream, 16) && aligned(branch_a, piece) && aligned(branch_b, piece) && aligned(out1, piece) &&
-               aligned(out2, piece);
+               aligned(out2, piece) && aligned(parts, 16);
     };
-#define CIE_DEPTH(KERNEL, T)                                                                                          \
-    KERNEL<T><<<rows, threads, hidden * sizeof(float), s>>>(                                                           \
+#define CIE_DEPTH(KERNEL, T, ...)                                                                                     \
+    KERNEL<T __VA_OPT__(,) __VA_ARGS__><<<rows, threads, hidden * sizeof(float), s>>>(                                                           \
         x, static_cast<const T*>(branch_a), static_cast<const T*>(branch_b), mult, history, layer_stride, newest,      \
-        weights, terms, stream, static_cast<T*>(out1), gain1, static_cast<T*>(out2), gain2, hidden, eps)
+        weights, terms, stream, static_cast<T*>(out1), gain1, static_cast<T*>(out2), gain2, hidden, eps, parts, n_parts)
     if ((dtype == CIE_F32 && wide(16)) || (dtype == CIE_BF16 && wide(8))) {
         const int threads = min(1024, (hidden / 4 + kWave - 1) / kWave * kWave);
-        if (dtype == CIE_F32) CIE_DEPTH(depth_stream_vec4_kernel, float);
-        else CIE_DEPTH(depth_stream_vec4_kernel, bf16_t);
+#define CIE_DEPTH4(T)                                                                                                 \
+    if (n_parts && branch_b) CIE_DEPTH(depth_stream_vec4_kernel, T, 2, true);                                          \
+    else if (n_parts) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, true);                                                 \
+    else if (branch_b) CIE_DEPTH(depth_stream_vec4_kernel, T, 2, false);                                               \
+    else if (branch_a) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, false);                                               \
+    else CIE_DEPTH(depth_stream_vec4_kernel, T, 0, false)
+        if (dtype == CIE_F32) {
+            CIE_DEPTH4(float);
+        } else {
+            CIE_DEPTH4(bf16_t);
+        }
+#undef CIE_DEPTH4
         return cie_after_launch();
     }
     // few rows (a decode step): a row is one workgroup's, so its width is spread over as many threads as it has

@@ -1050,11 +1050,12 @@ def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor] = None,
 def depth_stream(x: torch.Tensor, branch_a: Optional[torch.Tensor] = None, branch_b: Optional[torch.Tensor] = None,
                  mult: float = 1.0, history: Optional[torch.Tensor] = None, newest: int = -1,
                  weights: Optional[torch.Tensor] = None, gains: tuple = (), out_dtype: torch.dtype = torch.float32,
-                 eps: float = 1e-6, want_stream: bool = True):
+                 eps: float = 1e-6, want_stream: bool = True, parts: Optional[torch.Tensor] = None):
     """One layer boundary of a stream whose layers add two parallel branches and whose next input is a weighted
     average of what the embedding and every layer so far left:
 
-    ``v = x + mult * (branch_a + branch_b)`` (float32; without branches ``v = x``); ``history[newest] = v``;
+    ``v = x + mult * (branch_a + branch_b)`` (float32; without branches ``v = x``; ``parts`` [P, T, H] float32, beside a
+    ``branch_a``: their sum, in order, is one more branch); ``history[newest] = v``;
     with ``weights`` (float32 [terms]) ``v = sum_j weights[j] * history[j]``; then for every gain ``g`` in
     ``gains`` (up to two) the rows ``v / sqrt(mean(v^2) + eps) * g`` in ``out_dtype``.
 
@@ -1071,6 +1072,10 @@ def depth_stream(x: torch.Tensor, branch_a: Optional[torch.Tensor] = None, branc
                 raise ValueError(f"{name} {tuple(branch.shape)} vs the stream {tuple(x.shape)}")
     if branch_b is not None and branch_a is None:
         raise ValueError("a second branch needs a first")
+    if parts is not None:
+        _gpu("parts", parts, torch.float32, 3)
+        if branch_a is None or tuple(parts.shape[1:]) != (rows, hidden):
+            raise ValueError(f"parts {tuple(parts.shape)} beside a first branch of {tuple(x.shape)}")
     terms, stride = 0, 0
     if history is not None:
         _gpu("history", history, torch.float32, 3)
@@ -1093,7 +1098,8 @@ def depth_stream(x: torch.Tensor, branch_a: Optional[torch.Tensor] = None, branc
     _run("cie_depth_stream", load_library().cie_depth_stream(
         _stream(), _i(_code(out_dtype)), _ptr(x), _ptr(branch_a), _ptr(branch_b), _f(mult), _ptr(history), stride,
         _i(newest), _ptr(weights), _i(terms), _ptr(stream), _ptr(outs[0] if outs else None), _f(g[0]),
-        _ptr(outs[1] if len(outs) > 1 else None), _f(g[1]), _i(rows), _i(hidden), _f(eps)))
+        _ptr(outs[1] if len(outs) > 1 else None), _f(g[1]), _i(rows), _i(hidden), _f(eps), _ptr(parts),
+        _i(0 if parts is None else parts.shape[0])))
     return (stream if stream is not None else (x if want_stream else None)), outs
 
 

@@ -289,10 +289,15 @@ class ParallelDepthBlock:
                                          want_stream=False)
             first, second = normed[0], normed[1] if len(normed) > 1 else None
         mixed = self.mixer.forward(first, batch, view, writes)
-        fed = self.feed_forward.forward(second) if self.has_feed_forward else None
+        fed = parts = None
+        if self.has_feed_forward:  # (its last product may come as parts of K: the boundary's kernel sums them)
+            takes = {"sums_parts": True} if getattr(self.feed_forward, "sums_parts", False) else {}
+            fed = self.feed_forward.forward(second, **takes)
+        if isinstance(fed, KParts):
+            fed, parts = None, fed.parts
         follower = self.next_block
         stream, normed = ops.depth_stream(
-            residual, mixed, fed, mult=self.mult, history=history, newest=self.depth + 1, weights=self.average,
+            residual, mixed, fed, parts=parts, mult=self.mult, history=history, newest=self.depth + 1, weights=self.average,
             gains=follower.gains() if follower is not None else (), out_dtype=self.dtype,
             eps=follower.norm1.eps if follower is not None else self.norm1.eps)
         if follower is None:

@@ -306,7 +306,7 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
     :class:`RowSumsq` comes back, or (a product whose K was cut into parts that
     each add their share) an :class:`Added`; otherwise the plain
     result comes back and the caller adds it (the next norm kernel does).
-    ``sums_parts`` (with ``into``): the caller's block takes :class:`KParts` too.
+    ``sums_parts``: the caller's block takes :class:`KParts` too.
     ``then_norm`` (with ``into``): the norm that follows, if it can be folded into
     this product and the next (``RMSNorm.folds_into_products``): the residual
     epilogue then also leaves that norm's output short of the rows' scale.
@@ -343,6 +343,13 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
         ops.gemm_shared_rows(weight, ops.EPI_ATOMIC, x, bias=bias, column_tiles=column_tiles, waves=waves,
                              k_parts=parts, add_into=into)
         return Added()
+    if (fusable and into is None and sums_parts and not silu and not wants_f32 and rows <= FUSED_PARTS_ROWS and -(-n // 16) < PART_BELOW_TILES
+            and k >= PART_MIN_K and x.data_ptr() % 16 == 0):
+        # a branch that whoever adds it sums itself (the down product of the parallel block, 8 rows, K 11,008: 17 us whole,
+        # 11 in 8 parts, and 0.4 more in the kernel that adds them)
+        column_tiles, waves, parts = plan_shared_parts(-(-n // 16), k)
+        return KParts(ops.gemm_shared_rows(weight, ops.EPI_PARTIAL, x, bias=bias, column_tiles=column_tiles, waves=waves,
+                                           k_parts=parts))
     if fusable and silu and n % 2 == 0 and bias is None and into is None and not wants_f32 and rows <= SHARED_SILU_ROWS:
         waves, own_unit = plan_shared_silu(-(-n // 32))
         if rows > FUSED_ROWS or own_unit:
@@ -381,7 +388,9 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
             if tiles is not None:
                 return ops.gemm_tiles(weight, ops.TILE_SILU, x, *tiles[:2])
         elif into is None and not silu:
-            tiles = plan_tiles(rows, n, k)
+            tiles = plan_tiles(rows, n, k, most_parts=TILE_PARTS[-1] if sums_parts else 1)
+            if tiles is not None and tiles[2] > 1:
+                return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, *tiles[:2], bias=bias, parts=tiles[2]))
             if tiles is not None:
                 return ops.gemm_tiles(weight, ops.TILE_BF16, x, *tiles[:2], bias=bias)
     if weight.dtype == torch.float32:

@@ -379,23 +379,24 @@ def test_layer_boundary_kernel_over_depths_and_widths(dtype, rows, hidden, terms
     g = torch.Generator().manual_seed(2)
     layers = max(terms, newest + 1)
     weights = torch.randn(terms, generator=g)
-    for shift in (0, 1):
+    for shift, n_parts in ((0, 0), (1, 0), (0, 1), (0, 9), (1, 3)):
         def rand(*shape, kind=torch.float32):  # (a tensor whose first number lies `shift` numbers off the allocation's start)
             n = torch.Size(shape).numel()
             return torch.randn(n + shift, generator=g).to(kind).cuda()[shift:].view(shape)
         history, x = rand(layers, rows, hidden), rand(rows, hidden)
         a, b = rand(rows, hidden, kind=dtype), rand(rows, hidden, kind=dtype)
+        parts = rand(n_parts, rows, hidden) if n_parts else None  # (a branch that comes as the parts of a product)
         kept = history.clone()
         stream, normed = ops.depth_stream(x, a, b, mult=0.7, history=history, newest=newest, weights=weights.cuda(),
-                                          gains=(1.5, 0.25), out_dtype=dtype, eps=1e-5)
-        new = x.double() + 0.7 * (a.double() + b.double())
+                                          gains=(1.5, 0.25), out_dtype=dtype, eps=1e-5, parts=parts)
+        new = x.double() + 0.7 * (a.double() + b.double() + (parts.double().sum(0) if n_parts else 0.0))
         rest = [j for j in range(layers) if j != newest]
         assert torch.allclose(history[newest].double(), new, atol=1e-5) and torch.equal(history[rest], kept[rest])
         parts = [weights[j].double().item() * (new if j == newest else kept[j].double()) for j in range(terms)]
         want, size = sum(parts), sum(p.abs() for p in parts)
         # each of the sum's `terms` roundings is at most half a unit in the last place of a partial sum below `size`; three
-        # more make the row just made
-        assert torch.all((stream.double() - want).abs() <= (terms + 3) * 2.0 ** -24 * (size + 2.0))
+        # more, and one a part, make the row just made, whose own partial sums stay below 64
+        assert torch.all((stream.double() - want).abs() <= 2.0 ** -24 * ((terms + 3) * (size + 2.0) + n_parts * 64.0))
         unit = want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-5)
         tol = 1e-5 if dtype == torch.float32 else 2e-2
         assert torch.allclose(normed[0].double(), unit * 1.5, atol=tol, rtol=tol)
