@@ -64,8 +64,8 @@ __global__ void depth_stream_kernel(const float* __restrict__ x, const T* __rest
 // The same with four neighbouring numbers a thread, for rows whose pieces of 16 bytes lie on 16-byte lines.  What bounds it
 // is the memory's rate over the earlier layers' rows (a boundary in the middle of 13 reads some 7 of them), and a thread
 // has to keep enough of them on their way: up to eight rows' pieces are asked for before the first is used.  Measured (a
-// boundary in the middle of 12 layers of 2,048, us, single numbers -> this): 1,999 rows 64 -> 32 (6.1 TB/s over the caches),
-// 8 rows 6.8 -> 5.1.
+// boundary in the middle of 12 layers of 2,048, us, single numbers -> this): 1,999 rows 64 -> 34 (5.8 TB/s),
+// 8 rows 6.8 -> 5.1, and 5.3 where the feed-forward comes in eight parts.
 typedef float four_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ four_t load_four(const float* p) { return *reinterpret_cast<const four_t*>(p); }
@@ -79,9 +79,9 @@ __device__ __forceinline__ void store_four(bf16_t* p, four_t v) {
     *reinterpret_cast<uint2*>(p) = uint2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
 }
 
-constexpr int kDepthAhead = 8;
-
-template <typename T, int kBranches, bool kParts>
+// (kAhead earlier rows' pieces at once: eight for few rows, where the chain of loads is the time; four for many, whose
+// other workgroups fill the wait: 1,999 rows take 34 us with four and 35 with eight)
+template <typename T, int kBranches, bool kParts, int kAhead>
 __global__ void __launch_bounds__(1024)
 depth_stream_vec4_kernel(const float* __restrict__ x, const T* __restrict__ branch_a, const T* __restrict__ branch_b,
                          float mult, float* __restrict__ history, long layer_stride, int newest,
@@ -97,12 +97,12 @@ depth_stream_vec4_kernel(const float* __restrict__ x, const T* __restrict__ bran
     for (int h = threadIdx.x * 4; h < hidden; h += blockDim.x * 4) {
         // (no load stands behind a condition, and none may move to its use: each would be waited for alone)
         const float* past = history + row + h;
-        four_t v = load_four(x + row + h), branch[kBranches + 1], ahead[kDepthAhead];
+        four_t v = load_four(x + row + h), branch[kBranches + 1], ahead[kAhead];
         if constexpr (kBranches > 0) branch[0] = load_four(branch_a + row + h);
         if constexpr (kBranches > 1) branch[1] = load_four(branch_b + row + h);
-        const auto ask = [&](four_t (&piece)[kDepthAhead], const float* from, size_t apart, int first, int count, int leave_out) {
+        const auto ask = [&](four_t (&piece)[kAhead], const float* from, size_t apart, int first, int count, int leave_out) {
 #pragma unroll
-            for (int k = 0; k < kDepthAhead; ++k) {  // (a piece past the last reads the last again and is dropped)
+            for (int k = 0; k < kAhead; ++k) {  // (a piece past the last reads the last again and is dropped)
                 const int j = min(first + k, count - 1);
                 piece[k] = load_four(from + static_cast<size_t>(j + (j >= leave_out)) * apart);
             }
@@ -113,12 +113,12 @@ depth_stream_vec4_kernel(const float* __restrict__ x, const T* __restrict__ bran
             four_t s = branch[0];
             if constexpr (kBranches > 1) s += branch[1];
             if constexpr (kParts) {
-                for (int p0 = 0; p0 < n_parts; p0 += kDepthAhead) {
-                    four_t piece[kDepthAhead];
+                for (int p0 = 0; p0 < n_parts; p0 += kAhead) {
+                    four_t piece[kAhead];
                     ask(piece, parts + row + h, static_cast<size_t>(gridDim.x) * hidden, p0, n_parts, n_parts);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int k = 0; k < kDepthAhead; ++k) {
+                    for (int k = 0; k < kAhead; ++k) {
                         const four_t with = s + piece[k];
                         s = p0 + k < n_parts ? with : s;
                     }
@@ -131,11 +131,11 @@ depth_stream_vec4_kernel(const float* __restrict__ x, const T* __restrict__ bran
         if (terms > 0) {
             // (the terms in the layers' order, the row just made last, from its register)
             four_t acc = {0.f, 0.f, 0.f, 0.f};
-            for (int j0 = 0; j0 < earlier; j0 += kDepthAhead) {
+            for (int j0 = 0; j0 < earlier; j0 += kAhead) {
                 if (j0 > 0) ask(ahead, past, layer_stride, j0, earlier, own);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int k = 0; k < kDepthAhead; ++k) {
+                for (int k = 0; k < kAhead; ++k) {
                     const int j = min(j0 + k, earlier - 1);
                     const float weight = weights[j + (j >= own)];
                     four_t with;
@@ -188,16 +188,20 @@ CIE_API int cie_depth_stream(void* stream_handle, int dtype, const float* x, con
         weights, terms, stream, static_cast<T*>(out1), gain1, static_cast<T*>(out2), gain2, hidden, eps, parts, n_parts)
     if ((dtype == CIE_F32 && wide(16)) || (dtype == CIE_BF16 && wide(8))) {
         const int threads = min(1024, (hidden / 4 + kWave - 1) / kWave * kWave);
-#define CIE_DEPTH4(T)                                                                                                 \
-    if (n_parts && branch_b) CIE_DEPTH(depth_stream_vec4_kernel, T, 2, true);                                          \
-    else if (n_parts) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, true);                                                 \
-    else if (branch_b) CIE_DEPTH(depth_stream_vec4_kernel, T, 2, false);                                               \
-    else if (branch_a) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, false);                                               \
-    else CIE_DEPTH(depth_stream_vec4_kernel, T, 0, false)
-        if (dtype == CIE_F32) {
-            CIE_DEPTH4(float);
+#define CIE_DEPTH4(T, AHEAD)                                                                                          \
+    if (n_parts && branch_b) CIE_DEPTH(depth_stream_vec4_kernel, T, 2, true, AHEAD);                                   \
+    else if (n_parts) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, true, AHEAD);                                          \
+    else if (branch_b) CIE_DEPTH(depth_stream_vec4_kernel, T, 2, false, AHEAD);                                        \
+    else if (branch_a) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, false, AHEAD);                                        \
+    else CIE_DEPTH(depth_stream_vec4_kernel, T, 0, false, AHEAD)
+        if (dtype == CIE_F32 && rows <= 128) {
+            CIE_DEPTH4(float, 8);
+        } else if (dtype == CIE_F32) {
+            CIE_DEPTH4(float, 4);
+        } else if (rows <= 128) {
+            CIE_DEPTH4(bf16_t, 8);
         } else {
-            CIE_DEPTH4(bf16_t);
+            CIE_DEPTH4(bf16_t, 4);
         }
 #undef CIE_DEPTH4
         return cie_after_launch();
