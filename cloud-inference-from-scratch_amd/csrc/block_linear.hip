@@ -166,7 +166,13 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
-template <typename TC>
+// Four slices' pieces are on their way before the first is used, none behind a condition: with a slice's loads waited for
+// one slice at a time (and a tile's behind the question whether it has rows) the kernel was a chain of K / 32 round trips
+// (8 rows, K 256: 7.6 -> 4.9 us; K 96: 6.2 -> 4.8).  Of many rows it costs nothing and gives nothing (1,999 rows, float32
+// results of 4,096 columns 42 us either way), nor does dealing out the rows over the XCDs instead of the columns.
+constexpr int kSlicesAhead = 4;
+
+template <typename TC, int TILES>
 __global__ void __launch_bounds__(256)
 block_linear_mfma_kernel(const bf16_t* __restrict__ A, long lda, long a_block, const bf16_t* __restrict__ W,
                          const bf16_t* __restrict__ bias, TC* __restrict__ C, long ldc, long c_block,
@@ -177,42 +183,54 @@ block_linear_mfma_kernel(const bf16_t* __restrict__ A, long lda, long a_block, c
     const int r = lane & 15;
     const int g = lane >> 4;
     const int n0 = (blockIdx.x * 4 + wave) * 16;
-    const int m0 = blockIdx.y * 64;
+    const int m0 = blockIdx.y * (16 * TILES);
     if (n0 >= N) return;  // (a wave leaves whole)
-    const int tiles = min(4, (M - m0 + 15) / 16);
     const bf16_t* w_row = W + (static_cast<size_t>(b) * N + min(n0 + r, N - 1)) * K;
     const bf16_t* a_base = A + static_cast<size_t>(b) * a_block;
-    const bf16_t* a_row[4];
+    const bf16_t* a_row[TILES];  // (a row past the last reads the last and is not stored)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) a_row[t] = a_base + static_cast<size_t>(min(m0 + t * 16 + r, M - 1)) * lda;
-    floatx4_t acc[4];
+    for (int t = 0; t < TILES; ++t) a_row[t] = a_base + static_cast<size_t>(min(m0 + t * 16 + r, M - 1)) * lda;
+    floatx4_t acc[TILES];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < TILES; ++t) acc[t] = floatx4_t{0.f, 0.f, 0.f, 0.f};
     const u32x4_t nothing = {0u, 0u, 0u, 0u};
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        // (a group of 8 past the end of K reads the last group again and counts as zeros: no load under a condition)
-        const int k = k0 + g * 8;
-        const int at = min(k, K - 8);
-        u32x4_t wt = *reinterpret_cast<const u32x4_t*>(w_row + at);
-        if (k >= K) wt = nothing;
+    for (int k0 = 0; k0 < K; k0 += 32 * kSlicesAhead) {
+        u32x4_t wt[kSlicesAhead], av[kSlicesAhead][TILES];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            if (t < tiles) {
-                u32x4_t av = *reinterpret_cast<const u32x4_t*>(a_row[t] + at);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
-                                                                 __builtin_bit_cast(bf16x8_t, wt), acc[t], 0, 0, 0);
+        for (int s = 0; s < kSlicesAhead; ++s) {
+            // (a group of 8 past the end of K reads the last group again and counts as zeros, on both sides)
+            const int at = min(k0 + 32 * s + g * 8, K - 8);
+            wt[s] = *reinterpret_cast<const u32x4_t*>(w_row + at);
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) av[s][t] = *reinterpret_cast<const u32x4_t*>(a_row[t] + at);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const bool tail = k0 + 32 * kSlicesAhead > K;
+#pragma unroll
+        for (int s = 0; s < kSlicesAhead; ++s) {
+            if (tail) {
+                const bool past = k0 + 32 * s + g * 8 >= K;
+                wt[s] = past ? nothing : wt[s];
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) av[s][t] = past ? nothing : av[s][t];
             }
         }
+#pragma unroll
+        for (int s = 0; s < kSlicesAhead; ++s)
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[s][t]),
+                                                                 __builtin_bit_cast(bf16x8_t, wt[s]), acc[t], 0, 0, 0);
     }
     const int n = n0 + r;
     if (n >= N) return;
     const float add = bias ? to_float(bias[static_cast<size_t>(b) * N + n]) : 0.f;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < TILES; ++t) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int m = m0 + t * 16 + g * 4 + i;
-            if (t < tiles && m < M) {
+            if (m < M) {
                 float v = acc[t][i] + add;
                 if (gate) {
                     const float gv = to_float(gate[static_cast<size_t>(m) * ldg + static_cast<size_t>(b) * g_block + n]);
@@ -246,15 +264,17 @@ CIE_API int cie_block_linear(void* stream, int dtype, int out_f32, const void* A
         return CIE_BAD_ARGUMENT;
     }
     if (cores) {
-        dim3 tiles((N + 63) / 64, grid_y, B);
-        if (out_f32)
-            block_linear_mfma_kernel<float><<<tiles, 256, 0, s>>>(
-                static_cast<const bf16_t*>(A), lda, a_block, static_cast<const bf16_t*>(W), static_cast<const bf16_t*>(bias),
-                static_cast<float*>(C), ldc, c_block, static_cast<const bf16_t*>(gate), ldg, g_block, M, N, K);
-        else
-            block_linear_mfma_kernel<bf16_t><<<tiles, 256, 0, s>>>(
-                static_cast<const bf16_t*>(A), lda, a_block, static_cast<const bf16_t*>(W), static_cast<const bf16_t*>(bias),
-                static_cast<bf16_t*>(C), ldc, c_block, static_cast<const bf16_t*>(gate), ldg, g_block, M, N, K);
+        const int rows = M <= 16 ? 16 : 64;
+        dim3 tiles((N + 63) / 64, (M + rows - 1) / rows, B);
+#define CIE_BLOCK(TC, TILES)                                                                                           \
+    block_linear_mfma_kernel<TC, TILES><<<tiles, 256, 0, s>>>(                                                          \
+        static_cast<const bf16_t*>(A), lda, a_block, static_cast<const bf16_t*>(W), static_cast<const bf16_t*>(bias),    \
+        static_cast<TC*>(C), ldc, c_block, static_cast<const bf16_t*>(gate), ldg, g_block, M, N, K)
+        if (out_f32 && rows == 16) CIE_BLOCK(float, 1);
+        else if (out_f32) CIE_BLOCK(float, 4);
+        else if (rows == 16) CIE_BLOCK(bf16_t, 1);
+        else CIE_BLOCK(bf16_t, 4);
+#undef CIE_BLOCK
         return cie_after_launch();
     }
     if (dtype == CIE_F32)

@@ -337,6 +337,34 @@ def test_block_diagonal_product_in_all_its_forms(rows, dtype):
         assert torch.equal(alone, out[:1])
 
 
+@pytest.mark.parametrize("rows", [5, 16, 17, 64, 65, 520, 600])
+@pytest.mark.parametrize("blocks,n,k", [(1, 16, 8), (3, 72, 40), (2, 130, 128), (2, 64, 136), (5, 24, 256), (1, 200, 264)])
+def test_block_diagonal_product_on_the_matrix_cores(rows, blocks, n, k):
+    """Operands that take them: one tile of 16 rows and tiles of 64, fewer and more blocks of rows than XCDs; one group of
+    8 k, K inside a round of four slices, one round, one group more, two rounds and one group more."""
+    from cie_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(rows + k)
+    a_block = k + 16
+    a = torch.randn(rows, 8 + blocks * a_block, generator=g).bfloat16().cuda()
+    w = (torch.randn(blocks, n, k, generator=g) / k ** 0.5).bfloat16().cuda()
+    bias = torch.randn(blocks, n, generator=g).bfloat16().cuda()
+    gate = torch.randn(rows, blocks * n, generator=g).bfloat16().cuda()
+    picked = torch.stack([a[:, 8 + b * a_block: 8 + b * a_block + k] for b in range(blocks)], 1).cpu().double()
+    plain = torch.stack([picked[:, b] @ w[b].cpu().double().t() for b in range(blocks)], 1)
+    size = torch.stack([picked[:, b].abs() @ w[b].cpu().double().abs().t() for b in range(blocks)], 1)
+    out = ops.block_linear(a, w, a_block=a_block, a_offset=8, out_dtype=torch.float32).cpu().double().reshape(rows, blocks, n)
+    # exact products of bfloat16 numbers, k float32 sums: each rounds by at most 2^-24 of what it has summed
+    assert torch.all((out - plain).abs() <= k * 2.0 ** -24 * size)
+    wide = torch.full((rows, 8 + blocks * (n + 8)), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.block_linear(a, w, bias, a_block=a_block, a_offset=8, out=wide, out_offset=8, c_block=n + 8, gate=gate)
+    gated = (plain + bias.cpu().double()) * torch.sigmoid(gate.cpu().double().reshape(rows, blocks, n))
+    got = wide[:, 8:].cpu().double().reshape(rows, blocks, n + 8)
+    assert torch.all((got[:, :, :n] - gated).abs() <= 2.0 ** -8 * gated.abs() + 1e-5 * (size + 1))  # (rounded once)
+    assert bool((wide[:, :8] == 7).all()) and bool((got[:, :, n:] == 7).all())
+
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_layer_boundary_kernel(dtype):
     from cie_amd.kernels import ops
