@@ -253,16 +253,34 @@ __device__ __forceinline__ void decay_table(float* pw, float fade) {
     }
 }
 
+// What the block kernels read from memory they ask for several loads at a time, in straight-line code that ends in a
+// barrier to the compiler's scheduler: in loops of one load and its use a workgroup of four waves, two to a compute unit,
+// waited for some thirty loads one after another (1,999 tokens of 8 heads of 128 x 256, us: block sums 51 -> 39, reads
+// 28 -> 19).
+constexpr int kStageAhead = 4;
+constexpr int kStageValues = 8;
+
 // a block's queries (side 0) or keys (side 1) into LDS rows of `stride` floats; rows past the block's last token are zero
 __device__ __forceinline__ void stage_rows(float* dst, int stride, const float* __restrict__ turned, int first_token,
                                            int cn, int heads, int head, int padded, int side) {
-    const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
-    for (int t = wave; t < kBlockTokens; t += 4) {
-        const float* src = turned + ((static_cast<size_t>(first_token + min(t, cn - 1)) * heads + head) * 2 + side) * padded;
-        for (int piece = lane; piece < padded / 4; piece += kWave) {
-            const piece_t value = *reinterpret_cast<const piece_t*>(src + 4 * piece);
-            *reinterpret_cast<piece_t*>(dst + t * stride + 4 * piece) = t < cn ? value : piece_t{0.f, 0.f, 0.f, 0.f};
+    const int row_pieces = padded / 4, pieces = kBlockTokens * row_pieces;
+    for (int base = 0; base < pieces; base += kStageAhead * 256) {
+        piece_t value[kStageAhead];
+#pragma unroll
+        for (int i = 0; i < kStageAhead; ++i) {  // (what lies past the end reads the last piece again)
+            const int idx = min(base + i * 256 + static_cast<int>(threadIdx.x), pieces - 1);
+            const int t = idx / row_pieces;
+            value[i] = *reinterpret_cast<const piece_t*>(
+                turned + ((static_cast<size_t>(first_token + min(t, cn - 1)) * heads + head) * 2 + side) * padded +
+                4 * (idx - t * row_pieces));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kStageAhead; ++i) {  // (... and writes it again: a store under a condition takes its load along)
+            const int idx = min(base + i * 256 + static_cast<int>(threadIdx.x), pieces - 1);
+            const int t = idx / row_pieces;
+            *reinterpret_cast<piece_t*>(dst + t * stride + 4 * (idx - t * row_pieces)) =
+                t < cn ? value[i] : piece_t{0.f, 0.f, 0.f, 0.f};
         }
     }
 }
@@ -299,11 +317,22 @@ retention_block_sums_kernel(const T* __restrict__ proj, long ldp, int v_off, con
     decay_table(pw, decay[head]);
     stage_rows(q_s, stride, turned, first + c0, cn, heads, head, padded, 0);
     stage_rows(k_s, stride, turned, first + c0, cn, heads, head, padded, 1);
-    for (int t = wave; t < kBlockTokens; t += 4) {
-        const T* src = proj + static_cast<size_t>(first + c0 + min(t, cn - 1)) * ldp + v_off + head * vdim;
-        for (int c = lane; c < cols; c += kWave) {
-            const float value = activated(to_float(src[min(panel0 + c, vdim - 1)]), act);
-            v_s[t * vstride + c] = (t < cn && panel0 + c < vdim) ? value : 0.f;
+    for (int base = 0; base < kBlockTokens * cols; base += kStageValues * 256) {
+        T value[kStageValues];
+#pragma unroll
+        for (int i = 0; i < kStageValues; ++i) {
+            const int idx = min(base + i * 256 + static_cast<int>(threadIdx.x), kBlockTokens * cols - 1);
+            const int t = idx / cols;
+            value[i] = proj[static_cast<size_t>(first + c0 + min(t, cn - 1)) * ldp + v_off + head * vdim +
+                            min(panel0 + idx - t * cols, vdim - 1)];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kStageValues; ++i) {
+            const int idx = min(base + i * 256 + static_cast<int>(threadIdx.x), kBlockTokens * cols - 1);
+            const int t = idx / cols, c = idx - t * cols;
+            const float number = activated(to_float(value[i]), act);
+            v_s[t * vstride + c] = (t < cn && panel0 + c < vdim) ? number : 0.f;
         }
     }
     __syncthreads();
@@ -436,20 +465,26 @@ retention_block_reads_kernel(const float* __restrict__ turned, const float* __re
     for (int ct = wave; ct < col_tiles; ct += 4) {
         acc4_t o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
         const float* rows = before + static_cast<size_t>(4 * g) * vdim16 + 16 * ct + l16;
-#pragma unroll 2
-        for (int m = 0; m < tiles; ++m) {
-            const float4 a0 = *reinterpret_cast<const float4*>(q_s + l16 * stride + 16 * m + 4 * g);
-            const float4 a1 = *reinterpret_cast<const float4*>(q_s + (16 + l16) * stride + 16 * m + 4 * g);
-            const float* s = rows + static_cast<size_t>(16 * m) * vdim16;
-            const float b0 = s[0], b1 = s[vdim16], b2 = s[2 * vdim16], b3 = s[3 * vdim16];
-            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0.x, b0, o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1.x, b0, o1, 0, 0, 0);
-            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0.y, b1, o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1.y, b1, o1, 0, 0, 0);
-            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0.z, b2, o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1.z, b2, o1, 0, 0, 0);
-            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0.w, b3, o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1.w, b3, o1, 0, 0, 0);
+        for (int m0 = 0; m0 < tiles; m0 += kStageAhead) {
+            float mem[kStageAhead][4];
+#pragma unroll
+            for (int i = 0; i < kStageAhead; ++i)  // (a tile past the last reads the last again and is left out)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) mem[i][j] = rows[static_cast<size_t>(16 * min(m0 + i, tiles - 1) + j) * vdim16];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < kStageAhead; ++i) {
+                const bool there = m0 + i < tiles;
+                const int m = min(m0 + i, tiles - 1);
+                const piece_t a0 = *reinterpret_cast<const piece_t*>(q_s + l16 * stride + 16 * m + 4 * g);
+                const piece_t a1 = *reinterpret_cast<const piece_t*>(q_s + (16 + l16) * stride + 16 * m + 4 * g);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float b = there ? mem[i][j] : 0.f;
+                    o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(there ? a0[j] : 0.f, b, o0, 0, 0, 0);
+                    o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(there ? a1[j] : 0.f, b, o1, 0, 0, 0);
+                }
+            }
         }
         const int col = panel0 + 16 * ct + l16;
         if (col < vdim) {
@@ -496,6 +531,64 @@ retention_norm_kernel(float* __restrict__ raw, long plane, int parts, const T* _
         float y = o[c] * inv;
         if (weight) y *= weight[first + c];
         dst[c] = from_float<T>(y * open);
+    }
+}
+
+// The same for runs of up to four columns a lane: the parts' columns and the gate's are asked for together and stay in
+// registers (1,999 tokens of 8 heads of 256, two parts: 12.1 us, 15.8 in the kernel above, which stores the sums and reads
+// them again).
+constexpr int kNormColumns = 4;
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+retention_norm_narrow_kernel(const float* __restrict__ raw, long plane, int parts, const T* __restrict__ proj, long ldp,
+                             int g_off, T* __restrict__ out, int tokens, int heads, int vdim, float eps, int span,
+                             const float* __restrict__ weight, int gate_act) {
+    const int runs = heads / span;
+    const int item = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    if (item >= tokens * runs) return;  // (whole waves leave together)
+    const int lane = threadIdx.x % kWave;
+    const int token = item / runs;
+    const int first = (item - token * runs) * span * vdim;  // the run's first column
+    const int width = span * vdim;
+    const float* o = raw + static_cast<size_t>(token) * heads * vdim + first;
+    const T* gate = proj + static_cast<size_t>(token) * ldp + g_off + first;
+    T g_in[kNormColumns];
+    float v[kNormColumns] = {}, gain[kNormColumns];
+#pragma unroll
+    for (int i = 0; i < kNormColumns; ++i) {  // (a column past the run reads its last and counts as zero)
+        const int c = min(lane + i * kWave, width - 1);
+        g_in[i] = gate[c];
+        gain[i] = weight ? weight[first + c] : 1.f;
+    }
+    for (int p0 = 0; p0 < parts; p0 += 4) {
+        float piece[4][kNormColumns];
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+            for (int i = 0; i < kNormColumns; ++i)
+                piece[p][i] = o[static_cast<size_t>(min(p0 + p, parts - 1)) * plane + min(lane + i * kWave, width - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+            for (int i = 0; i < kNormColumns; ++i) {  // (the parts in their order)
+                const float with = p0 + p == 0 ? piece[p][i] : v[i] + piece[p][i];
+                v[i] = p0 + p < parts && lane + i * kWave < width ? with : v[i];
+            }
+    }
+    float sum_sq = 0.f;
+#pragma unroll
+    for (int i = 0; i < kNormColumns; ++i) sum_sq += v[i] * v[i];
+    const float inv = 1.0f / sqrtf(wave_sum(sum_sq) / static_cast<float>(width) + eps);
+    T* dst = out + static_cast<size_t>(token) * heads * vdim + first;
+#pragma unroll
+    for (int i = 0; i < kNormColumns; ++i) {
+        const float g = to_float(g_in[i]);
+        const float open = gate_act == 1 ? sigmoidf(g) : g * sigmoidf(g);
+        float y = v[i] * inv;
+        if (weight) y *= gain[i];
+        if (lane + i * kWave < width) dst[lane + i * kWave] = from_float<T>(y * open);
     }
 }
 
@@ -952,14 +1045,17 @@ CIE_API int cie_retention(void* stream, int dtype, const void* proj, long ldp, i
         return cie_after_launch();
     }
     const int norm_blocks = (items + 3) / 4;
-    if (dtype == CIE_F32)
-        retention_norm_kernel<float><<<norm_blocks, 256, 0, s>>>(raw, plane, parts, static_cast<const float*>(proj), ldp, g_off,
-                                                           static_cast<float*>(out), tokens, heads, vdim, eps, norm_span,
-                                                           norm_weight, gate_act);
-    else
-        retention_norm_kernel<bf16_t><<<norm_blocks, 256, 0, s>>>(raw, plane, parts, static_cast<const bf16_t*>(proj), ldp, g_off,
-                                                            static_cast<bf16_t*>(out), tokens, heads, vdim, eps, norm_span,
-                                                            norm_weight, gate_act);
+#define CIE_NORM(KERNEL, T)                                                                                           \
+    KERNEL<T><<<norm_blocks, 256, 0, s>>>(raw, plane, parts, static_cast<const T*>(proj), ldp, g_off, static_cast<T*>(out), \
+                                          tokens, heads, vdim, eps, norm_span, norm_weight, gate_act)
+    if (width <= kNormColumns * kWave) {
+        if (dtype == CIE_F32) CIE_NORM(retention_norm_narrow_kernel, float);
+        else CIE_NORM(retention_norm_narrow_kernel, bf16_t);
+    } else {  // (a run that not even the wide kernel's LDS holds)
+        if (dtype == CIE_F32) CIE_NORM(retention_norm_kernel, float);
+        else CIE_NORM(retention_norm_kernel, bf16_t);
+    }
+#undef CIE_NORM
     return cie_after_launch();
 }
 

@@ -478,3 +478,48 @@ def test_gated_recurrence_and_its_convolution(dtype, lengths, channels, taps, se
         # (S fades by 1 - a^2 against what it takes in: its float32 roundings do not add up over the tokens)
         assert torch.allclose(out[at: at + n].double().cpu(), want, **tol)
         assert torch.allclose(state[slot].double().cpu(), S, atol=3e-5, rtol=3e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lengths,heads,dim,vdim,span", [
+    ((33,), 2, 40, 24, 1), ((70, 5, 129), 1, 128, 128, 1), ((64, 31), 2, 160, 72, 2), ((200,), 3, 16, 256, 1),
+    ((1, 1, 1), 2, 128, 128, 1), ((1, 2), 4, 16, 16, 4), ((40,), 2, 24, 136, 2)])
+def test_retention_over_the_edges_of_its_pieces(dtype, lengths, heads, dim, vdim, span):
+    """Blocks that end inside their 32 tokens, heads of fewer and of more pieces than one round of loads, columns in one
+    panel and two, norms over one lane's column, over four and over more; both walks; against 64 bits token by token."""
+    from cie_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(4)
+    tokens, slots = sum(lengths), list(range(len(lengths)))[::-1]
+    width = heads * (2 * dim + 2 * vdim)
+    proj = torch.randn(tokens, width + 8, generator=g).to(dtype).cuda()
+    offsets = (0, heads * dim, 2 * heads * dim, 2 * heads * dim + heads * vdim)
+    decay = torch.linspace(0.9, 0.99, heads).cuda()
+    state = torch.randn(len(lengths), heads, dim, vdim, generator=g).cuda()
+    old = state.cpu().double()
+    weight = torch.rand(heads * vdim, generator=g).cuda() + 0.5
+    starts = [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    meta = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+    positions = meta([t for n in lengths for t in range(n)])
+    out = ops.retention(proj, offsets, None, None, 0, decay, state, meta(slots), positions, meta(starts), len(lengths),
+                        heads, dim, vdim, 1e-6, dim ** -0.5, max(lengths), norm_span=span, norm_weight=weight, gate="sigmoid")
+    p = proj.cpu().double()
+    q, k = (p[:, o: o + heads * dim].view(tokens, heads, dim) for o in offsets[:2])
+    v, gate = (p[:, o: o + heads * vdim].view(tokens, heads, vdim) for o in offsets[2:])
+    f = decay.cpu().double()[:, None, None]
+    for i, n in enumerate(lengths):
+        S, size = old[slots[i]].clone(), old[slots[i]].abs()
+        for t in range(starts[i], starts[i] + n):
+            add = (k[t] * dim ** -0.5)[:, :, None] * v[t][:, None, :]
+            S, size = f * S + add, f * size + add.abs()
+            o, o_size = (S * q[t][:, :, None]).sum(1), (size * q[t].abs()[:, :, None]).sum(1)
+            rms = torch.sqrt((o.view(heads // span, -1) ** 2).mean(-1) + 1e-6).repeat_interleave(span)[:, None]
+            factor = weight.cpu().double().view(heads, vdim) * torch.sigmoid(gate[t]) / rms
+            want = o * factor
+            # float32 sums of n + dim terms and the powers of the decay in front of them, then the norm's own few roundings
+            # (its sum of squares carries the error of all its columns)
+            bound = (2 * n + dim + 16) * 2.0 ** -24 * (o_size + o_size.max() * want.abs() / factor.abs().clamp_min(1e-30) / rms) * factor.abs()
+            if dtype == torch.bfloat16:
+                bound = bound + 2.0 ** -8 * want.abs()
+            assert torch.all((out[t].cpu().double().view(heads, vdim) - want).abs() <= bound + 1e-6)
+        assert torch.all((state[slots[i]].cpu().double() - S).abs() <= (2 * n + 16) * 2.0 ** -24 * (size + 1))
