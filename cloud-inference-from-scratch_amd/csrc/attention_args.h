@@ -57,6 +57,5 @@ __host__ __device__ inline bool all_in_first_share(int first_begin, int hi, int 
 int launch_prompt_form(hipStream_t stream, const AttentionArgs& a, int head_dim, int waves);
 
 constexpr int kPromptWaves = 8;       // waves of a workgroup in that form
-constexpr int kPromptTileRows = 128;  // (token, head) rows of its tiles
 
 }  // namespace cie_attention

@@ -715,15 +715,29 @@ attention_merge_kernel(AttentionArgs a, int head_dim, int rows_per_tile) {
 // The same merge for tiles of many rows and few shares (prompt portions whose keys are cut): a workgroup
 // takes 16 rows of a (tile, kv head), a thread four head dimensions at a time of one row; every thread
 // of a row makes the shares' weights for itself from the few statistics.  (With one workgroup for each row,
-// as above, a step of 2,048 tokens would start 32,768 workgroups.)
+// as above, a step of 2,048 tokens would start 32,768 workgroups.)  What bounds it is the chain of loads: the statistics
+// and the first sums of all shares are asked for together, before anything about the tile is known (a share past the
+// last reads the last again, a row past the tile's own what its place holds, and a select or the return drops both).
+// 256 rows of 16 heads in four shares, tiles of 32 rows: 9.4 us a row a workgroup, 3.9 here.
 constexpr int kMergeFewShares = 16;
 
+template <int SHARES>
 __global__ void __launch_bounds__(256)
 attention_merge_rows_kernel(AttentionArgs a, int head_dim, int rows_per_tile) {
     const int tile = blockIdx.x;
     const int kv_head = blockIdx.y;
     const int row = blockIdx.z * 16 + threadIdx.x / 16;
     const int lane16 = threadIdx.x % 16;
+    const size_t unit0 = (static_cast<size_t>(tile) * a.kv_heads + kv_head) * a.n_splits;
+    const auto place = [&](int s) { return (unit0 + min(s, a.n_splits - 1)) * rows_per_tile + row; };
+    float2 ml[SHARES];
+    floatx4 sums[SHARES];
+    const int d0 = min(lane16 * 4, head_dim - 4);
+#pragma unroll
+    for (int s = 0; s < SHARES; ++s) ml[s] = *reinterpret_cast<const float2*>(a.part_ml + place(s) * 2);
+#pragma unroll
+    for (int s = 0; s < SHARES; ++s) sums[s] = *reinterpret_cast<const floatx4*>(a.part_o + place(s) * head_dim + d0);
+    __builtin_amdgcn_sched_barrier(0);
     const int group = a.q_heads / a.kv_heads;
     const int seq = a.tile_seq ? a.tile_seq[tile] : tile;
     const int q0 = a.tile_seq ? a.tile_q0[tile] : 0;
@@ -740,20 +754,20 @@ attention_merge_rows_kernel(AttentionArgs a, int head_dim, int rows_per_tile) {
         }
         if (all_in_first_share(lo & ~(kKeysPerBlock - 1), hi, per_split)) return;
     }
-    const size_t unit0 = (static_cast<size_t>(tile) * a.kv_heads + kv_head) * a.n_splits;
-    float weight[kMergeFewShares];
+    float weight[SHARES];
     float m_all = -INFINITY;
 #pragma unroll
-    for (int s = 0; s < kMergeFewShares; ++s) {
-        weight[s] = (s < a.n_splits) ? a.part_ml[((unit0 + s) * rows_per_tile + row) * 2] : -INFINITY;
+    for (int s = 0; s < SHARES; ++s) {
+        weight[s] = s < a.n_splits ? ml[s].x : -INFINITY;
         m_all = fmaxf(m_all, weight[s]);
     }
     float den = 0.f;
 #pragma unroll
-    for (int s = 0; s < kMergeFewShares; ++s) {
+    for (int s = 0; s < SHARES; ++s) {
         const float w = (weight[s] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(weight[s] - m_all);  // maxima are kept in base 2
         weight[s] = w;
-        if (s < a.n_splits) den += a.part_ml[((unit0 + s) * rows_per_tile + row) * 2 + 1] * w;
+        const float with = den + ml[s].y * w;
+        den = s < a.n_splits ? with : den;
     }
     const float inv = 1.0f / den;
     const int tok = row / group;
@@ -761,11 +775,17 @@ attention_merge_rows_kernel(AttentionArgs a, int head_dim, int rows_per_tile) {
     bf16_t* dst = a.out + static_cast<size_t>(a.q_start_loc[seq] + q0 + tok) * a.q_heads * head_dim +
                   static_cast<size_t>(kv_head * group + head) * head_dim;
     for (int d = lane16 * 4; d < head_dim; d += 64) {
+        if (d >= 64) {
+#pragma unroll
+            for (int s = 0; s < SHARES; ++s) sums[s] = *reinterpret_cast<const floatx4*>(a.part_o + place(s) * head_dim + d);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         floatx4 num = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int s = 0; s < kMergeFewShares; ++s)
-            if (s < a.n_splits && weight[s] != 0.f)  // (a share without keys wrote no sums)
-                num += *reinterpret_cast<const floatx4*>(a.part_o + ((unit0 + s) * rows_per_tile + row) * head_dim + d) * weight[s];
+        for (int s = 0; s < SHARES; ++s) {
+            const floatx4 with = num + sums[s] * weight[s];
+            num = weight[s] != 0.f ? with : num;  // (a share without keys wrote no sums)
+        }
         uint2 packed;
         packed.x = from_float<bf16_t>(num[0] * inv).bits | (static_cast<uint32_t>(from_float<bf16_t>(num[1] * inv).bits) << 16);
         packed.y = from_float<bf16_t>(num[2] * inv).bits | (static_cast<uint32_t>(from_float<bf16_t>(num[3] * inv).bits) << 16);
@@ -776,8 +796,13 @@ attention_merge_rows_kernel(AttentionArgs a, int head_dim, int rows_per_tile) {
 // Which of the two merges a step's shape takes.
 int launch_merge(hipStream_t s, const AttentionArgs& a, int n_tiles, int head_dim, int rows_per_tile) {
     const int rows = a.tokens_per_tile * (a.q_heads / a.kv_heads);
-    if (rows_per_tile >= kPromptTileRows && a.n_splits <= kMergeFewShares)  // (with fewer rows a tile the first is the faster one)
-        attention_merge_rows_kernel<<<dim3(n_tiles, a.kv_heads, (rows + 15) / 16), 256, 0, s>>>(a, head_dim, rows_per_tile);
+    const dim3 by_rows(n_tiles, a.kv_heads, (rows + 15) / 16);
+    if (rows_per_tile > 16 && a.n_splits <= 4)
+        attention_merge_rows_kernel<4><<<by_rows, 256, 0, s>>>(a, head_dim, rows_per_tile);
+    else if (rows_per_tile > 16 && a.n_splits <= 8)
+        attention_merge_rows_kernel<8><<<by_rows, 256, 0, s>>>(a, head_dim, rows_per_tile);
+    else if (rows_per_tile > 16 && a.n_splits <= kMergeFewShares)
+        attention_merge_rows_kernel<kMergeFewShares><<<by_rows, 256, 0, s>>>(a, head_dim, rows_per_tile);
     else
         attention_merge_kernel<<<dim3(n_tiles, a.kv_heads, rows), kMergeThreads, 0, s>>>(a, head_dim, rows_per_tile);
     return cie_after_launch();
