@@ -1,7 +1,8 @@
 // Paged grouped-query attention, generic form: any head size that is a multiple
 // of 8 up to 256, any group size, float32 or bfloat16 storage, optional window.
-// It is the whole of the float32 path's attention and the fallback of the
-// bfloat16 path for shapes the matrix-core kernels refuse.
+// It is the fallback of both paths for shapes that the matrix-core kernels
+// refuse (float32: heads of other than 32, 64, 96 or 128 dimensions, groups of
+// more than 64 heads, pages that are no power of two or smaller than 4).
 //
 // One workgroup (4 waves) per (query token, query head).  A token at position p
 // sees keys [lo, p] with lo = max(0, p + 1 - window) (window <= 0: all keys).
