@@ -363,6 +363,7 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
 # less than the second kernel that joins blocks), and the bytes that the blocks' workspace may take (sequences beyond
 # that go in further launches, which share it)
 F32_WHOLE_KEYS = 128
+F32_CUT_TILES = 0.6  # tiles a compute unit up to which prompts' tiles may be cut into blocks
 F32_WORKSPACE_BYTES = 64 << 20
 
 
@@ -386,7 +387,12 @@ def attend_f32(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int
             blocks = min(blocks, -(-(window + tokens) // ops.F32_BLOCK_KEYS) + 1)
         rows = tokens * group
         per = num_kv_heads * blocks * rows
-        if whole or (tokens > 1 and (2 * n_tiles * num_kv_heads > cus
+        # Whole tiles take some 8.3 us a block of the longest tile, tiles in blocks 0.055 us a block of all of them and 8 more
+        # (the parts' way through memory), over 256 units (us, whole against in blocks, 16 heads of 128 on 2: a prompt of
+        # 130 tokens 30, 24; 256 tokens 39, 31; 517 tokens 79, 66; 1,024 tokens 138, 160; 8 prompts of 64 tokens 16, 36; 8 of
+        # 128 25, 68; 14 heads of 64 on 2: 600 tokens 51, 40)
+        units = F32_CUT_TILES * cus - n_tiles * num_kv_heads
+        if whole or (tokens > 1 and (blocks * units <= F32_CUT_TILES * cus
                                      or n_tiles * per * (head_dim + 2) * 4 > F32_WORKSPACE_BYTES)):
             ops.paged_attention_f32(qkv, qkv.stride(0), view.k_pool, view.v_pool, view.block_table, tile_seq, tile_q0,
                                     n_tiles, *common, tokens)
