@@ -370,7 +370,7 @@ F32_WORKSPACE_BYTES = 64 << 20
 def attend_f32(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, head_dim: int,
                window: Optional[int], scale: float) -> torch.Tensor:
     """Attention in true float32 on the matrix cores: single tokens in blocks of keys (a wave each, joined behind),
-    prompt portions a workgroup per 64 rows, or in blocks too where such tiles would leave half of the units idle."""
+    prompt portions a workgroup per 64 rows, or in blocks too where there are few such tiles of many blocks."""
     out = torch.empty((batch.tokens, num_heads * head_dim), dtype=qkv.dtype, device=qkv.device)
     group = num_heads // num_kv_heads
     per_tile = ops.F32_TILE_ROWS // group
