@@ -14,7 +14,8 @@ Interfaces (``x`` is ``[tokens, hidden]`` in the engine's activation dtype,
                 adds ``branch`` into ``residual`` (in place, float32) and returns
                 the normalised rows.  A norm that sets ``takes_row_sumsq`` is
                 also handed the ``RowSumsq`` / ``Added`` forms of a branch
-                (``parts/linear.py``); any other gets a tensor or ``None``.
+                (``parts/linear.py``), and one that sets ``takes_parts`` the
+                ``KParts`` form; any other gets a tensor or ``None``.
 ``Position``    ``tables(device) -> (cos, sin)`` or whatever its mixer asks of it.
 ``Mixer``       ``cache_need() -> PagedKV | FixedState | None`` and
                 ``forward(x, batch, view, writes) -> y``; ``view`` is the cache
@@ -28,7 +29,8 @@ Interfaces (``x`` is ``[tokens, hidden]`` in the engine's activation dtype,
                 embedding's rows; ``plus`` (float32) still joins the new stream.
 ``Block``       ``forward(residual, pending, batch, view, writes) -> (residual, pending)``
                 ``pending`` is a branch output not yet added to the residual, so
-                that the add fuses with the next norm.
+                that the add fuses with the next norm (``normalise`` in
+                ``parts/block.py`` turns its forms into what a norm takes).
 """
 
 from __future__ import annotations
@@ -71,6 +73,18 @@ def build_part(role: str, spec: PartSpec) -> Any:
     return registry[spec.kind](**spec.as_dict())
 
 
+def declares(part: Any, flag: str) -> bool:
+    """Whether ``flag`` holds for the ``forward`` that ``part`` runs: what its class says, unless the class brings a
+    ``forward`` of its own and says nothing (a variant written against the plain interface takes no argument and no form
+    of a branch that only its base class knows)."""
+    for cls in type(part).__mro__:
+        if flag in vars(cls):
+            return bool(vars(cls)[flag])
+        if "forward" in vars(cls):
+            return False
+    return False
+
+
 class Part:
     """Default behaviour of a part without tensors.
 
@@ -83,6 +97,9 @@ class Part:
     # ``adds_to_residual``: ``forward`` takes ``residual=`` and may add its output there itself
     # (returning a ``RowSumsq`` or an ``Added``).
     adds_to_residual = False
+    # ``sums_parts``: ``forward`` takes ``sums_parts=``, and where that is true its output may come back as ``KParts``: the
+    # float32 parts of its last product, which whoever adds the branch sums.  (Asked with ``declares``.)
+    sums_parts = False
     # ``joins_products``: the part is one product in, something between, one product out.  Two such parts that read the
     # same rows and whose results are added may share both products: ``product_in()`` and ``product_out()`` give the
     # weights, and the part's own step between them takes the first product's rows and writes into a given matrix.

@@ -31,7 +31,7 @@ import torch
 from ..config.specs import LayerSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
-from .base import build_part, register_part
+from .base import build_part, declares, register_part
 from .linear import Added, KParts, RawRows, RowSumsq, StreamRows, WeightedPair, linear, linear_beside
 
 
@@ -84,7 +84,7 @@ class PreNormBlock:
         norm that says ``takes_plus`` adds them in its own kernel; for any other they are added here."""
         if plus is not None:
             if getattr(self.norm1, "takes_plus", False):
-                x = self.norm1.forward(residual, pending, self.dtype, plus=plus)
+                x = normalise(self.norm1, residual, pending, self.dtype, plus=plus)
                 return self._behind_first_norm(x, residual, batch, view, writes)
             x = normalise(self.norm1, residual, pending, self.dtype)  # (the pending branch joins the stream)
             residual.add_(plus)
@@ -99,7 +99,7 @@ class PreNormBlock:
 
     def _behind_first_norm(self, x, residual: torch.Tensor, batch, view, writes: bool):
         extra = {"residual": residual} if getattr(self.mixer, "adds_to_residual", False) else {}
-        if extra and getattr(self.mixer, "sums_parts", False):
+        if extra and declares(self.mixer, "sums_parts"):
             extra["sums_parts"] = True
         if (extra and self.has_feed_forward and getattr(self.mixer, "folds_next_norm", False)
                 and getattr(self.norm2, "folds_into_products", False)
@@ -110,24 +110,29 @@ class PreNormBlock:
             return residual, mixed  # (the next norm adds it)
         x = normalise(self.norm2, residual, mixed, self.dtype)
         extra = {"residual": residual} if getattr(self.feed_forward, "adds_to_residual", False) else {}
-        if extra and getattr(self.feed_forward, "sums_parts", False):
+        if extra and declares(self.feed_forward, "sums_parts"):
             extra["sums_parts"] = True
         return residual, self.feed_forward.forward(x, **extra)
 
 
-def normalise(norm, residual: torch.Tensor, pending, dtype: torch.dtype, rows=None):
-    """Run ``norm`` on the residual stream plus what is pending.  Only a norm that
-    says so (``takes_row_sumsq``) is shown the fused forms of a branch; for any
-    other an already added branch becomes ``None``."""
-    if not getattr(norm, "takes_row_sumsq", False) and isinstance(pending, (RowSumsq, Added, KParts)):
-        if isinstance(pending, KParts):
-            pending.join(residual)
+def normalise(norm, residual: torch.Tensor, pending, dtype: torch.dtype, rows=None, plus=None):
+    """Run ``norm`` on the residual stream plus what is pending (and ``plus``, for a norm
+    that takes it).  Only a norm that says so (``takes_row_sumsq``, ``takes_parts``) is
+    shown the fused forms of a branch; for any other an already added branch becomes
+    ``None``, and parts of a product join the stream here."""
+    if isinstance(pending, KParts) and not declares(norm, "takes_parts"):
+        pending.join(residual)
+        pending = None
+    if not getattr(norm, "takes_row_sumsq", False) and isinstance(pending, (RowSumsq, Added)):
         pending = None
     if isinstance(pending, WeightedPair):
         pending = pending.combined()
+    extra = {}
     if rows is not None:
-        return norm.forward(residual, pending, dtype, rows=rows)
-    return norm.forward(residual, pending, dtype)
+        extra["rows"] = rows
+    if plus is not None:
+        extra["plus"] = plus
+    return norm.forward(residual, pending, dtype, **extra)
 
 
 def whole_stream(residual: torch.Tensor, pending) -> torch.Tensor:
@@ -291,7 +296,7 @@ class ParallelDepthBlock:
         mixed = self.mixer.forward(first, batch, view, writes)
         fed = parts = None
         if self.has_feed_forward:  # (its last product may come as parts of K: the boundary's kernel sums them)
-            takes = {"sums_parts": True} if getattr(self.feed_forward, "sums_parts", False) else {}
+            takes = {"sums_parts": True} if declares(self.feed_forward, "sums_parts") else {}
             fed = self.feed_forward.forward(second, **takes)
         if isinstance(fed, KParts):
             fed, parts = None, fed.parts
@@ -372,7 +377,7 @@ class SandwichNormBlock(PreNormBlock):
         if isinstance(pending, NormedRows) and pending.owner is self and plus is None:
             x = pending.first
         elif plus is not None and getattr(self.norm1, "takes_plus", False):
-            x = self.norm1.forward(residual, None if isinstance(pending, NormedRows) else pending, self.dtype, plus=plus)
+            x = normalise(self.norm1, residual, None if isinstance(pending, NormedRows) else pending, self.dtype, plus=plus)
         else:
             if plus is not None:
                 raise ValueError("the first norm of this layer cannot add rows to the stream")
@@ -474,7 +479,7 @@ class ParallelBlock:
         if isinstance(pending, NormedRows) and pending.owner is self and plus is None:
             x = pending.first
         elif plus is not None:
-            x = self.norm1.forward(residual, None if isinstance(pending, NormedRows) else pending, self.dtype, plus=plus)
+            x = normalise(self.norm1, residual, None if isinstance(pending, NormedRows) else pending, self.dtype, plus=plus)
         else:
             x = normalise(self.norm1, residual, None if isinstance(pending, NormedRows) else pending, self.dtype)
         if self.joined:

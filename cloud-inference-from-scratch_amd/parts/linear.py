@@ -190,7 +190,7 @@ class Added:
 @dataclass
 class KParts:
     """Stands where a branch output would: the branch is the sum of ``parts`` [P, rows, hidden] (float32), still to be
-    added into the stream, in order: a product whose K was cut.  A norm that says ``takes_row_sumsq`` sums them itself."""
+    added into the stream, in order: a product whose K was cut.  A norm that says ``takes_parts`` sums them itself."""
 
     parts: torch.Tensor
 

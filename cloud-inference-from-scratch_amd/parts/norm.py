@@ -21,6 +21,7 @@ from .linear import Added, KParts, RowSumsq, ScaledRows, SummedBranch, WeightedP
 class RMSNorm(Part):
     graph_safe = True
     takes_row_sumsq = True
+    takes_parts = True  # its kernel sums the parts of a product whose K was cut
     # between a product that adds into the residual and a product that reads the norm's output, the norm can
     # ride along: the first writes residual * weight, the second applies the rows' 1 / rms to its sums
     folds_into_products = True

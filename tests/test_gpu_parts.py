@@ -1184,3 +1184,65 @@ def test_a_layer_that_reads_the_cache_another_layer_writes(tmp_path, dtype):
             rows = replay_util.by_position(steps, replay_util.drive_runner(runner, steps))
             replay_util.compare(rows, reference, **tolerance)
             assert runner.cache.stats().pages_used == 0
+
+
+@pytest.mark.parametrize("norm", ["rms_norm_groups", "layer_norm", "rms_norm"])
+def test_parts_of_k_reach_a_layer_that_adds_rows(norm, monkeypatch):
+    """A layer whose down product leaves the parts of its K, and behind it one that adds the embedding's rows in its first
+    norm's kernel (a norm that cannot sum parts, and one that can): the same bits as with the parts joined beforehand."""
+    from dataclasses import replace
+
+    from cie_amd.config import PartSpec, Qwen2Config
+    from cie_amd.parts import linear
+    from cie_amd.parts.block import PreNormBlock
+    from cie_amd.parts.linear import KParts
+
+    monkeypatch.setattr(linear, "plan_tiles", lambda rows, n, k, most_parts=1, behind_us=0.0: (64, 64, 2) if most_parts > 1 else None)
+    rows, hidden = 200, 64
+    raw = dict(model_type="qwen2", hidden_size=hidden, num_hidden_layers=2, num_attention_heads=2, num_key_value_heads=1,
+               intermediate_size=136, vocab_size=32, rms_norm_eps=1e-5, rope_theta=1e4, max_position_embeddings=256)
+    layers = Qwen2Config.from_hf_config(raw).model_spec().layers
+    first = PreNormBlock(layers[0])
+    second = PreNormBlock(layers[1] if norm == "rms_norm" else replace(layers[1], norm1=PartSpec.of(norm, size=hidden, eps=1e-5)))
+    bound(first, "model.layers.0.", "bfloat16", 5)
+    bound(second, "model.layers.1.", "bfloat16", 6)
+    manager, device_cache = harness([first.cache_need(), second.cache_need()], [rows], dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(7)
+    stream, plus = torch.randn((rows, hidden), generator=g).cuda(), torch.randn((rows, hidden), generator=g).cuda()
+    batch = batch_of(manager, [(0, 0, rows)])
+    residual, pending = first.forward(stream, None, batch, device_cache.view(0))
+    assert isinstance(pending, KParts) and pending.parts.shape == (2, rows, hidden)
+    joined = residual.clone()
+    pending.join(joined)
+    expect, branch = second.forward(joined, None, batch, device_cache.view(1), plus=plus.clone())
+    got, other = second.forward(residual, pending, batch, device_cache.view(1), plus=plus.clone())
+    assert torch.equal(got, expect) and torch.equal(other.parts, branch.parts)
+
+
+def test_a_feed_forward_with_a_forward_of_its_own_runs_in_a_layer(monkeypatch):
+    """A variant written against the plain interface (no ``sums_parts``) inside a layer, at rows whose products are cut."""
+    from cie_amd.config import Qwen2Config
+    from cie_amd.parts import linear
+    from cie_amd.parts.block import PreNormBlock
+    from cie_amd.parts.feed_forward import GatedMLP
+    from cie_amd.parts.linear import KParts
+
+    class Doubled(GatedMLP):
+        def forward(self, x, residual=None):
+            return super().forward(x) * 2
+
+    monkeypatch.setattr(linear, "plan_tiles", lambda rows, n, k, most_parts=1, behind_us=0.0: (64, 64, 2) if most_parts > 1 else None)
+    raw = dict(model_type="qwen2", hidden_size=64, num_hidden_layers=1, num_attention_heads=2, num_key_value_heads=1,
+               intermediate_size=136, vocab_size=32, rms_norm_eps=1e-5, rope_theta=1e4, max_position_embeddings=256)
+    block = PreNormBlock(Qwen2Config.from_hf_config(raw).model_spec().layers[0])
+    block.feed_forward = Doubled(64, 136)
+    bound(block, "model.layers.0.", "bfloat16", 5)
+    manager, device_cache = harness([block.cache_need()], [200], dtype=torch.bfloat16)
+    stream = torch.randn((200, 64), generator=torch.Generator().manual_seed(8)).cuda()
+    plain_block = PreNormBlock(Qwen2Config.from_hf_config(raw).model_spec().layers[0])
+    bound(plain_block, "model.layers.0.", "bfloat16", 5)
+    batch = batch_of(manager, [(0, 0, 200)])
+    _, doubled = block.forward(stream.clone(), None, batch, device_cache.view(0))
+    _, parts = plain_block.forward(stream.clone(), None, batch, device_cache.view(0))
+    assert isinstance(parts, KParts)
+    check(doubled.float().cpu(), 2 * parts.parts.sum(0).cpu(), "bfloat16")

@@ -1,0 +1,96 @@
+"""What a layer's parts hand to one another, without a GPU: the forms of a pending branch, the arguments that a part is
+given, and the rules that pick a kernel by sizes alone."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+
+class Norm:
+    """A norm of the plain interface: a tensor or nothing to add, rows that join the stream."""
+
+    takes_plus = True
+
+    def forward(self, residual, branch, out_dtype, rows=None, plus=None):
+        assert branch is None or isinstance(branch, torch.Tensor)
+        residual += (0 if branch is None else branch) + (0 if plus is None else plus)
+        return residual.to(out_dtype)
+
+
+def parts_of(*values):
+    from cie_amd.parts.linear import KParts
+
+    return KParts(torch.stack([torch.full((3, 4), float(v)) for v in values]))
+
+
+def test_parts_of_a_product_join_the_stream_for_a_norm_that_cannot_sum_them():
+    from cie_amd.parts.block import normalise, whole_stream
+    from cie_amd.parts.norm import GroupedRMSNorm, LayerNorm, OnePlusRMSNorm, RMSNorm, ScalarRMSNorm
+    from cie_amd.parts.base import declares
+
+    assert all(declares(kind(8, 1e-5), "takes_parts") for kind in (RMSNorm, OnePlusRMSNorm))
+    assert not any(declares(kind(8, 1e-5), "takes_parts") for kind in (GroupedRMSNorm, LayerNorm, ScalarRMSNorm))
+    for plus in (None, torch.full((3, 4), 0.5)):
+        residual = torch.ones(3, 4)
+        rows = normalise(Norm(), residual, parts_of(2, 3), torch.float32, plus=plus)
+        assert torch.equal(rows, torch.full((3, 4), 6.0 if plus is None else 6.5)) and torch.equal(residual, rows)
+    assert torch.equal(whole_stream(torch.ones(3, 4), parts_of(2, 3)), torch.full((3, 4), 6.0))
+
+
+@pytest.mark.parametrize("arrangement", ["pre_norm", "sandwich_norm", "parallel"])
+def test_a_layer_that_adds_rows_takes_a_branch_in_parts(arrangement):
+    """The layer in front leaves the parts of its last product; this one's first norm adds rows in its own kernel and
+    knows no parts."""
+    from cie_amd.parts.block import BranchNormBlock, ParallelBlock, PreNormBlock, SandwichNormBlock  # noqa: F401
+
+    class Mixer:
+        def forward(self, x, batch, view, writes=True):
+            return x
+
+    kind = {"pre_norm": PreNormBlock, "sandwich_norm": SandwichNormBlock, "parallel": ParallelBlock}[arrangement]
+    block = kind.__new__(kind)
+    block.norm1, block.mixer, block.has_feed_forward, block.dtype = Norm(), Mixer(), False, torch.float32
+    block.joined, block.side = False, None
+    residual, seen = torch.ones(3, 4), []
+    if arrangement == "sandwich_norm":
+        class Out:
+            def joins_into(self, then):
+                return False
+
+            def add_normed(self, residual, branch, dtype, **_):
+                seen.append(branch)
+
+        block.norm1_out, block.scale1 = Out(), None
+    _, pending = block.forward(residual, parts_of(2, 3), None, None, plus=torch.full((3, 4), 0.5))
+    assert torch.equal(residual, torch.full((3, 4), 6.5))
+    assert torch.equal(seen[0] if seen else pending, residual)
+
+
+def test_a_variant_with_a_forward_of_its_own_is_not_given_what_its_base_declares():
+    from cie_amd.parts.attention import Attention
+    from cie_amd.parts.base import declares
+    from cie_amd.parts.feed_forward import GatedMLP
+
+    class Reuses(GatedMLP):
+        pass
+
+    class Plain(GatedMLP):
+        def forward(self, x, residual=None):
+            return x
+
+    class Own(GatedMLP):
+        sums_parts = True
+
+        def forward(self, x, residual=None, sums_parts=False):
+            return x
+
+    class Shaped(Attention):
+        def shape_projection(self, qkv, batch):
+            return qkv
+
+    class Declines(GatedMLP):
+        sums_parts = False
+
+    of = lambda kind: declares(kind.__new__(kind), "sums_parts")  # noqa: E731
+    assert [of(k) for k in (GatedMLP, Reuses, Plain, Own, Attention, Shaped, Declines)] == [True, True, False, True, True, True, False]
