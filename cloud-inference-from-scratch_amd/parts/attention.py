@@ -22,8 +22,8 @@ from ..config.specs import PartSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import Part, build_part, register_part
-from .linear import (BEHIND_RATE, FUSED_PARTS_ROWS, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, linear,
-                     plan_tiles)
+from .linear import (BEHIND_RATE, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, linear, plan_tiles,
+                     takes_tiles)
 
 
 ROTATION_US = 5.0  # what the rotation's kernel costs behind the library's q/k/v product, beside its traffic
@@ -147,7 +147,7 @@ class Attention(Part):
                  and x.shape[1] % 8 == 0 and (rows == 1 or x.stride(0) % 8 == 0))
         # (the tiles' epilogue saves the rotation's kernel)
         tiles = (plan_tiles(rows, self.w_qkv.shape[0], x.shape[1], behind_us=ROTATION_US + rows * self.w_qkv.shape[0] * 4e-6 / BEHIND_RATE)
-                 if fused and not few and rows > FUSED_PARTS_ROWS and x.data_ptr() % 16 == 0 else None)
+                 if fused and not few and takes_tiles(rows, x, self.w_qkv) else None)
         if tiles is not None:
             qkv = ops.gemm_tiles_rope(self.w_qkv, x, self.b_qkv, self.cos, self.sin, batch.positions, batch.seq_of_token,
                                       batch.seq_slot, view.block_table, view.k_pool, view.v_pool, self.num_heads,

@@ -294,6 +294,15 @@ def _fusable(rows: int, k: int, row_stride: int, weight: torch.Tensor) -> bool:
     return weight.dtype == torch.bfloat16 and rows >= 1 and k % 8 == 0 and row_stride % 8 == 0
 
 
+def takes_tiles(rows: int, x: torch.Tensor, weight: torch.Tensor, into: Optional[torch.Tensor] = None) -> bool:
+    """Whether the tile kernels take these operands (of a product that is ``_fusable``): beyond the rows of the streaming
+    kernels, on the GPU, in rows and at addresses that 16-byte loads and stores can use.  Whatever else a caller brings
+    (rows read across, a stream that starts off a 16-byte line, host tensors) is the library's or torch's, as it was."""
+    return (rows > FUSED_PARTS_ROWS and x.is_cuda and x.stride(1) == 1 and x.data_ptr() % 16 == 0
+            and weight.data_ptr() % 16 == 0
+            and (into is None or (into.is_cuda and into.dtype == torch.float32 and into.data_ptr() % 16 == 0)))
+
+
 def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out_dtype: Optional[torch.dtype] = None, epilogue: Optional[str] = None,
            into: Optional[torch.Tensor] = None, then_norm: Any = None,
@@ -374,7 +383,7 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
             return ops.gemm_fused(weight, ops.EPI_SILU, x)
         elif not silu:
             return ops.gemm_fused(weight, ops.EPI_F32 if wants_f32 else ops.EPI_BF16, x, bias=bias)
-    if fusable and rows > FUSED_PARTS_ROWS and not wants_f32 and x.data_ptr() % 16 == 0:
+    if fusable and not wants_f32 and takes_tiles(rows, x, weight, into):
         tiles = None
         if into is not None and not silu and into.is_contiguous() and tuple(into.shape) == (rows, n):
             tiles = plan_tiles(rows, n, k, most_parts=TILE_PARTS[-1] if sums_parts else 1)

@@ -1246,3 +1246,20 @@ def test_a_feed_forward_with_a_forward_of_its_own_runs_in_a_layer(monkeypatch):
     _, parts = plain_block.forward(stream.clone(), None, batch, device_cache.view(0))
     assert isinstance(parts, KParts)
     check(doubled.float().cpu(), 2 * parts.parts.sum(0).cpu(), "bfloat16")
+
+
+def test_products_whose_operands_the_tiles_do_not_take():
+    """Some hundred rows of an operand that is read across its rows, and a stream that starts off a 16-byte line: the plain
+    result comes back, as it does for any product that nothing fuses."""
+    from cie_amd.parts.linear import linear, plan_tiles
+
+    rows, n, k = 200, 98, 512
+    assert plan_tiles(rows, n, k) is not None
+    g = torch.Generator().manual_seed(9)
+    wide, w = torch.randn((rows, 2 * k), generator=g).bfloat16().cuda(), torch.randn((n, k), generator=g).bfloat16().cuda()
+    expect = wide[:, ::2].double() @ w.double().t()
+    stream = torch.zeros(rows * n + 2).cuda()[2:].view(rows, n)
+    for got in (linear(wide[:, ::2], w), linear(wide[:, ::2].contiguous(), w, into=stream)):
+        assert isinstance(got, torch.Tensor) and not stream.any()
+        # float32 sums of k products of numbers about 1, rounded once to 8 mantissa bits
+        torch.testing.assert_close(got.double(), expect, rtol=2.0 ** -8, atol=1e-4 * math.sqrt(k))

@@ -94,3 +94,13 @@ def test_a_variant_with_a_forward_of_its_own_is_not_given_what_its_base_declares
 
     of = lambda kind: declares(kind.__new__(kind), "sums_parts")  # noqa: E731
     assert [of(k) for k in (GatedMLP, Reuses, Plain, Own, Attention, Shaped, Declines)] == [True, True, False, True, True, True, False]
+
+
+def test_products_of_many_rows_on_the_host_are_torchs():
+    from cie_amd.parts.linear import linear, plan_tiles
+
+    g = torch.Generator().manual_seed(1)
+    x, w = torch.randn(200, 512, generator=g).bfloat16(), torch.randn(96, 512, generator=g).bfloat16()
+    assert plan_tiles(200, 96, 512) is not None  # (on the GPU this product goes to the tiles)
+    assert torch.equal(linear(x, w), torch.nn.functional.linear(x, w))
+    assert torch.equal(linear(x, w, into=torch.zeros(200, 96)), torch.nn.functional.linear(x, w))
