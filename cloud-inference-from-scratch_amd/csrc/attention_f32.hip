@@ -44,12 +44,13 @@ struct Args {
     const int* block_table;
     int table_width;
     const int *tile_seq, *tile_q0;  // both or neither: tile i is the first of sequence i
-    int first_tile;
     const int *seq_slot, *seq_start, *seq_q_len, *q_start_loc;
     float* out;
-    float *part_o, *part_ml;  // [tiles, kv_heads, blocks, rows, D] and [.., rows, 2]
+    float *part_o, *part_ml;  // [tiles, kv_heads, blocks, rows, D] and [.., rows, 2]; packed: a tile has the blocks it needs
     int rows;                 // of a tile in the workspace
-    int blocks;               // ... and blocks of a tile
+    int blocks;               // ... and the most blocks of a tile
+    int capacity;             // 0: every tile has `blocks` places in the workspace; else places that a round of tiles shares
+    int round;                // packed: the round that runs (prompt form: the first that it runs)
     int q_heads, kv_heads, page_shift, window;
     float scale;
     int tokens_per_tile;
@@ -71,6 +72,31 @@ __device__ __forceinline__ Tile tile_of(const Args& a, int index) {
     t.lo = a.window > 0 ? max(0, t.start + t.q0 + 1 - a.window) : 0;
     t.table = a.block_table + static_cast<size_t>(a.seq_slot[seq]) * a.table_width;
     return t;
+}
+
+__device__ __forceinline__ int blocks_of(const Tile& t) { return (t.hi - 1) / kKeys - t.lo / kKeys + 1; }
+
+// Packed, the tiles' blocks lie one behind the other in the workspace, in rounds of `capacity` places (a round's last tile may
+// reach beyond it, by less than `blocks`): what a captured step launches, and the memory it takes, then follow the lengths
+// that the device knows, not the longest contexts that it may ever see.  The blocks of the tiles before this one; every lane
+// of a wave calls it.
+__device__ __forceinline__ int blocks_before(const Args& a, int index) {
+    int before = 0;
+    for (int j = threadIdx.x % kWave; j < index; j += kWave) before += blocks_of(tile_of(a, j));
+#pragma unroll
+    for (int offset = kWave / 2; offset > 0; offset >>= 1) before += __shfl_xor(before, offset, kWave);
+    return before;
+}
+
+// Where the parts of (tile, kv head) begin in the workspace, in rows; false: the tile is another round's.
+__device__ __forceinline__ bool tile_place(const Args& a, int index, int count, int kv_head, size_t& at) {
+    if (a.capacity == 0) {
+        at = (static_cast<size_t>(index) * a.kv_heads + kv_head) * a.blocks * a.rows;
+        return true;
+    }
+    const int before = blocks_before(a, index);
+    at = (static_cast<size_t>(before % a.capacity) * a.kv_heads + static_cast<size_t>(kv_head) * count) * a.rows;
+    return before / a.capacity == a.round;
 }
 
 __device__ __forceinline__ bool is_finite_bits(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
@@ -177,7 +203,9 @@ __global__ void __launch_bounds__(kTileWaves * kWave, 2) attention_f32_prompt_ke
     const int kv_head = blockIdx.y;
     const int group = a.q_heads / a.kv_heads;
     // (the longest tiles first)
-    const Tile t = tile_of(a, a.first_tile + (gridDim.x - 1 - blockIdx.x));
+    const int index = gridDim.x - 1 - blockIdx.x;
+    const Tile t = tile_of(a, index);
+    if (a.capacity && blocks_before(a, index) / a.capacity < a.round) return;  // (a tile of the block form's rounds)
     const int page_mask = (1 << a.page_shift) - 1;
 
     // this lane's row
@@ -309,9 +337,12 @@ __global__ void __launch_bounds__(kWave, 1) attention_f32_block_kernel(Args a) {
     const int group = a.q_heads / a.kv_heads;
     const int row_tiles = gridDim.y / a.kv_heads;
     const int kv_head = blockIdx.y / row_tiles, row_tile = blockIdx.y % row_tiles;
-    const Tile t = tile_of(a, a.first_tile + blockIdx.x);
+    const Tile t = tile_of(a, blockIdx.x);
     const int rows = t.tokens * group;
     if (16 * row_tile >= rows) return;
+    const int first_block = t.lo / kKeys, last_block = (t.hi - 1) / kKeys;
+    size_t place;
+    if (!tile_place(a, blockIdx.x, last_block - first_block + 1, kv_head, place)) return;
     const int page_mask = (1 << a.page_shift) - 1;
     const int row = 16 * row_tile + r;
     const bool valid = row < rows;
@@ -328,7 +359,6 @@ __global__ void __launch_bounds__(kWave, 1) attention_f32_block_kernel(Args a) {
 #pragma unroll
     for (int i = 0; i < kG; ++i) q[i] = across_quarters(q[i]);
 
-    const int first_block = t.lo / kKeys, last_block = (t.hi - 1) / kKeys;
     for (int block = first_block + blockIdx.z; block <= last_block; block += gridDim.z) {
         const int kb = block * kKeys;
         const bool edge = kb + kKeys - 1 > first_pos || (a.window > 0 && kb < t.hi - a.window);
@@ -380,7 +410,7 @@ __global__ void __launch_bounds__(kWave, 1) attention_f32_block_kernel(Args a) {
         }
         float m, l;
         block_softmax(s, kb, pos, row_lo, a.scale, g, m, l);
-        const size_t at = ((static_cast<size_t>(blockIdx.x) * a.kv_heads + kv_head) * a.blocks + (block - first_block)) * a.rows;
+        const size_t at = place + static_cast<size_t>(block - first_block) * a.rows;
         if (g == 0 && row < a.rows) {
             a.part_ml[(at + row) * 2] = m;
             a.part_ml[(at + row) * 2 + 1] = l;
@@ -414,15 +444,17 @@ constexpr int kJoin = 16;  // blocks that a thread asks for at once (16 blocks a
 
 // One workgroup per (tile, token of the tile, query head), a thread a dimension: the row's blocks joined in order.
 template <int D>
-__global__ void __launch_bounds__(D < 64 ? 64 : D) attention_f32_join_kernel(Args a) {
+__global__ void __launch_bounds__((D + kWave - 1) / kWave * kWave) attention_f32_join_kernel(Args a) {
     const int group = a.q_heads / a.kv_heads;
     const int tok = blockIdx.y / a.q_heads, q_head = blockIdx.y % a.q_heads;
-    const Tile t = tile_of(a, a.first_tile + blockIdx.x);
+    const Tile t = tile_of(a, blockIdx.x);
     const int d = threadIdx.x;
-    if (tok >= t.tokens || d >= D) return;
+    if (tok >= t.tokens) return;
     const int kv_head = q_head / group, row = tok * group + q_head % group;
-    const int count = (t.hi - 1) / kKeys - t.lo / kKeys + 1;
-    const size_t base = ((static_cast<size_t>(blockIdx.x) * a.kv_heads + kv_head) * a.blocks) * a.rows + row;
+    const int count = blocks_of(t);
+    size_t base;
+    if (!tile_place(a, blockIdx.x, count, kv_head, base) || d >= D) return;
+    base += row;
     float M = -INFINITY, L = 0.f, o = 0.f;
     for (int first = 0; first < count; first += kJoin) {
         float m[kJoin], l[kJoin], part[kJoin];
@@ -454,33 +486,35 @@ int run(hipStream_t s, const Args& a, int n_tiles, int row_tiles, int turns) {
         attention_f32_prompt_kernel<D><<<dim3(n_tiles, a.kv_heads), kTileWaves * kWave, 0, s>>>(a);
     } else {
         attention_f32_block_kernel<D><<<dim3(n_tiles, a.kv_heads * row_tiles, turns), kWave, 0, s>>>(a);
-        attention_f32_join_kernel<D><<<dim3(n_tiles, a.tokens_per_tile * a.q_heads), D < 64 ? 64 : D, 0, s>>>(a);
+        attention_f32_join_kernel<D><<<dim3(n_tiles, a.tokens_per_tile * a.q_heads), (D + kWave - 1) / kWave * kWave, 0, s>>>(a);
     }
     return cie_after_launch();
 }
 
 }  // namespace
 
-// Tiles first_tile .. first_tile + n_tiles - 1.  `turns` 0: the prompt form.  Otherwise the block form with that many
-// waves to a tile's 16 rows, and the workspaces part_o [n_tiles, kv_heads, blocks, rows, D] and part_ml [.., 2] with
-// rows >= tokens_per_tile * group and blocks enough for every tile's keys.
+// `turns` 0: the prompt form.  Otherwise the block form with that many waves to a tile's 16 rows, and the workspaces part_o
+// [n_tiles, kv_heads, blocks, rows, D] and part_ml [.., 2] with rows >= tokens_per_tile * group and blocks enough for every
+// tile's keys.  `capacity` > 0: the tiles of round `round`, packed into workspaces of (capacity + blocks) * kv_heads * rows
+// rows; the prompt form then runs the tiles of that round and all later ones.
 CIE_API int cie_paged_attention_f32(void* stream, const float* q, int q_row_stride, const float* k_pool, const float* v_pool,
                                     const int* block_table, int table_width, const int* tile_seq, const int* tile_q0,
-                                    int first_tile, int n_tiles, const int* seq_slot, const int* seq_start,
-                                    const int* seq_q_len, const int* q_start_loc, float* out, float* part_o, float* part_ml,
-                                    int rows, int blocks, int turns, int q_heads, int kv_heads, int head_dim, int page_size,
+                                    int n_tiles, const int* seq_slot, const int* seq_start, const int* seq_q_len,
+                                    const int* q_start_loc, float* out, float* part_o, float* part_ml, int rows, int blocks,
+                                    int capacity, int round, int turns, int q_heads, int kv_heads, int head_dim, int page_size,
                                     int window, float scale, int tokens_per_tile) {
-    if (n_tiles < 0 || first_tile < 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads || page_size < 4 ||
+    if (n_tiles < 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads || page_size < 4 ||
         (page_size & (page_size - 1)) || tokens_per_tile < 1 || tokens_per_tile * (q_heads / kv_heads) > kRowsTile ||
         q_row_stride % 4 || table_width < 1 || (tile_seq == nullptr) != (tile_q0 == nullptr) || kv_heads > 16383 ||
-        static_cast<long>(tokens_per_tile) * q_heads > 65535 || turns < 0 || turns > 65535)
+        static_cast<long>(tokens_per_tile) * q_heads > 65535 || turns < 0 || turns > 65535 || capacity < 0 || round < 0)
         return CIE_BAD_ARGUMENT;
     if (turns && (!part_o || !part_ml || blocks < 1 || rows < tokens_per_tile * (q_heads / kv_heads))) return CIE_BAD_ARGUMENT;
+    if (capacity && static_cast<long>(n_tiles) * blocks > (1L << 30)) return CIE_BAD_ARGUMENT;
     if (n_tiles == 0) return CIE_OK;
     int shift = 0;
     while ((1 << shift) < page_size) ++shift;
-    const Args a{q, q_row_stride, k_pool, v_pool, block_table, table_width, tile_seq, tile_q0, first_tile, seq_slot, seq_start,
-                 seq_q_len, q_start_loc, out, part_o, part_ml, rows, blocks, q_heads, kv_heads, shift, window, scale, tokens_per_tile};
+    const Args a{q, q_row_stride, k_pool, v_pool, block_table, table_width, tile_seq, tile_q0, seq_slot, seq_start,
+                 seq_q_len, q_start_loc, out, part_o, part_ml, rows, blocks, capacity, round, q_heads, kv_heads, shift, window, scale, tokens_per_tile};
     const int row_tiles = (tokens_per_tile * (q_heads / kv_heads) + 15) / 16;
     hipStream_t s = static_cast<hipStream_t>(stream);
     switch (head_dim) {

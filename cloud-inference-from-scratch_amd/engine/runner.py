@@ -57,7 +57,7 @@ class PendingTokens:
 
 
 # What a running engine needs of the device memory beside weights and cache, set aside before the cache takes
-# its share of what is free: the vendor library's workspace, the copies of a weight its timing runs stream
+# its share of what is free: the vendor library's workspace or the float32 kernels', the copies of a weight its timing runs stream
 # through (gemm_library.hip keeps up to 640 MB of them while a shape's candidates are timed), and a full step's
 # activations (per token and number of the model's width: the float32 stream, the 16-bit rows of the norms,
 # projections and feed-forward, and partial sums, some 64 bytes) and float32 logits.
@@ -75,7 +75,7 @@ def flat_needs(needs: Sequence[Any]) -> list[Any]:
 
 def reserve_bytes(config: EngineConfig, hidden_size: int, vocab_size: int) -> int:
     """Device memory kept out of the cache's reach (see above)."""
-    reserve = ops.LIBRARY_WORKSPACE_BYTES
+    reserve = ops.F32_WORKSPACE_BYTES if config.dtype == "float32" else ops.LIBRARY_WORKSPACE_BYTES
     if config.search_library_algorithms:
         reserve += LIBRARY_TIMING_BYTES
     reserve += config.token_budget * hidden_size * ACTIVATION_BYTES_PER_NUMBER

@@ -351,21 +351,25 @@ def paged_attention_generic(q: torch.Tensor, q_row_stride: int, k_pool: torch.Te
 F32_HEAD_DIMS = (32, 64, 96, 128)  # head sizes of the float32 attention on the matrix cores
 F32_TILE_ROWS = 64   # (token, head) rows of its tiles
 F32_BLOCK_KEYS = 64  # keys of its blocks
+# the most bytes that the workspace of a float32 product or attention takes (an engine sets as much aside)
+F32_WORKSPACE_BYTES = 256 << 20
 
 
 def paged_attention_f32(q: torch.Tensor, q_row_stride: int, k_pool: torch.Tensor, v_pool: torch.Tensor,
                         block_table: torch.Tensor, tile_seq: Optional[torch.Tensor], tile_q0: Optional[torch.Tensor],
                         n_tiles: int, seq_slot: torch.Tensor, seq_start: torch.Tensor, seq_q_len: torch.Tensor,
                         q_start_loc: torch.Tensor, out: torch.Tensor, q_heads: int, kv_heads: int, head_dim: int,
-                        window: Optional[int], scale: float, tokens_per_tile: int, first_tile: int = 0, turns: int = 0,
-                        blocks: int = 0, part_o: Optional[torch.Tensor] = None,
-                        part_ml: Optional[torch.Tensor] = None) -> None:
-    """True float32 attention on the matrix cores for the tiles ``first_tile .. first_tile + n_tiles - 1``: tile i holds
+                        window: Optional[int], scale: float, tokens_per_tile: int, turns: int = 0, blocks: int = 0,
+                        part_o: Optional[torch.Tensor] = None, part_ml: Optional[torch.Tensor] = None,
+                        capacity: int = 0, round: int = 0) -> None:
+    """True float32 attention on the matrix cores: tile i holds
     up to ``tokens_per_tile`` tokens of sequence ``tile_seq[i]`` from its ``tile_q0[i]``-th token of this step on (both
     ``None``: tile i starts sequence i).  Rows of other tokens of ``out`` are left alone.  ``turns=0``: a workgroup to a
     tile and key head.  Otherwise that many waves to 16 rows of a tile, which take its blocks of 64 keys in turn and leave
     them in workspaces, of ``blocks`` blocks a tile (as many as any tile's keys need), that a second kernel joins.  Both
-    give a row the same bits."""
+    give a row the same bits.  ``capacity``: the tiles' blocks lie one behind the other instead, each tile with as many as
+    its keys need, in workspaces of ``capacity + blocks`` blocks; the call runs the tiles that begin in the ``round``-th
+    ``capacity`` of them, or, with ``turns=0``, there and behind it."""
     if not (q.is_cuda and q.dtype == torch.float32 and q.dim() == 2 and q.stride(1) == 1 and q.stride(0) == q_row_stride):
         raise ValueError("q must be a float32 GPU matrix with unit inner stride")
     if not (q.shape[1] >= q_heads * head_dim and q_row_stride % 4 == 0):
@@ -384,10 +388,10 @@ def paged_attention_f32(q: torch.Tensor, q_row_stride: int, k_pool: torch.Tensor
     for name, meta in (("tile_seq", tile_seq), ("tile_q0", tile_q0)):
         if meta is not None:
             _gpu(name, meta, torch.int32, 1)
-            if not (meta.shape[0] >= first_tile + n_tiles):
-                raise ValueError(f"{name} has {meta.shape[0]} entries for {first_tile + n_tiles} tiles")
-    if first_tile < 0 or (tile_seq is None and seq_q_len.shape[0] < first_tile + n_tiles):
-        raise ValueError(f"{n_tiles} tiles from {first_tile} on for {seq_q_len.shape[0]} sequences")
+            if not (meta.shape[0] >= n_tiles):
+                raise ValueError(f"{name} has {meta.shape[0]} entries for {n_tiles} tiles")
+    if tile_seq is None and seq_q_len.shape[0] < n_tiles:
+        raise ValueError(f"{n_tiles} tiles for {seq_q_len.shape[0]} sequences")
     for name, meta in (("seq_slot", seq_slot), ("seq_start", seq_start), ("seq_q_len", seq_q_len),
                        ("q_start_loc", q_start_loc)):
         _gpu(name, meta, torch.int32, 1)
@@ -400,13 +404,13 @@ def paged_attention_f32(q: torch.Tensor, q_row_stride: int, k_pool: torch.Tensor
             raise ValueError("attention in blocks needs its workspaces")
         _gpu("part_o", part_o, torch.float32)
         _gpu("part_ml", part_ml, torch.float32)
-        units = n_tiles * kv_heads * blocks * rows
+        units = (capacity + blocks if capacity else n_tiles * blocks) * kv_heads * rows
         if not (part_o.numel() >= units * head_dim and part_ml.numel() >= units * 2):
             raise ValueError("attention workspaces are too small")
     _run("cie_paged_attention_f32", load_library().cie_paged_attention_f32(
         _stream(), _ptr(q), _i(q_row_stride), _ptr(k_pool), _ptr(v_pool), _ptr(block_table), _i(block_table.shape[1]),
-        _ptr(tile_seq), _ptr(tile_q0), _i(first_tile), _i(n_tiles), _ptr(seq_slot), _ptr(seq_start), _ptr(seq_q_len),
-        _ptr(q_start_loc), _ptr(out), _ptr(part_o), _ptr(part_ml), _i(rows), _i(blocks), _i(turns), _i(q_heads),
+        _ptr(tile_seq), _ptr(tile_q0), _i(n_tiles), _ptr(seq_slot), _ptr(seq_start), _ptr(seq_q_len),
+        _ptr(q_start_loc), _ptr(out), _ptr(part_o), _ptr(part_ml), _i(rows), _i(blocks), _i(capacity), _i(round), _i(turns), _i(q_heads),
         _i(kv_heads), _i(head_dim), _i(page_size), _i(window or 0), _f(scale), _i(tokens_per_tile)))
 
 

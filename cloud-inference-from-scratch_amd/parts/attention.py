@@ -11,6 +11,7 @@ switches, scale, position encoding and an optional window are parameters.
 
 from __future__ import annotations
 
+import functools
 import math
 import warnings
 from typing import Optional
@@ -360,11 +361,10 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
 
 
 # Float32: contexts up to which single tokens take the prompt form too (a workgroup's two blocks of 64 keys in turn cost
-# less than the second kernel that joins blocks), and the bytes that the blocks' workspace may take (sequences beyond
-# that go in further launches, which share it)
+# less than the second kernel that joins blocks)
 F32_WHOLE_KEYS = 128
 F32_CUT_TILES = 0.6  # tiles a compute unit up to which prompts' tiles may be cut into blocks
-F32_WORKSPACE_BYTES = 64 << 20
+F32_CUT_BYTES = 64 << 20  # ... and the bytes that their blocks may take
 
 
 def attend_f32(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, head_dim: int,
@@ -380,44 +380,60 @@ def attend_f32(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int
     common = (batch.seq_slot, batch.seq_start, batch.seq_q_len, batch.q_start_loc, out, num_heads, num_kv_heads, head_dim,
               window, scale)
 
-    def run(tiles: tuple, tokens: int, whole: bool) -> None:
+    def run(tiles: tuple, tokens: int, whole: bool = False, decode: bool = False) -> None:
         tile_seq, tile_q0, n_tiles = tiles
         blocks = -(-bound // ops.F32_BLOCK_KEYS)
         if window is not None:  # (a window may begin inside a block)
             blocks = min(blocks, -(-(window + tokens) // ops.F32_BLOCK_KEYS) + 1)
         rows = tokens * group
-        per = num_kv_heads * blocks * rows
+        block_bytes = num_kv_heads * rows * (head_dim + 2) * 4
         # Whole tiles take some 8.3 us a block of the longest tile, tiles in blocks 0.055 us a block of all of them and 8 more
         # (the parts' way through memory), over 256 units (us, whole against in blocks, 16 heads of 128 on 2: a prompt of
         # 130 tokens 30, 24; 256 tokens 39, 31; 517 tokens 79, 66; 1,024 tokens 138, 160; 8 prompts of 64 tokens 16, 36; 8 of
         # 128 25, 68; 14 heads of 64 on 2: 600 tokens 51, 40)
         units = F32_CUT_TILES * cus - n_tiles * num_kv_heads
+        launch = functools.partial(ops.paged_attention_f32, qkv, qkv.stride(0), view.k_pool, view.v_pool, view.block_table,
+                                   tile_seq, tile_q0, n_tiles, *common, tokens)
         if whole or (tokens > 1 and (blocks * units <= F32_CUT_TILES * cus
-                                     or n_tiles * per * (head_dim + 2) * 4 > F32_WORKSPACE_BYTES)):
-            ops.paged_attention_f32(qkv, qkv.stride(0), view.k_pool, view.v_pool, view.block_table, tile_seq, tile_q0,
-                                    n_tiles, *common, tokens)
+                                     or n_tiles * blocks * block_bytes > F32_CUT_BYTES)):
+            launch()
             return
-        at_once = max(1, min(n_tiles, F32_WORKSPACE_BYTES // (per * (head_dim + 2) * 4)))
-        part_o = torch.empty(at_once * per * head_dim, dtype=torch.float32, device=qkv.device)
-        part_ml = torch.empty(at_once * per * 2, dtype=torch.float32, device=qkv.device)
-        for first in range(0, n_tiles, at_once):
-            count = min(at_once, n_tiles - first)
-            waves = count * num_kv_heads * -(-rows // 16)  # (some 16 waves a unit; more blocks than that are taken in turn)
-            ops.paged_attention_f32(qkv, qkv.stride(0), view.k_pool, view.v_pool, view.block_table, tile_seq, tile_q0, count,
-                                    *common, tokens, first_tile=first, turns=min(blocks, max(1, -(-16 * cus // waves))),
-                                    blocks=blocks, part_o=part_o, part_ml=part_ml)
+        places, capacity, rounds = n_tiles * blocks, 0, 1
+        if places * block_bytes > ops.F32_WORKSPACE_BYTES:
+            # Sequences of very different lengths, or a captured step whose bound is far above its contexts: the tiles'
+            # blocks lie packed, as many as the keys that are there need (64 sequences of 100 / 1,000 keys in a step captured
+            # for 131,072: 23 / 51 us, where workspaces of 64 MB that three tiles of 2,048 blocks at a time shared took 370 / 403
+            # and the generic kernel 35 / 298).
+            # The host counts an eager step's rounds; of a captured step it knows none, so one round runs, and
+            # whole tiles what begins behind it (millions of cached tokens in one step).
+            capacity = max(blocks, ops.F32_WORKSPACE_BYTES // block_bytes - blocks)
+            places = capacity + blocks
+            if plan is None:
+                size, behind = ops.F32_BLOCK_KEYS, batch.max_context if window is None else window
+                taken = [(start + min(first + tokens, n) - 1) // size - max(0, start + first + 1 - behind) // size + 1
+                         for start, n in zip(batch.host_starts, batch.host_q_lens) if (n == 1) == decode
+                         for first in range(0, n, tokens)]
+                rounds = -(-sum(taken) // capacity)
+        part_o = torch.empty(places * num_kv_heads * rows * head_dim, dtype=torch.float32, device=qkv.device)
+        part_ml = torch.empty(places * num_kv_heads * rows * 2, dtype=torch.float32, device=qkv.device)
+        waves = n_tiles * num_kv_heads * -(-rows // 16)  # (some 16 waves a unit; more blocks than that are taken in turn)
+        for turn in range(rounds):
+            launch(turns=min(blocks, max(1, -(-16 * cus // waves))), blocks=blocks, part_o=part_o, part_ml=part_ml,
+                   capacity=capacity, round=turn)
+        if capacity and plan is not None:
+            launch(capacity=capacity, blocks=blocks, round=rounds)
 
     single = batch.sequences if plan is not None and plan.decode_rows is None else plan.decode_rows if plan is not None else None
     if bound <= F32_WHOLE_KEYS:
-        run((None, None, batch.sequences) if single == batch.sequences else batch.tiles(per_tile, decode=None), per_tile, True)
+        run((None, None, batch.sequences) if single == batch.sequences else batch.tiles(per_tile, decode=None), per_tile, whole=True)
         return out
     tiles = (None, None, single) if single is not None else batch.tiles(1, decode=True)
     if tiles[2]:
-        run(tiles, 1, False)
+        run(tiles, 1, decode=True)
     if single != batch.sequences:
         tiles = batch.tiles(per_tile, decode=False)
         if tiles[2]:
-            run(tiles, per_tile, False)
+            run(tiles, per_tile)
     return out
 
 

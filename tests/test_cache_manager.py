@@ -498,6 +498,8 @@ def test_pool_size_from_free_memory_keeps_a_reserve():
     tokens = tokens_from_bytes(config, needs, 2, free, 2048, 150_000)
     assert tokens == int((free - reserve) * 0.9) // per_token // 16 * 16
     assert reserve_bytes(build_engine_config(search_library_algorithms=False), 2048, 150_000) < reserve - (600 << 20)
+    # a float32 engine: its kernels' workspace in place of the library's
+    assert reserve_bytes(build_engine_config(config, dtype="float32"), 2048, 150_000) == reserve + (256 << 20) - (64 << 20)
     # less free memory than the reserve: one page, not a negative pool
     assert tokens_from_bytes(config, needs, 2, reserve // 2, 2048, 150_000) == 16
     # bytes given: taken as they are; never more than every slot full can use

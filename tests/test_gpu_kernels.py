@@ -330,6 +330,55 @@ def test_paged_attention_f32(ops, geometry, window):
     assert all(torch.equal(out, outs[0]) for out in outs[1:])
 
 
+@pytest.mark.parametrize("geometry", [(16, 2, 128, 16), (3, 1, 96, 8), (64, 1, 32, 4)])
+@pytest.mark.parametrize("window", [None, 1, 65, 500])
+@pytest.mark.parametrize("captured", [False, True])
+def test_attend_float32_in_rounds(ops, monkeypatch, geometry, window, captured):
+    """Single tokens (and two prompt portions behind them) whose blocks exceed the workspace: an eager step runs as many
+    rounds as its lengths need, a step with a captured step's plan one round and whole tiles behind it, and with room for
+    every tile's bound none of both: all the bits of the whole form."""
+    from cie_amd.engine.batch import PagedView, StepBatch
+    from cie_amd.engine.graphs import StaticPlan
+    from cie_amd.parts import attention
+
+    q_heads, kv_heads, head_dim, page_size = geometry
+    contexts = [0, 62, 63, 1000, 1500, 130, 2000, 700, 64, 100]
+    q_lens = [1] * 8 + [40, 7]
+    k_pool, v_pool, table, slots, _ = build_cache(torch.float32, [c + n for c, n in zip(contexts, q_lens)], kv_heads, head_dim,
+                                                  page_size, seed=76)
+    view = PagedView(k_pool, v_pool, table, page_size)
+    qkv = rand((sum(q_lens), (q_heads + 2 * kv_heads) * head_dim), torch.float32, 77)
+    as_dev = lambda values: torch.tensor(values, dtype=torch.int32).cuda()  # noqa: E731
+    loc = [sum(q_lens[:i]) for i in range(len(q_lens) + 1)]
+    tokens = [(s, t) for s, n in enumerate(q_lens) for t in range(n)]
+    plan = StaticPlan(None, None, as_dev([2001]), 4096, decode_rows=8) if captured else None
+
+    def attend():
+        batch = StepBatch(tokens=len(tokens), sequences=len(q_lens), token_ids=as_dev([0] * len(tokens)),
+                          positions=as_dev([contexts[s] + t for s, t in tokens]), seq_of_token=as_dev([s for s, _ in tokens]),
+                          seq_slot=as_dev(slots), seq_start=as_dev(contexts), seq_q_len=as_dev(q_lens), q_start_loc=as_dev(loc),
+                          logit_rows=as_dev([0]), host_slots=slots, host_starts=[0] * 10 if captured else contexts,
+                          host_q_lens=q_lens, static_plan=plan)
+        return attention.attend(qkv, batch, view, q_heads, kv_heads, head_dim, window, 0.1)
+
+    calls, launch = [], ops.paged_attention_f32
+    monkeypatch.setattr(ops, "paged_attention_f32", lambda *a, **k: (calls.append((k.get("capacity", 0), k.get("round", 0), k.get("turns", 0))), launch(*a, **k)))
+    roomy = attend()
+    assert not any(capacity for capacity, _, _ in calls)
+    calls.clear()
+    monkeypatch.setattr(ops, "F32_WORKSPACE_BYTES", 1)  # (the least there is: places for one tile's bound a round)
+    tight = attend()
+    rounds = [(turn, turns > 0) for capacity, turn, turns in calls if capacity]
+    if captured:
+        assert rounds in ([(0, True), (1, False)], [(0, True), (1, False)] * 2)  # (the portions may be cut too)
+    else:
+        assert rounds[0] == (0, True) and all(turn in (0, last + 1) and cut for (last, _), (turn, cut) in zip(rounds, rounds[1:]))
+        assert len(rounds) > 2 or window is not None
+    monkeypatch.setattr(attention, "F32_WHOLE_KEYS", 1 << 20)
+    whole = attend()
+    assert torch.equal(roomy, whole) and torch.equal(tight, whole)
+
+
 @pytest.mark.parametrize("turns", [0, 2])
 def test_paged_attention_f32_odd_values_reach_the_rows_that_see_them(ops, turns):
     """An infinity and a NaN among the cached values: the rows before them in the same tile stay as they are, the rows
