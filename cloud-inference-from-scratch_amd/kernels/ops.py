@@ -509,12 +509,21 @@ def paged_attention_mfma(q: torch.Tensor, q_row_stride: int, k_pool: torch.Tenso
 F32_STRETCH = 1024  # k that one workgroup takes where the float32 product cuts K
 
 
+def f32_bands(rows: int, columns: int, k: int) -> tuple[int, int]:
+    """(bands, rows of a band) in which the float32 product with K in stretches takes its rows: as few bands, in multiples
+    of the tiles' 64 rows, as keep the stretches' sums of one within ``F32_WORKSPACE_BYTES`` (7B down of 1,500 rows: two
+    bands of 768 instead of 409 MB)."""
+    most = max(64, F32_WORKSPACE_BYTES // (-(-k // F32_STRETCH) * columns * 4) // 64 * 64)
+    bands = -(-rows // most)
+    return bands, -(-(-(-rows // bands)) // 64) * 64
+
+
 def plan_gemm_f32(rows: int, columns: int, k: int) -> int:
     """Which form of the float32 product runs (the numbers of ``cie_gemm_f32``): 0 few rows, 1 tiles of 64 x 64, 2 such
     tiles with K cut in stretches.  Up to 16 rows the first, bound by the weight's stream; beyond that the one whose
     turns over the units take least, in us as measured on MI355X: a turn of workgroups of 32 rows and 16 columns takes
     9.5 per 2,048 k (eight waves; 3.9 where K is up to 1,024 and four waves do), a tile 21.5 per 1,000 k when alone on its
-    unit and 17.5 behind another, a stretch 19 and the join behind it 10.  (N = K = 2,048: 64 / 128 rows 13 / 23 in
+    unit and 17.5 behind another, a stretch 19 and the join behind it 10, a band.  (N = K = 2,048: 64 / 128 rows 13 / 23 in
     the first, 47 / 48 in the second, 28 / 29 in the third form; N 22,016: 101 / 177, 81 / 115, 69 / 125; N 2,048, K
     11,008: 53 / 106, 236 / 237, 52 / 75.)"""
     if rows <= 16:
@@ -525,7 +534,10 @@ def plan_gemm_f32(rows: int, columns: int, k: int) -> int:
     tiles = -(-rows // 64) * -(-columns // 64)
     whole = 2 + k / 1000 * (21.5 + 17.5 * (-(-tiles // units) - 1))
     stretches = -(-k // F32_STRETCH)
-    cut = 10 + 19 * min(k, F32_STRETCH) / F32_STRETCH * -(-tiles * stretches // units) if stretches > 1 and rows <= 65535 else whole
+    cut = whole
+    if stretches > 1 and 64 * stretches * columns * 4 <= F32_WORKSPACE_BYTES:
+        bands, band = f32_bands(rows, columns, k)
+        cut = bands * (10 + 19 * -(-(band // 64 * -(-columns // 64) * stretches) // units))
     return 0 if few <= min(whole, cut) else 1 if whole <= cut else 2
 
 
@@ -556,12 +568,14 @@ def gemm_f32(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
     lda = a.stride(0) if m > 1 else max(a.stride(0), k)
     if form is None:
         form = plan_gemm_f32(m, n, k)
-    parts = None
-    if form == 2:
-        parts = torch.empty((-(-k // F32_STRETCH), m, n), dtype=torch.float32, device=a.device)
-    _run("cie_gemm_f32", load_library().cie_gemm_f32(_stream(), _ptr(a), _ptr(weight), _ptr(bias), _ptr(out), _ptr(parts),
-                                                     _i(m), _i(n), _i(k), _i(lda), _i(width), _i(bool(gate)), _i(form),
-                                                     _i(compute_units(a.device))))
+    band, parts = m, None
+    if form == 2 and m:
+        _, band = f32_bands(m, n, k)
+        parts = torch.empty((-(-k // F32_STRETCH), min(m, band), n), dtype=torch.float32, device=a.device)
+    for first in range(0, max(m, 1), max(band, 1)):
+        _run("cie_gemm_f32", load_library().cie_gemm_f32(
+            _stream(), _ptr(a) + 4 * first * lda, _ptr(weight), _ptr(bias), _ptr(out) + 4 * first * width, _ptr(parts),
+            _i(min(band, m - first)), _i(n), _i(k), _i(lda), _i(width), _i(bool(gate)), _i(form), _i(compute_units(a.device))))
     return out
 
 

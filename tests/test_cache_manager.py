@@ -498,8 +498,6 @@ def test_pool_size_from_free_memory_keeps_a_reserve():
     tokens = tokens_from_bytes(config, needs, 2, free, 2048, 150_000)
     assert tokens == int((free - reserve) * 0.9) // per_token // 16 * 16
     assert reserve_bytes(build_engine_config(search_library_algorithms=False), 2048, 150_000) < reserve - (600 << 20)
-    # a float32 engine: its kernels' workspace in place of the library's
-    assert reserve_bytes(build_engine_config(config, dtype="float32"), 2048, 150_000) == reserve + (256 << 20) - (64 << 20)
     # less free memory than the reserve: one page, not a negative pool
     assert tokens_from_bytes(config, needs, 2, reserve // 2, 2048, 150_000) == 16
     # bytes given: taken as they are; never more than every slot full can use
@@ -508,3 +506,12 @@ def test_pool_size_from_free_memory_keeps_a_reserve():
     small = build_engine_config(max_model_len=64, max_running=2, page_size=16, prefix_cache_pages=3)
     assert tokens_from_bytes(small, needs, 2, free, 2048, 150_000) == (2 * 4 + 3) * 16
     assert tokens_from_bytes(config, [FixedState((4,))], 2, free, 64, 100) == 16  # nothing is paged
+
+
+def test_a_float32_engine_sets_its_kernels_workspace_aside():
+    from cie_amd.config import build_engine_config
+    from cie_amd.engine.runner import reserve_bytes
+    from cie_amd.kernels import ops
+
+    apart = reserve_bytes(build_engine_config(dtype="float32"), 2048, 1000) - reserve_bytes(build_engine_config(), 2048, 1000)
+    assert apart == ops.F32_WORKSPACE_BYTES - ops.LIBRARY_WORKSPACE_BYTES

@@ -121,6 +121,18 @@ def test_gemm_f32_forms(ops, shape):
         assert all(torch.equal(ops.gemm_f32(a, w, gate=True, form=form), unit) for form in (0, 1, 2))
 
 
+@pytest.mark.parametrize("shape", [(200, 66, 1028), (129, 130, 4100)])
+def test_gemm_f32_in_bands_of_rows(ops, monkeypatch, shape):
+    """Stretches of K whose sums do not fit the workspace: the rows go in bands, with the bits of the other forms."""
+    m, n, k = shape
+    wide = rand((m, k + 12), torch.float32, 13)
+    a, w, b = wide[:, :k], rand((n, k), torch.float32, 14), rand((n,), torch.float32, 15)
+    expect, unit = ops.gemm_f32(a, w, b, form=1), ops.gemm_f32(a, w, gate=True, form=1)
+    monkeypatch.setattr(ops, "F32_WORKSPACE_BYTES", 1)
+    assert ops.f32_bands(m, n, k) == (-(-m // 64), 64)
+    assert torch.equal(ops.gemm_f32(a, w, b, form=2), expect) and torch.equal(ops.gemm_f32(a, w, gate=True, form=2), unit)
+
+
 @pytest.mark.parametrize("shape", [(1, 40, 24), (5, 515, 96), (16, 64, 128), (17, 130, 200), (33, 70, 1032),
                                    (64, 256, 264), (150, 99, 72)])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])

@@ -104,3 +104,16 @@ def test_products_of_many_rows_on_the_host_are_torchs():
     assert plan_tiles(200, 96, 512) is not None  # (on the GPU this product goes to the tiles)
     assert torch.equal(linear(x, w), torch.nn.functional.linear(x, w))
     assert torch.equal(linear(x, w, into=torch.zeros(200, 96)), torch.nn.functional.linear(x, w))
+
+
+@pytest.mark.parametrize("rows,columns,k", [(2100, 3584, 18944), (4100, 2048, 11008), (1500, 3584, 18944), (20, 896, 4864),
+                                            (70000, 1024, 4096), (64, 152064, 8192), (517, 2048, 11008)])
+def test_float32_products_in_stretches_keep_their_workspace_bounded(rows, columns, k):
+    from cie_amd.kernels import ops
+
+    bands, band = ops.f32_bands(rows, columns, k)
+    assert band % 64 == 0 and (bands - 1) * band < rows <= bands * band
+    held = -(-k // ops.F32_STRETCH) * min(rows, band) * columns * 4
+    assert held <= ops.F32_WORKSPACE_BYTES or (band == 64 and ops.plan_gemm_f32(rows, columns, k) != 2)
+    if (rows, columns, k) == (1500, 3584, 18944):  # (2,005 us in whole tiles, 1,878 in stretches at once)
+        assert (bands, band) == (2, 768) and ops.plan_gemm_f32(rows, columns, k) == 2
