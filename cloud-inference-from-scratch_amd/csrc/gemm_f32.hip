@@ -404,8 +404,13 @@ template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec>
 void run_rows(hipStream_t s, const Product& p) {
     const int step = kGate ? kColumns / 2 : kColumns;
     const int tiles = ((kGate ? p.N / 2 : p.N) + step - 1) / step;
-    // as many workgroups as the units hold at a time by their LDS (two of the wide ones, four of the others)
-    const int most = p.units * ((kColumns == 32 || kRows == 32 || kWaves == 16 ? 2 : 4) * (kWaves == 4 ? 2 : 1));
+    // as many workgroups as the units hold at a time by their LDS (2 KB a wave for each staged tile and each tile of sums):
+    // further ones would start cold behind them instead of fetching across the end of a tile (N 22,016, K 2,048 with the
+    // gate at 32 rows 54.3 -> 49.3 us, N 3,584, K 18,944 at 16 rows 88 -> 83).  Not for 16 columns of up to 16 rows, three to
+    // a unit, whose columns never exceed four a unit: all at once (N 14,000, K 2,048 at 4 rows 25.9; by their LDS 27.4)
+    constexpr int kRowTiles = (kRows + 15) / 16, kColumnTiles = (kColumns + 15) / 16;
+    constexpr int kLds = kWaves * 2048 * (kRowTiles + kColumnTiles + kRowTiles * kColumnTiles);
+    const int most = p.units * (kRows <= 16 && kColumns == 16 ? 32 / kWaves : 160 * 1024 / kLds);
     dim3 grid(tiles < most ? tiles : most, (p.M + kRows - 1) / kRows);
     gemm_f32_rows_kernel<kRows, kColumns, kWaves, kGate, kVec><<<grid, kWaves * kWave, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc);
 }
