@@ -23,7 +23,8 @@
 //
 // Measured (MI355X, 3B shape, us; the library's product, and the kernel behind it, in brackets): 256 rows: down in 4 parts
 // 26 (38), o_proj 9 (15), q/k/v with rotation and cache write 15 (16 + 5); 613 rows: down in 3 parts 47 (63), q/k/v 19
-// (18 + 5); 1,024 rows: down in 4 parts 56 (74).  Gate/up of 256 rows and more is the library's.
+// (18 + 5); 1,024 rows: down in 4 parts 56 (74).  Gate/up, with the library's gate kernel in its figure: 256 rows 40 (41),
+// 613 rows 77 (72), where it stays the library's; of the 0.5B shape 20.8 (26.4) at 613 rows, 48 (49) at 2,048.
 #include "common.h"
 
 namespace {

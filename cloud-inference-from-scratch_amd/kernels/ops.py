@@ -793,6 +793,8 @@ def library_search(rows):
 
 
 def _tune_level(rows: int) -> int:
+    """How the library's algorithm for products of this many rows is chosen: 0 its first choice, 1 its candidates timed, 2 all
+    its algorithms timed."""
     if rows >= LIBRARY_TUNE_ROWS and rows in _search_rows:
         return 2
     if (rows >= LIBRARY_TUNE_ROWS and rows % 256 == 0) or (rows >= 32 and rows & (rows - 1) == 0):

@@ -23,11 +23,10 @@ from ..config.specs import PartSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import Part, build_part, register_part
-from .linear import (BEHIND_RATE, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, linear, plan_tiles,
-                     takes_tiles)
+from .linear import FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, behind, linear, plan_tiles, takes_tiles
 
 
-ROTATION_US = 5.0  # what the rotation's kernel costs behind the library's q/k/v product, beside its traffic
+ROTATION_US = (1.1, 1.8)  # the rotation's kernel behind the library's q/k/v product: us, and us per million numbers
 
 
 class Attention(Part):
@@ -147,7 +146,7 @@ class Attention(Part):
         fused = (x.dtype == torch.bfloat16 and untouched and head_dim % 32 == 0
                  and x.shape[1] % 8 == 0 and (rows == 1 or x.stride(0) % 8 == 0))
         # (the tiles' epilogue saves the rotation's kernel)
-        tiles = (plan_tiles(rows, self.w_qkv.shape[0], x.shape[1], behind_us=ROTATION_US + rows * self.w_qkv.shape[0] * 4e-6 / BEHIND_RATE)
+        tiles = (plan_tiles(rows, self.w_qkv.shape[0], x.shape[1], behind_us=behind(ROTATION_US, rows, self.w_qkv.shape[0]))
                  if fused and not few and takes_tiles(rows, x, self.w_qkv) else None)
         if tiles is not None:
             qkv = ops.gemm_tiles_rope(self.w_qkv, x, self.b_qkv, self.cos, self.sin, batch.positions, batch.seq_of_token,
@@ -409,8 +408,8 @@ def attend_f32(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int
             capacity = max(blocks, ops.F32_WORKSPACE_BYTES // block_bytes - blocks)
             places = capacity + blocks
             if plan is None:
-                size, behind = ops.F32_BLOCK_KEYS, batch.max_context if window is None else window
-                taken = [(start + min(first + tokens, n) - 1) // size - max(0, start + first + 1 - behind) // size + 1
+                size, sight = ops.F32_BLOCK_KEYS, batch.max_context if window is None else window
+                taken = [(start + min(first + tokens, n) - 1) // size - max(0, start + first + 1 - sight) // size + 1
                          for start, n in zip(batch.host_starts, batch.host_q_lens) if (n == 1) == decode
                          for first in range(0, n, tokens)]
                 rounds = -(-sum(taken) // capacity)

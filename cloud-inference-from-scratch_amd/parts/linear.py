@@ -20,6 +20,7 @@ package), as the reference leaves its products to a library
 from __future__ import annotations
 
 import functools
+import math
 import weakref
 from dataclasses import dataclass
 from typing import Any, Optional, Union
@@ -99,51 +100,66 @@ def plan_shared_parts(tiles: int, k: int) -> tuple[int, int, int]:
 
 
 # Products of more rows than the kernels above take (beyond ``FUSED_PARTS_ROWS``) go to tiles of this package or to the
-# vendor library, whichever the two models below say is faster.
-# Tiles: us per slice of 64 k of a workgroup alone on its unit, and of every further one that meets it there (measured on
-# MI355X at the 3B shape's widths, one to eleven workgroups a unit; what bounds them is the rate at which a unit is fed
-# from its L2, some 20 bytes a cycle, hence the advantage of large tiles where they are many).
-TILE_SLICE_US = {(64, 64): (0.28, 0.17), (128, 64): (0.39, 0.35), (128, 128): (0.63, 0.55), (128, 256): (0.94, 1.20)}
+# vendor library, whichever the two models below say is faster.  Both are fitted to 608 products timed inside captured
+# chains on MI355X with the kernels between them (q/k/v, o_proj, gate/up and down of six shapes from 896 to 8,192 wide, at
+# 16 to 30 row counts from 130 to 2,048).
+# Tiles (within 6 % of the measured, root mean square), us: a start, and per slice of 64 k of a workgroup alone on its unit
+# and of every further one that meets it there (what bounds them is the rate at which a unit is fed from its L2, some 20 bytes
+# a cycle, hence the advantage of large tiles where they are many).  The tiles are dealt to the 8 XCDs in equal runs and each
+# XCD has an eighth of the units: 33 workgroups on one of them take two turns, though there are fewer than 256 in all.
+TILE_US = {(64, 64): (4.9, 0.251, 0.233), (128, 64): (6.1, 0.405, 0.346), (128, 128): (7.8, 0.628, 0.525),
+           (128, 256): (9.5, 0.880, 1.04)}
 TILE_PARTS = (1, 2, 3, 4, 6, 8)
-TILE_START_US = 5.0
-# parts of K: float32 sums written by the product and read by the norm, MB per us
-TILE_PARTS_RATE = 4.5
-# The library, whose algorithms do not cut K: some 0.95 PFLOP/s (GFLOP per us) where tiles of 128 x 128 give every unit
-# one, less by the root of the share that have one, a little more where several meet on one, up to 1.25; and never faster
-# than 9 us and 2.8 per 1,000 k (measured, modelled in brackets, us: 3B down at 256 / 613 / 1,024 / 2,048 rows 38 / 63 /
-# 73 / 100 (40 / 52 / 69 / 97), gate/up 37 / 64 / 86 / 139 (24 / 49 / 75 / 147); o_proj 15-18 (15-17)).
-LIBRARY_RATE, LIBRARY_MOST = 0.95, 1.25
-LIBRARY_START_US, LIBRARY_K_US = 9.0, 2.8e-3
-# what a kernel behind the library's product costs that an epilogue saves: its launch, and its traffic
-BEHIND_US = 5.0
-BEHIND_RATE = 5.0
-TILES_MARGIN = 1.03  # the tiles are taken where they are modelled to be faster by this
+TILE_PARTS_US = 0.356  # parts of K: float32 sums written by the product and read by the norm, us per MB
+XCDS = 8
+# The library (within 12 %; it takes its first choice of algorithm for a row count that does not recur, now and then a bad
+# one: 7B down at 400 rows 200 us where this says 114 and the tiles take 90): the way through one tile's K and its weight rows
+# (us, per 1,000 k, per million weights), and the products at a rate (PFLOP/s) that goes by the tiles of 128 x 128 a unit.
+LIBRARY_US = (8.6, 1.0, 0.40)
+LIBRARY_RATE, LIBRARY_MOST = 0.85, 1.32
+LIBRARY_TUNED = (1.0, 0.90, 0.85)  # ... and its share of that where its candidates, or all its algorithms, were timed
+# What the library's product costs behind it beyond what the tiles' epilogue does: us, and us per million numbers of the
+# product: the gate's kernel; the branch, which is rounded, written and read again by the norm.
+GATE_US = (2.15, 1.2)
+BRANCH_US = (-1.3, 1.9)
+# The tiles are taken where they are modelled to be faster by this.  Of the products 31 are then more than 2 % slower than
+# the library's would be (the worst 1.25, the 72B down at 360 rows, where its first choice is a good one), and all
+# together 6.3 % faster, 1.4 % from the better of the two each time; with 1.03 48 and 6.2 %, with 1.1 24 and 6.3 %.
+TILES_MARGIN = 1.07
+
+
+def behind(us: tuple[float, float], rows: int, n: int) -> float:
+    """What ``plan_tiles`` is given as ``behind_us`` for a product of ``rows`` x ``n``."""
+    return us[0] + us[1] * rows * n * 1e-6
+
+
+def _tile_us(columns: int, tile_rows: int, parts: int, rows: int, n: int, k: int, units: int) -> float:
+    start, first, further = TILE_US[columns, tile_rows]
+    tiles = -(-rows // tile_rows) * -(-n // columns)
+    turns = -(-(-(-tiles // XCDS) * parts) // max(1, units // XCDS))
+    slices = -(-(-(-k // parts)) // 64)
+    return start + slices * (first + (turns - 1) * further) + (parts * rows * n * 4e-6 * TILE_PARTS_US if parts > 1 else 0.0)
+
+
+def _library_us(rows: int, n: int, k: int, units: int, tuned: int) -> float:
+    share = -(-rows // 128) * -(-n // 128) / units
+    rate = min(LIBRARY_MOST, LIBRARY_RATE * share ** (0.46 if share < 1.0 else 0.51))
+    start, per_k, per_weight = LIBRARY_US
+    return LIBRARY_TUNED[tuned] * math.hypot(start + per_k * 1e-3 * k + per_weight * 1e-6 * n * k, 2e-9 * rows * n * k / rate)
 
 
 @functools.lru_cache(maxsize=4096)
-def _plan_tiles(rows: int, n: int, k: int, most_parts: int, behind_us: float, units: int) -> Optional[tuple[int, int, int]]:
-    best = None
-    for (columns, tile_rows), (first, further) in TILE_SLICE_US.items():
-        tiles = -(-rows // tile_rows) * -(-n // columns)
-        for parts in TILE_PARTS:
-            per_part = -(-(-(-k // parts)) // 64) * 64
-            if parts > most_parts or per_part * (parts - 1) >= k:
-                continue
-            cost = TILE_START_US + per_part / 64 * (first + (-(-tiles * parts // units) - 1) * further)
-            if parts > 1:
-                cost += parts * rows * n * 8e-6 / TILE_PARTS_RATE
-            if best is None or cost < best[0]:
-                best = (cost, (columns, tile_rows, parts))
-    share = -(-rows // 128) * -(-n // 128) / units
-    rate = min(LIBRARY_MOST, LIBRARY_RATE * share ** (0.5 if share < 1.0 else 0.15))
-    library = max(LIBRARY_START_US + LIBRARY_K_US * k, 2e-9 * rows * n * k / rate) + behind_us
-    return best[1] if best[0] * TILES_MARGIN < library else None
+def _plan_tiles(rows: int, n: int, k: int, most_parts: int, behind_us: float, units: int, tuned: int) -> Optional[tuple[int, int, int]]:
+    forms = [(columns, tile_rows, parts) for columns, tile_rows in TILE_US for parts in TILE_PARTS
+             if parts <= most_parts and -(-(-(-k // parts)) // 64) * 64 * (parts - 1) < k]  # (every part has some of K)
+    cost, form = min((_tile_us(*form, rows, n, k, units), form) for form in forms)
+    return form if cost * TILES_MARGIN < _library_us(rows, n, k, units, tuned) + behind_us else None
 
 
 def plan_tiles(rows: int, n: int, k: int, most_parts: int = 1, behind_us: float = 0.0) -> Optional[tuple[int, int, int]]:
     """(columns, rows, parts of K) of the tiles that a bfloat16 product of some hundred rows takes, or ``None`` where the
     library's product (and a kernel of ``behind_us`` behind it, which the tiles' epilogue would save) is the faster one."""
-    return _plan_tiles(rows, n, k, most_parts, behind_us, ops.compute_units())
+    return _plan_tiles(rows, n, k, most_parts, behind_us, ops.compute_units(), ops._tune_level(rows))
 
 
 @dataclass
@@ -386,14 +402,14 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
     if fusable and not wants_f32 and takes_tiles(rows, x, weight, into):
         tiles = None
         if into is not None and not silu and into.is_contiguous() and tuple(into.shape) == (rows, n):
-            tiles = plan_tiles(rows, n, k, most_parts=TILE_PARTS[-1] if sums_parts else 1)
+            tiles = plan_tiles(rows, n, k, most_parts=TILE_PARTS[-1] if sums_parts else 1, behind_us=behind(BRANCH_US, rows, n))
             if tiles is not None and tiles[2] > 1:
                 return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, *tiles[:2], bias=bias, parts=tiles[2]))
             if tiles is not None:
                 ops.gemm_tiles(weight, ops.TILE_RESID, x, *tiles[:2], bias=bias, into=into)
                 return Added()
         elif into is None and silu and n % 2 == 0 and bias is None:
-            tiles = plan_tiles(rows, n, k, behind_us=BEHIND_US + rows * n * 3e-6 / BEHIND_RATE)
+            tiles = plan_tiles(rows, n, k, behind_us=behind(GATE_US, rows, n))
             if tiles is not None:
                 return ops.gemm_tiles(weight, ops.TILE_SILU, x, *tiles[:2])
         elif into is None and not silu:

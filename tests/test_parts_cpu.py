@@ -117,3 +117,24 @@ def test_float32_products_in_stretches_keep_their_workspace_bounded(rows, column
     assert held <= ops.F32_WORKSPACE_BYTES or (band == 64 and ops.plan_gemm_f32(rows, columns, k) != 2)
     if (rows, columns, k) == (1500, 3584, 18944):  # (2,005 us in whole tiles, 1,878 in stretches at once)
         assert (bands, band) == (2, 768) and ops.plan_gemm_f32(rows, columns, k) == 2
+
+
+# (what, rows, columns, K, us by the library with the kernel behind it, {tiles: us}), as measured on MI355X: products for
+# which an earlier rule took tiles that were slower than the library, or than whole tiles
+MEASURED = [
+    ("down", 613, 3584, 18944, 151.2, {(128, 256, 3): 193.0, (128, 128, 3): 134.1}),
+    ("down", 680, 3584, 18944, 169.8, {(128, 256, 3): 195.3, (128, 128, 3): 138.4}),
+    ("down", 768, 3584, 18944, 161.5, {(128, 256, 3): 198.8, (128, 128, 3): 145.2}),
+    ("down", 768, 896, 4864, 23.1, {(128, 64, 3): 28.3}),
+    ("o", 130, 3584, 3584, 20.4, {(128, 64, 3): 23.5, (64, 64, 3): 19.4}),
+    ("o", 330, 896, 896, 12.1, {(64, 64, 3): 11.2, (64, 64, 1): 10.6, (64, 64, 2): 10.2}),
+    ("o", 360, 2048, 2048, 16.3, {(128, 64, 2): 17.8, (64, 64, 1): 16.6}),
+]
+
+
+@pytest.mark.parametrize("what,rows,n,k,library,tiles", MEASURED)
+def test_tiles_are_not_taken_where_they_were_measured_to_lose(what, rows, n, k, library, tiles):
+    from cie_amd.parts.linear import BRANCH_US, behind, plan_tiles
+
+    picked = plan_tiles(rows, n, k, most_parts=8, behind_us=behind(BRANCH_US, rows, n))
+    assert (tiles[picked] if picked else library) <= 1.05 * min(library, *tiles.values())
