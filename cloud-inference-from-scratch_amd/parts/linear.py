@@ -122,10 +122,11 @@ LIBRARY_TUNED = (1.0, 0.90, 0.85)  # ... and its share of that where its candida
 # product: the gate's kernel; the branch, which is rounded, written and read again by the norm.
 GATE_US = (2.15, 1.2)
 BRANCH_US = (-1.3, 1.9)
-# The tiles are taken where they are modelled to be faster by this.  Of the products 31 are then more than 2 % slower than
-# the library's would be (the worst 1.25, the 72B down at 360 rows, where its first choice is a good one), and all
-# together 6.3 % faster, 1.4 % from the better of the two each time; with 1.03 48 and 6.2 %, with 1.1 24 and 6.3 %.
-TILES_MARGIN = 1.07
+# The tiles are taken where they are modelled to be faster by this: tiles of up to 25 us, and longer ones, where a good
+# algorithm that the library happens to have costs more.  Of the products 25 are then more than 2 % slower than the
+# library's would be (the worst 1.25, the 72B down at 360 rows), and all together 6.3 % faster, 1.4 % from the better of
+# the two each time; with 1.07 for all of them 31, 6.3 and 1.4 %, with 1.15 9, 6.1 and 1.6 %.
+TILES_MARGIN, TILES_SHORT_US, TILES_MARGIN_LONG = 1.05, 25.0, 1.12
 
 
 def behind(us: tuple[float, float], rows: int, n: int) -> float:
@@ -153,7 +154,8 @@ def _plan_tiles(rows: int, n: int, k: int, most_parts: int, behind_us: float, un
     forms = [(columns, tile_rows, parts) for columns, tile_rows in TILE_US for parts in TILE_PARTS
              if parts <= most_parts and -(-(-(-k // parts)) // 64) * 64 * (parts - 1) < k]  # (every part has some of K)
     cost, form = min((_tile_us(*form, rows, n, k, units), form) for form in forms)
-    return form if cost * TILES_MARGIN < _library_us(rows, n, k, units, tuned) + behind_us else None
+    margin = TILES_MARGIN if cost <= TILES_SHORT_US else TILES_MARGIN_LONG
+    return form if cost * margin < _library_us(rows, n, k, units, tuned) + behind_us else None
 
 
 def plan_tiles(rows: int, n: int, k: int, most_parts: int = 1, behind_us: float = 0.0) -> Optional[tuple[int, int, int]]:
