@@ -120,7 +120,7 @@ def test_float32_products_in_stretches_keep_their_workspace_bounded(rows, column
 
 
 # (what, rows, columns, K, us by the library with the kernel behind it, {tiles: us}), as measured on MI355X: products for
-# which an earlier rule took tiles that were slower than the library, or than whole tiles
+# which an earlier rule took tiles that were slower than the library (the first of each), and tiles that are not
 MEASURED = [
     ("down", 613, 3584, 18944, 151.2, {(128, 256, 3): 193.0, (128, 128, 3): 134.1}),
     ("down", 680, 3584, 18944, 169.8, {(128, 256, 3): 195.3, (128, 128, 3): 138.4}),
@@ -137,4 +137,4 @@ def test_tiles_are_not_taken_where_they_were_measured_to_lose(what, rows, n, k, 
     from cie_amd.parts.linear import BRANCH_US, behind, plan_tiles
 
     picked = plan_tiles(rows, n, k, most_parts=8, behind_us=behind(BRANCH_US, rows, n))
-    assert (tiles[picked] if picked else library) <= 1.05 * min(library, *tiles.values())
+    assert picked is None or tiles[picked] <= 1.03 * library
