@@ -186,11 +186,11 @@ CIE_API int cie_depth_stream(void* stream_handle, int dtype, const float* x, con
     KERNEL<T __VA_OPT__(,) __VA_ARGS__><<<rows, threads, hidden * sizeof(float), s>>>(                                                           \
         x, static_cast<const T*>(branch_a), static_cast<const T*>(branch_b), mult, history, layer_stride, newest,      \
         weights, terms, stream, static_cast<T*>(out1), gain1, static_cast<T*>(out2), gain2, hidden, eps, parts, n_parts)
-    if ((dtype == CIE_F32 && wide(16)) || (dtype == CIE_BF16 && wide(8))) {
+    // (two branches and parts beside them: the form of single numbers; no layer brings them)
+    if (!(n_parts && branch_b) && ((dtype == CIE_F32 && wide(16)) || (dtype == CIE_BF16 && wide(8)))) {
         const int threads = min(1024, (hidden / 4 + kWave - 1) / kWave * kWave);
 #define CIE_DEPTH4(T, AHEAD)                                                                                          \
-    if (n_parts && branch_b) CIE_DEPTH(depth_stream_vec4_kernel, T, 2, true, AHEAD);                                   \
-    else if (n_parts) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, true, AHEAD);                                          \
+    if (n_parts) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, true, AHEAD);                                          \
     else if (branch_b) CIE_DEPTH(depth_stream_vec4_kernel, T, 2, false, AHEAD);                                        \
     else if (branch_a) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, false, AHEAD);                                        \
     else CIE_DEPTH(depth_stream_vec4_kernel, T, 0, false, AHEAD)
