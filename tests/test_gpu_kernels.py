@@ -229,6 +229,24 @@ def test_add_rmsnorm_sums_parts(ops, dtype, hidden, parts):
     assert torch.equal(stream, whole)
 
 
+@pytest.mark.parametrize("hidden", [8192, 8200, 16384])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_add_rmsnorm_of_wide_rows(ops, dtype, hidden):
+    """Rows of which a thread has one piece of eight, and two (the second waits in LDS): a branch, parts, chosen rows."""
+    stream, weight, branch = rand((5, hidden), torch.float32, 29), rand((hidden,), dtype, 30), rand((5, hidden), dtype, 31)
+    pieces = rand((3, 5, hidden), torch.float32, 32)
+    added = stream + branch.float()
+    whole = added + pieces[0] + pieces[1] + pieces[2]
+    rows = torch.tensor([4, 0], dtype=torch.int32).cuda()
+    for extra, total in ((None, added), (pieces, whole)):
+        expect = plain_qwen2.rms_norm(total, weight.float(), 1e-6)
+        chosen = ops.add_rmsnorm(stream, branch, weight, 1e-6, dtype, rows=rows, parts=extra)
+        torch.testing.assert_close(chosen.float(), expect[[4, 0]], **tol(dtype))
+        left = stream.clone()
+        torch.testing.assert_close(ops.add_rmsnorm(left, branch, weight, 1e-6, dtype, parts=extra).float(), expect, **tol(dtype))
+        assert torch.equal(left, total)
+
+
 def build_cache(dtype, lengths, kv_heads, head_dim, page_size, seed, shuffle=True):
     """Random keys/values for sequences of the given lengths, scattered over the
     pages of a pool in a shuffled order.  Returns pools, block table and the

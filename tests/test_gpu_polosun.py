@@ -432,6 +432,55 @@ def test_layer_boundary_kernel_over_depths_and_widths(dtype, rows, hidden, terms
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,n_parts", [(3, 1), (5, 7), (5, 8), (128, 9), (129, 4), (130, 5), (2, 16)])
+def test_layer_boundary_kernel_that_sums_a_branch_in_parts(dtype, rows, n_parts):
+    """One branch and the parts of another, as a layer whose down product was cut leaves them: as many parts as are asked
+    for at once, one more and one less, in the forms for few rows and for many; the bits of the parts added in order."""
+    from cie_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(5)
+    hidden = 264
+    x, a = torch.randn(rows, hidden, generator=g).cuda(), torch.randn(rows, hidden, generator=g).to(dtype).cuda()
+    parts, weights = torch.randn(n_parts, rows, hidden, generator=g).cuda(), torch.randn(3, generator=g).cuda()
+    history = torch.randn(3, rows, hidden, generator=g).cuda()
+    kept = history.clone()
+    stream, normed = ops.depth_stream(x, a, None, mult=0.5, history=history, newest=2, weights=weights, gains=(1.5,), out_dtype=dtype,
+                                      eps=1e-5, parts=parts)
+    branch = a.float()
+    for part in parts:
+        branch = branch + part
+    assert torch.equal(history[2], x + 0.5 * branch) and torch.equal(history[:2], kept[:2])  # (half of it is exact)
+    want = sum(weights[j].double() * history[j].double() for j in range(3))
+    # three roundings of half a unit in the last place of sums whose terms stay below 64
+    assert torch.all((stream.double() - want).abs() <= 3 * 2.0 ** -24 * 64.0)
+    unit = want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-5)
+    tol = 1e-5 if dtype == torch.float32 else 2e-2
+    assert torch.allclose(normed[0].double(), unit * 1.5, atol=tol, rtol=tol)
+
+
+@pytest.mark.parametrize("captured", [False, True])
+def test_a_layer_whose_down_product_comes_in_parts(monkeypatch, captured):
+    """A feed-forward wide enough for its down product to be cut (few rows: the streaming kernel's parts; 150 rows: the
+    tiles'), against the plain implementation."""
+    from cie_amd.parts import linear
+
+    raw = pu.single({"type": "rglru", "mlp": {"kind": "dense", "ff": 4104}, "mixer": {"width": 16, "blocks": 2, "conv": 4}}, width=64)
+    weights = pu.make_weights(raw, seed=6)
+    requests = {"a": random_tokens(150, raw["vocab"], 1), "b": random_tokens(21, raw["vocab"], 2), "c": [7, 3]}
+    plain = plain_all(raw, weights, requests)
+    seen, parts_of = [], linear.KParts.__init__
+    monkeypatch.setattr(linear.KParts, "__init__", lambda self, parts: (seen.append(parts.shape[:2]), parts_of(self, parts))[1])
+    monkeypatch.setattr(linear, "plan_tiles", lambda rows, n, k, most_parts=1, behind_us=0.0: (64, 64, 3) if most_parts > 1 and k > 4000 else None)
+    steps = replay_util.fixed_portions(requests, portion=150, live=3, decode_tail=8) if captured else replay_util.tail_one_by_one(requests, tail=8)
+    pool = max(replay_util.max_live_tokens(steps, page=16), 16)
+    runner = pu.make_runner(raw, weights, "bfloat16", pool, 16, 4, graph_decode=captured)
+    rows = replay_util.by_position(steps, replay_util.drive_runner(runner, steps))
+    worst, rms = pu.spread(rows, plain)
+    assert worst <= LIMIT["bfloat16"] and rms <= RMS_LIMIT["bfloat16"], (worst, rms)
+    assert any(parts > 1 and count <= 128 for parts, count in seen) and any(parts == 3 and count > 128 for parts, count in seen), seen
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("lengths,channels,taps,segments", [
     ((64, 1, 129), 48, 4, 64), ((63, 65), 16, 4, 64), ((2048,), 128, 4, 64), ((2049, 70), 40, 3, 64), ((4100,), 16, 4, 64),
     ((300, 5), 24, 4, 2), ((97,), 40, 4, 16), ((9, 2, 3), 72, 4, 1)])
