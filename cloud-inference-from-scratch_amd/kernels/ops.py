@@ -32,6 +32,10 @@ _COMPUTE_UNITS: dict[int, int] = {}
 def compute_units(device: "torch.device | int | None" = None) -> int:
     """Compute units of the GPU the kernels run on, asked of the device once (the plans that spread
     workgroups over the units are made from it); 256, an MI355X's, where no GPU is visible."""
+    if device is None and _COMPUTE_UNITS:  # (asked several times a layer)
+        known = _COMPUTE_UNITS.get(torch._C._cuda_getDevice())
+        if known is not None:
+            return known
     if not torch.cuda.is_available():
         return 256
     index = torch.cuda.current_device() if device is None else torch.device(device).index if not isinstance(device, int) else device

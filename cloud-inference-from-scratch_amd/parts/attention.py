@@ -23,10 +23,7 @@ from ..config.specs import PartSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import Part, build_part, register_part
-from .linear import FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, behind, linear, plan_tiles, takes_tiles
-
-
-ROTATION_US = (1.1, 1.8)  # the rotation's kernel behind the library's q/k/v product: us, and us per million numbers
+from .linear import BEHIND_ROTATION, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, linear, plan_tiles, takes_tiles
 
 
 class Attention(Part):
@@ -146,7 +143,7 @@ class Attention(Part):
         fused = (x.dtype == torch.bfloat16 and untouched and head_dim % 32 == 0
                  and x.shape[1] % 8 == 0 and (rows == 1 or x.stride(0) % 8 == 0))
         # (the tiles' epilogue saves the rotation's kernel)
-        tiles = (plan_tiles(rows, self.w_qkv.shape[0], x.shape[1], behind_us=behind(ROTATION_US, rows, self.w_qkv.shape[0]))
+        tiles = (plan_tiles(rows, self.w_qkv.shape[0], x.shape[1], behind=BEHIND_ROTATION)
                  if fused and not few and takes_tiles(rows, x, self.w_qkv) else None)
         if tiles is not None:
             qkv = ops.gemm_tiles_rope(self.w_qkv, x, self.b_qkv, self.cos, self.sin, batch.positions, batch.seq_of_token,

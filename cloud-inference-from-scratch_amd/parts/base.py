@@ -35,6 +35,7 @@ Interfaces (``x`` is ``[tokens, hidden]`` in the engine's activation dtype,
 
 from __future__ import annotations
 
+import functools
 from typing import Any, Callable
 
 import torch
@@ -77,7 +78,12 @@ def declares(part: Any, flag: str) -> bool:
     """Whether ``flag`` holds for the ``forward`` that ``part`` runs: what its class says, unless the class brings a
     ``forward`` of its own and says nothing (a variant written against the plain interface takes no argument and no form
     of a branch that only its base class knows)."""
-    for cls in type(part).__mro__:
+    return _class_declares(type(part), flag)
+
+
+@functools.lru_cache(maxsize=1024)
+def _class_declares(kind: type, flag: str) -> bool:
+    for cls in kind.__mro__:
         if flag in vars(cls):
             return bool(vars(cls)[flag])
         if "forward" in vars(cls):

@@ -118,20 +118,32 @@ XCDS = 8
 LIBRARY_US = (8.6, 1.0, 0.40)
 LIBRARY_RATE, LIBRARY_MOST = 0.85, 1.32
 LIBRARY_TUNED = (1.0, 0.90, 0.85)  # ... and its share of that where its candidates, or all its algorithms, were timed
-# What the library's product costs behind it beyond what the tiles' epilogue does: us, and us per million numbers of the
-# product: the gate's kernel; the branch, which is rounded, written and read again by the norm.
-GATE_US = (2.15, 1.2)
-BRANCH_US = (-1.3, 1.9)
-# The tiles are taken where they are modelled to be faster by this: tiles of up to 25 us, and longer ones, where a good
-# algorithm that the library happens to have costs more.  Of the products 25 are then more than 2 % slower than the
-# library's would be (the worst 1.25, the 72B down at 360 rows), and all together 6.3 % faster, 1.4 % from the better of
-# the two each time; with 1.07 for all of them 31, 6.3 and 1.4 %, with 1.15 9, 6.1 and 1.6 %.
-TILES_MARGIN, TILES_SHORT_US, TILES_MARGIN_LONG = 1.05, 25.0, 1.12
+@dataclass(frozen=True, eq=False)
+class Behind:
+    """What the library's product costs beyond what the tiles and their epilogue do.  ``us`` and ``us_per_million`` numbers of
+    the product: the kernel behind it, or the branch that is rounded, written and read again.  ``host_us``: a step of more
+    than 128 rows runs launch by launch, and where a layer's kernels together take less than some 120 us the host is the
+    slower side: the library's call costs it 3 us more than the tiles', a kernel behind it 8.  ``host_upto`` (us of the
+    tiles) is where the layer around such a product has that length; beyond it the GPU is the slower side.
+
+    Whole prompts, 12 layers, without regard for the host and with it, us: 0.5B shape, 400 rows 1,622, 1,330; 800 1,698,
+    1,317; 1,500 1,698, 1,646; 3B shape, 150 rows 1,714, 1,411; 800 2,932, 2,819."""
+
+    us: float
+    us_per_million: float
+    host_us: float
+    host_upto: float
 
 
-def behind(us: tuple[float, float], rows: int, n: int) -> float:
-    """What ``plan_tiles`` is given as ``behind_us`` for a product of ``rows`` x ``n``."""
-    return us[0] + us[1] * rows * n * 1e-6
+BEHIND_NOTHING = Behind(0.0, 0.0, 3.0, 15.0)
+BEHIND_GATE = Behind(2.15, 1.2, 11.0, 40.0)      # the gate's kernel
+BEHIND_BRANCH = Behind(-1.3, 1.9, 3.0, 15.0)     # the norm that adds the branch
+BEHIND_ROTATION = Behind(1.1, 1.8, 11.0, 21.0)   # the rotation and cache write
+# Where the host does not matter the tiles are taken if they are modelled to be faster by the first of these, beyond 25 us by the
+# second (a good algorithm that the library happens to have costs more there).  Of the 608 products 32 are then more than
+# 2 % slower than the library's inside a captured chain (the worst 1.25, the 72B down at 360 rows), and all together 6.4 %
+# faster, 1.3 % from the better of the two each time.
+TILES_MARGIN, TILES_MARGIN_LONG, TILES_LONG_US = 1.05, 1.12, 25.0
 
 
 def _tile_us(columns: int, tile_rows: int, parts: int, rows: int, n: int, k: int, units: int) -> float:
@@ -150,18 +162,21 @@ def _library_us(rows: int, n: int, k: int, units: int, tuned: int) -> float:
 
 
 @functools.lru_cache(maxsize=4096)
-def _plan_tiles(rows: int, n: int, k: int, most_parts: int, behind_us: float, units: int, tuned: int) -> Optional[tuple[int, int, int]]:
+def _plan_tiles(rows: int, n: int, k: int, most_parts: int, behind: Behind, units: int,
+                searched: frozenset) -> Optional[tuple[int, int, int]]:
     forms = [(columns, tile_rows, parts) for columns, tile_rows in TILE_US for parts in TILE_PARTS
              if parts <= most_parts and -(-(-(-k // parts)) // 64) * 64 * (parts - 1) < k]  # (every part has some of K)
     cost, form = min((_tile_us(*form, rows, n, k, units), form) for form in forms)
-    margin = TILES_MARGIN if cost <= TILES_SHORT_US else TILES_MARGIN_LONG
-    return form if cost * margin < _library_us(rows, n, k, units, tuned) + behind_us else None
+    library = _library_us(rows, n, k, units, ops._tune_level(rows)) + behind.us + behind.us_per_million * rows * n * 1e-6
+    if cost <= behind.host_upto:
+        return form if cost * TILES_MARGIN < library + behind.host_us else None
+    return form if cost * (TILES_MARGIN if cost <= TILES_LONG_US else TILES_MARGIN_LONG) < library else None
 
 
-def plan_tiles(rows: int, n: int, k: int, most_parts: int = 1, behind_us: float = 0.0) -> Optional[tuple[int, int, int]]:
+def plan_tiles(rows: int, n: int, k: int, most_parts: int = 1, behind: Behind = BEHIND_NOTHING) -> Optional[tuple[int, int, int]]:
     """(columns, rows, parts of K) of the tiles that a bfloat16 product of some hundred rows takes, or ``None`` where the
-    library's product (and a kernel of ``behind_us`` behind it, which the tiles' epilogue would save) is the faster one."""
-    return _plan_tiles(rows, n, k, most_parts, behind_us, ops.compute_units(), ops._tune_level(rows))
+    library's product, with what it costs ``behind`` it, is the faster one."""
+    return _plan_tiles(rows, n, k, most_parts, behind, ops.compute_units(), ops._search_rows)
 
 
 @dataclass
@@ -404,14 +419,14 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
     if fusable and not wants_f32 and takes_tiles(rows, x, weight, into):
         tiles = None
         if into is not None and not silu and into.is_contiguous() and tuple(into.shape) == (rows, n):
-            tiles = plan_tiles(rows, n, k, most_parts=TILE_PARTS[-1] if sums_parts else 1, behind_us=behind(BRANCH_US, rows, n))
+            tiles = plan_tiles(rows, n, k, most_parts=TILE_PARTS[-1] if sums_parts else 1, behind=BEHIND_BRANCH)
             if tiles is not None and tiles[2] > 1:
                 return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, *tiles[:2], bias=bias, parts=tiles[2]))
             if tiles is not None:
                 ops.gemm_tiles(weight, ops.TILE_RESID, x, *tiles[:2], bias=bias, into=into)
                 return Added()
         elif into is None and silu and n % 2 == 0 and bias is None:
-            tiles = plan_tiles(rows, n, k, behind_us=behind(GATE_US, rows, n))
+            tiles = plan_tiles(rows, n, k, behind=BEHIND_GATE)
             if tiles is not None:
                 return ops.gemm_tiles(weight, ops.TILE_SILU, x, *tiles[:2])
         elif into is None and not silu:

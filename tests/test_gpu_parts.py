@@ -1197,7 +1197,7 @@ def test_parts_of_k_reach_a_layer_that_adds_rows(norm, monkeypatch):
     from cie_amd.parts.block import PreNormBlock
     from cie_amd.parts.linear import KParts
 
-    monkeypatch.setattr(linear, "plan_tiles", lambda rows, n, k, most_parts=1, behind_us=0.0: (64, 64, 2) if most_parts > 1 and k > 64 else None)
+    monkeypatch.setattr(linear, "plan_tiles", lambda rows, n, k, most_parts=1, behind=None: (64, 64, 2) if most_parts > 1 and k > 64 else None)
     rows, hidden = 200, 64
     raw = dict(model_type="qwen2", hidden_size=hidden, num_hidden_layers=2, num_attention_heads=2, num_key_value_heads=1,
                intermediate_size=136, vocab_size=32, rms_norm_eps=1e-5, rope_theta=1e4, max_position_embeddings=256)
@@ -1231,7 +1231,7 @@ def test_a_feed_forward_with_a_forward_of_its_own_runs_in_a_layer(monkeypatch):
         def forward(self, x, residual=None):
             return super().forward(x) * 2
 
-    monkeypatch.setattr(linear, "plan_tiles", lambda rows, n, k, most_parts=1, behind_us=0.0: (64, 64, 2) if most_parts > 1 and k > 64 else None)
+    monkeypatch.setattr(linear, "plan_tiles", lambda rows, n, k, most_parts=1, behind=None: (64, 64, 2) if most_parts > 1 and k > 64 else None)
     raw = dict(model_type="qwen2", hidden_size=64, num_hidden_layers=1, num_attention_heads=2, num_key_value_heads=1,
                intermediate_size=136, vocab_size=32, rms_norm_eps=1e-5, rope_theta=1e4, max_position_embeddings=256)
     block = PreNormBlock(Qwen2Config.from_hf_config(raw).model_spec().layers[0])

@@ -470,7 +470,7 @@ def test_a_layer_whose_down_product_comes_in_parts(monkeypatch, captured):
     plain = plain_all(raw, weights, requests)
     seen, parts_of = [], linear.KParts.__init__
     monkeypatch.setattr(linear.KParts, "__init__", lambda self, parts: (seen.append(parts.shape[:2]), parts_of(self, parts))[1])
-    monkeypatch.setattr(linear, "plan_tiles", lambda rows, n, k, most_parts=1, behind_us=0.0: (64, 64, 3) if most_parts > 1 and k > 4000 else None)
+    monkeypatch.setattr(linear, "plan_tiles", lambda rows, n, k, most_parts=1, behind=None: (64, 64, 3) if most_parts > 1 and k > 4000 else None)
     steps = replay_util.fixed_portions(requests, portion=150, live=3, decode_tail=8) if captured else replay_util.tail_one_by_one(requests, tail=8)
     pool = max(replay_util.max_live_tokens(steps, page=16), 16)
     runner = pu.make_runner(raw, weights, "bfloat16", pool, 16, 4, graph_decode=captured)

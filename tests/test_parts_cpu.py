@@ -134,7 +134,7 @@ MEASURED = [
 
 @pytest.mark.parametrize("what,rows,n,k,library,tiles", MEASURED)
 def test_tiles_are_not_taken_where_they_were_measured_to_lose(what, rows, n, k, library, tiles):
-    from cie_amd.parts.linear import BRANCH_US, behind, plan_tiles
+    from cie_amd.parts.linear import BEHIND_BRANCH, plan_tiles
 
-    picked = plan_tiles(rows, n, k, most_parts=8, behind_us=behind(BRANCH_US, rows, n))
+    picked = plan_tiles(rows, n, k, most_parts=8, behind=BEHIND_BRANCH)
     assert picked is None or tiles[picked] <= 1.03 * library
