@@ -837,7 +837,7 @@ gated_recurrence_kernel(const T* __restrict__ y_pre, long ldy, const T* __restri
 //
 // What bounds it is the way to memory: 14 bytes a token and channel, and a thread that waits for one token's loads at a
 // time waits some hundred times.  So a stretch is short, its a_t and x_t stay in registers between the walks (no second
-// read, no second exponential and root), and eight tokens' loads travel together.  16 channels a workgroup, and
+// read, no second exponential and root), and four tokens' loads travel together.  16 channels a workgroup, and
 // neighbouring workgroups' channels on one XCD, whose L2 then serves both halves of a 128-byte line.  1,999 tokens of 2,048
 // channels: 107 us in 16 stretches that were read twice, 44 in 64 stretches (16 us is the memory's part).
 constexpr int kMaxSegments = 64;

@@ -211,7 +211,9 @@ class MixedGraphs:
 
     Such a step is a few hundred launches too, and with few tokens the host cannot queue them as fast as the
     GPU runs them (8 decode rows and a 32-token portion of the 3B shape: 4.1 ms launch by launch, 3.6 ms
-    replayed; with a 64-token portion 4.4 and 4.2 ms; with 256 tokens the GPU is the slower one either way).  A capture costs as
+    replayed; with a 64-token portion 4.4 and 4.2 ms).  Larger steps gain less and their graphs keep more memory (12 layers
+    of the 3B shape, eight decode rows and a portion, launch by launch and replayed, ms: 128 rows 1.84, 1.70; 200 rows 1.99,
+    1.83; 256 rows 1.88, 1.85; 512 rows 2.51, 2.44): they are not captured.  A capture costs as
     much as ten such steps, so only shapes that come again are captured: a step's shape is (bucket of its
     single-token rows, the lengths of its portions); one that comes a second time (the portions of one
     long prompt beside the same decoding requests do) is captured, on rows of padding, and replayed from
@@ -220,7 +222,7 @@ class MixedGraphs:
     ``limit`` are dropped.  The reference captures decode steps only (src/cloud_engine/engine.py:316-437)."""
 
     MAX_PORTIONS = 4
-    MAX_TOKENS = 128  # rows of a step (decode bucket and portions) up to which the host is the slower side
+    MAX_TOKENS = 128  # rows of a step (decode bucket and portions) up to which it is captured
 
     def __init__(self, runner: Any, decode_graphs: "DecodeGraphs", limit: int) -> None:
         self.runner = runner

@@ -263,7 +263,10 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
         # (64 sequences x 2 heads x 256 keys: 9.2 us against 11.1 us with one wave per part).  A second part pays for
         # its merge where a unit has more to read than MANY_PART_BYTES (64 x 2 heads of 128, us, whole against two
         # parts: 512 keys 12.5, 15.5; 1,024 keys 20.2, 21.5; 1,200 keys 24.7, 24.1; 1,536 keys 29.6, 28.0; 48 x 2
-        # heads: 700 keys 14.8, 15.7; 1,024 keys 19.8, 18.8; 64 x 2 heads of 64: 1,280 keys 14.1, 16.5).
+        # heads: 700 keys 14.8, 15.7; 1,024 keys 19.8, 18.8; 64 x 2 heads of 64: 1,280 keys 14.1, 16.5; the two parts
+        # joined by a workgroup a row).  A captured step's bound is the longest context it may ever see: a limit of
+        # WIDE_DECODE_KEYS and more has the form above, with 1,000 keys as with many (64 x 2 heads of 128 over 1,000 keys:
+        # 19 us at a bound of 1,000, 22 at 4,096).
         if wide and units >= MANY_DECODE_UNITS and bound >= SHARED_DECODE_KEYS:
             return ops.TILE_WAVES, dict(target_waves=4 * cus // ops.TILE_WAVES,
                                         min_keys=max(512, MANY_PART_BYTES // (4 * head_dim)))
