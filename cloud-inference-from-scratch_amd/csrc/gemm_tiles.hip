@@ -18,7 +18,7 @@
 // What bounds it: few tiles, the chain of one tile's slices (0.28 to 0.94 us each); many, the rate at which a unit is fed
 // from its L2, some 20 bytes a cycle in every shape of tile (2,048 rows, N 22,016, K 2,048: the matrix cores busy 31 % of
 // the time, LDS 31 %, no bank conflicts; 128 x 128 tiles 0.84 PFLOP/s, where the library's tiles of 256 x 256, fed at the
-// same rate, reach 1.2: 256 x 256 from this source spills).  Reading LDS for the next half slice while the matrix cores
+// same rate, reach 1.2: 256 x 256 spills here while its slices wait in registers).  Reading LDS for the next half slice while the matrix cores
 // work on this one gave 0-20 % where a unit holds one tile (qkv 128 x 64 22.5 -> 17.5 us) and nothing where it holds many.
 //
 // Measured (MI355X, 3B shape, us; the library's product, and the kernel behind it, in brackets): 256 rows: down in 4 parts
