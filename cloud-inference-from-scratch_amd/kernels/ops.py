@@ -861,6 +861,16 @@ def folds_norm(rows: int, k: int) -> bool:
 
 TILE_BF16, TILE_SILU, TILE_RESID, TILE_PARTS = 0, 1, 2, 3
 TILE_SHAPES = ((64, 64), (128, 64), (128, 128), (128, 256))  # columns x rows of a workgroup's tile
+# ... of the kernel whose operands go straight into LDS (K a multiple of 64)
+DIRECT_SHAPES = ((64, 64), (96, 64), (96, 128), (128, 64), (128, 128), (128, 192), (128, 256), (192, 128), (192, 192),
+                 (192, 256), (256, 128), (256, 160), (256, 256))
+DIRECT_SLICE = 64
+DIRECT_NUMBERS = 1 << 31  # an operand holds fewer numbers (their places are 32-bit numbers of bytes)
+
+
+def direct_fits(rows: int, n: int, k: int, lda: int) -> bool:
+    """Whether the kernel that loads straight into LDS takes a product of these sizes."""
+    return k % DIRECT_SLICE == 0 and n * k < DIRECT_NUMBERS and rows * lda < DIRECT_NUMBERS
 
 
 def _tile_rows(a: torch.Tensor, weight: torch.Tensor) -> tuple[int, int, int, int]:
@@ -878,14 +888,23 @@ def _tile_rows(a: torch.Tensor, weight: torch.Tensor) -> tuple[int, int, int, in
     return m, n, k, lda
 
 
+def _check_tile_shape(columns: int, rows: int, direct: bool, m: int, n: int, k: int, lda: int) -> None:
+    shapes = DIRECT_SHAPES if direct else TILE_SHAPES
+    if (columns, rows) not in shapes:
+        raise ValueError(f"tiles are one of {shapes}, not {(columns, rows)}")
+    if direct and not direct_fits(m, n, k, lda):
+        raise ValueError(f"{m} x {n} x {k} with row stride {lda}: K is a multiple of {DIRECT_SLICE}, an operand below 2^31 numbers")
+
+
 def gemm_tiles(weight: torch.Tensor, epilogue: int, a: torch.Tensor, columns: int, rows: int,
-               bias: Optional[torch.Tensor] = None, into: Optional[torch.Tensor] = None, parts: int = 1) -> torch.Tensor:
+               bias: Optional[torch.Tensor] = None, into: Optional[torch.Tensor] = None, parts: int = 1,
+               direct: bool = False) -> torch.Tensor:
     """``a @ weight.T + bias`` in bfloat16 for some hundred rows, in tiles of ``columns`` x ``rows``: the bf16 result, its
     gated unit (``TILE_SILU``), added in place to the float32 stream ``into`` (``TILE_RESID``), or K in ``parts`` parts
-    whose float32 sums come back as [parts, M, N] (``TILE_PARTS``)."""
+    whose float32 sums come back as [parts, M, N] (``TILE_PARTS``).  ``direct``: by the kernel that loads its operands
+    straight into LDS (``DIRECT_SHAPES``; K a multiple of 64)."""
     m, n, k, lda = _tile_rows(a, weight)
-    if (columns, rows) not in TILE_SHAPES:
-        raise ValueError(f"tiles are one of {TILE_SHAPES}, not {(columns, rows)}")
+    _check_tile_shape(columns, rows, direct, m, n, k, lda)
     if bias is not None:
         _gpu("bias", bias, torch.bfloat16, 1)
         if not (bias.shape[0] == n and epilogue != TILE_SILU):
@@ -899,7 +918,8 @@ def gemm_tiles(weight: torch.Tensor, epilogue: int, a: torch.Tensor, columns: in
         out = torch.empty((parts, m, n), dtype=torch.float32, device=a.device)
     else:
         out = torch.empty((m, n // 2 if epilogue == TILE_SILU else n), dtype=torch.bfloat16, device=a.device)
-    _run("cie_gemm_tiles", load_library().cie_gemm_tiles(
+    entry = "cie_gemm_direct" if direct else "cie_gemm_tiles"
+    _run(entry, getattr(load_library(), entry)(
         _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(out), _i(out.shape[-1]), _i(m), _i(n), _i(k), _i(epilogue),
         _i(columns), _i(rows), _i(parts)))
     return out
@@ -908,10 +928,13 @@ def gemm_tiles(weight: torch.Tensor, epilogue: int, a: torch.Tensor, columns: in
 def gemm_tiles_rope(weight: torch.Tensor, a: torch.Tensor, bias: Optional[torch.Tensor], cos: torch.Tensor,
                     sin: torch.Tensor, positions: torch.Tensor, seq_of_token: torch.Tensor, seq_slot: torch.Tensor,
                     block_table: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, q_heads: int, kv_heads: int,
-                    head_dim: int, columns: int, rows: int, rotate: bool = True, write_kv: bool = True) -> torch.Tensor:
-    """What :func:`gemm_qkv_rope` does, for some hundred rows in tiles of ``columns`` x ``rows``."""
+                    head_dim: int, columns: int, rows: int, rotate: bool = True, write_kv: bool = True,
+                    direct: bool = False) -> torch.Tensor:
+    """What :func:`gemm_qkv_rope` does, for some hundred rows in tiles of ``columns`` x ``rows`` (``direct``: as in
+    :func:`gemm_tiles`)."""
     m, n, k, lda = _tile_rows(a, weight)
-    if (columns, rows) not in TILE_SHAPES or head_dim % 32 or n != (q_heads + 2 * kv_heads) * head_dim:
+    _check_tile_shape(columns, rows, direct, m, n, k, lda)
+    if head_dim % 32 or n != (q_heads + 2 * kv_heads) * head_dim:
         raise ValueError(f"tiles of {columns} x {rows}, heads of {head_dim}, {n} weight rows do not fit")
     if bias is not None:
         _gpu("bias", bias, torch.bfloat16, 1)
@@ -929,7 +952,8 @@ def gemm_tiles_rope(weight: torch.Tensor, a: torch.Tensor, bias: Optional[torch.
     _gpu("block_table", block_table, torch.int32, 2)
     page_size = _check_pools(k_pool, v_pool, torch.bfloat16, kv_heads, head_dim)
     out = torch.empty((m, n), dtype=torch.bfloat16, device=a.device)
-    _run("cie_gemm_tiles_rope", load_library().cie_gemm_tiles_rope(
+    entry = "cie_gemm_direct_rope" if direct else "cie_gemm_tiles_rope"
+    _run(entry, getattr(load_library(), entry)(
         _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k), _i(columns), _i(rows),
         _ptr(cos), _ptr(sin), _ptr(positions), _ptr(seq_of_token), _ptr(seq_slot), _ptr(block_table),
         _i(block_table.shape[1]), _ptr(k_pool), _ptr(v_pool), _i(q_heads), _i(kv_heads), _i(head_dim), _i(page_size),

@@ -23,7 +23,7 @@ from ..config.specs import PartSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import Part, build_part, register_part
-from .linear import BEHIND_ROTATION, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, linear, plan_tiles, takes_tiles
+from .linear import BEHIND_ROTATION, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, choose_tiles, linear, takes_tiles
 
 
 class Attention(Part):
@@ -143,12 +143,13 @@ class Attention(Part):
         fused = (x.dtype == torch.bfloat16 and untouched and head_dim % 32 == 0
                  and x.shape[1] % 8 == 0 and (rows == 1 or x.stride(0) % 8 == 0))
         # (the tiles' epilogue saves the rotation's kernel)
-        tiles = (plan_tiles(rows, self.w_qkv.shape[0], x.shape[1], behind=BEHIND_ROTATION)
+        tiles = (choose_tiles(rows, self.w_qkv.shape[0], x.shape[1], x.stride(0), behind=BEHIND_ROTATION)
                  if fused and not few and takes_tiles(rows, x, self.w_qkv) else None)
         if tiles is not None:
             qkv = ops.gemm_tiles_rope(self.w_qkv, x, self.b_qkv, self.cos, self.sin, batch.positions, batch.seq_of_token,
                                       batch.seq_slot, view.block_table, view.k_pool, view.v_pool, self.num_heads,
-                                      self.num_kv_heads, head_dim, *tiles[:2], rotate=self.position.rotates, write_kv=writes)
+                                      self.num_kv_heads, head_dim, tiles.columns, tiles.rows,
+                                      rotate=self.position.rotates, write_kv=writes, direct=tiles.direct)
         elif fused and few:
             # few rows (where the hand-written product is the faster one): its epilogue rotates and writes the cache
             qkv = ops.gemm_qkv_rope(self.w_qkv, x, self.b_qkv, self.cos, self.sin, batch.positions,

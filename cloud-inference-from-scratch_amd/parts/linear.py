@@ -10,8 +10,8 @@ residual stream (``into=residual``), or float32 results for the logits.  They
 come in two forms: waves that share K and own all rows (few rows; the q/k/v,
 o_proj and head products), and waves that own columns and share the rows through
 LDS (the SiLU-gate product up to 64 rows and every product whose K is cut).
-bfloat16 with more rows: tiles of this package's own (``csrc/gemm_tiles.hip``) where
-few tiles or a kernel behind the product would cost the library more, else the
+bfloat16 with more rows: tiles of this package's own (``csrc/gemm_direct.hip``, and
+``csrc/gemm_tiles.hip`` for a K that is no multiple of 64) where they are the faster ones, else the
 vendor library's product (hipBLASLt through a thin cached interface of this
 package), as the reference leaves its products to a library
 (src/cloud_engine/model.py:89-137), with the small kernels around it.
@@ -23,7 +23,7 @@ import functools
 import math
 import weakref
 from dataclasses import dataclass
-from typing import Any, Optional, Union
+from typing import Any, NamedTuple, Optional, Union
 
 import torch
 
@@ -100,7 +100,7 @@ def plan_shared_parts(tiles: int, k: int) -> tuple[int, int, int]:
 
 
 # Products of more rows than the kernels above take (beyond ``FUSED_PARTS_ROWS``) go to tiles of this package or to the
-# vendor library, whichever the two models below say is faster.  Both are fitted to 608 products timed inside captured
+# vendor library, whichever the models below say is faster.  These two are fitted to 608 products timed inside captured
 # chains on MI355X with the kernels between them (q/k/v, o_proj, gate/up and down of six shapes from 896 to 8,192 wide, at
 # 16 to 30 row counts from 130 to 2,048).
 # Tiles (within 6 % of the measured, root mean square), us: a start, and per slice of 64 k of a workgroup alone on its unit
@@ -148,8 +148,8 @@ BEHIND_ROTATION = Behind(1.1, 1.8, 11.0, 21.0)   # the rotation and cache write
 TILES_MARGIN, TILES_MARGIN_LONG, TILES_LONG_US = 1.05, 1.15, 25.0
 
 
-def _tile_us(columns: int, tile_rows: int, parts: int, rows: int, n: int, k: int, units: int) -> float:
-    start, first, further = TILE_US[columns, tile_rows]
+def _tile_us(columns: int, tile_rows: int, parts: int, rows: int, n: int, k: int, units: int, times: dict = TILE_US) -> float:
+    start, first, further = times[columns, tile_rows]
     tiles = -(-rows // tile_rows) * -(-n // columns)
     turns = -(-(-(-tiles // XCDS) * parts) // max(1, units // XCDS))
     slices = -(-(-(-k // parts)) // 64)
@@ -161,6 +161,25 @@ def _library_us(rows: int, n: int, k: int, units: int, tuned: int) -> float:
     rate = min(LIBRARY_MOST, LIBRARY_RATE * share ** (0.46 if share < 1.0 else 0.51))
     start, per_k, per_weight = LIBRARY_US
     return LIBRARY_TUNED[tuned] * math.hypot(start + per_k * 1e-3 * k + per_weight * 1e-6 * n * k, 2e-9 * rows * n * k / rate)
+
+
+# The tiles whose operands go straight into LDS (csrc/gemm_direct.hip; K a multiple of 64), by the same model, fitted to 7,500
+# timings (0.5B, 3B, 7B and 14B widths at 16 row counts from 112 to 2,048; 10 % root mean square): the form it picks takes
+# 1.7 % more than the best of all in the mean.  Against the tiles above and the library, us, each product alone (the kernel
+# behind the library's not counted): 3B gate/up 256 rows 40 -> 33, 777 81 -> 72, 2,048 186 -> 157; down 613 47 -> 36, 2,048
+# 100 -> 91; 7B gate/up 777 272 -> 175, 2,048 541 -> 445, down 777 167 -> 98.  What decides is how the turns come out: 777 rows
+# x 37,888 are 740 tiles of 256 x 160, three turns of 256 units, and 1,036 of 256 x 128, five.
+DIRECT_US = {(64, 64): (3.1, 0.239, 0.246), (96, 64): (3.4, 0.301, 0.299), (96, 128): (5.3, 0.390, 0.494),
+             (128, 64): (3.0, 0.405, 0.340), (128, 128): (4.8, 0.467, 0.554), (128, 192): (5.4, 0.577, 0.671),
+             (128, 256): (6.8, 0.662, 0.821), (192, 128): (5.7, 0.604, 0.684), (192, 192): (7.3, 0.713, 0.856),
+             (192, 256): (6.9, 1.078, 1.208), (256, 128): (6.2, 0.750, 0.854), (256, 160): (7.7, 0.826, 0.977),
+             (256, 256): (8.1, 1.299, 1.481)}
+# Of the forms within this share of the fastest the one that reads least: level in the timings, less power inside a step (3B
+# gate/up of 2,048 rows, tiles of 192 x 192 that the model prefers by 3 %: 161 us alone, 174 inside a prompt).
+DIRECT_LEVEL = 1.04
+DIRECT_MARGIN = 1.03  # ... taken where they are modelled to be faster than the library by this
+# Sums of K in parts are at most this many bytes (2,048 rows: 4 parts of the 3B shape's down product 67 MB, 2 of 7B's 59)
+PARTS_BYTES = 128 << 20
 
 
 @functools.lru_cache(maxsize=4096)
@@ -179,6 +198,39 @@ def plan_tiles(rows: int, n: int, k: int, most_parts: int = 1, behind: Behind = 
     """(columns, rows, parts of K) of the tiles that a bfloat16 product of some hundred rows takes, or ``None`` where the
     library's product, with what it costs ``behind`` it, is the faster one."""
     return _plan_tiles(rows, n, k, most_parts, behind, ops.compute_units(), ops._search_rows)
+
+
+class Tiles(NamedTuple):
+    """How a product of many rows runs: tiles of ``columns`` x ``rows``, K in ``parts`` parts, and whether its operands go
+    straight into LDS."""
+
+    columns: int
+    rows: int
+    parts: int
+    direct: bool
+
+
+@functools.lru_cache(maxsize=4096)
+def _choose_direct(rows: int, n: int, k: int, most_parts: int, behind: Behind, units: int, searched: frozenset) -> Optional[Tiles]:
+    forms = [(columns, tile_rows, parts) for columns, tile_rows in DIRECT_US for parts in TILE_PARTS
+             if parts <= most_parts and -(-(-(-k // parts)) // 64) * 64 * (parts - 1) < k
+             and (parts == 1 or parts * rows * n * 4 <= PARTS_BYTES)]
+    times = {form: _tile_us(*form, rows, n, k, units, DIRECT_US) for form in forms}
+    cost = min(times.values())
+    reads = lambda f: (-(-rows // f[1]) * -(-n // f[0]) * (f[0] + f[1]), f[2])  # noqa: E731
+    form = min((f for f in forms if times[f] <= cost * DIRECT_LEVEL), key=reads)
+    library = _library_us(rows, n, k, units, ops._tune_level(rows)) + behind.us + behind.us_per_million * rows * n * 1e-6
+    library += behind.host_us if cost <= behind.host_upto else 0.0
+    return Tiles(*form, True) if cost * DIRECT_MARGIN < library else None
+
+
+def choose_tiles(rows: int, n: int, k: int, row_stride: int, most_parts: int = 1, behind: Behind = BEHIND_NOTHING) -> Optional[Tiles]:
+    """The tiles that a product of many rows takes, or ``None``: the library.  Whatever fits the kernel that loads straight
+    into LDS is that kernel's or the library's; the other tiles have what is left (a K that is no multiple of 64)."""
+    if ops.direct_fits(rows, n, k, row_stride):
+        return _choose_direct(rows, n, k, most_parts, behind, ops.compute_units(), ops._search_rows)
+    form = plan_tiles(rows, n, k, most_parts=most_parts, behind=behind)
+    return None if form is None else Tiles(*form, False)
 
 
 @dataclass
@@ -419,24 +471,24 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
         elif not silu:
             return ops.gemm_fused(weight, ops.EPI_F32 if wants_f32 else ops.EPI_BF16, x, bias=bias)
     if fusable and not wants_f32 and takes_tiles(rows, x, weight, into):
-        tiles = None
+        stride, most = x.stride(0), TILE_PARTS[-1] if sums_parts else 1
         if into is not None and not silu and into.is_contiguous() and tuple(into.shape) == (rows, n):
-            tiles = plan_tiles(rows, n, k, most_parts=TILE_PARTS[-1] if sums_parts else 1, behind=BEHIND_BRANCH)
-            if tiles is not None and tiles[2] > 1:
-                return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, *tiles[:2], bias=bias, parts=tiles[2]))
+            tiles = choose_tiles(rows, n, k, stride, most_parts=most, behind=BEHIND_BRANCH)
+            if tiles is not None and tiles.parts > 1:
+                return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, tiles.columns, tiles.rows, bias, None, tiles.parts, tiles.direct))
             if tiles is not None:
-                ops.gemm_tiles(weight, ops.TILE_RESID, x, *tiles[:2], bias=bias, into=into)
+                ops.gemm_tiles(weight, ops.TILE_RESID, x, tiles.columns, tiles.rows, bias, into, 1, tiles.direct)
                 return Added()
         elif into is None and silu and n % 2 == 0 and bias is None:
-            tiles = plan_tiles(rows, n, k, behind=BEHIND_GATE)
+            tiles = choose_tiles(rows, n, k, stride, behind=BEHIND_GATE)
             if tiles is not None:
-                return ops.gemm_tiles(weight, ops.TILE_SILU, x, *tiles[:2])
+                return ops.gemm_tiles(weight, ops.TILE_SILU, x, tiles.columns, tiles.rows, None, None, 1, tiles.direct)
         elif into is None and not silu:
-            tiles = plan_tiles(rows, n, k, most_parts=TILE_PARTS[-1] if sums_parts else 1)
-            if tiles is not None and tiles[2] > 1:
-                return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, *tiles[:2], bias=bias, parts=tiles[2]))
+            tiles = choose_tiles(rows, n, k, stride, most_parts=most)
+            if tiles is not None and tiles.parts > 1:
+                return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, tiles.columns, tiles.rows, bias, None, tiles.parts, tiles.direct))
             if tiles is not None:
-                return ops.gemm_tiles(weight, ops.TILE_BF16, x, *tiles[:2], bias=bias)
+                return ops.gemm_tiles(weight, ops.TILE_BF16, x, tiles.columns, tiles.rows, bias, None, 1, tiles.direct)
     if weight.dtype == torch.float32:
         if silu and n % 2 == 0 and bias is None:
             return ops.gemm_f32(x, weight, gate=True)

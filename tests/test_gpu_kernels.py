@@ -186,6 +186,58 @@ def test_gemm_tiles(ops, shape, tile):
             torch.testing.assert_close(got.double().sum(0), product + b.double(), **sums)
 
 
+# (rows, columns, K): a stage or fewer of k, fewer slices than stages, edges of 16 and of the tiles, columns that are no
+# multiple of 8 or of 4, as many slices as the loop takes at once and one more
+@pytest.mark.parametrize("shape", [(1, 32, 64), (63, 64, 128), (65, 130, 192), (129, 256, 320), (200, 99, 448), (257, 100, 512),
+                                   (530, 776, 576)])
+@pytest.mark.parametrize("tile", [(64, 64), (96, 64), (96, 128), (128, 64), (128, 128), (128, 192), (128, 256), (192, 128),
+                                  (192, 192), (192, 256), (256, 128), (256, 160), (256, 256)])
+def test_gemm_direct(ops, shape, tile):
+    """The products of :func:`test_gemm_tiles` by the kernel whose operands go straight into LDS."""
+    m, n, k = shape
+    assert tile in ops.DIRECT_SHAPES
+    wide = torch.zeros((m, k + 24), dtype=torch.bfloat16).cuda()
+    wide[:, :k] = rand((m, k), torch.bfloat16, 16)
+    a, w, b = wide[:, :k], rand((n, k), torch.bfloat16, 17), rand((n,), torch.bfloat16, 18)
+    product = a.double() @ w.double().t()
+    sums = dict(rtol=1e-4, atol=1e-4 * math.sqrt(k))       # float32 sums of k products of numbers about 1
+    rounded = dict(rtol=1e-2, atol=1e-2 * math.sqrt(k))    # ... rounded to bfloat16
+    run = lambda epilogue, **more: ops.gemm_tiles(w, epilogue, a, *tile, direct=True, **more)  # noqa: E731
+    torch.testing.assert_close(run(ops.TILE_BF16, bias=b).double(), product + b.double(), **rounded)
+    if n % 2 == 0:
+        gate, up = product[:, : n // 2], product[:, n // 2:]
+        torch.testing.assert_close(run(ops.TILE_SILU).double(), torch.nn.functional.silu(gate) * up, rtol=1e-2, atol=1e-2 * k)
+    stream = rand((m, n), torch.float32, 19)
+    expect = stream.double() + product + b.double()
+    run(ops.TILE_RESID, bias=b, into=stream)
+    torch.testing.assert_close(stream.double(), expect, **sums)
+    for parts in (1, 2, 3):
+        if (parts - 1) * (-(-(-(-k // parts)) // 64) * 64) < k:  # (every part has some of K)
+            got = run(ops.TILE_PARTS, bias=b, parts=parts)
+            assert got.shape == (parts, m, n)
+            torch.testing.assert_close(got.double().sum(0), product + b.double(), **sums)
+
+
+@pytest.mark.parametrize("heads", [(4, 2, 128), (3, 1, 96), (14, 2, 64), (2, 2, 32)])
+@pytest.mark.parametrize("tile", [(64, 64), (128, 64), (128, 128), (192, 128), (256, 160), (256, 256)])
+def test_gemm_direct_rope(ops, heads, tile):
+    """... and its q/k/v epilogue: the bits of the plain one and the rotation's kernel behind it."""
+    q_heads, kv_heads, dim = heads
+    m, k, page, n = 300, 192, 8, (heads[0] + 2 * heads[1]) * heads[2]
+    a, w, b = rand((m, k), torch.bfloat16, 20), rand((n, k), torch.bfloat16, 21), rand((n,), torch.bfloat16, 22)
+    as_dev = lambda values: torch.tensor(values, dtype=torch.int32).cuda()  # noqa: E731
+    positions, seqs, slots = as_dev(list(range(3, 203)) + list(range(100))), as_dev([0] * 200 + [1] * 100), as_dev([2, 0])
+    table = torch.randperm(96, generator=torch.Generator().manual_seed(23)).to(torch.int32).reshape(3, 32).cuda()
+    cos, sin = rand((256, dim // 2), torch.float32, 24), rand((256, dim // 2), torch.float32, 25)
+    pools = [torch.zeros((96, kv_heads, page, dim), dtype=torch.bfloat16).cuda(), torch.zeros((96, kv_heads, dim, page), dtype=torch.bfloat16).cuda()]
+    plain_pools = [p.clone() for p in pools]
+    got = ops.gemm_tiles_rope(w, a, b, cos, sin, positions, seqs, slots, table, *pools, q_heads, kv_heads, dim, *tile, direct=True)
+    expect = ops.gemm_tiles(w, ops.TILE_BF16, a, *tile, bias=b, direct=True)
+    ops.rope_kv_write(expect, cos, sin, positions, seqs, slots, table, *plain_pools, q_heads, kv_heads, dim)
+    assert torch.equal(got[:, : q_heads * dim], expect[:, : q_heads * dim])
+    assert all(torch.equal(x, y) for x, y in zip(pools, plain_pools))
+
+
 @pytest.mark.parametrize("heads", [(4, 2, 128), (3, 1, 96), (14, 2, 64), (2, 2, 32)])
 @pytest.mark.parametrize("tile", [(64, 64), (128, 64), (128, 128), (128, 256)])
 @pytest.mark.parametrize("rotate,write", [(True, True), (False, True), (True, False)])
