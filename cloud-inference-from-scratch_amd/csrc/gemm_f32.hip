@@ -21,16 +21,19 @@
 //   registers (one slice ahead a tile alone on its unit took twice as long: 89 -> 45 us at 256 rows, N = K = 2,048).
 //   Where the tiles leave units idle a workgroup takes one stretch of K and leaves its sum in a workspace, and
 //   gemm_f32_join_kernel adds the stretches in order.
+//   gemm_f32_direct_kernel: the same tiles, loaded straight into LDS, where a unit takes five and more (goes_direct); the
+//   matrix cores are busy 77 % of its time, with zeros for numbers too, so it is not the power.
 //
 // Measured (MI355X, us): 4 rows: N 22,016, K 2,048 42 (4.3 TB/s), N 2,048, K 11,008 27 (3.4 TB/s), N = K = 2,048 10;
-// 517 rows: 473 (99 TFLOP/s), 264 with K in stretches (88 TFLOP/s; 420 without), 68; 2,048 rows: 1,622 (114 TFLOP/s),
-// 824, 170.  Plain fused multiply-adds in tiles of 64 x 64, whatever the rows, took 370 for the median product of a step
+// 517 rows: 460 (101 TFLOP/s), 256 with K in stretches (91 TFLOP/s; 359 without), 68; 2,048 rows: 1,555 (119 TFLOP/s),
+// 753, 150.  Plain fused multiply-adds in tiles of 64 x 64, whatever the rows, took 370 for the median product of a step
 // of 4 rows and 833 of one of 517 (23 TFLOP/s).
 #include "common.h"
 
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* lds_pointer;
 
 constexpr int kBlockK = 256;   // a block of K: its sum joins the total
 constexpr int kPiece = 32;     // k of a piece: 128 bytes of a row
@@ -366,6 +369,189 @@ gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, c
     }
 }
 
+// The tiles of gemm_f32_direct_kernel: those whose 64 rows are all there, and the last row block's where they are not.
+struct DirectGrid {
+    int whole_blocks, whole, ragged, whole_each, ragged_each;  // (..._each: of an XCD)
+    __host__ __device__ DirectGrid(int M, int row_blocks, int tiles) {
+        const bool ends_early = M % 64 != 0 && row_blocks > 1;
+        const int columns = tiles / row_blocks;
+        whole_blocks = row_blocks - (ends_early ? 1 : 0);
+        whole = columns * whole_blocks;
+        ragged = ends_early ? columns : 0;
+        whole_each = (whole + 7) / 8;
+        ragged_each = (ragged + 7) / 8;
+    }
+    __host__ __device__ int workgroups() const { return 8 * (whole_each + ragged_each); }
+};
+
+// Tiles of 64 x 64 by four waves, two by two, whose operands go straight into LDS: K a multiple of 32.  Four stages of 32 k
+// (16 KB), so that three slices are under way and two workgroups share a unit; one barrier a slice, between its halves of 16
+// k, as in gemm_direct.hip.  A wave whose rows lie partly past M leaves those products out.
+template <bool kGate>
+__global__ void __launch_bounds__(256, 2)
+gemm_f32_direct_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                       float* __restrict__ C, int M, int N, int K, int lda, int ldc, int row_blocks, int tiles,
+                       float* __restrict__ parts) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the host's pass has no type for a buffer's description)
+    constexpr int kN = 2, kM = 2, kStages = 4, kWaves = 4;
+    constexpr int kRows = 32 * (kN + kM), kStageFloats = kRows * kPiece;
+    constexpr int kLoads = kRows / 8 / kWaves;      // of 8 rows, a wave and slice: half of them W's, half A's
+    constexpr int kStep = kGate ? 16 * kN : 32 * kN;
+    static_assert(kPiecesPerChain == kStages, "the loop takes a chain at a time");
+    __shared__ __attribute__((aligned(1024))) float stages[kStages * kStageFloats];
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    // each XCD takes a run of neighbouring whole tiles, row blocks first, and behind them its share of those whose rows end
+    // early (less work: what is left to do when the last turn is short)
+    const DirectGrid grid(M, row_blocks, tiles);
+    const int xcd = blockIdx.x % 8, local = blockIdx.x / 8;
+    const bool ragged = local >= grid.whole_each;
+    const int at = ragged ? xcd * grid.ragged_each + local - grid.whole_each : xcd * grid.whole_each + local;
+    if (at >= (ragged ? grid.ragged : grid.whole)) return;
+    const int m0 = (ragged ? row_blocks - 1 : at % grid.whole_blocks) * 32 * kM;
+    const int n0 = (ragged ? at : at / grid.whole_blocks) * kStep;
+    const int width = kGate ? N / 2 : N;
+    const int k_first = parts ? blockIdx.y * kStretch : 0;
+    const int slices = ((parts ? min(K, k_first + kStretch) : K) - k_first) / kPiece;
+
+    unsigned from[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int r = (wave + kWaves * i) * 8 + lane / 8;
+        const int chunk = (lane % 8) ^ ((r >> 1) & 7);
+        const int n = kGate ? min(n0 + r / 32 * 16 + r % 16, width - 1) + (r / 16 % 2) * width : min(n0 + r, N - 1);
+        const int m = min(m0 + r - 32 * kN, M - 1);
+        from[i] = 4u * (r < 32 * kN ? static_cast<unsigned>(n) * K + k_first + 4 * chunk : static_cast<unsigned>(m) * lda + k_first + 4 * chunk);
+    }
+    const __amdgpu_buffer_rsrc_t of_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(W), 0, 0xffffffffu, 0x00027000);
+    const __amdgpu_buffer_rsrc_t of_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, 0xffffffffu, 0x00027000);
+    auto fetch = [&](int slice, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(i < kLoads / 2 ? of_w : of_a,
+                                                     (lds_pointer)(stages + stage * kStageFloats + (wave + kWaves * i) * 8 * kPiece), 16,
+                                                     from[i], slice * kPiece * 4, 0, 0);
+    };
+
+    const int wn = (wave % 2) * 16 * kN, wm = 32 * kN + (wave / 2) * 16 * kM;  // this wave's rows in a stage
+    const int row_tiles = max(0, min(kM, (M - m0 - (wm - 32 * kN) + 15) / 16));  // ... of which so many hold rows
+    floatx4 acc[kN][kM] = {}, block[kN][kM] = {}, stretch[kN][kM] = {}, total[kN][kM] = {};
+    auto join = [](floatx4 (&to)[kN][kM], floatx4 (&from)[kN][kM]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int in = 0; in < kN; ++in)
+#pragma unroll
+            for (int im = 0; im < kM; ++im) {
+                to[in][im] += from[in][im];
+                from[in][im] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
+    };
+    struct Operands {
+        floatx4 w[kN], x[kM];
+    };
+    auto read = [&](Operands& to, const float* at, int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kN; ++i) to.w[i] = operand(at, wn + 16 * i + lane % 16, g, lane / 16);
+#pragma unroll
+        for (int i = 0; i < kM; ++i) to.x[i] = operand(at, wm + 16 * i + lane % 16, g, lane / 16);
+    };
+    auto products = [&](const Operands& o, int im) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int in = 0; in < kN; ++in)
+                acc[in][im] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[in][j], o.x[im][j], acc[in][im], 0, 0, 0);
+    };
+    auto multiply = [&](const Operands& o) __attribute__((always_inline)) {
+        if (row_tiles == kM) {  // (the same for the wave)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int in = 0; in < kN; ++in)
+#pragma unroll
+                    for (int im = 0; im < kM; ++im)
+                        acc[in][im] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[in][j], o.x[im][j], acc[in][im], 0, 0, 0);
+        } else if (row_tiles == 1) {
+            products(o, 0);
+        }
+    };
+    // A product's sums are read (join) only when it has finished: the wait states between the two are written here, for
+    // every way that leads from a product to a join.
+    auto settle = [] __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Operands even, odd;
+    auto meet = [&](bool more) __attribute__((always_inline)) {
+        if (more) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kStages - 2) * kLoads) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        asm volatile("s_barrier" ::: "memory");
+    };
+#pragma unroll
+    for (int s = 0; s < kStages; ++s)
+        if (s < slices) fetch(s, s);
+    if (slices >= kStages) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStages - 1) * kLoads) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+    read(even, stages, 0);
+    for (int first = 0; first < slices; first += kStages) {
+#pragma unroll
+        for (int j = 0; j < kStages; ++j) {
+            const int slice = first + j;
+            if (slice < slices) {  // (the same for all)
+                read(odd, stages + j * kStageFloats, 1);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(even);
+                __builtin_amdgcn_sched_barrier(0);
+                meet(slice + kStages <= slices);  // the next slice is there, and nobody reads this one any more
+                if (slice + kStages < slices) fetch(slice + kStages, j);
+                read(even, stages + (j + 1) % kStages * kStageFloats, 0);  // (past the last slice: read and dropped)
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(odd);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        const int past = first + kStages;
+        const bool end = past >= slices;
+        settle();
+        join(block, acc);
+        if (end || past % kPiecesPerBlock == 0) join(stretch, block);
+        if (end || past % (kPiecesPerBlock * kBlocksPerStretch) == 0) join(total, stretch);
+    }
+    if (parts) C = parts + static_cast<size_t>(blockIdx.y) * M * N;
+    const bool wide = ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+#pragma unroll
+    for (int in = 0; in < kN; in += kGate ? 2 : 1) {
+        const int n = n0 + (kGate ? wn / 2 + 8 * in : wn + 16 * in) + 4 * (lane / 16);
+        floatx4 b = {0.f, 0.f, 0.f, 0.f};
+        if (bias)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b[i] = bias[min(n + i, N - 1)];
+#pragma unroll
+        for (int im = 0; im < kM; ++im) {
+            const int m = m0 + (wm - 32 * kN) + 16 * im + lane % 16;
+            if (m >= M) continue;
+            floatx4 v = total[in][im];
+            if constexpr (kGate) {
+                const floatx4 u = total[in + 1][im];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = gated(v[i], u[i]);
+            } else {
+                v += b;
+            }
+            float* to = C + static_cast<size_t>(m) * ldc + n;
+            if (wide && n + 3 < width) {
+                *reinterpret_cast<floatx4*>(to) = v;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n + i < width) to[i] = v[i];
+            }
+        }
+    }
+#endif
+}
+
 // C = the sums of `stretches` parts [M, N] in order (+ bias), or the gated unit of their halves; a thread an output number.
 template <bool kGate>
 __global__ void __launch_bounds__(256)
@@ -400,6 +586,15 @@ struct Product {
     int M, N, K, lda, ldc, units;
 };
 
+// Whether `workgroups` tiles load straight into LDS: whole slices of K, places in the operands in 32 bits of bytes, and five
+// tiles and more to a unit (N 22,016, K 2,048 with the gate, us, before and so: 100 rows, 2.7 to a unit, 129, 133; 256 rows,
+// 5.4, 249, 237; 517 rows 486, 460; N 2,048, K 11,008 in stretches: 517 rows, 12 to a unit, 264, 256; N 2,560, K 2,048: 800
+// rows, 4 to a unit, 106, 110).
+bool goes_direct(const Product& p, long workgroups) {
+    return workgroups >= 5L * p.units && p.K % kPiece == 0 && static_cast<long>(p.N) * p.K < (1L << 30) &&
+           static_cast<long>(p.M) * p.lda < (1L << 30);
+}
+
 template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec>
 void run_rows(hipStream_t s, const Product& p) {
     const int step = kGate ? kColumns / 2 : kColumns;
@@ -420,7 +615,8 @@ void run_tiles(hipStream_t s, const Product& p) {
     const int step = kGate ? 32 : 64;
     const int row_blocks = (p.M + 63) / 64;
     const int tiles = row_blocks * (((kGate ? p.N / 2 : p.N) + step - 1) / step);
-    gemm_f32_tile_kernel<2, 2, kVec ? 4 : 2, kGate, kVec><<<(tiles + 7) / 8 * 8, 256, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, row_blocks, tiles, nullptr);
+    if (kVec && goes_direct(p, tiles)) gemm_f32_direct_kernel<kGate><<<DirectGrid(p.M, row_blocks, tiles).workgroups(), 256, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, row_blocks, tiles, nullptr);
+    else gemm_f32_tile_kernel<2, 2, kVec ? 4 : 2, kGate, kVec><<<(tiles + 7) / 8 * 8, 256, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, row_blocks, tiles, nullptr);
 }
 
 template <bool kVec>
@@ -429,7 +625,8 @@ void run_stretches(hipStream_t s, const Product& p, bool gate) {
     const int tiles = row_blocks * ((p.N + 63) / 64);
     const int stretches = (p.K + kStretch - 1) / kStretch;
     dim3 grid((tiles + 7) / 8 * 8, stretches);
-    gemm_f32_tile_kernel<2, 2, kVec ? 4 : 2, false, kVec><<<grid, 256, 0, s>>>(p.A, p.W, nullptr, nullptr, p.M, p.N, p.K, p.lda, p.N, row_blocks, tiles, p.parts);
+    if (kVec && goes_direct(p, static_cast<long>(tiles) * stretches)) gemm_f32_direct_kernel<false><<<dim3(DirectGrid(p.M, row_blocks, tiles).workgroups(), stretches), 256, 0, s>>>(p.A, p.W, nullptr, nullptr, p.M, p.N, p.K, p.lda, p.N, row_blocks, tiles, p.parts);
+    else gemm_f32_tile_kernel<2, 2, kVec ? 4 : 2, false, kVec><<<grid, 256, 0, s>>>(p.A, p.W, nullptr, nullptr, p.M, p.N, p.K, p.lda, p.N, row_blocks, tiles, p.parts);
     dim3 join(((gate ? p.N / 2 : p.N) + 255) / 256, p.M);
     if (gate) gemm_f32_join_kernel<true><<<join, 256, 0, s>>>(p.parts, stretches, nullptr, p.C, p.M, p.N, p.ldc);
     else gemm_f32_join_kernel<false><<<join, 256, 0, s>>>(p.parts, stretches, p.bias, p.C, p.M, p.N, p.ldc);

@@ -121,6 +121,19 @@ def test_gemm_f32_forms(ops, shape):
         assert all(torch.equal(ops.gemm_f32(a, w, gate=True, form=form), unit) for form in (0, 1, 2))
 
 
+# five and more tiles of 64 x 64 to each of 256 units: whole row blocks, rows of which one and more than 48 are left, a
+# number of slices that is no multiple of a chain's four, K in stretches of which the last is short
+@pytest.mark.parametrize("shape", [(640, 8192, 96), (641, 8194, 160), (700, 8130, 32), (321, 4098, 4128)])
+def test_gemm_f32_many_tiles(ops, shape):
+    """The tiles that load straight into LDS give the bits of the form for few rows."""
+    m, n, k = shape
+    a, w, b = rand((m, k), torch.float32, 13), rand((n, k), torch.float32, 14), rand((n,), torch.float32, 15)
+    assert -(-m // 64) * -(-n // 64) * -(-k // 1024) >= 5 * ops.compute_units()
+    expect, unit = ops.gemm_f32(a, w, b, form=0), ops.gemm_f32(a, w, gate=True, form=0)
+    assert all(torch.equal(ops.gemm_f32(a, w, b, form=form), expect) for form in (1, 2))
+    assert all(torch.equal(ops.gemm_f32(a, w, gate=True, form=form), unit) for form in (1, 2))
+
+
 @pytest.mark.parametrize("shape", [(200, 66, 1028), (129, 130, 4100)])
 def test_gemm_f32_in_bands_of_rows(ops, monkeypatch, shape):
     """Stretches of K whose sums do not fit the workspace: the rows go in bands, with the bits of the other forms."""
