@@ -63,10 +63,12 @@ PART_K = 1024           # the shortest stretch of K a part takes
 # at 96 rows 29.6 / 69.6 / 65.0 against 32.2 / 71.1 / 64.6); beyond that the library is level or ahead (3B at 128
 # rows: 35 against 30 + 5 us; 7B: 111 against 66).
 SHARED_SILU_ROWS = 96
-# float32 logits take that form up to this many rows (the head of the 3B / 7B / 14B shape, us: 64 rows 156 against
-# 173 in the form whose waves share K; 72 rows 165 / 239 / 333 against the library's 174 / 249 / 349; 96 rows
-# 172 / 255 / 346 against 174 / 238 / 338)
-SHARED_LOGIT_ROWS = 80
+# float32 logits of this many rows take that form (the head of the 0.5B / 3B / 7B / 14B shape, us, in the form whose waves share
+# K and in this one: 1 row 42.6, 43.3 / 109, 110 / - / -; 4 rows 54.6, 52.9 / 114, 114 / 199, 193 / 279, 271; 8 rows 56, 54 /
+# 121, 116 / 211, 190 / 299, 275; 16 rows 64, 56 / 137, 118 / 238, 195 / 346, 272; the library and this one: 72 rows 85, 73 / 169,
+# 142 / 237, 226 / 338, 313; 96 rows 82, 78 / 171, 149 / 235, 239 / 333, 327; 112 rows 89, 102 / 170, 169 / 244, 278 / 333, 398)
+SHARED_LOGIT_ROWS_FROM = 4
+SHARED_LOGIT_ROWS = 96
 
 
 def plan_shared_silu(pairs: int) -> tuple[int, bool]:
@@ -450,8 +452,8 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
         waves, own_unit = plan_shared_silu(-(-n // 32))
         if rows > FUSED_ROWS or own_unit:
             return ops.gemm_shared_rows(weight, ops.EPI_SILU, x, waves=waves)
-    if fusable and wants_f32 and FUSED_ROWS < rows <= SHARED_LOGIT_ROWS and into is None and not silu:
-        # logits of 17 to 80 rows: the shared-rows form
+    if fusable and wants_f32 and SHARED_LOGIT_ROWS_FROM <= rows <= SHARED_LOGIT_ROWS and into is None and not silu:
+        # logits of 4 to 96 rows: the shared-rows form
         return ops.gemm_shared_rows(weight, ops.EPI_F32, x, bias=bias, waves=4)
     if fusable and wants_f32 and rows > FUSED_LOGIT_ROWS and into is None and not silu and bias is None:
         out = ops.gemm_library(x, weight, out_dtype=torch.float32)  # logits of many rows: one pass over the weight
