@@ -1278,6 +1278,27 @@ def test_gemm_shared_rows_matches_float64(ops, shape, waves):
         torch.testing.assert_close(out.double(), torch.nn.functional.silu(gate * scale) * (up * scale), rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("shape", [(1, 2048, 96), (8, 2048, 22016), (16, 4096, 200), (40, 2048, 328), (96, 6144, 72), (5, 2048, 33)])
+def test_products_whose_rows_lie_4_kb_apart_match_float64(ops, shape):
+    """Where K is a multiple of 2,048 the workgroups begin with different k: logits in both forms, the SiLU product, sums of K in
+    parts.  The operands are exact in bf16; K float32 adds of partial sums that grow like sqrt(K) miss the float64 product by some
+    K 2^-24 of a term in the root mean square, and four roundings of the sum of the terms' magnitudes are several times that."""
+    m, k, n = shape
+    a, w = rand((m, k), torch.bfloat16, 71), rand((n, k), torch.bfloat16, 72, 0.3)
+    want = a.double() @ w.double().t()
+    close = dict(rtol=0.0, atol=float(2.0 ** -22 * (a.double().abs() @ w.double().abs().t()).max()))
+    torch.testing.assert_close(ops.gemm_fused(w, ops.EPI_F32, a).double(), want, **close)
+    torch.testing.assert_close(ops.gemm_shared_rows(w, ops.EPI_F32, a).double(), want, **close)
+    for parts in (1, 3):
+        out = ops.gemm_shared_rows(w, ops.EPI_PARTIAL, a, k_parts=parts, column_tiles=1)
+        torch.testing.assert_close(out.double().sum(dim=0), want, **close)
+    if n % 2 == 0:
+        gate, up = want[:, : n // 2], want[:, n // 2:]
+        torch.testing.assert_close(ops.gemm_shared_rows(w, ops.EPI_SILU, a).double(), gate * torch.sigmoid(gate) * up,
+                                   rtol=2 ** -7, atol=2e-3)
+
+
+
 def test_gemm_shared_rows_refuses_what_it_does_not_take(ops):
     a, w = rand((129, 64), torch.bfloat16, 44), rand((32, 64), torch.bfloat16, 45)
     with pytest.raises(ValueError):
