@@ -54,6 +54,10 @@ FUSED_LOGIT_ROWS = 64
 PART_BELOW_TILES = 512
 PART_MIN_K = 4096
 PART_K = 1024           # the shortest stretch of K a part takes
+# ... and of a product that has at least this many workgroups side by side (narrower ones were not measured).  896 columns,
+# K 4,864, us: 4 parts 7.2 at 8 rows, 13.7 at 96; 8 parts 5.4, 10.2; 10 parts 4.7, 8.8; 16 parts 4.8, 9.7.  1,536 columns,
+# K 8,960: 8 parts 8.3, 16.0; 10 parts 7.5, 15.4.
+PART_K_WIDE, PART_WIDE_BLOCKS = 512, 8
 
 
 # SiLU-gate products of up to this many rows take the form whose waves own columns and share the rows of A
@@ -97,7 +101,8 @@ def plan_shared_parts(tiles: int, k: int) -> tuple[int, int, int]:
     column_tiles = 1 if tiles <= units else 2
     waves = 4
     blocks = -(-tiles // (column_tiles * waves))
-    parts = max(1, min(units // blocks, 16, k // PART_K))
+    most = -(-k // PART_K_WIDE) if blocks >= PART_WIDE_BLOCKS and PART_K > PART_K_WIDE else k // PART_K
+    parts = max(1, min(units // blocks, 16, most))
     return column_tiles, waves, parts
 
 

@@ -78,6 +78,20 @@ def test_cut_products_and_silu_products_plan_by_compute_units():
     assert plan_shared_silu(1) == (2, True)        # a narrow one: no idle waves
 
 
+def test_narrow_products_of_a_long_k_take_more_parts():
+    """Stretches of 512 k where eight workgroups and more stand side by side and units are left; none without K of its own."""
+    from cie_amd.parts.linear import plan_shared_parts
+
+    assert plan_shared_parts(56, 4864) == (1, 4, 10)      # the 0.5B down product
+    assert plan_shared_parts(96, 8960) == (1, 4, 10)      # 1.5B: as many as there are units for
+    assert plan_shared_parts(28, 4096) == (1, 4, 4) and plan_shared_parts(29, 4096) == (1, 4, 8)  # seven workgroups, eight
+    for tiles, k in ((56, 4864), (40, 4104), (96, 8960), (32, 5000)):
+        parts = plan_shared_parts(tiles, k)[2]
+        stretch = -(-(-(-k // parts)) // 128) * 128       # what the kernel gives each part
+        assert stretch * (parts - 1) < k, (tiles, k)
+
+
+
 def test_a_widened_head_is_made_once_and_let_go_with_its_weight():
     import gc
 
