@@ -61,7 +61,7 @@ PART_K_WIDE, PART_WIDE_BLOCKS = 512, 8
 
 
 # SiLU-gate products of up to this many rows take the form whose waves own columns and share the rows of A
-# through LDS (gate/up of the 3B shape at 32 / 64 rows: 21 / 24 us against the library's 26 / 27 us and 5 us
+# through LDS (gate/up of the 3B shape at 32 / 64 rows: 19 / 22.5 us against the library's 26 / 27 us and 5 us
 # for the SiLU kernel behind it; 14B: 50 / 56 against 55 / 62 + 6; 7B: level); from 65 to 96 rows, on six row tiles
 # (3B / 7B / 14B at 72 rows: 28.3 / 67.7 / 63.7 us against 31.4 / 75.2 / 70.4 for the library and its SiLU kernel,
 # at 96 rows 29.6 / 69.6 / 65.0 against 32.2 / 71.1 / 64.6); beyond that the library is level or ahead (3B at 128
