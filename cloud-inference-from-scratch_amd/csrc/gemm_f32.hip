@@ -586,12 +586,15 @@ struct Product {
     int M, N, K, lda, ldc, units;
 };
 
-// Whether `workgroups` tiles load straight into LDS: whole slices of K, places in the operands in 32 bits of bytes, and five
-// tiles and more to a unit (N 22,016, K 2,048 with the gate, us, before and so: 100 rows, 2.7 to a unit, 129, 133; 256 rows,
-// 5.4, 249, 237; 517 rows 486, 460; N 2,048, K 11,008 in stretches: 517 rows, 12 to a unit, 264, 256; N 2,560, K 2,048: 800
-// rows, 4 to a unit, 106, 110).
-bool goes_direct(const Product& p, long workgroups) {
-    return workgroups >= 5L * p.units && p.K % kPiece == 0 && static_cast<long>(p.N) * p.K < (1L << 30) &&
+// Whether `workgroups` tiles load straight into LDS: whole slices of K, places in the operands in 32 bits of bytes, and so many
+// tiles to a unit: five and more over all of K (N 22,016, K 2,048 with the gate, us, before and so: 100 rows, 2.7 to a unit,
+// 129, 133; 256 rows, 5.4, 228, 229; 264 rows 269, 253; 448 rows 377, 361; 517 rows 486, 460; N 2,560,
+// K 2,048: 800 rows, 4 to a unit, 106, 110), twelve in stretches (N 2,048, K 11,008: 288 rows, 6.9 to a unit, 147, 150; 384 rows,
+// 8.3, 176, 182; 448 rows, 9.6, 196, 197; 517 rows, 12.4, 264, 256; 2,048 rows 821, 753).
+constexpr long kDirectTiles = 5, kDirectStretches = 12;
+
+bool goes_direct(const Product& p, long workgroups, long per_unit) {
+    return workgroups >= per_unit * p.units && p.K % kPiece == 0 && static_cast<long>(p.N) * p.K < (1L << 30) &&
            static_cast<long>(p.M) * p.lda < (1L << 30);
 }
 
@@ -615,7 +618,7 @@ void run_tiles(hipStream_t s, const Product& p) {
     const int step = kGate ? 32 : 64;
     const int row_blocks = (p.M + 63) / 64;
     const int tiles = row_blocks * (((kGate ? p.N / 2 : p.N) + step - 1) / step);
-    if (kVec && goes_direct(p, tiles)) gemm_f32_direct_kernel<kGate><<<DirectGrid(p.M, row_blocks, tiles).workgroups(), 256, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, row_blocks, tiles, nullptr);
+    if (kVec && goes_direct(p, tiles, kDirectTiles)) gemm_f32_direct_kernel<kGate><<<DirectGrid(p.M, row_blocks, tiles).workgroups(), 256, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, row_blocks, tiles, nullptr);
     else gemm_f32_tile_kernel<2, 2, kVec ? 4 : 2, kGate, kVec><<<(tiles + 7) / 8 * 8, 256, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, row_blocks, tiles, nullptr);
 }
 
@@ -625,7 +628,7 @@ void run_stretches(hipStream_t s, const Product& p, bool gate) {
     const int tiles = row_blocks * ((p.N + 63) / 64);
     const int stretches = (p.K + kStretch - 1) / kStretch;
     dim3 grid((tiles + 7) / 8 * 8, stretches);
-    if (kVec && goes_direct(p, static_cast<long>(tiles) * stretches)) gemm_f32_direct_kernel<false><<<dim3(DirectGrid(p.M, row_blocks, tiles).workgroups(), stretches), 256, 0, s>>>(p.A, p.W, nullptr, nullptr, p.M, p.N, p.K, p.lda, p.N, row_blocks, tiles, p.parts);
+    if (kVec && goes_direct(p, static_cast<long>(tiles) * stretches, kDirectStretches)) gemm_f32_direct_kernel<false><<<dim3(DirectGrid(p.M, row_blocks, tiles).workgroups(), stretches), 256, 0, s>>>(p.A, p.W, nullptr, nullptr, p.M, p.N, p.K, p.lda, p.N, row_blocks, tiles, p.parts);
     else gemm_f32_tile_kernel<2, 2, kVec ? 4 : 2, false, kVec><<<grid, 256, 0, s>>>(p.A, p.W, nullptr, nullptr, p.M, p.N, p.K, p.lda, p.N, row_blocks, tiles, p.parts);
     dim3 join(((gate ? p.N / 2 : p.N) + 255) / 256, p.M);
     if (gate) gemm_f32_join_kernel<true><<<join, 256, 0, s>>>(p.parts, stretches, nullptr, p.C, p.M, p.N, p.ldc);

@@ -134,6 +134,15 @@ def test_gemm_f32_many_tiles(ops, shape):
     assert all(torch.equal(ops.gemm_f32(a, w, gate=True, form=form), unit) for form in (1, 2))
 
 
+def test_gemm_f32_many_stretches(ops):
+    """Twelve and more tiles to a unit with K in stretches, the last one short: loaded straight into LDS, the same bits."""
+    m, n, k = 600, 4098, 4128
+    a, w, b = rand((m, k), torch.float32, 16), rand((n, k), torch.float32, 17), rand((n,), torch.float32, 18)
+    assert -(-m // 64) * -(-n // 64) * -(-k // 1024) >= 12 * ops.compute_units()
+    assert torch.equal(ops.gemm_f32(a, w, b, form=2), ops.gemm_f32(a, w, b, form=0))
+
+
+
 @pytest.mark.parametrize("shape", [(200, 66, 1028), (129, 130, 4100)])
 def test_gemm_f32_in_bands_of_rows(ops, monkeypatch, shape):
     """Stretches of K whose sums do not fit the workspace: the rows go in bands, with the bits of the other forms."""
