@@ -67,12 +67,29 @@ PART_K_WIDE, PART_WIDE_BLOCKS = 512, 8
 # at 96 rows 29.6 / 69.6 / 65.0 against 32.2 / 71.1 / 64.6); beyond that the library is level or ahead (3B at 128
 # rows: 35 against 30 + 5 us; 7B: 111 against 66).
 SHARED_SILU_ROWS = 96
-# float32 logits of this many rows take that form (the head of the 0.5B / 3B / 7B / 14B shape, us, in the form whose waves share
-# K and in this one: 1 row 42.6, 43.3 / 109, 110 / - / -; 4 rows 54.6, 52.9 / 114, 114 / 199, 193 / 279, 271; 8 rows 56, 54 /
-# 121, 116 / 211, 190 / 299, 275; 16 rows 64, 56 / 137, 118 / 238, 195 / 346, 272; the library and this one: 72 rows 85, 73 / 169,
-# 142 / 237, 226 / 338, 313; 96 rows 82, 78 / 171, 149 / 235, 239 / 333, 327; 112 rows 89, 102 / 170, 169 / 244, 278 / 333, 398)
-SHARED_LOGIT_ROWS_FROM = 4
-SHARED_LOGIT_ROWS = 96
+# Float32 results take that form at 17 to 80 rows (the head of the 3B shape at 64 rows 137 us, 169 in the form whose waves share
+# K), and with fewer or more rows where the columns give each unit a workgroup (of 128 columns) all the time: what the form
+# takes is what its fullest unit takes, and a narrow product leaves the others idle while one workgroup walks all of K.
+# us, the form whose waves share K and this one, K 2,048, 4 / 8 / 16 rows:
+#   columns      32  4.2, 11.2 / 4.4, 11.2 / 4.8, 11.2       2,048 (K 4,096)  7.6, 24.0 / 8.1, 24.2 / 9.4, 24.4
+#            32,768  27.5, 25.3 / 28.2, 25.2 / 29.6, 24.6 (one turn of 256 units)       40,000 (two turns, 61 % of them)
+#                    31.4, 36.0 / 32.4, 36.1 / 35.1, 35.6       65,536 (two turns)  49.4, 48.3 / 50.5, 47.2 / 55.8, 47.1
+#            73,728 (three turns, 75 %)  56.4, 57.5 / 58.1, 58.0 / 66.8, 59.0       152,064 (93 %)  111, 110 / 114, 111 / 132, 115
+# Hence the share of the turns' units that must have work, up to so many rows:
+SHARED_LOGIT_FILL = ((3, None), (8, 0.9), (16, 0.75), (80, 0.0))
+# The library and this one, 81 / 96 rows: 32 columns 6.0, 25.2 / 5.9, 25.3; 32,768 (K 1,024) 18.5, 19.5 / 17.8, 19.9; 50,304
+# (K 4,096) 103, 96 / 105, 98, (K 5,120) 106, 123 / 106, 125; 65,536 (K 1,024, 4,096, 5,120) 37, 34, 131, 109, 126, 139 at 81;
+# 152,064 166, 144 / 168, 147, (K 5,120) 342, 320 / 331, 327: from so many turns on, up to and beyond this K.
+SHARED_LOGIT_ROWS, SHARED_LOGIT_TURNS, SHARED_LOGIT_K = 96, (2, 4), 4096
+
+
+def shares_rows_f32(rows: int, n: int, k: int) -> bool:
+    """Whether a float32 result of ``rows`` rows and ``n`` columns takes the shared-rows form."""
+    units, groups = ops.compute_units(), -(-n // 128)
+    for upto, fill in SHARED_LOGIT_FILL:
+        if rows <= upto:
+            return fill is not None and groups >= fill * units * -(-groups // units)
+    return rows <= SHARED_LOGIT_ROWS and groups >= SHARED_LOGIT_TURNS[k > SHARED_LOGIT_K] * units
 
 
 def plan_shared_silu(pairs: int) -> tuple[int, bool]:
@@ -457,8 +474,7 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
         waves, own_unit = plan_shared_silu(-(-n // 32))
         if rows > FUSED_ROWS or own_unit:
             return ops.gemm_shared_rows(weight, ops.EPI_SILU, x, waves=waves)
-    if fusable and wants_f32 and SHARED_LOGIT_ROWS_FROM <= rows <= SHARED_LOGIT_ROWS and into is None and not silu:
-        # logits of 4 to 96 rows: the shared-rows form
+    if fusable and wants_f32 and into is None and not silu and shares_rows_f32(rows, n, k):
         return ops.gemm_shared_rows(weight, ops.EPI_F32, x, bias=bias, waves=4)
     if fusable and wants_f32 and rows > FUSED_LOGIT_ROWS and into is None and not silu and bias is None:
         out = ops.gemm_library(x, weight, out_dtype=torch.float32)  # logits of many rows: one pass over the weight

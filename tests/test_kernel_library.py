@@ -92,6 +92,21 @@ def test_narrow_products_of_a_long_k_take_more_parts():
 
 
 
+def test_float32_results_share_rows_only_where_the_units_have_work():
+    """Heads take the form whose waves own 128 columns a workgroup; a router, an expert's gate, a mixer's or an entry's
+    float32 rows, whose few workgroups would walk all of K one after another, do not (17 to 80 rows take it at any width)."""
+    from cie_amd.parts.linear import shares_rows_f32
+
+    for n, k in ((1, 2048), (32, 2048), (64, 5120), (2048, 2048), (2048, 4096), (4096, 8192), (16384, 1024)):
+        assert not any(shares_rows_f32(rows, n, k) for rows in (*range(1, 17), *range(81, 129))), (n, k)
+        assert all(shares_rows_f32(rows, n, k) for rows in (17, 64, 80))
+    for n, k in ((151936, 896), (151936, 2048), (152064, 3584), (152064, 5120)):
+        assert [rows for rows in range(1, 200) if shares_rows_f32(rows, n, k)] == list(range(4, 97))
+    assert not shares_rows_f32(4, 40000, 2048) and not shares_rows_f32(16, 40000, 2048)  # a second turn of a few units
+    assert not shares_rows_f32(8, 73728, 2048) and shares_rows_f32(9, 73728, 2048)
+    assert shares_rows_f32(81, 65536, 4096) and not shares_rows_f32(81, 65536, 5120)
+
+
 def test_a_widened_head_is_made_once_and_let_go_with_its_weight():
     import gc
 
