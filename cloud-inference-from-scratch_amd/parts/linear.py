@@ -474,7 +474,9 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
         waves, own_unit = plan_shared_silu(-(-n // 32))
         if rows > FUSED_ROWS or own_unit:
             return ops.gemm_shared_rows(weight, ops.EPI_SILU, x, waves=waves)
-    if fusable and wants_f32 and into is None and not silu and shares_rows_f32(rows, n, k):
+    if (fusable and wants_f32 and into is None and not silu and shares_rows_f32(rows, n, k)
+            # (beyond these rows the library is the other way, which takes operands that start off a 16-byte line too)
+            and (rows <= SHARED_LOGIT_FILL[-1][0] or (x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0))):
         return ops.gemm_shared_rows(weight, ops.EPI_F32, x, bias=bias, waves=4)
     if fusable and wants_f32 and rows > FUSED_LOGIT_ROWS and into is None and not silu and bias is None:
         out = ops.gemm_library(x, weight, out_dtype=torch.float32)  # logits of many rows: one pass over the weight

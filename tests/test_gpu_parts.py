@@ -1263,3 +1263,20 @@ def test_products_whose_operands_the_tiles_do_not_take():
         assert isinstance(got, torch.Tensor) and not stream.any()
         # float32 sums of k products of numbers about 1, rounded once to 8 mantissa bits
         torch.testing.assert_close(got.double(), expect, rtol=2.0 ** -8, atol=1e-4 * math.sqrt(k))
+
+
+def test_float32_results_of_operands_off_a_16_byte_line():
+    """81 to 96 rows that start between two 16-byte lines, a product wide enough for the form that asks for whole lines: the
+    library's, as it is for more rows."""
+    from cie_amd.parts.linear import linear, shares_rows_f32
+
+    n, k = 65600, 64
+    g = torch.Generator().manual_seed(10)
+    w = torch.randn((n, k), generator=g).bfloat16().cuda()
+    for rows in (88, 100):
+        x = torch.randn((rows, k + 8), generator=g).bfloat16().cuda()[:, 4: k + 4]
+        assert shares_rows_f32(rows, n, k) == (rows == 88) and x.data_ptr() % 16 == 8
+        got = linear(x, w, out_dtype=torch.float32)
+        assert got.dtype == torch.float32
+        # float32 sums of k products of numbers about 1
+        torch.testing.assert_close(got.double(), x.double() @ w.double().t(), rtol=1e-5, atol=1e-5 * math.sqrt(k))
