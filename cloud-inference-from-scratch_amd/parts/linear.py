@@ -407,10 +407,11 @@ def _fusable(rows: int, k: int, row_stride: int, weight: torch.Tensor) -> bool:
 
 def takes_tiles(rows: int, x: torch.Tensor, weight: torch.Tensor, into: Optional[torch.Tensor] = None) -> bool:
     """Whether the tile kernels take these operands (of a product that is ``_fusable``): beyond the rows of the streaming
-    kernels, on the GPU, in rows and at addresses that 16-byte loads and stores can use.  Whatever else a caller brings
-    (rows read across, a stream that starts off a 16-byte line, host tensors) is the library's or torch's, as it was."""
-    return (rows > FUSED_PARTS_ROWS and x.is_cuda and x.stride(1) == 1 and x.data_ptr() % 16 == 0
-            and weight.data_ptr() % 16 == 0
+    kernels, on the GPU, in rows that lie apart and at addresses that 16-byte loads and stores can use.  Whatever else a
+    caller brings (rows read across, rows that share their numbers, as one row expanded to many does, a stream that starts
+    off a 16-byte line, host tensors) is the library's or torch's, as it was."""
+    return (rows > FUSED_PARTS_ROWS and x.is_cuda and x.stride(1) == 1 and x.stride(0) >= x.shape[1]
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
             and (into is None or (into.is_cuda and into.dtype == torch.float32 and into.data_ptr() % 16 == 0)))
 
 

@@ -1280,3 +1280,25 @@ def test_float32_results_of_operands_off_a_16_byte_line():
         assert got.dtype == torch.float32
         # float32 sums of k products of numbers about 1
         torch.testing.assert_close(got.double(), x.double() @ w.double().t(), rtol=1e-5, atol=1e-5 * math.sqrt(k))
+
+
+@pytest.mark.parametrize("rows,n,k", [(200, 96, 512), (300, 4096, 128)])
+def test_products_of_rows_that_share_their_numbers(rows, n, k):
+    """One row expanded to many, and rows that begin eight numbers apart: torch's products of them, in every form that tiles
+    have an epilogue for."""
+    from cie_amd.parts.linear import linear
+
+    g = torch.Generator().manual_seed(11)
+    w = torch.randn((n, k), generator=g).bfloat16().cuda()
+    base = torch.randn(8 * rows + k, generator=g).bfloat16().cuda()
+    for x in (base[:k].expand(rows, k), base.as_strided((rows, k), (8, 1))):
+        expect = x.double() @ w.double().t()
+        # float32 sums of k products of numbers about 1, rounded once to 8 mantissa bits
+        close = dict(rtol=2.0 ** -8, atol=1e-4 * math.sqrt(k))
+        stream = torch.zeros((rows, n)).cuda()
+        torch.testing.assert_close(linear(x, w).double(), expect, **close)
+        torch.testing.assert_close(linear(x, w, into=stream).double(), expect, **close)
+        gate, up = expect[:, : n // 2], expect[:, n // 2:]
+        # (the gate and the unit come rounded: three roundings of 2^-8, and the sums' own error times the other factor)
+        torch.testing.assert_close(linear(x, w, epilogue="silu").double(), torch.nn.functional.silu(gate) * up,
+                                   rtol=3 * 2.0 ** -8, atol=1e-2 * k)
