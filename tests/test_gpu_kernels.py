@@ -1308,6 +1308,22 @@ def test_products_whose_rows_lie_4_kb_apart_match_float64(ops, shape):
 
 
 
+@pytest.mark.parametrize("rows", [4, 16, 40, 90])
+@pytest.mark.parametrize("k", [8, 136, 384, 896, 2048])
+def test_an_infinite_weight_shows_as_infinity(ops, rows, k):
+    """One infinite weight in a column, among the first, the middle or the last k: the column's float32 results are infinite
+    in both forms, and no other result is; also where K ends inside a slice or the slices are odd in number."""
+    n = 160
+    a, w = rand((rows, k), torch.bfloat16, 73), rand((n, k), torch.bfloat16, 74)
+    a[a == 0] = 1.0
+    for column, at, value in ((3, 0, math.inf), (17, k - 1, math.inf), (40, k // 2, -math.inf), (159, k - 8, -math.inf)):
+        w[column, at] = value
+    for out in (ops.gemm_fused(w, ops.EPI_F32, a), ops.gemm_shared_rows(w, ops.EPI_F32, a)):
+        assert not out.isnan().any()
+        assert torch.equal(out.isinf().any(0).nonzero().flatten().cpu(), torch.tensor([3, 17, 40, 159]))
+        assert torch.equal(out[:, 17], math.inf * a[:, k - 1].float().sign())
+
+
 def test_gemm_shared_rows_refuses_what_it_does_not_take(ops):
     a, w = rand((129, 64), torch.bfloat16, 44), rand((32, 64), torch.bfloat16, 45)
     with pytest.raises(ValueError):
