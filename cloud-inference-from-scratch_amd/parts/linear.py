@@ -118,9 +118,10 @@ def plan_shared_parts(tiles: int, k: int) -> tuple[int, int, int]:
     column_tiles = 1 if tiles <= units else 2
     waves = 4
     blocks = -(-tiles // (column_tiles * waves))
-    most = -(-k // PART_K_WIDE) if blocks >= PART_WIDE_BLOCKS and PART_K > PART_K_WIDE else k // PART_K
+    most = -(-k // PART_K_WIDE) if blocks >= PART_WIDE_BLOCKS else k // PART_K
     parts = max(1, min(units // blocks, 16, most))
-    return column_tiles, waves, parts
+    stretch = -(-(-(-k // parts)) // 128) * 128  # (what the kernel gives a part: whole slices, and none a part without k)
+    return column_tiles, waves, -(-k // stretch)
 
 
 # Products of more rows than the kernels above take (beyond ``FUSED_PARTS_ROWS``) go to tiles of this package or to the

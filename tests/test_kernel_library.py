@@ -85,10 +85,12 @@ def test_narrow_products_of_a_long_k_take_more_parts():
     assert plan_shared_parts(56, 4864) == (1, 4, 10)      # the 0.5B down product
     assert plan_shared_parts(96, 8960) == (1, 4, 10)      # 1.5B: as many as there are units for
     assert plan_shared_parts(28, 4096) == (1, 4, 4) and plan_shared_parts(29, 4096) == (1, 4, 8)  # seven workgroups, eight
-    for tiles, k in ((56, 4864), (40, 4104), (96, 8960), (32, 5000)):
-        parts = plan_shared_parts(tiles, k)[2]
-        stretch = -(-(-(-k // parts)) // 128) * 128       # what the kernel gives each part
-        assert stretch * (parts - 1) < k, (tiles, k)
+    assert plan_shared_parts(64, 11008) == (1, 4, 15) and plan_shared_parts(113, 4104) == (1, 4, 7)
+    for tiles in (1, 3, 28, 29, 32, 40, 56, 63, 64, 96, 113, 128, 224, 257, 320, 511):
+        for k in (*range(4096, 9000, 8), 8960, 11008, 13824, 16400, 18944, 29568):
+            _, _, parts = plan_shared_parts(tiles, k)
+            stretch = -(-(-(-k // parts)) // 128) * 128   # what the kernel gives each part
+            assert 1 <= parts <= 16 and stretch * (parts - 1) < k <= stretch * parts, (tiles, k)
 
 
 
