@@ -18,7 +18,10 @@
 // turns: parts/linear.py picks the tile whose turns come out best.
 //
 // A lane stores 16 bytes whose neighbours are its neighbours' (64 bytes a row and instruction): sums of K in parts, 3B down
-// at 2,048 rows, 101 -> 92 us.  The q/k/v epilogue asks for its rows' places between the last slices: 256 rows 14.8 -> 14.1.
+// at 2,048 rows, 101 -> 92 us.  Where the result's rows lie no multiple of that apart, in pieces of 8 or 4 bytes (bf16, 777 rows, K
+// 2,048, 4,098 columns, which are stored two at a time, 18.9 us; one at a time 24.8; 768 rows, K 768, 10,508 columns, four at a
+// time, 18.0 and 32.5).  The q/k/v epilogue asks for its rows' places between the last slices: 256 rows 14.8 -> 14.1; at 256 x 256
+// it spills 14 registers (60 bytes a lane), no other form any.
 //
 // Measured (MI355X, us, weights from memory; before: the library with the kernel behind its product, or gemm_tiles.hip):
 // 3B: gate/up 256 rows 40 -> 33, 613 rows 72 -> 61, 777 81 -> 72, 2,048 186 -> 157; down 256 rows 27 -> 23, 613 47 -> 36, 2,048
@@ -338,7 +341,7 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
 #pragma unroll
     for (int u = 0; u < kOut; u += kPair) {
         const int n = first + column_of<EPI, kN>(EPI == DIRECT_SILU ? 2 * u : u, lane / 16 * 4);
-        const bool whole = n + 4 * kPair <= width && p.ldc % (4 * kPair) == 0;
+        const bool whole = n + 4 * kPair <= width;
         float b[4 * kPair] = {};
         if (EPI != DIRECT_SILU && p.bias && blockIdx.y == 0)
 #pragma unroll
@@ -359,21 +362,41 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
             }
             if constexpr (EPI == DIRECT_BF16 || EPI == DIRECT_SILU) {
                 bf16_t* to = static_cast<bf16_t*>(p.c) + static_cast<size_t>(m) * p.ldc + n;
-                if (!whole) {
+                if (!whole || p.ldc % 2) {
 #pragma unroll
                     for (int i = 0; i < 4 * kPair; ++i)
                         if (n + i < width) to[i] = from_float<bf16_t>(v[i]);
-                } else if constexpr (kPair == 2) {
-                    *reinterpret_cast<u32x4*>(to) = u32x4{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
+                    continue;
+                }
+                unsigned packed[2 * kPair];
+#pragma unroll
+                for (int i = 0; i < 2 * kPair; ++i) packed[i] = pack_bf16(v[2 * i], v[2 * i + 1]);
+                if (kPair == 2 && p.ldc % 8 == 0) {
+                    *reinterpret_cast<u32x4*>(to) = u32x4{packed[0], packed[1], packed[2 * kPair - 2], packed[2 * kPair - 1]};
+                } else if (p.ldc % 4 == 0) {
+#pragma unroll
+                    for (int i = 0; i < kPair; ++i) reinterpret_cast<uint2*>(to)[i] = uint2{packed[2 * i], packed[2 * i + 1]};
                 } else {
-                    *reinterpret_cast<uint2*>(to) = uint2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+#pragma unroll
+                    for (int i = 0; i < 2 * kPair; ++i) reinterpret_cast<unsigned*>(to)[i] = packed[i];
                 }
             } else {
                 float* to = static_cast<float*>(p.c) + (static_cast<size_t>(EPI == DIRECT_PARTS ? blockIdx.y : 0) * p.M + m) * p.ldc + n;
-                if (whole) {
+                if (whole && p.ldc % 4 == 0) {
                     floatx4 sum = {v[0], v[1], v[2], v[3]};
                     if (EPI == DIRECT_RESID) sum += *reinterpret_cast<const floatx4*>(to);
                     *reinterpret_cast<floatx4*>(to) = sum;
+                } else if (whole && p.ldc % 2 == 0) {
+#pragma unroll
+                    for (int i = 0; i < 4; i += 2) {
+                        float2 sum = {v[i], v[i + 1]};
+                        if (EPI == DIRECT_RESID) {
+                            const float2 was = *reinterpret_cast<const float2*>(to + i);
+                            sum.x += was.x;
+                            sum.y += was.y;
+                        }
+                        *reinterpret_cast<float2*>(to + i) = sum;
+                    }
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
