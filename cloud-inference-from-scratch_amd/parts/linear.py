@@ -160,10 +160,11 @@ class Behind:
     us_per_million: float
     host_us: float
     host_upto: float
+    margin_timed: float = 1.15  # (``DIRECT_MARGIN`` where the library's algorithms are timed)
 
 
 BEHIND_NOTHING = Behind(0.0, 0.0, 3.0, 15.0)
-BEHIND_GATE = Behind(2.15, 1.2, 11.0, 40.0)      # the gate's kernel
+BEHIND_GATE = Behind(2.15, 1.2, 11.0, 40.0, 1.03)  # the gate's kernel
 BEHIND_BRANCH = Behind(-1.3, 1.9, 3.0, 15.0)     # the norm that adds the branch
 BEHIND_ROTATION = Behind(1.1, 1.8, 11.0, 21.0)   # the rotation and cache write
 # Where the host does not matter the tiles are taken if they are modelled to be faster by the first of these, beyond 25 us by the
@@ -202,7 +203,12 @@ DIRECT_US = {(64, 64): (3.1, 0.239, 0.246), (96, 64): (3.4, 0.301, 0.299), (96, 
 # Of the forms within this share of the fastest the one that reads least: level in the timings, less power inside a step (3B
 # gate/up of 2,048 rows, tiles of 192 x 192 that the model prefers by 3 %: 161 us alone, 174 inside a prompt).
 DIRECT_LEVEL = 1.04
-DIRECT_MARGIN = 1.03  # ... taken where they are modelled to be faster than the library by this
+# ... taken where they are modelled to be faster than the library by this, or, at the row counts whose algorithms it times, by
+# ``Behind.margin_timed``: of 500 products at 256 to 2,048 such rows 399 were taken by 1.03, 29 of them more than 4 % slower than
+# the library where the host is not what takes the time (512 rows x 4,096, K 11,136, 94 us against 82); by 1.15, and 1.03 for the
+# gate, 346 and 7, the gain in the mean the same 13.4 %.  At 400 row counts that do not recur, where the library takes its first
+# choice, eight of the 336 taken by 1.03.
+DIRECT_MARGIN = 1.03
 # Sums of K in parts are at most this many bytes (2,048 rows: 4 parts of the 3B shape's down product 67 MB, 2 of 7B's 59)
 PARTS_BYTES = 128 << 20
 
@@ -244,9 +250,10 @@ def _choose_direct(rows: int, n: int, k: int, most_parts: int, behind: Behind, u
     cost = min(times.values())
     reads = lambda f: (-(-rows // f[1]) * -(-n // f[0]) * (f[0] + f[1]), f[2])  # noqa: E731
     form = min((f for f in forms if times[f] <= cost * DIRECT_LEVEL), key=reads)
-    library = _library_us(rows, n, k, units, ops._tune_level(rows)) + behind.us + behind.us_per_million * rows * n * 1e-6
+    timed = ops._tune_level(rows)
+    library = _library_us(rows, n, k, units, timed) + behind.us + behind.us_per_million * rows * n * 1e-6
     library += behind.host_us if cost <= behind.host_upto else 0.0
-    return Tiles(*form, True) if cost * DIRECT_MARGIN < library else None
+    return Tiles(*form, True) if cost * (behind.margin_timed if timed else DIRECT_MARGIN) < library else None
 
 
 def choose_tiles(rows: int, n: int, k: int, row_stride: int, most_parts: int = 1, behind: Behind = BEHIND_NOTHING) -> Optional[Tiles]:

@@ -119,22 +119,33 @@ def test_float32_products_in_stretches_keep_their_workspace_bounded(rows, column
         assert (bands, band) == (2, 768) and ops.plan_gemm_f32(rows, columns, k) == 2
 
 
-# (what, rows, columns, K, us by the library with the kernel behind it, {tiles: us}), as measured on MI355X: products for
-# which an earlier rule took tiles that were slower than the library (the first of each), and tiles that are not
+# (what stands behind it, whether in parts of K, rows, columns, K, us by the library with the kernel behind it, {tiles: us}),
+# as measured on MI355X: products for which earlier rules took tiles that were slower than the library, and products whose
+# tiles are much the faster ones
 MEASURED = [
-    ("down", 613, 3584, 18944, 151.2, {(128, 256, 3): 193.0, (128, 128, 3): 134.1}),
-    ("down", 680, 3584, 18944, 169.8, {(128, 256, 3): 195.3, (128, 128, 3): 138.4}),
-    ("down", 768, 3584, 18944, 161.5, {(128, 256, 3): 198.8, (128, 128, 3): 145.2}),
-    ("down", 768, 896, 4864, 23.1, {(128, 64, 3): 28.3}),
-    ("o", 130, 3584, 3584, 20.4, {(128, 64, 3): 23.5, (64, 64, 3): 19.4}),
-    ("o", 330, 896, 896, 12.1, {(64, 64, 3): 11.2, (64, 64, 1): 10.6, (64, 64, 2): 10.2}),
-    ("o", 360, 2048, 2048, 16.3, {(128, 64, 2): 17.8, (64, 64, 1): 16.6}),
+    ("BRANCH", 8, 613, 3584, 18944, 152.5, {(256, 160, 4): 115.0}),
+    ("BRANCH", 8, 680, 3584, 18944, 168.5, {(192, 192, 3): 111.2}),
+    ("BRANCH", 8, 768, 3584, 18944, 160.5, {(192, 192, 3): 111.0}),
+    ("BRANCH", 8, 768, 896, 4864, 22.4, {(96, 128, 4): 21.9}),
+    ("BRANCH", 8, 130, 3584, 3584, 24.1, {(96, 64, 2): 18.0}),
+    ("BRANCH", 8, 330, 896, 896, 11.6, {(64, 64, 2): 9.8}),
+    ("BRANCH", 8, 360, 2048, 2048, 15.9, {(64, 64, 1): 13.7}),
+    ("BRANCH", 8, 400, 3584, 18944, 201.5, {(128, 256, 4): 80.6}),
+    ("BRANCH", 1, 512, 4096, 11136, 77.2, {(96, 128, 1): 92.4}),
+    ("BRANCH", 1, 512, 2560, 5120, 35.0, {(96, 64, 1): 38.8}),
+    ("BRANCH", 1, 2048, 1140, 11136, 85.1, {(96, 128, 1): 94.4}),
+    ("NOTHING", 1, 768, 1746, 8192, 43.9, {(96, 64, 1): 46.9}),
+    ("NOTHING", 1, 512, 4516, 5632, 42.4, {(96, 128, 1): 47.8}),
+    ("GATE", 1, 256, 22016, 2048, 42.0, {(192, 128, 1): 34.2}),
+    ("GATE", 1, 777, 37888, 3584, 273.0, {(256, 160, 1): 202.0}),
+    ("GATE", 1, 2048, 22016, 2048, 201.0, {(256, 256, 1): 167.8}),
 ]
 
 
-@pytest.mark.parametrize("what,rows,n,k,library,tiles", MEASURED)
-def test_tiles_are_not_taken_where_they_were_measured_to_lose(what, rows, n, k, library, tiles):
-    from cie_amd.parts.linear import BEHIND_BRANCH, plan_tiles
+@pytest.mark.parametrize("behind,parts,rows,n,k,library,tiles", MEASURED)
+def test_tiles_are_taken_where_they_were_measured_to_win(behind, parts, rows, n, k, library, tiles):
+    from cie_amd.parts import linear
 
-    picked = plan_tiles(rows, n, k, most_parts=8, behind=BEHIND_BRANCH)
-    assert picked is None or tiles[picked] <= 1.03 * library
+    picked = linear.choose_tiles(rows, n, k, k, most_parts=parts, behind=getattr(linear, "BEHIND_" + behind))
+    assert picked is None or (picked.direct and tiles[picked[:3]] <= 1.03 * library)
+    assert picked is not None or min(tiles.values()) > 0.9 * library
