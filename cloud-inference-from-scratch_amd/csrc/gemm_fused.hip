@@ -876,15 +876,19 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
     Slot ring0, ring1;
     // Workgroups that walk K in step read the same k of many rows at a time.  Where the rows lie a multiple of 4 KB apart these
     // are lines of a few memory channels, so there each workgroup begins with another slice and ends with those before it
-    // (3B gate/up, K 2,048, us: 8 rows 20.0 -> 18.1, 32 rows 20.6 -> 18.9, 64 rows 23.0 -> 22.5; K 5,120, whose rows spread by
-    // themselves, 49.2 -> 50.1, K 13,824 in parts 27.2 -> 28.6).  A step past the last slice stays there.
+    // (3B gate/up, K 2,048, us: 8 rows 20.2 -> 17.7, 32 rows 20.9 -> 18.3, 64 rows 22.9 -> 22.0; K 5,120, whose rows spread by
+    // themselves, 49.2 -> 50.1, K 13,824 in parts 27.2 -> 28.6).  A step past the last slice stays there.  The others have
+    // a loop of their own (sums in parts, 64 rows x 1,536, K 8,960: 12.2 -> 11.7) but for the SiLU product, which two loops cost more
+    // than a slice's place in turns (32 rows, 3B gate/up, 18.3 -> 19.0; 96 rows, 7B, 68 -> 81).
+    constexpr bool kTwoLoops = EPI == EPI_F32 || EPI == EPI_ATOMIC || EPI == EPI_PARTIAL;
     const int turn = slices > 0 && a.K % kChannelK == 0 ? static_cast<int>(blockIdx.x + (blockIdx.x >> 3)) % slices : 0;
-    auto first_k = [&](int slice) __attribute__((always_inline)) {
+    auto first_k = [&](int slice, auto turned) __attribute__((always_inline)) {
+        if constexpr (!decltype(turned)::value) return k_begin + slice * 128;
         const int s = slice + turn;
         return k_begin + (slice >= slices ? slices : s >= slices ? s - slices : s) * 128;
     };
-    auto fetch = [&](Slot& into, int slice) __attribute__((always_inline)) {
-        const int k = min(first_k(slice) + load_col, k_end - 8);
+    auto fetch = [&](Slot& into, int from) __attribute__((always_inline)) {
+        const int k = min(from + load_col, k_end - 8);
 #pragma unroll
         for (int i = 0; i < kPasses; ++i) into.a[i] = *reinterpret_cast<const u32x4*>(a_rows[i] + k);
 #pragma unroll
@@ -900,28 +904,24 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
         for (int t = 0; t < NT; ++t) acc[mt][t] = floatx4{0.f, 0.f, 0.f, 0.f};
     const int row_tiles_used = (a.M + 15) / 16;  // (row tiles past the last row are not multiplied)
 
-    auto step = [&](const Slot& now, Slot& ahead, int slice) __attribute__((always_inline)) {
+    // One slice, which begins at `at`, while the next one, at `next`, comes in.  kEnd: the slice may end behind the part.
+    auto step = [&](const Slot& now, Slot& ahead, int slice, int at, int next, auto end) __attribute__((always_inline)) {
+        constexpr bool kEnd = decltype(end)::value;
         char* stage_a = shared + (kStagesA == 2 ? (slice & 1) * kStageBytesA : 0);
         if (kStagesA == 1) __syncthreads();  // every wave has read the slice before
-        const int at = first_k(slice);
-        const bool inside = at + load_col < k_end;
+        const bool inside = !kEnd || at + load_col < k_end;
 #pragma unroll
         for (int i = 0; i < kPasses; ++i)
             *reinterpret_cast<u32x4*>(stage_a + a_stage_row[i] * kStageRow + load_col * 2) =
                 inside ? now.a[i] : u32x4{0u, 0u, 0u, 0u};
-        fetch(ahead, slice + 1);
+        fetch(ahead, next);
         u32x4 bt[NT][4];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {  // through the wave's staging area (its LDS operations keep their order)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                *reinterpret_cast<u32x4*>(stage_w + (i * 4 + load_row) * kStageRow + load_col * 2) = now.w[t][i];
-            // (float32 results: no zeros of A times a last piece of W that is infinite.  Head of K 896, us: 8 rows 53.0 -> 53.2, 64
-            // rows 66.0 -> 66.8; K 2,048 level; the other epilogues would pay up to 4 %)
-            if (EPI == EPI_F32 && at + 128 > k_end && !inside)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    *reinterpret_cast<u32x4*>(stage_w + (i * 4 + load_row) * kStageRow + load_col * 2) = u32x4{0u, 0u, 0u, 0u};
+                *reinterpret_cast<u32x4*>(stage_w + (i * 4 + load_row) * kStageRow + load_col * 2) =
+                    EPI != EPI_F32 || inside ? now.w[t][i] : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
             for (int j = 0; j < 4; ++j) bt[t][j] = *reinterpret_cast<const u32x4*>(stage_w + r * kStageRow + j * 64 + g * 16);
         }
@@ -959,7 +959,7 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
         for (int i = 0; i < kHeld; ++i)  // (past the end: the last four again, not added below)
             held[i] = *reinterpret_cast<const float4*>(scale_from + min((scale_sub + i * kPerRow) * 4, a.sumsq_parts - 4));
     }
-    fetch(ring0, 0);
+    fetch(ring0, k_begin + turn * 128);
     if (scaled_rows) {
         float sq = 0.f;
         if (scale_by_four) {
@@ -977,12 +977,32 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
         for (int offset = kPerRow / 2; offset > 0; offset >>= 1) sq += __shfl_xor(sq, offset, kWave);
         if (scale_lane && scale_sub == 0) scale_lds[scale_row] = 1.0f / sqrtf(sq / static_cast<float>(a.K) + a.eps);
     }
-    // (whole turns of the ring: a step past the last slice multiplies zeros)
+    auto walk = [&](auto turned) __attribute__((always_inline)) {
+        int base = 0;
+        if constexpr (EPI == EPI_F32) {
+            // whole slices, and what is left behind them, where the piece of W past the end is zeroed too: no zeros of A times a
+            // last piece that is infinite (a mask in every step, or a step past the last slice, cost up to 12 %)
+            const int whole = (k_end - k_begin) / 128;
 #pragma unroll 1
-    for (int base = 0; base < slices; base += 2) {
-        step(ring0, ring1, base);
-        step(ring1, ring0, base + 1);
-    }
+            for (; base + 2 <= whole; base += 2) {
+                step(ring0, ring1, base, first_k(base, turned), first_k(base + 1, turned), std::false_type{});
+                step(ring1, ring0, base + 1, first_k(base + 1, turned), first_k(base + 2, turned), std::false_type{});
+            }
+            if (base < slices) {
+                step(ring0, ring1, base, first_k(base, turned), first_k(base + 1, turned), std::true_type{});
+                if (base + 1 < slices) step(ring1, ring0, base + 1, first_k(base + 1, turned), first_k(base + 2, turned), std::true_type{});
+            }
+        } else {
+            // (whole turns of the ring: a step past the last slice multiplies zeros)
+#pragma unroll 1
+            for (; base < slices; base += 2) {
+                step(ring0, ring1, base, first_k(base, turned), first_k(base + 1, turned), std::true_type{});
+                step(ring1, ring0, base + 1, first_k(base + 1, turned), first_k(base + 2, turned), std::true_type{});
+            }
+        }
+    };
+    if (kTwoLoops && turn == 0) walk(std::false_type{});
+    else walk(std::true_type{});
     if (scaled_rows && slices == 0) __syncthreads();  // (the scales, if no step stood between)
 
 #pragma unroll
