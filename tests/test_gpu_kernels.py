@@ -122,25 +122,35 @@ def test_gemm_f32_forms(ops, shape):
 
 
 # five and more tiles of 64 x 64 to each of 256 units: whole row blocks, rows of which one and more than 48 are left, a
-# number of slices that is no multiple of a chain's four, K in stretches of which the last is short
-@pytest.mark.parametrize("shape", [(640, 8192, 96), (641, 8194, 160), (700, 8130, 32), (321, 4098, 4128)])
+# number of slices that is no multiple of a chain's four, blocks of K behind one another, two stretches and a part of a third
+@pytest.mark.parametrize("shape", [(640, 8192, 96), (641, 8194, 160), (700, 8130, 32), (1281, 4098, 2080)])
 def test_gemm_f32_many_tiles(ops, shape):
-    """The tiles that load straight into LDS give the bits of the form for few rows."""
+    """The tiles that load straight into LDS give the bits of the form for few rows, and of its gated unit, also for rows
+    that lie apart."""
     m, n, k = shape
     a, w, b = rand((m, k), torch.float32, 13), rand((n, k), torch.float32, 14), rand((n,), torch.float32, 15)
-    assert -(-m // 64) * -(-n // 64) * -(-k // 1024) >= 5 * ops.compute_units()
+    assert -(-m // 64) * -(-(n // 2) // 32) >= 5 * ops.compute_units()  # (with the gate a tile takes 32 of either half)
+    wide = torch.zeros((m, k + 12)).cuda()
+    wide[:, :k] = a
     expect, unit = ops.gemm_f32(a, w, b, form=0), ops.gemm_f32(a, w, gate=True, form=0)
-    assert all(torch.equal(ops.gemm_f32(a, w, b, form=form), expect) for form in (1, 2))
-    assert all(torch.equal(ops.gemm_f32(a, w, gate=True, form=form), unit) for form in (1, 2))
+    for rows in (a, wide[:, :k]):
+        assert torch.equal(ops.gemm_f32(rows, w, b, form=1), expect) and torch.equal(ops.gemm_f32(rows, w, gate=True, form=1), unit)
+    assert torch.equal(ops.gemm_f32(a, w, form=1), ops.gemm_f32(a, w, form=0))
+    assert torch.equal(ops.gemm_f32(a, w, b, form=2), expect) and torch.equal(ops.gemm_f32(a, w, gate=True, form=2), unit)
 
 
-def test_gemm_f32_many_stretches(ops):
-    """Twelve and more tiles to a unit with K in stretches, the last one short: loaded straight into LDS, the same bits."""
-    m, n, k = 600, 4098, 4128
+@pytest.mark.parametrize("shape", [(600, 4098, 4128), (449, 4160, 6144)])
+def test_gemm_f32_many_stretches(ops, shape):
+    """Twelve and more tiles to a unit with K in stretches (the last one short, or all of them whole): loaded straight into
+    LDS, the same bits, the gated unit's too, and for rows that lie apart."""
+    m, n, k = shape
     a, w, b = rand((m, k), torch.float32, 16), rand((n, k), torch.float32, 17), rand((n,), torch.float32, 18)
-    assert -(-m // 64) * -(-n // 64) * -(-k // 1024) >= 12 * ops.compute_units()
-    assert torch.equal(ops.gemm_f32(a, w, b, form=2), ops.gemm_f32(a, w, b, form=0))
-
+    assert -(-m // 64) * -(-n // 64) * -(-k // 1024) >= 12 * ops.compute_units() and ops.f32_bands(m, n, k)[0] == 1
+    wide = torch.zeros((m, k + 4)).cuda()
+    wide[:, :k] = a
+    expect, unit = ops.gemm_f32(a, w, b, form=0), ops.gemm_f32(a, w, gate=True, form=0)
+    for rows in (a, wide[:, :k]):
+        assert torch.equal(ops.gemm_f32(rows, w, b, form=2), expect) and torch.equal(ops.gemm_f32(rows, w, gate=True, form=2), unit)
 
 
 @pytest.mark.parametrize("shape", [(200, 66, 1028), (129, 130, 4100)])
@@ -209,9 +219,10 @@ def test_gemm_tiles(ops, shape, tile):
 
 
 # (rows, columns, K): a stage or fewer of k, fewer slices than stages, edges of 16 and of the tiles, columns that are no
-# multiple of 8 or of 4, as many slices as the loop takes at once and one more
+# multiple of 8, of 4 or of 2.  The loop over whole turns of the stages is entered from twice as many slices as a tile has
+# stages (two to five): never, once and several times, with and without slices that are left behind it
 @pytest.mark.parametrize("shape", [(1, 32, 64), (63, 64, 128), (65, 130, 192), (129, 256, 320), (200, 99, 448), (257, 100, 512),
-                                   (530, 776, 576)])
+                                   (530, 776, 576), (150, 274, 960), (257, 516, 1024), (300, 200, 1088), (131, 72, 2112)])
 @pytest.mark.parametrize("tile", [(64, 64), (96, 64), (96, 128), (128, 64), (128, 128), (128, 192), (128, 256), (192, 128),
                                   (192, 192), (192, 256), (256, 128), (256, 160), (256, 256)])
 def test_gemm_direct(ops, shape, tile):
@@ -226,6 +237,7 @@ def test_gemm_direct(ops, shape, tile):
     rounded = dict(rtol=1e-2, atol=1e-2 * math.sqrt(k))    # ... rounded to bfloat16
     run = lambda epilogue, **more: ops.gemm_tiles(w, epilogue, a, *tile, direct=True, **more)  # noqa: E731
     torch.testing.assert_close(run(ops.TILE_BF16, bias=b).double(), product + b.double(), **rounded)
+    torch.testing.assert_close(run(ops.TILE_BF16).double(), product, **rounded)
     if n % 2 == 0:
         gate, up = product[:, : n // 2], product[:, n // 2:]
         torch.testing.assert_close(run(ops.TILE_SILU).double(), torch.nn.functional.silu(gate) * up, rtol=1e-2, atol=1e-2 * k)
@@ -241,23 +253,29 @@ def test_gemm_direct(ops, shape, tile):
 
 
 @pytest.mark.parametrize("heads", [(4, 2, 128), (3, 1, 96), (14, 2, 64), (2, 2, 32)])
-@pytest.mark.parametrize("tile", [(64, 64), (128, 64), (128, 128), (192, 128), (256, 160), (256, 256)])
-def test_gemm_direct_rope(ops, heads, tile):
-    """... and its q/k/v epilogue: the bits of the plain one and the rotation's kernel behind it."""
+@pytest.mark.parametrize("tile", [(64, 64), (96, 64), (96, 128), (128, 64), (128, 128), (128, 192), (128, 256), (192, 128),
+                                  (192, 192), (192, 256), (256, 128), (256, 160), (256, 256)])
+@pytest.mark.parametrize("k,rotate,write,biased", [(192, True, True, True), (1088, True, True, False), (1024, False, True, True),
+                                                   (576, True, False, True)])
+def test_gemm_direct_rope(ops, heads, tile, k, rotate, write, biased):
+    """... and its q/k/v epilogue, whose rows' places are asked for between the last slices, behind none, one and several
+    turns of the stages: the bits of the plain one and the rotation's kernel behind it."""
     q_heads, kv_heads, dim = heads
-    m, k, page, n = 300, 192, 8, (heads[0] + 2 * heads[1]) * heads[2]
-    a, w, b = rand((m, k), torch.bfloat16, 20), rand((n, k), torch.bfloat16, 21), rand((n,), torch.bfloat16, 22)
+    m, page, n = 300, 8, (heads[0] + 2 * heads[1]) * heads[2]
+    a, w = rand((m, k), torch.bfloat16, 20), rand((n, k), torch.bfloat16, 21)
+    b = rand((n,), torch.bfloat16, 22) if biased else None
     as_dev = lambda values: torch.tensor(values, dtype=torch.int32).cuda()  # noqa: E731
     positions, seqs, slots = as_dev(list(range(3, 203)) + list(range(100))), as_dev([0] * 200 + [1] * 100), as_dev([2, 0])
     table = torch.randperm(96, generator=torch.Generator().manual_seed(23)).to(torch.int32).reshape(3, 32).cuda()
     cos, sin = rand((256, dim // 2), torch.float32, 24), rand((256, dim // 2), torch.float32, 25)
     pools = [torch.zeros((96, kv_heads, page, dim), dtype=torch.bfloat16).cuda(), torch.zeros((96, kv_heads, dim, page), dtype=torch.bfloat16).cuda()]
     plain_pools = [p.clone() for p in pools]
-    got = ops.gemm_tiles_rope(w, a, b, cos, sin, positions, seqs, slots, table, *pools, q_heads, kv_heads, dim, *tile, direct=True)
+    how = dict(rotate=rotate, write_kv=write)
+    got = ops.gemm_tiles_rope(w, a, b, cos, sin, positions, seqs, slots, table, *pools, q_heads, kv_heads, dim, *tile, direct=True, **how)
     expect = ops.gemm_tiles(w, ops.TILE_BF16, a, *tile, bias=b, direct=True)
-    ops.rope_kv_write(expect, cos, sin, positions, seqs, slots, table, *plain_pools, q_heads, kv_heads, dim)
+    ops.rope_kv_write(expect, cos, sin, positions, seqs, slots, table, *plain_pools, q_heads, kv_heads, dim, **how)
     assert torch.equal(got[:, : q_heads * dim], expect[:, : q_heads * dim])
-    assert all(torch.equal(x, y) for x, y in zip(pools, plain_pools))
+    assert all(torch.equal(x, y) for x, y in zip(pools, plain_pools)) and bool(pools[0].any()) == write
 
 
 @pytest.mark.parametrize("heads", [(4, 2, 128), (3, 1, 96), (14, 2, 64), (2, 2, 32)])
@@ -1296,6 +1314,8 @@ def test_products_whose_rows_lie_4_kb_apart_match_float64(ops, shape):
     a, w = rand((m, k), torch.bfloat16, 71), rand((n, k), torch.bfloat16, 72, 0.3)
     want = a.double() @ w.double().t()
     close = dict(rtol=0.0, atol=float(2.0 ** -22 * (a.double().abs() @ w.double().abs().t()).max()))
+    # (the form whose waves share K begins at different k only with one wave over all of it, and one tile of rows)
+    torch.testing.assert_close(ops.gemm_fused(w, ops.EPI_F32, a, plan=(1, 1, 1)).double(), want, **close)
     torch.testing.assert_close(ops.gemm_fused(w, ops.EPI_F32, a).double(), want, **close)
     torch.testing.assert_close(ops.gemm_shared_rows(w, ops.EPI_F32, a).double(), want, **close)
     for parts in (1, 3):
@@ -1305,7 +1325,6 @@ def test_products_whose_rows_lie_4_kb_apart_match_float64(ops, shape):
         gate, up = want[:, : n // 2], want[:, n // 2:]
         torch.testing.assert_close(ops.gemm_shared_rows(w, ops.EPI_SILU, a).double(), gate * torch.sigmoid(gate) * up,
                                    rtol=2 ** -7, atol=2e-3)
-
 
 
 @pytest.mark.parametrize("rows", [4, 16, 40, 90])

@@ -1251,10 +1251,10 @@ def test_a_feed_forward_with_a_forward_of_its_own_runs_in_a_layer(monkeypatch):
 def test_products_whose_operands_the_tiles_do_not_take():
     """Some hundred rows of an operand that is read across its rows, and a stream that starts off a 16-byte line: the plain
     result comes back, as it does for any product that nothing fuses."""
-    from cie_amd.parts.linear import linear, plan_tiles
+    from cie_amd.parts.linear import choose_tiles, linear
 
     rows, n, k = 200, 98, 512
-    assert plan_tiles(rows, n, k) is not None
+    assert choose_tiles(rows, n, k, k) is not None
     g = torch.Generator().manual_seed(9)
     wide, w = torch.randn((rows, 2 * k), generator=g).bfloat16().cuda(), torch.randn((n, k), generator=g).bfloat16().cuda()
     expect = wide[:, ::2].double() @ w.double().t()

@@ -93,7 +93,6 @@ def test_narrow_products_of_a_long_k_take_more_parts():
             assert 1 <= parts <= 16 and stretch * (parts - 1) < k <= stretch * parts, (tiles, k)
 
 
-
 def test_float32_results_share_rows_only_where_the_units_have_work():
     """Heads take the form whose waves own 128 columns a workgroup; a router, an expert's gate, a mixer's or an entry's
     float32 rows, whose few workgroups would walk all of K one after another, do not (17 to 80 rows take it at any width)."""

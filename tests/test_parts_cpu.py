@@ -97,11 +97,11 @@ def test_a_variant_with_a_forward_of_its_own_is_not_given_what_its_base_declares
 
 
 def test_products_of_many_rows_on_the_host_are_torchs():
-    from cie_amd.parts.linear import linear, plan_tiles
+    from cie_amd.parts.linear import choose_tiles, linear
 
     g = torch.Generator().manual_seed(1)
     x, w = torch.randn(200, 512, generator=g).bfloat16(), torch.randn(96, 512, generator=g).bfloat16()
-    assert plan_tiles(200, 96, 512) is not None  # (on the GPU this product goes to the tiles)
+    assert choose_tiles(200, 96, 512, 512) is not None  # (on the GPU this product goes to the tiles)
     assert torch.equal(linear(x, w), torch.nn.functional.linear(x, w))
     assert torch.equal(linear(x, w, into=torch.zeros(200, 96)), torch.nn.functional.linear(x, w))
 
@@ -149,3 +149,32 @@ def test_tiles_are_taken_where_they_were_measured_to_win(behind, parts, rows, n,
     picked = linear.choose_tiles(rows, n, k, k, most_parts=parts, behind=getattr(linear, "BEHIND_" + behind))
     assert picked is None or (picked.direct and tiles[picked[:3]] <= 1.03 * library)
     assert picked is not None or min(tiles.values()) > 0.9 * library
+
+
+@pytest.mark.parametrize("behind", ["NOTHING", "GATE", "BRANCH", "ROTATION"])
+def test_the_tiles_that_are_chosen_are_tiles_there_are(behind):
+    """Over rows, widths and K: a form that the kernel has, parts of K that all have some, sums within their limit, and the
+    tiles that load straight into LDS only for sizes they take; every other K has the other tiles or the library."""
+    from cie_amd.kernels import ops
+    from cie_amd.parts import linear
+
+    taken = 0
+    for rows in (129, 200, 256, 613, 777, 1024, 1999, 2048, 5000):
+        for n in (32, 98, 896, 2048, 4608, 22016, 37888):
+            for k in (64, 512, 896, 2048, 3584, 4104, 11008, 18944, 29568):
+                for most in (1, 8):
+                    picked = linear.choose_tiles(rows, n, k, k + 64, most_parts=most, behind=getattr(linear, "BEHIND_" + behind))
+                    if picked is None:
+                        continue
+                    taken += 1
+                    assert picked.direct == (k % 64 == 0) and 1 <= picked.parts <= most
+                    assert picked[:2] in (ops.DIRECT_SHAPES if picked.direct else ops.TILE_SHAPES)
+                    stretch = -(-(-(-k // picked.parts)) // 64) * 64
+                    assert stretch * (picked.parts - 1) < k
+                    assert picked.parts == 1 or not picked.direct or picked.parts * rows * n * 4 <= linear.PARTS_BYTES
+    assert taken > 400
+    # operands of 2^31 numbers and more are not the tiles' whose places are 32-bit numbers of bytes
+    for rows, n, k, stride in ((256, 1 << 21, 1024, 1024), (1 << 20, 64, 1024, 2048)):
+        assert not ops.direct_fits(rows, n, k, stride)
+        picked = linear.choose_tiles(rows, n, k, stride)
+        assert picked is None or not picked.direct
