@@ -83,13 +83,18 @@ SHARED_LOGIT_FILL = ((3, None), (8, 0.9), (16, 0.75), (80, 0.0))
 SHARED_LOGIT_ROWS, SHARED_LOGIT_TURNS, SHARED_LOGIT_K = 96, (2, 4), 4096
 
 
-def shares_rows_f32(rows: int, n: int, k: int) -> bool:
-    """Whether a float32 result of ``rows`` rows and ``n`` columns takes the shared-rows form."""
-    units, groups = ops.compute_units(), -(-n // 128)
+@functools.lru_cache(maxsize=4096)
+def _shares_rows_f32(rows: int, n: int, k: int, units: int) -> bool:
+    groups = -(-n // 128)
     for upto, fill in SHARED_LOGIT_FILL:
         if rows <= upto:
             return fill is not None and groups >= fill * units * -(-groups // units)
     return rows <= SHARED_LOGIT_ROWS and groups >= SHARED_LOGIT_TURNS[k > SHARED_LOGIT_K] * units
+
+
+def shares_rows_f32(rows: int, n: int, k: int) -> bool:
+    """Whether a float32 result of ``rows`` rows and ``n`` columns takes the shared-rows form."""
+    return _shares_rows_f32(rows, n, k, ops.compute_units())
 
 
 def plan_shared_silu(pairs: int) -> tuple[int, bool]:
@@ -418,8 +423,10 @@ def takes_tiles(rows: int, x: torch.Tensor, weight: torch.Tensor, into: Optional
     kernels, on the GPU, in rows that lie apart and at addresses that 16-byte loads and stores can use.  Whatever else a
     caller brings (rows read across, rows that share their numbers, as one row expanded to many does, a stream that starts
     off a 16-byte line, host tensors) is the library's or torch's, as it was."""
-    return (rows > FUSED_PARTS_ROWS and x.is_cuda and x.stride(1) == 1 and x.stride(0) >= x.shape[1]
-            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+    if rows <= FUSED_PARTS_ROWS or not x.is_cuda:
+        return False
+    apart, inner = x.stride()
+    return (inner == 1 and apart >= x.shape[1] and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
             and (into is None or (into.is_cuda and into.dtype == torch.float32 and into.data_ptr() % 16 == 0)))
 
 
