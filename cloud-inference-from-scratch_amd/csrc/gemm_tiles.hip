@@ -1,5 +1,6 @@
 // bfloat16 products of some hundred rows on the matrix cores: C = A * W^T with A [M, K], W [N, K] bf16 and float32 sums.
 // Products whose K is a multiple of 64 are gemm_direct.hip's (faster at every size measured); this one takes any multiple of 8.
+// What is measured below are products of such a K, from when they were its own: another K takes as many slices.
 //
 // Between the few rows that the streaming kernels take (gemm_fused.hip) and the thousands for which the vendor library
 // is tuned such a product has few tiles: its time is how many tiles meet on one unit, and the launches behind it.  The

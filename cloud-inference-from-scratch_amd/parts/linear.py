@@ -7,9 +7,10 @@ it is the faster one (a small weight, a long K): the hand-written
 matrix-core kernels that stream the weight once and take over their neighbours'
 work: a SiLU-gate behind (``epilogue="silu"``), the add into the float32
 residual stream (``into=residual``), or float32 results for the logits.  They
-come in two forms: waves that share K and own all rows (few rows; the q/k/v,
-o_proj and head products), and waves that own columns and share the rows through
-LDS (the SiLU-gate product up to 64 rows and every product whose K is cut).
+come in two forms: waves that share K and own all rows (few rows; the q/k/v and
+o_proj products, logits of up to 3 rows and narrow float32 results), and waves that
+own columns and share the rows through LDS (the SiLU-gate product up to 96 rows, every
+product whose K is cut, logits of 4 to 96 rows).
 bfloat16 with more rows: tiles of this package's own (``csrc/gemm_direct.hip``, and
 ``csrc/gemm_tiles.hip`` for a K that is no multiple of 64) where they are the faster ones, else the
 vendor library's product (hipBLASLt through a thin cached interface of this
@@ -130,10 +131,12 @@ def plan_shared_parts(tiles: int, k: int) -> tuple[int, int, int]:
 
 
 # Products of more rows than the kernels above take (beyond ``FUSED_PARTS_ROWS``) go to tiles of this package or to the
-# vendor library, whichever the models below say is faster.  These two are fitted to 608 products timed inside captured
-# chains on MI355X with the kernels between them (q/k/v, o_proj, gate/up and down of six shapes from 896 to 8,192 wide, at
-# 16 to 30 row counts from 130 to 2,048).
-# Tiles (within 6 % of the measured, root mean square), us: a start, and per slice of 64 k of a workgroup alone on its unit
+# vendor library, whichever the models below say is faster: the tiles that load straight into LDS (``DIRECT_US``) where K is a
+# multiple of 64, else those of csrc/gemm_tiles.hip (``TILE_US``), each against the one model of the library.
+# ``TILE_US`` and the library's are fitted to 608 products timed inside captured chains on MI355X with the kernels between them
+# (q/k/v, o_proj, gate/up and down of six shapes from 896 to 8,192 wide, at 16 to 30 row counts from 130 to 2,048).  Their K are
+# multiples of 64, which these tiles no longer see; any other K takes them as many slices as the next multiple.
+# Those tiles (within 6 % of the measured, root mean square), us: a start, and per slice of 64 k of a workgroup alone on its unit
 # and of every further one that meets it there (what bounds them is the rate at which a unit is fed from its L2, some 20 bytes
 # a cycle, hence the advantage of large tiles where they are many).  The tiles are dealt to the 8 XCDs in equal runs and each
 # XCD has an eighth of the units: 33 workgroups on one of them take two turns, though there are fewer than 256 in all.
@@ -143,7 +146,8 @@ TILE_PARTS = (1, 2, 3, 4, 6, 8)
 TILE_PARTS_US = 0.356  # parts of K: float32 sums written by the product and read by the norm, us per MB
 XCDS = 8
 # The library (within 12 %; it takes its first choice of algorithm for a row count that does not recur, now and then a bad
-# one: 7B down at 400 rows 200 us where this says 114 and the tiles take 90): the way through one tile's K and its weight rows
+# one: 7B down at 400 rows 200 us where this says 114 and the tiles take 81; 1,999 rows x 6,144 and 4,736, K 2,048, inside a
+# prompt 57 and 55 where it says 41 and 33): the way through one tile's K and its weight rows
 # (us, per 1,000 k, per million weights), and the products at a rate (PFLOP/s) that goes by the tiles of 128 x 128 a unit.
 LIBRARY_US = (8.6, 1.0, 0.40)
 LIBRARY_RATE, LIBRARY_MOST = 0.85, 1.32
@@ -172,10 +176,9 @@ BEHIND_NOTHING = Behind(0.0, 0.0, 3.0, 15.0)
 BEHIND_GATE = Behind(2.15, 1.2, 11.0, 40.0, 1.03)  # the gate's kernel
 BEHIND_BRANCH = Behind(-1.3, 1.9, 3.0, 15.0)     # the norm that adds the branch
 BEHIND_ROTATION = Behind(1.1, 1.8, 11.0, 21.0)   # the rotation and cache write
-# Where the host does not matter the tiles are taken if they are modelled to be faster by the first of these, beyond 25 us by the
-# second (a good algorithm that the library happens to have costs more there).  Of the 608 products 27 are then more than
-# 2 % slower than the library's inside a captured chain (the worst 1.25, the 72B down at 360 rows), and all together 6.3 %
-# faster, 1.3 % from the better of the two each time.
+# Where the host does not matter the tiles of csrc/gemm_tiles.hip are taken if they are modelled to be faster by the first of
+# these, beyond 25 us by the second (a good algorithm that the library happens to have costs more there): of the 608 products 27
+# were then more than 2 % slower than the library's inside a captured chain, and all together 6.3 % faster.
 TILES_MARGIN, TILES_MARGIN_LONG, TILES_LONG_US = 1.05, 1.15, 25.0
 
 
@@ -196,7 +199,9 @@ def _library_us(rows: int, n: int, k: int, units: int, tuned: int) -> float:
 
 # The tiles whose operands go straight into LDS (csrc/gemm_direct.hip; K a multiple of 64), by the same model, fitted to 7,500
 # timings (0.5B, 3B, 7B and 14B widths at 16 row counts from 112 to 2,048; 10 % root mean square): the form it picks takes
-# 1.7 % more than the best of all in the mean.  Against the tiles above and the library, us, each product alone (the kernel
+# 1.7 % more than the best of all in the mean.  (Over 500 further products of any width and K, without and with the gate, 19 %:
+# it leaves out the weight's way from memory and the result's to it, some 0.3 us a million weights and 0.6 a million results,
+# which hardly choose between the forms.)  Against the tiles above and the library, us, each product alone (the kernel
 # behind the library's not counted): 3B gate/up 256 rows 40 -> 33, 777 81 -> 72, 2,048 186 -> 157; down 613 47 -> 36, 2,048
 # 100 -> 91; 7B gate/up 777 272 -> 175, 2,048 541 -> 445, down 777 167 -> 98.  What decides is how the turns come out: 777 rows
 # x 37,888 are 740 tiles of 256 x 160, three turns of 256 units, and 1,036 of 256 x 128, five.
