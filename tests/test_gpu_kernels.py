@@ -252,6 +252,25 @@ def test_gemm_direct(ops, shape, tile):
             torch.testing.assert_close(got.double().sum(0), product + b.double(), **sums)
 
 
+@pytest.mark.parametrize("gate", [0.0, 0.5, -0.5, 9.0, -9.0, 40.0, -40.0, -80.0, 1e30, -1e30, math.inf])
+def test_gemm_direct_gate_over_its_range(ops, gate):
+    """Each row's one number k = 0 is its gate, k = 1 its up; the result is rounded once to bf16 (2^-9), behind float32
+    steps of a few 2^-24; what lies below float32's normal numbers is nothing."""
+    a = torch.zeros((130, 64), dtype=torch.bfloat16, device="cuda")
+    a[:, 0], a[:, 1] = gate, 1.5
+    w = torch.zeros((64, 64), dtype=torch.bfloat16, device="cuda")
+    w[:32, 0], w[32:, 1] = 1.0, 1.0
+    if math.isinf(gate):
+        w[32:, 0], a[:, 1] = 1.0, 0.0  # (no 0 x inf in the up columns)
+    got = ops.gemm_tiles(w, ops.TILE_SILU, a, 64, 64, direct=True).double()
+    x = a[0, 0].double().cpu()
+    expect = x * torch.sigmoid(x) * (x if math.isinf(gate) else 1.5)
+    if math.isinf(gate):
+        assert torch.isinf(got).all() and (got > 0).all()
+    else:
+        assert (got.cpu() - expect).abs().max() <= expect.abs() * 2.0 ** -8.9 + 2.0 ** -126
+
+
 @pytest.mark.parametrize("heads", [(4, 2, 128), (3, 1, 96), (14, 2, 64), (2, 2, 32)])
 @pytest.mark.parametrize("tile", [(64, 64), (96, 64), (96, 128), (128, 64), (128, 128), (128, 192), (128, 256), (192, 128),
                                   (192, 192), (192, 256), (256, 128), (256, 160), (256, 256)])
