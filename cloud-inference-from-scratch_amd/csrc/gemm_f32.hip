@@ -10,7 +10,10 @@
 //
 // Two forms:
 //
-// * gemm_f32_rows_kernel, few rows: bound by the stream of W.  A workgroup owns 8 to 32 columns and 8 to 32 rows and
+// * gemm_f32_rows_kernel, few rows: bound by the stream of W and, in a decode layer, by its launches (some 4.8 us each before
+//   one streams anything).  It can take its neighbours' work with it, all of it in the bits that their own kernels give: the
+//   RMS norm in front of it (every workgroup sums the few rows' squares while its first pieces of W are on their way), the add
+//   into the stream behind it, the rotation and the cache write of q/k/v.  A decode layer has six kernels so, not nine.  A workgroup owns 8 to 32 columns and 8 to 32 rows and
 //   goes on to the next columns until none are left; its waves take the blocks of K in turn, each wave fetching W and
 //   A as 128-byte row segments (8 lanes to a segment: a load in which every lane reads another row keeps the address
 //   unit busy four times as long), four 32-wide pieces ahead in registers and across the end of a tile, and turning
@@ -81,33 +84,74 @@ __device__ __forceinline__ floatx4 inside(floatx4 v, int k, int K) {
 
 __device__ __forceinline__ float gated(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
 
+// What the rows kernel does beside the product: nothing; the norm of its rows; that, the rotation and the cache write.
+enum { kPlain = 0, kNormed = 1, kRotated = 2 };
+
+struct RowsBeside {
+    const float* norm_weight;  // kNormed, kRotated: A is the stream, its rows' norm is multiplied
+    float eps;
+    int into;                  // kPlain: C is added to, not written
+    // kRotated: W stacks the rows of q, k and v heads; queries go to C, keys and values to the cache
+    const float *cos_table, *sin_table;  // [positions, rotary_dim / 2]
+    const int *positions, *seq_of_token, *seq_slot, *block_table;
+    int table_width;
+    float *k_pool, *v_pool;    // [pages, Hkv, page_size, D], [pages, Hkv, D, page_size]
+    int q_heads, kv_heads, head_dim, rotary_dim, page_size, rotate, write_kv;
+};
+
+// Where pair i (0..7) of group j (0..head_dim / 16 - 1) of a head lies: its first dimension, and how far on its partner is.  The
+// first rotary_dim / 16 groups are dimensions of the rotated part's first half, the others of what does not rotate.
+struct HeadPair {
+    int first, apart;
+    bool rotates;
+};
+__device__ __forceinline__ HeadPair head_pair(const RowsBeside& b, int j, int i) {
+    const int turning = b.rotary_dim / 16;
+    if (j < turning) return {j * 8 + i, b.rotary_dim / 2, b.rotate != 0};
+    return {b.rotary_dim + (j - turning) * 8 + i, (b.head_dim - b.rotary_dim) / 2, false};
+}
+
+constexpr int kSegment = 8 * kWave;      // of a row: what a wave of the norm's own kernel sums
+constexpr int kNormSegments = 16;        // rows of up to this many segments ...
+constexpr int kNormTasks = 32;           // ... and so many segments in all: what 64 KB of LDS hold
+
 // kRows rows (8, 16 or 32) by kColumns columns (8, 16 or 32; with the gate kColumns / 2 of each half), in tiles of 16
 // of which the last may be half empty.  kWaves waves share K.  Workgroup x takes the columns' tiles x, x + gridDim.x, ...
-template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec>
+template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec, int kBeside = kPlain>
 __global__ void __launch_bounds__(kWaves * kWave)
 gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-                     float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
+                     float* __restrict__ C, int M, int N, int K, int lda, int ldc, RowsBeside beside) {
     constexpr int kRowTiles = (kRows + 15) / 16, kColumnTiles = (kColumns + 15) / 16;
-    constexpr int kTiles = kRowTiles + kColumnTiles;
+    constexpr bool kOwnRows = kBeside != kPlain;  // the normed rows lie in LDS, whole
+    constexpr int kTiles = kRowTiles + kColumnTiles, kStaged = kOwnRows ? kColumnTiles : kTiles;
     constexpr int kSums = kRowTiles * kColumnTiles * 256;
     constexpr int kAhead = kPiecesPerChain;  // pieces on their way
     constexpr int kThreads = kWaves * kWave;
     constexpr int kOwned = (kSums + kThreads - 1) / kThreads;
     constexpr int kStep = kGate ? kColumns / 2 : kColumns;  // output columns of a tile
     static_assert(!kGate || kColumns == 32 || kColumns == 16, "a gate's tile holds as many columns of either half");
-    __shared__ float stage_all[kWaves * kTiles * kTileFloats];
+    static_assert(kBeside == kPlain || (kVec && kRows <= 16), "a few rows in 16-byte pieces");
+    static_assert(kBeside != kRotated || (!kGate && kColumns == 16 && kRows * 8 <= kThreads), "8 dimensions and their partners");
+    __shared__ float stage_all[kWaves * kStaged * kTileFloats];
     __shared__ float sums[2][kWaves * kSums];
     const int lane = threadIdx.x % kWave;
     const int wave = threadIdx.x / kWave;
-    float* stage = stage_all + wave * kTiles * kTileFloats;
+    float* stage = stage_all + wave * kStaged * kTileFloats;
     const int m0 = blockIdx.y * kRows;
     const int width = kGate ? N / 2 : N;  // output columns
     const int column_tiles = (width + kStep - 1) / kStep;
     const int blocks = (K + kBlockK - 1) / kBlockK;
     const int rounds = (blocks + kWaves - 1) / kWaves;
 
+    // kRotated: tile t takes the eight pairs of group j of head h, t = h * D / 16 + j
+    const int per_head = kBeside == kRotated ? beside.head_dim / 16 : 1;
     // row r (0..kColumns - 1) of a tile of W
     auto weight_row = [&](int tile, int r) {
+        if constexpr (kBeside == kRotated) {
+            const int head = tile / per_head;
+            const HeadPair pair = head_pair(beside, tile - head * per_head, r % 8);
+            return W + static_cast<size_t>(head * beside.head_dim + pair.first + r / 8 * pair.apart) * K;
+        }
         const int n = kGate ? min(tile * kStep + r % kStep, width - 1) + (r / kStep) * width : min(tile * kStep + r, N - 1);
         return W + static_cast<size_t>(n) * K;
     };
@@ -117,6 +161,8 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 #pragma unroll
     for (int i = 0; i < kALoads; ++i) a_row[i] = A + static_cast<size_t>(min(m0 + 8 * i + lane / 8, M - 1)) * lda;
 
+    // (a K of up to one chain's has no second chain)
+    const int halves = K <= kBlockK / 2 ? 1 : 2, pieces = halves * kPiecesPerChain;
     // the piece that is fetched next: its place in the block, the round and the tile
     int f_piece = 0, f_round = 0, f_tile = blockIdx.x;
     const float* w_row[kWLoads];
@@ -127,9 +173,10 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
         const int k = (wave + f_round * kWaves) * kBlockK + f_piece * kPiece + 4 * chunk;
 #pragma unroll
         for (int i = 0; i < kWLoads; ++i) w[i] = load4<kVec>(w_row[i], k, K);
+        if constexpr (!kOwnRows)
 #pragma unroll
-        for (int i = 0; i < kALoads; ++i) a[i] = load4<kVec>(a_row[i], k, K);
-        if (++f_piece == kPiecesPerBlock) {
+            for (int i = 0; i < kALoads; ++i) a[i] = load4<kVec>(a_row[i], k, K);
+        if (++f_piece == pieces) {
             f_piece = 0;
             if (++f_round == rounds) {
                 f_round = 0;
@@ -139,15 +186,92 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
             }
         }
     };
+    // where the token of this thread's result (row threadIdx.x / 8, pair threadIdx.x % 8 of a tile) sits: three loads, each of
+    // which needs the one before, between what else is on its way
+    const int place_row = min(m0 + static_cast<int>(threadIdx.x) / 8 % kRows, M - 1);
+    int pos = 0, page = -1;
+    if constexpr (kBeside == kRotated) {
+        pos = beside.positions[place_row];
+        if (beside.write_kv) page = beside.seq_of_token[place_row];
+    }
+    // The norm's rows: asked for in front of the first pieces of W (behind them they would wait for all of these), summed
+    // segment by segment as the norm's kernel sums them, and left in LDS, where the product takes its operand from: rows
+    // `apart` numbers apart, zeros behind K up to the last block's end.
+    __shared__ __attribute__((aligned(16))) float own_rows[kOwnRows ? kNormTasks * kSegment + 4 * kRows : 1];
+    const int apart = blocks * kBlockK + 4;
+    constexpr int kTogether = kNormTasks / kWaves;
+    const int segments = (K + kSegment - 1) / kSegment, tasks = min(kRows, M - m0) * segments;
+    eight_t own[kTogether] = {}, gain[kTogether] = {};
+    if constexpr (kOwnRows) {
+        const int first = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll
+        for (int i = 0; i < kTogether; ++i) {
+            if (first + i * kWaves >= tasks) break;
+            const int task = first + i * kWaves, row = task / segments;
+            const int h = min((task - row * segments) * kSegment + lane * 8, K - 8);
+            own[i] = load_eight(A + static_cast<size_t>(m0 + row) * lda + h);
+            gain[i] = load_eight(beside.norm_weight + h);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int s = 0; s < kAhead; ++s) fetch(w_ahead[s], a_ahead[s]);
+    if constexpr (kOwnRows) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (kBeside == kRotated && beside.write_kv) page = beside.seq_slot[page];
+        __shared__ float segment_sums[kNormTasks];
+        const int first = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll
+        for (int i = 0; i < kTogether; ++i) {
+            const int task = first + i * kWaves, row = task / segments, h = (task - row * segments) * kSegment + lane * 8;
+            if (task >= tasks) break;
+            const float sum = wave_sum(h < K ? 0.f + sum_of_squares(own[i]) : 0.f);
+            if (lane == 0) segment_sums[task] = sum;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kTogether; ++i) {
+            const int task = first + i * kWaves, row = task / segments, h = (task - row * segments) * kSegment + lane * 8;
+            if (task >= tasks) break;
+            float sum = 0.f;
+            for (int s = 0; s < segments; ++s) sum += segment_sums[row * segments + s];
+            const float inverse = 1.0f / sqrtf(sum / static_cast<float>(K) + beside.eps);
+            if (h < blocks * kBlockK) store_eight(own_rows + row * apart + h, h < K ? (own[i] * inverse) * gain[i] : eight_t{});
+        }
+        if (kBeside == kRotated && beside.write_kv)
+            page = beside.block_table[static_cast<size_t>(page) * beside.table_width + pos / beside.page_size];
+        __syncthreads();
+    }
+    const float* own_row[kRowTiles];  // this lane's rows of A (one past the last reads that one again, and is not stored)
+#pragma unroll
+    for (int rt = 0; rt < kRowTiles; ++rt) own_row[rt] = own_rows + min(16 * rt + lane % 16, min(kRows, M - m0) - 1) * apart;
 
     int turn = 0;  // two sets of sums take turns: the next block's are written while others still read this one's
     for (int tile = blockIdx.x; tile < column_tiles; tile += gridDim.x) {
         float total[kOwned] = {}, stretch[kOwned] = {};
+        // a thread's sum e: tile e / 256 (column tiles outer), column 4 * (place / 16) + e % 4, row place % 16
+        auto column_of = [&](int e) { return 16 * (e / 256 / kRowTiles) + 4 * ((e / 4) % kWave / 16) + e % 4; };
+        auto row_of = [&](int e) { return 16 * (e / 256 % kRowTiles) + (e / 4) % kWave % 16; };
+        float old[kOwned] = {};  // (of a C that is added to: on its way while W streams)
+        if (kBeside == kPlain && !kGate && beside.into)
+#pragma unroll
+            for (int o = 0; o < kOwned; ++o) {
+                const int e = min(static_cast<int>(threadIdx.x) + o * kThreads, kSums - 1);
+                old[o] = C[static_cast<size_t>(min(m0 + row_of(e), M - 1)) * ldc + min(tile * kStep + column_of(e), N - 1)];
+            }
+        float c = 1.f, s = 0.f;  // this thread's angle
+        if constexpr (kBeside == kRotated) {
+            const int head = tile / per_head;
+            const HeadPair pair = head_pair(beside, tile - head * per_head, threadIdx.x % 8);
+            if (pair.rotates && head < beside.q_heads + beside.kv_heads) {
+                const size_t at = static_cast<size_t>(pos) * (beside.rotary_dim / 2) + pair.first;
+                c = beside.cos_table[at];
+                s = beside.sin_table[at];
+            }
+        }
         for (int round = 0; round < rounds; ++round) {
             floatx4 block[kColumnTiles][kRowTiles] = {};
-            for (int half = 0; half < 2; ++half) {
+            for (int half = 0; half < halves; ++half) {
                 floatx4 acc[kColumnTiles][kRowTiles] = {};
 #pragma unroll
                 for (int s = 0; s < kAhead; ++s) {
@@ -156,21 +280,28 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 #pragma unroll
                     for (int i = 0; i < kWLoads; ++i)
                         *reinterpret_cast<floatx4*>(stage + chunk_at(8 * i + lane / 8, chunk)) = inside<kVec>(w_ahead[s][i], k, K);
+                    if constexpr (!kOwnRows)
 #pragma unroll
-                    for (int i = 0; i < kALoads; ++i)
-                        *reinterpret_cast<floatx4*>(stage + kColumnTiles * kTileFloats + chunk_at(8 * i + lane / 8, chunk)) =
-                            inside<kVec>(a_ahead[s][i], k, K);
+                        for (int i = 0; i < kALoads; ++i)
+                            *reinterpret_cast<floatx4*>(stage + kColumnTiles * kTileFloats + chunk_at(8 * i + lane / 8, chunk)) =
+                                inside<kVec>(a_ahead[s][i], k, K);
                     fetch(w_ahead[s], a_ahead[s]);
                     __builtin_amdgcn_wave_barrier();
 #pragma unroll
                     for (int g = 0; g < kPiece / 16; ++g) {
                         floatx4 f[kTiles];
 #pragma unroll
-                        for (int t = 0; t < kTiles; ++t) {
+                        for (int t = 0; t < kStaged; ++t) {
                             // (a half empty tile reads its 8 rows twice; what comes of the copies is not stored)
                             const int r = (t < kColumnTiles ? kColumns : kRows) == 8 ? lane % 8 : lane % 16;
                             f[t] = operand(stage + t * kTileFloats, r, g, lane / 16);
                         }
+                        if constexpr (kOwnRows)
+#pragma unroll
+                            for (int rt = 0; rt < kRowTiles; ++rt)
+#pragma unroll
+                                for (int t = 0; t < 4; ++t)  // (a block past the last reads that one, and is not summed)
+                                    f[kColumnTiles + rt][t] = own_row[rt][min(wave + round * kWaves, blocks - 1) * kBlockK + (half * kAhead + s) * kPiece + 16 * g + 4 * t + lane / 16];
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -209,8 +340,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
                     }
             }
         }
-        // a thread's sum: tile e / 256 (column tiles outer), column 4 * (place / 16) + e % 4, row place % 16
-        if constexpr (kGate) {
+        if constexpr (kGate || kBeside == kRotated) {
             // the two halves of a column belong to two threads (or to one thread's two sums): they meet in LDS
             float* all = sums[turn];
             turn ^= 1;
@@ -220,24 +350,50 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
                 if (e < kSums) all[e] = total[o];
             }
             __syncthreads();
-            for (int at = threadIdx.x; at < kRows * kStep; at += kThreads) {
-                const int c = at % kStep, r = at / kStep;
-                const int n = tile * kStep + c, m = m0 + r;
-                auto sum_of = [&](int column) {
-                    return all[(column / 16 * kRowTiles + r / 16) * 256 + ((column % 16) / 4 * 16 + r % 16) * 4 + column % 4];
-                };
-                if (m < M && n < width)
-                    C[static_cast<size_t>(m) * ldc + n] = gated(sum_of(c), sum_of(kStep + c));
+            auto sum_of = [&](int r, int column) {
+                return all[(column / 16 * kRowTiles + r / 16) * 256 + ((column % 16) / 4 * 16 + r % 16) * 4 + column % 4];
+            };
+            if constexpr (kBeside == kRotated) {
+                const int r = threadIdx.x / 8, i = threadIdx.x % 8, m = m0 + r;
+                if (r < kRows && m < M) {
+                    const int head = tile / per_head, D = beside.head_dim;
+                    const HeadPair pair = head_pair(beside, tile - head * per_head, i);
+                    const int d = pair.first, half = pair.apart, n = head * D + d;
+                    const float x1 = sum_of(r, i) + (bias ? bias[n] : 0.f), x2 = sum_of(r, 8 + i) + (bias ? bias[n + half] : 0.f);
+                    const bool turns = pair.rotates && head < beside.q_heads + beside.kv_heads;
+                    const float y1 = turns ? __builtin_fmaf(x1, c, -(x2 * s)) : x1;  // (rounded as the rotation's kernel does)
+                    const float y2 = turns ? __builtin_fmaf(x2, c, x1 * s) : x2;
+                    if (head < beside.q_heads) {
+                        C[static_cast<size_t>(m) * ldc + n] = y1;
+                        C[static_cast<size_t>(m) * ldc + n + half] = y2;
+                    } else if (page >= 0) {  // (no page: nothing is to be written)
+                        const int in_page = pos % beside.page_size;
+                        const size_t head_base = (static_cast<size_t>(page) * beside.kv_heads + (head - beside.q_heads) % beside.kv_heads) * beside.page_size * D;
+                        if (head < beside.q_heads + beside.kv_heads) {
+                            beside.k_pool[head_base + static_cast<size_t>(in_page) * D + d] = y1;
+                            beside.k_pool[head_base + static_cast<size_t>(in_page) * D + d + half] = y2;
+                        } else {  // element d of the token goes to [d, in_page]
+                            beside.v_pool[head_base + static_cast<size_t>(d) * beside.page_size + in_page] = y1;
+                            beside.v_pool[head_base + static_cast<size_t>(d + half) * beside.page_size + in_page] = y2;
+                        }
+                    }
+                }
+            } else {
+                for (int at = threadIdx.x; at < kRows * kStep; at += kThreads) {
+                    const int n = tile * kStep + at % kStep, m = m0 + at / kStep;
+                    if (m < M && n < width)
+                        C[static_cast<size_t>(m) * ldc + n] = gated(sum_of(at / kStep, at % kStep), sum_of(at / kStep, kStep + at % kStep));
+                }
             }
         } else {
 #pragma unroll
             for (int o = 0; o < kOwned; ++o) {
                 const int e = threadIdx.x + o * kThreads;
-                const int at = (e / 4) % kWave;
-                const int c = 16 * (e / 256 / kRowTiles) + 4 * (at / 16) + e % 4, r = 16 * (e / 256 % kRowTiles) + at % 16;
-                const int n = tile * kStep + c, m = m0 + r;
-                if (e < kSums && c < kColumns && r < kRows && m < M && n < N)
-                    C[static_cast<size_t>(m) * ldc + n] = total[o] + (bias ? bias[n] : 0.f);
+                const int n = tile * kStep + column_of(e), m = m0 + row_of(e);
+                if (e < kSums && column_of(e) < kColumns && row_of(e) < kRows && m < M && n < N) {
+                    const float sum = total[o] + (bias ? bias[n] : 0.f);
+                    C[static_cast<size_t>(m) * ldc + n] = beside.into ? old[o] + sum : sum;
+                }
             }
         }
     }
@@ -584,6 +740,7 @@ struct Product {
     const float *A, *W, *bias;
     float *C, *parts;
     int M, N, K, lda, ldc, units;
+    RowsBeside beside;
 };
 
 // Whether `workgroups` tiles load straight into LDS: whole slices of K, places in the operands in 32 bits of bytes, and so many
@@ -598,7 +755,7 @@ bool goes_direct(const Product& p, long workgroups, long per_unit) {
            static_cast<long>(p.M) * p.lda < (1L << 30);
 }
 
-template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec>
+template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec, int kBeside = kPlain>
 void run_rows(hipStream_t s, const Product& p) {
     const int step = kGate ? kColumns / 2 : kColumns;
     const int tiles = ((kGate ? p.N / 2 : p.N) + step - 1) / step;
@@ -608,9 +765,9 @@ void run_rows(hipStream_t s, const Product& p) {
     // a unit, whose columns never exceed four a unit: all at once (N 14,000, K 2,048 at 4 rows 25.9; by their LDS 27.4)
     constexpr int kRowTiles = (kRows + 15) / 16, kColumnTiles = (kColumns + 15) / 16;
     constexpr int kLds = kWaves * 2048 * (kRowTiles + kColumnTiles + kRowTiles * kColumnTiles);
-    const int most = p.units * (kRows <= 16 && kColumns == 16 ? 32 / kWaves : 160 * 1024 / kLds);
+    const int most = p.units * (kBeside != kPlain ? 1 : kRows <= 16 && kColumns == 16 ? 32 / kWaves : 160 * 1024 / kLds);
     dim3 grid(tiles < most ? tiles : most, (p.M + kRows - 1) / kRows);
-    gemm_f32_rows_kernel<kRows, kColumns, kWaves, kGate, kVec><<<grid, kWaves * kWave, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc);
+    gemm_f32_rows_kernel<kRows, kColumns, kWaves, kGate, kVec, kBeside><<<grid, kWaves * kWave, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, p.beside);
 }
 
 template <bool kGate, bool kVec>
@@ -663,6 +820,30 @@ void run_few(hipStream_t s, const Product& p, bool vec) {
     else eight ? run_rows<8, 16, 8, kGate, true>(s, p) : run_rows<16, 16, 8, kGate, true>(s, p);
 }
 
+// The same choice for up to 16 rows with their norm (and the rotation) beside the product; no width takes 8 columns here.
+template <bool kGate, int kBeside>
+void run_few_beside(hipStream_t s, const Product& p) {
+    const bool wide = kBeside == kNormed && p.N >= 64 * p.units, shallow = p.K <= 4 * kBlockK, eight = p.M <= 8;
+    if constexpr (kBeside == kNormed) {
+        if (wide) {
+            if (shallow) eight ? run_rows<8, 32, 4, kGate, true, kBeside>(s, p) : run_rows<16, 32, 4, kGate, true, kBeside>(s, p);
+            else eight ? run_rows<8, 32, 8, kGate, true, kBeside>(s, p) : run_rows<16, 32, 8, kGate, true, kBeside>(s, p);
+            return;
+        }
+    }
+    if (shallow) eight ? run_rows<8, 16, 4, kGate, true, kBeside>(s, p) : run_rows<16, 16, 4, kGate, true, kBeside>(s, p);
+    else eight ? run_rows<8, 16, 8, kGate, true, kBeside>(s, p) : run_rows<16, 16, 8, kGate, true, kBeside>(s, p);
+}
+
+bool on_16_bytes(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+// Up to 16 rows of a float32 stream whose norm the product makes itself.
+bool takes_norm(const float* stream, const float* W, const float* norm_weight, float eps, int M, int K) {
+    return M >= 1 && M <= 16 && K >= 8 && K % 8 == 0 && K <= kNormSegments * kSegment &&
+           M * ((K + kSegment - 1) / kSegment) <= kNormTasks && eps > 0.f && stream && W && norm_weight &&
+           on_16_bytes(stream) && on_16_bytes(W) && on_16_bytes(norm_weight);
+}
+
 template <bool kGate>
 void run_form(hipStream_t s, const Product& p, int form, bool vec) {
     if (form == 0) run_few<kGate>(s, p, vec);
@@ -684,8 +865,56 @@ CIE_API int cie_gemm_f32(void* stream, const float* A, const float* W, const flo
     if ((form == 0 && M > 8 * 65535) || (form == 2 && (M > 65535 || K > 65535 * kStretch))) return CIE_BAD_ARGUMENT;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool vec = K % 4 == 0 && lda % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0;
-    const Product p{A, W, bias, C, parts, M, N, K, lda, ldc, units};
+    const Product p{A, W, bias, C, parts, M, N, K, lda, ldc, units, {}};
     if (gate) run_form<true>(s, p, form, vec);
     else run_form<false>(s, p, form, vec);
+    return cie_after_launch();
+}
+
+// Few rows: C [M, N] (rows ldc apart) += A W^T (+ bias), added to as the norm's kernel would add the product to its stream.
+CIE_API int cie_gemm_f32_into(void* stream, const float* A, const float* W, const float* bias, float* C, int M, int N, int K,
+                              int lda, int ldc, int units) {
+    if (M < 0 || N <= 0 || K <= 0 || lda < K || ldc < N || units < 1 || M > 8 * 65535) return CIE_BAD_ARGUMENT;
+    if (M == 0) return CIE_OK;
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && on_16_bytes(A) && on_16_bytes(W);
+    Product p{A, W, bias, C, nullptr, M, N, K, lda, ldc, units, {}};
+    p.beside.into = 1;
+    run_few<false>(static_cast<hipStream_t>(stream), p, vec);
+    return cie_after_launch();
+}
+
+// Up to 16 rows, and rows * ceil(K / 512) up to 32: C = norm(rows of the stream [M, K], contiguous) W^T (+ bias), or its gated unit.  K a multiple of 8, up to
+// 8,192; stream, W and the norm's weight at multiples of 16 bytes.
+CIE_API int cie_gemm_f32_normed(void* stream, const float* rows, const float* norm_weight, float eps, const float* W, const float* bias,
+                                float* C, int M, int N, int K, int ldc, int gate, int units) {
+    if (!takes_norm(rows, W, norm_weight, eps, M, K) || N <= 0 || units < 1 || !C) return CIE_BAD_ARGUMENT;
+    if (ldc < (gate ? N / 2 : N) || (gate && (N % 2 || bias))) return CIE_BAD_ARGUMENT;
+    Product p{rows, W, bias, C, nullptr, M, N, K, K, ldc, units, {}};
+    p.beside.norm_weight = norm_weight;
+    p.beside.eps = eps;
+    if (gate) run_few_beside<true, kNormed>(static_cast<hipStream_t>(stream), p);
+    else run_few_beside<false, kNormed>(static_cast<hipStream_t>(stream), p);
+    return cie_after_launch();
+}
+
+// The same for a q/k/v weight (heads of head_dim dimensions, of which the first rotary_dim rotate, multiples of 16): rotated queries go to C [M, N], rotated keys
+// and values to the cache.
+CIE_API int cie_gemm_f32_normed_rope(void* stream, const float* rows, const float* norm_weight, float eps, const float* W, const float* bias,
+                                     float* C, int M, int N, int K, const float* cos_table, const float* sin_table,
+                                     const int* positions, const int* seq_of_token, const int* seq_slot, const int* block_table,
+                                     int table_width, float* k_pool, float* v_pool, int q_heads, int kv_heads, int head_dim,
+                                     int rotary_dim, int page_size, int rotate, int write_kv, int units) {
+    if (!takes_norm(rows, W, norm_weight, eps, M, K) || units < 1 || !C) return CIE_BAD_ARGUMENT;
+    if (q_heads <= 0 || kv_heads <= 0 || head_dim <= 0 || head_dim % 16 || rotary_dim <= 0 || rotary_dim % 16 ||
+        rotary_dim > head_dim || page_size <= 0 || table_width <= 0 ||
+        N != (q_heads + 2 * kv_heads) * head_dim)
+        return CIE_BAD_ARGUMENT;
+    if (!positions || (rotate && (!cos_table || !sin_table)) ||
+        (write_kv && (!seq_of_token || !seq_slot || !block_table || !k_pool || !v_pool)))
+        return CIE_BAD_ARGUMENT;
+    const Product p{rows, W, bias, C, nullptr, M, N, K, K, N, units,
+                    {norm_weight, eps, 0, cos_table, sin_table, positions, seq_of_token, seq_slot, block_table, table_width, k_pool,
+                     v_pool, q_heads, kv_heads, head_dim, rotary_dim, page_size, rotate, write_kv}};
+    run_few_beside<false, kRotated>(static_cast<hipStream_t>(stream), p);
     return cie_after_launch();
 }

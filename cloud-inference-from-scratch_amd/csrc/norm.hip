@@ -38,23 +38,11 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ residual, const T* __rest
         dst[h] = from_float<T>((staged[h] * inv) * to_float(weight[h]));
 }
 
-// Eight neighbouring numbers as float32, in 16-byte pieces.
-typedef float eight_t __attribute__((ext_vector_type(8)));
-typedef float half_eight_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ eight_t load_eight(const float* p) {
-    const half_eight_t lo = reinterpret_cast<const half_eight_t*>(p)[0], hi = reinterpret_cast<const half_eight_t*>(p)[1];
-    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-}
 __device__ __forceinline__ eight_t load_eight(const bf16_t* p) {
     const uint4 raw = *reinterpret_cast<const uint4*>(p);
     return eight_t{__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xffff0000u), __uint_as_float(raw.y << 16),
                    __uint_as_float(raw.y & 0xffff0000u), __uint_as_float(raw.z << 16), __uint_as_float(raw.z & 0xffff0000u),
                    __uint_as_float(raw.w << 16), __uint_as_float(raw.w & 0xffff0000u)};
-}
-__device__ __forceinline__ void store_eight(float* p, eight_t v) {
-    reinterpret_cast<half_eight_t*>(p)[0] = __builtin_shufflevector(v, v, 0, 1, 2, 3);
-    reinterpret_cast<half_eight_t*>(p)[1] = __builtin_shufflevector(v, v, 4, 5, 6, 7);
 }
 __device__ __forceinline__ void store_eight(bf16_t* p, eight_t v) {
     *reinterpret_cast<uint4*>(p) = uint4{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
@@ -99,8 +87,7 @@ add_rmsnorm_vec8_kernel(float* __restrict__ residual, const T* __restrict__ bran
         if (store) store_eight(res + h, x);
         if (h == h0) own = x;
         else store_eight(staged + h, x);
-        sum_sq += ((x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3])) +
-                  ((x[4] * x[4] + x[5] * x[5]) + (x[6] * x[6] + x[7] * x[7]));
+        sum_sq += sum_of_squares(x);
     }
     const float total = block_sum(sum_sq, scratch);
     const float inv = 1.0f / sqrtf(total / static_cast<float>(hidden) + eps);

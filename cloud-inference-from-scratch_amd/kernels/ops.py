@@ -583,6 +583,111 @@ def gemm_f32(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
     return out
 
 
+F32_FEW_ROWS = 16  # the most rows that the float32 product of few rows takes its neighbours' work along for
+F32_NORM_WIDTH = 8192  # ... the widest rows whose norm it makes,
+F32_NORM_SEGMENT, F32_NORM_SEGMENTS = 512, 32  # and how many segments of a row in all, which lie in LDS
+
+
+def folds_norm_f32(stream: torch.Tensor) -> bool:
+    """Whether :func:`gemm_f32_normed` and :func:`gemm_f32_qkv_rope` take this float32 stream."""
+    rows, width = stream.shape
+    return (1 <= rows <= F32_FEW_ROWS and 8 <= width <= F32_NORM_WIDTH and width % 8 == 0
+            and rows * -(-width // F32_NORM_SEGMENT) <= F32_NORM_SEGMENTS and stream.is_cuda
+            and stream.dtype == torch.float32 and stream.is_contiguous() and stream.data_ptr() % 16 == 0)
+
+
+def _check_normed_f32(stream: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor,
+                      bias: Optional[torch.Tensor]) -> tuple[int, int, int]:
+    if not (stream.dim() == 2 and folds_norm_f32(stream)):
+        raise ValueError(f"the product makes the norm of 1 to {F32_FEW_ROWS} contiguous float32 rows of up to {F32_NORM_WIDTH} "
+                         f"numbers (a multiple of 8; {F32_NORM_SEGMENTS} segments of {F32_NORM_SEGMENT} in all) on a 16-byte "
+                         f"line itself, not of {tuple(stream.shape)}")
+    _gpu("weight", weight, torch.float32, 2)
+    _gpu("norm_weight", norm_weight, torch.float32, 1)
+    m, k = stream.shape
+    n = weight.shape[0]
+    if not (weight.shape[1] == k and norm_weight.shape[0] == k and eps > 0):
+        raise ValueError(f"weight {tuple(weight.shape)} and norm weight {tuple(norm_weight.shape)} do not fit rows of K={k}")
+    if weight.data_ptr() % 16 or norm_weight.data_ptr() % 16:
+        raise ValueError("operands must be 16-byte aligned")
+    if bias is not None:
+        _gpu("bias", bias, torch.float32, 1)
+        if not (bias.shape[0] == n):
+            raise ValueError(f"bias must be [{n}]")
+    return m, n, k
+
+
+def gemm_f32_normed(stream: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor,
+                    bias: Optional[torch.Tensor] = None, gate: bool = False) -> torch.Tensor:
+    """:func:`gemm_f32` of the RMS norm of ``stream``'s few rows, made inside the product: the bits are those of
+    :func:`add_rmsnorm` followed by the product."""
+    m, n, k = _check_normed_f32(stream, norm_weight, eps, weight, bias)
+    if gate and (bias is not None or n % 2):
+        raise ValueError("a gated unit takes an even number of weight rows and no bias")
+    width = n // 2 if gate else n
+    out = torch.empty((m, width), dtype=torch.float32, device=stream.device)
+    _run("cie_gemm_f32_normed", load_library().cie_gemm_f32_normed(
+        _stream(), _ptr(stream), _ptr(norm_weight), _f(eps), _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k),
+        _i(width), _i(bool(gate)), _i(compute_units(stream.device))))
+    return out
+
+
+def gemm_f32_into(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], into: torch.Tensor) -> None:
+    """``into += a @ weight.T + bias`` for up to ``F32_FEW_ROWS`` rows, in the bits of :func:`gemm_f32` and an add behind it."""
+    if not (a.is_cuda and a.dtype == torch.float32 and a.dim() == 2 and a.stride(1) == 1):
+        raise ValueError("a must be a float32 GPU matrix with unit inner stride")
+    _gpu("weight", weight, torch.float32, 2)
+    _gpu("into", into, torch.float32, 2)
+    m, k = a.shape
+    n = weight.shape[0]
+    if not (weight.shape[1] == k and into.shape == (m, n) and m <= F32_FEW_ROWS):
+        raise ValueError(f"a is [{m},{k}], weight {tuple(weight.shape)}, into {tuple(into.shape)}; up to {F32_FEW_ROWS} rows")
+    if bias is not None:
+        _gpu("bias", bias, torch.float32, 1)
+        if not (bias.shape[0] == n):
+            raise ValueError(f"bias must be [{n}]")
+    lda = a.stride(0) if m > 1 else max(a.stride(0), k)
+    _run("cie_gemm_f32_into", load_library().cie_gemm_f32_into(
+        _stream(), _ptr(a), _ptr(weight), _ptr(bias), _ptr(into), _i(m), _i(n), _i(k), _i(lda), _i(n), _i(compute_units(a.device))))
+
+
+def gemm_f32_qkv_rope(stream: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor,
+                      bias: Optional[torch.Tensor], cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor,
+                      seq_of_token: torch.Tensor, seq_slot: torch.Tensor, block_table: torch.Tensor, k_pool: torch.Tensor,
+                      v_pool: torch.Tensor, q_heads: int, kv_heads: int, head_dim: int, rotate: bool = True,
+                      write_kv: bool = True, rotary_dim: Optional[int] = None) -> torch.Tensor:
+    """The q/k/v product of :func:`gemm_f32_normed` with the rotation and the cache write of :func:`rope_kv_write` in its
+    epilogue, in their bits (heads of a size in steps of 16, of which the first ``rotary_dim`` dimensions, a number in steps
+    of 16 too, rotate; all without it).  Returns [M, N] whose query columns hold the
+    rotated queries; the others are not written."""
+    m, n, k = _check_normed_f32(stream, norm_weight, eps, weight, bias)
+    if head_dim % 16 or n != (q_heads + 2 * kv_heads) * head_dim:
+        raise ValueError(f"weight has {n} rows, heads say {(q_heads + 2 * kv_heads) * head_dim}, of {head_dim} (in steps of 16)")
+    rotary_dim = head_dim if rotary_dim is None else rotary_dim
+    if not (0 < rotary_dim <= head_dim and rotary_dim % 16 == 0):
+        raise ValueError(f"rotary_dim must be in steps of 16 up to {head_dim}, is {rotary_dim}")
+    for name, table in (("cos", cos), ("sin", sin)):
+        _gpu(name, table, torch.float32, 2)
+        if rotate and not (table.shape[1] == rotary_dim // 2):
+            raise ValueError(f"{name} must be [max_position, {rotary_dim // 2}]")
+    if not (cos.shape == sin.shape):
+        raise ValueError("cos and sin tables differ in shape")
+    for name, meta in (("positions", positions), ("seq_of_token", seq_of_token)):
+        _gpu(name, meta, torch.int32, 1)
+        if not (meta.shape[0] >= m):
+            raise ValueError(f"{name} has {meta.shape[0]} entries for {m} rows")
+    _gpu("seq_slot", seq_slot, torch.int32, 1)
+    _gpu("block_table", block_table, torch.int32, 2)
+    page_size = _check_pools(k_pool, v_pool, torch.float32, kv_heads, head_dim)
+    out = torch.empty((m, n), dtype=torch.float32, device=weight.device)
+    _run("cie_gemm_f32_normed_rope", load_library().cie_gemm_f32_normed_rope(
+        _stream(), _ptr(stream), _ptr(norm_weight), _f(eps), _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k), _ptr(cos),
+        _ptr(sin), _ptr(positions), _ptr(seq_of_token), _ptr(seq_slot), _ptr(block_table), _i(block_table.shape[1]), _ptr(k_pool),
+        _ptr(v_pool), _i(q_heads), _i(kv_heads), _i(head_dim), _i(rotary_dim), _i(page_size), _i(bool(rotate)), _i(bool(write_kv)),
+        _i(compute_units(weight.device))))
+    return out
+
+
 EPI_BF16, EPI_F32, EPI_SILU, EPI_RESID, EPI_PARTIAL = 0, 1, 2, 3, 4
 EPI_ATOMIC = 7  # (the shared-rows form: parts of K add into a float32 stream with atomic adds)
 FUSED_TARGET_WAVES = 2048

@@ -139,6 +139,15 @@ class Attention(Part):
                 context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, head_dim,
                                  self.window, self.scale)
                 return linear(context, self.w_o, self.b_o, into=residual, then_norm=next_norm, sums_parts=sums_parts)
+            turning = head_dim if rotary_dim is None else rotary_dim
+            if (type(self).shape_projection is Attention.shape_projection and head_dim % 16 == 0 and turning % 16 == 0
+                    and x.joins_f32(self.w_qkv)):
+                qkv = ops.gemm_f32_qkv_rope(
+                    x.residual, x.norm.weight_f32, x.norm.eps, self.w_qkv, self.b_qkv, self.cos, self.sin, batch.positions,
+                    batch.seq_of_token, batch.seq_slot, view.block_table, view.k_pool, view.v_pool, self.num_heads,
+                    self.num_kv_heads, head_dim, rotate=self.position.rotates, write_kv=writes, rotary_dim=turning)
+                context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, head_dim, self.window, self.scale)
+                return linear(context, self.w_o, self.b_o, into=residual, then_norm=next_norm, sums_parts=sums_parts)
             x = x.complete()
         fused = (x.dtype == torch.bfloat16 and untouched and head_dim % 32 == 0
                  and x.shape[1] % 8 == 0 and (rows == 1 or x.stride(0) % 8 == 0))

@@ -78,27 +78,38 @@ class PreNormBlock:
             if warm is not None:
                 warm(rows)
 
-    def forward(self, residual: torch.Tensor, pending: Optional[torch.Tensor], batch, view,
-                writes: bool = True, plus: Optional[torch.Tensor] = None) -> tuple[torch.Tensor, torch.Tensor]:
+    takes_added = True
+
+    def forward(self, residual: torch.Tensor, pending: Optional[torch.Tensor], batch, view, writes: bool = True,
+                plus: Optional[torch.Tensor] = None, added: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
         """``plus``: float32 rows that join the stream in front of this layer (behind what is pending).  A first
-        norm that says ``takes_plus`` adds them in its own kernel; for any other they are added here."""
+        norm that says ``takes_plus`` adds them in its own kernel; for any other they are added here.  ``added``: in
+        float32 too the feed-forward's branch may come back added to the stream (what follows need not read it)."""
         if plus is not None:
             if getattr(self.norm1, "takes_plus", False):
                 x = normalise(self.norm1, residual, pending, self.dtype, plus=plus)
-                return self._behind_first_norm(x, residual, batch, view, writes)
+                return self._behind_first_norm(x, residual, batch, view, writes, added)
             x = normalise(self.norm1, residual, pending, self.dtype)  # (the pending branch joins the stream)
             residual.add_(plus)
             pending = None
         if ((pending is None or isinstance(pending, Added)) and getattr(self.mixer, "takes_raw_rows", False)
+                and (self.dtype != torch.float32 or declares(self.mixer, "takes_raw_rows"))
                 and getattr(self.norm1, "folds_into_products", False) and RawRows.fits(residual, self.dtype)):
             # a few rows, the stream complete: the mixer's first product makes the norm itself (a kernel less)
             x = RawRows(residual, self.norm1, self.dtype)
         else:
             x = normalise(self.norm1, residual, pending, self.dtype)
-        return self._behind_first_norm(x, residual, batch, view, writes)
+        return self._behind_first_norm(x, residual, batch, view, writes, added)
 
-    def _behind_first_norm(self, x, residual: torch.Tensor, batch, view, writes: bool):
-        extra = {"residual": residual} if getattr(self.mixer, "adds_to_residual", False) else {}
+    def _joins(self, part, residual: Optional[torch.Tensor]) -> dict:
+        """What a part that can add to the stream is handed; in float32 one with a ``forward`` of its own, which may expect
+        its products to come back as tensors there, is not."""
+        if not getattr(part, "adds_to_residual", False):
+            return {}
+        return {"residual": residual if self.dtype != torch.float32 or declares(part, "adds_to_residual") else None}
+
+    def _behind_first_norm(self, x, residual: torch.Tensor, batch, view, writes: bool, added: bool = False):
+        extra = self._joins(self.mixer, residual if added or self.has_feed_forward or self.dtype != torch.float32 else None)
         if extra and declares(self.mixer, "sums_parts"):
             extra["sums_parts"] = True
         if (extra and self.has_feed_forward and getattr(self.mixer, "folds_next_norm", False)
@@ -108,8 +119,12 @@ class PreNormBlock:
         mixed = self.mixer.forward(x, batch, view, writes, **extra)
         if not self.has_feed_forward:
             return residual, mixed  # (the next norm adds it)
-        x = normalise(self.norm2, residual, mixed, self.dtype)
-        extra = {"residual": residual} if getattr(self.feed_forward, "adds_to_residual", False) else {}
+        if (self.dtype == torch.float32 and isinstance(mixed, Added) and declares(self.feed_forward, "takes_raw_rows")
+                and getattr(self.norm2, "folds_into_products", False) and RawRows.fits(residual, self.dtype)):
+            x = RawRows(residual, self.norm2, self.dtype)  # a few rows: the feed-forward's first product makes the norm
+        else:
+            x = normalise(self.norm2, residual, mixed, self.dtype)
+        extra = self._joins(self.feed_forward, residual if added or self.dtype != torch.float32 else None)
         if extra and declares(self.feed_forward, "sums_parts"):
             extra["sums_parts"] = True
         return residual, self.feed_forward.forward(x, **extra)

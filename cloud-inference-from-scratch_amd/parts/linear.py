@@ -1,7 +1,7 @@
 """``x @ W^T + b`` for a Linear's weight ``[out, in]``, and its fused forms.
 
 float32: the hand-written true-float32 kernels, always (the gated unit in their
-epilogue).  bfloat16 with up to
+epilogue; of up to ``ops.F32_FEW_ROWS`` rows also the norm in front and the add into the stream).  bfloat16 with up to
 ``FUSED_ROWS`` rows (decode steps, the output head), and up to 64 or 128 rows where
 it is the faster one (a small weight, a long K): the hand-written
 matrix-core kernels that stream the weight once and take over their neighbours'
@@ -368,9 +368,10 @@ class WeightedPair:
 @dataclass
 class RawRows:
     """Stands where an RMSNorm's output would, before anything was computed: the rows are the norm ``norm``
-    of the float32 stream ``residual``.  Only a mixer that says ``takes_raw_rows`` is shown it (the attention
+    of the float32 stream ``residual``.  Only a part that says ``takes_raw_rows`` is shown it (the attention
     part's q/k/v product then makes its rows itself, with up to ``ops.FOLDED_NORM_ROWS`` rows: every workgroup
-    reads the few rows once, where a kernel of its own for the norm costs a decode layer 4.6 us)."""
+    reads the few rows once, where a kernel of its own for the norm costs a decode layer 4.6 us; in float32 the
+    feed-forward's first product too)."""
 
     residual: torch.Tensor
     norm: Any
@@ -379,11 +380,18 @@ class RawRows:
     @staticmethod
     def fits(residual: torch.Tensor, dtype: torch.dtype) -> bool:
         rows, width = residual.shape
+        if dtype == torch.float32:
+            return ops.folds_norm_f32(residual)
         return dtype == torch.bfloat16 and residual.is_cuda and ops.folds_norm(rows, width)
 
     @property
     def shape(self):
         return self.residual.shape
+
+    def joins_f32(self, weight: torch.Tensor) -> bool:
+        """Whether the float32 product with this weight can make the norm itself."""
+        return (self.dtype == weight.dtype == torch.float32 and weight.data_ptr() % 16 == 0
+                and self.norm.weight_f32.data_ptr() % 16 == 0)
 
     def complete(self) -> torch.Tensor:
         """The norm's output after all."""
@@ -435,7 +443,7 @@ def takes_tiles(rows: int, x: torch.Tensor, weight: torch.Tensor, into: Optional
             and (into is None or (into.is_cuda and into.dtype == torch.float32 and into.data_ptr() % 16 == 0)))
 
 
-def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out_dtype: Optional[torch.dtype] = None, epilogue: Optional[str] = None,
            into: Optional[torch.Tensor] = None, then_norm: Any = None,
            sums_parts: bool = False) -> Union[torch.Tensor, RowSumsq, Added, KParts]:
@@ -452,7 +460,8 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
     this product and the next (``RMSNorm.folds_into_products``): the residual
     epilogue then also leaves that norm's output short of the rows' scale.
     ``x`` may be such rows (:class:`ScaledRows`): the SiLU product of few rows
-    applies the scale itself, any other reader gets the completed rows."""
+    applies the scale itself, any other reader gets the completed rows.  :class:`RawRows` in float32:
+    the SiLU product of few rows makes their norm itself."""
     if isinstance(x, ScaledRows):
         rows, k = x.rows.shape
         if epilogue == "silu" and weight.shape[0] % 2 == 0 and bias is None and weight.dtype == torch.bfloat16:
@@ -466,6 +475,10 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
             out = ops.gemm_library(x.rows, weight) if x.rows.stride(1) == 1 else None
             if out is not None:
                 return ops.silu_mul(out, row_sumsq=x.sumsq, hidden=k, eps=x.eps)
+        x = x.complete()
+    if isinstance(x, RawRows):
+        if epilogue == "silu" and weight.shape[0] % 2 == 0 and bias is None and into is None and x.joins_f32(weight):
+            return ops.gemm_f32_normed(x.residual, x.norm.weight_f32, x.norm.eps, weight, gate=True)
         x = x.complete()
     rows, k = x.shape
     n = weight.shape[0]
@@ -538,6 +551,10 @@ def linear(x: Union[torch.Tensor, ScaledRows], weight: torch.Tensor, bias: Optio
     if weight.dtype == torch.float32:
         if silu and n % 2 == 0 and bias is None:
             return ops.gemm_f32(x, weight, gate=True)
+        if (into is not None and not silu and 1 <= rows <= ops.F32_FEW_ROWS and into.is_cuda and into.dtype == torch.float32
+                and into.is_contiguous() and tuple(into.shape) == (rows, n)):
+            ops.gemm_f32_into(x, weight, bias, into)  # (the next norm need not add it: it may ride in the product behind it)
+            return Added()
         out = ops.gemm_f32(x, weight, bias)
     elif wants_f32:
         # a shape the kernel refuses (a width that is no multiple of 8): widened operands, exact products,

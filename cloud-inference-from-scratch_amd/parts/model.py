@@ -14,7 +14,7 @@ from ..config.specs import ModelSpec
 from ..kernels import ops
 from ..weights.loader import torch_dtype
 from ..weights.tensors import TensorSpec
-from .base import BLOCKS, build_part
+from .base import BLOCKS, build_part, declares
 from .block import NormedRows, normalise, whole_stream
 from .linear import StreamRows, linear
 
@@ -222,6 +222,8 @@ class DecoderModel:
                 residual, extra["plus"] = self.entry.forward(joint, call.entry)
                 pending = None
             left = False
+            if declares(block, "takes_added"):
+                extra["added"] = True
             if getattr(block, "takes_follower", False):
                 extra["follower"] = self.followers[index]
                 if index + 1 < len(self.spec.order) and self.spec.order[index + 1].entry is not None:
