@@ -77,25 +77,44 @@ class PageAllocator:
             raise DoubleFreeError(f"page {page} is already held by {holder!r}")
         holders.append(holder)
 
+    def retain_all(self, pages: Sequence[int], holder: str) -> None:
+        """:meth:`retain` for each page; raises before changing anything if any page cannot be retained."""
+        if len(set(pages)) != len(pages):
+            raise DoubleFreeError("same page retained twice in one call")
+        held = self._holders
+        found = []
+        for page in pages:
+            holders = held.get(page)
+            if holders is None:
+                raise DoubleFreeError(f"page {page} is free and cannot be retained by {holder!r}")
+            if holder in holders:
+                raise DoubleFreeError(f"page {page} is already held by {holder!r}")
+            found.append(holders)
+        for holders in found:
+            holders.append(holder)
+
     def free(self, pages: Sequence[int], holder: str) -> list[int]:
         """Drop ``holder`` from each page; returns the pages that became free.
         Raises before changing anything if any page is not held by ``holder``."""
         if len(set(pages)) != len(pages):
             raise DoubleFreeError("same page freed twice in one call")
+        held = self._holders
+        found = []
         for page in pages:
-            holders = self._holders.get(page)
+            holders = held.get(page)
             if holders is None:
                 raise DoubleFreeError(f"page {page} is already free")
             if holder not in holders:
                 raise DoubleFreeError(f"page {page} held by {holders!r}, freed by {holder!r}")
+            found.append(holders)
         returned = []
-        for page in pages:
-            holders = self._holders[page]
-            holders.remove(holder)
-            if not holders:
-                del self._holders[page]
-                self._free.append(page)
+        for page, holders in zip(pages, found):
+            if len(holders) > 1:
+                holders.remove(holder)
+            else:
+                del held[page]
                 returned.append(page)
+        self._free.extend(returned)
         return returned
 
     def free_for(self, holder: str) -> list[int]:

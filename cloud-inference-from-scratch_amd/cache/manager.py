@@ -414,9 +414,9 @@ class CacheManager:
         candidate_pages = (len(tokens) - 1) // self.page_size
         matched: list[_PrefixNode] = []
         parent_id: int | None = None
-        for i in range(candidate_pages):
-            key = (parent_id, tuple(tokens[i * self.page_size:(i + 1) * self.page_size]))
-            node = self._prefix.get(key)
+        size, find = self.page_size, self._prefix.get
+        for first in range(0, candidate_pages * size, size):
+            node = find((parent_id, tuple(tokens[first:first + size])))
             if node is None:
                 break
             matched.append(node)
@@ -425,11 +425,12 @@ class CacheManager:
             if candidate_pages:
                 self.prefix_cache_misses += 1
             return 0
-        table = group.tables[request_id]
+        pages = [node.page for node in matched]
+        group.allocator.retain_all(pages, request_id)
+        group.tables[request_id].extend(pages)
+        renew = self._prefix.move_to_end
         for node in matched:
-            group.allocator.retain(node.page, request_id)
-            table.append(node.page)
-            self._prefix.move_to_end(node.key)
+            renew(node.key)
         self._dirty.add((0, self._slots[request_id]))
         length = len(matched) * self.page_size
         self._length[request_id] = length
