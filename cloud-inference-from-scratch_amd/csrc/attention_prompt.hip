@@ -2,9 +2,14 @@
 //
 // A workgroup takes one tile (up to 128 rows = tokens_per_tile tokens x the heads of one kv head's group)
 // and walks the tile's keys 64 at a time.  The keys and values of those 64 positions are read from the
-// cache once per workgroup, in 16-byte pieces that follow one another in memory, and laid into LDS in the
-// order the matrix instructions take their operands; every wave then reads them from there.  Two stages
-// of LDS take turns, so that the loads of the keys after next are under way while a block is worked on.
+// cache once per workgroup, by loads that write LDS themselves (1 KB each, 16 bytes a lane), in the order the matrix
+// instructions take their operands; every wave then reads them from there.  Two stages of LDS take turns, so that the loads of
+// the next 64 keys are under way while a block is worked on, and one barrier a stage frees the one and has the other whole.
+// (Carried through registers and stored to LDS by the waves, as far ahead, the pieces held 32 registers and took 12 stores a
+// wave and stage: MI355X, us, 2,048 tokens of one prompt, 3B heads 43.6 -> 36.4, behind 14,336 keys 342 -> 270; 777 tokens behind
+// 4,000, 7B heads 104 -> 80; 14 heads of 64 dimensions 30.3 -> 24.6.  A third stage changes nothing.)  The products run at a
+// raised priority where the head has 128 dimensions: a wave that multiplies goes before the one beside it that does its
+// softmax (85 -> 80 and 284 -> 270 of these; with 64 dimensions, half the products, 41.5 -> 44.5: not there).
 //
 // Wave w owns rows 32 * (w % 4) .. + 31 of the tile and, of each 64 keys, the half w / 4: four waves
 // cover the rows, two such sets the keys.  A wave holds 32 rows of the output (64 accumulator registers
@@ -16,13 +21,15 @@
 //   P = 2^(S * scale * log2 e - m)            float32; the reference m of a row moves lazily
 //   O[row, d] += P[row, key] * V[key, d]      A = P (registers), B = V^T (from LDS)
 //
+// Which row of a block's two 16-key products a key is, is free: row m of product kt is key 8 (m / 4) + 4 kt + m % 4 of the 32,
+// so that a lane ends with the probabilities of eight neighbouring keys, and takes their values as the cache has them.
+//
 // LDS layout of one stage (D = head size, C = D / 8 sixteen-byte chunks of a key):
 //   keys    64 rows of CS chunk slots (CS = C rounded up to a power of two); chunk c of key k lies in slot
 //           c ^ swizzle(k), so that the 16 lanes that read the same chunk of 16 different keys hit 16
 //           different groups of banks
-//   values  two blocks (one per half) of D rows of 64 bytes: row d holds, for each lane group g, the
-//           values of keys g*4 .. g*4+3 of the block's first 16 keys and of its second 16 keys (16 bytes,
-//           one read per product); the four 16-byte chunks of a row are swizzled by (d / 4) % 4
+//   values  four groups of 16 keys, each D rows of 32 bytes: dimension d's values of the keys, eight a chunk, the two
+//           chunks exchanged where d / 8 is odd
 #include "attention_args.h"
 #include "common.h"
 
@@ -61,27 +68,40 @@ struct PromptLayout {
     static constexpr int kKeyBytes = kKeysPerStage * CS * 16;
     static constexpr int kValueBlockBytes = D * 64;
     static constexpr int kStageBytes = kKeyBytes + 2 * kValueBlockBytes;
-    // the swizzle of a key's chunk slots: over 16 consecutive keys, the same chunk lands in 16 different
-    // sixteen-byte columns of the 256 bytes that the banks span
+    static constexpr int kKeyPieces = CS / 4, kValuePieces = D / 32;  // loads of 1 KB that a group of 16 keys takes
+    static constexpr int kKeysPerPiece = 64 / CS;
+    // the swizzle of a key's chunk slots: over the 16 keys that one product reads (bits 0, 1, 3 and 4 of their places take
+    // every value), the same chunk lands in 16 different sixteen-byte columns of the 256 bytes that the banks span
     __device__ static __forceinline__ int key_swizzle(int k) {
-        if (CS >= 16) return k & 15;
-        if (CS == 8) return (k >> 1) & 7;
-        return (k >> 2) & 3;
+        if (CS >= 16) return (k & 3) | (k >> 3 & 3) << 2;
+        if (CS == 8) return (k >> 1 & 1) | (k >> 3 & 3) << 1;
+        return k >> 3 & 3;
     }
 };
+
+typedef __attribute__((address_space(3))) void* lds_pointer;
+// (16 bytes as one value.  Read from a stage as a uint4, a structure, they made the compiler wait for every load that writes LDS
+// in front of each block's first read.)
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// Behind it all of this wave's loads but the youngest kYounger are in LDS, and what it read there is in registers.
+template <int kYounger>
+__device__ __forceinline__ void wait_for_loads() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kYounger) : "memory");
+}
 
 // WAVES = 8: tiles of 128 rows; WAVES = 4: the same with tiles of 64 rows, two such workgroups to a compute unit,
 // which then walk their keys independently of each other (one's matrix products beside the other's softmax).
 template <int D, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) paged_attention_prompt_kernel(AttentionArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the host's pass has no type for a buffer's description)
     using L = PromptLayout<D>;
     constexpr int NK = D / 32;
     constexpr int ND = D / 16;
     constexpr int RT = 2;  // 16-row tiles of a wave
     constexpr int QUARTERS = WAVES / 2;        // sets of 32 rows of the tile
     constexpr int kTileRows = 32 * QUARTERS;
-    constexpr int kLoaderThreads = 64 * QUARTERS;  // threads that fetch one group of 16 keys
-    extern __shared__ __align__(16) unsigned char lds[];
+    extern __shared__ __align__(1024) unsigned char lds[];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int quarter = wave % QUARTERS;   // which 32 rows of the tile
@@ -181,38 +201,19 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) paged_attentio
     }
     const bf16x8 ones = __builtin_bit_cast(bf16x8, (uint4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u}));
 
-    // ---- this thread's share of the loads.  A stage is four groups of 16 keys (each within one page).  The
-    // lower four waves fetch groups 0 and 2, the upper four groups 1 and 3, so that which page a load reads
-    // is one number per wave; within its group a thread always takes the same 16-byte piece of the keys
-    // and the same piece of the values, and puts them at the same places of the stage.
-    // (Where a group has fewer pieces than the 256 threads that share it, the threads left over fetch and
-    // store a piece a second time: the same bytes to the same place.)
-    const int loader = half;  // (the same split of the waves, used here for something else)
-    // (with four waves a loader's 128 threads take two pieces of each kind in a group: kPasses)
-    constexpr int kKeyPieces = 16 * L::C, kValuePieces = 2 * D;
-    constexpr int kPasses = (kKeyPieces > kValuePieces ? kKeyPieces : kValuePieces) > kLoaderThreads ? 2 : 1;
-    static_assert(kKeyPieces <= kPasses * kLoaderThreads && kValuePieces <= kPasses * kLoaderThreads,
-                  "at most two pieces of each kind per thread and group");
-    const int loader_thread = threadIdx.x % kLoaderThreads;
-    int key_from[kPasses], key_to[kPasses], value_from[kPasses], value_to_a[kPasses], value_to_b[kPasses];
+    // ---- this wave's share of the loads.  A stage is four groups of 16 keys (each within one page): wave w fetches group
+    // w % 4, with eight waves every second of its pieces, so that which page its loads read is one number.  A lane's place in
+    // LDS is given (16 bytes behind its neighbour's), so it picks the chunk that belongs there.
+    constexpr int kSharers = WAVES / 4, kPieces = L::kKeyPieces + L::kValuePieces;
+    const int loads_group = wave % 4, loads_first = wave / 4;
+    unsigned key_from[L::kKeyPieces];  // bytes from the group's first key
 #pragma unroll
-    for (int pass = 0; pass < kPasses; ++pass) {
-        const int key_piece = (loader_thread + pass * kLoaderThreads) % kKeyPieces;
-        const int piece_key = key_piece / L::C;           // which of the group's 16 keys
-        const int piece_chunk = key_piece - piece_key * L::C;
-        key_from[pass] = (piece_key * D + piece_chunk * 8) * 2;  // bytes from the group's first key
-        key_to[pass] = ((loader * 16 + piece_key) * L::CS + (piece_chunk ^ L::key_swizzle(piece_key))) * 16;  // + pair * 32 keys
-        const int value_piece = (loader_thread + pass * kLoaderThreads) % kValuePieces;
-        const int piece_d = value_piece >> 1;         // which dimension's row of values
-        const int piece_h = value_piece & 1;          // which 8 of the group's 16 keys
-        value_from[pass] = ((piece_d << a.page_shift) + piece_h * 8) * 2;  // bytes from the group's first key in row 0
-        // row d of the block (pair); the group's keys are the block's first 16 (loader 0) or second 16 (loader 1):
-        // the first or second 8 bytes of a chunk; keys h*8 .. +3 belong to lane group 2h, keys h*8+4 .. +7 to 2h+1
-        const int value_row = L::kKeyBytes + piece_d * 64 + loader * 8;  // + pair * kValueBlockBytes
-        const int value_sw = (piece_d >> 2) & 3;
-        value_to_a[pass] = value_row + (((2 * piece_h) ^ value_sw) << 4);
-        value_to_b[pass] = value_row + (((2 * piece_h + 1) ^ value_sw) << 4);
+    for (int i = 0; i < L::kKeyPieces; ++i) {
+        const int key = i * L::kKeysPerPiece + lane / L::CS;
+        const int chunk = (lane % L::CS) ^ L::key_swizzle(loads_group * 16 + key);
+        key_from[i] = (key * D + (chunk < L::C ? chunk : 0) * 8) * 2;  // (a slot that holds no chunk is never read)
     }
+    const unsigned value_from = ((lane / 2 << a.page_shift) + ((lane % 2) ^ (lane >> 4 & 1)) * 8) * 2;
 
     typedef const __attribute__((address_space(4))) int* const_int_ptr;
     const const_int_ptr table_c = (const_int_ptr)(uintptr_t)table;
@@ -221,78 +222,63 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) paged_attentio
     auto page_of = [&](int first) {
         return table_c[__builtin_amdgcn_readfirstlane(min(first, last_group) >> a.page_shift)];
     };
-    // the pages of this wave's two groups of the stage that starts at key kb
-    auto pages_of = [&](int kb, int (&page)[2]) {
+    auto page_at = [&](int kb) { return page_of(kb + loads_group * 16); };  // ... of this wave's group of the stage at key kb
+    auto fetch = [&](int kb, int page, int stage) __attribute__((always_inline)) {
+        const int first = min(kb + loads_group * 16, last_group);
+        const size_t page_head = static_cast<size_t>(page) * a.kv_heads + kv_head;
+        const __amdgpu_buffer_rsrc_t keys = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<bf16_t*>(a.k_pool + ((page_head << a.page_shift) + (first & page_mask)) * D), 0, 0xffffffffu, 0x00027000);
+        const __amdgpu_buffer_rsrc_t values = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<bf16_t*>(a.v_pool + (page_head * D << a.page_shift) + (first & page_mask)), 0, 0xffffffffu, 0x00027000);
+        unsigned char* key_to = lds + stage * L::kStageBytes + loads_group * (16 * L::CS * 16);
+        unsigned char* value_to = lds + stage * L::kStageBytes + L::kKeyBytes + loads_group * (D * 32);
 #pragma unroll
-        for (int pair = 0; pair < 2; ++pair) page[pair] = page_of(kb + (2 * pair + loader) * 16);
-    };
-    uint4 key_regs[2][kPasses], value_regs[2][kPasses];
-#pragma unroll
-    for (int pair = 0; pair < 2; ++pair)
-#pragma unroll
-        for (int pass = 0; pass < kPasses; ++pass) key_regs[pair][pass] = value_regs[pair][pass] = uint4{0, 0, 0, 0};
-    auto fetch = [&](int kb, const int (&page)[2]) {
-#pragma unroll
-        for (int pair = 0; pair < 2; ++pair) {
-            const int first = min(kb + (2 * pair + loader) * 16, last_group);
-            const size_t page_head = static_cast<size_t>(page[pair]) * a.kv_heads + kv_head;
-            const char* key_base = reinterpret_cast<const char*>(
-                a.k_pool + ((page_head << a.page_shift) + (first & page_mask)) * D);
-            const char* value_base = reinterpret_cast<const char*>(
-                a.v_pool + (page_head * D << a.page_shift) + (first & page_mask));
-#pragma unroll
-            for (int pass = 0; pass < kPasses; ++pass) {
-                key_regs[pair][pass] = *reinterpret_cast<const uint4*>(key_base + key_from[pass]);
-                value_regs[pair][pass] = *reinterpret_cast<const uint4*>(value_base + value_from[pass]);
-            }
-        }
-    };
-    auto stash = [&](int stage) {
-        unsigned char* base = lds + stage * L::kStageBytes;
-#pragma unroll
-        for (int pair = 0; pair < 2; ++pair) {
-            unsigned char* block = base + pair * L::kValueBlockBytes;
-#pragma unroll
-            for (int pass = 0; pass < kPasses; ++pass) {
-                *reinterpret_cast<uint4*>(base + key_to[pass] + pair * (32 * L::CS * 16)) = key_regs[pair][pass];
-                const uint4 values = value_regs[pair][pass];
-                *reinterpret_cast<uint2*>(block + value_to_a[pass]) = uint2{values.x, values.y};
-                *reinterpret_cast<uint2*>(block + value_to_b[pass]) = uint2{values.z, values.w};
-            }
+        for (int i = 0; i < kPieces; ++i) {
+            if (kSharers == 2 && i % 2 != loads_first) continue;
+            if (i < L::kKeyPieces)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(keys, (lds_pointer)(key_to + i * 1024), 16, key_from[i < L::kKeyPieces ? i : 0], 0, 0, 0);
+            else
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(values, (lds_pointer)(value_to + (i - L::kKeyPieces) * 1024), 16, value_from,
+                                                         (i - L::kKeyPieces) * 64 << a.page_shift, 0, 0);
         }
     };
 
     // ---- a lane's constant parts of its operand addresses in a stage
-    const int k_read = ((half * 32 + r) * L::CS) * 16;       // + kt * 16 * CS * 16, + swizzled chunk
-    const int k_sw = L::key_swizzle(r);
-    const int v_read = L::kKeyBytes + half * L::kValueBlockBytes + r * 64 + ((g ^ ((r >> 2) & 3)) << 4);  // + dt * 1024
+    // (row r of product kt is key 8 (r / 4) + r % 4 + 4 kt of the half; bit 2 of a key's place is not in its swizzle)
+    const int k_read = (half * 32 + r / 4 * 8 + r % 4) * L::CS * 16;  // + kt * 4 * CS * 16, + swizzled chunk
+    const int k_sw = L::key_swizzle(half * 32 + r / 4 * 8 + r % 4);
+    const int v_read = L::kKeyBytes + (half * 2 + g / 2) * (D * 32) + r * 32 + ((g % 2) ^ (r >> 3)) * 16;  // + dt * 512
 
     const int n_iter = (range_end - range_begin + kKeysPerStage - 1) / kKeysPerStage;
-    int page[2], page_next[2];
+    int page = 0;
     if (n_iter > 0) {
-        pages_of(range_begin, page);
-        pages_of(range_begin + kKeysPerStage, page_next);
-        fetch(range_begin, page);
-        stash(0);
-        __syncthreads();
-        if (n_iter > 1) fetch(range_begin + kKeysPerStage, page_next);
+        const int first_page = page_at(range_begin);
+        page = page_at(range_begin + kKeysPerStage);
+        fetch(range_begin, first_page, 0);
+        if (n_iter > 1) {
+            fetch(range_begin + kKeysPerStage, page, 1);
+            wait_for_loads<kPieces / kSharers>();
+        } else {
+            wait_for_loads<0>();
+        }
+        asm volatile("s_barrier" ::: "memory");
     }
 
     for (int it = 0; it < n_iter; ++it) {
         const int kb = range_begin + it * kKeysPerStage + half * kKeysPerBlock;  // this wave's 32 keys
         const unsigned char* stage = lds + (it & 1) * L::kStageBytes;
-        // pages of the stage after next, asked for early: the loads that need them come a whole block later
-        int page_after[2] = {0, 0};
-        if (it + 2 < n_iter) pages_of(range_begin + (it + 2) * kKeysPerStage, page_after);
+        // the page of the stage after next, asked for early: the loads that need it come a whole block later
+        if (it + 2 < n_iter) page = page_at(range_begin + (it + 2) * kKeysPerStage);
         if (wave_rows > 0 && kb < range_end && kb <= wave_last_pos) {
             // ---- S^T = K . Q^T for two 16-key tiles
             floatx4 s[RT][2];
+            if constexpr (D > 64) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) {
-                uint4 kf[NK];
+                u32x4 kf[NK];
 #pragma unroll
                 for (int j = 0; j < NK; ++j)
-                    kf[j] = *reinterpret_cast<const uint4*>(stage + k_read + kt * (16 * L::CS * 16) +
+                    kf[j] = *reinterpret_cast<const u32x4*>(stage + k_read + kt * (4 * L::CS * 16) +
                                                             (((j * 4 + g) ^ k_sw) << 4));
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
@@ -304,10 +290,11 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) paged_attentio
                     s[rt][kt] = acc;
                 }
             }
+            if constexpr (D > 64) __builtin_amdgcn_s_setprio(0);
             // ---- the block's values: asked for now, used after the softmax arithmetic
-            uint4 vf[ND];
+            u32x4 vf[ND];
 #pragma unroll
-            for (int dt = 0; dt < ND; ++dt) vf[dt] = *reinterpret_cast<const uint4*>(stage + v_read + dt * 1024);
+            for (int dt = 0; dt < ND; ++dt) vf[dt] = *reinterpret_cast<const u32x4*>(stage + v_read + dt * 512);
             // ---- running maxima; masks only in blocks that reach a row's edge
             const bool edge = kb + kKeysPerBlock - 1 > wave_first_pos || kb + kKeysPerBlock > range_end ||
                               (a.window > 0 && kb < wave_last_pos + 1 - a.window);
@@ -320,12 +307,12 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) paged_attentio
                 if (edge) {
                     const int pos = min(row_pos[rt], range_end - 1);  // (a row that does not exist has -1: nothing seen)
                     const int row_lo = (a.window > 0) ? row_pos[rt] + 1 - a.window : 0;
-                    const int first_key = kb + g * 4;
+                    const int first_key = kb + g * 8;
 #pragma unroll
                     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const int key = first_key + kt * 16 + i;
+                            const int key = first_key + kt * 4 + i;
                             if (!(key <= pos && key >= row_lo)) s[rt][kt][i] = -INFINITY;
                         }
                 }
@@ -371,8 +358,11 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) paged_attentio
                     pw[kt * 2 + 1] = pack_bf16(p2, p3);
                 }
                 p_frag[rt] = __builtin_bit_cast(bf16x8, (uint4{pw[0], pw[1], pw[2], pw[3]}));
-                l_acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p_frag[rt], ones, l_acc[rt], 0, 0, 0);
             }
+            if constexpr (D > 64) __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+                l_acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p_frag[rt], ones, l_acc[rt], 0, 0, 0);
 #pragma unroll
             for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
@@ -380,12 +370,11 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) paged_attentio
                     o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p_frag[rt], __builtin_bit_cast(bf16x8, vf[dt]),
                                                                         o[rt][dt], 0, 0, 0);
         }
-        // ---- the next stage's keys and values have arrived by now: into LDS; then ask for the ones after
-        if (it + 1 < n_iter) stash((it + 1) & 1);
-        __syncthreads();
-        if (it + 2 < n_iter) {
-            fetch(range_begin + (it + 2) * kKeysPerStage, page_after);
-        }
+        __builtin_amdgcn_s_setprio(0);
+        // ---- the next stage has arrived by now (and whoever reads this one has read it): ask for the one after
+        wait_for_loads<0>();
+        asm volatile("s_barrier" ::: "memory");
+        if (it + 2 < n_iter) fetch(range_begin + (it + 2) * kKeysPerStage, page, it & 1);
     }
 
     // ---- the two halves of the keys meet: the upper waves hand their sums to the lower ones through LDS,
@@ -454,6 +443,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) paged_attentio
             }
         }
     }
+#endif
 }
 
 template <int D, int WAVES>
