@@ -186,13 +186,18 @@ SPLIT_DECODE_KEYS = 192  # contexts from which the keys of decode rows are cut i
 JOINED_DECODE_ROWS = 32  # up to this many single-token sequences beside prompt portions ride in the prompt form's launch
 PROMPT_SPLIT_KEYS = 512  # the fewest keys of a part when a prompt portion's keys are cut
 # (cutting a prompt form's keys aims at as many workgroups as the GPU has compute units)
-# Tiles of 64 rows x kv heads (as a share of the compute units) from which prompt portions take the form that
-# shares keys and values through LDS: enough to give most compute units a workgroup without cutting the keys (whose parts, 64 KB of sums per tile and kv head, cost that
-# form more than they gain it: 512 tokens behind 1,536 keys, 7B heads, 60 us in two parts against 40 us in the form
-# of four waves).  Measured at head size 128 (us, four waves -> eight): 2,048 tokens of one prompt 55.7 -> 51.4
-# (3B heads), 101 -> 58 (7B), 144 -> 84 (14B); behind 2,048 keys 108 -> 91, 195 -> 135, 284 -> 201; beside 8 single
-# tokens 108 -> 64, 138 -> 75, 182 -> 111.
+# Tiles of 64 rows x kv heads (as a share of the compute units) from which prompt portions take the form that shares keys and
+# values through LDS, whatever is beside them; up to JOINED_DECODE_ROWS single tokens ride in the other form's launch, and have
+# one of their own beside this one (8 over 2,000 keys and 600 tokens of 3B heads, 150 tiles: 25.7 us joined, 26.8).
 EIGHT_WAVE_TILES = 0.75  # of the compute units
+# With nothing to join from fewer tiles on, or from so many tiles times keys of the longest: few tiles have their keys cut for
+# as many workgroups as the GPU has units in either form (MI355X, us, the form without LDS and this one; 3B heads: 600 tokens,
+# 150 tiles, 18.1, 15.1, behind 2,000 keys 51.6, 33.2; 400 tokens, 100 tiles, 12.8, 12.1, behind 500 18.3, 19.5, 2,000 43.9, 26.7;
+# 200 tokens, 50 tiles, 7.4, 9.5, behind 1,000 18.5, 18.2, 4,000 42.5, 26.2; 64 tokens, 16 tiles, behind 4,000 18.9, 19.2, 8,000 27.4,
+# 21.4; five prompts of 613 tokens in all 16.7, 10.8; 16 heads on 16, 600 tokens 18.3, 14.5; 14 heads of 64 dimensions, 132 tiles,
+# 10.5, 10.9, behind 1,000 25.4, 18.4).
+ALONE_TILES = 0.55  # of the compute units
+ALONE_TILE_KEYS = 96_000
 LARGE_TILES_ABOVE = 1.0  # tiles of 128 rows x kv heads (as a share of the compute units) above which that form takes them
 
 
@@ -208,6 +213,16 @@ def plan_splits(units: int, max_keys: int, target_waves: int = 1024, min_keys: i
         return 1, 0
     per_split = -(-(-(-max_keys // splits)) // 32) * 32
     return -(-max_keys // per_split), per_split
+
+
+def takes_prompt_form(tiles: int, keys: int, singles: int, captured: bool, cus: int) -> bool:
+    """Whether prompt portions of so many tiles of 64 rows x kv heads, over up to ``keys`` keys and beside ``singles`` single
+    tokens, take the form that shares keys and values through LDS.  (A captured step's keys are known when it is replayed.)"""
+    if tiles >= max(1, EIGHT_WAVE_TILES * cus):
+        return True
+    if tiles == 0 or 0 < singles <= JOINED_DECODE_ROWS:
+        return False
+    return tiles >= ALONE_TILES * cus or (not captured and tiles * keys >= ALONE_TILE_KEYS)
 
 
 def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, head_dim: int,
@@ -258,7 +273,8 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
     # -> 64: 2,048 tokens of one prompt, 3B heads, 256 large tiles: 50.8 -> 46.8, 1,024 tokens 27.5 -> 24.8; 7B
     # heads, 456 large tiles: 55.3 -> 70.5; heads of 64 dimensions, where the softmax arithmetic per key is the same
     # and the products are half: 2,048 tokens 40.2 -> 33.0, against 43.1 in the form of four waves without LDS).
-    eight = (wide and head_dim in (64, 128) and group <= 64 and small_tiles >= max(1, EIGHT_WAVE_TILES * cus))
+    eight = (wide and head_dim in (64, 128) and group <= 64
+             and takes_prompt_form(small_tiles, max_keys, sum(n == 1 for n in batch.host_q_lens), batch.static_plan is not None, cus))
     lds_row_tiles = 8 if head_dim == 128 and big_tiles > LARGE_TILES_ABOVE * cus else 4
 
     def decode_form(bound: int, units: int) -> tuple[int, dict]:

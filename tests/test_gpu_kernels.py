@@ -850,6 +850,43 @@ def test_attention_planning_of_steps_with_single_tokens_beside_portions(ops, geo
     torch.testing.assert_close(out.float().cpu(), torch.cat(expected), **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("alone", [0.0, 99.0])
+@pytest.mark.parametrize("geometry", [(16, 2, 128, 16), (6, 2, 64, 32), (7, 1, 128, 16)])
+@pytest.mark.parametrize("portions", [((613, 0),), ((17, 1500), (130, 911), (2, 63)), ((64, 0), (65, 64), (1, 700)), ((33, 2100),)])
+def test_attention_of_portions_with_little_beside_them(ops, geometry, portions, alone, monkeypatch):
+    """Portions of few tiles in the form that shares keys and values through LDS (cut and whole) and in the other one: parts of
+    a tile, of a page and of 64 keys, each against plain attention per sequence."""
+    from cie_amd.engine.batch import PagedView, StepBatch
+    from cie_amd.parts import attention
+
+    monkeypatch.setattr(attention, "ALONE_TILES", alone)
+    monkeypatch.setattr(attention, "ALONE_TILE_KEYS", 1 << 40)
+    monkeypatch.setattr(attention, "JOINED_DECODE_ROWS", 0)
+    q_heads, kv_heads, head_dim, page_size = geometry
+    q_lens, contexts = [n for n, _c in portions], [c for _n, c in portions]
+    k_pool, v_pool, table, slots, dense = build_cache(torch.bfloat16, [c + n for n, c in portions], kv_heads, head_dim, page_size, seed=97)
+    scale, total = 1.0 / math.sqrt(head_dim), sum(q_lens)
+    qkv = torch.zeros((total, (q_heads + 2 * kv_heads) * head_dim), dtype=torch.bfloat16)
+    q = (torch.randn((total, q_heads, head_dim), generator=torch.Generator().manual_seed(98)) * 2).to(torch.bfloat16)
+    qkv[:, : q_heads * head_dim] = q.reshape(total, -1)
+    loc = [sum(q_lens[:s]) for s in range(len(q_lens) + 1)]
+    expected = torch.cat([plain_qwen2.causal_attention(q[loc[s]: loc[s + 1]].float(), *dense[s], scale, past_len=contexts[s])
+                          for s in range(len(q_lens))])
+    as_dev = lambda values: torch.tensor(values, dtype=torch.int32, device="cuda")  # noqa: E731
+    batch = StepBatch(tokens=total, sequences=len(q_lens), token_ids=as_dev([0] * total),
+                      positions=as_dev([c + i for n, c in portions for i in range(n)]),
+                      seq_of_token=as_dev([s for s, n in enumerate(q_lens) for _ in range(n)]), seq_slot=as_dev(slots),
+                      seq_start=as_dev(contexts), seq_q_len=as_dev(q_lens), q_start_loc=as_dev(loc), logit_rows=as_dev([0]),
+                      host_slots=list(slots), host_starts=contexts, host_q_lens=q_lens)
+    forms = []
+    real = ops.paged_attention_mfma
+    monkeypatch.setattr(ops, "paged_attention_mfma", lambda *a, **k: (forms.append(k["tile_waves"]), real(*a, **k))[1])
+    out = attention.attend(qkv.cuda(), batch, PagedView(k_pool, v_pool, table, page_size), q_heads, kv_heads, head_dim, None, scale)
+    tiles = -(-sum(n for n in q_lens if n > 1) * (q_heads // kv_heads) // 64) * kv_heads
+    assert (ops.PROMPT_WAVES in forms) == (alone == 0.0 or tiles >= 0.75 * ops.compute_units())
+    torch.testing.assert_close(out.float().cpu(), expected.reshape(total, -1), **tol(torch.bfloat16))
+
+
 def test_paged_attention_mfma_far_key(ops):
     """One key among two thousand carries the weight: output = its value row, in
     the tiled form and in every split layout."""

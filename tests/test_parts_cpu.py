@@ -178,3 +178,14 @@ def test_the_tiles_that_are_chosen_are_tiles_there_are(behind):
         assert not ops.direct_fits(rows, n, k, stride)
         picked = linear.choose_tiles(rows, n, k, stride)
         assert picked is None or not picked.direct
+
+
+def test_which_portions_take_the_form_through_lds():
+    from cie_amd.parts.attention import takes_prompt_form
+
+    assert takes_prompt_form(192, 200, 8, True, 256)  # many tiles: whatever is beside them
+    assert not takes_prompt_form(191, 100_000, 8, False, 256) and not takes_prompt_form(191, 100_000, 32, False, 256)
+    assert takes_prompt_form(191, 100, 0, True, 256) and takes_prompt_form(141, 100, 33, False, 256)
+    assert not takes_prompt_form(140, 685, 0, False, 256) and takes_prompt_form(140, 686, 0, False, 256)
+    assert not takes_prompt_form(140, 100_000, 0, True, 256)  # (a captured step's keys are not known)
+    assert not takes_prompt_form(0, 100_000, 0, False, 256)
