@@ -41,7 +41,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* lds_pointer;
 
-enum { DIRECT_BF16 = 0, DIRECT_SILU = 1, DIRECT_RESID = 2, DIRECT_PARTS = 3, DIRECT_ROPE = 4 };
+enum { DIRECT_BF16 = 0, DIRECT_SILU = 1, DIRECT_RESID = 2, DIRECT_PARTS = 3, DIRECT_ROPE = 4, DIRECT_ATOMIC = 5 };
 
 constexpr int kSlice = 64;                   // k of a stage: 128 bytes of a row
 constexpr int kLdsBytes = 160 * 1024;
@@ -60,11 +60,15 @@ struct DirectRope {
 
 struct DirectArgs {
     const bf16_t *a, *w, *bias;
-    void* c;            // BF16, SILU: bf16 [M, ldc]; RESID: the float32 stream; PARTS: float32 [parts, M, N]
+    void* c;            // BF16, SILU: bf16 [M, ldc]; RESID, ATOMIC: the float32 stream; PARTS: float32 [parts, M, N]
     int M, N, K, lda, ldc;
     int k_per_part;     // a multiple of kSlice
     int row_blocks, tiles;
     DirectRope rope;    // ROPE only
+    // SILU, or null: partial sums of squares [M, sumsq_parts] of the rows of the stream that A is short of 1/rms of
+    const float* row_sumsq;
+    int sumsq_parts;
+    float eps;
 };
 
 // 16-byte chunk `c` (0..7) of row `row` of a stage: the chunks of 16 rows that are read at one time lie in different banks
@@ -241,6 +245,32 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
             __builtin_amdgcn_raw_ptr_buffer_load_lds(of_a, (lds_pointer)to, 16, from[i], slice * kSlice * 2, 0, 0);
     };
 
+    // The rows' 1/rms: behind the first loads, some lanes to a row, eight pieces each at a time
+    __shared__ float row_scale[EPI == DIRECT_SILU ? kTileRows : 1];
+    auto scale_rows = [&] __attribute__((always_inline)) {
+        constexpr int kSpare = 64 * kWaves / kTileRows, kPer = kSpare >= 8 ? 8 : kSpare >= 4 ? 4 : 2, kHeld = 8;
+        static_assert(kSpare >= 2, "");
+        const int row = threadIdx.x / kPer, sub = threadIdx.x % kPer;
+        const float* sums = p.row_sumsq + static_cast<size_t>(min(m0 + min(row, kTileRows - 1), p.M - 1)) * p.sumsq_parts;
+        float sum = 0.f;
+        if (p.sumsq_parts % 4 == 0) {
+            for (int first = sub * 4; first < p.sumsq_parts; first += kHeld * kPer * 4) {
+                floatx4 held[kHeld];
+#pragma unroll
+                for (int i = 0; i < kHeld; ++i) held[i] = *reinterpret_cast<const floatx4*>(sums + min(first + i * kPer * 4, p.sumsq_parts - 4));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < kHeld; ++i)
+                    if (first + i * kPer * 4 < p.sumsq_parts) sum += (held[i][0] + held[i][1]) + (held[i][2] + held[i][3]);
+            }
+        } else {
+            for (int at = sub; at < p.sumsq_parts; at += kPer) sum += sums[at];
+        }
+#pragma unroll
+        for (int apart = 1; apart < kPer; apart *= 2) sum += __shfl_xor(sum, apart, kWave);
+        if (sub == 0 && row < kTileRows) row_scale[row] = 1.0f / sqrtf(sum / static_cast<float>(p.K) + p.eps);
+    };
+
     const int wn = (wave % kWN) * 16 * kN, wm = kColumns + (wave / kWN) * 16 * kM;  // this wave's rows in a stage
     RowPlaces<kM> places;
     floatx4 acc[kN][kM] = {};
@@ -271,7 +301,9 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int im = 0; im < kM; ++im)
-                acc[g][im] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, o.w[g]), __builtin_bit_cast(bf16x8, o.x[im]), acc[g][im], 0, 0, 0);
+                acc[g][im] = EPI == DIRECT_ATOMIC  // (there a lane has one column of four rows)
+                    ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, o.x[im]), __builtin_bit_cast(bf16x8, o.w[g]), acc[g][im], 0, 0, 0)
+                    : __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, o.w[g]), __builtin_bit_cast(bf16x8, o.x[im]), acc[g][im], 0, 0, 0);
             __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -297,9 +329,13 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
         if (s < slices)
 #pragma unroll
             for (int i = 0; i < kLoads; ++i) fetch_one(i, s, s);
-    if (many) {
+    if (many)
 #pragma unroll
         for (int i = 0; i < kFirst; ++i) fetch_one(i, kStages - 1, kStages - 1);
+    if constexpr (EPI == DIRECT_SILU) {
+        if (p.row_sumsq) scale_rows();
+    }
+    if (many) {
         if (uneven_more) wait_for_all_but<kAhead * kLoads + kFirst>();
         else wait_for_all_but<kAhead * kFewer + (kFirst < kFewer ? kFirst : kFewer)>();
         asm volatile("s_barrier" ::: "memory");
@@ -339,6 +375,31 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
         while (places.known < 3) places.step(p, m0 + (wm - kColumns), lane);
         store_rope<kN, kM>(p, acc, places, n0 / 32 + wn / 32, m0 + (wm - kColumns), lane);
         return;
+    }
+    if constexpr (EPI == DIRECT_ATOMIC) {  // every part of K adds its share (the hardware's own float add), 16 neighbours at a time
+#pragma unroll
+        for (int in = 0; in < kN; ++in) {
+            const int n = n0 + wn + 16 * in + lane % 16;
+            if (n >= p.N) continue;
+            const float add = p.bias && blockIdx.y == 0 ? to_float(p.bias[n]) : 0.f;
+#pragma unroll
+            for (int im = 0; im < kM; ++im)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int m = m0 + (wm - kColumns) + 16 * im + 4 * (lane / 16) + i;
+                    if (m < p.M) unsafeAtomicAdd(static_cast<float*>(p.c) + static_cast<size_t>(m) * p.ldc + n, acc[in][im][i] + add);
+                }
+        }
+        return;
+    }
+    if constexpr (EPI == DIRECT_SILU) {
+        if (p.row_sumsq)
+#pragma unroll
+            for (int im = 0; im < kM; ++im) {
+                const float scale = row_scale[wm - kColumns + 16 * im + lane % 16];
+#pragma unroll
+                for (int in = 0; in < kN; ++in) acc[in][im] *= scale;
+            }
     }
     constexpr int kOut = EPI == DIRECT_SILU ? kN / 2 : kN;
     constexpr int kPair = (EPI == DIRECT_BF16 || EPI == DIRECT_SILU) && kOut % 2 == 0 ? 2 : 1;  // tiles whose columns are neighbours
@@ -467,15 +528,16 @@ bool fits(const void* a, int lda, const void* w, const void* c, int M, int N, in
 
 }  // namespace
 
-// epilogue: 0 bf16, 1 SiLU-gate (N even, no bias), 2 residual (c float32 [M, N]), 3 parts (c float32 [parts, M, N]).
+// epilogue: 0 bf16, 1 SiLU-gate (N even, no bias), 2 residual (c float32 [M, N]), 3 parts (c float32 [parts, M, N]), 5 parts
+// that add their shares into c (float32 [M, N]) with atomic adds.
 // `columns` x `rows`: the workgroup's tile of the product (with the gate: half of the columns of either half).
 // K is a multiple of 64, lda of 8; a, w and c lie at multiples of 16 bytes; the operands hold fewer than 2^31 numbers.
 CIE_API int cie_gemm_direct(void* stream, const void* a, int lda, const void* w, const void* bias, void* c, int ldc, int M,
                             int N, int K, int epilogue, int columns, int rows, int parts) {
     if (!fits(a, lda, w, c, M, N, K) || parts < 1 || parts > 64) return CIE_BAD_ARGUMENT;
-    if ((epilogue == DIRECT_SILU && (N % 2 || bias)) || (epilogue != DIRECT_PARTS && parts != 1)) return CIE_BAD_ARGUMENT;
+    if ((epilogue == DIRECT_SILU && (N % 2 || bias)) || (epilogue != DIRECT_PARTS && epilogue != DIRECT_ATOMIC && parts != 1)) return CIE_BAD_ARGUMENT;
     if (ldc < (epilogue == DIRECT_SILU ? N / 2 : N)) return CIE_BAD_ARGUMENT;
-    DirectArgs p{static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(w), static_cast<const bf16_t*>(bias), c, M, N, K, lda, ldc, 0, 0, 0, {}};
+    DirectArgs p{static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(w), static_cast<const bf16_t*>(bias), c, M, N, K, lda, ldc, 0, 0, 0, {}, nullptr, 0, 0.f};
     p.k_per_part = ((K + parts - 1) / parts + kSlice - 1) / kSlice * kSlice;
     if (static_cast<long>(p.k_per_part) * (parts - 1) >= K) return CIE_BAD_ARGUMENT;  // (a part without k)
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -484,8 +546,20 @@ CIE_API int cie_gemm_direct(void* stream, const void* a, int lda, const void* w,
         case DIRECT_SILU: return run_form<DIRECT_SILU>(s, p, parts, columns, rows);
         case DIRECT_RESID: return run_form<DIRECT_RESID>(s, p, parts, columns, rows);
         case DIRECT_PARTS: return run_form<DIRECT_PARTS>(s, p, parts, columns, rows);
+        case DIRECT_ATOMIC: return run_form<DIRECT_ATOMIC>(s, p, parts, columns, rows);
     }
     return CIE_BAD_ARGUMENT;
+}
+
+// The SiLU-gate product of rows `a` = bf16(row of the stream x norm weight), whose 1/rms it applies to its sums: `row_sumsq` [M,
+// sumsq_parts] are partial sums of squares of the stream's rows (of K numbers).
+CIE_API int cie_gemm_direct_silu_scaled(void* stream, const void* a, int lda, const void* w, void* c, int ldc, int M, int N, int K,
+                                        int columns, int rows, const float* row_sumsq, int sumsq_parts, float eps) {
+    if (!fits(a, lda, w, c, M, N, K) || N % 2 || ldc < N / 2 || !row_sumsq || sumsq_parts < 1 || !(eps > 0.f) ||
+        (reinterpret_cast<uintptr_t>(row_sumsq) & 15) != 0)
+        return CIE_BAD_ARGUMENT;
+    DirectArgs p{static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(w), nullptr, c, M, N, K, lda, ldc, K, 0, 0, {}, row_sumsq, sumsq_parts, eps};
+    return run_form<DIRECT_SILU>(static_cast<hipStream_t>(stream), p, 1, columns, rows);
 }
 
 // The q/k/v product with the rotation and the cache write in its epilogue: `w` [N, K] stacks the rows of q_heads query
@@ -505,7 +579,7 @@ CIE_API int cie_gemm_direct_rope(void* stream, const void* a, int lda, const voi
         return CIE_BAD_ARGUMENT;
     DirectArgs p{static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(w), static_cast<const bf16_t*>(bias), c, M, N, K, lda, N, 0, 0, 0,
                  {cos_table, sin_table, positions, seq_of_token, seq_slot, block_table, table_width, static_cast<bf16_t*>(k_pool),
-                  static_cast<bf16_t*>(v_pool), q_heads, kv_heads, head_dim, page_size, rotate, write_kv}};
+                  static_cast<bf16_t*>(v_pool), q_heads, kv_heads, head_dim, page_size, rotate, write_kv}, nullptr, 0, 0.f};
     p.k_per_part = K;
     return run_form<DIRECT_ROPE>(static_cast<hipStream_t>(stream), p, 1, columns, rows);
 }

@@ -11,6 +11,7 @@ derive a token's cache slot from the block table and its position.
 
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass, field
 from typing import Any
 
@@ -60,6 +61,12 @@ class StepBatch:
     @property
     def all_decode(self) -> bool:
         return all(n == 1 for n in self.host_q_lens)
+
+    @functools.cached_property
+    def portions(self) -> tuple[int, int]:
+        """(tokens of the sequences that bring more than one, sequences that bring one): asked for by every layer."""
+        singles = self.host_q_lens.count(1)
+        return sum(self.host_q_lens) - singles, singles
 
     @property
     def max_q_len(self) -> int:

@@ -965,6 +965,7 @@ def folds_norm(rows: int, k: int) -> bool:
 
 
 TILE_BF16, TILE_SILU, TILE_RESID, TILE_PARTS = 0, 1, 2, 3
+TILE_ATOMIC = 5  # (only straight into LDS: parts of K add into a float32 stream with atomic adds)
 TILE_SHAPES = ((64, 64), (128, 64), (128, 128), (128, 256))  # columns x rows of a workgroup's tile
 # ... of the kernel whose operands go straight into LDS (K a multiple of 64)
 DIRECT_SHAPES = ((64, 64), (96, 64), (96, 128), (128, 64), (128, 128), (128, 192), (128, 256), (192, 128), (192, 192),
@@ -1007,14 +1008,17 @@ def gemm_tiles(weight: torch.Tensor, epilogue: int, a: torch.Tensor, columns: in
     """``a @ weight.T + bias`` in bfloat16 for some hundred rows, in tiles of ``columns`` x ``rows``: the bf16 result, its
     gated unit (``TILE_SILU``), added in place to the float32 stream ``into`` (``TILE_RESID``), or K in ``parts`` parts
     whose float32 sums come back as [parts, M, N] (``TILE_PARTS``).  ``direct``: by the kernel that loads its operands
-    straight into LDS (``DIRECT_SHAPES``; K a multiple of 64)."""
+    straight into LDS (``DIRECT_SHAPES``; K a multiple of 64); there the parts may also add themselves into ``into``
+    (``TILE_ATOMIC``: in no fixed order)."""
+    if epilogue == TILE_ATOMIC and not direct:
+        raise ValueError("parts add themselves into the stream only in the kernel that loads straight into LDS")
     m, n, k, lda = _tile_rows(a, weight)
     _check_tile_shape(columns, rows, direct, m, n, k, lda)
     if bias is not None:
         _gpu("bias", bias, torch.bfloat16, 1)
         if not (bias.shape[0] == n and epilogue != TILE_SILU):
             raise ValueError("bias does not fit")
-    if epilogue == TILE_RESID:
+    if epilogue in (TILE_RESID, TILE_ATOMIC):
         _gpu("into", into, torch.float32, 2)
         if not (into.shape == (m, n) and into.data_ptr() % 16 == 0):
             raise ValueError(f"into must be {(m, n)}, is {tuple(into.shape)}")
@@ -1027,6 +1031,22 @@ def gemm_tiles(weight: torch.Tensor, epilogue: int, a: torch.Tensor, columns: in
     _run(entry, getattr(load_library(), entry)(
         _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(out), _i(out.shape[-1]), _i(m), _i(n), _i(k), _i(epilogue),
         _i(columns), _i(rows), _i(parts)))
+    return out
+
+
+def gemm_tiles_silu_scaled(weight: torch.Tensor, a: torch.Tensor, columns: int, rows: int, row_sumsq: torch.Tensor,
+                           eps: float) -> torch.Tensor:
+    """The gated unit of :func:`gemm_tiles` (``direct``) of rows that lack their 1/rms, which it applies to its sums:
+    ``row_sumsq`` [M, parts] holds partial sums of squares of the stream's rows (as ``gemm_fused`` takes them)."""
+    m, n, k, lda = _tile_rows(a, weight)
+    _check_tile_shape(columns, rows, True, m, n, k, lda)
+    _gpu("row_sumsq", row_sumsq, torch.float32, 2)
+    if not (n % 2 == 0 and row_sumsq.shape[0] == m and row_sumsq.shape[1] >= 1 and eps > 0 and row_sumsq.data_ptr() % 16 == 0):
+        raise ValueError(f"row_sumsq {tuple(row_sumsq.shape)} does not fit {m} rows, or the weight's {n} rows are no pairs")
+    out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=a.device)
+    _run("cie_gemm_direct_silu_scaled", load_library().cie_gemm_direct_silu_scaled(
+        _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(out), _i(n // 2), _i(m), _i(n), _i(k), _i(columns), _i(rows),
+        _ptr(row_sumsq), _i(row_sumsq.shape[1]), _f(eps)))
     return out
 
 

@@ -275,6 +275,57 @@ def choose_tiles(rows: int, n: int, k: int, row_stride: int, most_parts: int = 1
     return None if form is None else Tiles(*form, False)
 
 
+# Products of FEW_TILE_ROWS to FUSED_PARTS_ROWS rows (more: the model above).  The forms whose waves read every row for every 16
+# or 32 columns take longer with every row; the tiles that load straight into LDS read a row once for their 64 to 128 columns
+# (MI355X, us, chains of one product from memory, the other form or the library and tiles; down, parts added with atomic adds:
+# 3B 48 rows 13.6, 12.8, 64 14.9, 14.0, 96 18.8, 16.7, 128 23.3, 18.5; 7B 128 rows 53.6, 39.4; 0.5B 128 rows 10.5, 7.5; at 32 rows
+# level; output product of more than FUSED_SMALL_WEIGHT numbers, in parts: 7B 17 rows 12.3, 8.1, 96 rows 20.4, 11.9, 14B 128 rows
+# 27.9, 18.9; gate/up: 0.5B 48 rows 10.5, 7.3, 128 rows 14.5, 8.8, 1.5B 64 rows 17.6, 16.0, 128 rows 25.6, 20.8, 3B 64 rows 22.0, 21.5,
+# 96 rows 27.4, 25.7, 128 rows 31.8, 25.8, 14B 128 rows 72.6, 65.7; 7B, whose tiles of 128 rows do not meet the units in one turn,
+# 96 rows 68.2, 71.6).
+FEW_TILE_ROWS = 48
+FEW_TILE_PARTS = (1, 2, 4, 8)
+FEW_GATE_WIDTH = 72  # columns of gate and up a unit up to which 64 rows and fewer go to tiles (3B's 86: level, 1.5B's 70: 8 %)
+
+
+@functools.lru_cache(maxsize=4096)
+def plan_few_tiles(rows: int, n: int, k: int, most_parts: int, units: int) -> Optional[tuple[int, int, int]]:
+    """(columns, rows, parts) of the tiles of up to FUSED_PARTS_ROWS rows, or ``None`` if no form meets the units in one turn: of
+    those with nearly the most workgroups that do, the one that streams the weight the fewest times, in the fewest parts."""
+    forms = []
+    for tile_rows in (64,) if rows <= 64 else (64, 128):
+        for columns in (64, 96, 128):
+            if (columns, tile_rows) not in ops.DIRECT_SHAPES:
+                continue
+            for parts in FEW_TILE_PARTS:
+                groups = -(-n // columns) * -(-rows // tile_rows) * parts
+                if parts <= most_parts and groups <= units and -(-(-(-k // parts)) // ops.DIRECT_SLICE) * ops.DIRECT_SLICE * (parts - 1) < k:
+                    forms.append((groups, columns, tile_rows, parts))
+    if not forms:
+        return None
+    most = max(forms)[0]
+    _groups, columns, tile_rows, parts = min((f for f in forms if f[0] >= 0.9 * most), key=lambda f: (-(-rows // f[2]), f[3], -f[0], f[1]))
+    return columns, tile_rows, parts
+
+
+def few_tiles(x: torch.Tensor, weight: torch.Tensor, most_parts: int = 1, into: Optional[torch.Tensor] = None,
+              fewest: int = FEW_TILE_ROWS) -> Optional[tuple[int, int, int]]:
+    """What :func:`plan_few_tiles` says for these operands, if the tiles take them at all."""
+    rows, k = x.shape
+    if not fewest <= rows <= FUSED_PARTS_ROWS or not takes_tiles(rows, x, weight, into, beyond=FUSED_ROWS):
+        return None
+    if not ops.direct_fits(rows, weight.shape[0], k, x.stride(0)):
+        return None
+    return plan_few_tiles(rows, weight.shape[0], k, most_parts, ops.compute_units())
+
+
+def gate_tiles(x: torch.Tensor, weight: torch.Tensor) -> Optional[tuple[int, int, int]]:
+    """... for a gated unit's product."""
+    if x.shape[0] <= 64 and weight.shape[0] > FEW_GATE_WIDTH * ops.compute_units():
+        return None
+    return few_tiles(x, weight)
+
+
 @dataclass
 class RowSumsq:
     """Stands where a branch output would: the branch was already added into the
@@ -431,12 +482,13 @@ def _fusable(rows: int, k: int, row_stride: int, weight: torch.Tensor) -> bool:
     return weight.dtype == torch.bfloat16 and rows >= 1 and k % 8 == 0 and row_stride % 8 == 0
 
 
-def takes_tiles(rows: int, x: torch.Tensor, weight: torch.Tensor, into: Optional[torch.Tensor] = None) -> bool:
+def takes_tiles(rows: int, x: torch.Tensor, weight: torch.Tensor, into: Optional[torch.Tensor] = None,
+                beyond: int = FUSED_PARTS_ROWS) -> bool:
     """Whether the tile kernels take these operands (of a product that is ``_fusable``): beyond the rows of the streaming
     kernels, on the GPU, in rows that lie apart and at addresses that 16-byte loads and stores can use.  Whatever else a
     caller brings (rows read across, rows that share their numbers, as one row expanded to many does, a stream that starts
     off a 16-byte line, host tensors) is the library's or torch's, as it was."""
-    if rows <= FUSED_PARTS_ROWS or not x.is_cuda:
+    if rows <= beyond or not x.is_cuda:
         return False
     apart, inner = x.stride()
     return (inner == 1 and apart >= x.shape[1] and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
@@ -466,6 +518,9 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
         rows, k = x.rows.shape
         if epilogue == "silu" and weight.shape[0] % 2 == 0 and bias is None and weight.dtype == torch.bfloat16:
             if _fusable(rows, k, x.rows.stride(0) if rows > 1 else k, weight):
+                tiles = gate_tiles(x.rows, weight)
+                if tiles is not None:
+                    return ops.gemm_tiles_silu_scaled(weight, x.rows, tiles[0], tiles[1], x.sumsq, x.eps)
                 waves, own_unit = plan_shared_silu(-(-weight.shape[0] // 32))
                 if FUSED_ROWS < rows <= SHARED_SILU_ROWS or (rows <= FUSED_ROWS and own_unit):
                     return ops.gemm_shared_rows(weight, ops.EPI_SILU, x.rows, waves=waves, row_sumsq=x.sumsq, eps=x.eps)
@@ -493,6 +548,10 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
         # (atomic adds cost the product nothing, measured against partial products written for the next norm
         # kernel to sum: 10.3 us either way for the 3B shape's down product at 8 rows; and the kernel that summed
         # them falls away)
+        tiles = few_tiles(x, weight, FEW_TILE_PARTS[-1], into)
+        if tiles is not None:
+            ops.gemm_tiles(weight, ops.TILE_ATOMIC, x, tiles[0], tiles[1], bias, into, tiles[2], direct=True)
+            return Added()
         column_tiles, waves, parts = plan_shared_parts(-(-n // 16), k)
         ops.gemm_shared_rows(weight, ops.EPI_ATOMIC, x, bias=bias, column_tiles=column_tiles, waves=waves,
                              k_parts=parts, add_into=into)
@@ -501,9 +560,16 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
             and k >= PART_MIN_K and x.data_ptr() % 16 == 0):
         # a branch that whoever adds it sums itself (the down product of the parallel block, 8 rows, K 11,008: 17 us whole,
         # 11 in 8 parts, and 0.4 more in the kernel that adds them)
+        tiles = few_tiles(x, weight, FEW_TILE_PARTS[-1])
+        if tiles is not None:
+            return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, tiles[0], tiles[1], bias, None, tiles[2], direct=True))
         column_tiles, waves, parts = plan_shared_parts(-(-n // 16), k)
         return KParts(ops.gemm_shared_rows(weight, ops.EPI_PARTIAL, x, bias=bias, column_tiles=column_tiles, waves=waves,
                                            k_parts=parts))
+    if fusable and silu and n % 2 == 0 and bias is None and into is None and not wants_f32 and rows <= FUSED_PARTS_ROWS:
+        tiles = gate_tiles(x, weight)
+        if tiles is not None:
+            return ops.gemm_tiles(weight, ops.TILE_SILU, x, tiles[0], tiles[1], direct=True)
     if fusable and silu and n % 2 == 0 and bias is None and into is None and not wants_f32 and rows <= SHARED_SILU_ROWS:
         waves, own_unit = plan_shared_silu(-(-n // 32))
         if rows > FUSED_ROWS or own_unit:
@@ -529,6 +595,11 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
             return ops.gemm_fused(weight, ops.EPI_SILU, x)
         elif not silu:
             return ops.gemm_fused(weight, ops.EPI_F32 if wants_f32 else ops.EPI_BF16, x, bias=bias)
+    if (fusable and not wants_f32 and not silu and into is not None and sums_parts and FUSED_ROWS < rows <= FUSED_PARTS_ROWS
+            and into.is_contiguous() and tuple(into.shape) == (rows, n)):
+        tiles = few_tiles(x, weight, FEW_TILE_PARTS[-1], into, fewest=FUSED_ROWS + 1)
+        if tiles is not None:  # (the norm behind it sums the parts)
+            return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, tiles[0], tiles[1], bias, None, tiles[2], direct=True))
     if fusable and not wants_f32 and takes_tiles(rows, x, weight, into):
         stride, most = x.stride(0), TILE_PARTS[-1] if sums_parts else 1
         if into is not None and not silu and into.is_contiguous() and tuple(into.shape) == (rows, n):

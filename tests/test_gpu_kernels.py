@@ -321,6 +321,32 @@ def test_gemm_direct(ops, shape, tile):
             torch.testing.assert_close(got.double().sum(0), product + b.double(), **sums)
 
 
+@pytest.mark.parametrize("shape", [(41, 64, 512), (64, 130, 1088), (65, 100, 2112), (96, 520, 960), (128, 96, 1024), (1, 66, 128)])
+@pytest.mark.parametrize("tile", [(64, 64), (96, 64), (128, 64), (96, 128), (128, 128)])
+def test_gemm_direct_of_few_rows(ops, shape, tile):
+    """Parts that add themselves into a stream (in no fixed order: the bound is that of float32 sums of k products of numbers
+    about 1), and the gated unit of rows that lack their 1/rms, whose partial sums of squares come in any number."""
+    m, n, k = shape
+    a, w, b = rand((m, k), torch.bfloat16, 26), rand((n, k), torch.bfloat16, 27), rand((n,), torch.bfloat16, 28)
+    product = a.double() @ w.double().t()
+    for parts in (1, 2, 8):
+        if (parts - 1) * (-(-(-(-k // parts)) // 64) * 64) >= k:
+            continue
+        for bias in (None, b):
+            stream = rand((m, n), torch.float32, 29)
+            expect = stream.double() + product + (0.0 if bias is None else bias.double())
+            ops.gemm_tiles(w, ops.TILE_ATOMIC, a, *tile, bias=bias, into=stream, parts=parts, direct=True)
+            torch.testing.assert_close(stream.double(), expect, rtol=1e-4, atol=1e-4 * math.sqrt(k))
+    gate, up = product[:, : n // 2], product[:, n // 2:]
+    for sums in (1, 3, 8, 56, 260):
+        sumsq = rand((m, sums), torch.float32, 30).abs() * k
+        scale = torch.rsqrt(sumsq.double().sum(1, keepdim=True) / k + 1e-5)
+        got = ops.gemm_tiles_silu_scaled(w, a, *tile, sumsq, 1e-5).double()
+        torch.testing.assert_close(got, torch.nn.functional.silu(gate * scale) * (up * scale), rtol=1e-2, atol=1e-2 * k / float(sumsq.sum(1).min() / k))
+    with pytest.raises(ValueError, match="straight into LDS"):
+        ops.gemm_tiles(w, ops.TILE_ATOMIC, a, 64, 64, into=stream, parts=1)
+
+
 @pytest.mark.parametrize("gate", [0.0, 0.5, -0.5, 9.0, -9.0, 40.0, -40.0, -80.0, 1e30, -1e30, math.inf])
 def test_gemm_direct_gate_over_its_range(ops, gate):
     """Each row's one number k = 0 is its gate, k = 1 its up; the result is rounded once to bf16 (half of 2^-7), behind float32

@@ -189,3 +189,20 @@ def test_which_portions_take_the_form_through_lds():
     assert not takes_prompt_form(140, 685, 0, False, 256) and takes_prompt_form(140, 686, 0, False, 256)
     assert not takes_prompt_form(140, 100_000, 0, True, 256)  # (a captured step's keys are not known)
     assert not takes_prompt_form(0, 100_000, 0, False, 256)
+
+
+@pytest.mark.parametrize("rows", [17, 41, 64, 65, 128])
+@pytest.mark.parametrize("n,k", [(896, 4864), (2048, 11008), (3584, 18944), (5120, 5120), (64, 64), (9728, 896), (22016, 2048), (40000, 64)])
+@pytest.mark.parametrize("most", [1, 8])
+def test_tiles_of_few_rows_meet_the_units_once(rows, n, k, most):
+    from cie_amd.kernels import ops
+    from cie_amd.parts.linear import plan_few_tiles
+
+    form = plan_few_tiles(rows, n, k, most, 256)
+    if form is None:
+        assert min(-(-n // 128) * -(-rows // r) for r in ((64,) if rows <= 64 else (64, 128))) > 256
+        return
+    columns, tile_rows, parts = form
+    assert (columns, tile_rows) in ops.DIRECT_SHAPES and parts <= most
+    assert -(-n // columns) * -(-rows // tile_rows) * parts <= 256
+    assert -(-(-(-k // parts)) // 64) * 64 * (parts - 1) < k  # (no part without k)
