@@ -28,7 +28,7 @@ __device__ __forceinline__ float gelu_tanh(float z) {
 }
 
 // ---------------------------------------------------------------------------------------------- retention
-// Three kernels.  (a) Every token's queries and keys, turned by its position, the keys scaled, as float32 rows padded
+// Three kernels, or one for steps of one token a sequence (d).  (a) Every token's queries and keys, turned by its position, the keys scaled, as float32 rows padded
 // with zeros to `padded` numbers per head: [tokens, heads, 2, padded] (what passes through an activation on its way in
 // does so here).  (b) The walk over the tokens, below, token by token for steps of few tokens a sequence, or (b') in
 // blocks on the matrix cores for prompts' portions.  (c) The norm over a head's or over several heads' read-outs, the
@@ -641,6 +641,137 @@ int launch_retention(hipStream_t s, dim3 grid, int threads, size_t lds, const vo
     return cie_after_launch();
 }
 
+// (d) A step of one token a sequence: one workgroup per (sequence, head) does all of (a) to (c) at once.  Such a step reads
+// and writes the memory once and has next to no arithmetic, and three launches that hand float32 rows on through memory cost
+// more than that.  A thread takes four adjacent columns, 16 bytes, of kStepRows rows (a wave reads whole lines; the 4-byte
+// columns of (b) cost as much as the launches from some sixteen sequences on), the row groups' shares of o meet in LDS,
+// and because the workgroup has all columns of its head, the norm and the gate follow there.  What the token brings is asked
+// for in front of the memory's rows: behind them it waits for them, and the gate's columns asked for at the end were another
+// way to memory (7.1 us for one sequence, 10.2 for eight).  In place of the three kernels, 8 heads of 128 x 256: one
+// sequence 10.8 -> 6.2 us, eight 16.2 -> 9.1 (64 workgroups; the bytes take 3.2), 64 70.1 -> 33.8 (25.8); 32 heads of
+// 64 x 64: 10.3 -> 3.9, 13.4 -> 5.1, 55.2 -> 16.8.  2 or 4 rows a thread and more groups are up to 6 % faster for heads
+// of 64 numbers and fewer and up to 14 % slower for larger ones of many sequences.
+constexpr int kStepThreads = 1024;  // (most columns and rows of a head, too: a thread prepares one of each)
+constexpr int kStepRows = 8;
+
+template <typename T>
+__global__ void __launch_bounds__(kStepThreads)
+retention_step_kernel(const T* __restrict__ proj, long ldp, int q_off, int k_off, int v_off, int g_off,
+                      const float* __restrict__ cos_table, const float* __restrict__ sin_table, int rot,
+                      const float* __restrict__ decay, float* __restrict__ state, const int* __restrict__ seq_slot,
+                      const int* __restrict__ positions, const int* __restrict__ q_start_loc, T* __restrict__ out, int heads,
+                      int dim, int vdim, int quads, int groups, float eps, float key_scale, int act,
+                      const float* __restrict__ weight, int gate_act) {
+    extern __shared__ float4 lds4[];
+    float* o_s = reinterpret_cast<float*>(lds4);  // [groups][vdim]
+    float* v_s = o_s + groups * vdim;             // [vdim]
+    float* q_s = v_s + vdim;                      // [dim], then the keys
+    float* k_s = q_s + dim;
+    float* sums = k_s + dim;                      // [waves]
+    const int seq = blockIdx.x / heads;
+    const int head = blockIdx.x - seq * heads;
+    const int first = q_start_loc[seq];
+    const int end = q_start_loc[seq + 1];
+    if (end <= first) return;  // (a place without a token: the whole workgroup leaves)
+    const int quad = threadIdx.x % quads;
+    const int grp = threadIdx.x / quads;
+    const bool owner = grp < groups;
+    float* mem = state + (static_cast<size_t>(seq_slot[seq]) * heads + head) * dim * vdim + quad * 4;
+    const float fade = decay[head];
+    // what this thread prepares: a column's value and gate, and (from the last thread on down: where the columns leave waves
+    // over, those take them) a number of the query and the key with its partner in the rotation
+    const int back = blockDim.x - 1 - threadIdx.x;
+    const int c = min(static_cast<int>(threadIdx.x), vdim - 1);
+    const int d = min(back, dim - 1);
+    const int half = rot / 2;
+    const bool turns = d < rot;
+    const int pair = !turns ? 0 : d < half ? d : d - half;
+    const int other = !turns ? d : d < half ? d + half : pair;
+    const float gain = *(weight ? weight + head * vdim + c : decay);
+    const float* cos_at = turns ? cos_table : decay;  // (an address that can be read either way: loads under a condition
+    const float* sin_at = turns ? sin_table : decay;  // are waited for one by one)
+    T v_in, g_in, q_in, k_in, q_other, k_other;
+    float c_in, s_in;
+    auto fetch = [&](int t) {
+        const T* row = proj + static_cast<size_t>(t) * ldp;
+        const T* qh = row + q_off + head * dim;
+        const T* kh = row + k_off + head * dim;
+        const size_t at = turns ? static_cast<size_t>(positions[t]) * half + pair : 0;
+        q_in = qh[d];
+        k_in = kh[d];
+        q_other = qh[other];
+        k_other = kh[other];
+        v_in = row[v_off + head * vdim + c];
+        g_in = row[g_off + head * vdim + c];
+        c_in = cos_at[at];
+        s_in = sin_at[at];
+    };
+    fetch(first);
+    // (behind the token's numbers, which are needed first and would wait for whatever was asked for before them; a row past
+    // the last reads the last again)
+    piece_t S[kStepRows];
+#pragma unroll
+    for (int r = 0; r < kStepRows; ++r)
+        S[r] = *reinterpret_cast<const piece_t*>(mem + static_cast<size_t>(min(grp + r * groups, dim - 1)) * vdim);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int t = first; t < end; ++t) {
+        float qv = activated(to_float(q_in), act), kv = activated(to_float(k_in), act);
+        if (turns) {
+            const float q2 = activated(to_float(q_other), act), k2 = activated(to_float(k_other), act);
+            qv = d < half ? qv * c_in - q2 * s_in : qv * c_in + q2 * s_in;
+            kv = d < half ? kv * c_in - k2 * s_in : kv * c_in + k2 * s_in;
+        }
+        if (back < dim) {
+            q_s[d] = qv;
+            k_s[d] = kv * key_scale;
+        }
+        if (threadIdx.x < vdim) v_s[c] = activated(to_float(v_in), act);
+        const float g = to_float(g_in);
+        __syncthreads();
+        if (t + 1 < end) fetch(t + 1);
+        if (owner) {
+            const piece_t v = *reinterpret_cast<const piece_t*>(v_s + quad * 4);
+            piece_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < kStepRows; ++r) {
+                const int at = grp + r * groups;
+                const bool live = at < dim;
+                const float k = k_s[min(at, dim - 1)];
+                const float q = q_s[min(at, dim - 1)];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    S[r][j] = fmaf(fade, S[r][j], k * v[j]);
+                    o[j] = live ? fmaf(S[r][j], q, o[j]) : o[j];  // (a row that is not there adds nothing)
+                }
+            }
+            *reinterpret_cast<piece_t*>(o_s + grp * vdim + quad * 4) = o;
+        }
+        __syncthreads();
+        float o = 0.f;
+        if (threadIdx.x < vdim)
+#pragma unroll 8
+            for (int i = 0; i < groups; ++i) o += o_s[i * vdim + c];  // (the groups in their order)
+        const float wave_sq = wave_sum(o * o);
+        if (threadIdx.x % kWave == 0) sums[threadIdx.x / kWave] = wave_sq;
+        __syncthreads();
+        if (threadIdx.x < vdim) {
+            float sum_sq = 0.f;
+            for (int w = 0; w * kWave < vdim; ++w) sum_sq += sums[w];
+            const float inv = 1.0f / sqrtf(sum_sq / static_cast<float>(vdim) + eps);
+            const float open = gate_act == 1 ? sigmoidf(g) : g * sigmoidf(g);
+            float y = o * inv;
+            if (weight) y *= gain;
+            out[(static_cast<size_t>(t) * heads + head) * vdim + c] = from_float<T>(y * open);
+        }
+        // (the next token's numbers go where none but the threads before the second barrier read; `sums` is written behind
+        // two more)
+    }
+    if (owner)
+#pragma unroll
+        for (int r = 0; r < kStepRows; ++r)
+            if (grp + r * groups < dim) *reinterpret_cast<piece_t*>(mem + static_cast<size_t>(grp + r * groups) * vdim) = S[r];
+}
+
 // ---------------------------------------------------------------------------------------------- convolution
 // (`act`: what the sum passes through, 0 nothing, 1 silu; O: the type it is stored in)
 template <typename T, typename O>
@@ -1056,6 +1187,37 @@ CIE_API int cie_retention(void* stream, int dtype, const void* proj, long ldp, i
         else CIE_NORM(retention_norm_kernel, bf16_t);
     }
 #undef CIE_NORM
+    return cie_after_launch();
+}
+
+CIE_API int cie_retention_step(void* stream, int dtype, const void* proj, long ldp, int q_off, int k_off, int v_off, int g_off,
+                               const float* cos_table, const float* sin_table, int rot, const float* decay, float* state,
+                               const int* seq_slot, const int* positions, const int* q_start_loc, void* out, int sequences,
+                               int heads, int dim, int vdim, float eps, float key_scale, int act,
+                               const float* norm_weight, int gate_act) {
+    if (act < 0 || act > 1 || gate_act < 0 || gate_act > 1 || sequences < 0 || heads <= 0 || dim <= 0 || dim > kStepThreads ||
+        vdim <= 0 || vdim % 4 || vdim > kStepThreads || rot < 0 || rot % 2 || rot > dim ||
+        (rot > 0 && (!cos_table || !sin_table)) || !(eps > 0.f) || reinterpret_cast<size_t>(state) % 16 ||
+        static_cast<long>(sequences) * heads > 0x7fffffffL || (dtype != CIE_F32 && dtype != CIE_BF16))
+        return CIE_BAD_ARGUMENT;
+    const int quads = vdim / 4;
+    const int groups = (dim + kStepRows - 1) / kStepRows;
+    if (quads * groups > kStepThreads) return CIE_BAD_ARGUMENT;
+    if (sequences == 0) return CIE_OK;
+    int threads = quads * groups;
+    threads = threads < vdim ? vdim : threads;
+    threads = threads < dim ? dim : threads;
+    threads = (threads + kWave - 1) / kWave * kWave;
+    const size_t lds = sizeof(float) * (static_cast<size_t>(groups + 1) * vdim + 2 * static_cast<size_t>(dim) + threads / kWave);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+#define CIE_STEP(T)                                                                                                        \
+    retention_step_kernel<T><<<sequences * heads, threads, lds, s>>>(                                                      \
+        static_cast<const T*>(proj), ldp, q_off, k_off, v_off, g_off, cos_table, sin_table, rot, decay, state, seq_slot,   \
+        positions, q_start_loc, static_cast<T*>(out), heads, dim, vdim, quads, groups, eps, key_scale, act, norm_weight,   \
+        gate_act)
+    if (dtype == CIE_F32) CIE_STEP(float);
+    else CIE_STEP(bf16_t);
+#undef CIE_STEP
     return cie_after_launch();
 }
 

@@ -1459,6 +1459,18 @@ def plan_retention(dim: int, vdim: int, units: int = 1) -> tuple[int, int, int, 
     return rows, groups, parts, piece, chunk
 
 
+RETENTION_STEP_THREADS = 1024  # of a workgroup; no more columns and rows of a head either (csrc/recurrent.hip)
+RETENTION_STEP_ROWS = 8        # that a thread keeps, four columns each
+
+
+def steps_retention(tokens: int, sequences: int, dim: int, vdim: int, norm_span: int) -> bool:
+    """Whether a step goes to the kernel that turns, walks, norms and gates a head in one workgroup: one token a
+    sequence, a norm over single heads, and heads whose memory a workgroup's registers hold in 16-byte pieces.  (Faster
+    than the three kernels wherever it runs: heads of 4 x 72 to 256 x 128, 1 to 128 sequences, 1.7 to 3.5 times.)"""
+    return (tokens == sequences and norm_span == 1 and vdim % 4 == 0 and max(dim, vdim) <= RETENTION_STEP_THREADS
+            and vdim // 4 * -(-dim // RETENTION_STEP_ROWS) <= RETENTION_STEP_THREADS)
+
+
 def retention(proj: torch.Tensor, offsets: tuple[int, int, int, int], cos: Optional[torch.Tensor],
               sin: Optional[torch.Tensor], rot: int, decay: torch.Tensor, state: torch.Tensor, seq_slot: torch.Tensor,
               positions: torch.Tensor, q_start_loc: torch.Tensor, sequences: int, heads: int, dim: int, vdim: int,
@@ -1473,7 +1485,8 @@ def retention(proj: torch.Tensor, offsets: tuple[int, int, int, int], cos: Optio
     ``heads``: the token's whole row), multiplied by ``norm_weight`` (float32 [heads * vdim]) where given, and by
     ``silu`` or ``sigmoid`` (``gate``) of the gate columns.  Steps of ``RETENTION_BLOCKS_FROM`` tokens a sequence and more
     walk in blocks of 32 tokens on the matrix cores in float32 (heads of up to ``RETENTION_BLOCKS_MAX_DIM`` numbers a key,
-    scratch of up to ``RETENTION_BLOCKS_MAX_BYTES``), others token by token: the same sums in another order.
+    scratch of up to ``RETENTION_BLOCKS_MAX_BYTES``), others token by token, one token a sequence in one kernel
+    (``steps_retention``): the same sums in another order.
     Returns [T, heads * vdim] in ``proj``'s type."""
     if activation not in RETENTION_ACTIVATIONS or gate not in RETENTION_GATES:
         raise ValueError(f"activation is one of {list(RETENTION_ACTIVATIONS)}, gate one of {list(RETENTION_GATES)}")
@@ -1503,6 +1516,15 @@ def retention(proj: torch.Tensor, offsets: tuple[int, int, int, int], cos: Optio
         _gpu(name, meta, torch.int32, 1)
         if meta.shape[0] < least:
             raise ValueError(f"{name} has {meta.shape[0]} entries, {least} are needed")
+    ldp = proj.stride(0) if tokens > 1 else max(proj.stride(0), proj.shape[1])
+    if steps_retention(tokens, sequences, dim, vdim, norm_span) and state.data_ptr() % 16 == 0:
+        out = torch.empty((tokens, heads * vdim), dtype=proj.dtype, device=proj.device)
+        _run("cie_retention_step", load_library().cie_retention_step(
+            _stream(), _i(_code(proj.dtype)), _ptr(proj), ldp, _i(q_off), _i(k_off), _i(v_off),
+            _i(g_off), _ptr(cos if rot else None), _ptr(sin if rot else None), _i(rot), _ptr(decay), _ptr(state),
+            _ptr(seq_slot), _ptr(positions), _ptr(q_start_loc), _ptr(out), _i(sequences), _i(heads), _i(dim), _i(vdim),
+            _f(eps), _f(key_scale), _i(RETENTION_ACTIVATIONS[activation]), _ptr(norm_weight), _i(RETENTION_GATES[gate])))
+        return out
     rows, groups, parts, piece, chunk = plan_retention(dim, vdim, max(1, sequences * heads))
     # sequences that bring many tokens (prompts' portions) walk in blocks of 32 tokens on the matrix cores, float32
     # operands and sums, every block's own sums at once and only the memory itself in order; steps of few tokens a
@@ -1518,7 +1540,6 @@ def retention(proj: torch.Tensor, offsets: tuple[int, int, int, int], cos: Optio
     turned = torch.empty((tokens, heads, 2, parts * groups * rows), dtype=torch.float32, device=proj.device)
     raw = torch.empty((2 if blocks else parts, tokens, heads * vdim), dtype=torch.float32, device=proj.device)
     out = torch.empty((tokens, heads * vdim), dtype=proj.dtype, device=proj.device)
-    ldp = proj.stride(0) if tokens > 1 else max(proj.stride(0), proj.shape[1])
     _run("cie_retention", load_library().cie_retention(
         _stream(), _i(_code(proj.dtype)), _ptr(proj), ldp, _i(q_off), _i(k_off), _i(v_off), _i(g_off),
         _ptr(cos if rot else None), _ptr(sin if rot else None), _i(rot), _ptr(decay), _ptr(state), _ptr(seq_slot),

@@ -572,3 +572,69 @@ def test_retention_over_the_edges_of_its_pieces(dtype, lengths, heads, dim, vdim
                 bound = bound + 2.0 ** -8 * want.abs()
             assert torch.all((out[t].cpu().double().view(heads, vdim) - want).abs() <= bound + 1e-6)
         assert torch.all((state[slots[i]].cpu().double() - S).abs() <= (2 * n + 16) * 2.0 ** -24 * (size + 1))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lengths,heads,dim,vdim,rot,activation", [
+    ((1,), 1, 1, 4, 0, None), ((1, 1, 1), 3, 9, 72, 4, "silu"), ((1,) * 5, 8, 128, 256, 128, None), ((1, 1), 2, 1024, 32, 0, None),
+    ((1,), 2, 8, 1024, 6, "silu"), ((0, 2, 1, 1), 2, 72, 12, 72, None), ((1,) * 40, 4, 64, 64, 64, None)])
+def test_retention_of_one_token_a_sequence(dtype, lengths, heads, dim, vdim, rot, activation):
+    """The kernel that does a step in one workgroup a head, at the smallest and largest heads it takes, rows and columns
+    that leave threads over, whole, partial and no rotation, and a sequence without a token beside one with two; against
+    64 bits.  Columns that are no multiple of four, and a memory off a 16-byte line, take the general path."""
+    from cie_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(6)
+    tokens, slots = sum(lengths), list(range(len(lengths)))[::-1]
+    assert ops.steps_retention(tokens, len(lengths), dim, vdim, 1)
+    assert not ops.steps_retention(tokens, len(lengths), dim, vdim + 2, 1)
+    assert not ops.steps_retention(tokens + 1, len(lengths), dim, vdim, 1)
+    assert not ops.steps_retention(tokens, len(lengths), dim, vdim, 2)
+    proj = torch.randn(tokens, heads * (2 * dim + 2 * vdim) + 3, generator=g).to(dtype).cuda()  # (rows off 16-byte lines)
+    offsets = (3, 3 + heads * dim, 3 + 2 * heads * dim, 3 + 2 * heads * dim + heads * vdim)
+    decay, weight = torch.linspace(0.9, 0.99, heads).cuda(), torch.rand(heads * vdim, generator=g).cuda() + 0.5
+    kept = torch.randn(len(lengths), heads, dim, vdim, generator=g)
+    starts = [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    meta = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+    at = torch.randint(0, 500, (tokens,), generator=g)
+    angles = torch.arange(500)[:, None] * 0.7 ** torch.arange(rot // 2)[None, :]
+    cos, sin = angles.cos().float().cuda(), angles.sin().float().cuda()
+    run = lambda state: ops.retention(proj, offsets, cos if rot else None, sin if rot else None, rot, decay, state, meta(slots),
+                                      meta(at.tolist()), meta(starts), len(lengths), heads, dim, vdim, 1e-6, 0.25, 499,
+                                      activation=activation, norm_weight=weight)
+    state = kept.cuda()
+    off_line = torch.empty(kept.numel() + 1, device="cuda")[1:].view(kept.shape).copy_(kept)  # the general path
+    out, general = run(state), run(off_line)
+    p = proj.cpu().double()
+    act = (lambda z: z * torch.sigmoid(z)) if activation else (lambda z: z)
+    q, k = (act(p[:, o: o + heads * dim]).view(tokens, heads, dim) for o in offsets[:2])
+    v, gate = (p[:, o: o + heads * vdim].view(tokens, heads, vdim) for o in offsets[2:])
+    v = act(v)
+    c, s = cos.cpu().double()[at][:, None], sin.cpu().double()[at][:, None]
+
+    def turned(z):
+        a, b, rest = z[..., :rot // 2], z[..., rot // 2: rot], z[..., rot:]
+        size = torch.cat((a.abs() + b.abs(), a.abs() + b.abs(), rest.abs()), -1)
+        return torch.cat((a * c - b * s, b * c + a * s, rest), -1), size
+
+    (q, q_size), (k, k_size) = turned(q), turned(k)
+    f = decay.cpu().double()[:, None, None]
+    w = weight.cpu().double().view(heads, vdim)
+    for i, n in enumerate(lengths):
+        S, size = kept[slots[i]].double(), kept[slots[i]].double().abs()
+        for t in range(starts[i], starts[i] + n):
+            S = f * S + 0.25 * k[t][:, :, None] * v[t][:, None, :]
+            size = f * size + 0.25 * k_size[t][:, :, None] * v[t].abs()[:, None, :]
+            o, o_size = (S * q[t][:, :, None]).sum(1), (size * q_size[t][:, :, None]).sum(1)
+            rms = torch.sqrt((o ** 2).mean(-1) + 1e-6)[:, None]
+            factor = w * gate[t] * torch.sigmoid(gate[t]) / rms
+            want = o * factor
+            # a token's products, turns and activations are a dozen roundings each, o a float32 sum of dim terms, and the
+            # root mean square carries the error of its columns (o_size.max() over |o|, in parts of rms)
+            bound = (dim + 40) * 2.0 ** -24 * (o_size + o_size.max() * o.abs() / rms) * factor.abs()
+            if dtype == torch.bfloat16:
+                bound = bound + 2.0 ** -8 * want.abs()
+            for result in (out, general):
+                assert torch.all((result[t].cpu().double().view(heads, vdim) - want).abs() <= bound + 1e-6)
+        for memory in (state, off_line):
+            assert torch.all((memory[slots[i]].cpu().double() - S).abs() <= 40 * 2.0 ** -24 * (size + 1))
