@@ -5,93 +5,25 @@
 // part times the key expansion (C) | zeros], so that the kernels see one key head and as many query heads as the
 // layer has, and a head's weighted sum of cache entries holds, in its latent part, what the value expansion reads.
 //
-// This kernel lays the rows out for the rotation-and-cache-write kernel that follows it:
+// This kernel lays the queries out, turns them and the shared key part by the token's position, and writes the token's
+// entry into the cache:
 //
 //   proj  [tokens, ldp]: heads x [plain (P) | turned (R)] queries, then [latent (C) | turned key part (R)]
-//   rows  [tokens, (heads + 2) * D]:
-//     query head h : [0, R) = its turned part as projected (the next kernel turns it)   [R + C, D) = 0
-//                    ([R, R + C) is filled by the block-diagonal product with the key expansion)
-//     key          : [0, R) = the shared key part as projected   [R, R + C) = latent / rms(latent) * weight   rest 0
-//     value        : [0, R) = 0                                  [R, R + C) = the same normed latent         rest 0
+//   rows  [tokens, heads * D]: query head h at h * D: [0, R) = its turned part, turned   [R + C, D) = 0
+//         ([R, R + C) is filled by the block-diagonal product with the key expansion)
+//   key pool   [pages, page_size, D]: [0, R) = the shared key part, turned   [R, R + C) = latent / rms(latent) * weight   rest 0
+//   value pool [pages, D, page_size]: [0, R) = 0                             [R, R + C) = the same normed latent          rest 0
 //
-// The latent's mean square, the division and the weight are float32; one rounding to the activation type.
+// The latent's mean square, the division and the weight are float32, the angles and the products with them too; one
+// rounding to the activation type.
+//
+// A step of few tokens waits here for launches and for dependent loads (position, then angles; sequence, slot, page, then
+// the entry's place), not for bytes.  So the rotation and the write, which were a launch of their own behind the
+// block-diagonal product, take place here, and the queries have workgroups of their own (blockIdx.y > 0) beside the one
+// that norms the latent: 16 heads of 128 + 32, a latent of 96, 8 tokens 5.5 -> 2.8 us, 512 tokens 6.5 -> 3.4, 2,000 9.9 ->
+// 6.8.
 #include "common.h"
 
-template <typename T, typename W>
-__global__ void __launch_bounds__(256)
-latent_rows_kernel(const T* __restrict__ proj, long ldp, const W* __restrict__ weight, T* __restrict__ rows,
-                   int heads, int plain, int turned, int latent, int width, float eps) {
-    __shared__ float scratch[16];
-    const int token = blockIdx.x;
-    const T* src = proj + static_cast<size_t>(token) * ldp;
-    T* dst = rows + static_cast<size_t>(token) * (heads + 2) * width;
-    const T* down = src + static_cast<size_t>(heads) * (plain + turned);
-    float sum_sq = 0.f;
-    for (int i = threadIdx.x; i < latent; i += blockDim.x) {
-        const float c = to_float(down[i]);
-        sum_sq += c * c;
-    }
-    const float inv = 1.0f / sqrtf(block_sum(sum_sq, scratch) / static_cast<float>(latent) + eps);
-    T* key = dst + static_cast<size_t>(heads) * width;
-    T* value = key + width;
-    const T zero = from_float<T>(0.f);
-    for (int i = threadIdx.x; i < width; i += blockDim.x) {
-        T k = zero, v = zero;
-        if (i < turned) {
-            k = down[latent + i];
-        } else if (i < turned + latent) {
-            const int c = i - turned;
-            k = v = from_float<T>((to_float(down[c]) * inv) * to_float(weight[c]));
-        }
-        key[i] = k;
-        value[i] = v;
-    }
-    const int tail = width - turned - latent;
-    for (int i = threadIdx.x; i < heads * (turned + tail); i += blockDim.x) {
-        const int head = i / (turned + tail);
-        const int j = i - head * (turned + tail);
-        T* q = dst + static_cast<size_t>(head) * width;
-        if (j < turned)
-            q[j] = src[static_cast<size_t>(head) * (plain + turned) + plain + j];
-        else
-            q[turned + latent + (j - turned)] = zero;
-    }
-}
-
-CIE_API int cie_latent_rows(void* stream, int dtype, int wdtype, const void* proj, long ldp, const void* weight,
-                            void* rows, int tokens, int heads, int plain, int turned, int latent, int width, float eps) {
-    if (tokens < 0 || heads <= 0 || plain <= 0 || turned < 0 || latent <= 0 || width < turned + latent || !(eps > 0.f) ||
-        ldp < static_cast<long>(heads) * (plain + turned) + latent + turned)
-        return CIE_BAD_ARGUMENT;
-    if (tokens == 0) return CIE_OK;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == CIE_F32 && wdtype == CIE_F32)
-        latent_rows_kernel<float, float><<<tokens, 256, 0, s>>>(
-            static_cast<const float*>(proj), ldp, static_cast<const float*>(weight), static_cast<float*>(rows), heads, plain,
-            turned, latent, width, eps);
-    else if (dtype == CIE_BF16 && wdtype == CIE_BF16)
-        latent_rows_kernel<bf16_t, bf16_t><<<tokens, 256, 0, s>>>(
-            static_cast<const bf16_t*>(proj), ldp, static_cast<const bf16_t*>(weight), static_cast<bf16_t*>(rows), heads,
-            plain, turned, latent, width, eps);
-    else if (dtype == CIE_BF16 && wdtype == CIE_F32)
-        latent_rows_kernel<bf16_t, float><<<tokens, 256, 0, s>>>(
-            static_cast<const bf16_t*>(proj), ldp, static_cast<const float*>(weight), static_cast<bf16_t*>(rows), heads,
-            plain, turned, latent, width, eps);
-    else
-        return CIE_BAD_ARGUMENT;
-    return cie_after_launch();
-}
-
-// ---------------------------------------------------------------------------------------------- with a query latent
-// The same layer in a form whose cache keeps an entry [turned part (R) | normed latent (C) | zeros], D numbers wide, and
-// as its value the normed latent alone (DV numbers wide), and whose queries may come from a latent of their own.
-//
-// `latent_down_kernel`, one workgroup per token, stands behind the down projections: it norms the query latent
-// (RMS, weight) into `q_latent`, norms the key latent (RMS, weight), turns the first `rot` numbers of the shared key part
-// by the token's position, and writes both into the token's place in the cache.  `latent_queries_kernel` stands behind
-// the queries' projection [heads x (plain (P) | turned (R))]: it turns each head's turned part and lays it out, with the
-// zeros behind the latent's room, in rows [tokens, heads * D]; the room itself is filled by the block-diagonal product
-// with the key expansion.  Norms, angles and products with them are float32; one rounding to the activation type.
 struct Turn {
     const float* cos_table;  // [positions, rot / 2]
     const float* sin_table;
@@ -114,6 +46,102 @@ __device__ __forceinline__ float turned_number(const T* p, int d, int pos, const
     return is_u ? x * c - y * s : x * c + y * s;
 }
 
+struct EntryPlace {
+    const int* positions;
+    const int* seq_of_token;
+    const int* seq_slot;
+    const int* block_table;
+    int table_width;
+    int page_size;
+    int write_kv;
+};
+
+template <typename T, typename W>
+__global__ void __launch_bounds__(256)
+latent_rows_kernel(const T* __restrict__ proj, long ldp, const W* __restrict__ weight, T* __restrict__ rows,
+                   T* __restrict__ k_pool, T* __restrict__ v_pool, Turn turn, EntryPlace place, int heads, int plain,
+                   int turned, int latent, int width, float eps) {
+    __shared__ float scratch[16];
+    const int token = blockIdx.x;
+    const int pos = place.positions[token];
+    const T* src = proj + static_cast<size_t>(token) * ldp;
+    if (blockIdx.y > 0) {
+        T* dst = rows + static_cast<size_t>(token) * heads * width;
+        const int given = width - latent;  // numbers of a head that are written here
+        for (int i = (blockIdx.y - 1) * blockDim.x + threadIdx.x; i < heads * given; i += blockDim.x * (gridDim.y - 1)) {
+            const int head = i / given;
+            const int j = i - head * given;
+            T* q = dst + static_cast<size_t>(head) * width;
+            if (j < turned)
+                q[j] = from_float<T>(turned_number(src + static_cast<size_t>(head) * (plain + turned) + plain, j, pos, turn));
+            else
+                q[latent + j] = from_float<T>(0.f);
+        }
+        return;
+    }
+    if (!place.write_kv) return;
+    const int slot = place.seq_slot[place.seq_of_token[token]];
+    const int page = place.block_table[static_cast<size_t>(slot) * place.table_width + pos / place.page_size];
+    const T* down = src + static_cast<size_t>(heads) * (plain + turned);
+    float sum_sq = 0.f;
+    for (int i = threadIdx.x; i < latent; i += blockDim.x) {
+        const float c = to_float(down[i]);
+        sum_sq += c * c;
+    }
+    const float inv = 1.0f / sqrtf(block_sum(sum_sq, scratch) / static_cast<float>(latent) + eps);
+    if (page < 0) return;  // the host never schedules a token without a page
+    const size_t base = static_cast<size_t>(page) * place.page_size * width;
+    T* key = k_pool + base + static_cast<size_t>(pos % place.page_size) * width;
+    T* value = v_pool + base + pos % place.page_size;
+    for (int i = threadIdx.x; i < width; i += blockDim.x) {
+        float k = 0.f, v = 0.f;
+        if (i < turned)
+            k = turned_number(down + latent, i, pos, turn);
+        else if (i < turned + latent)
+            k = v = (to_float(down[i - turned]) * inv) * to_float(weight[i - turned]);
+        key[i] = from_float<T>(k);
+        value[static_cast<size_t>(i) * place.page_size] = from_float<T>(v);
+    }
+}
+
+CIE_API int cie_latent_rows(void* stream, int dtype, int wdtype, const void* proj, long ldp, const void* weight, void* rows,
+                            const float* cos_table, const float* sin_table, int rot, const int* positions,
+                            const int* seq_of_token, const int* seq_slot, const int* block_table, int table_width,
+                            void* k_pool, void* v_pool, int page_size, int write_kv, int tokens, int heads, int plain,
+                            int turned, int latent, int width, float eps) {
+    if (tokens < 0 || heads <= 0 || plain <= 0 || turned < 0 || latent <= 0 || width < turned + latent || !(eps > 0.f) ||
+        ldp < static_cast<long>(heads) * (plain + turned) + latent + turned || rot < 0 || rot % 2 || rot > turned ||
+        (rot > 0 && (!cos_table || !sin_table)) || page_size <= 0 || table_width <= 0)
+        return CIE_BAD_ARGUMENT;
+    if (tokens == 0) return CIE_OK;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const Turn turn{cos_table, sin_table, rot, 0};
+    const EntryPlace place{positions, seq_of_token, seq_slot, block_table, table_width, page_size, write_kv};
+    const int query_blocks = (heads * (width - latent) + 255) / 256;
+    const int most = tokens >= 256 ? 1 : 8;  // (many tokens fill the units by themselves)
+    const dim3 grid(tokens, 1 + (query_blocks < 1 ? 1 : query_blocks < most ? query_blocks : most));
+#define CIE_LATENT_ROWS(T, W)                                                                                              \
+    latent_rows_kernel<T, W><<<grid, 256, 0, s>>>(static_cast<const T*>(proj), ldp, static_cast<const W*>(weight),         \
+                                                  static_cast<T*>(rows), static_cast<T*>(k_pool), static_cast<T*>(v_pool), \
+                                                  turn, place, heads, plain, turned, latent, width, eps)
+    if (dtype == CIE_F32 && wdtype == CIE_F32) CIE_LATENT_ROWS(float, float);
+    else if (dtype == CIE_BF16 && wdtype == CIE_BF16) CIE_LATENT_ROWS(bf16_t, bf16_t);
+    else if (dtype == CIE_BF16 && wdtype == CIE_F32) CIE_LATENT_ROWS(bf16_t, float);
+    else return CIE_BAD_ARGUMENT;
+#undef CIE_LATENT_ROWS
+    return cie_after_launch();
+}
+
+// ---------------------------------------------------------------------------------------------- with a query latent
+// The same layer in a form whose cache keeps an entry [turned part (R) | normed latent (C) | zeros], D numbers wide, and
+// as its value the normed latent alone (DV numbers wide), and whose queries may come from a latent of their own.
+//
+// `latent_down_kernel`, one workgroup per token, stands behind the down projections: it norms the query latent
+// (RMS, weight) into `q_latent`, norms the key latent (RMS, weight), turns the first `rot` numbers of the shared key part
+// by the token's position, and writes both into the token's place in the cache.  `latent_queries_kernel` stands behind
+// the queries' projection [heads x (plain (P) | turned (R))]: it turns each head's turned part and lays it out, with the
+// zeros behind the latent's room, in rows [tokens, heads * D]; the room itself is filled by the block-diagonal product
+// with the key expansion.  Norms, angles and products with them are float32; one rounding to the activation type.
 template <typename T>
 __global__ void __launch_bounds__(256)
 latent_down_kernel(const T* __restrict__ proj, long ldp, int q_off, int q_rank, int c_off, const float* __restrict__ q_weight,

@@ -1326,11 +1326,15 @@ def block_linear(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
 
 
 def latent_rows(proj: torch.Tensor, weight: torch.Tensor, heads: int, plain: int, turned: int, latent: int,
-                width: int, eps: float) -> torch.Tensor:
-    """Lay out the rows ``[T, (heads + 2) * width]`` that the rotation-and-cache-write kernel and the attention
-    kernels read for a layer whose keys are compressed (``csrc/latent.hip``): per query head its turned part,
-    room for its folded plain part and zeros; one key ``[turned part | normed latent | zeros]`` and one value
-    ``[zeros | normed latent | zeros]``.  ``proj`` [T, heads * (plain + turned) + latent + turned]."""
+                width: int, eps: float, rotary: Optional[tuple[torch.Tensor, torch.Tensor]], positions: torch.Tensor,
+                seq_of_token: torch.Tensor, seq_slot: torch.Tensor, block_table: torch.Tensor, k_pool: torch.Tensor,
+                v_pool: torch.Tensor, write_kv: bool = True) -> torch.Tensor:
+    """What lies between the joint projection and the attention kernels of a layer whose keys are compressed
+    (``csrc/latent.hip``).  ``proj`` [T, heads * (plain + turned) + latent + turned].  Returns the query rows
+    ``[T, heads * width]``: per head its turned part, turned by the token's position, room for its folded plain part,
+    and zeros.  Writes every token's cache entry, key ``[turned part | normed latent | zeros]`` and value
+    ``[zeros | normed latent | zeros]``, where ``write_kv``.  ``rotary``: (cos, sin) float32 [max_position, turned / 2],
+    or ``None`` where nothing turns; pools as for ``rope_kv_write`` with one head of ``width``."""
     if not (proj.is_cuda and proj.dim() == 2 and proj.stride(1) == 1 and proj.dtype in _CODES):
         raise ValueError("proj must be a float32 or bfloat16 GPU matrix with unit inner stride")
     tokens = proj.shape[0]
@@ -1339,11 +1343,31 @@ def latent_rows(proj: torch.Tensor, weight: torch.Tensor, heads: int, plain: int
     _gpu("weight", weight, dims=1)
     if weight.shape[0] != latent or weight.dtype not in (proj.dtype, torch.float32):
         raise ValueError("the latent's norm weight does not fit")
-    rows = torch.empty((tokens, (heads + 2) * width), dtype=proj.dtype, device=proj.device)
+    cos = sin = None
+    if rotary is not None:
+        cos, sin = rotary
+        if turned <= 0 or turned % 2:
+            raise ValueError(f"the turned part must be even, is {turned}")
+        for name, table in (("cos", cos), ("sin", sin)):
+            _gpu(name, table, torch.float32, 2)
+            if not (table.shape[1] == turned // 2):
+                raise ValueError(f"{name} must be [max_position, {turned // 2}]")
+        if not (cos.shape == sin.shape):
+            raise ValueError("cos and sin tables differ in shape")
+    for name, meta in (("positions", positions), ("seq_of_token", seq_of_token)):
+        _gpu(name, meta, torch.int32, 1)
+        if not (meta.shape[0] >= tokens):
+            raise ValueError(f"{name} has {meta.shape[0]} entries for {tokens} tokens")
+    _gpu("seq_slot", seq_slot, torch.int32, 1)
+    _gpu("block_table", block_table, torch.int32, 2)
+    page_size = _check_pools(k_pool, v_pool, proj.dtype, 1, width)
+    rows = torch.empty((tokens, heads * width), dtype=proj.dtype, device=proj.device)
     ldp = proj.stride(0) if tokens > 1 else max(proj.stride(0), proj.shape[1])
     _run("cie_latent_rows", load_library().cie_latent_rows(
-        _stream(), _i(_code(proj.dtype)), _i(_code(weight.dtype)), _ptr(proj), ldp, _ptr(weight), _ptr(rows), _i(tokens),
-        _i(heads), _i(plain), _i(turned), _i(latent), _i(width), _f(eps)))
+        _stream(), _i(_code(proj.dtype)), _i(_code(weight.dtype)), _ptr(proj), ldp, _ptr(weight), _ptr(rows), _ptr(cos),
+        _ptr(sin), _i(turned if rotary is not None else 0), _ptr(positions), _ptr(seq_of_token), _ptr(seq_slot),
+        _ptr(block_table), _i(block_table.shape[1]), _ptr(k_pool), _ptr(v_pool), _i(page_size), _i(1 if write_kv else 0),
+        _i(tokens), _i(heads), _i(plain), _i(turned), _i(latent), _i(width), _f(eps)))
     return rows
 
 

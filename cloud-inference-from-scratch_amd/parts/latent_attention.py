@@ -93,13 +93,12 @@ class LatentAttention(Part):
             raise ValueError(f"position {batch.max_context - 1} is beyond the rotary table of {self.position.max_position}")
         queries = h * (p + r)
         proj = linear(x, self.w_in)
-        rows = ops.latent_rows(proj[:, : queries + c + r], self.latent_weight, h, p, r, c, width, self.eps)
-        ops.block_linear(proj, self.w_fold, a_block=p + r, out=rows, out_offset=r, c_block=width)
         turns = bool(r) and self.position.rotates
-        cos, sin = self.position.tables(x.device, positions_bound(batch))
-        ops.rope_kv_write(rows, cos, sin, batch.positions, batch.seq_of_token, batch.seq_slot, view.block_table,
-                          view.k_pool, view.v_pool, h, 1, width, rotate=turns, write_kv=writes,
-                          rotary_dim=r if turns else None)
+        rotary = self.position.tables(x.device, positions_bound(batch)) if turns else None
+        rows = ops.latent_rows(proj[:, : queries + c + r], self.latent_weight, h, p, r, c, width, self.eps, rotary,
+                               batch.positions, batch.seq_of_token, batch.seq_slot, view.block_table, view.k_pool,
+                               view.v_pool, write_kv=writes)
+        ops.block_linear(proj, self.w_fold, a_block=p + r, out=rows, out_offset=r, c_block=width)
         context = attend(rows, batch, view, h, 1, width, None, self.scale)
         gated = ops.block_linear(context, self.w_unfold, gate=proj, gate_offset=queries + c + r)
         return linear(gated, self.w_o)

@@ -638,3 +638,67 @@ def test_retention_of_one_token_a_sequence(dtype, lengths, heads, dim, vdim, rot
                 assert torch.all((result[t].cpu().double().view(heads, vdim) - want).abs() <= bound + 1e-6)
         for memory in (state, off_line):
             assert torch.all((memory[slots[i]].cpu().double() - S).abs() <= 40 * 2.0 ** -24 * (size + 1))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens,heads,plain,turned,latent,width,page_size", [
+    (1, 16, 24, 32, 96, 128, 16), (7, 3, 5, 6, 11, 32, 4), (3, 40, 128, 64, 64, 256, 16), (300, 4, 16, 32, 96, 128, 32),
+    (5, 2, 8, 0, 64, 64, 3), (2, 1, 1, 2, 1, 4, 1)])
+@pytest.mark.parametrize("mode", ["turned", "unturned", "reads"])
+def test_rows_and_entries_of_compressed_keys(dtype, tokens, heads, plain, turned, latent, width, page_size, mode):
+    """Query rows and cache entries of one launch: heads that leave lanes over or take several workgroups, entries with and
+    without zeros behind the latent, a part that does not turn or is not there, odd pages, a token without a page, and a
+    layer that only reads; places that are nobody's stay as they are."""
+    from cie_amd.kernels import ops
+
+    if not turned and mode == "turned":
+        mode = "unturned"
+    g = torch.Generator().manual_seed(8)
+    columns = heads * (plain + turned) + latent + turned
+    proj = torch.randn(tokens, columns + 5, generator=g).to(dtype).cuda()[:, :columns]
+    weight = torch.rand(latent, generator=g).cuda() + 0.5
+    at = torch.randint(0, 40, (tokens,), generator=g)
+    pages_each = -(-40 // page_size)
+    table = torch.randperm(tokens * pages_each, generator=g).view(tokens, pages_each).int()
+    lost = tokens - 1 if tokens > 2 else -1
+    if lost >= 0:
+        table[0, at[lost] // page_size] = -1  # (the last token's sequence has slot 0)
+    slots = torch.arange(tokens).flip(0)
+    angles = torch.arange(40)[:, None] * 0.7 ** torch.arange(turned // 2)[None, :]
+    cos, sin = angles.cos().float(), angles.sin().float()
+    keys = torch.full((tokens * pages_each, 1, page_size, width), 3.0, dtype=dtype, device="cuda")
+    values = torch.full((tokens * pages_each, 1, width, page_size), 3.0, dtype=dtype, device="cuda")
+    rows = ops.latent_rows(proj, weight, heads, plain, turned, latent, width, 1e-6,
+                           (cos.cuda(), sin.cuda()) if mode == "turned" else None, at.int().cuda(),
+                           torch.arange(tokens).int().cuda(), slots.int().cuda(), table.cuda(), keys, values,
+                           write_kv=mode != "reads")
+    p, c, s = proj.cpu().double(), cos.double()[at], sin.double()[at]
+    half = turned // 2
+
+    def turn(z):  # [tokens, ..., turned] -> turned, and what its roundings are relative to
+        if mode != "turned":
+            return z, z.abs()
+        shape = (tokens,) + (1,) * (z.dim() - 2) + (half,)
+        a, b, cc, ss = z[..., :half], z[..., half:], c.view(shape), s.view(shape)
+        return torch.cat((a * cc - b * ss, b * cc + a * ss), -1), torch.cat((a.abs() + b.abs(),) * 2, -1)
+
+    one = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24  # the last rounding; four more of float32 in front of it
+    close = lambda got, want, size: bool(((got.cpu().double() - want).abs() <= one * want.abs() + 4 * 2.0 ** -24 * size).all())
+    q = rows.view(tokens, heads, width)
+    want, size = turn(p[:, : heads * (plain + turned)].view(tokens, heads, plain + turned)[..., plain:])
+    assert close(q[..., :turned], want, size) and not q[..., turned + latent:].any()
+    down = p[:, heads * (plain + turned):]
+    normed = down[:, :latent] / torch.sqrt((down[:, :latent] ** 2).mean(-1, keepdim=True) + 1e-6) * weight.cpu().double()
+    key, key_size = turn(down[:, latent:])
+    untouched = torch.ones(keys.shape[0], page_size, dtype=torch.bool)
+    for t in range(tokens):
+        page, row = int(table[slots[t], at[t] // page_size]), int(at[t] % page_size)
+        if mode == "reads" or page < 0:
+            continue
+        untouched[page, row] = False
+        k, v = keys[page, 0, row], values[page, 0, :, row]
+        assert close(k[:turned], key[t], key_size[t]) and not v[:turned].any()
+        for entry in (k, v):  # (the mean square: `latent` squares and their sum, a root, a quotient, two products)
+            assert close(entry[turned: turned + latent], normed[t], (latent + 4) * normed[t].abs())
+            assert not entry[turned + latent:].any()
+    assert (keys.cpu()[:, 0][untouched] == 3).all() and (values.cpu()[:, 0].transpose(1, 2)[untouched] == 3).all()
