@@ -961,6 +961,108 @@ gated_recurrence_kernel(const T* __restrict__ y_pre, long ldy, const T* __restri
         keep_inputs(past + static_cast<size_t>(slot) * (taps - 1) * channels, x_in, ldx, first, count, c, channels, taps - 1);
 }
 
+// A step in which no sequence brings more than one token, in bfloat16: the gates' block-diagonal product and the walk's one
+// step at once.  A workgroup owns 16 channels of 16 sequences.  Its four waves take every fourth slice of 32 k of both gates
+// (v_mfma_f32_16x16x32_bf16), the sums meet in LDS in the waves' order, and every thread then moves the state of one channel
+// and sequence: the float32 gates never go through memory and a launch falls away.  What bounds it are chains, not bytes (a
+// layer's gates are 2 MB): a wave's slices and what the step itself needs are all asked for before the first product,
+// and a lane of one wave that moved the four states whose gates it held spent 0.65 us on each, one after the other.
+// In place of the product and the walk, 8 blocks of 256: one sequence 6.6 -> 4.2 us, eight 7.2 -> 4.3, 64 11.4 -> 6.5.  From
+// some eight workgroups a unit on every 16 sequences' new reading of the weights costs more than the launch (16 blocks, 128
+// sequences 15.8 -> 16.7; at five a unit 13.5 -> 12.4): kernels/ops.py draws the line between.
+typedef __bf16 gate_piece_t __attribute__((ext_vector_type(8)));
+constexpr int kGateSlices = 4;  // of 32 k under way at once, a wave
+constexpr int kStepTaps = 4;    // inputs kept beside the token's own, at most (longer convolutions take the general path)
+
+__global__ void __launch_bounds__(256)
+gated_recurrence_step_kernel(const bf16_t* __restrict__ y_pre, long ldy, const bf16_t* __restrict__ x_in, long ldx,
+                             const bf16_t* __restrict__ u, const bf16_t* __restrict__ weight, const bf16_t* __restrict__ bias,
+                             int block_width, int tiles, const float* __restrict__ rate, float* __restrict__ state,
+                             float* __restrict__ past, const int* __restrict__ seq_slot, const int* __restrict__ q_start_loc,
+                             bf16_t* __restrict__ out, int sequences, int tokens, int channels, int keep_n) {
+    __shared__ float sums[4][2][16][17];  // [wave][gate][sequence][channel]
+    const int lane = threadIdx.x % kWave;
+    const int wave = threadIdx.x / kWave;
+    const int r = lane & 15;
+    const int g = lane >> 4;
+    const int groups = gridDim.x;  // (neighbouring channels on one XCD, whose L2 then holds a line's both halves and a block's rows)
+    const int group = groups % 8 == 0 ? (blockIdx.x % 8) * (groups / 8) + blockIdx.x / 8 : blockIdx.x;
+    const int block = group / tiles;
+    const int n0 = (group - block * tiles) * 16;
+    const int seq0 = blockIdx.y * 16;
+    // (a channel past the block's last reads the last, a sequence past the last too; a place without a token reads some token
+    // and stores nothing)
+    const int n = min(n0 + r, block_width - 1);
+    const bf16_t* a_row = u + static_cast<size_t>(min(q_start_loc[min(seq0 + r, sequences - 1)], tokens - 1)) * channels +
+                          static_cast<size_t>(block) * block_width;
+    const bf16_t* r_row = weight + (static_cast<size_t>(block) * 2 * block_width + n) * block_width;
+    const bf16_t* i_row = r_row + static_cast<size_t>(block_width) * block_width;
+    words_t av[kGateSlices], rv[kGateSlices], iv[kGateSlices];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int s = 0; s < kGateSlices; ++s) {
+            const int at = min(k0 + 32 * (4 * s + wave) + g * 8, block_width - 8);
+            rv[s] = *reinterpret_cast<const words_t*>(r_row + at);
+            iv[s] = *reinterpret_cast<const words_t*>(i_row + at);
+            av[s] = *reinterpret_cast<const words_t*>(a_row + at);
+        }
+    };
+    fetch(0);
+    // the step's own: one channel of one sequence a thread
+    const int mine = threadIdx.x / 16;
+    const int col = threadIdx.x % 16;
+    const int seq = min(seq0 + mine, sequences - 1);
+    const int inside = min(n0 + col, block_width - 1);
+    const int c = block * block_width + inside;
+    const int start = q_start_loc[seq];
+    const bool steps = n0 + col < block_width && seq0 + mine < sequences && q_start_loc[seq + 1] > start;
+    const size_t token = static_cast<size_t>(min(start, tokens - 1));
+    const size_t slot = static_cast<size_t>(seq_slot[seq]);
+    const bf16_t* b_row = bias + static_cast<size_t>(block) * 2 * block_width + inside;
+    const bf16_t r_bias = b_row[0], i_bias = b_row[block_width];
+    const float coef = rate[c];
+    const float S = state[slot * channels + c];
+    const bf16_t y_in = y_pre[token * ldy + c], u_in = u[token * channels + c], x_new = x_in[token * ldx + c];
+    float* before = past + slot * max(keep_n, 1) * channels + c;
+    float old[kStepTaps];
+#pragma unroll
+    for (int j = 0; j < kStepTaps; ++j) old[j] = before[static_cast<size_t>(min(j, max(keep_n - 1, 0))) * channels];
+    __builtin_amdgcn_sched_barrier(0);
+    acc4_t r_sum = {0.f, 0.f, 0.f, 0.f}, i_sum = {0.f, 0.f, 0.f, 0.f};
+    const words_t nothing = {0u, 0u, 0u, 0u};
+    for (int k0 = 0; k0 < block_width; k0 += 4 * 32 * kGateSlices) {
+        if (k0 > 0) fetch(k0);
+#pragma unroll
+        for (int s = 0; s < kGateSlices; ++s) {
+            // (a group of 8 past the end read the last group again and counts as zeros, on both sides)
+            const bool there = k0 + 32 * (4 * s + wave) + g * 8 < block_width;
+            const gate_piece_t a = __builtin_bit_cast(gate_piece_t, there ? av[s] : nothing);
+            r_sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(gate_piece_t, there ? rv[s] : nothing), r_sum, 0, 0, 0);
+            i_sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(gate_piece_t, there ? iv[s] : nothing), i_sum, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        sums[wave][0][g * 4 + i][r] = r_sum[i];
+        sums[wave][1][g * 4 + i][r] = i_sum[i];
+    }
+    __syncthreads();
+    if (!steps) return;
+    float r_pre = sums[0][0][mine][col], i_pre = sums[0][1][mine][col];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+        r_pre += sums[w][0][mine][col];
+        i_pre += sums[w][1][mine][col];
+    }
+    const GateStep now = gate_step(r_pre + to_float(r_bias), i_pre + to_float(i_bias), to_float(u_in), coef);
+    const float next = fmaf(now.a, S, now.x);
+    out[token * channels + c] = from_float<bf16_t>(next * gelu_tanh(to_float(y_in)));
+    state[slot * channels + c] = next;
+#pragma unroll
+    for (int j = 0; j < kStepTaps; ++j)
+        if (j < keep_n) before[static_cast<size_t>(j) * channels] = j + 1 < keep_n ? old[j + 1 < kStepTaps ? j + 1 : j] : to_float(x_new);
+}
+
 // Long portions.  S_t = a_t S_(t-1) + x_t is linear in S, so `segments` stretches of up to 32 tokens run side by side:
 // thread (channel, stretch) folds its stretch into (A, B) with S_out = A S_in + B, the stretches before it give its
 // S_in (a chain of at most `segments` multiply-adds), and a second walk makes the outputs.  A portion of more than
@@ -1307,5 +1409,23 @@ CIE_API int cie_gated_recurrence(void* stream, int dtype, const void* y_pre, lon
 #undef CIE_SCAN
     else
         return CIE_BAD_ARGUMENT;
+    return cie_after_launch();
+}
+
+CIE_API int cie_gated_recurrence_step(void* stream, const void* y_pre, long ldy, const void* x_in, long ldx, const void* u,
+                                      const void* weight, const void* bias, int block_width, const float* rate, float* state,
+                                      float* past, const int* seq_slot, const int* q_start_loc, void* out, int sequences,
+                                      int tokens, int channels, int taps) {
+    if (sequences < 0 || tokens < 0 || channels <= 0 || block_width <= 0 || block_width % 8 || channels % block_width ||
+        taps < 1 || taps > kStepTaps + 1 || ldy < channels || ldx < channels || sequences > 16 * 65535 ||
+        reinterpret_cast<size_t>(u) % 16 || reinterpret_cast<size_t>(weight) % 16)
+        return CIE_BAD_ARGUMENT;
+    if (sequences == 0 || tokens == 0) return CIE_OK;
+    const int tiles = (block_width + 15) / 16;
+    gated_recurrence_step_kernel<<<dim3(channels / block_width * tiles, (sequences + 15) / 16), 256, 0,
+                                   static_cast<hipStream_t>(stream)>>>(
+        static_cast<const bf16_t*>(y_pre), ldy, static_cast<const bf16_t*>(x_in), ldx, static_cast<const bf16_t*>(u),
+        static_cast<const bf16_t*>(weight), static_cast<const bf16_t*>(bias), block_width, tiles, rate, state, past, seq_slot,
+        q_start_loc, static_cast<bf16_t*>(out), sequences, tokens, channels, taps - 1);
     return cie_after_launch();
 }

@@ -1669,6 +1669,52 @@ def gated_recurrence(y_pre: torch.Tensor, x_in: torch.Tensor, u: torch.Tensor, g
     return out
 
 
+SCAN_STEP_TAPS = 5         # of a convolution in front of the kernel of single tokens, at most
+SCAN_STEP_WORKGROUPS = 5   # ... and workgroups of 16 channels and 16 sequences a compute unit (csrc/recurrent.hip)
+
+
+def steps_gated_recurrence(u: torch.Tensor, weight: torch.Tensor, sequences: int, block_width: int, taps: int) -> bool:
+    """Whether the kernel that makes the gates and moves the states of single tokens is the faster one for these and takes
+    them: bfloat16, blocks in 16-byte pieces."""
+    groups = u.shape[1] // block_width * -(-block_width // 16) * -(-sequences // 16)
+    return (u.dtype == torch.bfloat16 and weight.dtype == u.dtype and block_width % 8 == 0 and taps <= SCAN_STEP_TAPS
+            and groups <= SCAN_STEP_WORKGROUPS * compute_units() and u.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+def gated_recurrence_step(y_pre: torch.Tensor, x_in: torch.Tensor, u: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,
+                          rate: torch.Tensor, state: torch.Tensor, past: torch.Tensor, seq_slot: torch.Tensor,
+                          q_start_loc: torch.Tensor, sequences: int, taps: int) -> torch.Tensor:
+    """``gated_recurrence`` with its gates' product ``block_linear(u, weight, bias)`` (``weight``
+    [blocks, 2 * block_width, block_width]) in one kernel, for a step in which no sequence brings more than one token
+    (the caller's to know: of a sequence with more, only the first would be walked)."""
+    tokens, channels = u.shape
+    for name, t in (("y_pre", y_pre), ("x_in", x_in)):
+        if not (t.is_cuda and t.dim() == 2 and t.stride(1) == 1 and t.dtype == u.dtype and tuple(t.shape) == (tokens, channels)):
+            raise ValueError(f"{name} must be a [{tokens}, {channels}] view of u's type with unit inner stride")
+    _gpu("u", u, torch.bfloat16, 2)
+    _gpu("weight", weight, torch.bfloat16, 3)
+    _gpu("bias", bias, torch.bfloat16, 2)
+    _gpu("rate", rate, torch.float32, 1)
+    _gpu("state", state, torch.float32, 2)
+    _gpu("past", past, torch.float32, 3)
+    blocks, twice, width = weight.shape
+    if (twice != 2 * width or blocks * width != channels or tuple(bias.shape) != (blocks, twice) or rate.shape[0] != channels
+            or state.shape[1] != channels or tuple(past.shape[1:]) != (max(taps - 1, 1), channels)
+            or past.shape[0] != state.shape[0] or not 1 <= taps <= SCAN_STEP_TAPS or width % 8):
+        raise ValueError("weight, bias, rate, state or past do not fit the channels")
+    for name, meta, least in (("seq_slot", seq_slot, sequences), ("q_start_loc", q_start_loc, sequences + 1)):
+        _gpu(name, meta, torch.int32, 1)
+        if meta.shape[0] < least:
+            raise ValueError(f"{name} has {meta.shape[0]} entries for {sequences} sequences")
+    out = torch.empty((tokens, channels), dtype=u.dtype, device=u.device)
+    ld = lambda t: t.stride(0) if tokens > 1 else max(t.stride(0), channels)
+    _run("cie_gated_recurrence_step", load_library().cie_gated_recurrence_step(
+        _stream(), _ptr(y_pre), ld(y_pre), _ptr(x_in), ld(x_in), _ptr(u), _ptr(weight), _ptr(bias), _i(width), _ptr(rate),
+        _ptr(state), _ptr(past), _ptr(seq_slot), _ptr(q_start_loc), _ptr(out), _i(sequences), _i(tokens), _i(channels),
+        _i(taps)))
+    return out
+
+
 # ---------------------------------------------------------------------------
 WALK_ROWS = (4, 8, 16, 32, 64)   # rows of a memory that one thread of the walk keeps in registers
 WALK_MAX_ROWS = 1024

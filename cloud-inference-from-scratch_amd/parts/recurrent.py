@@ -237,6 +237,12 @@ class GatedLinearRecurrence(Part):
         proj = linear(x, self.w_in, self.b_in)
         y_pre, x_in = proj[:, :w], proj[:, w:]
         u = ops.causal_conv(x_in, self.conv_w, self.conv_b, past, batch.seq_of_token, batch.seq_slot, batch.q_start_loc)
+        if (batch.max_q_len == 1
+                and ops.steps_gated_recurrence(u, self.w_gates, batch.sequences, w // self.blocks, self.taps)):
+            # (no sequence brings more than one token: the gates and the step at once)
+            out = ops.gated_recurrence_step(y_pre, x_in, u, self.w_gates, self.b_gates, self.rate, state, past, batch.seq_slot,
+                                            batch.q_start_loc, batch.sequences, self.taps)
+            return linear(out, self.w_o)
         gates = ops.block_linear(u, self.w_gates, self.b_gates, out_dtype=torch.float32)
         # long portions run as stretches side by side (the portion lengths are the host's, and a captured step's own)
         segments = scan_segments(batch.max_q_len)

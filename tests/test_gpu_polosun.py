@@ -702,3 +702,40 @@ def test_rows_and_entries_of_compressed_keys(dtype, tokens, heads, plain, turned
             assert close(entry[turned: turned + latent], normed[t], (latent + 4) * normed[t].abs())
             assert not entry[turned + latent:].any()
     assert (keys.cpu()[:, 0][untouched] == 3).all() and (values.cpu()[:, 0].transpose(1, 2)[untouched] == 3).all()
+
+
+@pytest.mark.parametrize("lengths,blocks,width,taps", [
+    ((1,), 1, 8, 1), ((1,) * 5, 3, 24, 2), ((1,) * 16, 8, 256, 4), ((1,) * 17, 2, 264, 5), ((1, 0, 1, 0, 0), 2, 40, 4),
+    ((1,) * 64, 4, 128, 4), ((1, 1), 1, 520, 3)])
+def test_gated_recurrence_of_single_tokens(lengths, blocks, width, taps):
+    """The kernel that makes the gates and moves the states, at blocks that end inside a tile of 16 channels, inside a slice
+    of 32 and behind eight slices, rows that end inside a tile of 16 sequences, and places without a token, against the
+    product and the walk by themselves."""
+    from cie_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(9)
+    tokens, channels = sum(lengths), blocks * width
+    slots = list(range(len(lengths) + 2))[::-1][: len(lengths)]
+    make = lambda *shape: torch.randn(*shape, generator=g)
+    proj = make(tokens, 2 * channels + 1).bfloat16().cuda()  # (rows off 16-byte lines)
+    y_pre, x_in = proj[:, 1: channels + 1], proj[:, channels + 1:]
+    u = make(tokens, channels).bfloat16().cuda()
+    weight, bias = (make(blocks, 2 * width, width) * width ** -0.5).bfloat16().cuda(), make(blocks, 2 * width).bfloat16().cuda()
+    rate = -8.0 * torch.rand(channels, generator=g).cuda()
+    state, past = make(len(lengths) + 2, channels).cuda(), make(len(lengths) + 2, max(taps - 1, 1), channels).cuda()
+    state2, past2 = state.clone(), past.clone()
+    starts = [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    meta = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+    takes, n = ops.steps_gated_recurrence, len(lengths)
+    assert takes(u, weight, n, width, taps) and not takes(u.float(), weight, n, width, taps)
+    assert not takes(u, weight, n, width + 4, taps) and not takes(u, weight, n, width, 6)
+    assert not takes(u, weight, 16 * 5 * 256 + 1, width, taps)
+    out = ops.gated_recurrence_step(y_pre, x_in, u, weight, bias, rate, state, past, meta(slots), meta(starts), len(lengths), taps)
+    gates = ops.block_linear(u, weight, bias, out_dtype=torch.float32)
+    want = ops.gated_recurrence(y_pre, x_in, u, gates, width, rate, state2, past2, meta(slots), meta(starts), len(lengths), taps)
+    # float32 sums of `width` terms of some 1 / sqrt(width) in another order, through slopes of at most 2 (the
+    # decay's, |rate| / 4) and the state's size of some 4; the bfloat16 result is rounded once, either way
+    near = width * 2.0 ** -24 * 8 + 1e-6
+    assert torch.allclose(state, state2, atol=near, rtol=near)
+    assert torch.allclose(out.float(), want.float(), atol=4 * near, rtol=2.0 ** -7)
+    assert torch.equal(past, past2)
