@@ -84,13 +84,14 @@ __device__ __forceinline__ floatx4 inside(floatx4 v, int k, int K) {
 
 __device__ __forceinline__ float gated(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
 
-// What the rows kernel does beside the product: nothing; the norm of its rows; that, the rotation and the cache write.
-enum { kPlain = 0, kNormed = 1, kRotated = 2 };
+// What the rows kernel does beside the product: nothing; the norm of its rows; that, the rotation and the cache write; the add
+// into C.
+enum { kPlain = 0, kNormed = 1, kRotated = 2, kAdded = 3 };
+constexpr bool norms_rows(int beside) { return beside == kNormed || beside == kRotated; }
 
 struct RowsBeside {
     const float* norm_weight;  // kNormed, kRotated: A is the stream, its rows' norm is multiplied
     float eps;
-    int into;                  // kPlain: C is added to, not written
     // kRotated: W stacks the rows of q, k and v heads; queries go to C, keys and values to the cache
     const float *cos_table, *sin_table;  // [positions, rotary_dim / 2]
     const int *positions, *seq_of_token, *seq_slot, *block_table;
@@ -117,12 +118,16 @@ constexpr int kNormTasks = 32;           // ... and so many segments in all: wha
 
 // kRows rows (8, 16 or 32) by kColumns columns (8, 16 or 32; with the gate kColumns / 2 of each half), in tiles of 16
 // of which the last may be half empty.  kWaves waves share K.  Workgroup x takes the columns' tiles x, x + gridDim.x, ...
-template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec, int kBeside = kPlain>
+// kHalves: 2, or 1 for a K of up to one chain's, which has no second chain (K 64 at 8 rows 4.2 -> 3.4 us).  Both this and kAdded are
+// known when the kernel is compiled: as numbers of the launch they cost every product 0.3 to 2 us (4 rows, 2,048 columns, K
+// 11,008 28.0 -> 25.8; 16 rows, 896 columns, K 4,864 19.4 -> 18.9), the loop over the chains no longer
+// being unrolled and the waits in it being for what the add might have asked for.
+template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec, int kBeside, int kHalves>
 __global__ void __launch_bounds__(kWaves * kWave)
 gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
                      float* __restrict__ C, int M, int N, int K, int lda, int ldc, RowsBeside beside) {
     constexpr int kRowTiles = (kRows + 15) / 16, kColumnTiles = (kColumns + 15) / 16;
-    constexpr bool kOwnRows = kBeside != kPlain;  // the normed rows lie in LDS, whole
+    constexpr bool kOwnRows = norms_rows(kBeside);  // the normed rows lie in LDS, whole
     constexpr int kTiles = kRowTiles + kColumnTiles, kStaged = kOwnRows ? kColumnTiles : kTiles;
     constexpr int kSums = kRowTiles * kColumnTiles * 256;
     constexpr int kAhead = kPiecesPerChain;  // pieces on their way
@@ -130,7 +135,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
     constexpr int kOwned = (kSums + kThreads - 1) / kThreads;
     constexpr int kStep = kGate ? kColumns / 2 : kColumns;  // output columns of a tile
     static_assert(!kGate || kColumns == 32 || kColumns == 16, "a gate's tile holds as many columns of either half");
-    static_assert(kBeside == kPlain || (kVec && kRows <= 16), "a few rows in 16-byte pieces");
+    static_assert(!kOwnRows || (kVec && kRows <= 16), "a few rows in 16-byte pieces");
     static_assert(kBeside != kRotated || (!kGate && kColumns == 16 && kRows * 8 <= kThreads), "8 dimensions and their partners");
     __shared__ float stage_all[kWaves * kStaged * kTileFloats];
     __shared__ float sums[2][kWaves * kSums];
@@ -161,8 +166,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 #pragma unroll
     for (int i = 0; i < kALoads; ++i) a_row[i] = A + static_cast<size_t>(min(m0 + 8 * i + lane / 8, M - 1)) * lda;
 
-    // (a K of up to one chain's has no second chain)
-    const int halves = K <= kBlockK / 2 ? 1 : 2, pieces = halves * kPiecesPerChain;
+    constexpr int pieces = kHalves * kPiecesPerChain;
     // the piece that is fetched next: its place in the block, the round and the tile
     int f_piece = 0, f_round = 0, f_tile = blockIdx.x;
     const float* w_row[kWLoads];
@@ -253,7 +257,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
         auto column_of = [&](int e) { return 16 * (e / 256 / kRowTiles) + 4 * ((e / 4) % kWave / 16) + e % 4; };
         auto row_of = [&](int e) { return 16 * (e / 256 % kRowTiles) + (e / 4) % kWave % 16; };
         float old[kOwned] = {};  // (of a C that is added to: on its way while W streams)
-        if (kBeside == kPlain && !kGate && beside.into)
+        if constexpr (kBeside == kAdded)
 #pragma unroll
             for (int o = 0; o < kOwned; ++o) {
                 const int e = min(static_cast<int>(threadIdx.x) + o * kThreads, kSums - 1);
@@ -271,7 +275,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
         }
         for (int round = 0; round < rounds; ++round) {
             floatx4 block[kColumnTiles][kRowTiles] = {};
-            for (int half = 0; half < halves; ++half) {
+            for (int half = 0; half < kHalves; ++half) {
                 floatx4 acc[kColumnTiles][kRowTiles] = {};
 #pragma unroll
                 for (int s = 0; s < kAhead; ++s) {
@@ -392,7 +396,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
                 const int n = tile * kStep + column_of(e), m = m0 + row_of(e);
                 if (e < kSums && column_of(e) < kColumns && row_of(e) < kRows && m < M && n < N) {
                     const float sum = total[o] + (bias ? bias[n] : 0.f);
-                    C[static_cast<size_t>(m) * ldc + n] = beside.into ? old[o] + sum : sum;
+                    C[static_cast<size_t>(m) * ldc + n] = kBeside == kAdded ? old[o] + sum : sum;
                 }
             }
         }
@@ -757,6 +761,7 @@ bool goes_direct(const Product& p, long workgroups, long per_unit) {
 
 template <int kRows, int kColumns, int kWaves, bool kGate, bool kVec, int kBeside = kPlain>
 void run_rows(hipStream_t s, const Product& p) {
+    static_assert(kBeside != kAdded || !kGate, "a product's own result is added");
     const int step = kGate ? kColumns / 2 : kColumns;
     const int tiles = ((kGate ? p.N / 2 : p.N) + step - 1) / step;
     // as many workgroups as the units hold at a time by their LDS (2 KB a wave for each staged tile and each tile of sums):
@@ -765,9 +770,15 @@ void run_rows(hipStream_t s, const Product& p) {
     // a unit, whose columns never exceed four a unit: all at once (N 14,000, K 2,048 at 4 rows 25.9; by their LDS 27.4)
     constexpr int kRowTiles = (kRows + 15) / 16, kColumnTiles = (kColumns + 15) / 16;
     constexpr int kLds = kWaves * 2048 * (kRowTiles + kColumnTiles + kRowTiles * kColumnTiles);
-    const int most = p.units * (kBeside != kPlain ? 1 : kRows <= 16 && kColumns == 16 ? 32 / kWaves : 160 * 1024 / kLds);
+    const int most = p.units * (norms_rows(kBeside) ? 1 : kRows <= 16 && kColumns == 16 ? 32 / kWaves : 160 * 1024 / kLds);
     dim3 grid(tiles < most ? tiles : most, (p.M + kRows - 1) / kRows);
-    gemm_f32_rows_kernel<kRows, kColumns, kWaves, kGate, kVec, kBeside><<<grid, kWaves * kWave, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, p.beside);
+    if constexpr (kWaves == 4) {  // (a K that short has four waves, but for operands off 16 bytes)
+        if (p.K <= kBlockK / 2) {
+            gemm_f32_rows_kernel<kRows, kColumns, kWaves, kGate, kVec, kBeside, 1><<<grid, kWaves * kWave, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, p.beside);
+            return;
+        }
+    }
+    gemm_f32_rows_kernel<kRows, kColumns, kWaves, kGate, kVec, kBeside, 2><<<grid, kWaves * kWave, 0, s>>>(p.A, p.W, p.bias, p.C, p.M, p.N, p.K, p.lda, p.ldc, p.beside);
 }
 
 template <bool kGate, bool kVec>
@@ -792,32 +803,33 @@ void run_stretches(hipStream_t s, const Product& p, bool gate) {
     else gemm_f32_join_kernel<false><<<join, 256, 0, s>>>(p.parts, stretches, p.bias, p.C, p.M, p.N, p.ldc);
 }
 
-template <bool kGate>
+// (kAdded: up to 16 rows)
+template <bool kGate, int kBeside = kPlain>
 void run_few(hipStream_t s, const Product& p, bool vec) {
-    if (!vec) return run_rows<16, 16, 8, kGate, false>(s, p);
+    if (!vec) return run_rows<16, 16, 8, kGate, false, kBeside>(s, p);
     // columns enough for two workgroups of 32 on every unit; a short K has blocks for four waves only
     const bool wide = p.N >= 64 * p.units, shallow = p.K <= 4 * kBlockK;
-    if (p.M > 16) {
+    if constexpr (kBeside == kPlain) if (p.M > 16) {
         if (shallow) wide ? run_rows<32, 32, 4, kGate, true>(s, p) : run_rows<32, 16, 4, kGate, true>(s, p);
         else wide ? run_rows<32, 32, 8, kGate, true>(s, p) : run_rows<32, 16, 8, kGate, true>(s, p);
         return;
     }
     const bool eight = p.M <= 8;
     if (wide) {
-        if (shallow) eight ? run_rows<8, 32, 4, kGate, true>(s, p) : run_rows<16, 32, 4, kGate, true>(s, p);
-        else eight ? run_rows<8, 32, 8, kGate, true>(s, p) : run_rows<16, 32, 8, kGate, true>(s, p);
+        if (shallow) eight ? run_rows<8, 32, 4, kGate, true, kBeside>(s, p) : run_rows<16, 32, 4, kGate, true, kBeside>(s, p);
+        else eight ? run_rows<8, 32, 8, kGate, true, kBeside>(s, p) : run_rows<16, 32, 8, kGate, true, kBeside>(s, p);
         return;
     }
     if constexpr (!kGate) {
         // a long K and too few columns for a workgroup of 16 on every unit: 8 columns (a unit streams some 30 GB/s
         // however many loads it has under way: N 2,048, K 11,008 at 4 rows 32 -> 26 us; K 2,048 is as fast with 16)
         if (p.K > 8 * kBlockK && p.N < 16 * p.units) {
-            eight ? run_rows<8, 8, 16, false, true>(s, p) : run_rows<16, 8, 16, false, true>(s, p);
+            eight ? run_rows<8, 8, 16, false, true, kBeside>(s, p) : run_rows<16, 8, 16, false, true, kBeside>(s, p);
             return;
         }
     }
-    if (shallow) eight ? run_rows<8, 16, 4, kGate, true>(s, p) : run_rows<16, 16, 4, kGate, true>(s, p);
-    else eight ? run_rows<8, 16, 8, kGate, true>(s, p) : run_rows<16, 16, 8, kGate, true>(s, p);
+    if (shallow) eight ? run_rows<8, 16, 4, kGate, true, kBeside>(s, p) : run_rows<16, 16, 4, kGate, true, kBeside>(s, p);
+    else eight ? run_rows<8, 16, 8, kGate, true, kBeside>(s, p) : run_rows<16, 16, 8, kGate, true, kBeside>(s, p);
 }
 
 // The same choice for up to 16 rows with their norm (and the rotation) beside the product; no width takes 8 columns here.
@@ -871,15 +883,14 @@ CIE_API int cie_gemm_f32(void* stream, const float* A, const float* W, const flo
     return cie_after_launch();
 }
 
-// Few rows: C [M, N] (rows ldc apart) += A W^T (+ bias), added to as the norm's kernel would add the product to its stream.
+// Up to 16 rows: C [M, N] (rows ldc apart) += A W^T (+ bias), added to as the norm's kernel would add the product to its stream.
 CIE_API int cie_gemm_f32_into(void* stream, const float* A, const float* W, const float* bias, float* C, int M, int N, int K,
                               int lda, int ldc, int units) {
-    if (M < 0 || N <= 0 || K <= 0 || lda < K || ldc < N || units < 1 || M > 8 * 65535) return CIE_BAD_ARGUMENT;
+    if (M < 0 || M > 16 || N <= 0 || K <= 0 || lda < K || ldc < N || units < 1) return CIE_BAD_ARGUMENT;
     if (M == 0) return CIE_OK;
     const bool vec = K % 4 == 0 && lda % 4 == 0 && on_16_bytes(A) && on_16_bytes(W);
-    Product p{A, W, bias, C, nullptr, M, N, K, lda, ldc, units, {}};
-    p.beside.into = 1;
-    run_few<false>(static_cast<hipStream_t>(stream), p, vec);
+    const Product p{A, W, bias, C, nullptr, M, N, K, lda, ldc, units, {}};
+    run_few<false, kAdded>(static_cast<hipStream_t>(stream), p, vec);
     return cie_after_launch();
 }
 
@@ -913,7 +924,7 @@ CIE_API int cie_gemm_f32_normed_rope(void* stream, const float* rows, const floa
         (write_kv && (!seq_of_token || !seq_slot || !block_table || !k_pool || !v_pool)))
         return CIE_BAD_ARGUMENT;
     const Product p{rows, W, bias, C, nullptr, M, N, K, K, N, units,
-                    {norm_weight, eps, 0, cos_table, sin_table, positions, seq_of_token, seq_slot, block_table, table_width, k_pool,
+                    {norm_weight, eps, cos_table, sin_table, positions, seq_of_token, seq_slot, block_table, table_width, k_pool,
                      v_pool, q_heads, kv_heads, head_dim, rotary_dim, page_size, rotate, write_kv}};
     run_few_beside<false, kRotated>(static_cast<hipStream_t>(stream), p);
     return cie_after_launch();
