@@ -1,4 +1,4 @@
-// bfloat16 products of more than a hundred rows on the matrix cores, operands loaded straight into LDS: C = A * W^T with
+// bfloat16 products of some dozens of rows and more on the matrix cores, operands loaded straight into LDS: C = A * W^T with
 // A [M, K], W [N, K] bf16, K a multiple of 64, and float32 sums.  Epilogues: those of gemm_tiles.hip, which is left with the
 // other K.
 //
