@@ -23,10 +23,9 @@
 // time, 18.0 and 32.5).  The q/k/v epilogue asks for its rows' places between the last slices: 256 rows 14.8 -> 14.1; at 256 x 256
 // it spills 14 registers (60 bytes a lane), no other form any.
 //
-// The gate takes its quotient as a product with the reciprocal instruction's (1 unit in the last place; what is rounded to bf16
-// differs in 5 of a million numbers, its error against 64 bits in none of its first eight digits): a wave stores 64 of them a
-// lane, 10 instructions each where the division took 20, and the matrix cores wait.  3B gate/up 2,048 rows 170 -> 160 (three
-// turns of it), 613 rows 66.4 -> 63.6, 256 rows 34.1 -> 33.6.
+// The gate's quotient (gate_of) has the division's bits in fewer instructions than the compiler's division: a wave makes 64
+// of them a lane, and the matrix cores wait.  3B gate/up 2,048 rows 161 -> 158 (three turns of it), 613 rows 66.1 -> 64.6, 256
+// rows 33.1 -> 32.8.  (The reciprocal instruction's alone, 1 unit in the last place and 0 beyond 2^126: 154, 64.1, 32.6.)
 //
 // Measured (MI355X, us, weights from memory; before: the library with the kernel behind its product, or gemm_tiles.hip):
 // 3B: gate/up 256 rows 40 -> 33, 613 rows 72 -> 61, 777 81 -> 72, 2,048 186 -> 157; down 256 rows 27 -> 23, 613 47 -> 36, 2,048
@@ -175,6 +174,16 @@ __device__ __forceinline__ void store_rope(const DirectArgs& p, const floatx4 (&
             *reinterpret_cast<uint2*>(to + half) = uint2{pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
         }
     }
+}
+
+// x / (1 + e^-x), rounded as the division rounds it.  The reciprocal instruction's quotient is within a unit in the last place, and
+// adding what its remainder still gives rounds it right (Markstein, IBM J. Res. Dev. 34, 1990); the instruction's result is 0
+// where it lies below the normal numbers, so it is asked for a quarter of the denominator and scaled behind it; the last step
+// puts infinities, zeros and NaN right.  Equal to the division for each of the 2^32 floats, which were all compared.
+__device__ __forceinline__ float gate_of(float x) {
+    const float e = __expf(-x), y = 1.0f + e;
+    const float r = 0.25f * __builtin_amdgcn_rcpf(__builtin_fmaf(e, 0.25f, 0.25f)), q = x * r;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-y, q, x), r, q), y, x);
 }
 
 // All of this wave's loads but the youngest kYounger are in LDS, and all its reads of LDS in registers.
@@ -420,8 +429,7 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
 #pragma unroll
             for (int i = 0; i < 4 * kPair; ++i) {
                 if constexpr (EPI == DIRECT_SILU) {
-                    const float x = acc[2 * (u + i / 4)][im][i % 4];
-                    v[i] = x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)) * acc[2 * (u + i / 4) + 1][im][i % 4];
+                    v[i] = gate_of(acc[2 * (u + i / 4)][im][i % 4]) * acc[2 * (u + i / 4) + 1][im][i % 4];
                 } else {
                     v[i] = acc[u + i / 4][im][i % 4] + b[i];
                 }

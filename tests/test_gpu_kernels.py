@@ -347,7 +347,34 @@ def test_gemm_direct_of_few_rows(ops, shape, tile):
         ops.gemm_tiles(w, ops.TILE_ATOMIC, a, 64, 64, into=stream, parts=1)
 
 
-@pytest.mark.parametrize("gate", [0.0, 0.5, -0.5, 9.0, -9.0, 40.0, -40.0, -80.0, 1e30, -1e30, math.inf])
+@pytest.mark.parametrize("gates", ["of one", "of many sizes", "where 1 + e^-x passes 2^126", "tiny", "at the ends"])
+def test_gemm_direct_gate_is_the_division(ops, gates):
+    """The gate's quotient in the bits of the tiles that divide: a gate is three bf16 numbers (24 bits) times the column's scale,
+    in one group of 8 k, so that either kernel has the same float32 sums."""
+    g = torch.Generator().manual_seed(31)
+    x = torch.rand(4096, generator=g) * 2 - 1
+    if gates == "of many sizes":
+        x *= 2.0 ** torch.linspace(-20, 6.4, 4096)
+    elif gates == "where 1 + e^-x passes 2^126":
+        x = torch.linspace(-88.8, -87.2, 4096)
+    elif gates == "tiny":
+        x *= 2.0 ** torch.linspace(-132, -100, 4096)
+    elif gates == "at the ends":
+        x = torch.tensor([3e38, -3e38, 1e38, -1e38, 89.0, -89.0, -104.0, 0.0, -0.0, 2.0 ** 126, -(2.0 ** 126)]).repeat(373)[:4096]
+    hi = x.bfloat16()
+    mid = torch.where(hi.isinf(), 0.0, x - hi.float()).bfloat16()
+    lo = torch.where(hi.isinf(), 0.0, x - hi.float() - mid.float()).bfloat16()
+    a = torch.zeros((4096, 64), dtype=torch.bfloat16)
+    a[:, 0], a[:, 1], a[:, 2], a[:, 3] = hi, mid, lo, 1.0
+    w = torch.zeros((128, 64), dtype=torch.bfloat16)
+    w[:64, :3] = (torch.ones(64) if gates != "of many sizes" else 1.0 + torch.arange(64) / 64).bfloat16()[:, None]
+    w[64:, 3] = (0.5 + torch.arange(64) / 64).bfloat16()  # (the up halves)
+    a, w = a.cuda(), w.cuda()
+    got, divided = (ops.gemm_tiles(w, ops.TILE_SILU, a, 128, 64, direct=direct) for direct in (True, False))
+    assert torch.equal(got.isnan(), divided.isnan()) and torch.equal(got.nan_to_num(nan=7.0).view(torch.int16), divided.nan_to_num(nan=7.0).view(torch.int16))
+
+
+@pytest.mark.parametrize("gate", [0.0, 0.5, -0.5, 9.0, -9.0, 40.0, -40.0, -80.0, -87.5, -88.5, 1e30, -1e30, math.inf])
 def test_gemm_direct_gate_over_its_range(ops, gate):
     """Each row's one number k = 0 is its gate, k = 1 its up; the result is rounded once to bf16 (half of 2^-7), behind float32
     steps of a few 2^-24; what lies below float32's normal numbers is nothing."""
