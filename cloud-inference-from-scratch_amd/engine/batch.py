@@ -63,10 +63,12 @@ class StepBatch:
         return all(n == 1 for n in self.host_q_lens)
 
     @functools.cached_property
-    def portions(self) -> tuple[int, int]:
-        """(tokens of the sequences that bring more than one, sequences that bring one): asked for by every layer."""
+    def portions(self) -> tuple[int, int, int]:
+        """(tokens of the sequences that bring more than one, the longest context among these, sequences that bring one):
+        asked for by every layer."""
         singles = self.host_q_lens.count(1)
-        return sum(self.host_q_lens) - singles, singles
+        longest = max((s + n for s, n in zip(self.host_starts, self.host_q_lens) if n > 1), default=0)
+        return sum(self.host_q_lens) - singles, longest, singles
 
     @property
     def max_q_len(self) -> int:

@@ -216,8 +216,8 @@ def plan_splits(units: int, max_keys: int, target_waves: int = 1024, min_keys: i
 
 
 def takes_prompt_form(tiles: int, keys: int, singles: int, captured: bool, cus: int) -> bool:
-    """Whether prompt portions of so many tiles of 64 rows x kv heads, over up to ``keys`` keys and beside ``singles`` single
-    tokens, take the form that shares keys and values through LDS.  (A captured step's keys are known when it is replayed.)"""
+    """Whether prompt portions of so many tiles of 64 rows x kv heads, over up to ``keys`` keys of their own and beside ``singles``
+    single tokens, take the form that shares keys and values through LDS.  (A captured step's keys are known when it is replayed.)"""
     if tiles >= max(1, EIGHT_WAVE_TILES * cus):
         return True
     if tiles == 0 or 0 < singles <= JOINED_DECODE_ROWS:
@@ -263,7 +263,8 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
     wide = page_size >= 16 and scale > 0
     # Prompt portions with enough rows take tiles of 128 rows and eight waves, whose keys and values pass
     # through LDS once per tile.  (A short portion behind a long context also has its keys cut into parts.)
-    prompt_tokens, singles = batch.portions
+    prompt_tokens, prompt_keys, singles = batch.portions
+    prompt_keys = prompt_keys if window is None else min(prompt_keys, window + 64)
     bound = batch.static_plan.max_keys if batch.static_plan is not None else max_keys
     cuts = max(1, bound // PROMPT_SPLIT_KEYS) if wide and window is None else 1  # (a window's keys stay whole)
     big_tiles = -(-prompt_tokens * group // 128) * num_kv_heads
@@ -274,7 +275,7 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
     # heads, 456 large tiles: 55.3 -> 70.5; heads of 64 dimensions, where the softmax arithmetic per key is the same
     # and the products are half: 2,048 tokens 40.2 -> 33.0, against 43.1 in the form of four waves without LDS).
     eight = (wide and head_dim in (64, 128) and group <= 64
-             and takes_prompt_form(small_tiles, max_keys, singles, batch.static_plan is not None, cus))
+             and takes_prompt_form(small_tiles, prompt_keys, singles, batch.static_plan is not None, cus))
     lds_row_tiles = 8 if head_dim == 128 and big_tiles > LARGE_TILES_ABOVE * cus else 4
 
     def decode_form(bound: int, units: int) -> tuple[int, dict]:
