@@ -11,7 +11,7 @@ come in two forms: waves that share K and own all rows (few rows; the q/k/v and
 o_proj products, logits of up to 3 rows and narrow float32 results), and waves that
 own columns and share the rows through LDS (the SiLU-gate product up to 96 rows, every
 product whose K is cut, logits of 4 to 96 rows).
-bfloat16 with more rows, and from ``FEW_TILE_ROWS`` rows on what meets the units in one turn (``plan_few_tiles``,
+bfloat16 with more rows, and from ``FEW_TILE_ROWS`` rows on where they are the faster ones (``cut_tiles``, ``part_tiles``,
 ``gate_tiles``): tiles of this package's own (``csrc/gemm_direct.hip``, and
 ``csrc/gemm_tiles.hip`` for a K that is no multiple of 64) where they are the faster ones, else the
 vendor library's product (hipBLASLt through a thin cached interface of this
@@ -280,55 +280,127 @@ def choose_tiles(rows: int, n: int, k: int, row_stride: int, most_parts: int = 1
     return None if form is None else Tiles(*form, False)
 
 
-# Products of FEW_TILE_ROWS to FUSED_PARTS_ROWS rows (more: the model above).  The forms whose waves read every row for every 16
-# or 32 columns take longer with every row; the tiles that load straight into LDS read a row once for their 64 to 128 columns
-# (MI355X, us, chains of one product from memory, the other form or the library and tiles; down, parts added with atomic adds:
-# 3B 48 rows 13.6, 12.8, 64 14.9, 14.0, 96 18.8, 16.7, 128 23.3, 18.5; 7B 128 rows 53.6, 39.4; 0.5B 128 rows 10.5, 7.5; at 32 rows
-# level; output product of more than FUSED_SMALL_WEIGHT numbers, in parts: 7B 17 rows 12.3, 8.1, 96 rows 20.4, 11.9, 14B 128 rows
-# 27.9, 18.9; gate/up: 0.5B 48 rows 10.5, 7.3, 128 rows 14.5, 8.8, 1.5B 64 rows 17.6, 16.0, 128 rows 25.6, 20.8, 3B 64 rows 22.0, 21.5,
-# 96 rows 27.4, 25.7, 128 rows 31.8, 25.8, 14B 128 rows 72.6, 65.7; 7B, whose tiles of 128 rows do not meet the units in one turn,
-# 96 rows 68.2, 71.6).
-FEW_TILE_ROWS = 48
+# Products of up to FUSED_PARTS_ROWS rows (more: the models above).  The forms whose waves read every row for every 16 or 32
+# columns take longer with every row; the tiles that load straight into LDS read a row once for their 64 to 128 columns, but
+# stream a weight no faster, and add more sums: which is faster goes by shape (MI355X, us, the other way and the tiles: down 3B
+# 64 rows 14.9, 14.0, 128 23.3, 18.5; 4,096 x 4,096 in 8 parts of 128 rows at 96 rows 16.4, 20.3; 5,120 x 22,016 64 rows 51.7,
+# 59.4; gate/up 0.5B 128 rows 14.5, 8.8, 14B 72.6, 65.7, 28,672 x 6,144 72 rows 71.7, 80.0, 1,024 x 6,144 112 rows 15.3, 18.2).  So
+# both sides are modelled, each a sum of what it does, fitted to 28,000 timings inside captured chains, weights from memory
+# (260 products of any width and K added into the stream, 260 gates, 97 products in parts with the norm behind them, at 8 or 9
+# row counts from 17 to 128; 8 to 10 % root mean square for the tiles, 6 and 5 % for the forms of streaming waves, 10 for the
+# library).  Tiles: a start, per slice of 64 k, and per million weights (by the rows of a tile) and sums.
+FEW_CUT_US = {(64, 64): (1.83, 0.224), (96, 64): (1.95, 0.278), (128, 64): (1.63, 0.374), (96, 128): (2.38, 0.411),
+              (128, 128): (1.67, 0.493)}
+FEW_GATE_US = {(64, 64): (2.77, 0.166), (96, 64): (2.73, 0.217), (128, 64): (2.13, 0.305), (96, 128): (3.38, 0.325),
+               (128, 128): (2.39, 0.397)}
+FEW_CUT_WEIGHTS, FEW_CUT_SUMS = {64: 0.153, 128: 0.101}, 3.15
+FEW_GATE_WEIGHTS, FEW_GATE_SUMS = {64: 0.238, 128: 0.206}, 0.473
+# The other side: the cut product of streaming waves (a start, per 32 rows, per slice, the slice's 32 rows and those of all its
+# column tiles, per million sums and weights), their gate (a start, per slice and 32 rows, per slice and pair that
+# meets on a unit, per million weights and results), the library's gate with the kernel behind it (a start, per 1,000 k, per
+# million weights and results).
+SHARED_CUT_US = (1.90, 0.478, 0.0945, 0.0454, 0.0526, 2.62, 0.117)
+SHARED_GATE_US = (4.29, 0.1364, 0.0743, 0.0219, 0.855)
+LIBRARY_GATE_US = (8.28, 1.14, 0.385, 1.18)
+# Tiles are taken where they are modelled to be faster by this: of the 2,080 cut products 1,491 are then, 34 of them more than 2 %
+# slower than the other way (5,120 and 6,144 x 22,016 among them, 13 %: a K whose rows crowd few channels), of 1,560 gates against
+# streaming waves 1,165 and 4 (27,648 x 2,048 at 72 rows 26.9, 30.8), of 780 against the library 684 and 9 (narrow ones at 128
+# rows, where it times its candidates); in the mean 11, 23 and 19 % faster than without tiles.
+FEW_CUT_MARGIN, FEW_GATE_MARGIN = 0.95, 0.93
+FEW_TILE_ROWS = 48  # (at 32 rows the two are level)
 FEW_TILE_PARTS = (1, 2, 4, 8)
-FEW_GATE_WIDTH = 72  # columns of gate and up a unit up to which 64 rows and fewer go to tiles (3B's 86: level, 1.5B's 70: 8 %)
+# A product whose parts the next norm sums goes to tiles from FUSED_ROWS + 1 rows on (us, the library and the norm that adds its
+# branch, tiles and the norm that sums parts: 3,584 x 3,584 17 rows 16.2, 12.3, 96 24.5, 16.8; 8,192 x 29,568 32 rows 110, 93; up
+# to 40 million weights 584 timings, 11 more than 2 % slower, in the mean 20 % faster), but for a large weight whose rows lie a
+# multiple of 8 KB apart, which the library streams at up to 4.8 TB/s: that from 65 rows on (8,192 x 8,192 32 rows 34, 40, 64 39,
+# 38; 12,288 x 8,192 32 rows 49, 52, 72 63, 55; 8,192 x 16,384 48 rows 65, 72; from K 20,480 on it is the slower one again).  Of
+# 800 timings beyond 40 million weights 73 are then more than 2 % slower, by up to 15 % (K 11,008, 3,072 and 5,120 of the
+# widest most), in the mean 12 % faster.
+FEW_PARTS_WEIGHTS, FEW_PARTS_APART, FEW_PARTS_K, FEW_PARTS_ROWS = 40 << 20, 4096, 16384, 65
+
+
+def _few_us(form: tuple[int, int, int], rows: int, n: int, k: int, gate: bool) -> float:
+    columns, tile_rows, parts = form
+    times, weights, sums = ((FEW_GATE_US, FEW_GATE_WEIGHTS, FEW_GATE_SUMS) if gate else (FEW_CUT_US, FEW_CUT_WEIGHTS, FEW_CUT_SUMS))
+    start, per_slice = times[columns, tile_rows]
+    return (start + -(-(-(-k // parts)) // ops.DIRECT_SLICE) * per_slice + n * k * 1e-6 * weights[tile_rows]
+            + parts * rows * n * 1e-6 * sums)
 
 
 @functools.lru_cache(maxsize=4096)
-def plan_few_tiles(rows: int, n: int, k: int, most_parts: int, units: int) -> Optional[tuple[int, int, int]]:
-    """(columns, rows, parts) of the tiles of up to FUSED_PARTS_ROWS rows, or ``None`` if no form meets the units in one turn: of
-    those with nearly the most workgroups that do, the one that streams the weight the fewest times, in the fewest parts."""
+def plan_few_tiles(rows: int, n: int, k: int, most_parts: int, units: int, gate: bool = False) -> Optional[tuple[int, int, int]]:
+    """(columns, rows, parts) of the tiles of up to FUSED_PARTS_ROWS rows, or ``None`` if no form meets the units in one turn (each
+    XCD has an eighth of the tiles and of the units): of those that do the fastest by the model."""
     forms = []
-    for tile_rows in (64,) if rows <= 64 else (64, 128):
-        for columns in (64, 96, 128):
-            if (columns, tile_rows) not in ops.DIRECT_SHAPES:
-                continue
-            for parts in FEW_TILE_PARTS:
-                groups = -(-n // columns) * -(-rows // tile_rows) * parts
-                if parts <= most_parts and groups <= units and -(-(-(-k // parts)) // ops.DIRECT_SLICE) * ops.DIRECT_SLICE * (parts - 1) < k:
-                    forms.append((groups, columns, tile_rows, parts))
-    if not forms:
+    for columns, tile_rows in FEW_CUT_US:
+        if tile_rows > 64 >= rows:
+            continue
+        for parts in FEW_TILE_PARTS:
+            groups = -(-(-(-n // columns) * -(-rows // tile_rows)) // XCDS) * parts
+            if (parts <= most_parts and groups <= units // XCDS
+                    and -(-(-(-k // parts)) // ops.DIRECT_SLICE) * ops.DIRECT_SLICE * (parts - 1) < k):
+                forms.append((columns, tile_rows, parts))
+    return min(forms, key=lambda form: _few_us(form, rows, n, k, gate), default=None)
+
+
+@functools.lru_cache(maxsize=4096)
+def _cut_tiles(rows: int, n: int, k: int, units: int) -> Optional[tuple[int, int, int]]:
+    form = plan_few_tiles(rows, n, k, FEW_TILE_PARTS[-1], units)
+    if form is None:
         return None
-    most = max(forms)[0]
-    _groups, columns, tile_rows, parts = min((f for f in forms if f[0] >= 0.9 * most), key=lambda f: (-(-rows // f[2]), f[3], -f[0], f[1]))
-    return columns, tile_rows, parts
+    column_tiles, _waves, parts = plan_shared_parts(-(-n // 16), k)
+    slices, pairs = -(-(-(-k // parts)) // 64), -(-rows // 32)
+    start, per_rows, per_slice, per_pair, per_tile, per_sums, per_weights = SHARED_CUT_US
+    other = (start + pairs * per_rows + slices * (per_slice + pairs * (per_pair + column_tiles * per_tile))
+             + parts * rows * n * 1e-6 * per_sums + n * k * 1e-6 * per_weights)
+    return form if _few_us(form, rows, n, k, False) < FEW_CUT_MARGIN * other else None
 
 
-def few_tiles(x: torch.Tensor, weight: torch.Tensor, most_parts: int = 1, into: Optional[torch.Tensor] = None,
-              fewest: int = FEW_TILE_ROWS) -> Optional[tuple[int, int, int]]:
-    """What :func:`plan_few_tiles` says for these operands, if the tiles take them at all."""
+@functools.lru_cache(maxsize=4096)
+def _gate_tiles(rows: int, n: int, k: int, units: int) -> Optional[tuple[int, int, int]]:
+    form = plan_few_tiles(rows, n, k, 1, units, True)
+    if form is None:
+        return None
+    if rows <= SHARED_SILU_ROWS:
+        pairs = -(-n // 32)
+        waves, _own = plan_shared_silu(pairs)
+        start, per_rows, per_pair, per_weights, per_results = SHARED_GATE_US
+        other = start + k / 64 * (-(-rows // 32) * per_rows + -(-(-(-pairs // waves)) // units) * waves * per_pair)
+    else:
+        start, per_k, per_weights, per_results = LIBRARY_GATE_US
+        other = start + k * 1e-3 * per_k
+    other += n * k * 1e-6 * per_weights + rows * n * 1e-6 * per_results
+    return form if _few_us(form, rows, n, k, True) < FEW_GATE_MARGIN * other else None
+
+
+def _few_fits(x: torch.Tensor, weight: torch.Tensor, into: Optional[torch.Tensor], fewest: int) -> bool:
     rows, k = x.shape
-    if not fewest <= rows <= FUSED_PARTS_ROWS or not takes_tiles(rows, x, weight, into, beyond=FUSED_ROWS):
+    return (fewest <= rows <= FUSED_PARTS_ROWS and takes_tiles(rows, x, weight, into, beyond=FUSED_ROWS)
+            and ops.direct_fits(rows, weight.shape[0], k, x.stride(0)))
+
+
+def cut_tiles(x: torch.Tensor, weight: torch.Tensor, into: Optional[torch.Tensor] = None) -> Optional[tuple[int, int, int]]:
+    """(columns, rows, parts of K) of the tiles that a product takes whose other way is the cut form of streaming waves, or
+    ``None``: that one."""
+    if not _few_fits(x, weight, into, FEW_TILE_ROWS):
         return None
-    if not ops.direct_fits(rows, weight.shape[0], k, x.stride(0)):
+    return _cut_tiles(x.shape[0], weight.shape[0], x.shape[1], ops.compute_units())
+
+
+def part_tiles(x: torch.Tensor, weight: torch.Tensor, into: torch.Tensor) -> Optional[tuple[int, int, int]]:
+    """... whose other way is the library."""
+    n, k = weight.shape
+    large = n * k > FEW_PARTS_WEIGHTS and k % FEW_PARTS_APART == 0 and k <= FEW_PARTS_K
+    if not _few_fits(x, weight, into, FEW_PARTS_ROWS if large else FUSED_ROWS + 1):
         return None
-    return plan_few_tiles(rows, weight.shape[0], k, most_parts, ops.compute_units())
+    return plan_few_tiles(x.shape[0], n, k, FEW_TILE_PARTS[-1], ops.compute_units())
 
 
 def gate_tiles(x: torch.Tensor, weight: torch.Tensor) -> Optional[tuple[int, int, int]]:
-    """... for a gated unit's product."""
-    if x.shape[0] <= 64 and weight.shape[0] > FEW_GATE_WIDTH * ops.compute_units():
+    """(columns, rows, 1) of the tiles that a gated unit's product takes, or ``None``: the form of streaming waves, or the library."""
+    if not _few_fits(x, weight, None, FEW_TILE_ROWS):
         return None
-    return few_tiles(x, weight)
+    return _gate_tiles(x.shape[0], weight.shape[0], x.shape[1], ops.compute_units())
 
 
 @dataclass
@@ -553,7 +625,7 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
         # (atomic adds cost the product nothing, measured against partial products written for the next norm
         # kernel to sum: 10.3 us either way for the 3B shape's down product at 8 rows; and the kernel that summed
         # them falls away)
-        tiles = few_tiles(x, weight, FEW_TILE_PARTS[-1], into)
+        tiles = cut_tiles(x, weight, into)
         if tiles is not None:
             ops.gemm_tiles(weight, ops.TILE_ATOMIC, x, tiles[0], tiles[1], bias, into, tiles[2], direct=True)
             return Added()
@@ -565,7 +637,7 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
             and k >= PART_MIN_K and x.data_ptr() % 16 == 0):
         # a branch that whoever adds it sums itself (the down product of the parallel block, 8 rows, K 11,008: 17 us whole,
         # 11 in 8 parts, and 0.4 more in the kernel that adds them)
-        tiles = few_tiles(x, weight, FEW_TILE_PARTS[-1])
+        tiles = cut_tiles(x, weight)
         if tiles is not None:
             return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, tiles[0], tiles[1], bias, None, tiles[2], direct=True))
         column_tiles, waves, parts = plan_shared_parts(-(-n // 16), k)
@@ -602,7 +674,7 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
             return ops.gemm_fused(weight, ops.EPI_F32 if wants_f32 else ops.EPI_BF16, x, bias=bias)
     if (fusable and not wants_f32 and not silu and into is not None and sums_parts and FUSED_ROWS < rows <= FUSED_PARTS_ROWS
             and into.is_contiguous() and tuple(into.shape) == (rows, n)):
-        tiles = few_tiles(x, weight, FEW_TILE_PARTS[-1], into, fewest=FUSED_ROWS + 1)
+        tiles = part_tiles(x, weight, into)
         if tiles is not None:  # (the norm behind it sums the parts)
             return KParts(ops.gemm_tiles(weight, ops.TILE_PARTS, x, tiles[0], tiles[1], bias, None, tiles[2], direct=True))
     if fusable and not wants_f32 and takes_tiles(rows, x, weight, into):

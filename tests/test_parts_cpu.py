@@ -238,3 +238,33 @@ def test_tiles_of_few_rows_meet_the_units_once(rows, n, k, most):
     assert (columns, tile_rows) in ops.DIRECT_SHAPES and parts <= most
     assert -(-n // columns) * -(-rows // tile_rows) * parts <= 256
     assert -(-(-(-k // parts)) // 64) * 64 * (parts - 1) < k  # (no part without k)
+    assert -(-(-(-n // columns) * -(-rows // tile_rows)) // 8) * parts <= 32  # (and an eighth of the tiles an eighth of the units)
+
+
+@pytest.mark.parametrize("rows,n,k,gate,tiles", [
+    # (us, the other way and the tiles, measured)
+    (64, 2048, 11008, False, True), (96, 2048, 11008, False, True), (128, 3584, 18944, False, True), (72, 896, 4864, False, True),
+    (96, 5120, 5120, False, True),
+    (64, 5120, 22016, False, False),   # 51.7, 59.4
+    (48, 6144, 8192, False, False),    # 23.0, 26.0
+    (56, 8128, 8192, False, False),    # 27.4, 29.9
+    (64, 6144, 24576, False, False),   # 64.5, 70.8
+    (64, 9728, 896, True, True), (128, 22016, 2048, True, True), (56, 20480, 1024, True, True),
+    (64, 28672, 6144, True, False),    # 65.3, 78.1
+    (72, 28672, 6144, True, False),    # 71.7, 80.0
+    (112, 1024, 6144, True, False),    # 15.3, 18.2
+    (112, 1120, 5120, True, False),    # 14.7, 16.8
+    (128, 16384, 5120, True, False)])  # 49.4, 52.4
+def test_tiles_of_few_rows_where_they_are_the_faster_ones(monkeypatch, rows, n, k, gate, tiles):
+    from cie_amd.kernels import ops
+    from cie_amd.parts import linear
+
+    monkeypatch.setattr(ops, "compute_units", lambda *_: 256)
+    assert ((linear._gate_tiles if gate else linear._cut_tiles)(rows, n, k, 256) is not None) == tiles
+
+
+def test_tiles_of_few_rows_cut_a_short_k_little():
+    """4,096 x 4,096, 96 rows: 8 parts of 128 x 128 20.3 us, 2 of 64 x 64 13.7, the streaming waves 16.4."""
+    from cie_amd.parts.linear import plan_few_tiles
+
+    assert plan_few_tiles(96, 4096, 4096, 8, 256)[2] <= 4
