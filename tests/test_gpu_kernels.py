@@ -321,6 +321,19 @@ def test_gemm_direct(ops, shape, tile):
             torch.testing.assert_close(got.double().sum(0), product + b.double(), **sums)
 
 
+def close_to_gated_unit(got, a, w, scale, sums):
+    """bf16(silu(g) * u) for g, u = scale x halves of a @ w.T: each row by its own numbers.  A float32 sum of k products is off by at
+    most k 2^-24 of its terms' sizes, its scale (of `sums` partial sums, a root, a quotient) by (sums + 8) 2^-24; silu's slope is
+    at most 1.1; the exponential and the last rounding to bf16 stay below 2^-8 of the result."""
+    n, k = w.shape
+    product, size = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    g, u = (scale * half for half in (product[:, : n // 2], product[:, n // 2:]))
+    g_off, u_off = (scale * half * (k + sums + 8) * 2.0 ** -24 for half in (size[:, : n // 2], size[:, n // 2:]))
+    expect = torch.nn.functional.silu(g) * u
+    bound = 1.1 * g_off * (u.abs() + u_off) + torch.nn.functional.silu(g).abs() * u_off + 2.0 ** -8 * expect.abs() + 1e-30
+    assert ((got.double() - expect).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("shape", [(41, 64, 512), (64, 130, 1088), (65, 100, 2112), (96, 520, 960), (128, 96, 1024), (1, 66, 128)])
 @pytest.mark.parametrize("tile", [(64, 64), (96, 64), (128, 64), (96, 128), (128, 128)])
 def test_gemm_direct_of_few_rows(ops, shape, tile):
@@ -337,14 +350,61 @@ def test_gemm_direct_of_few_rows(ops, shape, tile):
             expect = stream.double() + product + (0.0 if bias is None else bias.double())
             ops.gemm_tiles(w, ops.TILE_ATOMIC, a, *tile, bias=bias, into=stream, parts=parts, direct=True)
             torch.testing.assert_close(stream.double(), expect, rtol=1e-4, atol=1e-4 * math.sqrt(k))
-    gate, up = product[:, : n // 2], product[:, n // 2:]
     for sums in (1, 3, 8, 56, 260):
         sumsq = rand((m, sums), torch.float32, 30).abs() * k
         scale = torch.rsqrt(sumsq.double().sum(1, keepdim=True) / k + 1e-5)
-        got = ops.gemm_tiles_silu_scaled(w, a, *tile, sumsq, 1e-5).double()
-        torch.testing.assert_close(got, torch.nn.functional.silu(gate * scale) * (up * scale), rtol=1e-2, atol=1e-2 * k / float(sumsq.sum(1).min() / k))
+        close_to_gated_unit(ops.gemm_tiles_silu_scaled(w, a, *tile, sumsq, 1e-5), a, w, scale, sums)
     with pytest.raises(ValueError, match="straight into LDS"):
         ops.gemm_tiles(w, ops.TILE_ATOMIC, a, 64, 64, into=stream, parts=1)
+
+
+@pytest.mark.parametrize("rows", [17, 47, 48, 64, 65, 96, 128])
+def test_linear_of_some_dozens_of_rows(ops, rows, monkeypatch):
+    """What linear() makes of products that may go to the tiles that load straight into LDS, by rows: the form, what comes back, and
+    its numbers against 64 bits (a float32 sum of k products is off by at most k 2^-24 of its terms' sizes)."""
+    from cie_amd.parts import linear as L
+    from cie_amd.parts.norm import RMSNorm
+
+    forms = []
+    for name in ("gemm_tiles", "gemm_tiles_silu_scaled"):
+        real = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda *a, real=real, scaled="scaled" in name, **k: (forms.append("scaled" if scaled else a[1]), real(*a, **k))[1])
+    tiles = rows >= L.FEW_TILE_ROWS
+
+    def product(n, k):
+        x, w, b = rand((rows, k), torch.bfloat16, 61), rand((n, k), torch.bfloat16, 62, 0.1), rand((n,), torch.bfloat16, 63)
+        return x, w, b, x.double() @ w.double().t(), (x.double().abs() @ w.double().abs().t()) * (k + 8) * 2.0 ** -24
+
+    x, w, b, expect, bound = product(896, 4864)  # a narrow one of a long K: its parts add themselves into the stream
+    for bias in (None, b):
+        stream = rand((rows, 896), torch.float32, 64)
+        whole = stream.double() + expect + (0.0 if bias is None else bias.double())
+        assert type(L.linear(x, w, bias, into=stream, sums_parts=True)) is L.Added
+        assert ((stream.double() - whole).abs() <= bound + 16 * 2.0 ** -24 * (whole.abs() + expect.abs() + 4)).all()
+        # ... or come back
+        branch = L.linear(x, w, bias, sums_parts=True)
+        assert type(branch) is L.KParts
+        assert ((branch.parts.double().sum(0) - expect - (0.0 if bias is None else bias.double())).abs() <= bound + 2.0 ** -22 * (expect.abs() + 4)).all()
+    assert forms == [ops.TILE_ATOMIC, ops.TILE_PARTS] * 2 if tiles else not forms
+    forms.clear()
+    x, w, b, expect, bound = product(2112, 3200)  # one of more than FUSED_SMALL_WEIGHT numbers whose K is too short for that
+    for bias in (None, b):
+        stream = rand((rows, 2112), torch.float32, 65)
+        before = stream.clone()
+        branch = L.linear(x, w, bias, into=stream, sums_parts=True)
+        assert type(branch) is L.KParts and torch.equal(stream, before)
+        assert ((branch.parts.double().sum(0) - expect - (0.0 if bias is None else bias.double())).abs() <= bound + 2.0 ** -22 * (expect.abs() + 4)).all()
+    assert forms == [ops.TILE_PARTS] * 2
+    forms.clear()
+    x, w, _b, _expect, _bound = product(9728, 896)  # a gate, and one of rows without their 1/rms
+    one = torch.ones((rows, 1), dtype=torch.float64, device="cuda")
+    close_to_gated_unit(L.linear(x, w, epilogue="silu"), x, w, one, 0)
+    norm = RMSNorm(896, 1e-6)
+    norm.bind({"weight": torch.ones(896, dtype=torch.bfloat16, device="cuda")}, "", torch.bfloat16, "cuda")
+    sumsq = torch.rand((rows, 14), generator=torch.Generator().manual_seed(66)).cuda() * torch.arange(1, rows + 1, device="cuda")[:, None]
+    scale = torch.rsqrt(sumsq.double().sum(1, keepdim=True) / 896 + 1e-6)
+    close_to_gated_unit(L.linear(L.ScaledRows(x, sumsq, 1e-6, x.float(), norm), w, epilogue="silu"), x, w, scale, 14)
+    assert forms == [ops.TILE_SILU, "scaled"] if tiles else not forms
 
 
 @pytest.mark.parametrize("gates", ["of one", "of many sizes", "where 1 + e^-x passes 2^126", "tiny", "at the ends"])
