@@ -135,7 +135,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
     constexpr int kOwned = (kSums + kThreads - 1) / kThreads;
     constexpr int kStep = kGate ? kColumns / 2 : kColumns;  // output columns of a tile
     static_assert(!kGate || kColumns == 32 || kColumns == 16, "a gate's tile holds as many columns of either half");
-    static_assert(!kOwnRows || (kVec && kRows <= 16), "a few rows in 16-byte pieces");
+    static_assert(!kOwnRows || (kVec && kRows == 8), "a few rows in 16-byte pieces");
     static_assert(kBeside != kRotated || (!kGate && kColumns == 16 && kRows * 8 <= kThreads), "8 dimensions and their partners");
     __shared__ float stage_all[kWaves * kStaged * kTileFloats];
     __shared__ float sums[2][kWaves * kSums];
@@ -803,55 +803,49 @@ void run_stretches(hipStream_t s, const Product& p, bool gate) {
     else gemm_f32_join_kernel<false><<<join, 256, 0, s>>>(p.parts, stretches, p.bias, p.C, p.M, p.N, p.ldc);
 }
 
-// (kAdded: up to 16 rows)
+// (kAdded: up to 8 rows)
 template <bool kGate, int kBeside = kPlain>
 void run_few(hipStream_t s, const Product& p, bool vec) {
     if (!vec) return run_rows<16, 16, 8, kGate, false, kBeside>(s, p);
     // columns enough for two workgroups of 32 on every unit; a short K has blocks for four waves only
     const bool wide = p.N >= 64 * p.units, shallow = p.K <= 4 * kBlockK;
-    if constexpr (kBeside == kPlain) if (p.M > 16) {
-        if (shallow) wide ? run_rows<32, 32, 4, kGate, true>(s, p) : run_rows<32, 16, 4, kGate, true>(s, p);
-        else wide ? run_rows<32, 32, 8, kGate, true>(s, p) : run_rows<32, 16, 8, kGate, true>(s, p);
-        return;
-    }
-    const bool eight = p.M <= 8;
-    if (wide) {
-        if (shallow) eight ? run_rows<8, 32, 4, kGate, true, kBeside>(s, p) : run_rows<16, 32, 4, kGate, true, kBeside>(s, p);
-        else eight ? run_rows<8, 32, 8, kGate, true, kBeside>(s, p) : run_rows<16, 32, 8, kGate, true, kBeside>(s, p);
-        return;
-    }
-    if constexpr (!kGate) {
-        // a long K and too few columns for a workgroup of 16 on every unit: 8 columns (a unit streams some 30 GB/s
-        // however many loads it has under way: N 2,048, K 11,008 at 4 rows 32 -> 26 us; K 2,048 is as fast with 16)
-        if (p.K > 8 * kBlockK && p.N < 16 * p.units) {
-            eight ? run_rows<8, 8, 16, false, true, kBeside>(s, p) : run_rows<16, 8, 16, false, true, kBeside>(s, p);
+    // a long K and too few columns for a workgroup of 16 on every unit: 8 columns (a unit streams some 30 GB/s
+    // however many loads it has under way: N 2,048, K 11,008 at 4 rows 32 -> 26 us; K 2,048 is as fast with 16)
+    const bool narrow = !kGate && p.K > 8 * kBlockK && p.N < 16 * p.units;
+    if constexpr (kBeside == kPlain) {
+        if (p.M > 16) {
+            if (shallow) wide ? run_rows<32, 32, 4, kGate, true>(s, p) : run_rows<32, 16, 4, kGate, true>(s, p);
+            else wide ? run_rows<32, 32, 8, kGate, true>(s, p) : run_rows<32, 16, 8, kGate, true>(s, p);
             return;
         }
+        if (p.M > 8) {
+            if (wide) return shallow ? run_rows<16, 32, 4, kGate, true>(s, p) : run_rows<16, 32, 8, kGate, true>(s, p);
+            if constexpr (!kGate)
+                if (narrow) return run_rows<16, 8, 16, false, true>(s, p);
+            return shallow ? run_rows<16, 16, 4, kGate, true>(s, p) : run_rows<16, 16, 8, kGate, true>(s, p);
+        }
     }
-    if (shallow) eight ? run_rows<8, 16, 4, kGate, true, kBeside>(s, p) : run_rows<16, 16, 4, kGate, true, kBeside>(s, p);
-    else eight ? run_rows<8, 16, 8, kGate, true, kBeside>(s, p) : run_rows<16, 16, 8, kGate, true, kBeside>(s, p);
+    if (wide) return shallow ? run_rows<8, 32, 4, kGate, true, kBeside>(s, p) : run_rows<8, 32, 8, kGate, true, kBeside>(s, p);
+    if constexpr (!kGate)
+        if (narrow) return run_rows<8, 8, 16, false, true, kBeside>(s, p);
+    shallow ? run_rows<8, 16, 4, kGate, true, kBeside>(s, p) : run_rows<8, 16, 8, kGate, true, kBeside>(s, p);
 }
 
-// The same choice for up to 16 rows with their norm (and the rotation) beside the product; no width takes 8 columns here.
-template <bool kGate, int kBeside>
-void run_few_beside(hipStream_t s, const Product& p) {
-    const bool wide = kBeside == kNormed && p.N >= 64 * p.units, shallow = p.K <= 4 * kBlockK, eight = p.M <= 8;
-    if constexpr (kBeside == kNormed) {
-        if (wide) {
-            if (shallow) eight ? run_rows<8, 32, 4, kGate, true, kBeside>(s, p) : run_rows<16, 32, 4, kGate, true, kBeside>(s, p);
-            else eight ? run_rows<8, 32, 8, kGate, true, kBeside>(s, p) : run_rows<16, 32, 8, kGate, true, kBeside>(s, p);
-            return;
-        }
-    }
-    if (shallow) eight ? run_rows<8, 16, 4, kGate, true, kBeside>(s, p) : run_rows<16, 16, 4, kGate, true, kBeside>(s, p);
-    else eight ? run_rows<8, 16, 8, kGate, true, kBeside>(s, p) : run_rows<16, 16, 8, kGate, true, kBeside>(s, p);
+// The same choice for up to 8 rows with their norm beside the gated product, or beside that of q/k/v; no width takes 8 columns here.
+void run_normed_gate(hipStream_t s, const Product& p) {
+    const bool wide = p.N >= 64 * p.units, shallow = p.K <= 4 * kBlockK;
+    if (wide) shallow ? run_rows<8, 32, 4, true, true, kNormed>(s, p) : run_rows<8, 32, 8, true, true, kNormed>(s, p);
+    else shallow ? run_rows<8, 16, 4, true, true, kNormed>(s, p) : run_rows<8, 16, 8, true, true, kNormed>(s, p);
+}
+void run_normed_rope(hipStream_t s, const Product& p) {
+    p.K <= 4 * kBlockK ? run_rows<8, 16, 4, false, true, kRotated>(s, p) : run_rows<8, 16, 8, false, true, kRotated>(s, p);
 }
 
 bool on_16_bytes(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
-// Up to 16 rows of a float32 stream whose norm the product makes itself.
+// Up to 8 rows of a float32 stream whose norm the product makes itself.
 bool takes_norm(const float* stream, const float* W, const float* norm_weight, float eps, int M, int K) {
-    return M >= 1 && M <= 16 && K >= 8 && K % 8 == 0 && K <= kNormSegments * kSegment &&
+    return M >= 1 && M <= 8 && K >= 8 && K % 8 == 0 && K <= kNormSegments * kSegment &&
            M * ((K + kSegment - 1) / kSegment) <= kNormTasks && eps > 0.f && stream && W && norm_weight &&
            on_16_bytes(stream) && on_16_bytes(W) && on_16_bytes(norm_weight);
 }
@@ -883,10 +877,10 @@ CIE_API int cie_gemm_f32(void* stream, const float* A, const float* W, const flo
     return cie_after_launch();
 }
 
-// Up to 16 rows: C [M, N] (rows ldc apart) += A W^T (+ bias), added to as the norm's kernel would add the product to its stream.
+// Up to 8 rows: C [M, N] (rows ldc apart) += A W^T (+ bias), added to as the norm's kernel would add the product to its stream.
 CIE_API int cie_gemm_f32_into(void* stream, const float* A, const float* W, const float* bias, float* C, int M, int N, int K,
                               int lda, int ldc, int units) {
-    if (M < 0 || M > 16 || N <= 0 || K <= 0 || lda < K || ldc < N || units < 1) return CIE_BAD_ARGUMENT;
+    if (M < 0 || M > 8 || N <= 0 || K <= 0 || lda < K || ldc < N || units < 1) return CIE_BAD_ARGUMENT;
     if (M == 0) return CIE_OK;
     const bool vec = K % 4 == 0 && lda % 4 == 0 && on_16_bytes(A) && on_16_bytes(W);
     const Product p{A, W, bias, C, nullptr, M, N, K, lda, ldc, units, {}};
@@ -894,17 +888,15 @@ CIE_API int cie_gemm_f32_into(void* stream, const float* A, const float* W, cons
     return cie_after_launch();
 }
 
-// Up to 16 rows, and rows * ceil(K / 512) up to 32: C = norm(rows of the stream [M, K], contiguous) W^T (+ bias), or its gated unit.  K a multiple of 8, up to
-// 8,192; stream, W and the norm's weight at multiples of 16 bytes.
-CIE_API int cie_gemm_f32_normed(void* stream, const float* rows, const float* norm_weight, float eps, const float* W, const float* bias,
-                                float* C, int M, int N, int K, int ldc, int gate, int units) {
-    if (!takes_norm(rows, W, norm_weight, eps, M, K) || N <= 0 || units < 1 || !C) return CIE_BAD_ARGUMENT;
-    if (ldc < (gate ? N / 2 : N) || (gate && (N % 2 || bias))) return CIE_BAD_ARGUMENT;
-    Product p{rows, W, bias, C, nullptr, M, N, K, K, ldc, units, {}};
+// Up to 8 rows, and rows * ceil(K / 512) up to 32: C [M, N / 2] = the gated unit of norm(rows of the stream [M, K], contiguous) W^T.
+// K a multiple of 8, up to 8,192; stream, W and the norm's weight at multiples of 16 bytes.
+CIE_API int cie_gemm_f32_normed(void* stream, const float* rows, const float* norm_weight, float eps, const float* W, float* C, int M,
+                                int N, int K, int ldc, int units) {
+    if (!takes_norm(rows, W, norm_weight, eps, M, K) || N <= 0 || N % 2 || ldc < N / 2 || units < 1 || !C) return CIE_BAD_ARGUMENT;
+    Product p{rows, W, nullptr, C, nullptr, M, N, K, K, ldc, units, {}};
     p.beside.norm_weight = norm_weight;
     p.beside.eps = eps;
-    if (gate) run_few_beside<true, kNormed>(static_cast<hipStream_t>(stream), p);
-    else run_few_beside<false, kNormed>(static_cast<hipStream_t>(stream), p);
+    run_normed_gate(static_cast<hipStream_t>(stream), p);
     return cie_after_launch();
 }
 
@@ -926,6 +918,6 @@ CIE_API int cie_gemm_f32_normed_rope(void* stream, const float* rows, const floa
     const Product p{rows, W, bias, C, nullptr, M, N, K, K, N, units,
                     {norm_weight, eps, cos_table, sin_table, positions, seq_of_token, seq_slot, block_table, table_width, k_pool,
                      v_pool, q_heads, kv_heads, head_dim, rotary_dim, page_size, rotate, write_kv}};
-    run_few_beside<false, kRotated>(static_cast<hipStream_t>(stream), p);
+    run_normed_rope(static_cast<hipStream_t>(stream), p);
     return cie_after_launch();
 }

@@ -583,7 +583,10 @@ def gemm_f32(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
     return out
 
 
-F32_FEW_ROWS = 16  # the most rows that the float32 product of few rows takes its neighbours' work along for
+# Rows up to which a float32 product takes the norm in front, the rotation or the add into the stream along (every workgroup makes
+# the norm of as many rows).  Decode steps of 12 layers, kernels of their own and joined, us: 3B 4 sequences, eight steps 12,061,
+# 11,211; 0.5B 8 sequences, four steps 3,586, 3,442; 16 sequences, with kernels for as many rows, 3,757, 3,770.
+F32_FEW_ROWS = 8
 F32_NORM_WIDTH = 8192  # ... the widest rows whose norm it makes,
 F32_NORM_SEGMENT, F32_NORM_SEGMENTS = 512, 32  # and how many segments of a row in all, which lie in LDS
 
@@ -617,18 +620,16 @@ def _check_normed_f32(stream: torch.Tensor, norm_weight: torch.Tensor, eps: floa
     return m, n, k
 
 
-def gemm_f32_normed(stream: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor,
-                    bias: Optional[torch.Tensor] = None, gate: bool = False) -> torch.Tensor:
-    """:func:`gemm_f32` of the RMS norm of ``stream``'s few rows, made inside the product: the bits are those of
+def gemm_f32_normed(stream: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor) -> torch.Tensor:
+    """The gated unit of :func:`gemm_f32` of the RMS norm of ``stream``'s few rows, made inside the product: the bits are those of
     :func:`add_rmsnorm` followed by the product."""
-    m, n, k = _check_normed_f32(stream, norm_weight, eps, weight, bias)
-    if gate and (bias is not None or n % 2):
-        raise ValueError("a gated unit takes an even number of weight rows and no bias")
-    width = n // 2 if gate else n
-    out = torch.empty((m, width), dtype=torch.float32, device=stream.device)
+    m, n, k = _check_normed_f32(stream, norm_weight, eps, weight, None)
+    if n % 2:
+        raise ValueError("a gated unit takes an even number of weight rows")
+    out = torch.empty((m, n // 2), dtype=torch.float32, device=stream.device)
     _run("cie_gemm_f32_normed", load_library().cie_gemm_f32_normed(
-        _stream(), _ptr(stream), _ptr(norm_weight), _f(eps), _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k),
-        _i(width), _i(bool(gate)), _i(compute_units(stream.device))))
+        _stream(), _ptr(stream), _ptr(norm_weight), _f(eps), _ptr(weight), _ptr(out), _i(m), _i(n), _i(k), _i(n // 2),
+        _i(compute_units(stream.device))))
     return out
 
 

@@ -1,7 +1,7 @@
 """``x @ W^T + b`` for a Linear's weight ``[out, in]``, and its fused forms.
 
 float32: the hand-written true-float32 kernels, always (the gated unit in their
-epilogue; of up to ``F32_JOINED_ROWS`` rows also the norm in front and the add into the stream).  bfloat16 with up to
+epilogue; of up to ``ops.F32_FEW_ROWS`` rows also the norm in front and the add into the stream).  bfloat16 with up to
 ``FUSED_ROWS`` rows (decode steps, the output head), and up to 64 or 128 rows where
 it is the faster one (a small weight, a long K): the hand-written
 matrix-core kernels that stream the weight once and take over their neighbours'
@@ -11,8 +11,8 @@ come in two forms: waves that share K and own all rows (few rows; the q/k/v and
 o_proj products, logits of up to 3 rows and narrow float32 results), and waves that
 own columns and share the rows through LDS (the SiLU-gate product up to 96 rows, every
 product whose K is cut, logits of 4 to 96 rows).
-bfloat16 with more rows, and from ``FEW_TILE_ROWS`` rows on where they are the faster ones (``cut_tiles``, ``part_tiles``,
-``gate_tiles``): tiles of this package's own (``csrc/gemm_direct.hip``, and
+bfloat16 with more rows, and from ``FEW_TILE_ROWS`` or 17 rows on (``cut_tiles``, ``gate_tiles``;
+``part_tiles``): tiles of this package's own (``csrc/gemm_direct.hip``, and
 ``csrc/gemm_tiles.hip`` for a K that is no multiple of 64) where they are the faster ones, else the
 vendor library's product (hipBLASLt through a thin cached interface of this
 package), as the reference leaves its products to a library
@@ -41,10 +41,6 @@ FUSED_ROWS = 16
 # 36.3 / 39.8 / 48.2 against 50.0 / 61.6 / 60.9: the library has no good algorithm for a long K and few rows, and at
 # row counts that do not recur it takes its heuristic's first choice)
 FUSED_PARTS_ROWS = 128
-# Rows up to which a float32 product takes the norm in front, the rotation or the add into the stream along (its kernels take
-# 16: every workgroup then makes the norm of as many rows).  Decode steps of 12 layers, kernels of their own and joined, us: 3B
-# 4 sequences, eight steps 12,061, 11,211; 0.5B 8 sequences, four steps 3,586, 3,442; 16 sequences 3,757, 3,770.
-F32_JOINED_ROWS = 8
 # With 17 to 128 rows it also wins where the weight is small (q/k/v and o_proj of the 3B shape: 7-9 us against
 # the library's 12-18 us inside a step at up to 64 rows, 9.3 and 8.2 us against 9.5-12.4 and 9.1 us at 72 and 128
 # rows, where the weight is streamed twice; and the rotation, the cache write, the residual add and the next
@@ -509,7 +505,7 @@ class RawRows:
     def fits(residual: torch.Tensor, dtype: torch.dtype) -> bool:
         rows, width = residual.shape
         if dtype == torch.float32:
-            return rows <= F32_JOINED_ROWS and ops.folds_norm_f32(residual)
+            return ops.folds_norm_f32(residual)
         return dtype == torch.bfloat16 and residual.is_cuda and ops.folds_norm(rows, width)
 
     @property
@@ -610,7 +606,7 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
         x = x.complete()
     if isinstance(x, RawRows):
         if epilogue == "silu" and weight.shape[0] % 2 == 0 and bias is None and into is None and x.joins_f32(weight):
-            return ops.gemm_f32_normed(x.residual, x.norm.weight_f32, x.norm.eps, weight, gate=True)
+            return ops.gemm_f32_normed(x.residual, x.norm.weight_f32, x.norm.eps, weight)
         x = x.complete()
     rows, k = x.shape
     n = weight.shape[0]
@@ -699,7 +695,7 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
     if weight.dtype == torch.float32:
         if silu and n % 2 == 0 and bias is None:
             return ops.gemm_f32(x, weight, gate=True)
-        if (into is not None and not silu and 1 <= rows <= F32_JOINED_ROWS and into.is_cuda and into.dtype == torch.float32
+        if (into is not None and not silu and 1 <= rows <= ops.F32_FEW_ROWS and into.is_cuda and into.dtype == torch.float32
                 and into.is_contiguous() and tuple(into.shape) == (rows, n)):
             ops.gemm_f32_into(x, weight, bias, into)  # (the next norm need not add it: it may ride in the product behind it)
             return Added()

@@ -123,12 +123,12 @@ def test_gemm_f32_forms(ops, shape):
 
 # (rows, columns, K): a part of a piece, segments of 512 numbers that are full and not, four and eight waves, one and several
 # rounds of blocks, narrow, middle and wide workgroups (with the gate columns of either half past the last), the widest rows
-@pytest.mark.parametrize("shape", [(1, 64, 8), (3, 384, 64), (8, 2560, 896), (9, 130, 1032), (4, 16384, 520), (13, 16386, 1104),
-                                   (2, 48, 8192), (16, 48, 2048), (3, 100, 4104), (8, 16448, 2048),
-                                   (16, 16386, 1000), (2, 22, 512)])
+@pytest.mark.parametrize("shape", [(1, 64, 8), (3, 384, 64), (8, 2560, 896), (7, 130, 1032), (4, 16384, 520), (6, 16386, 1104),
+                                   (2, 48, 8192), (8, 48, 2048), (3, 100, 4104), (8, 16448, 2048),
+                                   (8, 16386, 1000), (2, 22, 512), (5, 64, 4096)])
 def test_gemm_f32_with_its_neighbours(ops, shape):
-    """The float32 product of few rows that makes the norm in front of it, or adds into the stream, gives the bits of the
-    kernels that it takes the place of."""
+    """The gated float32 product of few rows that makes the norm in front of it, and the one that adds into the stream, give the bits
+    of the kernels that they take the place of."""
     m, n, k = shape
     x, w, b = rand((m, k), torch.float32, 71, 3.0), rand((n, k), torch.float32, 72), rand((n,), torch.float32, 73)
     x *= torch.linspace(0.01, 5.0, m, device="cuda")[:, None]
@@ -138,9 +138,7 @@ def test_gemm_f32_with_its_neighbours(ops, shape):
         assert not ops.folds_norm_f32(x)
     else:
         normed = ops.add_rmsnorm(x.clone(), None, gain, eps, torch.float32)
-        assert torch.equal(ops.gemm_f32_normed(x, gain, eps, w, b), ops.gemm_f32(normed, w, b, form=0))
-        assert torch.equal(ops.gemm_f32_normed(x, gain, eps, w), ops.gemm_f32(normed, w, form=0))
-        assert torch.equal(ops.gemm_f32_normed(x, gain, eps, w, gate=True), ops.gemm_f32(normed, w, gate=True, form=0))
+        assert torch.equal(ops.gemm_f32_normed(x, gain, eps, w), ops.gemm_f32(normed, w, gate=True, form=0))
     assert torch.equal(x, before)
     wide = torch.zeros((m, k + 3)).cuda()
     wide[:, :k] = x
@@ -153,17 +151,17 @@ def test_gemm_f32_with_its_neighbours(ops, shape):
 
 def test_gemm_f32_with_its_neighbours_refuses(ops):
     w, gain = torch.zeros((16, 64), device="cuda"), torch.ones(64, device="cuda")
-    for stream in (torch.zeros((17, 64), device="cuda"), torch.zeros((0, 64), device="cuda"), torch.zeros((4, 128), device="cuda")[:, ::2],
+    for stream in (torch.zeros((9, 64), device="cuda"), torch.zeros((0, 64), device="cuda"), torch.zeros((4, 128), device="cuda")[:, ::2],
                    torch.zeros(4 * 64 + 1, device="cuda")[1:].view(4, 64)):
         assert not ops.folds_norm_f32(stream)
         with pytest.raises(ValueError, match="makes the norm"):
             ops.gemm_f32_normed(stream, gain, 1e-6, w)
-    with pytest.raises(ValueError, match="up to 16 rows"):
-        ops.gemm_f32_into(torch.zeros((17, 64), device="cuda"), w, None, torch.zeros((17, 16), device="cuda"))
+    with pytest.raises(ValueError, match="up to 8 rows"):
+        ops.gemm_f32_into(torch.zeros((9, 64), device="cuda"), w, None, torch.zeros((9, 16), device="cuda"))
 
 
 @pytest.mark.parametrize("geometry", [(16, 2, 128, 16, 2048), (4, 2, 16, 8, 64), (3, 1, 64, 4, 328), (5, 5, 96, 32, 200), (2, 1, 48, 1, 1040)])
-@pytest.mark.parametrize("rows", [1, 3, 8, 13, 16])
+@pytest.mark.parametrize("rows", [1, 3, 7, 8])
 @pytest.mark.parametrize("rotate,write,biased", [(True, True, True), (False, True, False), (True, False, True)])
 @pytest.mark.parametrize("part", [False, True])
 def test_gemm_f32_qkv_rope(ops, geometry, rows, rotate, write, biased, part):
@@ -172,7 +170,7 @@ def test_gemm_f32_qkv_rope(ops, geometry, rows, rotate, write, biased, part):
     if rows * -(-hidden // 512) > 32:
         rows = 32 // -(-hidden // 512)
     n = (q_heads + 2 * kv_heads) * head_dim
-    lengths = [40, 35, 100, 33, 64, 1, 17, 90, 41, 36, 101, 34, 65, 2, 18, 91][:rows]
+    lengths = [40, 35, 100, 33, 64, 1, 17, 90][:rows]
     k_pool, v_pool, table, slots, _ = build_cache(torch.float32, lengths, kv_heads, head_dim, page_size, seed=81)
     k_two, v_two = k_pool.clone(), v_pool.clone()
     x = rand((rows, hidden), torch.float32, 82, 2.0)
