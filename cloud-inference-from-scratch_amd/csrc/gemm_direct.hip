@@ -40,7 +40,8 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* lds_pointer;
 
-enum { DIRECT_BF16 = 0, DIRECT_SILU = 1, DIRECT_RESID = 2, DIRECT_PARTS = 3, DIRECT_ROPE = 4, DIRECT_ATOMIC = 5 };
+enum { DIRECT_BF16 = 0, DIRECT_SILU = 1, DIRECT_RESID = 2, DIRECT_PARTS = 3, DIRECT_ROPE = 4, DIRECT_ATOMIC = 5, DIRECT_SCALED = 6 };
+constexpr bool gates(int epilogue) { return epilogue == DIRECT_SILU || epilogue == DIRECT_SCALED; }
 
 constexpr int kSlice = 64;                   // k of a stage: 128 bytes of a row
 constexpr int kLdsBytes = 160 * 1024;
@@ -59,12 +60,12 @@ struct DirectRope {
 
 struct DirectArgs {
     const bf16_t *a, *w, *bias;
-    void* c;            // BF16, SILU: bf16 [M, ldc]; RESID, ATOMIC: the float32 stream; PARTS: float32 [parts, M, N]
+    void* c;            // BF16, SILU, SCALED: bf16 [M, ldc]; RESID, ATOMIC: the float32 stream; PARTS: float32 [parts, M, N]
     int M, N, K, lda, ldc;
     int k_per_part;     // a multiple of kSlice
     int row_blocks, tiles;
     DirectRope rope;    // ROPE only
-    // SILU, or null: partial sums of squares [M, sumsq_parts] of the rows of the stream that A is short of 1/rms of
+    // SCALED only: partial sums of squares [M, sumsq_parts] of the rows of the stream whose 1/rms A lacks
     const float* row_sumsq;
     int sumsq_parts;
     float eps;
@@ -77,9 +78,9 @@ __device__ __forceinline__ int chunk_at(int row, int c) { return row * 128 + 16 
 // lane ends with eight neighbouring columns and four lanes with 32.
 template <int EPI, int kN>
 __device__ __forceinline__ int column_of(int t, int i) {
-    constexpr int kOut = EPI == DIRECT_SILU ? kN / 2 : kN;
-    if (EPI == DIRECT_SILU) t /= 2;
-    if ((EPI == DIRECT_BF16 || EPI == DIRECT_SILU) && kOut % 2 == 0) return t / 2 * 32 + i / 4 * 8 + t % 2 * 4 + i % 4;
+    constexpr int kOut = gates(EPI) ? kN / 2 : kN;
+    if (gates(EPI)) t /= 2;
+    if ((EPI == DIRECT_BF16 || gates(EPI)) && kOut % 2 == 0) return t / 2 * 32 + i / 4 * 8 + t % 2 * 4 + i % 4;
     return 16 * t + i;
 }
 
@@ -192,6 +193,12 @@ __device__ __forceinline__ void wait_for_all_but() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kYounger) : "memory");
 }
 
+// The stages, and behind them each row's scale.
+template <int EPI>
+constexpr int lds_bytes(int columns, int rows, int stages) {
+    return stages * (columns + rows) * 128 + (EPI == DIRECT_SCALED ? rows * static_cast<int>(sizeof(float)) : 0);
+}
+
 // kN x kM tiles of 16 columns x 16 rows per wave, kWN waves side by side along the columns and kWM along the rows.
 template <int EPI, int kWN, int kWM, int kN, int kM, int kStages>
 __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectArgs p) {
@@ -202,8 +209,8 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
     constexpr int kPieces = (kColumns + kTileRows) / 8;         // loads of 8 rows that a stage takes
     constexpr int kLoads = (kPieces + kWaves - 1) / kWaves;     // ... of a wave; some waves have one fewer
     constexpr int kUneven = kPieces % kWaves;                   // (the first so many waves have kLoads, if it is not 0)
-    constexpr int kStep = EPI == DIRECT_SILU ? kColumns / 2 : kColumns;
-    static_assert(kStages >= 2 && kStages * kStageBytes <= kLdsBytes && (EPI != DIRECT_SILU || kN % 2 == 0) && (EPI != DIRECT_ROPE || kN % 2 == 0), "");
+    constexpr int kStep = gates(EPI) ? kColumns / 2 : kColumns;
+    static_assert(kStages >= 2 && lds_bytes<EPI>(kColumns, kTileRows, kStages) <= kLdsBytes && (!gates(EPI) || kN % 2 == 0) && (EPI != DIRECT_ROPE || kN % 2 == 0), "");
     extern __shared__ __attribute__((aligned(1024))) char stages[];
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -214,7 +221,7 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
     if (static_cast<int>(blockIdx.x) / 8 >= per || tile >= p.tiles) return;
     const int m0 = (tile % p.row_blocks) * kTileRows;
     const int n0 = (tile / p.row_blocks) * kStep;
-    const int width = EPI == DIRECT_SILU ? p.N / 2 : p.N;
+    const int width = gates(EPI) ? p.N / 2 : p.N;
     const int k_first = blockIdx.y * p.k_per_part;
     const int slices = (min(p.K, k_first + p.k_per_part) - k_first) / kSlice;
 
@@ -228,7 +235,7 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
         if (row < kColumns) {
             const int t = row % (16 * kN) / 16, j = row % 16;
             int n;
-            if (EPI == DIRECT_SILU) {
+            if (gates(EPI)) {
                 n = min(n0 + row / (16 * kN) * 8 * kN + column_of<EPI, kN>(t, j), width - 1) + t % 2 * width;
             } else if (EPI == DIRECT_ROPE) {  // 16 dimensions of a head's first half, then the 16 they rotate with
                 const int per_head = p.rope.head_dim / 32, pair = min((n0 + row) / 32, p.N / 32 - 1);
@@ -255,7 +262,7 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
     };
 
     // The rows' 1/rms: behind the first loads, some lanes to a row, eight pieces each at a time
-    __shared__ float row_scale[EPI == DIRECT_SILU ? kTileRows : 1];
+    float* row_scale = reinterpret_cast<float*>(stages + kStages * kStageBytes);  // (SCALED only)
     auto scale_rows = [&] __attribute__((always_inline)) {
         constexpr int kSpare = 64 * kWaves / kTileRows, kPer = kSpare >= 8 ? 8 : kSpare >= 4 ? 4 : 2, kHeld = 8;
         static_assert(kSpare >= 2, "");
@@ -341,9 +348,7 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
     if (many)
 #pragma unroll
         for (int i = 0; i < kFirst; ++i) fetch_one(i, kStages - 1, kStages - 1);
-    if constexpr (EPI == DIRECT_SILU) {
-        if (p.row_sumsq) scale_rows();
-    }
+    if constexpr (EPI == DIRECT_SCALED) scale_rows();
     if (many) {
         if (uneven_more) wait_for_all_but<kAhead * kLoads + kFirst>();
         else wait_for_all_but<kAhead * kFewer + (kFirst < kFewer ? kFirst : kFewer)>();
@@ -401,24 +406,23 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
         }
         return;
     }
-    if constexpr (EPI == DIRECT_SILU) {
-        if (p.row_sumsq)
+    if constexpr (EPI == DIRECT_SCALED) {
 #pragma unroll
-            for (int im = 0; im < kM; ++im) {
-                const float scale = row_scale[wm - kColumns + 16 * im + lane % 16];
+        for (int im = 0; im < kM; ++im) {
+            const float scale = row_scale[wm - kColumns + 16 * im + lane % 16];
 #pragma unroll
-                for (int in = 0; in < kN; ++in) acc[in][im] *= scale;
-            }
+            for (int in = 0; in < kN; ++in) acc[in][im] *= scale;
+        }
     }
-    constexpr int kOut = EPI == DIRECT_SILU ? kN / 2 : kN;
-    constexpr int kPair = (EPI == DIRECT_BF16 || EPI == DIRECT_SILU) && kOut % 2 == 0 ? 2 : 1;  // tiles whose columns are neighbours
-    const int first = n0 + (EPI == DIRECT_SILU ? wn / 2 : wn);
+    constexpr int kOut = gates(EPI) ? kN / 2 : kN;
+    constexpr int kPair = (EPI == DIRECT_BF16 || gates(EPI)) && kOut % 2 == 0 ? 2 : 1;  // tiles whose columns are neighbours
+    const int first = n0 + (gates(EPI) ? wn / 2 : wn);
 #pragma unroll
     for (int u = 0; u < kOut; u += kPair) {
-        const int n = first + column_of<EPI, kN>(EPI == DIRECT_SILU ? 2 * u : u, lane / 16 * 4);
+        const int n = first + column_of<EPI, kN>(gates(EPI) ? 2 * u : u, lane / 16 * 4);
         const bool whole = n + 4 * kPair <= width;
         float b[4 * kPair] = {};
-        if (EPI != DIRECT_SILU && p.bias && blockIdx.y == 0)
+        if (!gates(EPI) && p.bias && blockIdx.y == 0)
 #pragma unroll
             for (int i = 0; i < 4 * kPair; ++i) b[i] = to_float(p.bias[min(n + i, width - 1)]);
 #pragma unroll
@@ -428,13 +432,13 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
             float v[4 * kPair];
 #pragma unroll
             for (int i = 0; i < 4 * kPair; ++i) {
-                if constexpr (EPI == DIRECT_SILU) {
+                if constexpr (gates(EPI)) {
                     v[i] = gate_of(acc[2 * (u + i / 4)][im][i % 4]) * acc[2 * (u + i / 4) + 1][im][i % 4];
                 } else {
                     v[i] = acc[u + i / 4][im][i % 4] + b[i];
                 }
             }
-            if constexpr (EPI == DIRECT_BF16 || EPI == DIRECT_SILU) {
+            if constexpr (EPI == DIRECT_BF16 || gates(EPI)) {
                 bf16_t* to = static_cast<bf16_t*>(p.c) + static_cast<size_t>(m) * p.ldc + n;
                 if (!whole || p.ldc % 2) {
 #pragma unroll
@@ -485,7 +489,7 @@ __global__ void __launch_bounds__(64 * kWN * kWM, 2) gemm_direct_kernel(DirectAr
 template <int EPI, int kWN, int kWM, int kN, int kM, int kStages>
 int run(hipStream_t s, DirectArgs& p, int parts) {
     constexpr int kColumns = 16 * kN * kWN, kTileRows = 16 * kM * kWM;
-    constexpr int kBytes = kStages * (kColumns + kTileRows) * 128;
+    constexpr int kBytes = lds_bytes<EPI>(kColumns, kTileRows, kStages);
     if (kBytes > 64 * 1024) {  // more than a kernel gets without asking: once per kernel (and again is harmless)
         static bool asked = false;
         if (!asked) {
@@ -497,14 +501,27 @@ int run(hipStream_t s, DirectArgs& p, int parts) {
             asked = true;
         }
     }
-    const int step = EPI == DIRECT_SILU ? kColumns / 2 : kColumns;
-    const int width = EPI == DIRECT_SILU ? p.N / 2 : p.N;
+    const int step = gates(EPI) ? kColumns / 2 : kColumns;
+    const int width = gates(EPI) ? p.N / 2 : p.N;
     p.row_blocks = (p.M + kTileRows - 1) / kTileRows;
     const long tiles = static_cast<long>(p.row_blocks) * ((width + step - 1) / step);
     if (tiles > (1L << 27)) return CIE_BAD_ARGUMENT;
     p.tiles = static_cast<int>(tiles);
     gemm_direct_kernel<EPI, kWN, kWM, kN, kM, kStages><<<dim3((p.tiles + 7) / 8 * 8, parts), 64 * kWN * kWM, kBytes, s>>>(p);
     return cie_after_launch();
+}
+
+// Tiles of up to 128 columns and rows: all there are for parts that add atomically and for rows that are scaled.
+template <int EPI>
+int run_few_form(hipStream_t s, DirectArgs& p, int parts, int columns, int rows) {
+    switch (columns * 1000 + rows) {
+        case 128128: return run<EPI, 2, 4, 4, 2, 4>(s, p, parts);
+        case 128064: return run<EPI, 4, 2, 2, 2, 3>(s, p, parts);
+        case 96128: return run<EPI, 1, 8, 6, 1, 5>(s, p, parts);
+        case 96064: return run<EPI, 1, 4, 6, 1, 4>(s, p, parts);
+        case 64064: return run<EPI, 2, 2, 2, 2, 4>(s, p, parts);
+    }
+    return CIE_BAD_ARGUMENT;
 }
 
 template <int EPI>
@@ -518,13 +535,8 @@ int run_form(hipStream_t s, DirectArgs& p, int parts, int columns, int rows) {
         case 192128: return run<EPI, 2, 4, 6, 2, 3>(s, p, parts);
         case 128256: return run<EPI, 2, 4, 4, 4, 3>(s, p, parts);
         case 128192: return run<EPI, 2, 4, 4, 3, 3>(s, p, parts);
-        case 128128: return run<EPI, 2, 4, 4, 2, 4>(s, p, parts);
-        case 128064: return run<EPI, 4, 2, 2, 2, 3>(s, p, parts);
-        case 96128: return run<EPI, 1, 8, 6, 1, 5>(s, p, parts);
-        case 96064: return run<EPI, 1, 4, 6, 1, 4>(s, p, parts);
-        case 64064: return run<EPI, 2, 2, 2, 2, 4>(s, p, parts);
     }
-    return CIE_BAD_ARGUMENT;
+    return run_few_form<EPI>(s, p, parts, columns, rows);
 }
 
 bool fits(const void* a, int lda, const void* w, const void* c, int M, int N, int K) {
@@ -537,7 +549,7 @@ bool fits(const void* a, int lda, const void* w, const void* c, int M, int N, in
 }  // namespace
 
 // epilogue: 0 bf16, 1 SiLU-gate (N even, no bias), 2 residual (c float32 [M, N]), 3 parts (c float32 [parts, M, N]), 5 parts
-// that add their shares into c (float32 [M, N]) with atomic adds.
+// that add their shares into c (float32 [M, N]) with atomic adds (tiles of up to 128 columns and 128 rows).
 // `columns` x `rows`: the workgroup's tile of the product (with the gate: half of the columns of either half).
 // K is a multiple of 64, lda of 8; a, w and c lie at multiples of 16 bytes; the operands hold fewer than 2^31 numbers.
 CIE_API int cie_gemm_direct(void* stream, const void* a, int lda, const void* w, const void* bias, void* c, int ldc, int M,
@@ -554,20 +566,20 @@ CIE_API int cie_gemm_direct(void* stream, const void* a, int lda, const void* w,
         case DIRECT_SILU: return run_form<DIRECT_SILU>(s, p, parts, columns, rows);
         case DIRECT_RESID: return run_form<DIRECT_RESID>(s, p, parts, columns, rows);
         case DIRECT_PARTS: return run_form<DIRECT_PARTS>(s, p, parts, columns, rows);
-        case DIRECT_ATOMIC: return run_form<DIRECT_ATOMIC>(s, p, parts, columns, rows);
+        case DIRECT_ATOMIC: return run_few_form<DIRECT_ATOMIC>(s, p, parts, columns, rows);
     }
     return CIE_BAD_ARGUMENT;
 }
 
 // The SiLU-gate product of rows `a` = bf16(row of the stream x norm weight), whose 1/rms it applies to its sums: `row_sumsq` [M,
-// sumsq_parts] are partial sums of squares of the stream's rows (of K numbers).
+// sumsq_parts] are partial sums of squares of the stream's rows (of K numbers).  Tiles of up to 128 columns and 128 rows.
 CIE_API int cie_gemm_direct_silu_scaled(void* stream, const void* a, int lda, const void* w, void* c, int ldc, int M, int N, int K,
                                         int columns, int rows, const float* row_sumsq, int sumsq_parts, float eps) {
     if (!fits(a, lda, w, c, M, N, K) || N % 2 || ldc < N / 2 || !row_sumsq || sumsq_parts < 1 || !(eps > 0.f) ||
         (reinterpret_cast<uintptr_t>(row_sumsq) & 15) != 0)
         return CIE_BAD_ARGUMENT;
     DirectArgs p{static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(w), nullptr, c, M, N, K, lda, ldc, K, 0, 0, {}, row_sumsq, sumsq_parts, eps};
-    return run_form<DIRECT_SILU>(static_cast<hipStream_t>(stream), p, 1, columns, rows);
+    return run_few_form<DIRECT_SCALED>(static_cast<hipStream_t>(stream), p, 1, columns, rows);
 }
 
 // The q/k/v product with the rotation and the cache write in its epilogue: `w` [N, K] stacks the rows of q_heads query

@@ -971,6 +971,7 @@ TILE_SHAPES = ((64, 64), (128, 64), (128, 128), (128, 256))  # columns x rows of
 # ... of the kernel whose operands go straight into LDS (K a multiple of 64)
 DIRECT_SHAPES = ((64, 64), (96, 64), (96, 128), (128, 64), (128, 128), (128, 192), (128, 256), (192, 128), (192, 192),
                  (192, 256), (256, 128), (256, 160), (256, 256))
+DIRECT_FEW_SHAPES = DIRECT_SHAPES[:5]  # ... where its parts add atomically, or its rows are scaled
 DIRECT_SLICE = 64
 DIRECT_NUMBERS = 1 << 31  # an operand holds fewer numbers (their places are 32-bit numbers of bytes)
 
@@ -995,8 +996,8 @@ def _tile_rows(a: torch.Tensor, weight: torch.Tensor) -> tuple[int, int, int, in
     return m, n, k, lda
 
 
-def _check_tile_shape(columns: int, rows: int, direct: bool, m: int, n: int, k: int, lda: int) -> None:
-    shapes = DIRECT_SHAPES if direct else TILE_SHAPES
+def _check_tile_shape(columns: int, rows: int, direct: bool, m: int, n: int, k: int, lda: int, few: bool = False) -> None:
+    shapes = DIRECT_FEW_SHAPES if few else DIRECT_SHAPES if direct else TILE_SHAPES
     if (columns, rows) not in shapes:
         raise ValueError(f"tiles are one of {shapes}, not {(columns, rows)}")
     if direct and not direct_fits(m, n, k, lda):
@@ -1014,7 +1015,7 @@ def gemm_tiles(weight: torch.Tensor, epilogue: int, a: torch.Tensor, columns: in
     if epilogue == TILE_ATOMIC and not direct:
         raise ValueError("parts add themselves into the stream only in the kernel that loads straight into LDS")
     m, n, k, lda = _tile_rows(a, weight)
-    _check_tile_shape(columns, rows, direct, m, n, k, lda)
+    _check_tile_shape(columns, rows, direct, m, n, k, lda, epilogue == TILE_ATOMIC)
     if bias is not None:
         _gpu("bias", bias, torch.bfloat16, 1)
         if not (bias.shape[0] == n and epilogue != TILE_SILU):
@@ -1040,7 +1041,7 @@ def gemm_tiles_silu_scaled(weight: torch.Tensor, a: torch.Tensor, columns: int, 
     """The gated unit of :func:`gemm_tiles` (``direct``) of rows that lack their 1/rms, which it applies to its sums:
     ``row_sumsq`` [M, parts] holds partial sums of squares of the stream's rows (as ``gemm_fused`` takes them)."""
     m, n, k, lda = _tile_rows(a, weight)
-    _check_tile_shape(columns, rows, True, m, n, k, lda)
+    _check_tile_shape(columns, rows, True, m, n, k, lda, True)
     _gpu("row_sumsq", row_sumsq, torch.float32, 2)
     if not (n % 2 == 0 and row_sumsq.shape[0] == m and row_sumsq.shape[1] >= 1 and eps > 0 and row_sumsq.data_ptr() % 16 == 0):
         raise ValueError(f"row_sumsq {tuple(row_sumsq.shape)} does not fit {m} rows, or the weight's {n} rows are no pairs")

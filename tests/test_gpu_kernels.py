@@ -354,6 +354,8 @@ def test_gemm_direct_of_few_rows(ops, shape, tile):
         close_to_gated_unit(ops.gemm_tiles_silu_scaled(w, a, *tile, sumsq, 1e-5), a, w, scale, sums)
     with pytest.raises(ValueError, match="straight into LDS"):
         ops.gemm_tiles(w, ops.TILE_ATOMIC, a, 64, 64, into=stream, parts=1)
+    with pytest.raises(ValueError, match="tiles are one of"):
+        ops.gemm_tiles(w, ops.TILE_ATOMIC, a, 256, 128, into=stream, parts=1, direct=True)
 
 
 @pytest.mark.parametrize("rows", [17, 47, 48, 64, 65, 96, 128])

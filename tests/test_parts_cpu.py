@@ -235,7 +235,7 @@ def test_tiles_of_few_rows_meet_the_units_once(rows, n, k, most):
         assert min(-(-n // 128) * -(-rows // r) for r in ((64,) if rows <= 64 else (64, 128))) > 256
         return
     columns, tile_rows, parts = form
-    assert (columns, tile_rows) in ops.DIRECT_SHAPES and parts <= most
+    assert (columns, tile_rows) in ops.DIRECT_FEW_SHAPES and parts <= most
     assert -(-n // columns) * -(-rows // tile_rows) * parts <= 256
     assert -(-(-(-k // parts)) // 64) * 64 * (parts - 1) < k  # (no part without k)
     assert -(-(-(-n // columns) * -(-rows // tile_rows)) // 8) * parts <= 32  # (and an eighth of the tiles an eighth of the units)
