@@ -198,6 +198,10 @@ EIGHT_WAVE_TILES = 0.75  # of the compute units
 # 10.5, 10.9, behind 1,000 25.4, 18.4).
 ALONE_TILES = 0.55  # of the compute units
 ALONE_TILE_KEYS = 96_000
+# (A window's keys are not cut, and few tiles then have few workgroups: with pages of 16, whose table the form through LDS reads
+# for every 16 keys, it is 9 % slower in the mean of 46 such batches, 135 tokens of 12 heads on 2 under a window of 4,096 73.7, 89.8;
+# with larger pages 5 to 34 % faster in 46.)
+WINDOW_PAGE = 32
 LARGE_TILES_ABOVE = 1.0  # tiles of 128 rows x kv heads (as a share of the compute units) above which that form takes them
 
 
@@ -264,7 +268,8 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
     # Prompt portions with enough rows take tiles of 128 rows and eight waves, whose keys and values pass
     # through LDS once per tile.  (A short portion behind a long context also has its keys cut into parts.)
     prompt_tokens, prompt_keys, singles = batch.portions
-    prompt_keys = prompt_keys if window is None else min(prompt_keys, window + 64)
+    if window is not None:
+        prompt_keys = min(prompt_keys, window + 64) if page_size >= WINDOW_PAGE else 0
     bound = batch.static_plan.max_keys if batch.static_plan is not None else max_keys
     cuts = max(1, bound // PROMPT_SPLIT_KEYS) if wide and window is None else 1  # (a window's keys stay whole)
     big_tiles = -(-prompt_tokens * group // 128) * num_kv_heads

@@ -191,15 +191,15 @@ def test_which_portions_take_the_form_through_lds():
     assert not takes_prompt_form(0, 100_000, 0, False, 256)
 
 
-@pytest.mark.parametrize("window", [None, 1024])
+@pytest.mark.parametrize("window,page", [(None, 16), (1024, 32), (1024, 16)])
 @pytest.mark.parametrize("singles,single_start,portion,portion_start,through_lds", [
     (40, 3999, 200, 0, False),    # 50 tiles over 200 keys: the 40 tokens' 4,000 keys are not theirs
     (40, 99, 200, 1800, True),    # ... over 2,000
     (40, 99, 200, 1700, False),   # (95,000 tiles x keys)
     (0, 0, 200, 1800, True), (0, 0, 400, 1000, True)])
-def test_the_keys_of_the_portions_choose_their_form(monkeypatch, window, singles, single_start, portion, portion_start, through_lds):
+def test_the_keys_of_the_portions_choose_their_form(monkeypatch, window, page, singles, single_start, portion, portion_start, through_lds):
     """Single tokens beside the portions have a launch of their own here; their contexts do not choose the portions' form.  (A
-    window of 1,024 keys leaves the portions some 1,088.)"""
+    window of 1,024 keys leaves the portions some 1,088; with pages of 16 few tiles do not take the form for its keys.)"""
     from cie_amd.engine.batch import PagedView, StepBatch
     from cie_amd.kernels import ops
     from cie_amd.parts import attention
@@ -213,13 +213,13 @@ def test_the_keys_of_the_portions_choose_their_form(monkeypatch, window, singles
     batch = StepBatch(tokens=total, sequences=len(q_lens), token_ids=some, positions=some, seq_of_token=some, seq_slot=some,
                       seq_start=some, seq_q_len=some, q_start_loc=some, logit_rows=some, host_slots=list(range(len(q_lens))),
                       host_starts=starts, host_q_lens=q_lens)
-    pool = torch.zeros((1, 2, 16, 128), dtype=torch.bfloat16)
-    view = PagedView(pool, pool.transpose(2, 3), some[None], 16)
+    pool = torch.zeros((1, 2, page, 128), dtype=torch.bfloat16)
+    view = PagedView(pool, pool.transpose(2, 3), some[None], page)
     attention.attend(torch.zeros((total, 20 * 128), dtype=torch.bfloat16), batch, view, 16, 2, 128, window, 0.1)
     keys = portion_start + portion if window is None else min(portion_start + portion, window + 64)
     tiles = -(-portion * 8 // 64) * 2
     if window is not None:
-        through_lds = tiles >= 0.55 * 256 or tiles * keys >= 96_000
+        through_lds = tiles >= 0.55 * 256 or (page == 32 and tiles * keys >= 96_000)
     assert [w for tokens, w in waves if tokens > 1] == [ops.PROMPT_WAVES if through_lds else ops.TILE_WAVES]
 
 
