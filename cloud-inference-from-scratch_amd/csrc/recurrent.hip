@@ -968,8 +968,9 @@ gated_recurrence_kernel(const T* __restrict__ y_pre, long ldy, const T* __restri
 // layer's gates are 2 MB): a wave's slices and what the step itself needs are all asked for before the first product,
 // and a lane of one wave that moved the four states whose gates it held spent 0.65 us on each, one after the other.
 // In place of the product and the walk, 8 blocks of 256: one sequence 6.6 -> 4.2 us, eight 7.2 -> 4.3, 64 11.4 -> 6.5.  From
-// some eight workgroups a unit on every 16 sequences' new reading of the weights costs more than the launch (16 blocks, 128
-// sequences 15.8 -> 16.7; at five a unit 13.5 -> 12.4): kernels/ops.py draws the line between.
+// four to six workgroups a unit on, by the blocks' width, every 16 sequences' new reading of the weights costs more than the launch
+// (16 blocks of 256, 128 sequences 15.9 -> 16.9; at five a unit 14.0 -> 13.2; 20 blocks of 128 11.7 -> 13.5): kernels/ops.py
+// draws the line.
 typedef __bf16 gate_piece_t __attribute__((ext_vector_type(8)));
 constexpr int kGateSlices = 4;  // of 32 k under way at once, a wave
 constexpr int kStepTaps = 4;    // inputs kept beside the token's own, at most (longer convolutions take the general path)

@@ -1672,15 +1672,20 @@ def gated_recurrence(y_pre: torch.Tensor, x_in: torch.Tensor, u: torch.Tensor, g
 
 
 SCAN_STEP_TAPS = 5         # of a convolution in front of the kernel of single tokens, at most
-SCAN_STEP_WORKGROUPS = 5   # ... and workgroups of 16 channels and 16 sequences a compute unit (csrc/recurrent.hip)
+# ... and workgroups of 16 channels and 16 sequences a compute unit: blocks of up to so many numbers have little K for what a
+# fifth costs (us, the two kernels and this one: 20 blocks of 128, 4.4 a unit 11.0, 12.1, 5 11.7, 13.5; 16 blocks of 128, 4 a unit
+# 10.8, 10.0, 5 11.4, 12.8; 32 blocks of 64 10.8, 10.0 and 11.9, 13.1; 8 blocks of 256 12.7, 10.1 and 13.5, 13.1, 6 a unit 14.3,
+# 14.5; 16 of 160 5 a unit 13.7, 10.6; 4 of 640 21.3, 19.2, 6.3 a unit 22.5, 24.5)
+SCAN_STEP_WORKGROUPS, SCAN_STEP_NARROW, SCAN_STEP_WORKGROUPS_NARROW = 5, 128, 4
 
 
 def steps_gated_recurrence(u: torch.Tensor, weight: torch.Tensor, sequences: int, block_width: int, taps: int) -> bool:
     """Whether the kernel that makes the gates and moves the states of single tokens is the faster one for these and takes
     them: bfloat16, blocks in 16-byte pieces."""
     groups = u.shape[1] // block_width * -(-block_width // 16) * -(-sequences // 16)
+    most = SCAN_STEP_WORKGROUPS if block_width > SCAN_STEP_NARROW else SCAN_STEP_WORKGROUPS_NARROW
     return (u.dtype == torch.bfloat16 and weight.dtype == u.dtype and block_width % 8 == 0 and taps <= SCAN_STEP_TAPS
-            and groups <= SCAN_STEP_WORKGROUPS * compute_units() and u.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+            and groups <= most * compute_units() and u.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
 def gated_recurrence_step(y_pre: torch.Tensor, x_in: torch.Tensor, u: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,

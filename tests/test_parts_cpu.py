@@ -268,3 +268,16 @@ def test_tiles_of_few_rows_cut_a_short_k_little():
     from cie_amd.parts.linear import plan_few_tiles
 
     assert plan_few_tiles(96, 4096, 4096, 8, 256)[2] <= 4
+
+
+@pytest.mark.parametrize("blocks,width,sequences,takes", [
+    (16, 128, 128, True), (16, 128, 129, False), (20, 128, 128, False), (32, 64, 128, True), (40, 64, 112, False),
+    (8, 256, 160, True), (8, 256, 161, False), (16, 160, 128, True), (4, 640, 128, True)])
+def test_which_steps_of_single_tokens_make_their_gates_themselves(monkeypatch, blocks, width, sequences, takes):
+    """Up to four workgroups a unit for blocks of up to 128 numbers, up to five for wider ones."""
+    from cie_amd.kernels import ops
+
+    monkeypatch.setattr(ops, "compute_units", lambda *_: 256)
+    u = torch.zeros((sequences, blocks * width), dtype=torch.bfloat16)
+    weight = torch.zeros((blocks, 2 * width, width), dtype=torch.bfloat16)
+    assert ops.steps_gated_recurrence(u, weight, sequences, width, 4) == takes
