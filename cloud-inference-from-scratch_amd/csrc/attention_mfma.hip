@@ -845,6 +845,8 @@ int launch_for_dim(hipStream_t s, const AttentionArgs& a, int n_tiles, int row_t
 // Workspace sizes (floats) the caller provides when n_splits > 1:
 //   part_o  n_tiles * kv_heads * n_splits * 16*row_tiles * head_dim
 //   part_ml n_tiles * kv_heads * n_splits * 16*row_tiles * 2
+// merge: 0 leaves the shares there (whoever reads them merges them: csrc/merge_project.hip; not with tile_waves 8, whose tiles may
+// write their result themselves), and writes nothing to `out`.
 CIE_API int cie_paged_attention_mfma(void* stream, const void* q, int q_row_stride, const void* k_pool,
                                      const void* v_pool, const int* block_table, int table_width,
                                      const int* tile_seq, const int* tile_q0, const int* seq_slot,
@@ -852,7 +854,7 @@ CIE_API int cie_paged_attention_mfma(void* stream, const void* q, int q_row_stri
                                      void* out, float* part_o, float* part_ml, int n_tiles, int q_heads,
                                      int kv_heads, int head_dim, int page_size, int window, float scale,
                                      int n_splits, int tokens_per_tile, int row_tiles, int keys_per_split,
-                                     const int* max_context_dev, int tile_waves) {
+                                     const int* max_context_dev, int tile_waves, int merge) {
     if (n_tiles < 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads || page_size < 4 ||
         (page_size & (page_size - 1)) || table_width <= 0 || n_splits < 1 || n_splits > 65535 ||
         kv_heads > 65535 || tokens_per_tile < 1 || q_row_stride % 8)
@@ -860,6 +862,7 @@ CIE_API int cie_paged_attention_mfma(void* stream, const void* q, int q_row_stri
     const int group = q_heads / kv_heads;
     if (tokens_per_tile * group > 16 * row_tiles) return CIE_BAD_ARGUMENT;
     if (n_splits > kMergeMaxSplits) return CIE_BAD_ARGUMENT;
+    if (!merge && (n_splits == 1 || tile_waves == kPromptWaves)) return CIE_BAD_ARGUMENT;
     // the prompt form takes maxima before scaling, which needs a positive scale, and keeps the 16 keys of a
     // product in one page
     if (tile_waves != 1 && ((tile_waves != kTileWaves && tile_waves != kPromptWaves) || !(scale > 0.f) || page_size < 16))
@@ -916,6 +919,6 @@ CIE_API int cie_paged_attention_mfma(void* stream, const void* q, int q_row_stri
         case 256: rc = launch_for_dim<256>(s, a, n_tiles, row_tiles, tile_waves); break;
         default: return CIE_BAD_ARGUMENT;
     }
-    if (rc != CIE_OK || n_splits == 1) return rc;
+    if (rc != CIE_OK || n_splits == 1 || !merge) return rc;
     return launch_merge(s, a, n_tiles, head_dim, 16 * row_tiles);
 }

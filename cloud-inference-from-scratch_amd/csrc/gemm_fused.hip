@@ -81,7 +81,7 @@ struct FusedArgs {
     const float* row_sumsq;    // SILU: [M, sumsq_parts] or null
     int sumsq_parts;
     float eps;
-    // ROPE with the norm in front of it folded in (up to 16 rows): the rows of A are not read but made here, as
+    // ROPE, or SILU in the second form, with the norm in front of it folded in (up to 16 rows): the rows of A are not read but made here, as
     // bf16(fold_residual * fold_weight), a lane making the very values its matrix operand holds, and the
     // product is multiplied by each row's 1/rms, whose sums of squares the lanes gather on the way.
     const float* fold_residual;  // [M, K] float32 or null
@@ -816,8 +816,14 @@ struct SharedRowsLds {
     static constexpr int kBytes = kStagesA * kStageBytesA + kRest;
 };
 
-template <int EPI, int MT, int NT, int WAVES>
+// FOLD: 0, or the rows (8 or 16) that are made from the float32 stream, the norm in front of the SiLU product folded in (see
+// FusedArgs): a thread's piece of a row is then eight numbers of the stream times the norm's weight, rounded on their way into LDS.
+// The weight's way from memory hides it (MI355X, us, rows short of their scale read and rows made here, 8 / 16 rows: 3B gate/up 18.0,
+// 18.1 / 18.0, 18.6; 0.5B 7.1, 7.3 / 7.1, 7.8; 14B 50.1, 50.5 / 50.2, 51.2; 7B, against the first form, 52.6, 54.0 / 56.4, 57.4, where
+// the first form with its norm folded in takes 54.8 / 67.3).
+template <int EPI, int MT, int NT, int WAVES, int FOLD = 0>
 __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs a) {
+    static_assert(FOLD == 0 || (EPI == EPI_SILU && MT == 1 && (FOLD == 8 || FOLD == 16)), "the folded norm: SiLU of one row tile");
     static_assert(EPI == EPI_SILU || EPI == EPI_PARTIAL || EPI == EPI_BF16 || EPI == EPI_F32 || EPI == EPI_ATOMIC,
                   "epilogues of this form");
     static_assert(EPI != EPI_SILU || NT == 2, "the SiLU epilogue pairs a gate tile with its up tile");
@@ -852,14 +858,18 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
     // the slice of A: thread t takes the piece (t % 16) of rows t / 16 + (threads / 16) i (a row past the
     // last one computes a copy that is not stored; past the last row tile, a thread repeats the last row)
     constexpr int kRowsPerPass = kThreads / 16;
-    constexpr int kPasses = (kRows + kRowsPerPass - 1) / kRowsPerPass;
+    constexpr int kMadeRows = FOLD > 0 ? FOLD : kRows;  // (row tiles' rows past these are whatever LDS holds: theirs are not stored)
+    constexpr int kPasses = (kMadeRows + kRowsPerPass - 1) / kRowsPerPass;
     const int a_row = threadIdx.x >> 4;
     const bf16_t* a_rows[kPasses];
+    const float* fold_rows[kPasses];
     int a_stage_row[kPasses];
 #pragma unroll
     for (int i = 0; i < kPasses; ++i) {
-        a_stage_row[i] = min(i * kRowsPerPass + a_row, kRows - 1);
-        a_rows[i] = a.a + static_cast<size_t>(min(a_stage_row[i], a.M - 1)) * a.lda;
+        a_stage_row[i] = min(i * kRowsPerPass + a_row, kMadeRows - 1);
+        const int row = min(a_stage_row[i], a.M - 1);
+        a_rows[i] = FOLD > 0 ? nullptr : a.a + static_cast<size_t>(row) * a.lda;
+        fold_rows[i] = FOLD > 0 ? a.fold_residual + static_cast<size_t>(row) * a.K : nullptr;
     }
     const int k_begin = blockIdx.z * a.k_per_part;
     const int k_end = min(a.K, k_begin + a.k_per_part);
@@ -871,9 +881,11 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
     // results the piece of W too).
     struct Slot {
         u32x4 w[NT][4];
-        u32x4 a[kPasses];
+        u32x4 a[FOLD > 0 ? 1 : kPasses];
+        floatx4 x[FOLD > 0 ? kPasses : 1][2], norm[2];  // FOLD: the pieces of the stream and of the norm's weight
     };
     Slot ring0, ring1;
+    float fold_sq[kPasses] = {};  // FOLD: this thread's share of its rows' sums of squares
     // Workgroups that walk K in step read the same k of many rows at a time.  Where the rows lie a multiple of 4 KB apart these
     // are lines of a few memory channels, so there each workgroup begins with another slice and ends with those before it
     // (3B gate/up, K 2,048, us: 8 rows 20.2 -> 17.7, 32 rows 20.9 -> 18.3, 64 rows 22.9 -> 22.0; K 5,120, whose rows spread by
@@ -889,8 +901,17 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
     };
     auto fetch = [&](Slot& into, int from) __attribute__((always_inline)) {
         const int k = min(from + load_col, k_end - 8);
+        if constexpr (FOLD > 0) {
 #pragma unroll
-        for (int i = 0; i < kPasses; ++i) into.a[i] = *reinterpret_cast<const u32x4*>(a_rows[i] + k);
+            for (int h = 0; h < 2; ++h) {
+                into.norm[h] = *reinterpret_cast<const floatx4*>(a.fold_weight + k + h * 4);
+#pragma unroll
+                for (int i = 0; i < kPasses; ++i) into.x[i][h] = *reinterpret_cast<const floatx4*>(fold_rows[i] + k + h * 4);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kPasses; ++i) into.a[i] = *reinterpret_cast<const u32x4*>(a_rows[i] + k);
+        }
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -911,9 +932,20 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
         if (kStagesA == 1) __syncthreads();  // every wave has read the slice before
         const bool inside = !kEnd || at + load_col < k_end;
 #pragma unroll
-        for (int i = 0; i < kPasses; ++i)
-            *reinterpret_cast<u32x4*>(stage_a + a_stage_row[i] * kStageRow + load_col * 2) =
-                inside ? now.a[i] : u32x4{0u, 0u, 0u, 0u};
+        for (int i = 0; i < kPasses; ++i) {
+            u32x4 piece;
+            if constexpr (FOLD > 0) {
+                const floatx4 lo = now.x[i][0], hi = now.x[i][1];
+                const float sq = ((lo[0] * lo[0] + lo[1] * lo[1]) + (lo[2] * lo[2] + lo[3] * lo[3])) +
+                                 ((hi[0] * hi[0] + hi[1] * hi[1]) + (hi[2] * hi[2] + hi[3] * hi[3]));
+                fold_sq[i] += inside ? sq : 0.f;
+                const floatx4 a0 = lo * now.norm[0], a1 = hi * now.norm[1];
+                piece = u32x4{pack_bf16(a0[0], a0[1]), pack_bf16(a0[2], a0[3]), pack_bf16(a1[0], a1[1]), pack_bf16(a1[2], a1[3])};
+            } else {
+                piece = now.a[i];
+            }
+            *reinterpret_cast<u32x4*>(stage_a + a_stage_row[i] * kStageRow + load_col * 2) = inside ? piece : u32x4{0u, 0u, 0u, 0u};
+        }
         fetch(ahead, next);
         u32x4 bt[NT][4];
 #pragma unroll
@@ -1004,13 +1036,25 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
     if (kTwoLoops && turn == 0) walk(std::false_type{});
     else walk(std::true_type{});
     if (scaled_rows && slices == 0) __syncthreads();  // (the scales, if no step stood between)
+    if constexpr (FOLD > 0) {  // the rows' 1/rms: sixteen lanes hold a row's squares
+#pragma unroll
+        for (int i = 0; i < kPasses; ++i) {
+            float sq = fold_sq[i];
+            sq += turned<8>(sq);
+            sq += turned<4>(sq);
+            sq += turned<2>(sq);
+            sq += turned<1>(sq);
+            if ((lane & 15) == 0) scale_lds[a_stage_row[i]] = 1.0f / sqrtf(sq / static_cast<float>(a.K) + a.eps);
+        }
+        __syncthreads();
+    }
 
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         if (mt >= row_tiles_used) break;
         if (EPI == EPI_SILU) {
             float row_scale[4] = {1.f, 1.f, 1.f, 1.f};
-            if (scaled_rows) {
+            if (scaled_rows || FOLD > 0) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) row_scale[i] = scale_lds[mt * 16 + g * 4 + i];
             }
@@ -1025,13 +1069,13 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
     }
 }
 
-template <int EPI, int MT, int NT, int WAVES>
+template <int EPI, int MT, int NT, int WAVES, int FOLD = 0>
 int launch_shared_rows_tiles(hipStream_t s, dim3 grid, const FusedArgs& a) {
     constexpr int kBytes = SharedRowsLds<MT, WAVES>::kBytes;
     if (kBytes > 64 * 1024) {  // more than a kernel gets without asking: once per kernel (and again is harmless)
         static bool asked = false;
         if (!asked) {
-            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_shared_rows_kernel<EPI, MT, NT, WAVES>),
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_shared_rows_kernel<EPI, MT, NT, WAVES, FOLD>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kBytes) != hipSuccess) {
                 (void)hipGetLastError();
                 return CIE_LAUNCH_FAILED;
@@ -1039,7 +1083,7 @@ int launch_shared_rows_tiles(hipStream_t s, dim3 grid, const FusedArgs& a) {
             asked = true;
         }
     }
-    gemm_shared_rows_kernel<EPI, MT, NT, WAVES><<<grid, WAVES * 64, kBytes, s>>>(a);
+    gemm_shared_rows_kernel<EPI, MT, NT, WAVES, FOLD><<<grid, WAVES * 64, kBytes, s>>>(a);
     return cie_after_launch();
 }
 
@@ -1057,6 +1101,14 @@ int launch_shared_rows_waves(hipStream_t s, int k_parts, const FusedArgs& a) {
     if constexpr (EPI == EPI_ATOMIC || EPI == EPI_SILU || EPI == EPI_F32)
         if (a.M <= 96) return launch_shared_rows_tiles<EPI, 6, NT, WAVES>(s, grid, a);
     return launch_shared_rows_tiles<EPI, 8, NT, WAVES>(s, grid, a);
+}
+
+template <int WAVES>
+int launch_shared_rows_normed(hipStream_t s, const FusedArgs& a) {
+    const int tiles = (a.up_offset + 15) / 16;
+    const dim3 grid((tiles + WAVES - 1) / WAVES, 1, 1);
+    return a.M <= 8 ? launch_shared_rows_tiles<EPI_SILU, 1, 2, WAVES, 8>(s, grid, a)
+                    : launch_shared_rows_tiles<EPI_SILU, 1, 2, WAVES, 16>(s, grid, a);
 }
 
 template <int EPI, int NT>
@@ -1303,6 +1355,34 @@ CIE_API int cie_gemm_shared_rows(void* stream, const void* a, int lda, const voi
         case EPI_ATOMIC:
             return column_tiles == 2 ? launch_shared_rows<EPI_ATOMIC, 2>(s, waves, k_parts, f)
                                      : launch_shared_rows<EPI_ATOMIC, 1>(s, waves, k_parts, f);
+    }
+    return CIE_BAD_ARGUMENT;
+}
+
+// The SiLU-gate product of up to 16 rows in that form, which makes the RMSNorm of its rows itself: the rows are residual [M, K]
+// (float32, at a 16-byte address, as norm_weight [K]) * norm_weight * 1/rms.
+CIE_API int cie_gemm_shared_rows_normed(void* stream, const float* residual, const float* norm_weight, float eps, const void* w, void* c,
+                                        int M, int N, int K, int waves) {
+    if (M <= 0 || M > kFoldRows || N <= 0 || N % 2 || K <= 0 || K % 8 || !residual || !norm_weight || !(eps > 0.f) || !w || !c)
+        return CIE_BAD_ARGUMENT;
+    FusedArgs f{};
+    f.lda = K;
+    f.w = static_cast<const bf16_t*>(w);
+    f.c = c;
+    f.M = M;
+    f.N = N;
+    f.K = K;
+    f.up_offset = N / 2;
+    f.k_per_part = (K + 127) / 128 * 128;
+    f.eps = eps;
+    f.fold_residual = residual;
+    f.fold_weight = norm_weight;
+    f.split = N;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    switch (waves) {
+        case 2: return launch_shared_rows_normed<2>(s, f);
+        case 3: return launch_shared_rows_normed<3>(s, f);
+        case 4: return launch_shared_rows_normed<4>(s, f);
     }
     return CIE_BAD_ARGUMENT;
 }

@@ -432,7 +432,7 @@ def paged_attention_mfma(q: torch.Tensor, q_row_stride: int, k_pool: torch.Tenso
                          n_splits: int = 1, keys_per_split: int = 0,
                          max_context_dev: Optional[torch.Tensor] = None,
                          part_o: Optional[torch.Tensor] = None, part_ml: Optional[torch.Tensor] = None,
-                         tile_waves: int = 1) -> None:
+                         tile_waves: int = 1, merge: bool = True) -> None:
     """Matrix-core attention (bf16) for the tiles ``(tile_seq[i], tile_q0[i])``: tile i
     holds up to ``tokens_per_tile`` tokens of sequence ``tile_seq[i]`` from its
     ``tile_q0[i]``-th token of this step on (both ``None``: tile i starts sequence i, as in
@@ -444,7 +444,8 @@ def paged_attention_mfma(q: torch.Tensor, q_row_stride: int, k_pool: torch.Tenso
     blocks of 32 keys in turn; it needs pages of at least 16 keys.  ``tile_waves=8`` (heads of up to
     128 dimensions) is the form whose waves share the tile's keys and values through LDS: with
     ``row_tiles=8`` tiles of 128 rows and eight waves, with ``row_tiles=4`` tiles of 64 rows and four
-    waves, two such workgroups to a compute unit."""
+    waves, two such workgroups to a compute unit.  ``merge=False`` (several parts, not with ``tile_waves=8``) leaves the
+    parts in the workspaces for :func:`merge_project` and ``out`` as it is."""
     if not (
         q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 2 and q.stride(1) == 1 and q.stride(0) == q_row_stride
     ):
@@ -502,12 +503,50 @@ def paged_attention_mfma(q: torch.Tensor, q_row_stride: int, k_pool: torch.Tenso
         else:
             if not (keys_per_split > 0 and keys_per_split % 32 == 0):
                 raise ValueError(f"keys_per_split {keys_per_split} must be a multiple of 32")
+    if not merge and (n_splits == 1 or tile_waves == PROMPT_WAVES):
+        raise ValueError("only parts of the keys, and not those of the form through LDS, can be left unmerged")
     _run("cie_paged_attention_mfma", load_library().cie_paged_attention_mfma(
         _stream(), _ptr(q), _i(q_row_stride), _ptr(k_pool), _ptr(v_pool), _ptr(block_table),
         _i(block_table.shape[1]), _ptr(tile_seq), _ptr(tile_q0), _ptr(seq_slot), _ptr(seq_start), _ptr(seq_q_len),
         _ptr(q_start_loc), _ptr(out), _ptr(part_o), _ptr(part_ml), _i(n_tiles), _i(q_heads), _i(kv_heads),
         _i(head_dim), _i(page_size), _i(window or 0), _f(scale), _i(n_splits), _i(tokens_per_tile), _i(row_tiles),
-        _i(keys_per_split), _ptr(max_context_dev), _i(tile_waves)))
+        _i(keys_per_split), _ptr(max_context_dev), _i(tile_waves), _i(merge)))
+
+
+MERGE_PROJECT_ROWS = 16   # one row tile
+MERGE_PROJECT_SLICE = 128  # k of a workgroup
+
+
+def merge_project(part_o: torch.Tensor, part_ml: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
+                  residual: torch.Tensor, q_heads: int, kv_heads: int, head_dim: int, n_splits: int, tile_rows: int,
+                  tiles: Optional[int] = None) -> None:
+    """``residual += merged @ weight.T + bias`` (float32, in place, atomic adds), where row m of ``merged`` is the attention of
+    tile m, whose one token's ``n_splits`` parts :func:`paged_attention_mfma` left in the workspaces (``merge=False``;
+    ``tile_rows``: rows of its tiles).  ``weight`` is [N, q_heads * head_dim] in bf16."""
+    _gpu("weight", weight, torch.bfloat16, 2)
+    n, k = weight.shape
+    _gpu("residual", residual, torch.float32, 2)
+    m = residual.shape[0]
+    if not (1 <= m <= MERGE_PROJECT_ROWS and residual.shape[1] == n):
+        raise ValueError(f"residual {tuple(residual.shape)} for a weight of {n} rows; at most {MERGE_PROJECT_ROWS} rows")
+    if not (kv_heads >= 1 and q_heads % kv_heads == 0 and tile_rows >= q_heads // kv_heads and head_dim % 4 == 0
+            and k == q_heads * head_dim and k % MERGE_PROJECT_SLICE == 0 and weight.data_ptr() % 16 == 0):
+        raise ValueError(f"{q_heads} heads of {head_dim} on {kv_heads} and a weight {tuple(weight.shape)} do not fit")
+    _gpu("part_o", part_o, torch.float32)
+    _gpu("part_ml", part_ml, torch.float32)
+    units = m * kv_heads * n_splits * tile_rows
+    if not (n_splits >= 1 and part_o.numel() >= units * head_dim and part_ml.numel() >= units * 2
+            and part_o.data_ptr() % 16 == 0 and part_ml.data_ptr() % 8 == 0):
+        raise ValueError("attention workspaces are too small, or off a 16-byte line")
+    if bias is not None:
+        _gpu("bias", bias, torch.bfloat16, 1)
+        if bias.shape[0] != n:
+            raise ValueError(f"bias must be [{n}]")
+    if tiles is None:  # (128 columns a workgroup while every one has a unit of its own; else 512, fewer that merge the same shares)
+        tiles = 4 if -(-n // MERGE_PROJECT_SLICE) * (k // MERGE_PROJECT_SLICE) > compute_units() else 1
+    _run("cie_merge_project", load_library().cie_merge_project(
+        _stream(), _ptr(part_o), _ptr(part_ml), _ptr(weight), _ptr(bias), _ptr(residual), _i(m), _i(n), _i(q_heads),
+        _i(kv_heads), _i(head_dim), _i(n_splits), _i(tile_rows), _i(tiles)))
 
 
 F32_STRETCH = 1024  # k that one workgroup takes where the float32 product cuts K
@@ -875,6 +914,25 @@ def gemm_shared_rows(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias:
     _run("cie_gemm_shared_rows", load_library().cie_gemm_shared_rows(
         _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k), _i(epilogue),
         _i(column_tiles), _i(waves), _i(k_parts), _ptr(row_sumsq), _i(parts_in), _f(eps)))
+    return out
+
+
+def gemm_shared_rows_normed(stream: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor,
+                            waves: int = 4) -> torch.Tensor:
+    """:func:`gemm_shared_rows` with ``EPI_SILU`` over the RMSNorm of up to ``FOLDED_NORM_ROWS`` float32 rows, which the product
+    makes itself."""
+    _gpu("weight", weight, torch.bfloat16, 2)
+    n, k = weight.shape
+    _gpu("stream", stream, torch.float32, 2)
+    _gpu("norm_weight", norm_weight, torch.float32, 1)
+    m = stream.shape[0]
+    if not (folds_norm(m, k) and stream.shape[1] == k and norm_weight.shape[0] == k and n % 2 == 0 and eps > 0 and waves in (2, 3, 4)):
+        raise ValueError(f"{tuple(stream.shape)} rows, a norm of {norm_weight.shape[0]} and a weight {tuple(weight.shape)} do not fit")
+    if stream.data_ptr() % 16 or norm_weight.data_ptr() % 16 or weight.data_ptr() % 16:
+        raise ValueError("operands must be 16-byte aligned")
+    out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=weight.device)
+    _run("cie_gemm_shared_rows_normed", load_library().cie_gemm_shared_rows_normed(
+        _stream(), _ptr(stream), _ptr(norm_weight), _f(eps), _ptr(weight), _ptr(out), _i(m), _i(n), _i(k), _i(waves)))
     return out
 
 

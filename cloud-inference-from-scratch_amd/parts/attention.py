@@ -14,6 +14,7 @@ from __future__ import annotations
 import functools
 import math
 import warnings
+from dataclasses import dataclass
 from typing import Optional
 
 import torch
@@ -23,7 +24,7 @@ from ..config.specs import PartSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import Part, build_part, register_part
-from .linear import BEHIND_ROTATION, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, choose_tiles, linear, takes_tiles
+from .linear import Added, BEHIND_ROTATION, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, choose_tiles, linear, takes_tiles
 
 
 class Attention(Part):
@@ -136,9 +137,7 @@ class Attention(Part):
                     batch.seq_slot, view.block_table, view.k_pool, view.v_pool, self.num_heads, self.num_kv_heads,
                     head_dim, rotate=self.position.rotates, write_kv=writes,
                     folded=(x.residual, x.norm.weight_f32, x.norm.eps))
-                context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, head_dim,
-                                 self.window, self.scale)
-                return linear(context, self.w_o, self.b_o, into=residual, then_norm=next_norm, sums_parts=sums_parts)
+                return self._attended(qkv, batch, view, residual, next_norm, sums_parts)
             turning = head_dim if rotary_dim is None else rotary_dim
             if (type(self).shape_projection is Attention.shape_projection and head_dim % 16 == 0 and turning % 16 == 0
                     and x.joins_f32(self.w_qkv)):
@@ -146,8 +145,7 @@ class Attention(Part):
                     x.residual, x.norm.weight_f32, x.norm.eps, self.w_qkv, self.b_qkv, self.cos, self.sin, batch.positions,
                     batch.seq_of_token, batch.seq_slot, view.block_table, view.k_pool, view.v_pool, self.num_heads,
                     self.num_kv_heads, head_dim, rotate=self.position.rotates, write_kv=writes, rotary_dim=turning)
-                context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, head_dim, self.window, self.scale)
-                return linear(context, self.w_o, self.b_o, into=residual, then_norm=next_norm, sums_parts=sums_parts)
+                return self._attended(qkv, batch, view, residual, next_norm, sums_parts)
             x = x.complete()
         fused = (x.dtype == torch.bfloat16 and untouched and head_dim % 32 == 0
                  and x.shape[1] % 8 == 0 and (rows == 1 or x.stride(0) % 8 == 0))
@@ -170,8 +168,16 @@ class Attention(Part):
             ops.rope_kv_write(qkv, self.cos, self.sin, batch.positions, batch.seq_of_token, batch.seq_slot,
                               view.block_table, view.k_pool, view.v_pool, self.num_heads, self.num_kv_heads,
                               head_dim, rotate=self.position.rotates, write_kv=writes, rotary_dim=rotary_dim)
-        context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, head_dim,
-                         self.window, self.scale)
+        return self._attended(qkv, batch, view, residual, next_norm, sums_parts)
+
+    def _attended(self, qkv: torch.Tensor, batch, view, residual: Optional[torch.Tensor], next_norm, sums_parts: bool):
+        """The attention of rotated heads, and the product behind it."""
+        context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, self.kernel_head_dim, self.window, self.scale,
+                         unmerged=joins_merge(qkv.shape[0], self.w_o, residual))
+        if isinstance(context, Shares):
+            ops.merge_project(context.part_o, context.part_ml, self.w_o, self.b_o, residual, self.num_heads, self.num_kv_heads,
+                              self.kernel_head_dim, context.splits, context.tile_rows)
+            return Added()
         return linear(context, self.w_o, self.b_o, into=residual, then_norm=next_norm, sums_parts=sums_parts)
 
 
@@ -229,9 +235,39 @@ def takes_prompt_form(tiles: int, keys: int, singles: int, captured: bool, cus: 
     return tiles >= ALONE_TILES * cus or (not captured and tiles * keys >= ALONE_TILE_KEYS)
 
 
+@dataclass
+class Shares:
+    """Stands where the attention's output would: the keys of a step of single tokens were cut, row m is tile m, and its parts
+    are still to be merged."""
+
+    part_o: torch.Tensor
+    part_ml: torch.Tensor
+    splits: int
+    tile_rows: int
+
+
+# The output product merges a decode step's shares itself (``ops.merge_project``) where every workgroup, which reads the shares of
+# its 128 k, has no more than this many to read (of all rows, rounded up to a power of two; 512 bytes each), and where the weight
+# has no more numbers than this: beyond it the sums that meet in the stream cost more than the merge kernel (MI355X, us, attention,
+# merge and product apart and with the merge in the product, 1 / 8 rows over 4,000 keys: 3B heads, 4 million 15.9, 10.4 / 21.1, 16.1; 512
+# shares of one row 19.7, 14.1; 7B, 13 million 19.8, 17.1 / 30.1, 26.5; 32 heads on 8 and 4,096 columns, 17 million 21.3, 20.1 / 40.9, 39.9,
+# 16 rows 64.4, 64.3; 14B, 26 million 25.1, 28.3 / 45.1, 48.7).  The SiLU-gate product behind it, which then makes its norm itself, is 0 to
+# 0.6 us slower (7B 1.4).
+MERGE_SHARES = 512
+MERGE_WEIGHT = 14 << 20
+
+
+def joins_merge(rows: int, weight: torch.Tensor, residual: Optional[torch.Tensor]) -> bool:
+    """Whether the output product can take the keys' shares of a step of single tokens as they are."""
+    return (residual is not None and rows <= ops.MERGE_PROJECT_ROWS and weight.dtype == torch.bfloat16 and weight.is_cuda
+            and weight.shape[1] % ops.MERGE_PROJECT_SLICE == 0 and weight.numel() <= MERGE_WEIGHT and weight.data_ptr() % 16 == 0
+            and residual.dtype == torch.float32 and residual.is_contiguous() and tuple(residual.shape) == (rows, weight.shape[0]))
+
+
 def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, head_dim: int,
-           window: Optional[int], scale: float) -> torch.Tensor:
-    """Pick the attention kernel for this step's rows.
+           window: Optional[int], scale: float, unmerged: bool = False) -> "torch.Tensor | Shares":
+    """Pick the attention kernel for this step's rows.  ``unmerged``: of a step of single tokens whose keys are cut in a few
+    shares (``MERGE_SHARES``) these may come back instead.
 
     bfloat16 with a head size the matrix-core kernel takes: sequences that bring
     one token go to the split-context decode form, prompt portions to the tiled
@@ -311,6 +347,9 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
         # (8 x 128 keys: 6.5 against 6.9 us, 8 x 160: 7 against 11)
         return (ops.TILE_WAVES if wide and bound >= SHARED_DECODE_KEYS else 1), dict(target_waves=4 * cus, min_keys=bound + 1)
 
+    def leave(n_splits: int, rows: int) -> bool:
+        return unmerged and n_splits > 1 and rows == batch.tokens and n_splits << (rows - 1).bit_length() <= MERGE_SHARES
+
     plan = batch.static_plan
     longest_dev = None
     if plan is not None:
@@ -330,7 +369,9 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
             ops.paged_attention_mfma(qkv, qkv.stride(0), view.k_pool, view.v_pool, view.block_table, None,
                                      None, decode_rows, *common, tokens_per_tile=1, row_tiles=decode_tiles,
                                      n_splits=n_splits, max_context_dev=longest_dev, part_o=part_o, part_ml=part_ml,
-                                     tile_waves=decode_waves)
+                                     tile_waves=decode_waves, merge=not leave(n_splits, decode_rows))
+            if leave(n_splits, decode_rows):
+                return Shares(part_o, part_ml, n_splits, 16 * decode_tiles)
         if decode_rows == batch.sequences:
             return out
         n_tiles = 0  # (of the eager decode form below)
@@ -349,7 +390,10 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
             part_o, part_ml = _workspaces(qkv.device, n_tiles * num_kv_heads * n_splits, 16 * decode_tiles, head_dim)
         ops.paged_attention_mfma(qkv, qkv.stride(0), view.k_pool, view.v_pool, view.block_table, tile_seq, tile_q0,
                                  n_tiles, *common, tokens_per_tile=1, row_tiles=decode_tiles, n_splits=n_splits,
-                                 keys_per_split=per_split, part_o=part_o, part_ml=part_ml, tile_waves=decode_waves)
+                                 keys_per_split=per_split, part_o=part_o, part_ml=part_ml, tile_waves=decode_waves,
+                                 merge=not leave(n_splits, n_tiles))
+        if leave(n_splits, n_tiles):
+            return Shares(part_o, part_ml, n_splits, 16 * decode_tiles)
     if wide:
         # the prompt forms: waves share a tile's keys.  More rows per tile re-use each key more often,
         # fewer tiles leave compute units idle: the most rows that still give most units a workgroup, where a

@@ -119,7 +119,7 @@ class PreNormBlock:
         mixed = self.mixer.forward(x, batch, view, writes, **extra)
         if not self.has_feed_forward:
             return residual, mixed  # (the next norm adds it)
-        if (self.dtype == torch.float32 and isinstance(mixed, Added) and declares(self.feed_forward, "takes_raw_rows")
+        if (isinstance(mixed, Added) and declares(self.feed_forward, "takes_raw_rows")
                 and getattr(self.norm2, "folds_into_products", False) and RawRows.fits(residual, self.dtype)):
             x = RawRows(residual, self.norm2, self.dtype)  # a few rows: the feed-forward's first product makes the norm
         else:

@@ -20,7 +20,7 @@ class GatedMLP(Part):
     graph_safe = True
     adds_to_residual = True
     takes_scaled_rows = True  # its first product applies the scale of rows that come without it
-    takes_raw_rows = True  # in float32 its first product makes the norm of a few rows itself
+    takes_raw_rows = True  # its first product can make the norm of a few rows itself
     sums_parts = True  # its last product may come back as parts of K
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str = "silu",
                  names: tuple[str, str, str] = ("gate_proj.weight", "up_proj.weight", "down_proj.weight")) -> None:

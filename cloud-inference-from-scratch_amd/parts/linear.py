@@ -494,8 +494,8 @@ class RawRows:
     """Stands where an RMSNorm's output would, before anything was computed: the rows are the norm ``norm``
     of the float32 stream ``residual``.  Only a part that says ``takes_raw_rows`` is shown it (the attention
     part's q/k/v product then makes its rows itself, with up to ``ops.FOLDED_NORM_ROWS`` rows: every workgroup
-    reads the few rows once, where a kernel of its own for the norm costs a decode layer 4.6 us; in float32 the
-    feed-forward's first product too)."""
+    reads the few rows once, where a kernel of its own for the norm costs a decode layer 4.6 us; behind a branch that
+    was added in parts the feed-forward's first product too)."""
 
     residual: torch.Tensor
     norm: Any
@@ -516,6 +516,11 @@ class RawRows:
         """Whether the float32 product with this weight can make the norm itself."""
         return (self.dtype == weight.dtype == torch.float32 and weight.data_ptr() % 16 == 0
                 and self.norm.weight_f32.data_ptr() % 16 == 0)
+
+    def joins_silu(self, weight: torch.Tensor) -> bool:
+        """... and whether the bfloat16 SiLU-gate product can."""
+        return (self.dtype == weight.dtype == torch.bfloat16 and weight.data_ptr() % 16 == 0 and self.residual.is_contiguous()
+                and self.residual.data_ptr() % 16 == 0 and self.norm.weight_f32.data_ptr() % 16 == 0)
 
     def complete(self) -> torch.Tensor:
         """The norm's output after all."""
@@ -585,7 +590,7 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
     this product and the next (``RMSNorm.folds_into_products``): the residual
     epilogue then also leaves that norm's output short of the rows' scale.
     ``x`` may be such rows (:class:`ScaledRows`): the SiLU product of few rows
-    applies the scale itself, any other reader gets the completed rows.  :class:`RawRows` in float32:
+    applies the scale itself, any other reader gets the completed rows.  :class:`RawRows`:
     the SiLU product of few rows makes their norm itself."""
     if isinstance(x, ScaledRows):
         rows, k = x.rows.shape
@@ -607,6 +612,9 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
     if isinstance(x, RawRows):
         if epilogue == "silu" and weight.shape[0] % 2 == 0 and bias is None and into is None and x.joins_f32(weight):
             return ops.gemm_f32_normed(x.residual, x.norm.weight_f32, x.norm.eps, weight)
+        if epilogue == "silu" and weight.shape[0] % 2 == 0 and bias is None and into is None and x.joins_silu(weight):
+            waves, _own_unit = plan_shared_silu(-(-weight.shape[0] // 32))
+            return ops.gemm_shared_rows_normed(x.residual, x.norm.weight_f32, x.norm.eps, weight, waves)
         x = x.complete()
     rows, k = x.shape
     n = weight.shape[0]

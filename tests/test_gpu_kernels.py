@@ -1615,3 +1615,56 @@ def test_gemm_library_with_every_algorithm_timed(ops):
                 if exact is not None:
                     torch.testing.assert_close(exact.double(), expect, rtol=1e-4, atol=1e-4 * math.sqrt(k))
     assert ops._tune_level(768) == 1  # outside the block nothing is searched
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 8, 9, 16])
+@pytest.mark.parametrize("geometry", [(16, 2, 128, 2048, 16), (14, 2, 64, 896, 7), (2, 2, 64, 100, 1), (28, 4, 128, 3584, 33),
+                                      (32, 1, 64, 130, 129), (4, 4, 96, 33, 2), (8, 2, 32, 640, 5), (2, 1, 256, 1040, 3)])
+def test_merge_project(ops, geometry, rows):
+    """The merge of a decode step's shares and the output product in one: against 64 bits; shares without keys hold what they held."""
+    heads, kv, dim, n, splits = geometry
+    group, tile_rows = heads // kv, 16 if heads // kv <= 16 else 32
+    part_o = rand((rows, kv, splits, tile_rows, dim), torch.float32, 1)
+    part_ml = torch.stack([rand((rows, kv, splits, tile_rows), torch.float32, 2, 8.0),
+                           rand((rows, kv, splits, tile_rows), torch.float32, 3).abs() + 1], dim=-1).contiguous()
+    empty = torch.rand((rows, kv, splits, 1), generator=torch.Generator().manual_seed(4)).cuda().expand(-1, -1, -1, tile_rows) < 0.3
+    empty = empty & (torch.arange(splits).cuda() > 0)[None, None, :, None]  # (a row's first share has keys)
+    part_ml[empty] = torch.tensor([-math.inf, 0.0]).cuda()
+    part_o[empty] = math.nan
+    part_o[:, :, :, group:] = math.inf  # (rows of the tiles that are no head's)
+    w, b = rand((n, heads * dim), torch.bfloat16, 5, 0.05), rand((n,), torch.bfloat16, 6)
+    start = rand((rows, n), torch.float32, 7, 3.0)
+
+    m, l = part_ml[..., :group, 0].double(), part_ml[..., :group, 1].double()
+    weight = torch.exp2(m - m.amax(dim=2, keepdim=True))
+    sums = torch.where(empty[..., :group, None], 0.0, part_o[..., :group, :].double())
+    merged = (sums * weight[..., None]).sum(dim=2) / (l * weight).sum(dim=2)[..., None]
+    merged = merged.reshape(rows, heads * dim)
+    for bias in (b, None):
+        residual = start.clone()
+        ops.merge_project(part_o, part_ml, w, bias, residual, heads, kv, dim, splits, tile_rows)
+        want = start.double() + merged @ w.double().t() + (bias.double() if bias is not None else 0.0)
+        # merged rows are rounded to bf16 (half of 2^-8 of each number); float32 sums over K, and the stream's own last bits
+        bound = 2.0 ** -9 * (1 + 2.0 ** -7) * (merged.abs() @ w.double().abs().t()) + 1e-4
+        assert ((residual.double() - want).abs() <= bound).all()
+    with pytest.raises(ValueError):
+        ops.merge_project(part_o, part_ml, w, b, start[:, : n - 1].contiguous(), heads, kv, dim, splits, tile_rows)
+    with pytest.raises(ValueError):
+        ops.merge_project(part_o, part_ml, w, b, start, heads, kv, dim, splits + 1, tile_rows)
+
+
+@pytest.mark.parametrize("waves", [2, 3, 4])
+@pytest.mark.parametrize("shape", [(1, 64, 128), (8, 2208, 2048), (9, 96, 136), (16, 48, 328), (5, 34, 1032), (12, 1000, 264), (8, 22016, 8)])
+def test_gemm_shared_rows_that_makes_the_norm_itself(ops, shape, waves):
+    m, n, k = shape
+    stream, norm = rand((m, k), torch.float32, 1, 3.0), rand((k,), torch.float32, 2, 0.1) + 1
+    w = rand((n, k), torch.bfloat16, 3, 0.1)
+    rows = (stream * norm).bfloat16().double()  # (rounded short of the rows' scale)
+    scale = torch.rsqrt((stream.double() ** 2).mean(dim=1, keepdim=True) + 1e-6)
+    gate, up = ((rows @ w.double().t()) * scale).split(n // 2, dim=1)
+    want = gate * torch.sigmoid(gate) * up
+    out = ops.gemm_shared_rows_normed(stream, norm, 1e-6, w, waves=waves)
+    # the result's own rounding, and float32 sums of K terms in front of it
+    torch.testing.assert_close(out.double(), want, rtol=2.0 ** -8, atol=2e-5 * math.sqrt(k) * float(gate.abs().max() + up.abs().max()))
+    with pytest.raises(ValueError):
+        ops.gemm_shared_rows_normed(rand((17, k), torch.float32, 1), norm, 1e-6, w)
