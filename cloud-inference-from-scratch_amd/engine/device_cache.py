@@ -22,9 +22,11 @@ from __future__ import annotations
 
 from typing import Any
 
+import numpy as np
 import torch
 
 from ..cache.manager import CacheManager, FixedState
+from ..kernels import ops
 from .batch import PagedView, StateView, to_device_staging
 
 _STATE_DTYPES = {"float32": torch.float32, "bfloat16": torch.bfloat16, "int32": torch.int32}
@@ -56,6 +58,12 @@ class DeviceCache:
             assert isinstance(spec, FixedState)
             self.states[unit] = torch.zeros((manager.max_running + 1, *spec.shape),
                                             dtype=_STATE_DTYPES[spec.dtype], device=device)
+        # (address, bytes of a slot's row) of every state, for the kernel that clears a new request's rows: the states live as long
+        # as this object
+        row_bytes = [state[0].numel() * state.element_size() for state in self.states.values()]
+        self._most_state_bytes = max(row_bytes, default=0)
+        self._state_rows = torch.tensor([[state.data_ptr(), size] for state, size in zip(self.states.values(), row_bytes)],
+                                        dtype=torch.int64, device=device) if self.states else None
         self._views: dict[int, Any] = {}
         for unit in range(len(manager.unit_specs)):
             if unit in manager.unit_group:
@@ -85,6 +93,7 @@ class DeviceCache:
     def sync(self) -> None:
         """Bring the device block tables up to the host's; clear the state of
         slots that were handed to a new request."""
+        appended: dict[int, list[tuple[int, int, list[int]]]] = {}
         for group, slot, table in self.manager.take_dirty_rows():
             # A request's table only grows at its end (pages a window has passed turn to -1 in place, and
             # are never read again): copy what was appended since the last time, all of it once the slot
@@ -94,10 +103,28 @@ class DeviceCache:
             seen, synced = self._row_seen.get((group, slot), (-1, 0))
             first = synced if seen == serial and synced <= len(table) else 0
             if len(table) > first:
-                staged = to_device_staging([max(p, 0) for p in table[first:]], self.device)
-                self.tables[group][slot, first: len(table)].copy_(staged, non_blocking=True)
+                appended.setdefault(group, []).append((slot, first, table[first:]))
             self._row_seen[(group, slot)] = (serial, len(table))
+        for group, rows in appended.items():
+            if len(rows) == 1:
+                slot, first, entries = rows[0]
+                staged = to_device_staging([max(p, 0) for p in entries], self.device)
+                self.tables[group][slot, first: first + len(entries)].copy_(staged, non_blocking=True)
+                continue
+            # several rows: one copy and one launch for all of them
+            heads, at = [], 4 * len(rows)
+            for slot, first, entries in rows:
+                heads.extend((slot, first, len(entries), at))
+                at += len(entries)
+            plan = torch.empty(at, dtype=torch.int32, pin_memory=True)
+            host = plan.numpy()
+            host[: len(heads)] = heads
+            for (_slot, _first, entries), place in zip(rows, heads[3::4]):
+                host[place: place + len(entries)] = entries
+            np.maximum(host, 0, out=host)
+            ops.table_rows(plan.to(self.device, non_blocking=True), len(rows), self.tables[group])
         fresh = self.manager.take_fresh_slots()
         if fresh and self.states:
-            for state in self.states.values():
-                state[fresh] = 0
+            # (the slots' numbers as an asynchronous copy: an index made on the device from a list waits for the stream)
+            slots = to_device_staging(fresh, self.device).to(self.device, non_blocking=True)
+            ops.clear_rows(self._state_rows, slots, self._most_state_bytes)

@@ -15,12 +15,14 @@ from __future__ import annotations
 
 import contextlib
 import gc
+from array import array
 from collections.abc import Iterator, Sequence
 from dataclasses import dataclass
 from typing import Any
 
 import torch
 
+from ..kernels import ops
 from .batch import StepBatch, to_device_staging
 
 
@@ -93,6 +95,9 @@ class _Bucket:
             static_plan=StaticPlan(view("tile_seq"), view("tile_q0"), view("max_context", 1), max_keys),
             token_feed=view("token_feed") if token_pool is not None else None, token_pool=token_pool,
         )
+        # what a replay rewrites, for the kernel that does (its arguments carry the numbers: a pinned buffer, a copy into it and
+        # one to the device were 14 us of the host's 75 a step of the smallest model, and 3.6 against 2 us of the GPU's)
+        self.places = tuple(view(name) for name in ("token_ids", "positions", "seq_start", "seq_slot", "token_feed")) + (view("max_context", 1),)
         self.graph: Any = None
         self.logits: torch.Tensor | None = None
 
@@ -180,9 +185,15 @@ class DecodeGraphs:
         bucket = self.buckets.get(size) or self._capture(size)
         cache = runner.cache
         positions = [e.start_pos for e in entries]
-        bucket.fill([e.tokens[0] for e in entries], positions, [cache.slot(e.request_id) for e in entries],
-                    max(positions) + 1, feed)
-        bucket.dev.copy_(to_device_staging(bucket.host, runner.device), non_blocking=True)
+        tokens, slots = [e.tokens[0] for e in entries], [cache.slot(e.request_id) for e in entries]
+        if size <= ops.STEP_ROWS:
+            values = array("i", tokens)
+            for more in (positions, slots) if feed is None else (positions, slots, feed):
+                values.extend(more)
+            ops.step_rows(values, len(tokens), size, feed is not None, max(positions) + 1, bucket.pad_slot, *bucket.places)
+        else:
+            bucket.fill(tokens, positions, slots, max(positions) + 1, feed)
+            bucket.dev.copy_(to_device_staging(bucket.host, runner.device), non_blocking=True)
         bucket.graph.replay()
         self.replays += 1
         rows = [index for index, e in enumerate(entries) for _ in e.want]

@@ -182,6 +182,46 @@ def embed_normed(table: torch.Tensor, ids: torch.Tensor, weight: torch.Tensor, e
     return out, normed
 
 
+def table_rows(plan: torch.Tensor, rows: int, table: torch.Tensor) -> None:
+    """Write entries of ``rows`` rows of a block table: ``plan`` (int32) holds (row, first entry, how many, where they begin in
+    ``plan``) of each, and the entries behind them.  The caller vouches for the places."""
+    _gpu("plan", plan, torch.int32, 1)
+    _gpu("table", table, torch.int32, 2)
+    if not (1 <= rows and plan.shape[0] >= 4 * rows):
+        raise ValueError(f"a plan of {plan.shape[0]} numbers does not describe {rows} rows")
+    _run("cie_table_rows", load_library().cie_table_rows(_stream(), _ptr(plan), _i(rows), _ptr(table), _i(table.shape[1])))
+
+
+def clear_rows(states: torch.Tensor, slots: torch.Tensor, most_bytes: int) -> None:
+    """Zero rows ``slots`` (int32) of every state in ``states`` (int64 [n, 2]: its address, a multiple of 16, and the bytes of a
+    row, the largest of which is ``most_bytes``).  The caller vouches for addresses and slots."""
+    _gpu("states", states, torch.int64, 2)
+    _gpu("slots", slots, torch.int32, 1)
+    if not (states.shape[0] >= 1 and states.shape[1] == 2 and slots.shape[0] >= 1 and most_bytes >= 2):
+        raise ValueError(f"states {tuple(states.shape)}, slots {tuple(slots.shape)}, {most_bytes} bytes")
+    _run("cie_clear_rows", load_library().cie_clear_rows(
+        _stream(), _ptr(states), _i(states.shape[0]), _ptr(slots), _i(slots.shape[0]), _i(most_bytes)))
+
+
+STEP_ROWS = 128  # rows of a captured decode step whose numbers travel as a kernel's arguments
+
+
+def step_rows(values: "array.array", n: int, size: int, fed: bool, max_context: int, pad_slot: int, token_ids: torch.Tensor,
+              positions: torch.Tensor, seq_start: torch.Tensor, seq_slot: torch.Tensor, token_feed: torch.Tensor,
+              max_context_at: torch.Tensor) -> None:
+    """Write what changes between two replays of a captured decode step of ``size`` rows: ``values`` (a host array of C ints)
+    holds its ``n`` tokens, positions and slots and, if ``fed``, the places of the token pool they are taken from.  Rows beyond
+    ``n`` become padding on ``pad_slot``."""
+    if not (values.typecode == "i" and values.itemsize == 4 and len(values) == (4 if fed else 3) * n and 0 <= n <= size <= STEP_ROWS):
+        raise ValueError(f"{len(values)} numbers for {n} of {size} rows")
+    for at, least in ((token_ids, size), (positions, size), (seq_start, size), (seq_slot, size), (token_feed, size), (max_context_at, 1)):
+        if not (at.is_cuda and at.dtype == torch.int32 and at.is_contiguous() and at.numel() >= least):
+            raise ValueError(f"a place of {size} int32 numbers is {tuple(at.shape)} {at.dtype}")
+    _run("cie_step_rows", load_library().cie_step_rows(
+        _stream(), values.buffer_info()[0], _i(n), _i(size), _i(fed), _i(max_context), _i(pad_slot), _ptr(token_ids), _ptr(positions),
+        _ptr(seq_start), _ptr(seq_slot), _ptr(token_feed), _ptr(max_context_at)))
+
+
 MAX_NORM_WIDTH = 16384  # a row of the norm kernels is held in 64 KB of LDS as float32
 
 

@@ -1668,3 +1668,52 @@ def test_gemm_shared_rows_that_makes_the_norm_itself(ops, shape, waves):
     torch.testing.assert_close(out.double(), want, rtol=2.0 ** -8, atol=2e-5 * math.sqrt(k) * float(gate.abs().max() + up.abs().max()))
     with pytest.raises(ValueError):
         ops.gemm_shared_rows_normed(rand((17, k), torch.float32, 1), norm, 1e-6, w)
+
+
+@pytest.mark.parametrize("counts", [(1, 300), (0, 1, 255, 256, 257, 700, 3)])
+def test_table_rows(ops, counts):
+    table = torch.arange(40 * 1000, dtype=torch.int32).reshape(40, 1000).cuda()
+    want, heads, entries = table.clone(), [], []
+    for index, count in enumerate(counts):
+        slot, first = (index * 7 + 3) % 40, 1000 - count - (5 if index % 2 else 0)
+        if count + first > 1000 or first < 0:
+            first = 0
+        heads += [slot, first, count, 4 * len(counts) + len(entries)]
+        new = list(range(-count, 0))
+        entries += new
+        want[slot, first: first + count] = torch.tensor(new, dtype=torch.int32).cuda()
+    ops.table_rows(torch.tensor(heads + entries, dtype=torch.int32).cuda(), len(counts), table)
+    assert torch.equal(table, want)
+    with pytest.raises(ValueError):
+        ops.table_rows(torch.zeros(7, dtype=torch.int32).cuda(), 2, table)
+
+
+@pytest.mark.parametrize("slots", [[0], [5, 2, 6]])
+def test_clear_rows(ops, slots):
+    shapes = [(8, 128, 256), (2048,), (3, 5), (1,), (7,)]
+    types = [torch.float32, torch.float32, torch.float32, torch.int32, torch.bfloat16]
+    states = [torch.ones((7, *shape), dtype=dtype).cuda() for shape, dtype in zip(shapes, types)]
+    size = [s[0].numel() * s.element_size() for s in states]
+    rows = torch.tensor([[s.data_ptr(), b] for s, b in zip(states, size)], dtype=torch.int64).cuda()
+    ops.clear_rows(rows, torch.tensor(slots, dtype=torch.int32).cuda(), max(size))
+    for state in states:
+        for slot in range(7):
+            assert (state[slot] == (0 if slot in slots else 1)).all()
+
+
+@pytest.mark.parametrize("n,size,fed", [(1, 1, False), (3, 4, True), (5, 8, False), (64, 64, True), (70, 128, True), (128, 128, False)])
+def test_step_rows(ops, n, size, fed):
+    from array import array
+
+    places = [torch.full((size + 1,), 99, dtype=torch.int32).cuda() for _ in range(5)] + [torch.full((2,), 99, dtype=torch.int32).cuda()]
+    tokens, positions, slots = [7 * i for i in range(n)], [3 * i + 1 for i in range(n)], [n - i for i in range(n)]
+    feed = [i % 3 - 1 for i in range(n)]
+    ops.step_rows(array("i", tokens + positions + slots + (feed if fed else [])), n, size, fed, 4321, 200, *places)
+    rest = size - n
+    want = [tokens + [0] * rest, positions + [0] * rest, positions + [0] * rest, slots + [200] * rest,
+            (feed if fed else [-1] * n) + [-1] * rest]
+    for place, values in zip(places, want):
+        assert place.tolist() == values + [99]
+    assert places[5].tolist() == [4321, 99]
+    with pytest.raises(ValueError):
+        ops.step_rows(array("i", tokens), n, size, fed, 1, 200, *places)
