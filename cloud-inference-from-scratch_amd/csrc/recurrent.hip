@@ -1064,6 +1064,252 @@ gated_recurrence_step_kernel(const bf16_t* __restrict__ y_pre, long ldy, const b
         if (j < keep_n) before[static_cast<size_t>(j) * channels] = j + 1 < keep_n ? old[j + 1 < kStepTaps ? j + 1 : j] : to_float(x_new);
 }
 
+// Prompts' portions in bfloat16, whatever their number: the gates' block-diagonal product and the walk over the step's flat tokens
+// at once, in chunks of 64 tokens whose first token may be a sequence's or not.  (a) A workgroup owns 64 channels of a chunk: the
+// chunk's rows of the block's channels lie in LDS, a wave has its 16 channels' rows of both gates' weights in registers, and the
+// product comes out with a token a lane and four channels each, so that everything behind it moves in 16-byte pieces.  The walk
+// is linear in S, S_t = a_t S_(t-1) + x_t, and composed in the registers: 16 lanes' tokens by doubling, four such runs one after the
+// other.  (A, B) of every token, its state as A * (the state in front of the chunk) + B, go to memory, and the chunk's last pair
+// beside them.  A sequence's first token takes its slot's state in: A = 0 from there on.  (b) Every workgroup joins the chunks in front
+// of its own and makes the outputs; the token that ends a sequence writes the states.
+//
+// What bounds it: the way to memory, 16 bytes a token and channel between the two where the gates took as many, and the gates' five
+// transcendental functions (some 3,000 of a wave's instructions: 21 of (a)'s 30 us at 1,999 tokens of 2,048 channels; (b) 15.6).  In
+// place of the product, whose waves each fetched the same rows, and of a walk of 32 tokens a thread, 16 neighbouring channels a row: 87
+// -> 45 us there, 579 tokens of eight sequences 32.6 -> 25.5.  (b) also moves the convolutions' states, a workgroup a sequence behind its
+// tokens': done by the threads of a sequence's last token this took 8 us.
+constexpr int kChunkTokens = 64;
+constexpr int kChunkChannels = 64;
+constexpr int kOutputTokens = 32;  // of a workgroup of (b)
+
+// The value of the lane APART in front, of a row of 16 (the first ones keep theirs), and that of a row's last lane.
+template <int APART>
+__device__ __forceinline__ float lane_before(float v) {
+    const int own = static_cast<int>(__float_as_uint(v));
+    return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(own, own, 0x110 + APART, 0xf, 0xf, false)));
+}
+__device__ __forceinline__ float row_last(float v) {
+    const int own = static_cast<int>(__float_as_uint(v));
+    return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(own, own, 0x15f, 0xf, 0xf, false)));
+}
+
+// One doubling of the walk over a row's 16 tokens: what the tokens APART in front made joins, unless a sequence begins between.
+template <int APART>
+__device__ __forceinline__ void join_before(float (&a)[4], float (&b)[4], int r, int from, int place) {
+    const bool joins = r >= APART && from <= place - APART;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float pa = lane_before<APART>(a[i]), pb = lane_before<APART>(b[i]);
+        b[i] = joins ? fmaf(a[i], pb, b[i]) : b[i];
+        a[i] = joins ? a[i] * pa : a[i];
+    }
+}
+
+template <int BW>
+__global__ void __launch_bounds__(256, 4)
+gated_chunks_kernel(const bf16_t* __restrict__ u, const bf16_t* __restrict__ weight, const bf16_t* __restrict__ bias,
+                    const float* __restrict__ rate, const float* __restrict__ state, const int* __restrict__ seq_of_token,
+                    const int* __restrict__ seq_slot, const int* __restrict__ q_start_loc, float* __restrict__ plane_a,
+                    float* __restrict__ plane_b, float* __restrict__ carry, int tokens, int channels, int chunks) {
+    constexpr int kSlices = BW / 32;
+    constexpr int kRowBytes = BW * 2 + 16;  // the padding spreads the rows over the banks
+    constexpr int kTiles = kChunkTokens / 16;
+    __shared__ __attribute__((aligned(16))) char rows[kChunkTokens * kRowBytes];
+    // where a token's sequence begins, counted from the chunk's first token: what lies in front of it is never multiplied with what
+    // lies behind (its state may be infinite); the sequence's slot, if the token is its first, -1 for any other, -2 past the last
+    __shared__ int begins[kChunkTokens], first_slot[kChunkTokens];
+    const int lane = threadIdx.x % kWave;
+    const int wave = threadIdx.x / kWave;
+    const int r = lane & 15;
+    const int g = lane >> 4;
+    constexpr int kGroups = BW / kChunkChannels;
+    const int blocks = channels / BW, per = chunks * kGroups;
+    // (a block's rows and weights stay on one XCD where the blocks can be dealt out so)
+    const int own = blocks % 8 == 0 ? blockIdx.x / 8 : blockIdx.x;
+    const int block = blocks % 8 == 0 ? blockIdx.x % 8 + 8 * (own / per) : own / per;
+    const int chunk = own % per / kGroups;
+    const int n0 = own % kGroups * kChunkChannels + wave * 16;  // the wave's channels in the block
+    const int t0 = chunk * kChunkTokens;
+
+    words_t wr[kSlices], wi[kSlices], piece[kSlices];
+    const bf16_t* w_row = weight + (static_cast<size_t>(block) * 2 * BW + n0 + r) * BW + g * 8;
+    constexpr int kPieces = BW / 8;  // of 16 bytes, of a token's row
+#pragma unroll
+    for (int s = 0; s < kSlices; ++s) {
+        const int at = threadIdx.x + s * 256;
+        piece[s] = load_words(u + static_cast<size_t>(min(t0 + at / kPieces, tokens - 1)) * channels + block * BW + at % kPieces * 8);
+    }
+#pragma unroll
+    for (int s = 0; s < kSlices; ++s) {
+        wr[s] = load_words(w_row + s * 32);
+        wi[s] = load_words(w_row + static_cast<size_t>(BW) * BW + s * 32);
+    }
+    const int c = block * BW + n0 + g * 4;  // the lane's first channel
+    const piece_t coef = *reinterpret_cast<const piece_t*>(rate + c);
+    float r_bias[4], i_bias[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        r_bias[i] = to_float(bias[static_cast<size_t>(block) * 2 * BW + n0 + g * 4 + i]);
+        i_bias[i] = to_float(bias[static_cast<size_t>(block) * 2 * BW + BW + n0 + g * 4 + i]);
+    }
+    if (threadIdx.x < kChunkTokens) {
+        const int t = t0 + threadIdx.x;
+        const int seq = seq_of_token[min(t, tokens - 1)];
+        const int first = q_start_loc[seq];
+        begins[threadIdx.x] = first - t0;
+        first_slot[threadIdx.x] = t >= tokens ? -2 : first == t ? seq_slot[seq] : -1;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < kSlices; ++s) {
+        const int at = threadIdx.x + s * 256;
+        *reinterpret_cast<words_t*>(rows + at / kPieces * kRowBytes + at % kPieces * 16) = piece[s];
+    }
+    __syncthreads();
+    acc4_t r_sum[kTiles], i_sum[kTiles];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) r_sum[t] = i_sum[t] = acc4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < kSlices; ++s)
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            const gate_piece_t row = __builtin_bit_cast(gate_piece_t, *reinterpret_cast<const words_t*>(rows + (t * 16 + r) * kRowBytes + s * 64 + g * 16));
+            r_sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gate_piece_t, wr[s]), row, r_sum[t], 0, 0, 0);
+            i_sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gate_piece_t, wi[s]), row, i_sum[t], 0, 0, 0);
+        }
+    float before_a[4], before_b[4];  // all tokens of the chunk in front of the tile
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        before_a[i] = 1.f;
+        before_b[i] = 0.f;
+    }
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+        const int place = t * 16 + r;
+        const int slot = first_slot[place], from = begins[place];
+        const uint2 own_u = *reinterpret_cast<const uint2*>(rows + place * kRowBytes + (n0 + g * 4) * 2);
+        const float u_in[4] = {__uint_as_float(own_u.x << 16), __uint_as_float(own_u.x & 0xffff0000u),
+                               __uint_as_float(own_u.y << 16), __uint_as_float(own_u.y & 0xffff0000u)};
+        float a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const GateStep now = gate_step(r_sum[t][i] + r_bias[i], i_sum[t][i] + i_bias[i], u_in[i], coef[i]);
+            a[i] = slot == -2 ? 1.f : now.a;
+            b[i] = slot == -2 ? 0.f : now.x;
+        }
+        if (slot >= 0) {
+            const piece_t S = *reinterpret_cast<const piece_t*>(state + static_cast<size_t>(slot) * channels + c);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                b[i] = fmaf(a[i], S[i], b[i]);
+                a[i] = 0.f;
+            }
+        }
+        join_before<1>(a, b, r, from, place);
+        join_before<2>(a, b, r, from, place);
+        join_before<4>(a, b, r, from, place);
+        join_before<8>(a, b, r, from, place);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool joins = from < t * 16;
+            b[i] = joins ? fmaf(a[i], before_b[i], b[i]) : b[i];
+            a[i] = joins ? a[i] * before_a[i] : a[i];
+            before_a[i] = row_last(a[i]);
+            before_b[i] = row_last(b[i]);
+        }
+        if (t0 + place < tokens) {
+            const size_t at = static_cast<size_t>(t0 + place) * channels + c;
+            *reinterpret_cast<piece_t*>(plane_a + at) = piece_t{a[0], a[1], a[2], a[3]};
+            *reinterpret_cast<piece_t*>(plane_b + at) = piece_t{b[0], b[1], b[2], b[3]};
+        }
+    }
+    if (r == 15) {
+        float* to = carry + static_cast<size_t>(chunk) * 2 * channels + c;
+        *reinterpret_cast<piece_t*>(to) = piece_t{before_a[0], before_a[1], before_a[2], before_a[3]};
+        *reinterpret_cast<piece_t*>(to + channels) = piece_t{before_b[0], before_b[1], before_b[2], before_b[3]};
+    }
+}
+
+__global__ void __launch_bounds__(256)
+gated_outputs_kernel(const bf16_t* __restrict__ y_pre, long ldy, const bf16_t* __restrict__ x_in, long ldx,
+                     const float* __restrict__ plane_a, const float* __restrict__ plane_b, const float* __restrict__ carry,
+                     float* __restrict__ state, float* __restrict__ past, const int* __restrict__ seq_of_token,
+                     const int* __restrict__ seq_slot, const int* __restrict__ q_start_loc, bf16_t* __restrict__ out, int tokens,
+                     int channels, int keep_n, int token_groups) {
+    __shared__ float start[256];  // the channels' states in front of the chunk
+    const int c0 = blockIdx.x * 256;
+    if (blockIdx.y >= token_groups) {  // behind the tokens: a sequence's inputs, a channel a thread
+        const int keeps = blockIdx.y - token_groups, own = c0 + threadIdx.x;
+        if (own < channels)
+            keep_inputs(past + static_cast<size_t>(seq_slot[keeps]) * keep_n * channels, x_in, ldx, q_start_loc[keeps],
+                        q_start_loc[keeps + 1] - q_start_loc[keeps], own, channels, keep_n);
+        return;
+    }
+    const int t0 = blockIdx.y * kOutputTokens;
+    const int chunk = t0 / kChunkTokens;
+    const int c = c0 + threadIdx.x % 32 * 8;
+    const int cc = min(c, channels - 8);  // (a thread past the last channel reads and stores nothing of its own)
+    constexpr int kTurns = kOutputTokens / 8;
+    piece_t a[kTurns][2], b[kTurns][2];
+    words_t y[kTurns];
+    int seq[kTurns];
+#pragma unroll
+    for (int i = 0; i < kTurns; ++i) {
+        const int t = min(t0 + i * 8 + static_cast<int>(threadIdx.x) / 32, tokens - 1);
+        const size_t at = static_cast<size_t>(t) * channels + cc;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            a[i][h] = *reinterpret_cast<const piece_t*>(plane_a + at + 4 * h);
+            b[i][h] = *reinterpret_cast<const piece_t*>(plane_b + at + 4 * h);
+        }
+        y[i] = load_words(y_pre + static_cast<size_t>(t) * ldy + cc);
+        seq[i] = seq_of_token[t];
+    }
+    {
+        const int own = min(c0 + static_cast<int>(threadIdx.x), channels - 1);
+        const int from = q_start_loc[seq_of_token[chunk * kChunkTokens]] / kChunkTokens;
+        float S = 0.f;  // (the first of these chunks holds its sequence's first token: its A is 0)
+        for (int k0 = from; k0 < chunk; k0 += 8) {
+            float ka[8], kb[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float* pair = carry + static_cast<size_t>(min(k0 + k, chunk - 1)) * 2 * channels + own;
+                ka[k] = pair[0];
+                kb[k] = pair[channels];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) S = k0 + k < chunk ? fmaf(ka[k], S, kb[k]) : S;
+        }
+        start[threadIdx.x] = S;
+    }
+    __syncthreads();
+    if (c >= channels) return;
+    float S0[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) S0[e] = start[c - c0 + e];
+#pragma unroll
+    for (int i = 0; i < kTurns; ++i) {
+        const int t = t0 + i * 8 + static_cast<int>(threadIdx.x) / 32;
+        if (t >= tokens) break;
+        const int first = q_start_loc[seq[i]];
+        const bool joins = first < chunk * kChunkTokens;  // (its sequence does not begin in this chunk)
+        float S[8], o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float with = fmaf(a[i][e / 4][e % 4], S0[e], b[i][e / 4][e % 4]);
+            S[e] = joins ? with : b[i][e / 4][e % 4];
+            o[e] = S[e] * gelu_tanh(number(y[i], e));
+        }
+        *reinterpret_cast<words_t*>(out + static_cast<size_t>(t) * channels + c) =
+            words_t{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3]), pack_bf16(o[4], o[5]), pack_bf16(o[6], o[7])};
+        if (q_start_loc[seq[i] + 1] != t + 1) continue;
+        const int slot = seq_slot[seq[i]];  // the sequence ends here: its states
+        float* to = state + static_cast<size_t>(slot) * channels + c;
+        *reinterpret_cast<piece_t*>(to) = piece_t{S[0], S[1], S[2], S[3]};
+        *reinterpret_cast<piece_t*>(to + 4) = piece_t{S[4], S[5], S[6], S[7]};
+    }
+}
+
 // Long portions.  S_t = a_t S_(t-1) + x_t is linear in S, so `segments` stretches of up to 32 tokens run side by side:
 // thread (channel, stretch) folds its stretch into (A, B) with S_out = A S_in + B, the stretches before it give its
 // S_in (a chain of at most `segments` multiply-adds), and a second walk makes the outputs.  A portion of more than
@@ -1428,5 +1674,39 @@ CIE_API int cie_gated_recurrence_step(void* stream, const void* y_pre, long ldy,
         static_cast<const bf16_t*>(y_pre), ldy, static_cast<const bf16_t*>(x_in), ldx, static_cast<const bf16_t*>(u),
         static_cast<const bf16_t*>(weight), static_cast<const bf16_t*>(bias), block_width, tiles, rate, state, past, seq_slot,
         q_start_loc, static_cast<bf16_t*>(out), sequences, tokens, channels, taps - 1);
+    return cie_after_launch();
+}
+
+// The same for any portions of tokens, in chunks (see gated_chunks_kernel).  block_width 64, 128 or 256; u, weight, y_pre, planes, carry
+// and state at 16-byte addresses, ldy a multiple of 8.  planes: 2 * tokens * channels floats, carry: 2 * channels for every 64 tokens.
+CIE_API int cie_gated_recurrence_chunks(void* stream, const void* y_pre, long ldy, const void* x_in, long ldx, const void* u,
+                                        const void* weight, const void* bias, int block_width, const float* rate, float* state,
+                                        float* past, const int* seq_of_token, const int* seq_slot, const int* q_start_loc, void* out,
+                                        float* planes, float* carry, int sequences, int tokens, int channels, int taps) {
+    const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    if (sequences < 0 || tokens < 0 || channels <= 0 || (block_width != 64 && block_width != 128 && block_width != 256) || channels % block_width ||
+        taps < 1 || taps > kMaxTaps || ldy < channels || ldy % 8 || ldx < channels || !aligned(y_pre) || !aligned(u) || !aligned(weight) ||
+        !aligned(rate) || !aligned(state) || !aligned(out) || !aligned(planes) || !aligned(carry))
+        return CIE_BAD_ARGUMENT;
+    if (tokens == 0) return CIE_OK;
+    const int chunks = (tokens + kChunkTokens - 1) / kChunkTokens;
+    const long groups = static_cast<long>(chunks) * (channels / kChunkChannels);
+    const int token_groups = (tokens + kOutputTokens - 1) / kOutputTokens;
+    if (groups > 0x7fffffffL || static_cast<long>(token_groups) + sequences > 65535) return CIE_BAD_ARGUMENT;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    float* plane_b = planes + static_cast<size_t>(tokens) * channels;
+#define CIE_CHUNKS(BW)                                                                                                     \
+    gated_chunks_kernel<BW><<<static_cast<unsigned>(groups), 256, 0, s>>>(                                                  \
+        static_cast<const bf16_t*>(u), static_cast<const bf16_t*>(weight), static_cast<const bf16_t*>(bias), rate, state,   \
+        seq_of_token, seq_slot, q_start_loc, planes, plane_b, carry, tokens, channels, chunks)
+    if (block_width == 64) CIE_CHUNKS(64);
+    else if (block_width == 128) CIE_CHUNKS(128);
+    else CIE_CHUNKS(256);
+#undef CIE_CHUNKS
+    const int code = cie_after_launch();
+    if (code != CIE_OK) return code;
+    gated_outputs_kernel<<<dim3((channels + 255) / 256, token_groups + (taps > 1 ? sequences : 0)), 256, 0, s>>>(
+        static_cast<const bf16_t*>(y_pre), ldy, static_cast<const bf16_t*>(x_in), ldx, planes, plane_b, carry, state, past, seq_of_token,
+        seq_slot, q_start_loc, static_cast<bf16_t*>(out), tokens, channels, taps - 1, token_groups);
     return cie_after_launch();
 }

@@ -1769,6 +1769,53 @@ def gated_recurrence(y_pre: torch.Tensor, x_in: torch.Tensor, u: torch.Tensor, g
     return out
 
 
+SCAN_CHUNK_WIDTHS = (64, 128, 256)  # of a block
+SCAN_CHUNK_TOKENS = 64
+
+
+def chunks_gated_recurrence(y_pre: torch.Tensor, u: torch.Tensor, weight: torch.Tensor, block_width: int, taps: int) -> bool:
+    """Whether :func:`gated_recurrence_chunks` takes these: bfloat16, rows in 16-byte pieces."""
+    return (u.dtype == weight.dtype == y_pre.dtype == torch.bfloat16 and block_width in SCAN_CHUNK_WIDTHS and u.shape[0] > 1
+            and taps <= MAX_CONV_TAPS and y_pre.stride(0) % 8 == 0
+            and u.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and y_pre.data_ptr() % 16 == 0)
+
+
+def gated_recurrence_chunks(y_pre: torch.Tensor, x_in: torch.Tensor, u: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,
+                            rate: torch.Tensor, state: torch.Tensor, past: torch.Tensor, seq_of_token: torch.Tensor,
+                            seq_slot: torch.Tensor, q_start_loc: torch.Tensor, sequences: int, taps: int) -> torch.Tensor:
+    """``gated_recurrence`` with its gates' product ``block_linear(u, weight, bias)`` in front of it, over the step's flat tokens in
+    chunks of ``SCAN_CHUNK_TOKENS`` (the result differs from the walk in order by float32 rounding only)."""
+    tokens, channels = u.shape
+    for name, t in (("y_pre", y_pre), ("x_in", x_in)):
+        if not (t.is_cuda and t.dim() == 2 and t.stride(1) == 1 and t.dtype == u.dtype and tuple(t.shape) == (tokens, channels)):
+            raise ValueError(f"{name} must be a [{tokens}, {channels}] view of u's type with unit inner stride")
+    _gpu("u", u, torch.bfloat16, 2)
+    _gpu("weight", weight, torch.bfloat16, 3)
+    _gpu("bias", bias, torch.bfloat16, 2)
+    _gpu("rate", rate, torch.float32, 1)
+    _gpu("state", state, torch.float32, 2)
+    _gpu("past", past, torch.float32, 3)
+    blocks, twice, width = weight.shape
+    if (twice != 2 * width or blocks * width != channels or tuple(bias.shape) != (blocks, twice) or rate.shape[0] != channels
+            or state.shape[1] != channels or tuple(past.shape[1:]) != (max(taps - 1, 1), channels)
+            or past.shape[0] != state.shape[0] or not 1 <= taps <= MAX_CONV_TAPS or width not in SCAN_CHUNK_WIDTHS):
+        raise ValueError("weight, bias, rate, state or past do not fit the channels")
+    for name, meta, least in (("seq_of_token", seq_of_token, tokens), ("seq_slot", seq_slot, sequences),
+                              ("q_start_loc", q_start_loc, sequences + 1)):
+        _gpu(name, meta, torch.int32, 1)
+        if meta.shape[0] < least:
+            raise ValueError(f"{name} has {meta.shape[0]} entries for {sequences} sequences of {tokens} tokens")
+    out = torch.empty((tokens, channels), dtype=u.dtype, device=u.device)
+    planes = torch.empty((2, tokens, channels), dtype=torch.float32, device=u.device)
+    carry = torch.empty((-(-tokens // SCAN_CHUNK_TOKENS), 2, channels), dtype=torch.float32, device=u.device)
+    ld = lambda t: t.stride(0) if tokens > 1 else max(t.stride(0), channels)
+    _run("cie_gated_recurrence_chunks", load_library().cie_gated_recurrence_chunks(
+        _stream(), _ptr(y_pre), ld(y_pre), _ptr(x_in), ld(x_in), _ptr(u), _ptr(weight), _ptr(bias), _i(width), _ptr(rate),
+        _ptr(state), _ptr(past), _ptr(seq_of_token), _ptr(seq_slot), _ptr(q_start_loc), _ptr(out), _ptr(planes), _ptr(carry),
+        _i(sequences), _i(tokens), _i(channels), _i(taps)))
+    return out
+
+
 SCAN_STEP_TAPS = 5         # of a convolution in front of the kernel of single tokens, at most
 # ... and workgroups of 16 channels and 16 sequences a compute unit: blocks of up to so many numbers have little K for what a
 # fifth costs (us, the two kernels and this one: 20 blocks of 128, 4.4 a unit 11.0, 12.1, 5 11.7, 13.5; 16 blocks of 128, 4 a unit

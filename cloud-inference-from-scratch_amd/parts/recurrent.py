@@ -188,6 +188,17 @@ def scan_segments(longest: int) -> int:
     return min(ops.MAX_SCAN_SEGMENTS, max(16, -(-longest // (32 * 16)) * 16))
 
 
+# Tokens of a step, and of a portion that would else be walked in order, from which the gates and the walk go in chunks (us, product
+# and walk, and this: 2,048 channels in blocks of 256, one portion of 17 tokens 16.1, 16.7, 33 24.0, 17.8, 63 38.9, 18.2, 64 14.2, 18.1,
+# 128 16.3, 18.5, 200 21.3, 18.8, 1,999 87, 45; eight, 579 tokens 32.6, 25.5; 40 single tokens and 60 37.6, 19.3; 896 channels in blocks
+# of 128, 200 18.3, 17.2, 300 21.5, 17.8, 1,999 62.6, 31.1)
+CHUNKS_FROM_TOKENS, CHUNKS_FROM_WALK = 192, 24
+
+
+def takes_chunks(tokens: int, longest: int) -> bool:
+    return tokens >= CHUNKS_FROM_TOKENS or CHUNKS_FROM_WALK <= longest < SCAN_SEGMENT_TOKENS
+
+
 class GatedLinearRecurrence(Part):
     graph_safe = True
 
@@ -242,6 +253,11 @@ class GatedLinearRecurrence(Part):
             # (no sequence brings more than one token: the gates and the step at once)
             out = ops.gated_recurrence_step(y_pre, x_in, u, self.w_gates, self.b_gates, self.rate, state, past, batch.seq_slot,
                                             batch.q_start_loc, batch.sequences, self.taps)
+            return linear(out, self.w_o)
+        if (takes_chunks(u.shape[0], batch.max_q_len)
+                and ops.chunks_gated_recurrence(y_pre, u, self.w_gates, w // self.blocks, self.taps)):
+            out = ops.gated_recurrence_chunks(y_pre, x_in, u, self.w_gates, self.b_gates, self.rate, state, past, batch.seq_of_token,
+                                              batch.seq_slot, batch.q_start_loc, batch.sequences, self.taps)
             return linear(out, self.w_o)
         gates = ops.block_linear(u, self.w_gates, self.b_gates, out_dtype=torch.float32)
         # long portions run as stretches side by side (the portion lengths are the host's, and a captured step's own)

@@ -4,6 +4,7 @@ decoding, other sizes, and greedy generation through the engine's own entry poin
 
 from __future__ import annotations
 
+import math
 import random
 
 import numpy as np
@@ -739,3 +740,46 @@ def test_gated_recurrence_of_single_tokens(lengths, blocks, width, taps):
     assert torch.allclose(state, state2, atol=near, rtol=near)
     assert torch.allclose(out.float(), want.float(), atol=4 * near, rtol=2.0 ** -7)
     assert torch.equal(past, past2)
+
+
+@pytest.mark.parametrize("lengths,blocks,width,taps", [
+    ((2,), 1, 64, 1), ((64, 1, 129), 3, 64, 4), ((63, 65, 1, 1, 2), 8, 128, 4), ((1, 700), 2, 256, 3), ((17,) * 9, 1, 256, 4),
+    ((1999,), 8, 256, 4), ((3, 0, 61, 0, 1), 5, 128, 2)])
+def test_gated_recurrence_in_chunks(lengths, blocks, width, taps):
+    """Sequences that begin, end or both inside a chunk, at its first and last token, one over many chunks, and places without
+    a token, against the product and the walk by themselves; a sequence whose state is infinite keeps that to itself."""
+    from cie_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(10)
+    tokens, channels = sum(lengths), blocks * width
+    slots = list(range(len(lengths) + 2))[::-1][: len(lengths)]
+    make = lambda *shape: torch.randn(*shape, generator=g)
+    proj = make(tokens, 2 * channels + 8).bfloat16().cuda()
+    y_pre, x_in = proj[:, 8: channels + 8], proj[:, channels + 8:]
+    u = make(tokens, channels).bfloat16().cuda()
+    weight, bias = (make(blocks, 2 * width, width) * width ** -0.5).bfloat16().cuda(), make(blocks, 2 * width).bfloat16().cuda()
+    rate = -8.0 * torch.rand(channels, generator=g).cuda()
+    state, past = make(len(lengths) + 2, channels).cuda(), make(len(lengths) + 2, max(taps - 1, 1), channels).cuda()
+    starts = [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    meta = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+    of_token = meta([i for i, n in enumerate(lengths) for _ in range(n)])
+    assert ops.chunks_gated_recurrence(y_pre, u, weight, width, taps)
+    assert not ops.chunks_gated_recurrence(proj[:, 1: channels + 1], u, weight, width, taps)
+    assert not ops.chunks_gated_recurrence(y_pre, u.float(), weight, width, taps)
+    assert not ops.chunks_gated_recurrence(y_pre, u, weight, 32, taps)
+    for odd in (None, math.inf, math.nan):
+        if odd is not None:
+            state[slots[0], 3::7] = odd
+        state2, past2 = state.clone(), past.clone()
+        out = ops.gated_recurrence_chunks(y_pre, x_in, u, weight, bias, rate, state, past, of_token, meta(slots), meta(starts),
+                                          len(lengths), taps)
+        gates = ops.block_linear(u, weight, bias, out_dtype=torch.float32)
+        want = ops.gated_recurrence(y_pre, x_in, u, gates, width, rate, state2, past2, meta(slots), meta(starts), len(lengths), taps)
+        # as above; what fades joins in another order (a product of fades is some log2(64) + 4 roundings off)
+        near = width * 2.0 ** -24 * 8 + 2e-6
+        there = torch.isfinite(state2)
+        assert torch.allclose(state[there], state2[there], atol=near, rtol=near)
+        assert torch.equal(torch.isfinite(out[lengths[0]:]), torch.isfinite(want[lengths[0]:]))
+        there = torch.isfinite(want)
+        assert torch.allclose(out[there].float(), want[there].float(), atol=4 * near, rtol=2.0 ** -7)
+        assert torch.equal(past, past2)
