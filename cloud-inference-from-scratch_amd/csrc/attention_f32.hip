@@ -21,11 +21,11 @@
 //
 // * attention_f32_prompt_kernel: four waves share a tile's 64 keys and values through LDS, the next 64 on their way in
 //   registers; bound by the matrix cores (16 rows x 64 keys x 128 dimensions: 8,192 cycles a wave).
-// * attention_f32_block_kernel: a wave per 16 rows and block, straight from memory, the blocks' (m, l, o) to a workspace,
+// * attention_f32_block_kernel: a wave, or four, per 16 rows and block, straight from memory, the blocks' (m, l, o) to a workspace,
 //   and attention_f32_join_kernel joins them: single tokens, and tiles too few to fill the units.
 //
 // Measured (MI355X, us a layer; the generic kernel, one thread a key and an output number, in brackets): a prompt of 517
-// tokens with 16 query heads on 2 key heads of 128 66 in blocks, 79 in whole tiles (634), 4 tokens over 1,000 keys 17 for
+// tokens with 16 query heads on 2 key heads of 128 66 in blocks, 79 in whole tiles (634), 4 tokens over 1,000 keys 11.4 for
 // both kernels (117).
 #include "common.h"
 
@@ -151,10 +151,12 @@ __device__ __forceinline__ void join_factors(float& M, float m, float& stands, f
 
 // A block some of whose values are infinite or NaN, and which some row does not see whole: the product took such values
 // as 0 (0 times them is a NaN, in the rows that do not see them too), and here the rows that see them get them.  A lane
-// holds dimension 16 dt + r of rows 4 g + i; the probability of (row, key 16 kt + 4 gg + j) lies in lane 16 gg + row.
-template <int D>
+// holds dimension 16 dt + r of rows 4 g + i, its n-th dt = first + n * apart; the probability of (row, key 16 kt + 4 gg + j) lies in
+// lane 16 gg + row.
+template <int D, int kOwn>
 __device__ __forceinline__ void add_odd_values(const Args& a, const Tile& t, int kb, int kv_head, int pos, int r, int g,
-                                               const floatx4 (&p)[kKeys / 16], const float (&factor)[4], floatx4 (&o)[D / 16]) {
+                                               const floatx4 (&p)[kKeys / 16], const float (&factor)[4], floatx4 (&o)[kOwn],
+                                               int first = 0, int apart = 1) {
 #pragma unroll 1
     for (int c = 0; c < kKeys; ++c) {
         const int key = kb + c;
@@ -175,8 +177,8 @@ __device__ __forceinline__ void add_odd_values(const Args& a, const Tile& t, int
             sees[i] = key <= at && !(a.window > 0 && key < at + 1 - a.window);
         }
 #pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) {
-            const float x = v[static_cast<size_t>(16 * dt + r) << a.page_shift];
+        for (int dt = 0; dt < kOwn; ++dt) {
+            const float x = v[static_cast<size_t>(16 * min(first + dt * apart, D / 16 - 1) + r) << a.page_shift];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (sees[i] && !is_finite_bits(x)) o[dt][i] = fmaf(of_row[i], x, o[dt][i]);
@@ -315,7 +317,7 @@ __global__ void __launch_bounds__(kTileWaves * kWave, 2) attention_f32_prompt_ke
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[dt][i] = fmaf(part[i], row_comes[i], o[dt][i] * row_stands[i]);
         }
-        if (some_odd) add_odd_values<D>(a, t, kb, kv_head, pos, r, g, s, row_comes, o);
+        if (some_odd) add_odd_values<D, kG>(a, t, kb, kv_head, pos, r, g, s, row_comes, o);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -329,11 +331,20 @@ __global__ void __launch_bounds__(kTileWaves * kWave, 2) attention_f32_prompt_ke
     }
 }
 
-// blockIdx: (tile, kv head and 16 rows of the tile, first of the wave's blocks: it takes every gridDim.z-th).
-template <int D>
-__global__ void __launch_bounds__(kWave, 1) attention_f32_block_kernel(Args a) {
+// blockIdx: (tile, kv head and 16 rows of the tile, first of the workgroup's blocks: it takes every gridDim.z-th).
+// kWaves: 1, or 4 that share a block where there are few: each takes 16 of its keys and a quarter of the dimensions, so that a wave has
+// 16 KB to ask for and a fourth of the products, which a wave alone on its unit made one after the other; the scores meet in LDS, and every
+// sum stays in its order.  (A wave of the four makes the whole softmax, so where many blocks fill the units one wave is the better.)
+// Both kernels, 16 heads of 128 on 2, one sequence of 1,000 keys 15.5 -> 10.7 us, four 15.9 -> 11.4, eight 16.2 -> 12.2; 14 heads of 64 11.6
+// -> 9.6 of four.
+template <int D, int kWaves>
+__global__ void __launch_bounds__(kWaves * kWave, 1) attention_f32_block_kernel(Args a) {
     constexpr int kG = D / 16;
-    const int lane = threadIdx.x, r = lane % 16, g = lane / 16;
+    constexpr int kOwnKeys = kKeys / 16 / kWaves;               // tiles of 16 keys of a wave ...
+    constexpr int kOwnDims = (kG + kWaves - 1) / kWaves;        // ... and pieces of 16 dimensions: wave, wave + kWaves, ...
+    const int lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+    const int wave = kWaves > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0;
+    __shared__ floatx4 met[kWaves > 1 ? 2 : 1][kWaves > 1 ? kKeys / 16 : 1][kWaves > 1 ? kWave : 1];  // (two take turns)
     const int group = a.q_heads / a.kv_heads;
     const int row_tiles = gridDim.y / a.kv_heads;
     const int kv_head = blockIdx.y / row_tiles, row_tile = blockIdx.y % row_tiles;
@@ -359,27 +370,29 @@ __global__ void __launch_bounds__(kWave, 1) attention_f32_block_kernel(Args a) {
 #pragma unroll
     for (int i = 0; i < kG; ++i) q[i] = across_quarters(q[i]);
 
-    for (int block = first_block + blockIdx.z; block <= last_block; block += gridDim.z) {
+    int turn = 0;
+    for (int block = first_block + blockIdx.z; block <= last_block; block += gridDim.z, turn ^= 1) {
         const int kb = block * kKeys;
         const bool edge = kb + kKeys - 1 > first_pos || (a.window > 0 && kb < t.hi - a.window);
         // every load of the block is on its way before the first is used: the barriers keep the compiler from placing
         // each beside its use, where a wave that is alone on its SIMD waits for them one after another (four sequences of
         // 1,012 keys: 18.2 -> 12.6 us)
-        floatx4 s[kKeys / 16], k[kKeys / 16][kG], v[kG][kKeys / 16];
-        int key_page[kKeys / 16], value_page[kKeys / 16];
+        floatx4 s[kKeys / 16], k[kOwnKeys][kG], v[kOwnDims][kKeys / 16];
+        int key_page[kOwnKeys], value_page[kKeys / 16];
 #pragma unroll
-        for (int kt = 0; kt < kKeys / 16; ++kt) {
-            key_page[kt] = t.table[max(min(kb + 16 * kt + r, t.hi - 1), t.lo) >> a.page_shift];
+        for (int n = 0; n < kOwnKeys; ++n)
+            key_page[n] = t.table[max(min(kb + 16 * (wave + n) + r, t.hi - 1), t.lo) >> a.page_shift];
+#pragma unroll
+        for (int kt = 0; kt < kKeys / 16; ++kt)
             value_page[kt] = t.table[max(min(kb + 16 * kt + 4 * g, (t.hi - 1) & ~3), t.lo & ~3) >> a.page_shift];
-        }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int kt = 0; kt < kKeys / 16; ++kt) {
-            const int key = max(min(kb + 16 * kt + r, t.hi - 1), t.lo);
-            const float* k_row = a.k_pool + (((static_cast<size_t>(key_page[kt]) * a.kv_heads + kv_head) << a.page_shift) +
+        for (int n = 0; n < kOwnKeys; ++n) {
+            const int key = max(min(kb + 16 * (wave + n) + r, t.hi - 1), t.lo);
+            const float* k_row = a.k_pool + (((static_cast<size_t>(key_page[n]) * a.kv_heads + kv_head) << a.page_shift) +
                                              (key & page_mask)) * D + 4 * g;
 #pragma unroll
-            for (int i = 0; i < kG; ++i) k[kt][i] = *reinterpret_cast<const floatx4*>(k_row + 16 * i);
+            for (int i = 0; i < kG; ++i) k[n][i] = *reinterpret_cast<const floatx4*>(k_row + 16 * i);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -388,58 +401,72 @@ __global__ void __launch_bounds__(kWave, 1) attention_f32_block_kernel(Args a) {
             const float* v_base = a.v_pool + ((static_cast<size_t>(value_page[kt]) * a.kv_heads + kv_head) * D << a.page_shift) +
                                   (key & page_mask);
 #pragma unroll
-            for (int dt = 0; dt < kG; ++dt)
-                v[dt][kt] = *reinterpret_cast<const floatx4*>(v_base + (static_cast<size_t>(16 * dt + r) << a.page_shift));
+            for (int n = 0; n < kOwnDims; ++n)  // (a piece past the last reads that one, and is not stored)
+                v[n][kt] = *reinterpret_cast<const floatx4*>(
+                    v_base + (static_cast<size_t>(16 * min(wave + n * kWaves, kG - 1) + r) << a.page_shift));
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int kt = 0; kt < kKeys / 16; ++kt) s[kt] = scores<kG>([&](int i) { return across_quarters(k[kt][i]); }, q);
+        for (int n = 0; n < kOwnKeys; ++n) {
+            const floatx4 own = scores<kG>([&](int i) { return across_quarters(k[n][i]); }, q);
+            if constexpr (kWaves > 1) met[turn][wave][lane] = own;
+            else s[n] = own;
+        }
         bool any_odd = false;
         if (edge) {
 #pragma unroll
-            for (int dt = 0; dt < kG; ++dt)
+            for (int n = 0; n < kOwnDims; ++n)
 #pragma unroll
                 for (int kt = 0; kt < kKeys / 16; ++kt)
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const int key = kb + 16 * kt + 4 * g + j;
                         const bool there = key >= t.lo && key < t.hi;
-                        any_odd |= there && !is_finite_bits(v[dt][kt][j]);
-                        v[dt][kt][j] = there && is_finite_bits(v[dt][kt][j]) ? v[dt][kt][j] : 0.f;
+                        any_odd |= there && !is_finite_bits(v[n][kt][j]);
+                        v[n][kt][j] = there && is_finite_bits(v[n][kt][j]) ? v[n][kt][j] : 0.f;
                     }
+        }
+        if constexpr (kWaves > 1) {
+            __syncthreads();
+#pragma unroll
+            for (int kt = 0; kt < kKeys / 16; ++kt) s[kt] = met[turn][kt][lane];
         }
         float m, l;
         block_softmax(s, kb, pos, row_lo, a.scale, g, m, l);
         const size_t at = place + static_cast<size_t>(block - first_block) * a.rows;
-        if (g == 0 && row < a.rows) {
+        if (wave == 0 && g == 0 && row < a.rows) {
             a.part_ml[(at + row) * 2] = m;
             a.part_ml[(at + row) * 2 + 1] = l;
         }
         const bool some_odd = __any(any_odd);
-        floatx4 o[kG];
+        floatx4 o[kOwnDims];
 #pragma unroll
-        for (int dt = 0; dt < kG; ++dt) {
+        for (int n = 0; n < kOwnDims; ++n) {
             floatx4 part = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kt = 0; kt < kKeys / 16; ++kt)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) part = __builtin_amdgcn_mfma_f32_16x16x4f32(s[kt][j], v[dt][kt][j], part, 0, 0, 0);
-            o[dt] = part;
+                for (int j = 0; j < 4; ++j) part = __builtin_amdgcn_mfma_f32_16x16x4f32(s[kt][j], v[n][kt][j], part, 0, 0, 0);
+            o[n] = part;
         }
         if (some_odd) {
             const float whole[4] = {1.f, 1.f, 1.f, 1.f};
-            add_odd_values<D>(a, t, kb, kv_head, pos, r, g, s, whole, o);
+            add_odd_values<D, kOwnDims>(a, t, kb, kv_head, pos, r, g, s, whole, o, wave, kWaves);
         }
 #pragma unroll
-        for (int dt = 0; dt < kG; ++dt)
+        for (int n = 0; n < kOwnDims; ++n)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int out_row = 16 * row_tile + 4 * g + i;
-                if (out_row < a.rows) a.part_o[(at + out_row) * D + 16 * dt + r] = o[dt][i];
+                if (out_row < a.rows && wave + n * kWaves < kG) a.part_o[(at + out_row) * D + 16 * (wave + n * kWaves) + r] = o[n][i];
             }
     }
 }
 
+// Places of 16 rows and a block up to which four waves share one: heads of 64 dimensions and more, and of 32, whose wave has a fourth
+// to do (us, one wave and four: 16 heads of 128 on 2, 1,280 places 23.3, 18.6, 1,024 26.6, 25.9, 1,008 of 63 a tile level; of 64, 1,280
+// 14.8, 13.1; 4 heads of 32 on 2, 128 9.7, 9.0, 512 10.4, 10.5, 1,024 11.5, 11.9).
+constexpr long kShareUpTo = 2048, kShareUpToNarrow = 256;
 constexpr int kJoin = 16;  // blocks that a thread asks for at once (16 blocks a row: 8.0 -> 4.6 us)
 
 // One workgroup per (tile, token of the tile, query head), a thread a dimension: the row's blocks joined in order.
@@ -485,7 +512,11 @@ int run(hipStream_t s, const Args& a, int n_tiles, int row_tiles, int turns) {
     if (turns == 0) {
         attention_f32_prompt_kernel<D><<<dim3(n_tiles, a.kv_heads), kTileWaves * kWave, 0, s>>>(a);
     } else {
-        attention_f32_block_kernel<D><<<dim3(n_tiles, a.kv_heads * row_tiles, turns), kWave, 0, s>>>(a);
+        const dim3 grid(n_tiles, a.kv_heads * row_tiles, turns);
+        if (static_cast<long>(n_tiles) * a.kv_heads * row_tiles * turns <= (D >= 64 ? kShareUpTo : kShareUpToNarrow))
+            attention_f32_block_kernel<D, kTileWaves><<<grid, kTileWaves * kWave, 0, s>>>(a);
+        else
+            attention_f32_block_kernel<D, 1><<<grid, kWave, 0, s>>>(a);
         attention_f32_join_kernel<D><<<dim3(n_tiles, a.tokens_per_tile * a.q_heads), (D + kWave - 1) / kWave * kWave, 0, s>>>(a);
     }
     return cie_after_launch();

@@ -1717,3 +1717,34 @@ def test_step_rows(ops, n, size, fed):
     assert places[5].tolist() == [4321, 99]
     with pytest.raises(ValueError):
         ops.step_rows(array("i", tokens), n, size, fed, 1, 200, *places)
+
+
+@pytest.mark.parametrize("geometry", [(16, 2, 128, 16), (3, 1, 96, 8), (14, 2, 64, 8), (8, 1, 32, 4)])
+@pytest.mark.parametrize("window", [None, 70])
+def test_attention_f32_blocks_shared_by_four_waves_keep_their_bits(ops, geometry, window):
+    """The block form gives a row the same bits whether a wave takes a block (many places of 16 rows and a block) or four
+    share one (few); one sequence has infinities and a NaN among its last block's values."""
+    q_heads, kv_heads, dim, page = geometry
+    g = torch.Generator().manual_seed(21)
+    lengths = [1, 63, 64, 65, 200, 513] * 60  # (360 tiles of up to 9 blocks)
+    n = len(lengths)
+    width = -(-max(lengths) // page)
+    table = torch.arange(n * width, dtype=torch.int32).reshape(n, width).cuda()
+    k_pool = torch.randn((n * width, kv_heads, page, dim), generator=g).cuda()
+    v_pool = torch.randn((n * width, kv_heads, dim, page), generator=g).cuda()
+    v_pool[4 * width + 199 // page, 0, 3, 199 % page] = math.inf
+    v_pool[4 * width + 199 // page, 0, dim - 1, 198 % page] = math.nan
+    q = torch.randn((n, q_heads * dim), generator=g).cuda()
+    meta = lambda values: torch.tensor(values, dtype=torch.int32).cuda()
+
+    def run(count):
+        group, blocks = q_heads // kv_heads, 9
+        out = torch.zeros((count, q_heads * dim)).cuda()
+        part_o, part_ml = torch.empty(count * kv_heads * blocks * group * dim).cuda(), torch.empty(count * kv_heads * blocks * group * 2).cuda()
+        ops.paged_attention_f32(q[:count], q.stride(0), k_pool, v_pool, table, None, None, count, meta(range(count)),
+                                meta([m - 1 for m in lengths[:count]]), meta([1] * count), meta(range(count + 1)), out, q_heads, kv_heads,
+                                dim, window, dim ** -0.5, 1, turns=blocks, blocks=blocks, part_o=part_o, part_ml=part_ml)
+        return out
+
+    few, many = run(6), run(n)
+    assert torch.equal(torch.nan_to_num(few, 3.0, 5.0, 7.0), torch.nan_to_num(many[:6], 3.0, 5.0, 7.0))
