@@ -27,8 +27,8 @@ __global__ void depth_stream_kernel(const float* __restrict__ x, const T* __rest
     float sum_sq = 0.f;
     for (int h = threadIdx.x; h < hidden; h += blockDim.x) {
         float v = x[row + h];
-        if (branch_a) {
-            float s = to_float(branch_a[row + h]);
+        if (branch_a || n_parts) {
+            float s = branch_a ? to_float(branch_a[row + h]) : 0.f;
             if (branch_b) s += to_float(branch_b[row + h]);
             for (int p = 0; p < n_parts; ++p) s += parts[p * apart + row + h];
             v = v + mult * s;
@@ -109,8 +109,9 @@ depth_stream_vec4_kernel(const float* __restrict__ x, const T* __restrict__ bran
         };
         if (earlier > 0) ask(ahead, past, layer_stride, 0, earlier, own);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (kBranches > 0) {
-            four_t s = branch[0];
+        if constexpr (kBranches > 0 || kParts) {
+            four_t s = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (kBranches > 0) s = branch[0];
             if constexpr (kBranches > 1) s += branch[1];
             if constexpr (kParts) {
                 for (int p0 = 0; p0 < n_parts; p0 += kAhead) {
@@ -172,7 +173,7 @@ CIE_API int cie_depth_stream(void* stream_handle, int dtype, const float* x, con
     if (rows < 0 || hidden <= 0 || hidden * sizeof(float) > 64 * 1024 || !(eps > 0.f) || terms < 0) return CIE_BAD_ARGUMENT;
     if ((newest >= 0 || terms > 0) && (!history || layer_stride < static_cast<long>(rows) * hidden)) return CIE_BAD_ARGUMENT;
     if (terms > 0 && !weights) return CIE_BAD_ARGUMENT;
-    if ((branch_b || n_parts) && !branch_a) return CIE_BAD_ARGUMENT;
+    if (branch_b && !branch_a) return CIE_BAD_ARGUMENT;
     if (n_parts < 0 || (n_parts && !parts)) return CIE_BAD_ARGUMENT;
     if (rows == 0) return CIE_OK;
     hipStream_t s = static_cast<hipStream_t>(stream_handle);
@@ -190,7 +191,8 @@ CIE_API int cie_depth_stream(void* stream_handle, int dtype, const float* x, con
     if (!(n_parts && branch_b) && ((dtype == CIE_F32 && wide(16)) || (dtype == CIE_BF16 && wide(8)))) {
         const int threads = min(1024, (hidden / 4 + kWave - 1) / kWave * kWave);
 #define CIE_DEPTH4(T, AHEAD)                                                                                          \
-    if (n_parts) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, true, AHEAD);                                          \
+    if (n_parts && branch_a) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, true, AHEAD);                              \
+    else if (n_parts) CIE_DEPTH(depth_stream_vec4_kernel, T, 0, true, AHEAD);                                          \
     else if (branch_b) CIE_DEPTH(depth_stream_vec4_kernel, T, 2, false, AHEAD);                                        \
     else if (branch_a) CIE_DEPTH(depth_stream_vec4_kernel, T, 1, false, AHEAD);                                        \
     else CIE_DEPTH(depth_stream_vec4_kernel, T, 0, false, AHEAD)

@@ -821,8 +821,24 @@ struct SharedRowsLds {
 // The weight's way from memory hides it (MI355X, us, rows short of their scale read and rows made here, 8 / 16 rows: 3B gate/up 18.0,
 // 18.1 / 18.0, 18.6; 0.5B 7.1, 7.3 / 7.1, 7.8; 14B 50.1, 50.5 / 50.2, 51.2; 7B, against the first form, 52.6, 54.0 / 56.4, 57.4, where
 // the first form with its norm folded in takes 54.8 / 67.3).
-template <int EPI, int MT, int NT, int WAVES, int FOLD = 0>
-__global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs a) {
+// ARGS: FusedArgs, or BesideArgs with a second product in the launch.  Two products of a few rows that wait for the same things (a
+// layer's branches side by side: gate/up and a mixer's first product; down and a mixer's last) cost a launch less, and the smaller one,
+// which is little else, streams beside the larger.
+struct BesideArgs : FusedArgs {
+    const bf16_t* a2;    // the second product's rows, weight [N2, K2], and with SILU its bias and bf16 result [M, N2]
+    int lda2;
+    const bf16_t* w2;
+    const bf16_t* bias2;
+    bf16_t* c2;
+    int N2, K2, k_per_part2;
+    int first;           // workgroups (SILU, along x) or parts (PARTIAL, along z; N2 = N) of the first product
+};
+
+__device__ __forceinline__ int beside_first(const FusedArgs&) { return 0; }
+__device__ __forceinline__ int beside_first(const BesideArgs& a) { return a.first; }
+
+template <int EPI, int MT, int NT, int WAVES, int FOLD = 0, typename ARGS = FusedArgs>
+__global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(ARGS a) {
     static_assert(FOLD == 0 || (EPI == EPI_SILU && MT == 1 && (FOLD == 8 || FOLD == 16)), "the folded norm: SiLU of one row tile");
     static_assert(EPI == EPI_SILU || EPI == EPI_PARTIAL || EPI == EPI_BF16 || EPI == EPI_F32 || EPI == EPI_ATOMIC,
                   "epilogues of this form");
@@ -839,9 +855,26 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
     const int g = lane >> 4;
     char* stage_w = shared + kStagesA * kStageBytesA + wave * kStageTile;
     float* scale_lds = reinterpret_cast<float*>(shared + kStagesA * kStageBytesA + kWaves * kStageTile);
-    const int cols = (EPI == EPI_SILU) ? a.up_offset : a.N;
+    constexpr bool kBeside = std::is_same_v<ARGS, BesideArgs>;
+    static_assert(!kBeside || ((EPI == EPI_SILU || EPI == EPI_PARTIAL) && FOLD == 0), "two products: SiLU and plain, or parts");
+    bool second = false;  // (the same for the workgroup)
+    int part = blockIdx.z;
+    if constexpr (kBeside) {
+        second = EPI == EPI_SILU ? static_cast<int>(blockIdx.x) >= a.first : part >= a.first;
+        if (second) {
+            a.a = a.a2;
+            a.lda = a.lda2;
+            a.w = a.w2;
+            a.K = a.K2;
+            a.N = a.N2;
+            a.k_per_part = a.k_per_part2;
+            if (EPI == EPI_PARTIAL) part -= a.first;
+        }
+    }
+    const int cols = EPI == EPI_SILU && !second ? a.up_offset : a.N;
     // SILU: the wave's gate tile and its up tile; else NT adjacent tiles
-    const int tile_first = (EPI == EPI_SILU) ? blockIdx.x * kWaves + wave : (blockIdx.x * kWaves + wave) * NT;
+    const int tile_first = EPI == EPI_SILU && !second ? blockIdx.x * kWaves + wave
+                                                      : ((blockIdx.x - (EPI == EPI_SILU && kBeside ? beside_first(a) : 0)) * kWaves + wave) * NT;
 
     const int load_row = lane >> 4;        // of the four rows of a load of W
     const int load_col = (lane & 15) * 8;  // k offset inside the 128
@@ -851,8 +884,8 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int row = i * 4 + load_row;
-            const int n = (EPI == EPI_SILU) ? min(tile_first * 16 + row, cols - 1) + t * a.up_offset
-                                            : min((tile_first + t) * 16 + row, cols - 1);
+            const int n = EPI == EPI_SILU && !second ? min(tile_first * 16 + row, cols - 1) + t * a.up_offset
+                                                     : min((tile_first + t) * 16 + row, cols - 1);
             w_rows[t][i] = a.w + static_cast<size_t>(n) * a.K;
         }
     // the slice of A: thread t takes the piece (t % 16) of rows t / 16 + (threads / 16) i (a row past the
@@ -871,7 +904,7 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
         a_rows[i] = FOLD > 0 ? nullptr : a.a + static_cast<size_t>(row) * a.lda;
         fold_rows[i] = FOLD > 0 ? a.fold_residual + static_cast<size_t>(row) * a.K : nullptr;
     }
-    const int k_begin = blockIdx.z * a.k_per_part;
+    const int k_begin = part * a.k_per_part;
     const int k_end = min(a.K, k_begin + a.k_per_part);
     const int slices = (k_end - k_begin + 127) / 128;
 
@@ -1052,6 +1085,18 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(FusedArgs 
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         if (mt >= row_tiles_used) break;
+        if constexpr (kBeside && EPI == EPI_SILU) {
+            if (second) {
+                a.c = a.c2;
+                a.bias = a.bias2;
+                a.split = a.N;
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    if ((tile_first + t) * 16 < cols)  // wave-uniform
+                        store_tile<EPI_BF16>(a, acc[mt][t], acc[mt][t], mt * 16, (tile_first + t) * 16 + r, tile_first + t, lane);
+                continue;
+            }
+        }
         if (EPI == EPI_SILU) {
             float row_scale[4] = {1.f, 1.f, 1.f, 1.f};
             if (scaled_rows || FOLD > 0) {
@@ -1385,4 +1430,74 @@ CIE_API int cie_gemm_shared_rows_normed(void* stream, const float* residual, con
         case 4: return launch_shared_rows_normed<4>(s, f);
     }
     return CIE_BAD_ARGUMENT;
+}
+
+// Two products of up to 16 rows in that form and one launch: c [M, N / 2] = SiLU-gate of a * w^T (gate rows over up rows), and
+// c2 [M, N2] = a2 * w2^T + bias2, both of K.  waves: 2 to 4 a workgroup, which own a gate tile and its up tile each, or two tiles of w2.
+CIE_API int cie_gemm_silu_beside(void* stream, const void* a, int lda, const void* w, void* c, const void* a2, int lda2, const void* w2,
+                                 const void* bias2, void* c2, int M, int N, int N2, int K, int waves) {
+    if (M <= 0 || M > 16 || N <= 0 || N % 2 || N2 <= 0 || K <= 0 || K % 8 || !a || !w || !c || !a2 || !w2 || !c2 || lda < K || lda % 8 ||
+        lda2 < K || lda2 % 8)
+        return CIE_BAD_ARGUMENT;
+    BesideArgs f{};
+    f.a = static_cast<const bf16_t*>(a);
+    f.lda = lda;
+    f.w = static_cast<const bf16_t*>(w);
+    f.c = c;
+    f.M = M;
+    f.N = N;
+    f.K = K;
+    f.up_offset = N / 2;
+    f.k_per_part = (K + 127) / 128 * 128;
+    f.split = N;
+    f.a2 = static_cast<const bf16_t*>(a2);
+    f.lda2 = lda2;
+    f.w2 = static_cast<const bf16_t*>(w2);
+    f.bias2 = static_cast<const bf16_t*>(bias2);
+    f.c2 = static_cast<bf16_t*>(c2);
+    f.N2 = N2;
+    f.K2 = K;
+    f.k_per_part2 = f.k_per_part;
+    f.first = ((N / 2 + 15) / 16 + waves - 1) / (waves > 0 ? waves : 1);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int tiles2 = (N2 + 15) / 16;
+#define CIE_BESIDE(WAVES)                                                                                               \
+    gemm_shared_rows_kernel<EPI_SILU, 1, 2, WAVES, 0, BesideArgs>                                                       \
+        <<<f.first + (tiles2 + 2 * WAVES - 1) / (2 * WAVES), WAVES * 64, SharedRowsLds<1, WAVES>::kBytes, s>>>(f)
+    if (waves == 2) CIE_BESIDE(2);
+    else if (waves == 3) CIE_BESIDE(3);
+    else if (waves == 4) CIE_BESIDE(4);
+    else return CIE_BAD_ARGUMENT;
+#undef CIE_BESIDE
+    return cie_after_launch();
+}
+
+// ... and the partial sums of two products whose results are added: c [parts + parts2, M, N] float32 holds those of a * w^T [N, K]
+// and, behind them, those of a2 * w2^T [N, K2].
+CIE_API int cie_gemm_parts_beside(void* stream, const void* a, int lda, const void* w, int K, int parts, const void* a2, int lda2,
+                                  const void* w2, int K2, int parts2, float* c, int M, int N) {
+    if (M <= 0 || M > 16 || N <= 0 || K <= 0 || K % 8 || K2 <= 0 || K2 % 8 || parts < 1 || parts2 < 1 || parts + parts2 > 64 || !a || !w ||
+        !a2 || !w2 || !c || lda < K || lda % 8 || lda2 < K2 || lda2 % 8)
+        return CIE_BAD_ARGUMENT;
+    BesideArgs f{};
+    f.a = static_cast<const bf16_t*>(a);
+    f.lda = lda;
+    f.w = static_cast<const bf16_t*>(w);
+    f.c = c;
+    f.M = M;
+    f.N = N;
+    f.K = K;
+    f.k_per_part = ((K + parts - 1) / parts + 127) / 128 * 128;
+    f.split = N;
+    f.a2 = static_cast<const bf16_t*>(a2);
+    f.lda2 = lda2;
+    f.w2 = static_cast<const bf16_t*>(w2);
+    f.N2 = N;
+    f.K2 = K2;
+    f.k_per_part2 = ((K2 + parts2 - 1) / parts2 + 127) / 128 * 128;
+    f.first = parts;
+    const int groups = ((N + 15) / 16 + 3) / 4;
+    gemm_shared_rows_kernel<EPI_PARTIAL, 1, 1, 4, 0, BesideArgs>
+        <<<dim3(groups, 1, parts + parts2), 256, SharedRowsLds<1, 4>::kBytes, static_cast<hipStream_t>(stream)>>>(f);
+    return cie_after_launch();
 }

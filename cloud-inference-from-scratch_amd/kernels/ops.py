@@ -957,6 +957,56 @@ def gemm_shared_rows(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias:
     return out
 
 
+BESIDE_ROWS = 16  # of two products in one launch
+
+
+def _beside_rows(name: str, a: torch.Tensor, weight: torch.Tensor) -> int:
+    """The row stride of one of two products' rows, checked."""
+    _gpu(f"weight of {name}", weight, torch.bfloat16, 2)
+    if not (a.is_cuda and a.dtype == torch.bfloat16 and a.dim() == 2 and a.stride(1) == 1 and a.shape[1] == weight.shape[1]
+            and 1 <= a.shape[0] <= BESIDE_ROWS):
+        raise ValueError(f"{name} {tuple(a.shape)} must be up to {BESIDE_ROWS} bf16 rows with unit inner stride as long as the weight's")
+    lda = a.stride(0) if a.shape[0] > 1 else max(a.stride(0), a.shape[1])
+    if a.shape[1] % 8 or lda % 8 or a.data_ptr() % 16 or weight.data_ptr() % 16:
+        raise ValueError(f"{name}: K and the row stride must be multiples of 8 and the operands 16-byte aligned")
+    return lda
+
+
+def gemm_silu_beside(weight: torch.Tensor, a: torch.Tensor, weight2: torch.Tensor, a2: torch.Tensor, bias2: Optional[torch.Tensor],
+                     waves: int = 4) -> tuple[torch.Tensor, torch.Tensor]:
+    """Two products of up to ``BESIDE_ROWS`` rows in one launch: ``silu(gate) * up`` of ``a`` (``weight``: gate rows over up rows)
+    and ``a2 @ weight2.T + bias2``, in bf16."""
+    lda, lda2 = _beside_rows("a", a, weight), _beside_rows("a2", a2, weight2)
+    (n, k), n2, m = weight.shape, weight2.shape[0], a.shape[0]
+    if weight2.shape[1] != k or a2.shape[0] != m or n % 2 or waves not in (2, 3, 4):
+        raise ValueError(f"products {tuple(a.shape)} x {tuple(weight.shape)} and {tuple(a2.shape)} x {tuple(weight2.shape)}, {waves} waves")
+    if bias2 is not None:
+        _gpu("bias2", bias2, torch.bfloat16, 1)
+        if bias2.shape[0] != n2:
+            raise ValueError(f"bias2 must be [{n2}]")
+    out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=a.device)
+    out2 = torch.empty((m, n2), dtype=torch.bfloat16, device=a.device)
+    _run("cie_gemm_silu_beside", load_library().cie_gemm_silu_beside(
+        _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(out), _ptr(a2), _i(lda2), _ptr(weight2), _ptr(bias2), _ptr(out2), _i(m), _i(n),
+        _i(n2), _i(k), _i(waves)))
+    return out, out2
+
+
+def gemm_parts_beside(weight: torch.Tensor, a: torch.Tensor, parts: int, weight2: torch.Tensor, a2: torch.Tensor,
+                      parts2: int) -> torch.Tensor:
+    """The float32 partial sums [parts + parts2, M, N] of ``a @ weight.T + a2 @ weight2.T``, up to ``BESIDE_ROWS`` rows, in one
+    launch: ``parts`` parts of the first product's K, ``parts2`` of the second's."""
+    lda, lda2 = _beside_rows("a", a, weight), _beside_rows("a2", a2, weight2)
+    (n, k), m = weight.shape, a.shape[0]
+    if weight2.shape[0] != n or a2.shape[0] != m or parts < 1 or parts2 < 1 or parts + parts2 > 64:
+        raise ValueError(f"products {tuple(a.shape)} x {tuple(weight.shape)} and {tuple(a2.shape)} x {tuple(weight2.shape)} in {parts}, {parts2} parts")
+    out = torch.empty((parts + parts2, m, n), dtype=torch.float32, device=a.device)
+    _run("cie_gemm_parts_beside", load_library().cie_gemm_parts_beside(
+        _stream(), _ptr(a), _i(lda), _ptr(weight), _i(k), _i(parts), _ptr(a2), _i(lda2), _ptr(weight2), _i(weight2.shape[1]),
+        _i(parts2), _ptr(out), _i(m), _i(n)))
+    return out
+
+
 def gemm_shared_rows_normed(stream: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor,
                             waves: int = 4) -> torch.Tensor:
     """:func:`gemm_shared_rows` with ``EPI_SILU`` over the RMSNorm of up to ``FOLDED_NORM_ROWS`` float32 rows, which the product
@@ -1327,8 +1377,8 @@ def depth_stream(x: torch.Tensor, branch_a: Optional[torch.Tensor] = None, branc
     """One layer boundary of a stream whose layers add two parallel branches and whose next input is a weighted
     average of what the embedding and every layer so far left:
 
-    ``v = x + mult * (branch_a + branch_b)`` (float32; without branches ``v = x``; ``parts`` [P, T, H] float32, beside a
-    ``branch_a``: their sum, in order, is one more branch); ``history[newest] = v``;
+    ``v = x + mult * (branch_a + branch_b)`` (float32; without branches ``v = x``; ``parts`` [P, T, H] float32:
+    their sum, in order, is one more branch, or all there is); ``history[newest] = v``;
     with ``weights`` (float32 [terms]) ``v = sum_j weights[j] * history[j]``; then for every gain ``g`` in
     ``gains`` (up to two) the rows ``v / sqrt(mean(v^2) + eps) * g`` in ``out_dtype``.
 
@@ -1347,8 +1397,8 @@ def depth_stream(x: torch.Tensor, branch_a: Optional[torch.Tensor] = None, branc
         raise ValueError("a second branch needs a first")
     if parts is not None:
         _gpu("parts", parts, torch.float32, 3)
-        if branch_a is None or tuple(parts.shape[1:]) != (rows, hidden):
-            raise ValueError(f"parts {tuple(parts.shape)} beside a first branch of {tuple(x.shape)}")
+        if tuple(parts.shape[1:]) != (rows, hidden):
+            raise ValueError(f"parts {tuple(parts.shape)} for a stream of {tuple(x.shape)}")
     terms, stride = 0, 0
     if history is not None:
         _gpu("history", history, torch.float32, 3)
@@ -1364,7 +1414,7 @@ def depth_stream(x: torch.Tensor, branch_a: Optional[torch.Tensor] = None, branc
             raise ValueError(f"{terms} weights for a history of {0 if history is None else history.shape[0]}")
     if len(gains) > 2 or not eps > 0:
         raise ValueError("at most two norms, and a positive eps")
-    changed = branch_a is not None or terms > 0
+    changed = branch_a is not None or parts is not None or terms > 0
     stream = torch.empty_like(x) if (want_stream and changed) else None
     outs = [torch.empty((rows, hidden), dtype=out_dtype, device=x.device) for _ in gains]
     g = [float(v) for v in gains] + [0.0, 0.0]

@@ -110,6 +110,10 @@ class Part:
     # same rows and whose results are added may share both products: ``product_in()`` and ``product_out()`` give the
     # weights, and the part's own step between them takes the first product's rows and writes into a given matrix.
     joins_products = False
+    # ``splits_products``: the part is one product in, something between, one product out, which its block may run itself, each
+    # in one launch with another product that waits for the same things: ``first_product()`` gives the first one's weight and bias,
+    # ``between(proj, batch, view, writes)`` the last one's rows, ``last_product()`` its weight.  (Asked with ``declares``.)
+    splits_products = False
 
     def expected_tensors(self, prefix: str) -> dict[str, TensorSpec]:
         return {}

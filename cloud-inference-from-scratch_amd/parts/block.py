@@ -32,7 +32,8 @@ from ..config.specs import LayerSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import build_part, declares, register_part
-from .linear import Added, KParts, RawRows, RowSumsq, StreamRows, WeightedPair, linear, linear_beside
+from .linear import (Added, KParts, RawRows, RowSumsq, StreamRows, WeightedPair, linear, linear_beside, parts_beside,
+                     silu_beside)
 
 
 class PreNormBlock:
@@ -308,9 +309,21 @@ class ParallelDepthBlock:
             _, normed = ops.depth_stream(residual, gains=self.gains(), out_dtype=self.dtype, eps=self.norm1.eps,
                                          want_stream=False)
             first, second = normed[0], normed[1] if len(normed) > 1 else None
-        mixed = self.mixer.forward(first, batch, view, writes)
-        fed = parts = None
-        if self.has_feed_forward:  # (its last product may come as parts of K: the boundary's kernel sums them)
+        mixed = fed = parts = beside = None
+        if (self.has_feed_forward and self.dtype == torch.bfloat16 and declares(self.mixer, "splits_products")
+                and declares(self.feed_forward, "gates_products")):
+            # a few rows: the branches' first products in one launch, and their last ones, as parts of one sum
+            weight, bias = self.mixer.first_product()
+            beside = silu_beside(second, self.feed_forward.w_gate_up, first, weight, bias)
+        if beside is not None:
+            hidden, proj = beside
+            rows, last = self.mixer.between(proj, batch, view, writes), self.mixer.last_product()
+            fed = parts_beside(hidden, self.feed_forward.w_down, rows, last)
+            if fed is None:
+                mixed, fed = linear(rows, last), linear(hidden, self.feed_forward.w_down)
+        else:
+            mixed = self.mixer.forward(first, batch, view, writes)
+        if self.has_feed_forward and beside is None:  # (its last product may come as parts of K: the boundary's kernel sums them)
             takes = {"sums_parts": True} if declares(self.feed_forward, "sums_parts") else {}
             fed = self.feed_forward.forward(second, **takes)
         if isinstance(fed, KParts):

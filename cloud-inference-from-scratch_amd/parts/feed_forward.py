@@ -22,6 +22,7 @@ class GatedMLP(Part):
     takes_scaled_rows = True  # its first product applies the scale of rows that come without it
     takes_raw_rows = True  # its first product can make the norm of a few rows itself
     sums_parts = True  # its last product may come back as parts of K
+    gates_products = True  # its two products are the SiLU-gate one of ``w_gate_up`` and one of ``w_down``: a block may run them itself
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str = "silu",
                  names: tuple[str, str, str] = ("gate_proj.weight", "up_proj.weight", "down_proj.weight")) -> None:
         if activation != "silu":

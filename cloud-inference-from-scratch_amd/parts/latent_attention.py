@@ -32,6 +32,7 @@ from .scored_attention import scored_attend
 
 
 class LatentAttention(Part):
+    splits_products = True
     graph_safe = True  # (a captured step's rotation tables reach the bound the step was captured for)
 
     def __init__(self, hidden_size: int, num_heads: int, head_dim: int, rot_dim: int, value_dim: int, kv_rank: int,
@@ -87,21 +88,28 @@ class LatentAttention(Part):
         self.w_unfold = unfold.contiguous()
         self.w_o = tensors[prefix + "o"].contiguous()
 
+    def first_product(self) -> tuple:
+        return self.w_in, None
+
+    def last_product(self) -> torch.Tensor:
+        return self.w_o
+
     def forward(self, x: torch.Tensor, batch, view, writes: bool = True) -> torch.Tensor:
+        return linear(self.between(linear(x, self.w_in), batch, view, writes), self.w_o)
+
+    def between(self, proj: torch.Tensor, batch, view, writes: bool = True) -> torch.Tensor:
         h, p, r, c, width = self.num_heads, self.head_dim, self.rot_dim, self.kv_rank, self.entry_dim
         if batch.max_context > self.position.max_position and self.position.rotates:
             raise ValueError(f"position {batch.max_context - 1} is beyond the rotary table of {self.position.max_position}")
         queries = h * (p + r)
-        proj = linear(x, self.w_in)
         turns = bool(r) and self.position.rotates
-        rotary = self.position.tables(x.device, positions_bound(batch)) if turns else None
+        rotary = self.position.tables(proj.device, positions_bound(batch)) if turns else None
         rows = ops.latent_rows(proj[:, : queries + c + r], self.latent_weight, h, p, r, c, width, self.eps, rotary,
                                batch.positions, batch.seq_of_token, batch.seq_slot, view.block_table, view.k_pool,
                                view.v_pool, write_kv=writes)
         ops.block_linear(proj, self.w_fold, a_block=p + r, out=rows, out_offset=r, c_block=width)
         context = attend(rows, batch, view, h, 1, width, None, self.scale)
-        gated = ops.block_linear(context, self.w_unfold, gate=proj, gate_offset=queries + c + r)
-        return linear(gated, self.w_o)
+        return ops.block_linear(context, self.w_unfold, gate=proj, gate_offset=queries + c + r)
 
 
 register_part("mixer", "latent_attention", LatentAttention)

@@ -548,6 +548,52 @@ def linear_beside(x: torch.Tensor, weight: torch.Tensor, act_out: torch.Tensor) 
     return out[:, :split]
 
 
+# Two products of few rows that wait for the same things run in one launch (a layer whose mixer and feed-forward read the same
+# stream; MI355X, us, apart and together, 1 / 8 / 16 rows): gate/up and 6,144 columns of the 3B widths 27.5, 24.0 / 27.3, 23.3 / 28.4, 23.4,
+# 4,096 columns 24.0, 21.8 / 24.9, 22.0 / 25.7, 22.0; 0.5B and 2,304 10.7, 7.5 / 11.3, 7.6 / 11.5, 7.7; 7B and 7,168 65.7, 59.5 / 68.3,
+# 57.6 / 72.3, 57.8; down and an output product, as parts: 3B 16.9, 13.8 / 17.6, 14.1 / 18.3, 14.3; 0.5B 8.7, 5.1 / 9.1, 5.3 / 9.3, 5.4; 7B 36.0,
+# 35.8 / 37.2, 36.6 / 38.7, 37.2; 14B 44.9, 39.6 / 47.0, 39.9 / 50.8, 40.6.
+def plan_silu_beside(pairs: int, tiles: int, units: int) -> int:
+    """Waves per workgroup of the SiLU product of ``pairs`` gate tiles and a product of ``tiles`` column tiles in one launch: the
+    fewest pairs (or two tiles) that meet on a unit, each XCD's turns counted as :func:`plan_shared_silu` counts them."""
+    return min((4, 3, 2), key=lambda waves: -(-(-(-pairs // waves) + -(-tiles // (2 * waves))) // units) * waves)
+
+
+def plan_parts_beside(tiles: int, k: int, k2: int, units: int) -> tuple[int, int]:
+    """Parts of the two products' K: as many together as give about one workgroup per unit, the longest stretch the shortest."""
+    together = max(2, min(units // -(-tiles // 4), 16))
+    stretch = lambda k, parts: -(-(-(-k // parts)) // 128) * 128  # noqa: E731
+    parts2 = min(range(1, together), key=lambda p: max(stretch(k, together - p), stretch(k2, p)))
+    parts = together - parts2
+    return -(-k // stretch(k, parts)), -(-k2 // stretch(k2, parts2))  # (none a part without k)
+
+
+def _beside(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    rows, k = x.shape
+    return (x.dtype == torch.bfloat16 and x.is_cuda and x.stride(1) == 1 and 1 <= rows <= FUSED_ROWS
+            and _fusable(rows, k, x.stride(0) if rows > 1 else k, weight) and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+def silu_beside(x: torch.Tensor, weight: torch.Tensor, x2: torch.Tensor, weight2: torch.Tensor,
+                bias2: Optional[torch.Tensor]) -> Optional[tuple[torch.Tensor, torch.Tensor]]:
+    """(``silu(gate) * up`` of ``x``, ``x2 @ weight2.T + bias2``) in one launch, or ``None`` where that takes another form."""
+    if not (_beside(x, weight) and _beside(x2, weight2) and weight.shape[0] % 2 == 0 and weight.shape[1] == weight2.shape[1]
+            and x.shape[0] == x2.shape[0]):
+        return None
+    waves = plan_silu_beside(-(-weight.shape[0] // 32), -(-weight2.shape[0] // 16), ops.compute_units())
+    return ops.gemm_silu_beside(weight, x, weight2, x2, bias2, waves)
+
+
+def parts_beside(x: torch.Tensor, weight: torch.Tensor, x2: torch.Tensor, weight2: torch.Tensor) -> Optional[KParts]:
+    """``x @ weight.T + x2 @ weight2.T`` as parts, from one launch, or ``None`` where that takes another form."""
+    n, k = weight.shape
+    if not (_beside(x, weight) and _beside(x2, weight2) and weight2.shape[0] == n and x.shape[0] == x2.shape[0]
+            and -(-n // 16) < PART_BELOW_TILES):
+        return None
+    parts, parts2 = plan_parts_beside(-(-n // 16), k, weight2.shape[1], ops.compute_units())
+    return KParts(ops.gemm_parts_beside(weight, x, parts, weight2, x2, parts2))
+
+
 _WIDENED: dict[int, tuple["weakref.ref", torch.Tensor]] = {}
 
 

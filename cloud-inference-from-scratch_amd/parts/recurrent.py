@@ -46,6 +46,7 @@ from .position import positions_bound
 
 
 class Retention(Part):
+    splits_products = True
     graph_safe = True  # (a captured step's rotation tables reach the bound the step was captured for)
 
     def __init__(self, hidden_size: int, num_heads: int, head_dim: int, value_dim: int, decay: tuple, eps: float,
@@ -85,7 +86,16 @@ class Retention(Part):
         self.w_o = tensors[prefix + "o"].contiguous()
         self.decay = torch.tensor(self.decay_values, dtype=torch.float32, device=device)
 
+    def first_product(self) -> tuple:
+        return self.w_in, None
+
+    def last_product(self) -> torch.Tensor:
+        return self.w_o
+
     def forward(self, x: torch.Tensor, batch, view, writes: bool = True) -> torch.Tensor:
+        return linear(self.between(linear(x, self.w_in), batch, view, writes), self.w_o)
+
+    def between(self, proj: torch.Tensor, batch, view, writes: bool = True) -> torch.Tensor:
         if not writes:
             raise ValueError("a recurrent mixer moves its state on whenever it runs")
         h, d, v = self.num_heads, self.head_dim, self.value_dim
@@ -93,12 +103,10 @@ class Retention(Part):
         if rot and batch.max_context > self.position.max_position:
             raise ValueError(f"position {batch.max_context - 1} is beyond the rotary table of {self.position.max_position}")
         bound = positions_bound(batch)
-        cos, sin = self.position.tables(x.device, bound) if rot else (None, None)
-        proj = linear(x, self.w_in)
-        out = ops.retention(proj, (0, h * d, 2 * h * d, 2 * h * d + h * v), cos, sin, rot, self.decay, view.state,
-                            batch.seq_slot, batch.positions, batch.q_start_loc, batch.sequences, h, d, v, self.eps,
-                            d ** -0.5, bound - 1)
-        return linear(out, self.w_o)
+        cos, sin = self.position.tables(proj.device, bound) if rot else (None, None)
+        return ops.retention(proj, (0, h * d, 2 * h * d, 2 * h * d + h * v), cos, sin, rot, self.decay, view.state,
+                             batch.seq_slot, batch.positions, batch.q_start_loc, batch.sequences, h, d, v, self.eps,
+                             d ** -0.5, bound - 1)
 
 
 class LightningAttention(Part):
@@ -201,6 +209,7 @@ def takes_chunks(tokens: int, longest: int) -> bool:
 
 class GatedLinearRecurrence(Part):
     graph_safe = True
+    splits_products = True
 
     def __init__(self, hidden_size: int, width: int, blocks: int, taps: int) -> None:
         if min(hidden_size, width, blocks, taps) < 1 or width % blocks:
@@ -240,31 +249,36 @@ class GatedLinearRecurrence(Part):
         self.rate = (-8.0 * torch.nn.functional.softplus(tensors[prefix + "lam"].float())).contiguous()
         self.w_o = tensors[prefix + "o"].contiguous()
 
+    def first_product(self) -> tuple:
+        return self.w_in, self.b_in
+
+    def last_product(self) -> torch.Tensor:
+        return self.w_o
+
     def forward(self, x: torch.Tensor, batch, view, writes: bool = True) -> torch.Tensor:
+        return linear(self.between(linear(x, self.w_in, self.b_in), batch, view, writes), self.w_o)
+
+    def between(self, proj: torch.Tensor, batch, view, writes: bool = True) -> torch.Tensor:
         if not writes:
             raise ValueError("a recurrent mixer moves its state on whenever it runs")
         state, past = view[0].state, view[1].state
         w = self.width
-        proj = linear(x, self.w_in, self.b_in)
         y_pre, x_in = proj[:, :w], proj[:, w:]
         u = ops.causal_conv(x_in, self.conv_w, self.conv_b, past, batch.seq_of_token, batch.seq_slot, batch.q_start_loc)
         if (batch.max_q_len == 1
                 and ops.steps_gated_recurrence(u, self.w_gates, batch.sequences, w // self.blocks, self.taps)):
             # (no sequence brings more than one token: the gates and the step at once)
-            out = ops.gated_recurrence_step(y_pre, x_in, u, self.w_gates, self.b_gates, self.rate, state, past, batch.seq_slot,
-                                            batch.q_start_loc, batch.sequences, self.taps)
-            return linear(out, self.w_o)
+            return ops.gated_recurrence_step(y_pre, x_in, u, self.w_gates, self.b_gates, self.rate, state, past, batch.seq_slot,
+                                             batch.q_start_loc, batch.sequences, self.taps)
         if (takes_chunks(u.shape[0], batch.max_q_len)
                 and ops.chunks_gated_recurrence(y_pre, u, self.w_gates, w // self.blocks, self.taps)):
-            out = ops.gated_recurrence_chunks(y_pre, x_in, u, self.w_gates, self.b_gates, self.rate, state, past, batch.seq_of_token,
-                                              batch.seq_slot, batch.q_start_loc, batch.sequences, self.taps)
-            return linear(out, self.w_o)
+            return ops.gated_recurrence_chunks(y_pre, x_in, u, self.w_gates, self.b_gates, self.rate, state, past, batch.seq_of_token,
+                                               batch.seq_slot, batch.q_start_loc, batch.sequences, self.taps)
         gates = ops.block_linear(u, self.w_gates, self.b_gates, out_dtype=torch.float32)
         # long portions run as stretches side by side (the portion lengths are the host's, and a captured step's own)
         segments = scan_segments(batch.max_q_len)
-        out = ops.gated_recurrence(y_pre, x_in, u, gates, w // self.blocks, self.rate, state, past, batch.seq_slot,
-                                   batch.q_start_loc, batch.sequences, self.taps, segments)
-        return linear(out, self.w_o)
+        return ops.gated_recurrence(y_pre, x_in, u, gates, w // self.blocks, self.rate, state, past, batch.seq_slot,
+                                    batch.q_start_loc, batch.sequences, self.taps, segments)
 
 
 class StateSpace(Part):

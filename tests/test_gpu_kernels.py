@@ -1748,3 +1748,38 @@ def test_attention_f32_blocks_shared_by_four_waves_keep_their_bits(ops, geometry
 
     few, many = run(6), run(n)
     assert torch.equal(torch.nan_to_num(few, 3.0, 5.0, 7.0), torch.nan_to_num(many[:6], 3.0, 5.0, 7.0))
+
+
+@pytest.mark.parametrize("shape", [(1, 64, 32, 128), (8, 22016, 6144, 2048), (8, 9728, 2304, 896), (3, 34, 40, 136), (16, 1000, 4736, 328), (9, 96, 17, 2048)])
+@pytest.mark.parametrize("waves", [2, 3, 4])
+def test_gemm_silu_beside(ops, shape, waves):
+    """A SiLU-gate product and a plain one of other rows in one launch, against 64 bits."""
+    m, n, n2, k = shape
+    a, a2 = rand((m, k), torch.bfloat16, 1), rand((m, 2 * k), torch.bfloat16, 2)[:, :k]  # (rows that lie apart)
+    w, w2, b2 = rand((n, k), torch.bfloat16, 3, 0.05), rand((n2, k), torch.bfloat16, 4, 0.05), rand((n2,), torch.bfloat16, 5)
+    gate, up = (a.double() @ w.double().t()).split(n // 2, dim=1)
+    for bias in (b2, None):
+        out, out2 = ops.gemm_silu_beside(w, a, w2, a2, bias, waves=waves)
+        # (a bf16 result's own rounding, float32 sums of k terms in front of it)
+        torch.testing.assert_close(out.double(), gate * torch.sigmoid(gate) * up, rtol=2.0 ** -8, atol=1e-5 * math.sqrt(k))
+        want = a2.double() @ w2.double().t() + (bias.double() if bias is not None else 0.0)
+        torch.testing.assert_close(out2.double(), want, rtol=2.0 ** -8, atol=1e-5 * math.sqrt(k))
+    with pytest.raises(ValueError):
+        ops.gemm_silu_beside(w, rand((17, k), torch.bfloat16, 1), w2, rand((17, k), torch.bfloat16, 2), b2)
+
+
+@pytest.mark.parametrize("shape", [(1, 64, 128, 128), (8, 2048, 11008, 2048), (16, 896, 4864, 768), (5, 40, 1032, 3000), (9, 130, 8, 136)])
+def test_gemm_parts_beside(ops, shape):
+    from cie_amd.parts.linear import plan_parts_beside
+
+    m, n, k, k2 = shape
+    a, a2 = rand((m, k), torch.bfloat16, 1), rand((m, k2), torch.bfloat16, 2)
+    w, w2 = rand((n, k), torch.bfloat16, 3, 0.05), rand((n, k2), torch.bfloat16, 4, 0.05)
+    want = a.double() @ w.double().t() + a2.double() @ w2.double().t()
+    for parts, parts2 in ((1, 1), plan_parts_beside(-(-n // 16), k, k2, 256)):
+        out = ops.gemm_parts_beside(w, a, parts, w2, a2, parts2)
+        assert tuple(out.shape) == (parts + parts2, m, n)
+        torch.testing.assert_close(out.double().sum(dim=0), want, rtol=0, atol=2e-6 * math.sqrt(k + k2))
+    stream = rand((m, n), torch.float32, 6)
+    got, _ = ops.depth_stream(stream, parts=out, mult=0.5, out_dtype=torch.bfloat16)  # (parts and no other branch)
+    torch.testing.assert_close(got.double(), stream.double() + 0.5 * want, rtol=1e-6, atol=4e-6 * math.sqrt(k + k2))
