@@ -39,11 +39,14 @@ struct StepRows {
     int tokens[kStepRows], positions[kStepRows], slots[kStepRows], feed[kStepRows];
     int n, size, max_context, pad_slot;
     int *token_ids, *positions_at, *seq_start, *seq_slot, *token_feed, *max_context_at;
+    void** result_at;  // takes `result`, the address that the replay's last product writes to
+    void* result;
 };
 
 __global__ void __launch_bounds__(kStepRows) step_rows_kernel(StepRows a) {
     const int i = threadIdx.x;
     if (i == 0) *a.max_context_at = a.max_context;
+    if (i == 0 && a.result_at) *a.result_at = a.result;
     if (i >= a.size) return;
     const bool real = i < a.n;
     a.token_ids[i] = real ? a.tokens[i] : 0;
@@ -72,9 +75,10 @@ CIE_API int cie_clear_rows(void* stream, const long* states, int n_states, const
 }
 
 // A captured decode step's numbers: `values` (host memory, read before this returns) holds n tokens, n positions, n slots and, if
-// `fed`, n places of the token pool.  Rows n .. size - 1 become padding on pad_slot.
+// `fed`, n places of the token pool.  Rows n .. size - 1 become padding on pad_slot.  result_at (or null) takes `result`.
 CIE_API int cie_step_rows(void* stream, const int* values, int n, int size, int fed, int max_context, int pad_slot, int* token_ids,
-                          int* positions, int* seq_start, int* seq_slot, int* token_feed, int* max_context_at) {
+                          int* positions, int* seq_start, int* seq_slot, int* token_feed, int* max_context_at, void** result_at,
+                          void* result) {
     if (n < 0 || n > size || size < 1 || size > kStepRows || !values || !token_ids || !positions || !seq_start || !seq_slot || !token_feed ||
         !max_context_at)
         return CIE_BAD_ARGUMENT;
@@ -96,6 +100,8 @@ CIE_API int cie_step_rows(void* stream, const int* values, int n, int size, int 
     a.seq_slot = seq_slot;
     a.token_feed = token_feed;
     a.max_context_at = max_context_at;
+    a.result_at = result_at;
+    a.result = result;
     step_rows_kernel<<<1, kStepRows, 0, static_cast<hipStream_t>(stream)>>>(a);
     return cie_after_launch();
 }

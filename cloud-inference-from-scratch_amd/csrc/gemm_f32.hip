@@ -85,8 +85,8 @@ __device__ __forceinline__ floatx4 inside(floatx4 v, int k, int K) {
 __device__ __forceinline__ float gated(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
 
 // What the rows kernel does beside the product: nothing; the norm of its rows; that, the rotation and the cache write; the add
-// into C.
-enum { kPlain = 0, kNormed = 1, kRotated = 2, kAdded = 3 };
+// into C; nothing, into a C whose address lies on the device (a captured launch writes where its replay says).
+enum { kPlain = 0, kNormed = 1, kRotated = 2, kAdded = 3, kPointed = 4 };
 constexpr bool norms_rows(int beside) { return beside == kNormed || beside == kRotated; }
 
 struct RowsBeside {
@@ -98,6 +98,7 @@ struct RowsBeside {
     int table_width;
     float *k_pool, *v_pool;    // [pages, Hkv, page_size, D], [pages, Hkv, D, page_size]
     int q_heads, kv_heads, head_dim, rotary_dim, page_size, rotate, write_kv;
+    float* const* c_at;  // kPointed
 };
 
 // Where pair i (0..7) of group j (0..head_dim / 16 - 1) of a head lies: its first dimension, and how far on its partner is.  The
@@ -139,6 +140,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
     static_assert(kBeside != kRotated || (!kGate && kColumns == 16 && kRows * 8 <= kThreads), "8 dimensions and their partners");
     __shared__ float stage_all[kWaves * kStaged * kTileFloats];
     __shared__ float sums[2][kWaves * kSums];
+    if constexpr (kBeside == kPointed) C = *beside.c_at;
     const int lane = threadIdx.x % kWave;
     const int wave = threadIdx.x / kWave;
     float* stage = stage_all + wave * kStaged * kTileFloats;
@@ -888,6 +890,17 @@ CIE_API int cie_gemm_f32_into(void* stream, const float* A, const float* W, cons
     return cie_after_launch();
 }
 
+// Up to 8 rows: the contiguous [M, N] whose address is *c_at (on the device) = A W^T.
+CIE_API int cie_gemm_f32_at(void* stream, const float* A, const float* W, float* const* c_at, int M, int N, int K, int lda, int units) {
+    if (M < 0 || M > 8 || N <= 0 || K <= 0 || lda < K || units < 1 || !c_at) return CIE_BAD_ARGUMENT;
+    if (M == 0) return CIE_OK;
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && on_16_bytes(A) && on_16_bytes(W);
+    Product p{A, W, nullptr, nullptr, nullptr, M, N, K, lda, N, units, {}};
+    p.beside.c_at = c_at;
+    run_few<false, kPointed>(static_cast<hipStream_t>(stream), p, vec);
+    return cie_after_launch();
+}
+
 // Up to 8 rows, and rows * ceil(K / 512) up to 32: C [M, N / 2] = the gated unit of norm(rows of the stream [M, K], contiguous) W^T.
 // K a multiple of 8, up to 8,192; stream, W and the norm's weight at multiples of 16 bytes.
 CIE_API int cie_gemm_f32_normed(void* stream, const float* rows, const float* norm_weight, float eps, const float* W, float* C, int M,
@@ -917,7 +930,7 @@ CIE_API int cie_gemm_f32_normed_rope(void* stream, const float* rows, const floa
         return CIE_BAD_ARGUMENT;
     const Product p{rows, W, bias, C, nullptr, M, N, K, K, N, units,
                     {norm_weight, eps, cos_table, sin_table, positions, seq_of_token, seq_slot, block_table, table_width, k_pool,
-                     v_pool, q_heads, kv_heads, head_dim, rotary_dim, page_size, rotate, write_kv}};
+                     v_pool, q_heads, kv_heads, head_dim, rotary_dim, page_size, rotate, write_kv, nullptr}};
     run_normed_rope(static_cast<hipStream_t>(stream), p);
     return cie_after_launch();
 }

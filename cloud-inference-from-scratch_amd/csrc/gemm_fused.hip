@@ -92,6 +92,8 @@ struct FusedArgs {
     bf16_t* act_out;
     long act_ld;
     RopeArgs rope;         // ROPE only
+    // F32: where the result's address lies on the device, or null (`c` then): a captured launch writes where its replay says
+    float* const* c_at = nullptr;
 };
 
 // One 16x16 tile of results in its MFMA layout: lane (r, g) holds rows g*4+i of column r.
@@ -404,6 +406,7 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_rows_kernel(FusedArgs a) {
     float* reduce = reinterpret_cast<float*>(shared);
     char* stage = shared + (threadIdx.x / kWave) * kStageTile;
     __shared__ float fold_sq[FOLD > 0 ? WAVES * kFoldRows : 1];  // the waves' shares of the rows' sums of squares
+    if (EPI == EPI_F32 && a.c_at) a.c = *a.c_at;
 
     const int lane = threadIdx.x % kWave;
     const int wave = threadIdx.x / kWave;
@@ -855,6 +858,7 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_shared_rows_kernel(ARGS a) {
     const int g = lane >> 4;
     char* stage_w = shared + kStagesA * kStageBytesA + wave * kStageTile;
     float* scale_lds = reinterpret_cast<float*>(shared + kStagesA * kStageBytesA + kWaves * kStageTile);
+    if (EPI == EPI_F32 && a.c_at) a.c = *a.c_at;
     constexpr bool kBeside = std::is_same_v<ARGS, BesideArgs>;
     static_assert(!kBeside || ((EPI == EPI_SILU || EPI == EPI_PARTIAL) && FOLD == 0), "two products: SiLU and plain, or parts");
     bool second = false;  // (the same for the workgroup)
@@ -1178,19 +1182,21 @@ int launch_shared_rows(hipStream_t s, int waves, int k_parts, const FusedArgs& a
 // norm_weight [N] float32 and scaled_out [M, N] bf16 (both or neither; RESID only): the epilogue also writes
 // the new residual times the weight.  row_sumsq [M, sumsq_parts] and eps (SILU with one row tile only): the
 // rows of `a` lack the factor rsqrt(sum of the row's partial sums / K + eps), applied before the SiLU.
+// c_at (F32 only): see FusedArgs.
 // act_out (BF16 only): columns from `split` on go there, squared behind relu; `c` is [M, split].
 CIE_API int cie_gemm_fused(void* stream, const void* a, int lda, const void* w, const void* bias, void* c,
                            float* residual, float* sumsq, int M, int N, int K, int epilogue, int row_tiles,
                            int waves, int column_tiles, const float* norm_weight, void* scaled_out,
                            const float* row_sumsq, int sumsq_parts, float eps, int split, void* act_out,
-                           long act_ld) {
+                           long act_ld, float* const* c_at) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 8 || !a || !w || lda < K || lda % 8) return CIE_BAD_ARGUMENT;
     if (act_out && (epilogue != EPI_BF16 || split < 1 || split >= N || act_ld < N - split)) return CIE_BAD_ARGUMENT;
     if (row_tiles != 1 && row_tiles != 2 && row_tiles != 4) return CIE_BAD_ARGUMENT;
     if (waves != 1 && waves != 2 && waves != 4 && waves != 8) return CIE_BAD_ARGUMENT;
     if (epilogue == EPI_SILU && (N % 2 || bias)) return CIE_BAD_ARGUMENT;
     if (epilogue == EPI_RESID && (!residual || !sumsq)) return CIE_BAD_ARGUMENT;
-    if (epilogue != EPI_RESID && !c) return CIE_BAD_ARGUMENT;
+    if (epilogue != EPI_RESID && !c && !c_at) return CIE_BAD_ARGUMENT;
+    if (c_at && epilogue != EPI_F32) return CIE_BAD_ARGUMENT;
     // the folded norm: a scaled copy needs the weight and the RESID epilogue; rows that lack their scale
     // are taken by the SILU epilogue of one row tile
     if ((scaled_out != nullptr) != (norm_weight != nullptr) || (scaled_out && epilogue != EPI_RESID)) return CIE_BAD_ARGUMENT;
@@ -1220,6 +1226,7 @@ CIE_API int cie_gemm_fused(void* stream, const void* a, int lda, const void* w, 
     f.act_out = static_cast<bf16_t*>(act_out);
     f.act_ld = act_ld;
     f.rope = RopeArgs{};
+    f.c_at = c_at;
     hipStream_t s = static_cast<hipStream_t>(stream);
     switch (epilogue) {
         case EPI_BF16: return launch<EPI_BF16>(s, row_tiles, waves, column_tiles, f);
@@ -1354,8 +1361,9 @@ CIE_API int cie_gemm_qkv_rope_folded_norm(void* stream, const float* residual,
 // 16 columns per wave (SiLU: the gate tile and its up tile), 2 to 4 waves per workgroup.
 CIE_API int cie_gemm_shared_rows(void* stream, const void* a, int lda, const void* w, const void* bias, void* c, int M,
                                  int N, int K, int epilogue, int column_tiles, int waves, int k_parts,
-                                 const float* row_sumsq, int sumsq_parts, float eps) {
-    if (M <= 0 || M > 128 || N <= 0 || K <= 0 || K % 8 || !a || !w || !c || lda < K || lda % 8) return CIE_BAD_ARGUMENT;
+                                 const float* row_sumsq, int sumsq_parts, float eps, float* const* c_at) {
+    if (M <= 0 || M > 128 || N <= 0 || K <= 0 || K % 8 || !a || !w || (!c && !c_at) || lda < K || lda % 8) return CIE_BAD_ARGUMENT;
+    if (c_at && epilogue != EPI_F32) return CIE_BAD_ARGUMENT;
     if (epilogue != EPI_BF16 && epilogue != EPI_F32 && epilogue != EPI_SILU && epilogue != EPI_PARTIAL && epilogue != EPI_ATOMIC)
         return CIE_BAD_ARGUMENT;
     if (epilogue == EPI_SILU && (N % 2 || bias || column_tiles != 2)) return CIE_BAD_ARGUMENT;
@@ -1386,6 +1394,7 @@ CIE_API int cie_gemm_shared_rows(void* stream, const void* a, int lda, const voi
     f.act_out = nullptr;
     f.act_ld = 0;
     f.rope = RopeArgs{};
+    f.c_at = c_at;
     hipStream_t s = static_cast<hipStream_t>(stream);
     switch (epilogue) {
         case EPI_SILU: return launch_shared_rows<EPI_SILU, 2>(s, waves, 1, f);

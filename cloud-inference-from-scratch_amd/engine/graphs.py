@@ -20,6 +20,7 @@ from collections.abc import Iterator, Sequence
 from dataclasses import dataclass
 from typing import Any
 
+import numpy as np
 import torch
 
 from ..kernels import ops
@@ -58,6 +59,7 @@ class _Bucket:
                  token_pool: torch.Tensor | None = None) -> None:
         self.size = size
         count = 11 * size + 2
+        count += count % 2 + 2  # (behind them, on 8 bytes, the address of the logits)
         self.host = torch.zeros(count, dtype=torch.int32)  # the template; every replay stages a copy of it
         self.dev = torch.zeros(count, dtype=torch.int32, device=device)
         names = ["token_ids", "positions", "seq_of_token", "seq_slot", "seq_start", "seq_q_len"]
@@ -72,7 +74,8 @@ class _Bucket:
             self.offsets[name] = offset
             offset += size
         self.offsets["max_context"] = offset
-        assert offset + 1 == count
+        self.offsets["logits_at"] = count - 2
+        assert offset + 1 <= count - 2 and count % 2 == 0
         arange = torch.arange(size + 1, dtype=torch.int32)
         o = self.offsets
         self.host[o["seq_of_token"]: o["seq_of_token"] + size] = arange[:size]
@@ -94,17 +97,19 @@ class _Bucket:
             host_slots=[pad_slot] * size, host_starts=[0] * size, host_q_lens=[1] * size,
             static_plan=StaticPlan(view("tile_seq"), view("tile_q0"), view("max_context", 1), max_keys),
             token_feed=view("token_feed") if token_pool is not None else None, token_pool=token_pool,
+            logits_at=view("logits_at", 2).view(torch.int64),
         )
         # what a replay rewrites, for the kernel that does (its arguments carry the numbers: a pinned buffer, a copy into it and
         # one to the device were 14 us of the host's 75 a step of the smallest model, and 3.6 against 2 us of the GPU's)
         self.places = tuple(view(name) for name in ("token_ids", "positions", "seq_start", "seq_slot", "token_feed")) + (view("max_context", 1),)
         self.graph: Any = None
-        self.logits: torch.Tensor | None = None
+        self.logits: torch.Tensor | None = None  # the graph's own; None: they go where a replay's ``logits_at`` says
 
     def fill(self, tokens: Sequence[int], positions: Sequence[int], slots: Sequence[int], max_context: int,
-             feed: Sequence[int] | None = None) -> None:
+             feed: Sequence[int] | None = None, logits: torch.Tensor | None = None) -> None:
         """Real rows first, the rest padding: token 0 at position 0 of the pad slot.  ``feed[i] >= 0``:
-        row i takes the token at that place of the token pool on the device instead of ``tokens[i]``."""
+        row i takes the token at that place of the token pool on the device instead of ``tokens[i]``.  ``logits``: where the
+        step's logits go."""
         # (numpy views: five tensors made of lists took 25 us of the some 100 that the host needs for a step, and a small
         # model's step is no longer on the GPU)
         o, size, n = self.offsets, self.size, len(tokens)
@@ -121,6 +126,7 @@ class _Bucket:
         put("seq_start", positions, 0)
         put("seq_slot", slots, self.pad_slot)
         host[o["max_context"]] = max(1, max_context)
+        host[o["logits_at"]: o["logits_at"] + 2].view(np.int64)[0] = logits.data_ptr() if logits is not None else 0
 
 
 class DecodeGraphs:
@@ -145,6 +151,9 @@ class DecodeGraphs:
         runner = self.runner
         bucket = _Bucket(size, runner.device, runner.device_cache.pad_slot, runner.config.max_model_len,
                          self.token_pool)
+        logits = self._logits(size)  # (of the run on padding)
+        bucket.fill([], [], [], 1, logits=logits)
+        bucket.dev.copy_(bucket.host)
         torch.cuda.synchronize()
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
@@ -152,6 +161,7 @@ class DecodeGraphs:
             runner.model.forward(bucket.batch, runner.device_cache)
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
+        del logits
         graph = torch.cuda.CUDAGraph()
         if self.pool is None:
             self.pool = torch.cuda.graph_pool_handle()
@@ -161,6 +171,9 @@ class DecodeGraphs:
         self.buckets[size] = bucket
         self.captures += 1
         return bucket
+
+    def _logits(self, size: int) -> torch.Tensor:
+        return torch.empty((size, self.runner.model.head.shape[0]), dtype=torch.float32, device=self.runner.device)
 
     def capture_all(self) -> int:
         """Capture every bucket that is not captured yet (rows of padding only), so that no later step
@@ -177,32 +190,38 @@ class DecodeGraphs:
     def run(self, entries: Sequence[Any], feed: Sequence[int] | None = None, borrow: bool = False) -> torch.Tensor:
         """Replay the bucket's graph for single-token entries; logits [wanted, vocab].  ``feed[i] >= 0``:
         entry i's token is the one at that place of ``token_pool`` (its own ``tokens`` are ignored).
-        The graph writes its logits into one buffer of its own, which the bucket's next replay overwrites:
-        the caller gets a copy, unless it ``borrow``s the buffer (sampling that is queued on the same
-        stream right behind the replay has read it before the next replay can start)."""
+        The last product writes the logits into a matrix of this replay's (its address is one of the numbers that a replay
+        brings: a copy of them was 15 us of a step of 64 sequences, 4 and a launch of a step of one).  Where another kernel makes
+        the logits the graph has a buffer of its own, which the bucket's next replay overwrites: the caller then gets a copy,
+        unless it ``borrow``s the buffer (sampling that is queued on the same stream right behind the replay has read it before
+        the next replay can start)."""
         runner = self.runner
         size = self.bucket_of(len(entries))
         bucket = self.buckets.get(size) or self._capture(size)
         cache = runner.cache
         positions = [e.start_pos for e in entries]
         tokens, slots = [e.tokens[0] for e in entries], [cache.slot(e.request_id) for e in entries]
+        logits = self._logits(size) if bucket.logits is None else None
         if size <= ops.STEP_ROWS:
             values = array("i", tokens)
             for more in (positions, slots) if feed is None else (positions, slots, feed):
                 values.extend(more)
-            ops.step_rows(values, len(tokens), size, feed is not None, max(positions) + 1, bucket.pad_slot, *bucket.places)
+            ops.step_rows(values, len(tokens), size, feed is not None, max(positions) + 1, bucket.pad_slot, *bucket.places,
+                          None if logits is None else bucket.batch.logits_at, logits)
         else:
-            bucket.fill(tokens, positions, slots, max(positions) + 1, feed)
+            bucket.fill(tokens, positions, slots, max(positions) + 1, feed, logits)
             bucket.dev.copy_(to_device_staging(bucket.host, runner.device), non_blocking=True)
         bucket.graph.replay()
         self.replays += 1
         rows = [index for index, e in enumerate(entries) for _ in e.want]
         if rows == list(range(len(entries))):
+            if logits is not None:
+                return logits[: len(entries)]
             view = bucket.logits[: len(entries)]
             return view if borrow else view.clone()
         # (the index goes over as an asynchronous copy: a tensor made on the device from a list would wait for the replay)
         index = to_device_staging(rows, runner.device).to(runner.device, non_blocking=True).long()
-        return bucket.logits.index_select(0, index)
+        return (bucket.logits if logits is None else logits).index_select(0, index)
 
 
 @dataclass

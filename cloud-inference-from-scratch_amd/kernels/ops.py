@@ -208,10 +208,14 @@ STEP_ROWS = 128  # rows of a captured decode step whose numbers travel as a kern
 
 def step_rows(values: "array.array", n: int, size: int, fed: bool, max_context: int, pad_slot: int, token_ids: torch.Tensor,
               positions: torch.Tensor, seq_start: torch.Tensor, seq_slot: torch.Tensor, token_feed: torch.Tensor,
-              max_context_at: torch.Tensor) -> None:
+              max_context_at: torch.Tensor, result_at: Optional[torch.Tensor] = None, result: Optional[torch.Tensor] = None) -> None:
     """Write what changes between two replays of a captured decode step of ``size`` rows: ``values`` (a host array of C ints)
     holds its ``n`` tokens, positions and slots and, if ``fed``, the places of the token pool they are taken from.  Rows beyond
-    ``n`` become padding on ``pad_slot``."""
+    ``n`` become padding on ``pad_slot``.  ``result_at`` (int64 [1]) takes the address of ``result``, which the step's last product
+    writes to."""
+    if (result_at is None) != (result is None) or (result_at is not None and not (
+            result_at.is_cuda and result_at.dtype == torch.int64 and result_at.numel() == 1 and result.is_cuda)):
+        raise ValueError("a result and the place of its address come together")
     if not (values.typecode == "i" and values.itemsize == 4 and len(values) == (4 if fed else 3) * n and 0 <= n <= size <= STEP_ROWS):
         raise ValueError(f"{len(values)} numbers for {n} of {size} rows")
     for at, least in ((token_ids, size), (positions, size), (seq_start, size), (seq_slot, size), (token_feed, size), (max_context_at, 1)):
@@ -219,7 +223,12 @@ def step_rows(values: "array.array", n: int, size: int, fed: bool, max_context: 
             raise ValueError(f"a place of {size} int32 numbers is {tuple(at.shape)} {at.dtype}")
     _run("cie_step_rows", load_library().cie_step_rows(
         _stream(), values.buffer_info()[0], _i(n), _i(size), _i(fed), _i(max_context), _i(pad_slot), _ptr(token_ids), _ptr(positions),
-        _ptr(seq_start), _ptr(seq_slot), _ptr(token_feed), _ptr(max_context_at)))
+        _ptr(seq_start), _ptr(seq_slot), _ptr(token_feed), _ptr(max_context_at), _ptr(result_at), _ptr(result)))
+
+
+def _result_at(out_at: torch.Tensor) -> None:
+    if not (out_at.is_cuda and out_at.dtype == torch.int64 and out_at.numel() == 1):
+        raise ValueError("the place of a result's address is one int64 number on the GPU")
 
 
 MAX_NORM_WIDTH = 16384  # a row of the norm kernels is held in 64 KB of LDS as float32
@@ -731,6 +740,19 @@ def gemm_f32_into(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
         _stream(), _ptr(a), _ptr(weight), _ptr(bias), _ptr(into), _i(m), _i(n), _i(k), _i(lda), _i(n), _i(compute_units(a.device))))
 
 
+def gemm_f32_at(a: torch.Tensor, weight: torch.Tensor, out_at: torch.Tensor) -> None:
+    """``a @ weight.T`` of up to ``F32_FEW_ROWS`` rows into the contiguous float32 [M, N] whose address ``out_at`` (int64 [1], on
+    the GPU) holds when the kernel runs (the caller vouches for it), with the bits of :func:`gemm_f32`."""
+    _result_at(out_at)
+    _gpu("weight", weight, torch.float32, 2)
+    (m, k), n = a.shape, weight.shape[0]
+    if not (a.is_cuda and a.dtype == torch.float32 and a.stride(1) == 1 and weight.shape[1] == k and 1 <= m <= F32_FEW_ROWS):
+        raise ValueError(f"a {tuple(a.shape)} vs weight {tuple(weight.shape)}, up to {F32_FEW_ROWS} float32 rows with unit inner stride")
+    _run("cie_gemm_f32_at", load_library().cie_gemm_f32_at(
+        _stream(), _ptr(a), _ptr(weight), _ptr(out_at), _i(m), _i(n), _i(k), _i(a.stride(0) if m > 1 else max(a.stride(0), k)),
+        _i(compute_units(a.device))))
+
+
 def gemm_f32_qkv_rope(stream: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor,
                       bias: Optional[torch.Tensor], cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor,
                       seq_of_token: torch.Tensor, seq_slot: torch.Tensor, block_table: torch.Tensor, k_pool: torch.Tensor,
@@ -796,7 +818,7 @@ def gemm_fused(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias: Optio
                plan: Optional[tuple[int, int, int]] = None,
                norm_weight: Optional[torch.Tensor] = None, scaled_out: Optional[torch.Tensor] = None,
                row_sumsq: Optional[torch.Tensor] = None, eps: float = 0.0,
-               act_out: Optional[torch.Tensor] = None) -> torch.Tensor:
+               act_out: Optional[torch.Tensor] = None, out_at: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """Few-row matrix product ``a @ weight.T`` (bf16 operands, float32 sums) fused
     with its neighbour.  ``epilogue``: ``EPI_BF16`` / ``EPI_F32`` return
     ``a W^T + bias``; ``EPI_SILU`` (weight = gate rows over up rows) returns
@@ -809,7 +831,8 @@ def gemm_fused(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias: Optio
     given these rows as ``a`` with ``row_sumsq`` (the former's result) and ``eps``,
     multiplies its sums by each row's ``rsqrt(mean square + eps)`` before the SiLU.
     ``act_out`` (bf16 [M, n], rows may lie apart; ``EPI_BF16``): the last n columns go there, squared behind relu, and the
-    result that comes back holds the columns in front of them."""
+    result that comes back holds the columns in front of them.  ``out_at`` (int64 [1] on the GPU; ``EPI_F32``): the result goes
+    to the contiguous float32 [M, N] whose address it holds when the kernel runs (the caller vouches for it), and none comes back."""
     _gpu("weight", weight, torch.bfloat16, 2)
     n, k = weight.shape
     if not (a.is_cuda and a.dtype == torch.bfloat16 and a.dim() == 2 and a.stride(1) == 1):
@@ -847,7 +870,7 @@ def gemm_fused(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias: Optio
     if epilogue == EPI_BF16:
         out = torch.empty((m, split), dtype=torch.bfloat16, device=device)
     elif epilogue == EPI_F32:
-        out = torch.empty((m, n), dtype=torch.float32, device=device)
+        out = torch.empty((m, n), dtype=torch.float32, device=device) if out_at is None else None
     elif epilogue == EPI_SILU:
         if not (n % 2 == 0):
             raise ValueError(f"the SiLU epilogue needs an even N, got {n}")
@@ -874,6 +897,10 @@ def gemm_fused(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias: Optio
         _gpu("scaled_out", scaled_out, torch.bfloat16, 2)
         if not (norm_weight.shape[0] == n and scaled_out.shape == (m, n)):
             raise ValueError(f"norm_weight {tuple(norm_weight.shape)} / scaled_out {tuple(scaled_out.shape)} vs {(m, n)}")
+    if out_at is not None:
+        _result_at(out_at)
+        if epilogue != EPI_F32:
+            raise ValueError("only a float32 result goes to an address on the device")
     parts_in = 0
     if row_sumsq is not None:
         _gpu("row_sumsq", row_sumsq, torch.float32, 2)
@@ -883,7 +910,7 @@ def gemm_fused(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias: Optio
     _run("cie_gemm_fused", load_library().cie_gemm_fused(
         _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(None if epilogue == EPI_RESID else out),
         _ptr(residual), _ptr(sumsq), _i(m), _i(n), _i(k), _i(epilogue), _i(row_tiles), _i(waves), _i(column_tiles),
-        _ptr(norm_weight), _ptr(scaled_out), _ptr(row_sumsq), _i(parts_in), _f(eps), _i(split), _ptr(act_out), act_ld))
+        _ptr(norm_weight), _ptr(scaled_out), _ptr(row_sumsq), _i(parts_in), _f(eps), _i(split), _ptr(act_out), act_ld, _ptr(out_at)))
     return out
 
 
@@ -893,7 +920,7 @@ SHARED_ROWS_MAX = 128  # rows of the form whose waves share the rows of A
 def gemm_shared_rows(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias: Optional[torch.Tensor] = None,
                      column_tiles: int = 2, waves: int = 4, k_parts: int = 1,
                      row_sumsq: Optional[torch.Tensor] = None, eps: float = 0.0,
-                     add_into: Optional[torch.Tensor] = None) -> torch.Tensor:
+                     add_into: Optional[torch.Tensor] = None, out_at: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``a @ weight.T`` for 17 to 128 rows (it takes fewer too) in the form whose four waves per
     workgroup own columns and share each slice of ``a`` through LDS: ``EPI_BF16`` or ``EPI_F32`` (+ bias),
     ``EPI_SILU`` (weight = gate rows over up rows; with ``row_sumsq`` and ``eps`` the rows of ``a``
@@ -901,7 +928,8 @@ def gemm_shared_rows(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias:
     (``k_parts`` float32 partial products [k_parts, M, N], bias in part 0) or ``EPI_ATOMIC``
     (each of the ``k_parts`` parts of K adds its products into ``add_into``, float32 [M, N], with the
     hardware's atomic float add: no partial products to sum afterwards, and no fixed order of the sums;
-    ``add_into`` comes back).  ``column_tiles`` tiles of 16 columns per wave, ``waves`` waves per workgroup."""
+    ``add_into`` comes back).  ``column_tiles`` tiles of 16 columns per wave, ``waves`` waves per workgroup.
+    ``out_at`` (``EPI_F32``): as in :func:`gemm_fused`."""
     _gpu("weight", weight, torch.bfloat16, 2)
     n, k = weight.shape
     if not (a.is_cuda and a.dtype == torch.bfloat16 and a.dim() == 2 and a.stride(1) == 1):
@@ -941,7 +969,12 @@ def gemm_shared_rows(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias:
             raise ValueError("rows that lack their scale go to the SiLU epilogue, with a positive eps")
         parts_in = row_sumsq.shape[1]
     device = weight.device
-    if epilogue == EPI_BF16:
+    if out_at is not None:
+        _result_at(out_at)
+        if epilogue != EPI_F32:
+            raise ValueError("only a float32 result goes to an address on the device")
+        out = None
+    elif epilogue == EPI_BF16:
         out = torch.empty((m, n), dtype=torch.bfloat16, device=device)
     elif epilogue == EPI_F32:
         out = torch.empty((m, n), dtype=torch.float32, device=device)
@@ -953,7 +986,7 @@ def gemm_shared_rows(weight: torch.Tensor, epilogue: int, a: torch.Tensor, bias:
         out = torch.empty((k_parts, m, n), dtype=torch.float32, device=device)
     _run("cie_gemm_shared_rows", load_library().cie_gemm_shared_rows(
         _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k), _i(epilogue),
-        _i(column_tiles), _i(waves), _i(k_parts), _ptr(row_sumsq), _i(parts_in), _f(eps)))
+        _i(column_tiles), _i(waves), _i(k_parts), _ptr(row_sumsq), _i(parts_in), _f(eps), _ptr(out_at)))
     return out
 
 

@@ -548,6 +548,29 @@ def linear_beside(x: torch.Tensor, weight: torch.Tensor, act_out: torch.Tensor) 
     return out[:, :split]
 
 
+def logits_at(x: torch.Tensor, weight: torch.Tensor, out_at: torch.Tensor) -> bool:
+    """``x @ weight.T`` in float32 into the contiguous matrix whose address ``out_at`` holds when the kernel runs, if the form that
+    :func:`linear` takes for it can write there; else nothing is done."""
+    rows, k = x.shape
+    n = weight.shape[0]
+    if not (x.is_cuda and rows >= 1 and x.stride(1) == 1):
+        return False
+    if weight.dtype == torch.float32:
+        if x.dtype != torch.float32 or rows > ops.F32_FEW_ROWS:
+            return False
+        ops.gemm_f32_at(x, weight, out_at)
+        return True
+    if not _fusable(rows, k, x.stride(0) if rows > 1 else k, weight) or x.data_ptr() % 16 or weight.data_ptr() % 16:
+        return False
+    if shares_rows_f32(rows, n, k):
+        ops.gemm_shared_rows(weight, ops.EPI_F32, x, waves=4, out_at=out_at)
+        return True
+    if rows > FUSED_LOGIT_ROWS:
+        return False
+    ops.gemm_fused(weight, ops.EPI_F32, x, out_at=out_at)
+    return True
+
+
 # Two products of few rows that wait for the same things run in one launch (a layer whose mixer and feed-forward read the same
 # stream; MI355X, us, apart and together, 1 / 8 / 16 rows): gate/up and 6,144 columns of the 3B widths 27.5, 24.0 / 27.3, 23.3 / 28.4, 23.4,
 # 4,096 columns 24.0, 21.8 / 24.9, 22.0 / 25.7, 22.0; 0.5B and 2,304 10.7, 7.5 / 11.3, 7.6 / 11.5, 7.7; 7B and 7,168 65.7, 59.5 / 68.3,

@@ -6,7 +6,7 @@ src/cloud_engine/model.py:194-228).
 
 from __future__ import annotations
 
-from typing import Any
+from typing import Any, Optional
 
 import torch
 
@@ -16,7 +16,7 @@ from ..weights.loader import torch_dtype
 from ..weights.tensors import TensorSpec
 from .base import BLOCKS, build_part, declares
 from .block import NormedRows, normalise, whole_stream
-from .linear import StreamRows, linear
+from .linear import StreamRows, linear, logits_at
 
 
 def _blocks(spec: ModelSpec) -> list[Any]:
@@ -172,8 +172,9 @@ class DecoderModel:
                 for rows in row_counts:
                     warm(rows)
 
-    def forward(self, batch, cache) -> torch.Tensor:
-        """Run the step's tokens; float32 logits ``[len(logit_rows), vocab]``."""
+    def forward(self, batch, cache) -> Optional[torch.Tensor]:
+        """Run the step's tokens; float32 logits ``[len(logit_rows), vocab]``, or ``None`` if they went where ``batch.logits_at``
+        points."""
         history = None
         if self.keeps_history:
             history = torch.empty((len(self.spec.order) + 1, batch.token_ids.shape[0], self.embedding.shape[1]),
@@ -232,6 +233,9 @@ class DecoderModel:
         if batch.logit_rows.shape[0] == 0:  # a step of prompt portions that end before their prompts do
             return torch.empty((0, self.head.shape[0]), dtype=torch.float32, device=residual.device)
         selected = normalise(self.final_norm, residual, pending, self.dtype, rows=batch.logit_rows)
+        if getattr(batch, "logits_at", None) is not None and (self.spec.logit_scale == 1.0 or self.folded_scale) and self.spec.logit_softcap is None \
+                and logits_at(selected, self.head, batch.logits_at):
+            return None
         logits = linear(selected, self.head, None, out_dtype=torch.float32)
         if self.spec.logit_scale != 1.0 and not self.folded_scale:
             logits.mul_(self.spec.logit_scale)

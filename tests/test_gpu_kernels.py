@@ -1783,3 +1783,33 @@ def test_gemm_parts_beside(ops, shape):
     stream = rand((m, n), torch.float32, 6)
     got, _ = ops.depth_stream(stream, parts=out, mult=0.5, out_dtype=torch.bfloat16)  # (parts and no other branch)
     torch.testing.assert_close(got.double(), stream.double() + 0.5 * want, rtol=1e-6, atol=4e-6 * math.sqrt(k + k2))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 4099, 136), (3, 2050, 1024), (8, 40000, 256), (8, 513, 2056), (40, 300, 264), (80, 50304, 128)])
+def test_logits_go_where_an_address_says(ops, dtype, shape):
+    """A result whose address lies on the device has the bits of one that comes back, and nothing around it is touched; replays
+    of a captured launch follow the address."""
+    from cie_amd.parts import linear as L
+
+    m, n, k = shape
+    a, w = rand((m, k), dtype, 1), rand((n, k), dtype, 2)
+    want = L.linear(a, w, out_dtype=torch.float32)
+    outs = [torch.full((m + 2, n), 7.0).cuda() for _ in range(3)]
+    at = torch.tensor([outs[0].data_ptr() + 4 * n], dtype=torch.int64).cuda()
+    wrote = L.logits_at(a, w, at)
+    assert wrote == (dtype == torch.bfloat16 or m <= ops.F32_FEW_ROWS)
+    if not wrote:
+        assert (outs[0] == 7.0).all()
+        return
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert L.logits_at(a, w, at)
+    for out in outs[1:]:
+        at.copy_(torch.tensor([out.data_ptr() + 4 * n]))
+        graph.replay()
+    for out in outs:
+        assert torch.equal(out[1: m + 1], want) and (out[0] == 7.0).all() and (out[m + 1] == 7.0).all()
+    with pytest.raises(ValueError):
+        ops.gemm_fused(w.bfloat16(), ops.EPI_BF16, a.bfloat16()[:1], out_at=at)
