@@ -665,13 +665,22 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_rows_kernel(FusedArgs a) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             if (wave != mt % WAVES) continue;  // wave-uniform
+            // (this wave's own sums in their place: every form gives a row the same bits where as many waves share K)
+            floatx4 own[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) own[t] = acc[mt][t];
 #pragma unroll 1
-            for (int slot = 0; slot < WAVES - 1; ++slot)
+            for (int w = 0; w < WAVES; ++w) {
+                const int slot = min(w - (w > mt), WAVES - 2);
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        acc[mt][t][i] += reduce[(((mt * (WAVES - 1) + slot) * NT + t) * 4 + i) * 64 + lane];
+                    for (int i = 0; i < 4; ++i) {
+                        const float other = reduce[(((mt * (WAVES - 1) + slot) * NT + t) * 4 + i) * 64 + lane];
+                        const float part = w == mt ? own[t][i] : other;
+                        acc[mt][t][i] = w == 0 ? part : acc[mt][t][i] + part;
+                    }
+            }
             if constexpr (EPI == EPI_RESID) {
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
@@ -1241,11 +1250,9 @@ CIE_API int cie_gemm_fused(void* stream, const void* a, int lda, const void* w, 
 // streaming the weight again): `w` [N, K] stacks the rows of q_heads query
 // heads, kv_heads key heads and kv_heads value heads of head_dim dimensions each (a multiple of 32);
 // `c` [M, N] receives the rotated queries (its key and value columns are left alone); rotated keys and
-// values go to the cache page of each row's position.  `waves` waves per workgroup share K (1, 2, 4, 8;
-// with more than 16 rows 4 or 8).
-// (Below this many pairs of tiles a product of up to 64 rows takes one tile a workgroup: the 3B shape's 80 pairs
-// leave two thirds of the compute units without a workgroup; 64 rows 12.1 -> 10.9 us.)
-constexpr unsigned kSplitPairsBelow = 128;
+// values go to the cache page of each row's position.  row_tiles 1, 2, 4: 16, 32, 64 rows per workgroup (more rows: more
+// workgroups, each streaming W again); `waves` waves of it share K (1, 2, 4, 8; with more than one row tile 4 or 8); one_tile:
+// 16 columns a workgroup, else a pair of tiles.
 
 namespace {
 struct FoldedNorm {  // the norm in front of the q/k/v product, made by the product itself (see FusedArgs)
@@ -1255,16 +1262,17 @@ struct FoldedNorm {  // the norm in front of the q/k/v product, made by the prod
 };
 
 int qkv_rope(void* stream, const void* a, int lda, const void* w, const void* bias, void* c,
-             int M, int N, int K, int waves, const float* cos_table, const float* sin_table,
+             int M, int N, int K, int row_tiles, int waves, int one_tile, const float* cos_table, const float* sin_table,
              const int* positions, const int* seq_of_token, const int* seq_slot,
              const int* block_table, int table_width, void* k_pool, void* v_pool, int q_heads,
              int kv_heads, int head_dim, int page_size, int rotate, int write_kv, const FoldedNorm* fold) {
+    if (row_tiles != 1 && row_tiles != 2 && row_tiles != 4) return CIE_BAD_ARGUMENT;
     if (fold) {
-        if (M <= 0 || M > kFoldRows || K < 8 || K % 8 || !w || !c) return CIE_BAD_ARGUMENT;
+        if (M <= 0 || M > kFoldRows || row_tiles != 1 || K < 8 || K % 8 || !w || !c) return CIE_BAD_ARGUMENT;
         if (!fold->residual || !fold->weight || !(fold->eps > 0.f)) return CIE_BAD_ARGUMENT;
         a = nullptr;
         lda = K;
-    } else if (M <= 0 || (M + 63) / 64 > 65535 || K <= 0 || K % 8 || !a || !w || !c || lda < K || lda % 8) {
+    } else if (M <= 0 || (M + 16L * row_tiles - 1) / (16 * row_tiles) > 65535 || K <= 0 || K % 8 || !a || !w || !c || lda < K || lda % 8) {
         return CIE_BAD_ARGUMENT;
     }
     if (q_heads <= 0 || kv_heads <= 0 || head_dim <= 0 || head_dim % 32 || page_size <= 0 || table_width <= 0 ||
@@ -1299,10 +1307,9 @@ int qkv_rope(void* stream, const void* a, int lda, const void* w, const void* bi
     f.rope = RopeArgs{cos_table, sin_table, positions, seq_of_token, seq_slot, block_table, table_width,
                       static_cast<bf16_t*>(k_pool), static_cast<bf16_t*>(v_pool), q_heads, kv_heads, head_dim,
                       page_size, rotate, write_kv};
-    const dim3 grid((q_heads + 2 * kv_heads) * (head_dim / 32), M <= 64 ? 1 : (M + 63) / 64, 1);
+    const unsigned blocks = (M + 16 * row_tiles - 1) / (16 * row_tiles);
+    const dim3 grid((q_heads + 2 * kv_heads) * (head_dim / 32), blocks, 1), twice(2 * grid.x, blocks, 1);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 twice((q_heads + 2 * kv_heads) * (head_dim / 16), 1, 1);
-    const bool one_tile = M <= 16 && grid.x < kSplitPairsBelow;  // few columns: one tile a workgroup, twice the workgroups
     if (fold) {
         f.fold_residual = fold->residual;
         f.fold_weight = fold->weight;
@@ -1314,23 +1321,23 @@ int qkv_rope(void* stream, const void* a, int lda, const void* w, const void* bi
         if (one_tile) return launch_waves<EPI_ROPE8, 1, 1, 4>(s, waves, twice, f);
         return launch_waves<EPI_ROPE, 1, 2, 4>(s, waves, grid, f);
     }
-    if (one_tile) return launch_waves<EPI_ROPE8, 1, 1>(s, waves, twice, f);
-    if (M <= 64 && grid.x < kSplitPairsBelow) {  // the same with more row tiles
-        if (M <= 32) return launch_waves<EPI_ROPE8, 2, 1>(s, waves, twice, f);
+    if (one_tile) {
+        if (row_tiles == 1) return launch_waves<EPI_ROPE8, 1, 1>(s, waves, twice, f);
+        if (row_tiles == 2) return launch_waves<EPI_ROPE8, 2, 1>(s, waves, twice, f);
         return launch_waves<EPI_ROPE8, 4, 1>(s, waves, twice, f);
     }
-    if (M <= 16) return launch_waves<EPI_ROPE, 1, 2>(s, waves, grid, f);
-    if (M <= 32) return launch_waves<EPI_ROPE, 2, 2>(s, waves, grid, f);
+    if (row_tiles == 1) return launch_waves<EPI_ROPE, 1, 2>(s, waves, grid, f);
+    if (row_tiles == 2) return launch_waves<EPI_ROPE, 2, 2>(s, waves, grid, f);
     return launch_waves<EPI_ROPE, 4, 2>(s, waves, grid, f);
 }
 }  // namespace
 
 CIE_API int cie_gemm_qkv_rope(void* stream, const void* a, int lda, const void* w, const void* bias, void* c,
-                              int M, int N, int K, int waves, const float* cos_table, const float* sin_table,
-                              const int* positions, const int* seq_of_token, const int* seq_slot,
+                              int M, int N, int K, int row_tiles, int waves, int one_tile, const float* cos_table,
+                              const float* sin_table, const int* positions, const int* seq_of_token, const int* seq_slot,
                               const int* block_table, int table_width, void* k_pool, void* v_pool, int q_heads,
                               int kv_heads, int head_dim, int page_size, int rotate, int write_kv) {
-    return qkv_rope(stream, a, lda, w, bias, c, M, N, K, waves, cos_table, sin_table, positions, seq_of_token, seq_slot,
+    return qkv_rope(stream, a, lda, w, bias, c, M, N, K, row_tiles, waves, one_tile, cos_table, sin_table, positions, seq_of_token, seq_slot,
                     block_table, table_width, k_pool, v_pool, q_heads, kv_heads, head_dim, page_size, rotate, write_kv,
                     nullptr);
 }
@@ -1339,7 +1346,7 @@ CIE_API int cie_gemm_qkv_rope(void* stream, const void* a, int lda, const void* 
 // norm_weight * 1/rms.  A decode step of a few sequences saves the norm's kernel.
 CIE_API int cie_gemm_qkv_rope_folded_norm(void* stream, const float* residual,
                                           const float* norm_weight, float eps, const void* w,
-                                          const void* bias, void* c, int M, int N, int K, int waves,
+                                          const void* bias, void* c, int M, int N, int K, int waves, int one_tile,
                                           const float* cos_table, const float* sin_table, const int* positions,
                                           const int* seq_of_token, const int* seq_slot, const int* block_table,
                                           int table_width, void* k_pool, void* v_pool, int q_heads, int kv_heads,
@@ -1348,7 +1355,7 @@ CIE_API int cie_gemm_qkv_rope_folded_norm(void* stream, const float* residual,
     fold.residual = residual;
     fold.weight = norm_weight;
     fold.eps = eps;
-    return qkv_rope(stream, nullptr, K, w, bias, c, M, N, K, waves, cos_table, sin_table, positions, seq_of_token,
+    return qkv_rope(stream, nullptr, K, w, bias, c, M, N, K, 1, waves, one_tile, cos_table, sin_table, positions, seq_of_token,
                     seq_slot, block_table, table_width, k_pool, v_pool, q_heads, kv_heads, head_dim, page_size, rotate,
                     write_kv, &fold);
 }

@@ -9,6 +9,7 @@ on operands it was not written for.  Kernels run on torch's current stream.
 from __future__ import annotations
 
 import contextlib
+import functools
 
 from typing import Optional
 
@@ -797,15 +798,41 @@ FUSED_MAX_ROWS = 64  # rows one workgroup of ``gemm_fused`` takes; more rows run
 FUSED_PAIR_WORKGROUPS = 256  # workgroups that must remain when workgroups of many rows take two column tiles
 
 
+FUSED_SHORT_K = 1024  # of which four waves have all in flight at once (two slices of 128 each; one with four row tiles)
+FUSED_LONG_K = 4096   # from which more than 16 rows may run as blocks of 16
+
+
+def _row_blocks(rows: int, row_tiles: int, column_tiles: int, groups: int, units: int) -> int:
+    """What a product of more than 16 rows takes, in the time that 16 rows or columns take a workgroup: it reads its columns of
+    the weight and its rows of A, and more workgroups than units take turns."""
+    return -(-groups * -(-rows // (16 * row_tiles)) // units) * (column_tiles + row_tiles)
+
+
+@functools.lru_cache(maxsize=4096)
+def _plan_row_blocks(rows: int, tiles: int, k: int, units: int) -> tuple[int, int]:
+    """(row tiles, waves) of a workgroup with one column tile.  Four waves where they have all of K in flight, or where there are
+    workgroups for two on a unit (96 rows x 2,816, K 2,048 12.7 us, 13.8 with eight)."""
+    row_tiles = min((4, 2, 1) if k >= FUSED_LONG_K else (4, 2), key=lambda r: _row_blocks(rows, r, 1, tiles, units))
+    fills = tiles * -(-rows // (16 * row_tiles)) * 4 >= FUSED_TARGET_WAVES
+    short = k < FUSED_SHORT_K if row_tiles == 4 else k <= FUSED_SHORT_K
+    return row_tiles, 4 if fills or short else 8
+
+
 def plan_fused(rows: int, column_tiles: int, k: int) -> tuple[int, int, int]:
     """(row tiles, waves per workgroup, column tiles per workgroup) of ``gemm_fused``
     for ``rows`` rows, ``column_tiles`` tiles of 16 columns and a K of ``k``.  16, 32 or 64 rows per workgroup (more rows: more workgroups,
     each streaming the weight again).  With more than 16 rows a workgroup takes
     two column tiles if that still leaves enough workgroups (each activation
-    value a wave loads then meets two weight tiles).  As many waves share K as it
+    value a wave loads then meets two weight tiles), else as many rows as have the units read least (``_row_blocks``).  MI355X, us, up to 64 rows a workgroup and as many as are taken:
+    2,048 x 2,048 64 rows 10.2, 8.2 (128 and 256 workgroups), 128 rows 10.4 either way; 896 x 896 64 rows 7.3, 5.3, 128 7.4, 5.4;
+    1,024 x 4,096 64 rows 15.3, 9.8; 2,304 x 2,304 64 rows 10.9 either way, 96 14.9, 12.0; 4,096 x 1,024 32 rows with eight and four
+    waves 7.6, 6.5.  Up to 16 rows as many waves share K as it
     takes to fill the GPU, each with at least one 128-wide slice."""
+    pair = column_tiles >= 2 * FUSED_PAIR_WORKGROUPS
+    if rows > 16 and not pair:
+        return *_plan_row_blocks(rows, column_tiles, k, compute_units()), 1
     row_tiles = 1 if rows <= 16 else 2 if rows <= 32 else 4
-    pair = row_tiles > 1 and column_tiles >= 2 * FUSED_PAIR_WORKGROUPS
+    pair = pair and row_tiles > 1
     groups = (-(-column_tiles // 2) if pair else column_tiles) * -(-rows // FUSED_MAX_ROWS)
     waves = 1 if row_tiles == 1 else 4
     while waves < 8 and groups * waves < FUSED_TARGET_WAVES and waves * 2 * 128 <= k:
@@ -1129,7 +1156,7 @@ def gemm_library(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     return out
 
 
-QKV_SPLIT_PAIRS_BELOW = 128  # (as in the kernel library: below this many pairs of tiles, one tile a workgroup)
+QKV_SPLIT_PAIRS_BELOW = 128  # (of up to 16 rows: below this many pairs of tiles, one tile a workgroup)
 
 
 FOLDED_NORM_ROWS = 16      # the most rows whose norm the q/k/v product makes itself: one tile of rows
@@ -1269,11 +1296,35 @@ def gemm_tiles_rope(weight: torch.Tensor, a: torch.Tensor, bias: Optional[torch.
     return out
 
 
+@functools.lru_cache(maxsize=4096)
+def _plan_qkv_row_blocks(rows: int, pairs: int, k: int, units: int) -> tuple[int, int, bool]:
+    # (the waves of the plain product, so that both cut K alike: four keep too little of it in flight for four row tiles, and
+    # one row tile gained with the pair only)
+    _, waves = _plan_row_blocks(rows, 2 * pairs, k, units)
+    forms = ((2, 1), (2, 2)) if waves == 4 else ((4, 1), (4, 2), (2, 1), (2, 2), (1, 2))
+    row_tiles, tiles = min(forms, key=lambda f: _row_blocks(rows, f[0], f[1], 2 * pairs // f[1], units))
+    return row_tiles, 4 if row_tiles <= 2 and k <= FUSED_SHORT_K else waves, tiles == 1
+
+
+def plan_qkv_rope(rows: int, pairs: int, k: int) -> tuple[int, int, bool]:
+    """(row tiles, waves per workgroup, whether a workgroup takes one tile of 16 columns and not a pair) of ``gemm_qkv_rope``
+    for ``pairs`` pairs of tiles.  Up to 16 rows: one tile where the pairs leave half of the units without a workgroup (80 pairs
+    8.1 -> 7.2 us).  Beyond, as :func:`plan_fused` (MI355X, us, up to 64 rows a workgroup, one tile up to 64 rows and fewer than
+    128 pairs, and what is taken: 2,560 x 2,048 48 rows 10.6, 9.2, 64 10.9, 9.9, 96 12.6, 10.4; 1,152 x 896 64 rows 8.1, 6.3, 96
+    9.4, 6.4; 3,072 x 2,048 64 rows 11.7, 10.4; 5,120 x 1,024 96 rows 14.6, 10.2; 3,072 x 1,024 33 to 128 rows 0 to 12 % less)."""
+    if rows > 16:
+        return _plan_qkv_row_blocks(rows, pairs, k, compute_units())
+    _, waves, _ = plan_fused(rows, pairs, k)
+    one_tile = pairs < QKV_SPLIT_PAIRS_BELOW
+    return 1, min(waves, 4) if one_tile else waves, one_tile
+
+
 def gemm_qkv_rope(weight: torch.Tensor, a: Optional[torch.Tensor], bias: Optional[torch.Tensor], cos: torch.Tensor,
                   sin: torch.Tensor, positions: torch.Tensor, seq_of_token: torch.Tensor, seq_slot: torch.Tensor,
                   block_table: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, q_heads: int,
                   kv_heads: int, head_dim: int, rotate: bool = True, write_kv: bool = True,
-                  waves: Optional[int] = None, folded: Optional[tuple] = None) -> torch.Tensor:
+                  waves: Optional[int] = None, folded: Optional[tuple] = None,
+                  blocks: Optional[tuple[int, bool]] = None) -> torch.Tensor:
     """The q/k/v product of a few rows (64 per workgroup) fused with what ``rope_kv_write`` does:
     ``a @ weight.T + bias`` for weight [(Hq+2Hkv)*D, K], queries and keys rotated
     by each row's position, keys and values written into the cache.  Returns the
@@ -1283,7 +1334,9 @@ def gemm_qkv_rope(weight: torch.Tensor, a: Optional[torch.Tensor], bias: Optiona
 
     ``folded=(residual, norm_weight, eps)`` instead of ``a`` (``folds_norm`` says for which sizes): the rows
     are the RMSNorm of ``residual`` (float32 [M, K], float32 weight), made inside the product: a lane makes
-    the values of its matrix operand from the stream, and the rows' 1/rms multiplies the sums."""
+    the values of its matrix operand from the stream, and the rows' 1/rms multiplies the sums.
+
+    ``blocks``: (row tiles, one tile a workgroup) instead of the planned ones."""
     _gpu("weight", weight, torch.bfloat16, 2)
     n, k = weight.shape
     if folded is not None:
@@ -1334,23 +1387,23 @@ def gemm_qkv_rope(weight: torch.Tensor, a: Optional[torch.Tensor], bias: Optiona
     _gpu("seq_slot", seq_slot, torch.int32, 1)
     _gpu("block_table", block_table, torch.int32, 2)
     page_size = _check_pools(k_pool, v_pool, torch.bfloat16, kv_heads, head_dim)
-    if waves is None:
-        _, waves, _ = plan_fused(m, n // 32, k)
-        if m <= 16 and n // 32 < QKV_SPLIT_PAIRS_BELOW:
-            waves = min(waves, 4)  # (the kernel then takes one tile a workgroup, twice the workgroups: 8.1 -> 7.2 us)
-    if not (waves in ((1, 2, 4, 8) if m <= 16 else (4, 8))):
-        raise ValueError(f"{waves} waves per workgroup with {m} rows is not a form the kernel has")
+    row_tiles, planned, one_tile = plan_qkv_rope(m, n // 32, k)
+    waves = planned if waves is None else waves
+    if blocks is not None:
+        row_tiles, one_tile = blocks
+    if not (row_tiles in ((1,) if m <= 16 else (1, 2, 4)) and waves in ((1, 2, 4, 8) if row_tiles == 1 else (4, 8))):
+        raise ValueError(f"{waves} waves per workgroup and {row_tiles} row tiles with {m} rows is not a form the kernel has")
     out = torch.empty((m, n), dtype=torch.bfloat16, device=weight.device)
     if folded is not None:
         _run("cie_gemm_qkv_rope_folded_norm", load_library().cie_gemm_qkv_rope_folded_norm(
             _stream(), _ptr(residual), _ptr(norm_weight), _f(eps),
-            _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k), _i(waves), _ptr(cos), _ptr(sin), _ptr(positions),
+            _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k), _i(waves), _i(one_tile), _ptr(cos), _ptr(sin), _ptr(positions),
             _ptr(seq_of_token), _ptr(seq_slot), _ptr(block_table), _i(block_table.shape[1]), _ptr(k_pool), _ptr(v_pool),
             _i(q_heads), _i(kv_heads), _i(head_dim), _i(page_size), _i(1 if rotate else 0), _i(1 if write_kv else 0)))
         return out
     _run("cie_gemm_qkv_rope", load_library().cie_gemm_qkv_rope(
-        _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k), _i(waves), _ptr(cos),
-        _ptr(sin), _ptr(positions), _ptr(seq_of_token), _ptr(seq_slot), _ptr(block_table), _i(block_table.shape[1]),
+        _stream(), _ptr(a), _i(lda), _ptr(weight), _ptr(bias), _ptr(out), _i(m), _i(n), _i(k), _i(row_tiles), _i(waves), _i(one_tile),
+        _ptr(cos), _ptr(sin), _ptr(positions), _ptr(seq_of_token), _ptr(seq_slot), _ptr(block_table), _i(block_table.shape[1]),
         _ptr(k_pool), _ptr(v_pool), _i(q_heads), _i(kv_heads), _i(head_dim), _i(page_size),
         _i(1 if rotate else 0), _i(1 if write_kv else 0)))
     return out

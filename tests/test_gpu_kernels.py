@@ -1813,3 +1813,54 @@ def test_logits_go_where_an_address_says(ops, dtype, shape):
         assert torch.equal(out[1: m + 1], want) and (out[0] == 7.0).all() and (out[m + 1] == 7.0).all()
     with pytest.raises(ValueError):
         ops.gemm_fused(w.bfloat16(), ops.EPI_BF16, a.bfloat16()[:1], out_at=at)
+
+
+@pytest.mark.parametrize("shape", [(896, 896), (2048, 2048), (1024, 4096), (48, 136), (2304, 1032)])
+@pytest.mark.parametrize("rows", [17, 31, 33, 49, 64, 65, 97, 128])
+def test_products_of_more_rows_in_blocks_of_rows(ops, shape, rows):
+    """The product added into the stream in blocks of 16, 32 and 64 rows and as planned, against float64: the stream, the next
+    norm's rows and their sums of squares; the same bits where as many waves share K."""
+    n, k = shape
+    a, w, b = rand((rows, k), torch.bfloat16, 1), rand((n, k), torch.bfloat16, 2, 0.05), rand((n,), torch.bfloat16, 3)
+    stream, gain = rand((rows, n), torch.float32, 4), rand((n,), torch.float32, 5, 0.1) + 1
+    want = stream.double() + a.double() @ w.double().t() + b.double()
+    # float32 sums of k products and two more numbers: k + 2 roundings of at most the sum of the magnitudes
+    bound = (k + 2) * 2.0 ** -24 * (stream.double().abs() + a.double().abs() @ w.double().abs().t() + b.double().abs())
+    first = {}
+    for plan in (None, (1, 4, 1), (1, 8, 1), (2, 4, 1), (2, 8, 1), (4, 4, 1), (4, 8, 1)):
+        out, scaled = stream.clone(), torch.empty((rows, n), dtype=torch.bfloat16, device="cuda")
+        sumsq = ops.gemm_fused(w, ops.EPI_RESID, a, bias=b, residual_out=out, norm_weight=gain, scaled_out=scaled, plan=plan)
+        assert ((out.double() - want).abs() <= bound).all()
+        assert torch.equal(out, first.setdefault((plan or ops.plan_fused(rows, n // 16, k))[1], out))
+        assert torch.equal(scaled, (out * gain).to(torch.bfloat16))
+        torch.testing.assert_close(sumsq.sum(dim=1), out.double().pow(2).sum(dim=1).float(), rtol=1e-5, atol=0)
+
+
+@pytest.mark.parametrize("geometry", [(16, 2, 128, 16, 2048), (14, 2, 64, 16, 896), (3, 1, 32, 4, 328), (24, 8, 96, 16, 1024)])
+@pytest.mark.parametrize("rows", [17, 33, 48, 64, 65, 96, 128])
+def test_gemm_qkv_rope_in_blocks_of_rows(ops, geometry, rows):
+    """Every block of rows and columns that the q/k/v product may be planned in, against the plain product and the rotation's
+    kernel: the same values, and what two kernels make of one rotation (a bf16 step)."""
+    q_heads, kv_heads, head_dim, page_size, hidden = geometry
+    n, q_cols = (q_heads + 2 * kv_heads) * head_dim, q_heads * head_dim
+    lengths = [rows + 3, rows + 40]
+    k_pool, v_pool, table, slots, _ = build_cache(torch.bfloat16, lengths, kv_heads, head_dim, page_size, seed=9)
+    positions = torch.tensor([lengths[i % 2] - 1 - i // 2 for i in range(rows)], dtype=torch.int32).cuda()
+    meta = (positions, torch.tensor([i % 2 for i in range(rows)], dtype=torch.int32).cuda(),
+            torch.tensor(slots, dtype=torch.int32).cuda(), table)
+    a, w, b = rand((rows, hidden), torch.bfloat16, 1), rand((n, hidden), torch.bfloat16, 2, 0.3), rand((n,), torch.bfloat16, 3)
+    cos, sin = (t[:, : head_dim // 2].contiguous().cuda() for t in plain_qwen2.rope_tables(head_dim, 512, 1e6))
+    for waves in (4, 8):
+        plain = ops.gemm_fused(w, ops.EPI_BF16, a, bias=b, plan=(4, waves, 1))
+        k_want, v_want = k_pool.clone(), v_pool.clone()
+        ops.rope_kv_write(plain, cos, sin, *meta, k_want, v_want, q_heads, kv_heads, head_dim)
+        planned = ops.plan_qkv_rope(rows, n // 32, hidden)[1] == waves
+        for blocks in ((1, False), (1, True), (2, False), (2, True), (4, False), (4, True)) + ((None,) if planned else ()):
+            k_got, v_got = k_pool.clone(), v_pool.clone()
+            got = ops.gemm_qkv_rope(w, a, b, cos, sin, *meta, k_got, v_got, q_heads, kv_heads, head_dim,
+                                    waves=None if blocks is None else waves, blocks=blocks)
+            torch.testing.assert_close(got[:, :q_cols].float(), plain[:, :q_cols].float(), rtol=2 ** -7, atol=1e-6)
+            torch.testing.assert_close(k_got.float(), k_want.float(), rtol=2 ** -7, atol=1e-6)
+            assert torch.equal(v_got, v_want)
+    with pytest.raises(ValueError):
+        ops.gemm_qkv_rope(w, a, b, cos, sin, *meta, k_got, v_got, q_heads, kv_heads, head_dim, waves=2, blocks=(2, True))
