@@ -186,6 +186,9 @@ WIDE_DECODE_KEYS = 2048  # contexts from which decode rows go to the four-wave f
 FEW_DECODE_UNITS = 8  # (sequence, kv head) pairs below which they do not: parts of one wave fill the GPU better
 MANY_DECODE_UNITS = 96  # (sequence, kv head) pairs from which decode rows take the four-wave form at any context
 MANY_PART_BYTES = 300 << 10  # keys and values of one pair below which its keys are not cut then
+SOME_DECODE_UNITS = 33  # ... and from which they may with a merge of their own: whole while a pair reads no more than so many bytes,
+WHOLE_UNIT_BYTES = 176 << 10
+SOME_DECODE_KEYS = 48 << 10  # in parts where all pairs together have so many keys
 SHARED_DECODE_KEYS = 96  # contexts from which four waves share a decode row's keys without cutting them
 SPLIT_MIN_KEYS = 32  # the fewest keys of a one-wave part
 SPLIT_DECODE_KEYS = 192  # contexts from which the keys of decode rows are cut into parts at all
@@ -319,14 +322,28 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
              and takes_prompt_form(small_tiles, prompt_keys, singles, batch.static_plan is not None, cus))
     lds_row_tiles = 8 if head_dim == 128 and big_tiles > LARGE_TILES_ABOVE * cus else 4
 
-    def decode_form(bound: int, units: int) -> tuple[int, dict]:
+    def decode_form(bound: int, units: int, joined: bool) -> tuple[int, dict]:
         # Decode rows, `units` (sequence, kv head) pairs over up to `bound` keys.  Long contexts: four waves
         # per (sequence, kv head, part of the keys) take the part's blocks in turn with their loads running
         # ahead (15.8 against 18.1 us for 8 x 4,096 keys).  A few pairs do not fill the GPU that way: they take the
         # one-wave form below, whose parts are smaller (one sequence of the 3B shape over 32,000 keys: 333 -> 363
-        # tokens/s; from four sequences on the forms are level).
-        if wide and bound >= WIDE_DECODE_KEYS and units >= FEW_DECODE_UNITS:
-            return ops.TILE_WAVES, dict(target_waves=cus, min_keys=32 * ops.TILE_WAVES)
+        # tokens/s; from four sequences on the forms are level).  Where the output product merges the shares (``joined``) it
+        # reads every one of them: there the line is the number of keys in all, and a unit has no more shares than are needed for a
+        # workgroup each (MI355X, us, attention and output product, with parts of one wave down to 32 keys and so: 8 rows of 16
+        # heads on 2 over 1,600 keys 15.7 -> 13.4, 16 rows over 1,000 17.4 -> 14.4, 2,000 20.6 -> 17.7; heads of 64 13.7 -> 10.6,
+        # 14.6 -> 10.7, 17.1 -> 12.0; 28 heads on 4, 8 rows over 1,000 21.5 -> 20.0; one wave and four level at 8 rows over 1,000).
+        if wide and units >= FEW_DECODE_UNITS and (bound >= WIDE_DECODE_KEYS or (
+                joined and units < MANY_DECODE_UNITS and units * bound >= FEW_DECODE_UNITS * WIDE_DECODE_KEYS)):
+            return ops.TILE_WAVES, dict(target_waves=cus, min_keys=64 if joined else 32 * ops.TILE_WAVES)
+        # ... and with a merge of its own from some dozens of pairs on: whole where a pair has little to read, four waves where
+        # all have much (us, merge with it, one wave's parts, four waves whole, four waves' parts: 24 rows of 14 heads of 64 on 2 over 300
+        # keys 7.9, 6.3, 9.0, 640 10.4, 9.1, 10.3, 1,600 14.5, 14.6, 12.1; of 16 heads of 128 on 2 over 300 9.0, 9.1, 10.4, 640 11.9, 13.6,
+        # 12.6, 1,600 17.9, 25.1, 16.5; 32 rows 9.6, 9.3, 11.0, 12.9, 13.9, 13.1, 21, 25.9, 19.4).
+        if wide and not joined and SOME_DECODE_UNITS <= units < MANY_DECODE_UNITS:
+            if SHARED_DECODE_KEYS <= bound <= WHOLE_UNIT_BYTES // (4 * head_dim):
+                return ops.TILE_WAVES, dict(target_waves=cus, min_keys=bound + 1)
+            if units * bound >= SOME_DECODE_KEYS:
+                return ops.TILE_WAVES, dict(target_waves=cus, min_keys=32 * ops.TILE_WAVES)
         # Many pairs fill the GPU by themselves: the same form with the keys whole or in large parts
         # (64 sequences x 2 heads x 256 keys: 9.2 us against 11.1 us with one wave per part).  A second part pays for
         # its merge where a unit has more to read than MANY_PART_BYTES (64 x 2 heads of 128, us, whole against two
@@ -341,7 +358,10 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
         # Otherwise one wave per part, parts down to one block of 32 keys (8 x 256 keys: 7.3 us in 8 parts,
         # 10.2 us in 2; 8 x 512 keys: 8.1 us in 16 parts, 10.6 us in 4) ...
         if bound >= SPLIT_DECODE_KEYS:
-            return 1, dict(target_waves=4 * cus, min_keys=SPLIT_MIN_KEYS)
+            # (joined: shares of 128 keys and less only while all of them are fewer than the units; one row of 16 heads on 2 over
+            # 1,000 keys at a bound of 32,768 14.3 -> 11.8 us, over 32,000 20.5 -> 19.7; 8 rows over 800 keys 13.2 -> 12.0, 16 over 400 13.9 -> 12.7)
+            most = min(4 * cus, max(cus, units * (bound // 128))) if joined else 4 * cus
+            return 1, dict(target_waves=most, min_keys=SPLIT_MIN_KEYS)
         # ... and below some 200 keys, where the merge costs more than it saves, four waves that share a
         # sequence's few blocks inside one workgroup instead of one wave that takes them in turn
         # (8 x 128 keys: 6.5 against 6.9 us, 8 x 160: 7 against 11)
@@ -361,11 +381,16 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
         decode_rows = batch.sequences if plan.decode_rows is None else plan.decode_rows
         joined = wide and not eight and 0 < decode_rows <= JOINED_DECODE_ROWS and decode_rows < batch.sequences
         if decode_rows and not joined:
-            decode_waves, split_options = decode_form(max_keys, decode_rows * num_kv_heads)
-            n_splits, _ = plan_splits(decode_rows * num_kv_heads, max_keys, **split_options)
+            decode_waves, split_options = decode_form(max_keys, decode_rows * num_kv_heads, unmerged and decode_rows == batch.tokens)
+            units = decode_rows * num_kv_heads
+            n_splits, _ = plan_splits(units, max_keys, **split_options)
+            if n_splits > 1 and decode_waves > 1:
+                # (the device sizes the parts: as many as asked for, where the bound's own would come out fewer, as 1,040 keys in 8 of
+                # 160 do: 8 rows of 28 heads on 4 over 1,000 keys 19.7 us in 7, 19.3 in 8)
+                n_splits = min(split_options["target_waves"] // units, max_keys // split_options["min_keys"])
             part_o = part_ml = None
             if n_splits > 1:
-                part_o, part_ml = _workspaces(qkv.device, decode_rows * num_kv_heads * n_splits, 16 * decode_tiles, head_dim)
+                part_o, part_ml = _workspaces(qkv.device, units * n_splits, 16 * decode_tiles, head_dim)
             ops.paged_attention_mfma(qkv, qkv.stride(0), view.k_pool, view.v_pool, view.block_table, None,
                                      None, decode_rows, *common, tokens_per_tile=1, row_tiles=decode_tiles,
                                      n_splits=n_splits, max_context_dev=longest_dev, part_o=part_o, part_ml=part_ml,
@@ -383,7 +408,7 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
         # (not beside the form of eight waves, where a tile of one token would leave six of them idle)
         joined = wide and not eight and 0 < n_tiles <= JOINED_DECODE_ROWS and n_tiles < batch.sequences
     if n_tiles and not joined:
-        decode_waves, split_options = decode_form(max_keys, n_tiles * num_kv_heads)
+        decode_waves, split_options = decode_form(max_keys, n_tiles * num_kv_heads, unmerged and n_tiles == batch.tokens)
         n_splits, per_split = plan_splits(n_tiles * num_kv_heads, max_keys, **split_options)
         part_o = part_ml = None
         if n_splits > 1:

@@ -1864,3 +1864,47 @@ def test_gemm_qkv_rope_in_blocks_of_rows(ops, geometry, rows):
             assert torch.equal(v_got, v_want)
     with pytest.raises(ValueError):
         ops.gemm_qkv_rope(w, a, b, cos, sin, *meta, k_got, v_got, q_heads, kv_heads, head_dim, waves=2, blocks=(2, True))
+
+
+# (query heads, key heads, head size, rows, longest context): both sides of every line between the forms of a decode step's keys
+DECODE_LINES = [(16, 2, 128, 8, 1023), (16, 2, 128, 8, 1024), (14, 2, 64, 16, 511), (14, 2, 64, 16, 512), (16, 2, 128, 3, 2500), (16, 2, 128, 4, 2048),
+                (28, 4, 128, 9, 600), (32, 8, 64, 12, 700), (14, 2, 64, 17, 704), (14, 2, 64, 17, 705), (16, 2, 128, 30, 352), (16, 2, 128, 30, 353),
+                (16, 2, 128, 25, 983), (14, 2, 64, 32, 1700), (4, 2, 32, 20, 90), (8, 1, 128, 40, 1300)]
+
+
+@pytest.mark.parametrize("line", DECODE_LINES)
+def test_decode_forms_on_both_sides_of_their_lines(ops, line):
+    """A step of single tokens through the attention and, where that takes the keys' shares as they are, the output product."""
+    from cie_amd.engine.batch import PagedView, StepBatch
+    from cie_amd.engine.graphs import StaticPlan
+    from cie_amd.parts import attention as A
+
+    q_heads, kv_heads, dim, rows, longest = line
+    width, page = q_heads * dim, 16
+    contexts = [longest - 1 if i == rows // 2 else (i * 977) % longest for i in range(rows)]
+    lengths = [c + 1 for c in contexts]
+    k_pool, v_pool, table, slots, dense = build_cache(torch.bfloat16, lengths, kv_heads, dim, page, seed=5)
+    as_dev = lambda values: torch.tensor(values, dtype=torch.int32).cuda()  # noqa: E731
+    qkv = rand((rows, width + 2 * kv_heads * dim), torch.bfloat16, 1, 2.0)
+    w = rand((256, width), torch.bfloat16, 2, 0.05)
+    want = torch.cat([plain_qwen2.causal_attention(qkv[i: i + 1, :width].float().cpu().view(1, q_heads, dim), *dense[i], dim ** -0.5,
+                                                   past_len=contexts[i]) for i in range(rows)]).cuda()
+    batch = dict(tokens=rows, sequences=rows, token_ids=as_dev([0] * rows), positions=as_dev(contexts), seq_of_token=as_dev(range(rows)),
+                 seq_slot=as_dev(slots), seq_start=as_dev(contexts), seq_q_len=as_dev([1] * rows), q_start_loc=as_dev(range(rows + 1)),
+                 logit_rows=as_dev([0]), host_slots=slots, host_starts=contexts, host_q_lens=[1] * rows)
+    # launch by launch, and as in a captured step, for a tight and a loose bound
+    plans = [None] + [StaticPlan(as_dev(range(rows)), as_dev([0] * rows), as_dev([longest]), bound) for bound in (longest, longest + 900, 32768)]
+    for plan in plans:
+        view = PagedView(k_pool, v_pool, table, page)
+        step = StepBatch(**batch, static_plan=plan)
+        stream = torch.zeros((rows, 256), device="cuda")
+        joins = A.joins_merge(rows, w, stream)
+        assert joins == (rows <= 16 and width % 128 == 0)
+        out = A.attend(qkv, step, view, q_heads, kv_heads, dim, None, dim ** -0.5, unmerged=joins)
+        if isinstance(out, A.Shares):
+            ops.merge_project(out.part_o, out.part_ml, w, None, stream, q_heads, kv_heads, dim, out.splits, out.tile_rows)
+            # the rows' rounding (and their error, as below) through the product
+            bound = want.abs() @ w.float().abs().t() * 2 ** -7 + 1e-2 * w.float().abs().sum(dim=1)
+            assert ((stream - want @ w.float().t()).abs() <= bound).all()
+        else:
+            torch.testing.assert_close(out.float(), want, **tol(torch.bfloat16))
