@@ -1309,14 +1309,16 @@ def _plan_qkv_row_blocks(rows: int, pairs: int, k: int, units: int) -> tuple[int
 def plan_qkv_rope(rows: int, pairs: int, k: int) -> tuple[int, int, bool]:
     """(row tiles, waves per workgroup, whether a workgroup takes one tile of 16 columns and not a pair) of ``gemm_qkv_rope``
     for ``pairs`` pairs of tiles.  Up to 16 rows: one tile where the pairs leave half of the units without a workgroup (80 pairs
-    8.1 -> 7.2 us).  Beyond, as :func:`plan_fused` (MI355X, us, up to 64 rows a workgroup, one tile up to 64 rows and fewer than
+    8.1 -> 7.2 us), but for a short K, of which a pair's four waves have all in flight too, and read the rows once for twice the columns
+    (with the norm, one tile and a pair: 1,152 x 896 1 row 5.8, 5.2, 8 6.5 either way, 16 7.5, 7.0; 3,072 x 1,024 6.5, 6.1, 7.6 either way, 8.6, 8.0;
+    2,048 x 1,536 6.8, 8.1).  Beyond, as :func:`plan_fused` (MI355X, us, up to 64 rows a workgroup, one tile up to 64 rows and fewer than
     128 pairs, and what is taken: 2,560 x 2,048 48 rows 10.6, 9.2, 64 10.9, 9.9, 96 12.6, 10.4; 1,152 x 896 64 rows 8.1, 6.3, 96
     9.4, 6.4; 3,072 x 2,048 64 rows 11.7, 10.4; 5,120 x 1,024 96 rows 14.6, 10.2; 3,072 x 1,024 33 to 128 rows 0 to 12 % less)."""
     if rows > 16:
         return _plan_qkv_row_blocks(rows, pairs, k, compute_units())
     _, waves, _ = plan_fused(rows, pairs, k)
-    one_tile = pairs < QKV_SPLIT_PAIRS_BELOW
-    return 1, min(waves, 4) if one_tile else waves, one_tile
+    few = pairs < QKV_SPLIT_PAIRS_BELOW
+    return 1, min(waves, 4) if few else waves, few and k > FUSED_SHORT_K
 
 
 def gemm_qkv_rope(weight: torch.Tensor, a: Optional[torch.Tensor], bias: Optional[torch.Tensor], cos: torch.Tensor,
