@@ -1082,11 +1082,15 @@ constexpr int kChunkTokens = 64;
 constexpr int kChunkChannels = 64;
 constexpr int kOutputTokens = 32;  // of a workgroup of (b)
 
-// The value of the lane APART in front, of a row of 16 (the first ones keep theirs), and that of a row's last lane.
+// The value of the lane APART in front, of a row of 16 (the first ones have `first`, or keep theirs), and that of a row's last lane.
+template <int APART>
+__device__ __forceinline__ float lane_before(float v, float first) {
+    return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+        static_cast<int>(__float_as_uint(first)), static_cast<int>(__float_as_uint(v)), 0x110 + APART, 0xf, 0xf, false)));
+}
 template <int APART>
 __device__ __forceinline__ float lane_before(float v) {
-    const int own = static_cast<int>(__float_as_uint(v));
-    return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(own, own, 0x110 + APART, 0xf, 0xf, false)));
+    return lane_before<APART>(v, v);
 }
 __device__ __forceinline__ float row_last(float v) {
     const int own = static_cast<int>(__float_as_uint(v));
@@ -1205,6 +1209,7 @@ gated_chunks_kernel(const bf16_t* __restrict__ u, const bf16_t* __restrict__ wei
                 a[i] = 0.f;
             }
         }
+        const float own_a[4] = {a[0], a[1], a[2], a[3]}, own_b[4] = {b[0], b[1], b[2], b[3]};
         join_before<1>(a, b, r, from, place);
         join_before<2>(a, b, r, from, place);
         join_before<4>(a, b, r, from, place);
@@ -1214,6 +1219,15 @@ gated_chunks_kernel(const bf16_t* __restrict__ u, const bf16_t* __restrict__ wei
             const bool joins = from < t * 16;
             b[i] = joins ? fmaf(a[i], before_b[i], b[i]) : b[i];
             a[i] = joins ? a[i] * before_a[i] : a[i];
+            // Up to six roundings by now: the step over again from the token in front has the walk's one, and fades what the tokens
+            // in front have of them, twice (states off 64 bits by 7.9e-8 without, 7.2e-8 so, 7.1e-8 in order; 1,999 tokens of 2,048
+            // channels 43.9 -> 44.7 us).
+            const bool steps = from < place && place > 0;
+#pragma unroll
+            for (int again = 0; again < 2; ++again) {
+                const float in_front = lane_before<1>(b[i], before_b[i]);
+                b[i] = steps ? fmaf(own_a[i], in_front, own_b[i]) : b[i];
+            }
             before_a[i] = row_last(a[i]);
             before_b[i] = row_last(b[i]);
         }

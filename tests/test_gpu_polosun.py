@@ -783,3 +783,42 @@ def test_gated_recurrence_in_chunks(lengths, blocks, width, taps):
         there = torch.isfinite(want)
         assert torch.allclose(out[there].float(), want[there].float(), atol=4 * near, rtol=2.0 ** -7)
         assert torch.equal(past, past2)
+
+
+def test_gated_recurrence_in_chunks_is_as_near_to_64_bits_as_the_walk():
+    """The states of a portion in chunks, whose tokens compose by doubling, and those of the walk in order, at the fades of a model
+    whose parameters are drawn about zero."""
+    from cie_amd.kernels import ops
+
+    blocks, width, taps, off = 2, 256, 4, {"chunks": 0.0, "walk": 0.0}
+    channels = blocks * width
+    meta = lambda values: torch.tensor(values, dtype=torch.int32).cuda()  # noqa: E731
+    for seed, lengths in enumerate([(61, 128, 97, 33, 80, 111, 20, 49), (300, 17, 449), (640,), (255, 257)]):
+        g = torch.Generator().manual_seed(30 + seed)
+        make = lambda *shape: torch.randn(*shape, generator=g)  # noqa: E731, B023
+        tokens, n = sum(lengths), len(lengths)
+        proj, u = make(tokens, 2 * channels).bfloat16().cuda(), make(tokens, channels).bfloat16().cuda()
+        weight, bias = (make(blocks, 2 * width, width) * width ** -0.5).bfloat16().cuda(), make(blocks, 2 * width).bfloat16().cuda()
+        rate = -8.0 * torch.nn.functional.softplus(0.02 * make(channels)).cuda()
+        state, past = make(n, channels).cuda(), make(n, taps - 1, channels).cuda()
+        starts = [sum(lengths[:i]) for i in range(n + 1)]
+        rows = u.double().view(tokens, blocks, width).transpose(0, 1)
+        gates = torch.matmul(rows, weight.double().transpose(1, 2).contiguous()) + bias.double()[:, None]
+        gates = gates.transpose(0, 1).reshape(tokens, blocks, 2, width)
+        log_fade = rate.double() * torch.sigmoid(gates[:, :, 0]).reshape(tokens, channels)
+        fade, add = torch.exp(log_fade), torch.sqrt(-torch.expm1(2 * log_fade)) * torch.sigmoid(gates[:, :, 1]).reshape(tokens, channels) * u.double()
+        want = state.double()
+        for i in range(n):
+            for t in range(starts[i], starts[i + 1]):
+                want[i] = torch.addcmul(add[t], fade[t], want[i])
+        for name in off:
+            mine, kept = state.clone(), past.clone()
+            if name == "chunks":
+                ops.gated_recurrence_chunks(proj[:, :channels], proj[:, channels:], u, weight, bias, rate, mine, kept,
+                                            meta([i for i, k in enumerate(lengths) for _ in range(k)]), meta(range(n)), meta(starts), n, taps)
+            else:
+                ops.gated_recurrence(proj[:, :channels], proj[:, channels:], u, ops.block_linear(u, weight, bias, out_dtype=torch.float32),
+                                     width, rate, mine, kept, meta(range(n)), meta(starts), n, taps)
+            off[name] += float(((mine.double() - want).norm() / want.norm()) ** 2)
+    # (a token has the walk's own rounding and what fades of those in front, which is the same or, at a chunk's first tokens, one more)
+    assert off["chunks"] ** 0.5 <= 1.05 * off["walk"] ** 0.5, off
