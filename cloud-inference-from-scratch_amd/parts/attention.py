@@ -24,7 +24,7 @@ from ..config.specs import PartSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import Part, build_part, register_part
-from .linear import Added, BEHIND_ROTATION, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, choose_tiles, linear, takes_tiles
+from .linear import Added, BEHIND_ROTATION, FUSED_ROWS, FUSED_SMALL_ROWS, FUSED_SMALL_WEIGHT, RawRows, choose_tiles, cuts_k, linear, takes_tiles
 
 
 class Attention(Part):
@@ -33,6 +33,7 @@ class Attention(Part):
     folds_next_norm = True  # its output product can leave the next norm's rows short of their scale
     takes_raw_rows = True  # its first product can make the norm of a few rows itself
     sums_parts = True  # its last product may come back as parts of K
+    adds_unordered = True  # ... or merge a decode step's shares itself, and add their sums to the stream in no fixed order
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int,
                  qkv_bias: bool, out_bias: bool, position: PartSpec, window: Optional[int] = None,
                  scale: Optional[float] = None) -> None:
@@ -117,7 +118,7 @@ class Attention(Part):
         return qkv
 
     def forward(self, x, batch, view, writes: bool = True, residual: Optional[torch.Tensor] = None,
-                next_norm=None, sums_parts: bool = False):
+                next_norm=None, sums_parts: bool = False, unordered: bool = False):
         if batch.max_context > self.position.max_position and self.position.rotates:
             raise ValueError(
                 f"position {batch.max_context - 1} is beyond the rotary table of {self.position.max_position}"
@@ -137,7 +138,7 @@ class Attention(Part):
                     batch.seq_slot, view.block_table, view.k_pool, view.v_pool, self.num_heads, self.num_kv_heads,
                     head_dim, rotate=self.position.rotates, write_kv=writes,
                     folded=(x.residual, x.norm.weight_f32, x.norm.eps))
-                return self._attended(qkv, batch, view, residual, next_norm, sums_parts)
+                return self._attended(qkv, batch, view, residual, next_norm, sums_parts, unordered)
             turning = head_dim if rotary_dim is None else rotary_dim
             if (type(self).shape_projection is Attention.shape_projection and head_dim % 16 == 0 and turning % 16 == 0
                     and x.joins_f32(self.w_qkv)):
@@ -145,7 +146,7 @@ class Attention(Part):
                     x.residual, x.norm.weight_f32, x.norm.eps, self.w_qkv, self.b_qkv, self.cos, self.sin, batch.positions,
                     batch.seq_of_token, batch.seq_slot, view.block_table, view.k_pool, view.v_pool, self.num_heads,
                     self.num_kv_heads, head_dim, rotate=self.position.rotates, write_kv=writes, rotary_dim=turning)
-                return self._attended(qkv, batch, view, residual, next_norm, sums_parts)
+                return self._attended(qkv, batch, view, residual, next_norm, sums_parts, unordered)
             x = x.complete()
         fused = (x.dtype == torch.bfloat16 and untouched and head_dim % 32 == 0
                  and x.shape[1] % 8 == 0 and (rows == 1 or x.stride(0) % 8 == 0))
@@ -168,12 +169,13 @@ class Attention(Part):
             ops.rope_kv_write(qkv, self.cos, self.sin, batch.positions, batch.seq_of_token, batch.seq_slot,
                               view.block_table, view.k_pool, view.v_pool, self.num_heads, self.num_kv_heads,
                               head_dim, rotate=self.position.rotates, write_kv=writes, rotary_dim=rotary_dim)
-        return self._attended(qkv, batch, view, residual, next_norm, sums_parts)
+        return self._attended(qkv, batch, view, residual, next_norm, sums_parts, unordered)
 
-    def _attended(self, qkv: torch.Tensor, batch, view, residual: Optional[torch.Tensor], next_norm, sums_parts: bool):
+    def _attended(self, qkv: torch.Tensor, batch, view, residual: Optional[torch.Tensor], next_norm, sums_parts: bool,
+                  unordered: bool = False):
         """The attention of rotated heads, and the product behind it."""
         context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, self.kernel_head_dim, self.window, self.scale,
-                         unmerged=joins_merge(qkv.shape[0], self.w_o, residual))
+                         unmerged=(unordered or cuts_k(*self.w_o.shape)) and joins_merge(qkv.shape[0], self.w_o, residual))
         if isinstance(context, Shares):
             ops.merge_project(context.part_o, context.part_ml, self.w_o, self.b_o, residual, self.num_heads, self.num_kv_heads,
                               self.kernel_head_dim, context.splits, context.tile_rows)

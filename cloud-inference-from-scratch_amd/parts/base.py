@@ -106,6 +106,9 @@ class Part:
     # ``sums_parts``: ``forward`` takes ``sums_parts=``, and where that is true its output may come back as ``KParts``: the
     # float32 parts of its last product, which whoever adds the branch sums.  (Asked with ``declares``.)
     sums_parts = False
+    # ``adds_unordered``: ``forward`` takes ``unordered=``, and where that is true too (the layer's sums have no fixed order anyway)
+    # its output may be added to the stream in parts that have none.  (Asked with ``declares``.)
+    adds_unordered = False
     # ``joins_products``: the part is one product in, something between, one product out.  Two such parts that read the
     # same rows and whose results are added may share both products: ``product_in()`` and ``product_out()`` give the
     # weights, and the part's own step between them takes the first product's rows and writes into a given matrix.

@@ -32,8 +32,8 @@ from ..config.specs import LayerSpec
 from ..kernels import ops
 from ..weights.tensors import TensorSpec
 from .base import build_part, declares, register_part
-from .linear import (Added, KParts, RawRows, RowSumsq, StreamRows, WeightedPair, linear, linear_beside, parts_beside,
-                     silu_beside)
+from .linear import (Added, KParts, RawRows, RowSumsq, StreamRows, WeightedPair, cuts_k, linear, linear_beside,
+                     parts_beside, silu_beside)
 
 
 class PreNormBlock:
@@ -65,6 +65,9 @@ class PreNormBlock:
         self.dtype = dtype
         for role, part in self._parts():
             part.bind(tensors, f"{prefix}{self.spec.name_of(role)}.", dtype, device)
+        # the mixer's branch may be added in no fixed order where the feed-forward's is: a layer whose sums have one repeats its bits
+        self.unordered = (self.has_feed_forward and declares(self.feed_forward, "gates_products")
+                          and cuts_k(*self.feed_forward.w_down.shape))
 
     def cache_need(self):
         return self.mixer.cache_need()
@@ -80,6 +83,7 @@ class PreNormBlock:
                 warm(rows)
 
     takes_added = True
+    unordered = False
 
     def forward(self, residual: torch.Tensor, pending: Optional[torch.Tensor], batch, view, writes: bool = True,
                 plus: Optional[torch.Tensor] = None, added: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
@@ -113,6 +117,8 @@ class PreNormBlock:
         extra = self._joins(self.mixer, residual if added or self.has_feed_forward or self.dtype != torch.float32 else None)
         if extra and declares(self.mixer, "sums_parts"):
             extra["sums_parts"] = True
+        if extra and self.unordered and declares(self.mixer, "adds_unordered"):
+            extra["unordered"] = True
         if (extra and self.has_feed_forward and getattr(self.mixer, "folds_next_norm", False)
                 and getattr(self.norm2, "folds_into_products", False)
                 and getattr(self.feed_forward, "takes_scaled_rows", False)):

@@ -62,6 +62,11 @@ PART_K = 1024           # the shortest stretch of K a part takes
 PART_K_WIDE, PART_WIDE_BLOCKS = 512, 8
 
 
+def cuts_k(n: int, k: int) -> bool:
+    """Whether a product of few rows that joins the stream has its K cut, so that it is added in no fixed order."""
+    return -(-n // 16) < PART_BELOW_TILES and k >= PART_MIN_K
+
+
 # SiLU-gate products of up to this many rows take the form whose waves own columns and share the rows of A
 # through LDS (gate/up of the 3B shape at 32 / 64 rows: 19 / 22.5 us against the library's 26 / 27 us and 5 us
 # for the SiLU kernel behind it; 14B: 50 / 56 against 55 / 62 + 6; 7B: level); from 65 to 96 rows, on six row tiles
@@ -698,8 +703,7 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
     if rows == 0 and into is None:  # nothing to multiply: no kernel, and no widened copy of the weight
         return torch.empty((0, n // 2 if silu else n), dtype=torch.float32 if wants_f32 else x.dtype, device=x.device)
     fusable = _fusable(rows, k, x.stride(0) if rows > 1 else k, weight)
-    cut_k = (into is not None and -(-n // 16) < PART_BELOW_TILES and k >= PART_MIN_K and into.is_contiguous()
-             and tuple(into.shape) == (rows, n))
+    cut_k = into is not None and cuts_k(n, k) and into.is_contiguous() and tuple(into.shape) == (rows, n)
     if fusable and cut_k and rows <= FUSED_PARTS_ROWS:
         # (atomic adds cost the product nothing, measured against partial products written for the next norm
         # kernel to sum: 10.3 us either way for the 3B shape's down product at 8 rows; and the kernel that summed
@@ -712,8 +716,8 @@ def linear(x: Union[torch.Tensor, ScaledRows, RawRows], weight: torch.Tensor, bi
         ops.gemm_shared_rows(weight, ops.EPI_ATOMIC, x, bias=bias, column_tiles=column_tiles, waves=waves,
                              k_parts=parts, add_into=into)
         return Added()
-    if (fusable and into is None and sums_parts and not silu and not wants_f32 and rows <= FUSED_PARTS_ROWS and -(-n // 16) < PART_BELOW_TILES
-            and k >= PART_MIN_K and x.data_ptr() % 16 == 0):
+    if (fusable and into is None and sums_parts and not silu and not wants_f32 and rows <= FUSED_PARTS_ROWS and cuts_k(n, k)
+            and x.data_ptr() % 16 == 0):
         # a branch that whoever adds it sums itself (the down product of the parallel block, 8 rows, K 11,008: 17 us whole,
         # 11 in 8 parts, and 0.4 more in the kernel that adds them)
         tiles = cut_tiles(x, weight)

@@ -443,6 +443,31 @@ def test_block_whose_first_product_makes_the_norm_itself(rows, monkeypatch):
             check(pending[i: i + 1].float().cpu(), branch[prompt:], "bfloat16")
 
 
+@pytest.mark.parametrize("intermediate,ordered", [(1024, True), (4096, False)])
+def test_decode_rows_whose_sums_have_an_order_repeat_their_bits(intermediate, ordered, monkeypatch):
+    """Decode rows whose keys are cut: a layer whose feed-forward is summed in a fixed order sums its mixer's branch so too, and
+    gives the same bits again; the output product adds its shares in any order only where the down product does."""
+    from cie_amd.config import Qwen2Config
+    from cie_amd.kernels import ops
+    from cie_amd.parts.block import PreNormBlock
+
+    raw = dict(model_type="qwen2", hidden_size=256, num_hidden_layers=1, num_attention_heads=2, num_key_value_heads=1,
+               intermediate_size=intermediate, vocab_size=32, rms_norm_eps=1e-5, rope_theta=1e4, max_position_embeddings=256)
+    block = PreNormBlock(Qwen2Config.from_hf_config(raw).model_spec().layers[0])
+    bound(block, "model.layers.0.", "bfloat16", 25, scale=0.05)
+    prompt = 207  # (a step of 208 keys cuts them)
+    manager, device_cache = harness([block.cache_need()], [prompt + 1] * 2, page_size=16, dtype=block.dtype)
+    g, view = torch.Generator().manual_seed(26), device_cache.view(0)
+    block.forward(torch.randn((2 * prompt, 256), generator=g).cuda(), None, batch_of(manager, [(i, 0, prompt) for i in range(2)]), view)
+    manager.commit_lengths({f"r{i}": prompt for i in range(2)})
+    joined, real = [], ops.merge_project
+    monkeypatch.setattr(ops, "merge_project", lambda *a, **k: (joined.append(1), real(*a, **k))[1])
+    last, batch = torch.randn((2, 256), generator=g).cuda(), batch_of(manager, [(i, prompt, 1) for i in range(2)])
+    outs = [block.forward(last.clone(), None, batch, view)[0] for _ in range(8)]
+    assert bool(joined) != ordered
+    assert not ordered or all(torch.equal(out, outs[0]) for out in outs)
+
+
 # -- a toy mixer with state of its own -----------------------------------------------------
 def register_toy():
     """A decaying running sum per request: s_t = decay * s_{t-1} + W x_t, y_t = s_t.
