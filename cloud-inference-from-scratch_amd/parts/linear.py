@@ -225,11 +225,13 @@ DIRECT_LEVEL = 1.04
 # gate, 346 and 7, the gain in the mean the same 13.4 %.  At 400 row counts that do not recur, where the library takes its first
 # choice, eight of the 336 taken by 1.03.
 DIRECT_MARGIN = 1.03
-# ... but of up to this K also where they are modelled up to 1.15 times slower, at row counts that do not recur: of 131 products
-# between the two lines (150 to 2,047 rows, 1,024 to 16,384 columns, K 768 to 4,096, no epilogue) 112 were faster in the tiles, 11 % in the
-# mean (1,999 rows, K 2,048: 4,736 columns 45.4 -> 38.3 us, 6,144 49.0 -> 47.4; 1,283 rows x 6,144 44.1 -> 32.9), and ten more than 4 %
-# slower (8,192 and more columns most, 1,777 x 8,192 12 %); of 51 beyond it 14, 858 x 12,992, K 8,000, by 26 %.
-DIRECT_MARGIN_SHORT, DIRECT_SHORT_K = 1 / 1.15, 4096
+# ... but of up to this K also where they are modelled up to 1.15 times slower, at row counts that do not recur, and with nothing
+# behind them of fewer columns than this (products between the two lines, 129 to 2,047 rows, K 512 to 4,096, tiles over the library and
+# the kernel behind it in the mean, how many more than 4 % slower: plain, up to 8,191 columns 118, 0.87, 6; 8,192 to 28,000 222, 0.92, 49,
+# 1,315 rows x 17,920, K 2,176 106.9 us for 92.5; the gate, 5,000 to 40,000 columns 143, 0.92, 8, all of 522 to 564 rows x some
+# 17,000; a branch of 512 to 5,000 210, 0.89, 12, most of 232 to 280 rows; none with the rotation lies there.  1,999 rows x 4,736,
+# K 2,048 45.4 -> 38.3 us, x 6,144 49.0 -> 47.4).  Beyond this K 14 of 51 plain ones were slower, 858 x 12,992, K 8,000, by 26 %.
+DIRECT_MARGIN_SHORT, DIRECT_SHORT_K, DIRECT_SHORT_COLUMNS = 1 / 1.15, 4096, 8192
 # Sums of K in parts are at most this many bytes (2,048 rows: 4 parts of the 3B shape's down product 67 MB, 2 of 7B's 59)
 PARTS_BYTES = 128 << 20
 
@@ -274,7 +276,8 @@ def _choose_direct(rows: int, n: int, k: int, most_parts: int, behind: Behind, u
     timed = ops._tune_level(rows)
     library = _library_us(rows, n, k, units, timed) + behind.us + behind.us_per_million * rows * n * 1e-6
     library += behind.host_us if cost <= behind.host_upto else 0.0
-    margin = behind.margin_timed if timed else DIRECT_MARGIN_SHORT if k <= DIRECT_SHORT_K else DIRECT_MARGIN
+    short = k <= DIRECT_SHORT_K and (n < DIRECT_SHORT_COLUMNS or behind is not BEHIND_NOTHING)
+    margin = behind.margin_timed if timed else DIRECT_MARGIN_SHORT if short else DIRECT_MARGIN
     return Tiles(*form, True) if cost * margin < library else None
 
 

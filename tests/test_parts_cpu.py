@@ -151,6 +151,32 @@ def test_tiles_are_taken_where_they_were_measured_to_win(behind, parts, rows, n,
     assert picked is not None or min(tiles.values()) > 0.9 * library
 
 
+# the same at row counts that do not recur, of a short K, where the two models are nearly level
+MEASURED_SHORT = [
+    ("NOTHING", 1, 1999, 4736, 2048, 45.4, {(256, 160, 1): 38.3}, True),
+    ("NOTHING", 1, 2019, 5888, 576, 28.0, {(192, 256, 1): 18.8}, True),
+    ("NOTHING", 1, 366, 704, 3392, 16.5, {(64, 64, 1): 11.5}, True),
+    ("NOTHING", 1, 1310, 6656, 896, 29.1, {(192, 192, 1): 19.9}, True),
+    ("NOTHING", 1, 1315, 17920, 2176, 92.5, {(192, 192, 1): 106.9}, False),
+    ("NOTHING", 1, 1807, 19200, 1024, 76.5, {(192, 192, 1): 88.4}, False),
+    ("NOTHING", 1, 1518, 8704, 1664, 41.5, {(256, 256, 1): 46.8}, False),
+    ("NOTHING", 1, 1067, 11264, 3008, 66.4, {(256, 256, 1): 76.8}, False),
+    ("GATE", 1, 1202, 16512, 3904, 258.6, {(192, 256, 1): 159.3}, True),
+    ("GATE", 1, 524, 23168, 3456, 145.3, {(192, 192, 1): 100.9}, True),
+    ("BRANCH", 1, 345, 1024, 4032, 26.1, {(64, 64, 1): 17.7}, True),
+    ("BRANCH", 1, 565, 960, 3904, 26.9, {(64, 64, 1): 18.4}, True),
+]
+
+
+@pytest.mark.parametrize("behind,parts,rows,n,k,library,tiles,taken", MEASURED_SHORT)
+def test_tiles_of_a_short_k_are_taken_where_they_were_measured_to_win(behind, parts, rows, n, k, library, tiles, taken):
+    from cie_amd.parts import linear
+
+    picked = linear.choose_tiles(rows, n, k, k, most_parts=parts, behind=getattr(linear, "BEHIND_" + behind))
+    assert (picked is not None) == taken
+    assert picked is None or (picked.direct and tiles[picked[:3]] <= 1.03 * library)
+
+
 @pytest.mark.parametrize("behind", ["NOTHING", "GATE", "BRANCH", "ROTATION"])
 def test_the_tiles_that_are_chosen_are_tiles_there_are(behind):
     """Over rows, widths and K: a form that the kernel has, parts of K that all have some, sums within their limit, and the
