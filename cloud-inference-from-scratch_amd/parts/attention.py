@@ -190,7 +190,7 @@ MANY_DECODE_UNITS = 96  # (sequence, kv head) pairs from which decode rows take 
 MANY_PART_BYTES = 300 << 10  # keys and values of one pair below which its keys are not cut then
 SOME_DECODE_UNITS = 33  # ... and from which they may with a merge of their own: whole while a pair reads no more than so many bytes,
 WHOLE_UNIT_BYTES = 176 << 10
-SOME_DECODE_KEYS = 48 << 10  # in parts where all pairs together have so many keys
+SOME_DECODE_KEYS = 48 << 10  # in parts where all pairs together have so many keys (and not as many as they may come to have)
 SHARED_DECODE_KEYS = 96  # contexts from which four waves share a decode row's keys without cutting them
 SPLIT_MIN_KEYS = 32  # the fewest keys of a one-wave part
 SPLIT_DECODE_KEYS = 192  # contexts from which the keys of decode rows are cut into parts at all
@@ -340,11 +340,13 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
         # ... and with a merge of its own from some dozens of pairs on: whole where a pair has little to read, four waves where
         # all have much (us, merge with it, one wave's parts, four waves whole, four waves' parts: 24 rows of 14 heads of 64 on 2 over 300
         # keys 7.9, 6.3, 9.0, 640 10.4, 9.1, 10.3, 1,600 14.5, 14.6, 12.1; of 16 heads of 128 on 2 over 300 9.0, 9.1, 10.4, 640 11.9, 13.6,
-        # 12.6, 1,600 17.9, 25.1, 16.5; 32 rows 9.6, 9.3, 11.0, 12.9, 13.9, 13.1, 21, 25.9, 19.4).
+        # 12.6, 1,600 17.9, 25.1, 16.5; 32 rows 9.6, 9.3, 11.0, 12.9, 13.9, 13.1, 21, 25.9, 19.4).  Not by a captured step's bound: over
+        # few keys the four waves' parts are the slower form whatever the bound (32 rows, bound 1,500, one wave's parts and four waves'
+        # over 60 keys 7.9, 9.6, 300 9.2, 10.6, 1,000 15.3, 15.3).
         if wide and not joined and SOME_DECODE_UNITS <= units < MANY_DECODE_UNITS:
             if SHARED_DECODE_KEYS <= bound <= WHOLE_UNIT_BYTES // (4 * head_dim):
                 return ops.TILE_WAVES, dict(target_waves=cus, min_keys=bound + 1)
-            if units * bound >= SOME_DECODE_KEYS:
+            if batch.static_plan is None and units * bound >= SOME_DECODE_KEYS:
                 return ops.TILE_WAVES, dict(target_waves=cus, min_keys=32 * ops.TILE_WAVES)
         # Many pairs fill the GPU by themselves: the same form with the keys whole or in large parts
         # (64 sequences x 2 heads x 256 keys: 9.2 us against 11.1 us with one wave per part).  A second part pays for

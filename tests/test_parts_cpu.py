@@ -206,6 +206,44 @@ def test_the_tiles_that_are_chosen_are_tiles_there_are(behind):
         assert picked is None or not picked.direct
 
 
+def decode_form(monkeypatch, q_heads, kv_heads, dim, rows, longest, bound=None, unmerged=False, page=16):
+    """(waves a part, parts, whether they come back unmerged) of a step of ``rows`` single tokens over up to ``longest`` keys, launch by
+    launch, or as captured for up to ``bound`` keys."""
+    from cie_amd.engine.batch import PagedView, StepBatch
+    from cie_amd.engine.graphs import StaticPlan
+    from cie_amd.kernels import ops
+    from cie_amd.parts import attention
+
+    ints = lambda values: torch.tensor(list(values), dtype=torch.int32)  # noqa: E731
+    starts = [longest - 1 - i % min(longest, 7) for i in range(rows)]
+    step = StepBatch(tokens=rows, sequences=rows, token_ids=ints([0] * rows), positions=ints(starts), seq_of_token=ints(range(rows)),
+                     seq_slot=ints(range(rows)), seq_start=ints(starts), seq_q_len=ints([1] * rows), q_start_loc=ints(range(rows + 1)),
+                     logit_rows=ints([0]), host_slots=list(range(rows)), host_starts=starts, host_q_lens=[1] * rows,
+                     static_plan=None if bound is None else StaticPlan(ints(range(rows)), ints([0] * rows), ints([longest]), bound))
+    view = PagedView(torch.empty(1, kv_heads, page, dim), torch.empty(1, kv_heads, dim, page), ints([0] * rows).view(rows, 1), page)
+    calls = []
+    monkeypatch.setattr(ops, "paged_attention_mfma", lambda *a, **k: calls.append((k["tile_waves"], k["n_splits"], not k["merge"])))
+    out = attention.attend(torch.empty(rows, (q_heads + 2 * kv_heads) * dim, dtype=torch.bfloat16), step, view, q_heads, kv_heads, dim, None,
+                           dim ** -0.5, unmerged=unmerged)
+    (form,) = calls
+    assert form[2] == isinstance(out, attention.Shares) and (form[1] > 1 or not form[2])
+    return form
+
+
+@pytest.mark.parametrize("heads", [(16, 2, 128), (14, 2, 64)])
+@pytest.mark.parametrize("rows", [17, 24, 32, 47])
+def test_a_captured_steps_keys_are_not_cut_by_its_bound_alone(heads, rows, monkeypatch):
+    """Some dozens of pairs: parts of one wave, which are the faster ones over few keys, whatever the limit (below the one from which
+    every step has four waves); launch by launch the keys are known, and many of them are four waves'."""
+    for bound in (1024, 1500, 2047):
+        for longest in (60, 300, 1000):
+            waves, parts, _ = decode_form(monkeypatch, *heads, rows, longest, bound)
+            assert (waves, parts > 1) == (1, True)
+    assert decode_form(monkeypatch, *heads, rows, 1600)[0] == 4
+    assert decode_form(monkeypatch, *heads, rows, 60, 4096)[0] == 4
+    assert decode_form(monkeypatch, *heads, rows, 300, 304)[:2] == (4, 1)  # (whole: one kernel and no merge)
+
+
 def test_which_portions_take_the_form_through_lds():
     from cie_amd.parts.attention import takes_prompt_form
 
