@@ -324,7 +324,8 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
              and takes_prompt_form(small_tiles, prompt_keys, singles, batch.static_plan is not None, cus))
     lds_row_tiles = 8 if head_dim == 128 and big_tiles > LARGE_TILES_ABOVE * cus else 4
 
-    def decode_form(bound: int, units: int, joined: bool) -> tuple[int, dict]:
+    def decode_form(bound: int, units: int, room: int) -> tuple[int, dict]:
+        joined = room > 0  # (up to so many shares of a unit come back unmerged)
         # Decode rows, `units` (sequence, kv head) pairs over up to `bound` keys.  Long contexts: four waves
         # per (sequence, kv head, part of the keys) take the part's blocks in turn with their loads running
         # ahead (15.8 against 18.1 us for 8 x 4,096 keys).  A few pairs do not fill the GPU that way: they take the
@@ -365,14 +366,25 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
             # (joined: shares of 128 keys and less only while all of them are fewer than the units; one row of 16 heads on 2 over
             # 1,000 keys at a bound of 32,768 14.3 -> 11.8 us, over 32,000 20.5 -> 19.7; 8 rows over 800 keys 13.2 -> 12.0, 16 over 400 13.9 -> 12.7)
             most = min(4 * cus, max(cus, units * (bound // 128))) if joined else 4 * cus
+            # (a few pairs at a limit that gives more parts than the product takes: four waves a part, and as many parts as its threads read
+            # in whole turns, a power of two; with a merge of their own and so, a bound of 32,768, over 300 / 8,000 / 32,000 keys, 8 heads
+            # of 128 on 1, 4 rows 15.3, 20.3, 30.9 -> 11.1, 17.3, 29.4 us, 5 rows 15.2, 21.2, 35.1 -> 10.8, 16.0, 30.7; of 64 14.1, 18.4, 27.5
+            # -> 10.0, 12.5, 19.8; 16 heads on 2, 3 rows 15.7, 21.8, 38.0 -> 10.8, 15.9, 31.3.  85 parts of 3 rows 23.8 over 16,000, 64 20.1)
+            if joined and plan_splits(units, bound, most, SPLIT_MIN_KEYS)[0] > room:
+                if wide:
+                    return ops.TILE_WAVES, dict(target_waves=units << (cus // units).bit_length() - 1, min_keys=64)
+                most = 4 * cus
             return 1, dict(target_waves=most, min_keys=SPLIT_MIN_KEYS)
         # ... and below some 200 keys, where the merge costs more than it saves, four waves that share a
         # sequence's few blocks inside one workgroup instead of one wave that takes them in turn
         # (8 x 128 keys: 6.5 against 6.9 us, 8 x 160: 7 against 11)
         return (ops.TILE_WAVES if wide and bound >= SHARED_DECODE_KEYS else 1), dict(target_waves=4 * cus, min_keys=bound + 1)
 
+    def shares_taken(rows: int) -> int:
+        return MERGE_SHARES >> (rows - 1).bit_length() if unmerged and rows == batch.tokens else 0
+
     def leave(n_splits: int, rows: int) -> bool:
-        return unmerged and n_splits > 1 and rows == batch.tokens and n_splits << (rows - 1).bit_length() <= MERGE_SHARES
+        return 1 < n_splits <= shares_taken(rows)
 
     plan = batch.static_plan
     longest_dev = None
@@ -385,7 +397,7 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
         decode_rows = batch.sequences if plan.decode_rows is None else plan.decode_rows
         joined = wide and not eight and 0 < decode_rows <= JOINED_DECODE_ROWS and decode_rows < batch.sequences
         if decode_rows and not joined:
-            decode_waves, split_options = decode_form(max_keys, decode_rows * num_kv_heads, unmerged and decode_rows == batch.tokens)
+            decode_waves, split_options = decode_form(max_keys, decode_rows * num_kv_heads, shares_taken(decode_rows))
             units = decode_rows * num_kv_heads
             n_splits, _ = plan_splits(units, max_keys, **split_options)
             if n_splits > 1 and decode_waves > 1:
@@ -412,7 +424,7 @@ def attend(qkv: torch.Tensor, batch, view, num_heads: int, num_kv_heads: int, he
         # (not beside the form of eight waves, where a tile of one token would leave six of them idle)
         joined = wide and not eight and 0 < n_tiles <= JOINED_DECODE_ROWS and n_tiles < batch.sequences
     if n_tiles and not joined:
-        decode_waves, split_options = decode_form(max_keys, n_tiles * num_kv_heads, unmerged and n_tiles == batch.tokens)
+        decode_waves, split_options = decode_form(max_keys, n_tiles * num_kv_heads, shares_taken(n_tiles))
         n_splits, per_split = plan_splits(n_tiles * num_kv_heads, max_keys, **split_options)
         part_o = part_ml = None
         if n_splits > 1:

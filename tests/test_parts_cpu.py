@@ -244,6 +244,21 @@ def test_a_captured_steps_keys_are_not_cut_by_its_bound_alone(heads, rows, monke
     assert decode_form(monkeypatch, *heads, rows, 300, 304)[:2] == (4, 1)  # (whole: one kernel and no merge)
 
 
+@pytest.mark.parametrize("page", [8, 16])
+def test_shares_that_are_planned_for_the_output_product_are_left_to_it(page, monkeypatch):
+    """Up to 16 single tokens, at bounds that give more parts than the output product takes: a form of which it takes all, or, with
+    pages that have no such form, the one with a merge of its own."""
+    for heads in ((8, 1, 128), (16, 1, 64), (16, 2, 128), (14, 2, 64), (28, 4, 128), (32, 8, 64)):
+        for rows in range(1, 17):
+            for bound in (None, 300, 1000, 2040, 4096, 16384, 32768, 131072):
+                longest = 20000 if bound is None else min(bound, 1000)
+                waves, parts, unmerged = decode_form(monkeypatch, *heads, rows, longest, bound, unmerged=True, page=page)
+                if page >= 16:
+                    assert unmerged == (parts > 1)
+                elif parts > 1 and not unmerged:
+                    assert (waves, parts) == decode_form(monkeypatch, *heads, rows, longest, bound, page=page)[:2]
+
+
 def test_which_portions_take_the_form_through_lds():
     from cie_amd.parts.attention import takes_prompt_form
 
