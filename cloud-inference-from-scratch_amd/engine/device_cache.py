@@ -62,8 +62,9 @@ class DeviceCache:
         # as this object
         row_bytes = [state[0].numel() * state.element_size() for state in self.states.values()]
         self._most_state_bytes = max(row_bytes, default=0)
+        self._on_gpu = torch.device(device).type == "cuda"  # (a cache in host memory takes its rows one by one)
         self._state_rows = torch.tensor([[state.data_ptr(), size] for state, size in zip(self.states.values(), row_bytes)],
-                                        dtype=torch.int64, device=device) if self.states else None
+                                        dtype=torch.int64, device=device) if self.states and self._on_gpu else None
         self._views: dict[int, Any] = {}
         for unit in range(len(manager.unit_specs)):
             if unit in manager.unit_group:
@@ -106,10 +107,10 @@ class DeviceCache:
                 appended.setdefault(group, []).append((slot, first, table[first:]))
             self._row_seen[(group, slot)] = (serial, len(table))
         for group, rows in appended.items():
-            if len(rows) == 1:
-                slot, first, entries = rows[0]
-                staged = to_device_staging([max(p, 0) for p in entries], self.device)
-                self.tables[group][slot, first: first + len(entries)].copy_(staged, non_blocking=True)
+            if len(rows) == 1 or not self._on_gpu:
+                for slot, first, entries in rows:
+                    staged = to_device_staging([max(p, 0) for p in entries], self.device)
+                    self.tables[group][slot, first: first + len(entries)].copy_(staged, non_blocking=True)
                 continue
             # several rows: one copy and one launch for all of them
             heads, at = [], 4 * len(rows)
@@ -124,7 +125,10 @@ class DeviceCache:
             np.maximum(host, 0, out=host)
             ops.table_rows(plan.to(self.device, non_blocking=True), len(rows), self.tables[group])
         fresh = self.manager.take_fresh_slots()
-        if fresh and self.states:
+        if fresh and not self._on_gpu:
+            for state in self.states.values():
+                state[fresh] = 0
+        elif fresh and self.states:
             # (the slots' numbers as an asynchronous copy: an index made on the device from a list waits for the stream)
             slots = to_device_staging(fresh, self.device).to(self.device, non_blocking=True)
             ops.clear_rows(self._state_rows, slots, self._most_state_bytes)

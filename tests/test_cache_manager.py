@@ -515,3 +515,28 @@ def test_a_float32_engine_sets_its_kernels_workspace_aside():
 
     apart = reserve_bytes(build_engine_config(dtype="float32"), 2048, 1000) - reserve_bytes(build_engine_config(), 2048, 1000)
     assert apart == ops.F32_WORKSPACE_BYTES - ops.LIBRARY_WORKSPACE_BYTES
+
+
+def test_a_cache_in_host_memory_follows_the_tables_and_clears_fresh_states():
+    """Several requests between two syncs, where no kernel can bring their rows over."""
+    import torch
+
+    from cie_amd.engine.device_cache import DeviceCache
+
+    manager = CacheManager([PagedKV(2, 16), FixedState((3, 5))], 4, kv_tokens=64, max_running=4, max_model_len=32)
+    cache = DeviceCache(manager, torch.float32, torch.device("cpu"))
+    (state,) = cache.states.values()
+    state.fill_(1.0)
+    want = {}
+    for name, tokens in (("a", 9), ("b", 1), ("c", 17)):
+        manager.admit(name)
+        manager.ensure_capacity_batch({name: tokens})
+        want[name] = tokens
+    cache.sync()
+    entries = []
+    for name, tokens in want.items():
+        pages = -(-tokens // 4)
+        entries += cache.tables[0][manager.slot(name), :pages].tolist()
+        assert not state[manager.slot(name)].any()
+    assert sorted(entries) == sorted(set(entries)) and len(entries) == 9  # (3 + 1 + 5 pages, each once)
+    assert state[cache.pad_slot].all()
