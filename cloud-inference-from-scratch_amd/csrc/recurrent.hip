@@ -1251,15 +1251,17 @@ gated_outputs_kernel(const bf16_t* __restrict__ y_pre, long ldy, const bf16_t* _
                      const int* __restrict__ seq_slot, const int* __restrict__ q_start_loc, bf16_t* __restrict__ out, int tokens,
                      int channels, int keep_n, int token_groups) {
     __shared__ float start[256];  // the channels' states in front of the chunk
-    const int c0 = blockIdx.x * 256;
-    if (blockIdx.y >= token_groups) {  // behind the tokens: a sequence's inputs, a channel a thread
-        const int keeps = blockIdx.y - token_groups, own = c0 + threadIdx.x;
+    // (one grid dimension: portions and sequences together may be more than the others hold)
+    const int channel_groups = (channels + 255) / 256;
+    const int c0 = blockIdx.x % channel_groups * 256, place = blockIdx.x / channel_groups;
+    if (place >= token_groups) {  // behind the tokens: a sequence's inputs, a channel a thread
+        const int keeps = place - token_groups, own = c0 + threadIdx.x;
         if (own < channels)
             keep_inputs(past + static_cast<size_t>(seq_slot[keeps]) * keep_n * channels, x_in, ldx, q_start_loc[keeps],
                         q_start_loc[keeps + 1] - q_start_loc[keeps], own, channels, keep_n);
         return;
     }
-    const int t0 = blockIdx.y * kOutputTokens;
+    const int t0 = place * kOutputTokens;
     const int chunk = t0 / kChunkTokens;
     const int c = c0 + threadIdx.x % 32 * 8;
     const int cc = min(c, channels - 8);  // (a thread past the last channel reads and stores nothing of its own)
@@ -1706,7 +1708,8 @@ CIE_API int cie_gated_recurrence_chunks(void* stream, const void* y_pre, long ld
     const int chunks = (tokens + kChunkTokens - 1) / kChunkTokens;
     const long groups = static_cast<long>(chunks) * (channels / kChunkChannels);
     const int token_groups = (tokens + kOutputTokens - 1) / kOutputTokens;
-    if (groups > 0x7fffffffL || static_cast<long>(token_groups) + sequences > 65535) return CIE_BAD_ARGUMENT;
+    const long outputs = (channels + 255L) / 256 * (token_groups + (taps > 1 ? static_cast<long>(sequences) : 0L));
+    if (groups > 0x7fffffffL || outputs > 0x7fffffffL) return CIE_BAD_ARGUMENT;
     hipStream_t s = static_cast<hipStream_t>(stream);
     float* plane_b = planes + static_cast<size_t>(tokens) * channels;
 #define CIE_CHUNKS(BW)                                                                                                     \
@@ -1719,7 +1722,7 @@ CIE_API int cie_gated_recurrence_chunks(void* stream, const void* y_pre, long ld
 #undef CIE_CHUNKS
     const int code = cie_after_launch();
     if (code != CIE_OK) return code;
-    gated_outputs_kernel<<<dim3((channels + 255) / 256, token_groups + (taps > 1 ? sequences : 0)), 256, 0, s>>>(
+    gated_outputs_kernel<<<static_cast<unsigned>(outputs), 256, 0, s>>>(
         static_cast<const bf16_t*>(y_pre), ldy, static_cast<const bf16_t*>(x_in), ldx, planes, plane_b, carry, state, past, seq_of_token,
         seq_slot, q_start_loc, static_cast<bf16_t*>(out), tokens, channels, taps - 1, token_groups);
     return cie_after_launch();

@@ -822,3 +822,25 @@ def test_gated_recurrence_in_chunks_is_as_near_to_64_bits_as_the_walk():
             off[name] += float(((mine.double() - want).norm() / want.norm()) ** 2)
     # (a token has the walk's own rounding and what fades of those in front, which is the same or, at a chunk's first tokens, one more)
     assert off["chunks"] ** 0.5 <= 1.05 * off["walk"] ** 0.5, off
+
+
+def test_gated_recurrence_in_chunks_of_very_many_sequences():
+    """More sequences and groups of tokens together than a grid's second dimension holds, as the product and the walk take them."""
+    from cie_amd.kernels import ops
+
+    lengths, width, taps = (1,) * 64990 + (20000,), 64, 2
+    g = torch.Generator().manual_seed(11)
+    tokens, n = sum(lengths), len(lengths)
+    proj, u = (torch.randn(tokens, k * width, generator=g).bfloat16().cuda() for k in (2, 1))
+    weight, bias = (torch.randn(1, 2 * width, width, generator=g) * width ** -0.5).bfloat16().cuda(), torch.zeros(1, 2 * width).bfloat16().cuda()
+    rate = -8.0 * torch.rand(width, generator=g).cuda()
+    state, past = torch.randn(n, width, generator=g).cuda(), torch.randn(n, 1, width, generator=g).cuda()
+    of_token, slots = torch.arange(tokens, dtype=torch.int32).clamp(max=n - 1).cuda(), torch.arange(n, dtype=torch.int32).cuda()
+    starts = torch.tensor([*range(n), tokens], dtype=torch.int32).cuda()
+    state2, past2 = state.clone(), past.clone()
+    out = ops.gated_recurrence_chunks(proj[:, :width], proj[:, width:], u, weight, bias, rate, state, past, of_token, slots, starts, n, taps)
+    want = ops.gated_recurrence(proj[:, :width], proj[:, width:], u, ops.block_linear(u, weight, bias, out_dtype=torch.float32), width, rate,
+                                state2, past2, slots, starts, n, taps)
+    near = width * 2.0 ** -24 * 8 + 2e-6  # (as above)
+    assert torch.allclose(state, state2, atol=near, rtol=near) and torch.equal(past, past2)
+    assert torch.allclose(out.float(), want.float(), atol=4 * near, rtol=2.0 ** -7)
