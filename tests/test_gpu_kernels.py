@@ -1866,15 +1866,35 @@ def test_gemm_qkv_rope_in_blocks_of_rows(ops, geometry, rows):
         ops.gemm_qkv_rope(w, a, b, cos, sin, *meta, k_got, v_got, q_heads, kv_heads, head_dim, waves=2, blocks=(2, True))
 
 
-# (query heads, key heads, head size, rows, longest context): both sides of every line between the forms of a decode step's keys
-DECODE_LINES = [(16, 2, 128, 8, 1023), (16, 2, 128, 8, 1024), (14, 2, 64, 16, 511), (14, 2, 64, 16, 512), (16, 2, 128, 3, 2500), (16, 2, 128, 4, 2048),
-                (28, 4, 128, 9, 600), (32, 8, 64, 12, 700), (14, 2, 64, 17, 704), (14, 2, 64, 17, 705), (16, 2, 128, 30, 352), (16, 2, 128, 30, 353),
-                (16, 2, 128, 25, 983), (14, 2, 64, 32, 1700), (4, 2, 32, 20, 90), (8, 1, 128, 40, 1300)]
+# (query heads, key heads, head size, rows, longest context): both sides of every line between the forms of a decode step's keys, and
+# the (waves a part, parts, whether the output product merges them) of each step launch by launch, captured for that bound, for one
+# 900 keys longer and for 32,768
+DECODE_LINES = {
+    (16, 2, 128, 8, 1023): [(1, 16, True), (1, 16, True), (4, 16, True), (4, 16, True)],
+    (16, 2, 128, 8, 1024): [(4, 16, True), (4, 16, True), (4, 16, True), (4, 16, True)],
+    (14, 2, 64, 16, 511): [(1, 8, True), (1, 8, True), (4, 8, True), (4, 8, True)],
+    (14, 2, 64, 16, 512): [(4, 8, True), (4, 8, True), (4, 8, True), (4, 8, True)],
+    (16, 2, 128, 3, 2500): [(1, 40, True), (1, 40, True), (1, 36, True), (4, 32, True)],
+    (16, 2, 128, 4, 2048): [(4, 32, True), (4, 32, True), (4, 32, True), (4, 32, True)],
+    (28, 4, 128, 9, 600): [(4, 7, True), (4, 7, True), (4, 7, True), (4, 7, True)],
+    (32, 8, 64, 12, 700): [(4, 1, False), (4, 1, False), (4, 1, False), (4, 2, True)],
+    (8, 1, 128, 3, 700): [(1, 11, True), (1, 11, True), (1, 50, True), (4, 64, True)],
+    (14, 2, 64, 17, 704): [(4, 1, False), (4, 1, False), (1, 26, False), (4, 7, False)],
+    (14, 2, 64, 17, 705): [(1, 12, False), (1, 12, False), (1, 26, False), (4, 7, False)],
+    (16, 2, 128, 30, 352): [(4, 1, False), (4, 1, False), (1, 14, False), (4, 4, False)],
+    (16, 2, 128, 30, 353): [(1, 6, False), (1, 6, False), (1, 14, False), (4, 4, False)],
+    (16, 2, 128, 25, 983): [(1, 16, False), (1, 16, False), (1, 20, False), (4, 5, False)],
+    (16, 2, 128, 25, 984): [(4, 5, False), (1, 16, False), (1, 20, False), (4, 5, False)],
+    (14, 2, 64, 32, 1700): [(4, 4, False), (1, 14, False), (4, 4, False), (4, 4, False)],
+    (4, 2, 32, 20, 90): [(1, 1, False), (1, 1, False), (4, 1, False), (4, 6, False)],
+    (8, 1, 128, 40, 1300): [(4, 6, False), (1, 21, False), (4, 6, False), (4, 6, False)],
+}
 
 
-@pytest.mark.parametrize("line", DECODE_LINES)
-def test_decode_forms_on_both_sides_of_their_lines(ops, line):
-    """A step of single tokens through the attention and, where that takes the keys' shares as they are, the output product."""
+def decode_line(ops, monkeypatch, line, window=None):
+    """The (waves, parts, unmerged) of a step of single tokens launch by launch and as captured.  The step's context, or, where the
+    output product merges the parts, what that makes of them with an identity for its weight, is checked against the oracle, and
+    against what the merge kernel makes of the same parts; a part or a head that is lost would show."""
     from cie_amd.engine.batch import PagedView, StepBatch
     from cie_amd.engine.graphs import StaticPlan
     from cie_amd.parts import attention as A
@@ -1886,25 +1906,59 @@ def test_decode_forms_on_both_sides_of_their_lines(ops, line):
     k_pool, v_pool, table, slots, dense = build_cache(torch.bfloat16, lengths, kv_heads, dim, page, seed=5)
     as_dev = lambda values: torch.tensor(values, dtype=torch.int32).cuda()  # noqa: E731
     qkv = rand((rows, width + 2 * kv_heads * dim), torch.bfloat16, 1, 2.0)
-    w = rand((256, width), torch.bfloat16, 2, 0.05)
-    want = torch.cat([plain_qwen2.causal_attention(qkv[i: i + 1, :width].float().cpu().view(1, q_heads, dim), *dense[i], dim ** -0.5,
-                                                   past_len=contexts[i]) for i in range(rows)]).cuda()
+    one = torch.eye(width, dtype=torch.bfloat16, device="cuda")
+    query = lambda i: qkv[i: i + 1, :width].float().cpu().view(1, q_heads, dim)  # noqa: E731
+    want = torch.cat([plain_qwen2.causal_attention(query(i), *dense[i], dim ** -0.5, past_len=contexts[i], window=window)
+                      for i in range(rows)])
+    near = lambda got, expect: bool(torch.isclose(got.float().cpu(), expect, **tol(torch.bfloat16)).all())  # noqa: E731
+    # (what the bound sees: the oracle without 32 of the longest row's last keys, and without one head)
+    i = rows // 2
+    last = slice(contexts[i] - 40, contexts[i] - 8)
+    fewer = [torch.cat([t[: last.start], t[last.stop:]]) for t in dense[i]]
+    assert not near(plain_qwen2.causal_attention(query(i), *fewer, dim ** -0.5, past_len=contexts[i] - 32,
+                                                 window=None if window is None else window - 32), want[i: i + 1])
+    no_head = want.clone()
+    no_head[:, :dim] = 0
+    assert not near(no_head, want)
+
     batch = dict(tokens=rows, sequences=rows, token_ids=as_dev([0] * rows), positions=as_dev(contexts), seq_of_token=as_dev(range(rows)),
                  seq_slot=as_dev(slots), seq_start=as_dev(contexts), seq_q_len=as_dev([1] * rows), q_start_loc=as_dev(range(rows + 1)),
                  logit_rows=as_dev([0]), host_slots=slots, host_starts=contexts, host_q_lens=[1] * rows)
-    # launch by launch, and as in a captured step, for a tight and a loose bound
+    forms, merged, real = [], [], ops.paged_attention_mfma
+
+    def attention(*args, **kwargs):
+        forms.append((kwargs["tile_waves"], kwargs["n_splits"], not kwargs["merge"]))
+        if not kwargs["merge"]:
+            real(*args, **{**kwargs, "merge": True})
+            merged.append(args[12].clone())
+        real(*args, **kwargs)
+
+    monkeypatch.setattr(ops, "paged_attention_mfma", attention)
     plans = [None] + [StaticPlan(as_dev(range(rows)), as_dev([0] * rows), as_dev([longest]), bound) for bound in (longest, longest + 900, 32768)]
     for plan in plans:
         view = PagedView(k_pool, v_pool, table, page)
-        step = StepBatch(**batch, static_plan=plan)
-        stream = torch.zeros((rows, 256), device="cuda")
-        joins = A.joins_merge(rows, w, stream)
+        stream = torch.zeros((rows, width), device="cuda")
+        joins = A.joins_merge(rows, one, stream)
         assert joins == (rows <= 16 and width % 128 == 0)
-        out = A.attend(qkv, step, view, q_heads, kv_heads, dim, None, dim ** -0.5, unmerged=joins)
+        out = A.attend(qkv, StepBatch(**batch, static_plan=plan), view, q_heads, kv_heads, dim, window, dim ** -0.5, unmerged=joins)
         if isinstance(out, A.Shares):
-            ops.merge_project(out.part_o, out.part_ml, w, None, stream, q_heads, kv_heads, dim, out.splits, out.tile_rows)
-            # the rows' rounding (and their error, as below) through the product
-            bound = want.abs() @ w.float().abs().t() * 2 ** -7 + 1e-2 * w.float().abs().sum(dim=1)
-            assert ((stream - want @ w.float().t()).abs() <= bound).all()
-        else:
-            torch.testing.assert_close(out.float(), want, **tol(torch.bfloat16))
+            ops.merge_project(out.part_o, out.part_ml, one, None, stream, q_heads, kv_heads, dim, out.splits, out.tile_rows)
+            # (a row's numbers, rounded to bf16 and times 1; both roundings are of float32 sums of the same parts: one step apart at most)
+            assert ((stream - merged[-1].float()).abs() <= 2.0 ** -7 * merged[-1].float().abs()).all()
+            out = stream
+        torch.testing.assert_close(out.float().cpu(), want, **tol(torch.bfloat16))
+    return forms
+
+
+@pytest.mark.parametrize("line", DECODE_LINES)
+def test_decode_forms_on_both_sides_of_their_lines(ops, line, monkeypatch):
+    """A step of single tokens through the attention and, where that takes the keys' shares as they are, the output product."""
+    assert decode_line(ops, monkeypatch, line) == DECODE_LINES[line]
+
+
+@pytest.mark.parametrize("line,window", [((16, 2, 128, 8, 3000), 1000), ((14, 2, 64, 16, 1500), 300), ((16, 2, 128, 3, 900), 640),
+                                         ((28, 4, 128, 9, 600), 333)])
+def test_shares_under_a_window_left_to_the_output_product(ops, line, window, monkeypatch):
+    """... where a row's first shares begin behind its first key, and a short row's last ones have none."""
+    forms = decode_line(ops, monkeypatch, line, window)
+    assert all(parts > 1 and unmerged for _waves, parts, unmerged in forms)

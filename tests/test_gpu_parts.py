@@ -468,6 +468,50 @@ def test_decode_rows_whose_sums_have_an_order_repeat_their_bits(intermediate, or
     assert not ordered or all(torch.equal(out, outs[0]) for out in outs)
 
 
+@pytest.mark.parametrize("rows", [1, 5, 8, 9, 16])
+def test_block_whose_gate_product_makes_the_norm_itself(rows, monkeypatch):
+    """Decode rows whose keys are cut, in a layer whose output product merges them: the mixer's branch is added to the stream, and
+    the feed-forward's first product makes the norm behind it.  The layer agrees with the plain one, and with itself where the norm
+    has a kernel of its own."""
+    from cie_amd.cache import CacheManager
+    from cie_amd.config import Qwen2Config
+    from cie_amd.engine.device_cache import DeviceCache
+    from cie_amd.kernels import ops
+    from cie_amd.parts import block as blocks
+
+    hidden, prompt, p = 256, 207, "model.layers.0."
+    raw = dict(model_type="qwen2", hidden_size=hidden, num_hidden_layers=1, num_attention_heads=2, num_key_value_heads=1,
+               intermediate_size=4096, vocab_size=32, rms_norm_eps=1e-5, rope_theta=1e4, max_position_embeddings=256)
+    block = blocks.PreNormBlock(Qwen2Config.from_hf_config(raw).model_spec().layers[0])
+    w = bound(block, p, "bfloat16", 35, scale=0.05)
+    manager = CacheManager([block.cache_need()], 16, kv_tokens=224 * rows, max_running=rows, max_model_len=256)
+    device_cache = DeviceCache(manager, block.dtype, torch.device("cuda:0"))
+    for i in range(rows):
+        manager.admit(f"r{i}")
+    manager.ensure_capacity_batch({f"r{i}": prompt + 1 for i in range(rows)})
+    device_cache.sync()
+    g, view = torch.Generator().manual_seed(36), device_cache.view(0)
+    hs = [torch.randn((prompt + 1, hidden), generator=g) * (0.5 + 0.25 * i) for i in range(rows)]
+    block.forward(torch.cat([h[:prompt] for h in hs]).cuda(), None, batch_of(manager, [(i, 0, prompt) for i in range(rows)]), view)
+    manager.commit_lengths({f"r{i}": prompt for i in range(rows)})
+    made, real = [], ops.gemm_shared_rows_normed
+    monkeypatch.setattr(ops, "gemm_shared_rows_normed", lambda *a, **k: (made.append(1), real(*a, **k))[1])
+    last, batch = torch.cat([h[prompt:] for h in hs]).cuda(), batch_of(manager, [(i, prompt, 1) for i in range(rows)])
+    got = block.forward(last.clone(), None, batch, view)[0].cpu()
+    assert made == [1]
+    monkeypatch.setattr(blocks.RawRows, "fits", staticmethod(lambda residual, dtype: False))
+    apart = block.forward(last.clone(), None, batch, view)[0].cpu()
+    assert made == [1]
+    check(got, apart, "bfloat16")
+    cos, sin = plain.rope_tables(128, prompt + 1, 1e4)
+    for i, h in enumerate(hs):
+        a = plain.rms_norm(h, w[p + "input_layernorm.weight"], 1e-5)
+        mid = h + plain.attention_layer(a, w, p + "self_attn.", raw, cos, sin, torch.arange(prompt + 1))
+        m = plain.rms_norm(mid, w[p + "post_attention_layernorm.weight"], 1e-5)
+        branch = plain.swiglu(m, w[p + "mlp.gate_proj.weight"], w[p + "mlp.up_proj.weight"], w[p + "mlp.down_proj.weight"])
+        check(got[i: i + 1], (mid + branch)[prompt:], "bfloat16")
+
+
 # -- a toy mixer with state of its own -----------------------------------------------------
 def register_toy():
     """A decaying running sum per request: s_t = decay * s_{t-1} + W x_t, y_t = s_t.

@@ -844,3 +844,20 @@ def test_gated_recurrence_in_chunks_of_very_many_sequences():
     near = width * 2.0 ** -24 * 8 + 2e-6  # (as above)
     assert torch.allclose(state, state2, atol=near, rtol=near) and torch.equal(past, past2)
     assert torch.allclose(out.float(), want.float(), atol=4 * near, rtol=2.0 ** -7)
+
+
+@pytest.mark.parametrize("joined", [True, False])
+@pytest.mark.parametrize("name", sorted(pu.SMALL))
+def test_layers_whose_first_products_run_in_one_launch(models, name, joined, monkeypatch):
+    """Single tokens through layers whose branches start in one launch and end in one, or, where the last products' columns are too
+    many for that, in one each; against the plain implementation."""
+    from cie_amd.parts import block, linear
+
+    raw, weights, requests, plain = models[name]
+    if not joined:
+        monkeypatch.setattr(linear, "PART_BELOW_TILES", 1)
+    begun, ended = [], []
+    for kept, which in ((begun, "silu_beside"), (ended, "parts_beside")):
+        monkeypatch.setattr(block, which, lambda *a, kept=kept, real=getattr(block, which): (kept.append(real(*a)), kept[-1])[1])
+    run_and_compare(raw, weights, requests, replay_util.tail_one_by_one(requests, tail=8), "bfloat16", plain)
+    assert any(out is not None for out in begun) and ended and all((out is not None) == joined for out in ended)
