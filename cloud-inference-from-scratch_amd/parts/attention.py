@@ -101,6 +101,7 @@ class Attention(Part):
             if self.qkv_bias else None
         )
         self.w_o = per_head(tensors[prefix + "o_proj.weight"].t()).t().contiguous()
+        self.cuts_o = cuts_k(*self.w_o.shape)  # (whose sum has no fixed order then, whoever merges its rows)
         self.b_o = tensors[prefix + "o_proj.bias"].contiguous() if self.out_bias else None
         self.cos, self.sin = self.position.tables(device)
 
@@ -175,7 +176,7 @@ class Attention(Part):
                   unordered: bool = False):
         """The attention of rotated heads, and the product behind it."""
         context = attend(qkv, batch, view, self.num_heads, self.num_kv_heads, self.kernel_head_dim, self.window, self.scale,
-                         unmerged=(unordered or cuts_k(*self.w_o.shape)) and joins_merge(qkv.shape[0], self.w_o, residual))
+                         unmerged=(unordered or self.cuts_o) and joins_merge(qkv.shape[0], self.w_o, residual))
         if isinstance(context, Shares):
             ops.merge_project(context.part_o, context.part_ml, self.w_o, self.b_o, residual, self.num_heads, self.num_kv_heads,
                               self.kernel_head_dim, context.splits, context.tile_rows)
