@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import contextlib
 import functools
+import math
 
 from typing import Optional
 
@@ -802,17 +803,26 @@ FUSED_SHORT_K = 1024  # of which four waves have all in flight at once (two slic
 FUSED_LONG_K = 4096   # from which more than 16 rows may run as blocks of 16
 
 
-def _row_blocks(rows: int, row_tiles: int, column_tiles: int, groups: int, units: int) -> int:
+BLOCK_START = 4  # of a workgroup, in the time that 16 rows or columns of a slice take it
+
+
+def _row_blocks(rows: int, row_tiles: int, column_tiles: int, groups: int, units: int, k: int, whole: bool = True) -> float:
     """What a product of more than 16 rows takes, in the time that 16 rows or columns take a workgroup: it reads its columns of
-    the weight and its rows of A, and more workgroups than units take turns."""
-    return -(-groups * -(-rows // (16 * row_tiles)) // units) * (column_tiles + row_tiles)
+    the weight and its rows of A, and more workgroups than units take turns.  Of a short K the start counts too (q/k/v, 50 rows
+    x 10,240, K 136 6.7 us in blocks of 64 rows, 10.2 of 32; 121 x 5,120, K 88 6.5, 9.8), and the turns of the q/k/v
+    product, which hides a start behind the workgroup beside it, not only as ``whole`` ones."""
+    turns = groups * -(-rows // (16 * row_tiles)) / units
+    turns = math.ceil(turns) if whole or k > FUSED_SHORT_K else max(1.0, turns)
+    if k > FUSED_SHORT_K:
+        return turns * (column_tiles + row_tiles)
+    return turns * (BLOCK_START + -(-k // 512) * (column_tiles + row_tiles))
 
 
 @functools.lru_cache(maxsize=4096)
 def _plan_row_blocks(rows: int, tiles: int, k: int, units: int) -> tuple[int, int]:
     """(row tiles, waves) of a workgroup with one column tile.  Four waves where they have all of K in flight, or where there are
     workgroups for two on a unit (96 rows x 2,816, K 2,048 12.7 us, 13.8 with eight)."""
-    row_tiles = min((4, 2, 1) if k >= FUSED_LONG_K else (4, 2), key=lambda r: _row_blocks(rows, r, 1, tiles, units))
+    row_tiles = min((4, 2, 1) if k >= FUSED_LONG_K else (4, 2), key=lambda r: _row_blocks(rows, r, 1, tiles, units, k))
     fills = tiles * -(-rows // (16 * row_tiles)) * 4 >= FUSED_TARGET_WAVES
     short = k < FUSED_SHORT_K if row_tiles == 4 else k <= FUSED_SHORT_K
     return row_tiles, 4 if fills or short else 8
@@ -1298,11 +1308,11 @@ def gemm_tiles_rope(weight: torch.Tensor, a: torch.Tensor, bias: Optional[torch.
 
 @functools.lru_cache(maxsize=4096)
 def _plan_qkv_row_blocks(rows: int, pairs: int, k: int, units: int) -> tuple[int, int, bool]:
-    # (the waves of the plain product, so that both cut K alike: four keep too little of it in flight for four row tiles, and
+    # (the waves of the plain product, so that both cut K alike: four keep too little of a long K in flight for four row tiles, and
     # one row tile gained with the pair only)
     _, waves = _plan_row_blocks(rows, 2 * pairs, k, units)
-    forms = ((2, 1), (2, 2)) if waves == 4 else ((4, 1), (4, 2), (2, 1), (2, 2), (1, 2))
-    row_tiles, tiles = min(forms, key=lambda f: _row_blocks(rows, f[0], f[1], 2 * pairs // f[1], units))
+    forms = ((2, 1), (2, 2)) if waves == 4 and k > FUSED_SHORT_K else ((4, 1), (4, 2), (2, 1), (2, 2)) + (((1, 2),) if waves == 8 else ())
+    row_tiles, tiles = min(forms, key=lambda f: _row_blocks(rows, f[0], f[1], 2 * pairs // f[1], units, k, whole=False))
     return row_tiles, 4 if row_tiles <= 2 and k <= FUSED_SHORT_K else waves, tiles == 1
 
 

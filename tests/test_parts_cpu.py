@@ -206,6 +206,36 @@ def test_the_tiles_that_are_chosen_are_tiles_there_are(behind):
         assert picked is None or not picked.direct
 
 
+# (product, columns, rows, K, {(row tiles, waves, column tiles): us}) of 17 to 128 rows, as measured on MI355X
+BLOCKS = [
+    ("rope", 768, 59, 792, {(2, 4, 1): 5.64, (4, 4, 1): 7.76}),
+    ("rope", 1536, 36, 1008, {(2, 4, 1): 5.71, (1, 4, 2): 5.75, (4, 4, 1): 7.36}),
+    ("rope", 768, 122, 8176, {(2, 8, 1): 16.04, (1, 8, 2): 17.47, (4, 8, 2): 30.83}),
+    ("rope", 4608, 118, 512, {(4, 4, 2): 8.15, (1, 4, 2): 10.53, (2, 4, 2): 10.61, (2, 4, 1): 11.24}),
+    ("rope", 6144, 100, 64, {(4, 4, 2): 6.45, (1, 4, 2): 9.72, (2, 4, 2): 10.2}),
+    ("rope", 10240, 50, 136, {(4, 4, 2): 6.73, (1, 4, 2): 8.61, (2, 4, 2): 10.2}),
+    ("rope", 5120, 107, 600, {(4, 4, 2): 9.74, (1, 4, 2): 11.05, (2, 4, 2): 11.78}),
+    ("plain", 128, 104, 904, {(2, 4, 1): 4.27, (4, 4, 1): 6.21}),
+    ("plain", 912, 33, 864, {(2, 4, 1): 4.48, (4, 4, 1): 5.52}),
+    ("plain", 4496, 34, 280, {(4, 4, 1): 5.61, (2, 4, 1): 6.3}),
+    ("plain", 2224, 43, 352, {(4, 4, 1): 4.09, (2, 4, 1): 4.69}),
+    ("plain", 4832, 35, 416, {(4, 4, 1): 5.33, (2, 4, 1): 6.49}),
+    ("plain", 4000, 75, 352, {(4, 4, 1): 5.15, (2, 4, 1): 6.13}),
+]
+
+
+@pytest.mark.parametrize("product,n,rows,k,times", BLOCKS)
+def test_blocks_of_rows_are_those_that_were_measured_to_win(product, n, rows, k, times):
+    from cie_amd.kernels import ops
+
+    if product == "rope":
+        row_tiles, waves, one_tile = ops.plan_qkv_rope(rows, n // 32, k)
+        plan = (row_tiles, waves, 1 if one_tile else 2)
+    else:
+        plan = ops.plan_fused(rows, n // 16, k)
+    assert times[plan] <= 1.04 * min(times.values())
+
+
 def decode_form(monkeypatch, q_heads, kv_heads, dim, rows, longest, bound=None, unmerged=False, page=16):
     """(waves a part, parts, whether they come back unmerged) of a step of ``rows`` single tokens over up to ``longest`` keys, launch by
     launch, or as captured for up to ``bound`` keys."""
