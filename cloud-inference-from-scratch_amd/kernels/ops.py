@@ -1316,19 +1316,20 @@ def _plan_qkv_row_blocks(rows: int, pairs: int, k: int, units: int) -> tuple[int
     return row_tiles, 4 if row_tiles <= 2 and k <= FUSED_SHORT_K else waves, tiles == 1
 
 
-def plan_qkv_rope(rows: int, pairs: int, k: int) -> tuple[int, int, bool]:
+def plan_qkv_rope(rows: int, pairs: int, k: int, folded: bool = False) -> tuple[int, int, bool]:
     """(row tiles, waves per workgroup, whether a workgroup takes one tile of 16 columns and not a pair) of ``gemm_qkv_rope``
     for ``pairs`` pairs of tiles.  Up to 16 rows: one tile where the pairs leave half of the units without a workgroup (80 pairs
     8.1 -> 7.2 us), but for a short K, of which a pair's four waves have all in flight too, and read the rows once for twice the columns
-    (with the norm, one tile and a pair: 1,152 x 896 1 row 5.8, 5.2, 8 6.5 either way, 16 7.5, 7.0; 3,072 x 1,024 6.5, 6.1, 7.6 either way, 8.6, 8.0;
-    2,048 x 1,536 6.8, 8.1).  Beyond, as :func:`plan_fused` (MI355X, us, up to 64 rows a workgroup, one tile up to 64 rows and fewer than
+    (``folded``: with the norm made in the product, one tile and a pair: 1,152 x 896 1 row 5.8, 5.2, 8 6.5 either way, 16 7.5, 7.0; 3,072 x
+    1,024 6.5, 6.1, 7.6 either way, 8.6, 8.0; 2,048 x 1,536 6.8, 8.1; without it a pair gains up to a K of 512, 2 to 5 %, and loses beyond,
+    3,072 x 824, 16 rows 6.1, 6.6).  Beyond, as :func:`plan_fused` (MI355X, us, up to 64 rows a workgroup, one tile up to 64 rows and fewer than
     128 pairs, and what is taken: 2,560 x 2,048 48 rows 10.6, 9.2, 64 10.9, 9.9, 96 12.6, 10.4; 1,152 x 896 64 rows 8.1, 6.3, 96
     9.4, 6.4; 3,072 x 2,048 64 rows 11.7, 10.4; 5,120 x 1,024 96 rows 14.6, 10.2; 3,072 x 1,024 33 to 128 rows 0 to 12 % less)."""
     if rows > 16:
         return _plan_qkv_row_blocks(rows, pairs, k, compute_units())
     _, waves, _ = plan_fused(rows, pairs, k)
     few = pairs < QKV_SPLIT_PAIRS_BELOW
-    return 1, min(waves, 4) if few else waves, few and k > FUSED_SHORT_K
+    return 1, min(waves, 4) if few else waves, few and k > (FUSED_SHORT_K if folded else FUSED_SHORT_K // 2)
 
 
 def gemm_qkv_rope(weight: torch.Tensor, a: Optional[torch.Tensor], bias: Optional[torch.Tensor], cos: torch.Tensor,
@@ -1399,7 +1400,7 @@ def gemm_qkv_rope(weight: torch.Tensor, a: Optional[torch.Tensor], bias: Optiona
     _gpu("seq_slot", seq_slot, torch.int32, 1)
     _gpu("block_table", block_table, torch.int32, 2)
     page_size = _check_pools(k_pool, v_pool, torch.bfloat16, kv_heads, head_dim)
-    row_tiles, planned, one_tile = plan_qkv_rope(m, n // 32, k)
+    row_tiles, planned, one_tile = plan_qkv_rope(m, n // 32, k, folded is not None)
     waves = planned if waves is None else waves
     if blocks is not None:
         row_tiles, one_tile = blocks

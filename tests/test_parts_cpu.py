@@ -236,6 +236,16 @@ def test_blocks_of_rows_are_those_that_were_measured_to_win(product, n, rows, k,
     assert times[plan] <= 1.04 * min(times.values())
 
 
+@pytest.mark.parametrize("rows", [1, 10, 16])
+def test_few_rows_take_a_pair_of_column_tiles_where_that_was_measured_to_win(rows):
+    """q/k/v of a short K, whose workgroups make the norm of the rows, or read them."""
+    from cie_amd.kernels import ops
+
+    one_tile = lambda k, folded: ops.plan_qkv_rope(rows, 72, k, folded)[2]  # noqa: E731
+    assert [one_tile(k, True) for k in (64, 512, 824, 1024, 1032)] == [False, False, False, False, True]
+    assert [one_tile(k, False) for k in (64, 512, 520, 824, 1024)] == [False, False, True, True, True]
+
+
 def decode_form(monkeypatch, q_heads, kv_heads, dim, rows, longest, bound=None, unmerged=False, page=16):
     """(waves a part, parts, whether they come back unmerged) of a step of ``rows`` single tokens over up to ``longest`` keys, launch by
     launch, or as captured for up to ``bound`` keys."""
