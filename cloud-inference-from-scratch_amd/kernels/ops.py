@@ -804,24 +804,27 @@ FUSED_LONG_K = 4096   # from which more than 16 rows may run as blocks of 16
 
 
 BLOCK_START = 4  # of a workgroup, in the time that 16 rows or columns of a slice take it
+BLOCK_WAITS = 1.25  # ... a slice of four row tiles behind another, which have one in flight
 
 
 def _row_blocks(rows: int, row_tiles: int, column_tiles: int, groups: int, units: int, k: int, whole: bool = True) -> float:
     """What a product of more than 16 rows takes, in the time that 16 rows or columns take a workgroup: it reads its columns of
     the weight and its rows of A, and more workgroups than units take turns.  Of a short K the start counts too (q/k/v, 50 rows
-    x 10,240, K 136 6.7 us in blocks of 64 rows, 10.2 of 32; 121 x 5,120, K 88 6.5, 9.8), and the turns of the q/k/v
-    product, which hides a start behind the workgroup beside it, not only as ``whole`` ones."""
+    x 10,240, K 136 6.7 us in blocks of 64 rows, 10.2 of 32; 121 x 5,120, K 88 6.5, 9.8), four row tiles wait for the second of a wave's slices
+    (83 x 5,120, K 520 9.4, 7.8), and the q/k/v product, which hides a start behind the workgroup beside it, does not take ``whole`` turns
+    only."""
     turns = groups * -(-rows // (16 * row_tiles)) / units
     turns = math.ceil(turns) if whole or k > FUSED_SHORT_K else max(1.0, turns)
     if k > FUSED_SHORT_K:
         return turns * (column_tiles + row_tiles)
-    return turns * (BLOCK_START + -(-k // 512) * (column_tiles + row_tiles))
+    slices = -(-k // 512)  # of a wave
+    return turns * (BLOCK_START + slices * (column_tiles + row_tiles) * (BLOCK_WAITS if row_tiles == 4 and slices > 1 else 1.0))
 
 
 @functools.lru_cache(maxsize=4096)
 def _plan_row_blocks(rows: int, tiles: int, k: int, units: int) -> tuple[int, int]:
     """(row tiles, waves) of a workgroup with one column tile.  Four waves where they have all of K in flight, or where there are
-    workgroups for two on a unit (96 rows x 2,816, K 2,048 12.7 us, 13.8 with eight)."""
+    workgroups for two on a unit (96 rows x 2,816, K 2,048 12.0 us, a tenth more with eight)."""
     row_tiles = min((4, 2, 1) if k >= FUSED_LONG_K else (4, 2), key=lambda r: _row_blocks(rows, r, 1, tiles, units, k))
     fills = tiles * -(-rows // (16 * row_tiles)) * 4 >= FUSED_TARGET_WAVES
     short = k < FUSED_SHORT_K if row_tiles == 4 else k <= FUSED_SHORT_K
@@ -834,9 +837,9 @@ def plan_fused(rows: int, column_tiles: int, k: int) -> tuple[int, int, int]:
     each streaming the weight again).  With more than 16 rows a workgroup takes
     two column tiles if that still leaves enough workgroups (each activation
     value a wave loads then meets two weight tiles), else as many rows as have the units read least (``_row_blocks``).  MI355X, us, up to 64 rows a workgroup and as many as are taken:
-    2,048 x 2,048 64 rows 10.2, 8.2 (128 and 256 workgroups), 128 rows 10.4 either way; 896 x 896 64 rows 7.3, 5.3, 128 7.4, 5.4;
-    1,024 x 4,096 64 rows 15.3, 9.8; 2,304 x 2,304 64 rows 10.9 either way, 96 14.9, 12.0; 4,096 x 1,024 32 rows with eight and four
-    waves 7.6, 6.5.  Up to 16 rows as many waves share K as it
+    2,048 x 2,048 64 rows 9.7, 7.7 (128 and 256 workgroups), 128 rows 9.7 either way; 896 x 896 64 rows 6.7, 4.8, 128 6.8, 4.9;
+    1,024 x 4,096 64 rows 14.5, 9.4; 2,304 x 2,304 64 rows 10.2 either way, 96 14.0, 11.1; 4,096 x 1,024 32 rows with eight and four
+    waves 7.3, 6.3.  Up to 16 rows as many waves share K as it
     takes to fill the GPU, each with at least one 128-wide slice."""
     pair = column_tiles >= 2 * FUSED_PAIR_WORKGROUPS
     if rows > 16 and not pair:
@@ -1323,8 +1326,8 @@ def plan_qkv_rope(rows: int, pairs: int, k: int, folded: bool = False) -> tuple[
     (``folded``: with the norm made in the product, one tile and a pair: 1,152 x 896 1 row 5.8, 5.2, 8 6.5 either way, 16 7.5, 7.0; 3,072 x
     1,024 6.5, 6.1, 7.6 either way, 8.6, 8.0; 2,048 x 1,536 6.8, 8.1; without it a pair gains up to a K of 512, 2 to 5 %, and loses beyond,
     3,072 x 824, 16 rows 6.1, 6.6).  Beyond, as :func:`plan_fused` (MI355X, us, up to 64 rows a workgroup, one tile up to 64 rows and fewer than
-    128 pairs, and what is taken: 2,560 x 2,048 48 rows 10.6, 9.2, 64 10.9, 9.9, 96 12.6, 10.4; 1,152 x 896 64 rows 8.1, 6.3, 96
-    9.4, 6.4; 3,072 x 2,048 64 rows 11.7, 10.4; 5,120 x 1,024 96 rows 14.6, 10.2; 3,072 x 1,024 33 to 128 rows 0 to 12 % less)."""
+    128 pairs, and what is taken: 2,560 x 2,048 48 rows 9.8, 8.7, 64 10.1, 9.3, 96 11.7, 9.4; 1,152 x 896 64 rows 7.8, 5.7, 96
+    8.9, 5.7; 3,072 x 2,048 64 rows 10.6, 9.6)."""
     if rows > 16:
         return _plan_qkv_row_blocks(rows, pairs, k, compute_units())
     _, waves, _ = plan_fused(rows, pairs, k)

@@ -215,6 +215,8 @@ BLOCKS = [
     ("rope", 6144, 100, 64, {(4, 4, 2): 6.45, (1, 4, 2): 9.72, (2, 4, 2): 10.2}),
     ("rope", 10240, 50, 136, {(4, 4, 2): 6.73, (1, 4, 2): 8.61, (2, 4, 2): 10.2}),
     ("rope", 5120, 107, 600, {(4, 4, 2): 9.74, (1, 4, 2): 11.05, (2, 4, 2): 11.78}),
+    ("rope", 5120, 83, 520, {(2, 4, 2): 7.77, (4, 4, 2): 9.35, (1, 4, 2): 9.76}),
+    ("rope", 3072, 117, 800, {(4, 8, 2): 7.44, (2, 4, 2): 7.54, (1, 4, 2): 7.75, (4, 4, 2): 8.97}),
     ("plain", 128, 104, 904, {(2, 4, 1): 4.27, (4, 4, 1): 6.21}),
     ("plain", 912, 33, 864, {(2, 4, 1): 4.48, (4, 4, 1): 5.52}),
     ("plain", 4496, 34, 280, {(4, 4, 1): 5.61, (2, 4, 1): 6.3}),
