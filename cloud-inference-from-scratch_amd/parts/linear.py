@@ -41,8 +41,8 @@ FUSED_ROWS = 16
 # 36.3 / 39.8 / 48.2 against 50.0 / 61.6 / 60.9: the library has no good algorithm for a long K and few rows, and at
 # row counts that do not recur it takes its heuristic's first choice)
 FUSED_PARTS_ROWS = 128
-# With 17 to 128 rows it also wins where the weight is small (q/k/v and o_proj of the 3B shape at 32 / 64 / 96 rows: 8.5 / 9.9 /
-# 10.4 us and 8.0 / 8.2 / 9.6 against the library's 12-18 us inside a step at up to 64 rows and 9.1-12.4 beyond;
+# With 17 to 128 rows it also wins where the weight is small (q/k/v and o_proj of the 3B shape at 32 / 64 / 96 rows: 7.7 / 9.3 /
+# 9.4 us and 7.4 / 7.7 / 9.0 against the library's 12-18 us inside a step at up to 64 rows and 9.1-12.4 beyond;
 # and the rotation, the cache write, the residual add and the next
 # norm ride along); from about 6M weight values on the library is faster (7B o_proj at 64 rows: 12.6 us against
 # 11.1 us).
